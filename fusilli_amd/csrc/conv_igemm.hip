@@ -227,10 +227,12 @@ ConvPlan make_plan(const fhip_conv_desc *d, const fhip_conv_desc *orig = nullptr
   const FhipKnobs &knobs = fhip_knobs();
   if (knobs.conv_tile_bm) {
     const int bm = knobs.conv_tile_bm, bn = knobs.conv_tile_bn;
-    if ((bm == 128 || bm == 256 || (bm == 512 && bn == 128)) &&
-        (bn == 128 || bn == 256) && bm >= bn)
+    if ((bm == 128 || bm == 256) && (bn == 128 || bn == 256) && bm >= bn)
       p.bm = bm, p.bn = bn;
   }
+  // (that tile's gather keeps validity masks of 8 filter rows and columns)
+  if (p.bm == 256 && p.bn == 256 && (R > 8 || g.S > 8))
+    p.bm = p.bn = 128;
   // Halo mode (the slab of input pixels stays in LDS for all taps): unit
   // stride, output extent == input extent, and a slab small enough that two
   // workgroups still share a compute unit.  FUSILLI_HIP_CONV_HALO=0 / 1

@@ -235,9 +235,6 @@ __device__ __forceinline__ void mfma16(typename KindTraits<KIND>::AccVec4 &c,
   }
 }
 
-#ifndef GEMM_M16
-#define GEMM_M16 1
-#endif
 #define GEMM_AS1 __attribute__((address_space(1)))
 #define GEMM_AS3 __attribute__((address_space(3)))
 
@@ -289,16 +286,18 @@ template <int ELEM, int RB, int XB> __device__ __forceinline__ int nkc_chunk(int
 }
 
 // Per-thread byte offsets (from the tile's first row / column at K = 0) of the
-// chunks this thread's DMA instructions fetch; the same for every K slice.
-template <int ROWS, int ELEM, bool KCONTIG, int NW, int XB>
+// chunks this thread's DMA instructions fetch; the same for every K slice.  NW
+// wavefronts share the operand's loads: this one moves the 1 KB groups (8 rows,
+// or kRowsPerLoad K-rows) group0, group0 + STEP, ...
+template <int ROWS, int ELEM, bool KCONTIG, int NW, int STEP, int XB>
 __device__ __forceinline__ void
-dma_setup(int64_t ld_bytes, int64_t row0, int64_t rows_total,
+dma_setup(int group0, int64_t ld_bytes, int64_t row0, int64_t rows_total,
           uint32_t (&off)[SliceGeom<ROWS, ELEM, KCONTIG, NW>::kLoads]) {
   using G = SliceGeom<ROWS, ELEM, KCONTIG, NW>;
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  const int l = threadIdx.x & 63;
 #pragma unroll
   for (int j = 0; j < G::kLoads; ++j) {
-    const int group = j * NW + w;
+    const int group = group0 + j * STEP;
     if constexpr (KCONTIG) {
       const int row = group * 8 + (l >> 3);
       const int c = (l & 7) ^ kc_swz(row);
@@ -316,16 +315,16 @@ dma_setup(int64_t ld_bytes, int64_t row0, int64_t rows_total,
   }
 }
 
-// One K slice of one operand, global -> LDS: each wavefront instruction moves
+// This wavefront's loads of one K slice of one operand, global -> LDS (its first
+// group to `lds_dst`, the others STEP KB apart): each wavefront instruction moves
 // 64 x 16 bytes to 1024 consecutive LDS bytes.  Buffer addressing (uniform
 // 64-bit base + 32-bit lane offset) keeps these loads on the vector-memory
 // counter only, so waits on LDS reads stay exact while they are in flight;
 // offsets at or past `bytes` read as zero.
-template <int NW, int LOADS, int J0 = 0, int J1 = LOADS>
+template <int STEP, int LOADS, int J0 = 0, int J1 = LOADS>
 __device__ __forceinline__ void dma_issue(const char *base, uint32_t bytes,
                                           const uint32_t (&off)[LOADS],
-                                          uint32_t lds_stage) {
-  const int w = threadIdx.x >> 6;
+                                          uint32_t lds_dst) {
   // the descriptor must sit in scalar registers: say so, or 64-bit pointer
   // arithmetic done on the vector ALU forces a per-lane loop around each load
   const uint64_t b64 = (uint64_t)base;
@@ -336,7 +335,7 @@ __device__ __forceinline__ void dma_issue(const char *base, uint32_t bytes,
       (int)__builtin_amdgcn_readfirstlane(bytes), 0x00020000);
 #pragma unroll
   for (int j = J0; j < J1; ++j) {
-    const uint32_t dst = lds_stage + (uint32_t)(j * NW + w) * 1024u;
+    const uint32_t dst = lds_dst + (uint32_t)(j * STEP) * 1024u;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(
         rsrc, (GEMM_AS3 char *)__builtin_amdgcn_readfirstlane(dst), 16,
         (int)off[j], 0, 0, 0);
@@ -594,13 +593,13 @@ __device__ __forceinline__ void load_operand_vec(const void *p, int dt,
 // LDS bytes of the kernel: NSTAGE stages of (A slice + B slice); the epilogue
 // reuses it for four 32-row accumulator bands (one per wavefront).
 // Wavefront grid of a tile.  8 wavefronts (two per SIMD, scheduled in
-// alternating memory / MFMA phases): 256 x 256 as 2 x 4 and 512 x 128 as 4 x 2,
-// each wavefront owning 128 x 64 outputs, 256 x 128 as 4 x 2 of 64 x 64 and
+// alternating memory / MFMA phases): 256 x 256 as 2 x 4, each wavefront owning
+// 128 x 64 outputs, 256 x 128 as 4 x 2 of 64 x 64 and
 // 128 x 128 (GEMM, gather convolution) as 2 x 4 of 64 x 32; 4 wavefronts (the
 // halo convolution) as 2 x 2.
 template <int BM, int BN, int NW = 0> struct GemmLayout {
   static constexpr bool kWide = BM == 256 && BN == 256;
-  static constexpr bool kTall = (BM == 512 || (BM == 256 && NW == 8)) && BN == 128;
+  static constexpr bool kTall = BM == 256 && BN == 128 && NW == 8;
   static constexpr bool kSmall8 = BM == 128 && BN == 128 && NW == 8; // 64 x 32 per wavefront
   static constexpr int kWavesM = kTall ? 4 : 2;
   static constexpr int kWavesN = kWide || kSmall8 ? 4 : 2;
@@ -609,6 +608,11 @@ template <int BM, int BN, int NW = 0> struct GemmLayout {
 
 template <int BM, int BN, int NSTAGE, int NW, bool HALO = false> struct GemmLds {
   static constexpr int kStage = (BM + BN) * kTileKBytes;
+  // Eight wavefronts: two stages of A, filled by wavefronts 0..3, and three of
+  // B, filled by wavefronts 4..7 (see the loop)
+  // (the 256 x 256 gather deals out halves of both: the same bytes)
+  static constexpr int kRing =
+      NW == 8 ? (2 * BM + 3 * BN) * kTileKBytes : NSTAGE * kStage;
   static constexpr int kWN = BN / GemmLayout<BM, BN, NW>::kWavesN; // wave columns
   static constexpr int kEpiPitch = kWN * 4 + 32;
   static constexpr int kBand = 32 * kEpiPitch; // one wavefront, one tile row
@@ -616,12 +620,11 @@ template <int BM, int BN, int NSTAGE, int NW, bool HALO = false> struct GemmLds 
   // tile rows that leave together: as many as fit 160 KB, or 80 KB where the
   // stages leave room for two workgroups per compute unit
   static constexpr int kCap =
-      HALO || NSTAGE * kStage <= 80 * 1024 ? 80 * 1024 : 160 * 1024;
+      HALO || kRing <= 80 * 1024 ? 80 * 1024 : 160 * 1024;
   static constexpr int kBands =
       NW * kTM * kBand <= kCap ? kTM : (NW * 2 * kBand <= kCap ? 2 : 1);
   static constexpr int kEpiBytes = NW * kBands * kBand;
-  static constexpr int kBytes =
-      NSTAGE * kStage > kEpiBytes ? NSTAGE * kStage : kEpiBytes;
+  static constexpr int kBytes = kRing > kEpiBytes ? kRing : kEpiBytes;
 };
 
 // Halo kernels are laid out for two workgroups per compute unit (two
@@ -636,8 +639,17 @@ gemm_kernel(GemmArgs g) {
   constexpr int STEPB = KindTraits<KIND>::kStepBytes;
   constexpr int KSTEPS = kTileKBytes / STEPB;
   static_assert(KSTEPS % 2 == 0, "fragment double buffering needs even KSTEPS");
-  using GA = SliceGeom<BM, ELEM, A_KC, NW>;
-  using GB = SliceGeom<BN, ELEM, B_KC, NW>;
+  constexpr bool PINGPONG = NW == 8;
+  // Who loads what in the two-phase loop: wavefronts 0..3 (team 0) A and 4..7
+  // (team 1) B; in the 256 x 256 gather, where eight gathered loads per
+  // wavefront do not fit the registers, team 0 the upper half of either
+  // operand's rows and team 1 the lower half.
+  constexpr bool HALVES = A_MODE == A_CONV && BM == 256 && BN == 256;
+  constexpr bool TEAMS = PINGPONG && !HALVES;
+  constexpr int LSTEP = PINGPONG ? 4 : NW; // 1 KB groups between a wavefront's loads
+  constexpr int LW = TEAMS ? 4 : NW; // wavefronts that share an operand's loads
+  using GA = SliceGeom<BM, ELEM, A_KC, LW>;
+  using GB = SliceGeom<BN, ELEM, B_KC, LW>;
   using L = GemmLds<BM, BN, NSTAGE, NW, A_MODE == A_HALO>;
   constexpr int WAVES_M = GemmLayout<BM, BN, NW>::kWavesM;
   constexpr int WAVES_N = GemmLayout<BM, BN, NW>::kWavesN;
@@ -649,11 +661,11 @@ gemm_kernel(GemmArgs g) {
   // The ping-pong GEMM tiles use the 16 x 16 MFMA shapes (twice the K per
   // instruction): on operands with random bits the matrix pipe sustains 13 to
   // 21 % more with them than with the 32 x 32 shapes.
-  constexpr bool M16 = GEMM_M16 && NW == 8;
+  constexpr bool M16 = NW == 8;
   constexpr int XB = M16 ? Frag16Geom<KIND>::XB : 0; // (M/N-contiguous LDS layout)
   constexpr int KSTEPS16 = KSTEPS / 2;
   constexpr int TM16 = WM / 16, TN16 = WN / 16;
-  // DMA instructions per slice
+  // DMA instructions per slice and wavefront (in-order loop)
   constexpr int LPS = (HALO ? 0 : GA::kLoads) + GB::kLoads;
 
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -698,12 +710,23 @@ gemm_kernel(GemmArgs g) {
   // A and B tile base pointers at K = 0 and their per-slice advance.
   const char *a_base;
   int64_t a_step;
-  uint32_t off_a[GA::kLoads], off_b[GB::kLoads];
-  // implicit-GEMM gather: pixel index of tap (0, 0) and in-image row / column
-  // masks of the filter
-  int32_t cv_pix[A_MODE == A_CONV ? GA::kLoads : 1];
-  uint32_t cv_mask[A_MODE == A_CONV ? GA::kLoads : 1];
-  int cv_chunk = 0;
+  // (eight wavefronts: a wavefront loads one operand only, A's offsets -- for
+  // the gather its pixels -- or B's in the same registers)
+  const int team = PINGPONG ? __builtin_amdgcn_readfirstlane(wave >> 2) : 0;
+  constexpr int NOFF = TEAMS ? (GA::kLoads > GB::kLoads ? GA::kLoads : GB::kLoads)
+                             : GA::kLoads + GB::kLoads;
+  uint32_t off_t[NOFF];
+  uint32_t(&off_a)[GA::kLoads] = *(uint32_t(*)[GA::kLoads])&off_t[0];
+  uint32_t(&off_b)[GB::kLoads] = *(uint32_t(*)[GB::kLoads])&off_t[TEAMS ? 0 : GA::kLoads];
+  const int w_load = wave & (LSTEP - 1);
+  const int group_a = w_load + (HALVES && !team ? 4 * GA::kLoads : 0);
+  const int group_b = w_load + (HALVES && !team ? 4 * GB::kLoads : 0);
+  // implicit-GEMM gather: off_a holds the byte offset of tap (0, 0), modulo
+  // 2^32; in-image row / column masks of the filter
+  // (the 256 x 256 tile is short of registers: masks of at most 8 filter rows and
+  // columns, two loads to a register)
+  constexpr int MASK_BITS = HALVES ? 8 : 16;
+  uint32_t cv_mask[A_MODE == A_CONV ? GA::kLoads * MASK_BITS / 16 : 1] = {};
   // halo mode: slab row of tap (0, 0) and the validity masks of this lane's
   // fragment rows
   int32_t h_row[HALO ? TM : 1];
@@ -716,7 +739,7 @@ gemm_kernel(GemmArgs g) {
     a_step = 0;
 #pragma unroll
     for (int j = 0; j < GA::kLoads; ++j) {
-      const int row = (j * NW + wave) * 8 + (l >> 3);
+      const int row = (group_a + j * LSTEP) * 8 + (l >> 3);
       const int64_t m = m0 + row;
       const bool live = m < m_end;
       const int32_t mm = (int32_t)(live ? m : 0);
@@ -726,8 +749,10 @@ gemm_kernel(GemmArgs g) {
       const int32_t pp = pq - nn * g.conv.P;
       const int32_t ih0 = pp * g.conv.str_h - g.conv.pad_h;
       const int32_t iw0 = q * g.conv.str_w - g.conv.pad_w;
-      cv_pix[j] = (nn * g.conv.H + ih0) * g.conv.W + iw0;
-      // bits 0..15: filter rows inside the image, 16..31: filter columns
+      off_a[j] = (uint32_t)((nn * g.conv.H + ih0) * g.conv.W + iw0) *
+                     (uint32_t)g.conv.x_pitch +
+                 (uint32_t)(((l & 7) ^ kc_swz(row)) * 16);
+      // low half: filter rows inside the image, high half: filter columns
       uint32_t mask = 0;
       for (int fr = 0; fr < g.conv.R; ++fr)
         mask |= (uint32_t)(live && (uint32_t)(ih0 + fr * g.conv.dil_h) <
@@ -736,20 +761,22 @@ gemm_kernel(GemmArgs g) {
       for (int fs = 0; fs < g.conv.S; ++fs)
         mask |= (uint32_t)((uint32_t)(iw0 + fs * g.conv.dil_w) <
                            (uint32_t)g.conv.W)
-                << (16 + fs);
-      cv_mask[j] = mask;
-      cv_chunk = ((l & 7) ^ kc_swz(row)) * 16; // same for every j
+                << (MASK_BITS + fs);
+      if constexpr (HALVES)
+        cv_mask[j / 2] |= mask << (j & 1) * 16;
+      else
+        cv_mask[j] = mask;
     }
   } else if constexpr (A_KC) {
     a_step = kTileKBytes;
     a_base = g.a + (batch * g.a_batch + outer * g.a_outer) * ELEM + m0 * a_ldb +
              kt_base * a_step;
-    dma_setup<BM, ELEM, true, NW, XB>(a_ldb, m0, m_end, off_a);
+    dma_setup<BM, ELEM, true, LW, LSTEP, XB>(group_a, a_ldb, m0, m_end, off_a);
   } else {
     a_step = (int64_t)GA::kKRows * a_ldb;
     a_base = g.a + (batch * g.a_batch + outer * g.a_outer) * ELEM + m0 * ELEM +
              kt_base * a_step;
-    dma_setup<BM, ELEM, false, NW, XB>(a_ldb, m0, m_end, off_a);
+    dma_setup<BM, ELEM, false, LW, LSTEP, XB>(group_a, a_ldb, m0, m_end, off_a);
   }
   const char *b_base;
   int64_t b_step;
@@ -762,56 +789,79 @@ gemm_kernel(GemmArgs g) {
     b_base = g.b + (batch * g.b_batch + outer * g.b_outer) * ELEM + n0 * ELEM +
              kt_base * b_step;
   }
-  dma_setup<BN, ELEM, B_KC, NW, XB>(b_ldb, n0, g.N, off_b);
+  if (!TEAMS || team) // (after A's: they share registers)
+    dma_setup<BN, ELEM, B_KC, LW, LSTEP, XB>(group_b, b_ldb, n0, g.N, off_b);
 
-  // halo mode: [slab | ring of B slices]; otherwise a ring of (A, B) slices
+  // halo mode: [slab | ring of B slices]; four wavefronts: a ring of (A, B)
+  // slices; eight: a ring of A slices and one of B slices, or the rings of the
+  // halves (A's part first)
   constexpr uint32_t STAGE = HALO ? GB::kBytes : L::kStage;
   const uint32_t ring0 = HALO ? lds0 + g.conv.slab_bytes : lds0;
-  auto stage_a = [&](int st) { return ring0 + (uint32_t)st * STAGE; };
-  auto stage_b = [&](int st) {
-    return ring0 + (uint32_t)st * STAGE + (HALO ? 0 : GA::kBytes);
+  auto stage_a = [&](int st) {
+    return ring0 + (uint32_t)st * (PINGPONG ? (uint32_t)GA::kBytes : STAGE);
   };
-  // Part PART of PARTS of slice kt's loads (A and B split alike).
+  auto stage_b = [&](int st) {
+    if constexpr (PINGPONG)
+      return ring0 + 2u * GA::kBytes + (uint32_t)st * GB::kBytes;
+    else
+      return ring0 + (uint32_t)st * STAGE + (HALO ? 0 : GA::kBytes);
+  };
+  auto stage_half = [&](int t, int st) { // of the half that team t loads
+    return lds0 + (t ? 0u : 3u * GA::kBytes) + (uint32_t)st * GA::kBytes;
+  };
+  // Part PART of PARTS of slice kt's loads of one operand.
   // Slices past the end of K are not loaded at all; the loops' waits by count
   // become waits for everything where a batch is missing.  (They used to be
   // "loaded" through zero-sized buffers, which kept every iteration identical;
   // but such a load counts as complete before its zeros are written to LDS:
   // on tiles whose real loads return quickly the zeros of the last batch
   // could land in the epilogue's bands, after the final wait and barrier.)
-  auto issue = [&](int kt, int st, auto part_c, auto parts_c) {
+  auto issue_a = [&](int kt, int st, auto part_c, auto parts_c) {
     if (kt >= kt_count)
       return;
     const uint32_t lim = 0xffffffffu;
     constexpr int PART = decltype(part_c)::value;
     constexpr int PARTS = decltype(parts_c)::value;
     constexpr int A0 = PART * GA::kLoads / PARTS, A1 = (PART + 1) * GA::kLoads / PARTS;
-    constexpr int B0 = PART * GB::kLoads / PARTS, B1 = (PART + 1) * GB::kLoads / PARTS;
+    const uint32_t dst =
+        (HALVES ? stage_half(team, st) : stage_a(st)) + (uint32_t)w_load * 1024u;
     if constexpr (HALO) {
       // only the filter streams
     } else if constexpr (A_MODE == A_CONV) {
       const int32_t ktg = kt + kt_base;
       const int32_t tap = conv_div(ktg, g.conv.slices_per_tap, g.conv.magic_spt);
-      const int32_t cb =
-          (ktg - tap * g.conv.slices_per_tap) * kTileKBytes + cv_chunk;
       const int32_t fr = conv_div(tap, g.conv.S, g.conv.magic_s);
       const int32_t fs = tap - fr * g.conv.S;
-      const int32_t dpix = fr * g.conv.dil_h * g.conv.W + fs * g.conv.dil_w;
-      const int32_t cbytes = g.conv.x_pitch;
+      // (uniform: one addition and one mask test per load remain for the lanes)
+      const uint32_t at = (uint32_t)((fr * g.conv.dil_h * g.conv.W + fs * g.conv.dil_w) *
+                                         g.conv.x_pitch +
+                                     (ktg - tap * g.conv.slices_per_tap) * kTileKBytes);
+      const uint32_t need = (1u << fr) | (1u << (MASK_BITS + fs));
       uint32_t off[GA::kLoads];
 #pragma unroll
       for (int j = A0; j < A1; ++j) {
-        const bool in = (cv_mask[j] >> fr) & (cv_mask[j] >> (16 + fs)) & 1;
         // taps outside the image (and rows past M) read past the end: zeros
-        off[j] = in ? (uint32_t)((cv_pix[j] + dpix) * cbytes + cb) : 0x80000000u;
+        const uint32_t need_j = HALVES ? need << (j & 1) * 16 : need;
+        off[j] = (cv_mask[HALVES ? j / 2 : j] & need_j) == need_j ? off_a[j] + at : 0x80000000u;
       }
-      dma_issue<NW, GA::kLoads, A0, A1>(a_base, g.conv.x_bytes & lim, off,
-                                    stage_a(st));
+      dma_issue<LSTEP, GA::kLoads, A0, A1>(a_base, g.conv.x_bytes & lim, off, dst);
     } else {
-      dma_issue<NW, GA::kLoads, A0, A1>(a_base + kt * a_step, lim, off_a,
-                                    stage_a(st));
+      dma_issue<LSTEP, GA::kLoads, A0, A1>(a_base + kt * a_step, lim, off_a, dst);
     }
-    dma_issue<NW, GB::kLoads, B0, B1>(b_base + kt * b_step, lim, off_b,
-                                  stage_b(st));
+  };
+  auto issue_b = [&](int kt, int st, auto part_c, auto parts_c) {
+    if (kt >= kt_count)
+      return;
+    constexpr int PART = decltype(part_c)::value;
+    constexpr int PARTS = decltype(parts_c)::value;
+    constexpr int B0 = PART * GB::kLoads / PARTS, B1 = (PART + 1) * GB::kLoads / PARTS;
+    const uint32_t dst =
+        (HALVES ? stage_half(team, st) + GA::kBytes / 2 : stage_b(st)) + (uint32_t)w_load * 1024u;
+    dma_issue<LSTEP, GB::kLoads, B0, B1>(b_base + kt * b_step, 0xffffffffu, off_b, dst);
+  };
+  auto issue = [&](int kt, int st, auto part_c, auto parts_c) {
+    issue_a(kt, st, part_c, parts_c);
+    issue_b(kt, st, part_c, parts_c);
   };
   using One = std::integral_constant<int, 1>;
   using Zero = std::integral_constant<int, 0>;
@@ -850,13 +900,19 @@ gemm_kernel(GemmArgs g) {
       *(GEMM_AS3 u32x4 *)(uintptr_t)(ring0 - kTileKBytes + threadIdx.x * 16) =
           u32x4{0, 0, 0, 0};
   }
-  constexpr bool PINGPONG = NW == 8;
   if constexpr (PINGPONG) {
-    // slice 0, and the share of slice 1 that wavefronts 4..7 own (see the loop)
-    static_assert(NSTAGE == 2, "ping-pong tiles alternate two stages");
-    issue(0, 0, Zero{}, One{});
-    if (wave >= 4)
-      issue(1, 1, Zero{}, One{}); // (nothing when there is one slice)
+    // slice 0 of A from wavefronts 0..3, slices 0 and 1 of B from 4..7 (see the loop)
+    static_assert(NSTAGE == 2, "ping-pong tiles alternate two stages of A");
+    if constexpr (HALVES) {
+      issue(0, 0, Zero{}, One{});
+      if (team)
+        issue(1, 1, Zero{}, One{}); // (nothing when there is one slice)
+    } else if (team) {
+      issue_b(0, 0, Zero{}, One{});
+      issue_b(1, 1, Zero{}, One{});
+    } else {
+      issue_a(0, 0, Zero{}, One{});
+    }
   } else {
 #pragma unroll
     for (int p = 0; p < NSTAGE; ++p)
@@ -920,9 +976,9 @@ gemm_kernel(GemmArgs g) {
     }
   }
   if constexpr (PINGPONG) {
-    // slice 0 has landed (wavefronts 4..7 keep their share of slice 1 in flight)
-    if (wave >= 4 && kt_count > 1)
-      __builtin_amdgcn_s_waitcnt(gemm_wait_imm(LPS));
+    // slice 0 has landed (wavefronts 4..7 keep slice 1 of their part in flight)
+    if (team && kt_count > 1)
+      __builtin_amdgcn_s_waitcnt(gemm_wait_imm(HALVES ? LPS : GB::kLoads));
     else
       __builtin_amdgcn_s_waitcnt(gemm_wait_imm(0));
     gemm_barrier();
@@ -997,63 +1053,73 @@ gemm_kernel(GemmArgs g) {
     // wavefronts 0..3 (team 0), so on every SIMD one wavefront feeds the
     // matrix pipe while the other issues memory instructions.  With g = global
     // phase number:
-    //   g = 2 kt     : team 0 reads slice kt, loads its share of slice kt + 1
-    //                  into the other stage (team 1 finished reading that
+    //   g = 2 kt     : team 0 reads slice kt and loads A's slice kt + 1 into
+    //                  the other of two stages (team 1 finished reading that
     //                  stage in phase 2 kt - 1)            | team 1: MFMA(kt-1)
-    //   g = 2 kt + 1 : team 0: MFMA(kt), then waits for its share of slice
-    //                  kt + 1 | team 1 reads slice kt and, once those reads
-    //                  have returned, loads its share of slice kt + 2 into the
-    //                  same stage (team 0 read it in phase 2 kt); it then
-    //                  waits for its share of slice kt + 1
-    // so slice kt + 1 is complete when phase 2 kt + 2 starts, and every load
-    // has two phases to land.
-    // (A wavefront of team 1 requests its share of slice kt + 2 once ITS reads
-    // of the stage have returned; its three team mates, released by the same
-    // barrier and served by LDS in turns, finish theirs within a few hundred
-    // clocks of it, and the requested data is at least a cache round trip and
-    // the rest of the phase away.  Requesting after the next barrier instead,
-    // in front of the MFMAs, measured 4-5 % slower; dealt out between the
-    // MFMAs it needs a loop per team, and then the compiler no longer keeps
-    // the asm transposing reads' results where they land.)
-    const int team = __builtin_amdgcn_readfirstlane(wave >> 2);
-    Frag<KIND> pa[KSTEPS][TM], pb[KSTEPS][TN];
+    //   g = 2 kt + 1 : team 0: MFMA(kt), then waits for A's slice kt + 1 |
+    //                  team 1 reads slice kt and loads B's slice kt + 2 into
+    //                  the third stage of B, which held slice kt - 1 (team 1
+    //                  read that in phase 2 kt - 1, team 0 a phase earlier);
+    //                  it then waits for B's slice kt + 1
+    // so slice kt + 1 is complete when phase 2 kt + 2 starts, every load has
+    // two phases or more to land, and no load targets a stage that a wavefront
+    // may still be reading: a barrier lies between a stage's last read and the
+    // request that refills it, for both operands.  (With two stages of both
+    // operands and each team loading half of each, a wavefront of team 1 could
+    // only know that ITS reads of the stage had returned; a slower team mate
+    // then read columns of slice kt + 2: a 320 -> 128 channel 3 x 3 convolution
+    // at stride 2, N30 63 x 63, gave other bits in 20 runs of 20.  Times are
+    // those of the two-stage loop or better: bf16 4096^3 97 -> 96 us, fp8
+    // 4096 x 4096 x 8192 91.5 -> 90.9, bf16 2048^3 25.5 -> 24.6.)
     FragAddr16<KIND, BM, A_KC, TM16> fa16;
     FragAddr16<KIND, BN, B_KC, TN16> fb16;
-    Frag<KIND> qa[M16 ? KSTEPS16 : 1][TM16], qb[M16 ? KSTEPS16 : 1][TN16];
-    if constexpr (M16) {
-      fa16.setup(wm * TM16);
-      fb16.setup(wn * TN16);
-    }
+    Frag<KIND> qa[KSTEPS16][TM16], qb[KSTEPS16][TN16];
+    fa16.setup(wm * TM16);
+    fb16.setup(wn * TN16);
     if (team)
       gemm_barrier();
+    int cb = 0; // stage of B holding slice kt
     for (int kt = 0; kt < kt_count; ++kt) {
       const int nxt = cur ^ 1;
       // ---- memory phase
-      const uint32_t sa = stage_a(cur), sb = stage_b(cur);
-      if constexpr (M16) {
-        gemm_static_for<KSTEPS16>([&](auto uc) {
-          constexpr int u = decltype(uc)::value;
-          fa16.template load<u>(sa, qa[u]);
-          fb16.template load<u>(sb, qb[u]);
-        });
-      } else {
-        gemm_static_for<KSTEPS>([&](auto uc) {
-          constexpr int u = decltype(uc)::value;
-          fa_addr.template load<u>(sa, pa[u]);
-          fb_addr.template load<u>(sb, pb[u]);
-        });
+      uint32_t sa = stage_a(cur), sb = stage_b(cb);
+      if constexpr (HALVES) {
+        // the half that holds this wavefront's rows (the upper half's stages are
+        // addressed as if the lower lay in front of them)
+        const uint32_t lo = stage_half(1, cb), hi = stage_half(0, cur);
+        sa = wm * WM >= BM / 2 ? hi - GA::kBytes / 2 : lo;
+        sb = wn * WN >= BN / 2 ? hi : lo + GA::kBytes / 2;
+      } else if constexpr (A_MODE == A_CONV) {
+        // (a gathered load's address takes the lanes a while: ahead of the
+        // fragment reads it hides behind the other team's MFMAs -- 128 x 128
+        // tiles, C320 -> K128 3 x 3 at stride 2, N30 63 x 63: 41.0 -> 37.1 us)
+        if (!team)
+          issue_a(kt + 1, nxt, Zero{}, One{});
+        __builtin_amdgcn_sched_barrier(0);
       }
+      gemm_static_for<KSTEPS16>([&](auto uc) {
+        constexpr int u = decltype(uc)::value;
+        fa16.template load<u>(sa, qa[u]);
+        fb16.template load<u>(sb, qb[u]);
+      });
+      // (the reads have returned before the barrier: the other team may
+      // refill the stage in the next phase)
       if (team) {
-        __builtin_amdgcn_s_waitcnt(gemm_wait_imm(63)); // the reads returned
-        issue(kt + 2, cur, Zero{}, One{});
-        // its share of slice kt + 1 (one batch older) has landed
+        const int free3 = cb == 0 ? 2 : cb - 1;
+        if constexpr (HALVES)
+          issue(kt + 2, free3, Zero{}, One{});
+        else
+          issue_b(kt + 2, free3, Zero{}, One{});
+        // B's slice kt + 1 (one batch older) has landed
         if (kt + 2 < kt_count)
-          __builtin_amdgcn_s_waitcnt(gemm_wait_imm(LPS));
+          __builtin_amdgcn_s_waitcnt(gemm_wait_imm(HALVES ? LPS : GB::kLoads));
         else
           __builtin_amdgcn_s_waitcnt(gemm_wait_imm(0));
       } else {
-        issue(kt + 1, nxt, Zero{}, One{});
-        // the reads returned: the other team may overwrite the stage next
+        if constexpr (HALVES)
+          issue(kt + 1, nxt, Zero{}, One{});
+        else if constexpr (A_MODE != A_CONV)
+          issue_a(kt + 1, nxt, Zero{}, One{});
         __builtin_amdgcn_s_waitcnt(gemm_wait_imm(63));
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -1061,32 +1127,22 @@ gemm_kernel(GemmArgs g) {
       __builtin_amdgcn_sched_barrier(0);
       // ---- MFMA phase
       __builtin_amdgcn_s_setprio(1);
-      if constexpr (M16) {
-        gemm_static_for<KSTEPS16>([&](auto uc) {
-          constexpr int u = decltype(uc)::value;
+      gemm_static_for<KSTEPS16>([&](auto uc) {
+        constexpr int u = decltype(uc)::value;
 #pragma unroll
-          for (int i = 0; i < TM16; ++i)
+        for (int i = 0; i < TM16; ++i)
 #pragma unroll
-            for (int j = 0; j < TN16; ++j)
-              mfma16<KIND>(acc16[i][j], qa[u][i], qb[u][j]);
-        });
-      } else {
-        gemm_static_for<KSTEPS>([&](auto uc) {
-          constexpr int u = decltype(uc)::value;
-#pragma unroll
-          for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-              mfma32<KIND>(acc[i][j], pa[u][i], pb[u][j]);
-        });
-      }
+          for (int j = 0; j < TN16; ++j)
+            mfma16<KIND>(acc16[i][j], qa[u][i], qb[u][j]);
+      });
       __builtin_amdgcn_s_setprio(0);
       __builtin_amdgcn_sched_barrier(0);
       if (!team)
-        __builtin_amdgcn_s_waitcnt(gemm_wait_imm(0)); // its share of slice kt + 1
+        __builtin_amdgcn_s_waitcnt(gemm_wait_imm(0)); // A's slice kt + 1
       gemm_barrier();
       __builtin_amdgcn_sched_barrier(0);
       cur = nxt;
+      cb = cb == 2 ? 0 : cb + 1;
     }
     if (!team)
       gemm_barrier();
@@ -1603,8 +1659,6 @@ int gemm_launch_kind(fhip_ctx *ctx, const GemmPlan &p, const GemmArgs &g) {
 // Implicit-GEMM convolution launchers (A gathered, B = filter, K-contiguous).
 template <int KIND>
 int conv_launch_kind(fhip_ctx *ctx, int bm, int bn, const GemmArgs &g) {
-  if (bm == 512 && bn == 128)
-    return launch<KIND, 512, 128, A_CONV, true>(ctx, g, 1);
   if (bm == 256 && bn == 256)
     return launch<KIND, 256, 256, A_CONV, true>(ctx, g, 1);
   if (bm == 256 && bn == 128)

@@ -619,3 +619,27 @@ def test_conv_register_filter_kernel_chosen_rows(ctx, knobs):
     taps = np.full(28, 3.0); taps[[0, -1]] = 2.0
     assert np.array_equal(out, np.broadcast_to(64.0 * taps[:, None] * taps[None, :],
                                                out.shape))
+
+
+def test_conv_gather_repeats_its_bits(ctx):
+    # 320 -> 128 channels, 3x3 at stride 2: 240 gathered 128 x 128 tiles of 45 K
+    # slices, a long enough run of the two-phase loop that a wavefront reading a
+    # stage while it is refilled shows.  The batch repeats two images, so all
+    # copies of an image must agree bit for bit, within a launch and across
+    # launches; the two are compared with the oracle.
+    xd, wd = [30, 320, 63, 63], [128, 320, 3, 3]
+    pair = rand(53, 0, [2] + xd[1:])
+    x = HT.from_logical(np.concatenate([pair] * 15), capi.BFLOAT16, oracle.channels_last_strides(xd))
+    w = cl(wd, 53, 1, capi.BFLOAT16, std=0.02)
+    first = HT.from_logical(pair, capi.BFLOAT16, oracle.channels_last_strides([2] + xd[1:]))
+    ydims = oracle.conv_output_dims(xd, wd, [1, 1], [2, 2], [1, 1])
+    out = HT.empty(ydims, capi.FLOAT, oracle.channels_last_strides(ydims))
+    d = conv_desc(x, w, out, [1, 1], [2, 2], [1, 1], capi.FLOAT)
+    dx, dw, do = x.upload(ctx), w.upload(ctx), out.upload(ctx)
+    ref = oracle.conv_fprop(first.logical(), w.logical(), [1, 1], [2, 2], [1, 1])
+    for i in range(4):
+        ctx.conv_fprop(d, dx, dw, do)
+        assert ctx.last_kernel().startswith("conv_igemm gather 128x128"), ctx.last_kernel()
+        got = out.fetch(ctx, do).logical().reshape([15, 2] + ydims[1:])
+        assert np.array_equal(got, np.broadcast_to(got[:1], got.shape)), f"launch {i}"
+        assert_close(got[0], ref, capi.FLOAT, f"launch {i}", rtol=1e-4)
