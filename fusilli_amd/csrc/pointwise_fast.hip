@@ -345,13 +345,23 @@ bool float_like(int dt) {
   return dt == FHIP_FLOAT || dt == FHIP_BFLOAT16 || dt == FHIP_HALF;
 }
 
-// Row-major dense strides of `dims`, or false.
-bool dense_row_major(const fhip_tensor_desc &t) {
+// Dims of the output in memory order, outermost first; false where it is not
+// dense.
+bool dense_order(const fhip_tensor_desc &t, int (&order)[FHIP_MAX_RANK], int *n) {
+  *n = 0;
+  for (int i = 0; i < t.rank; ++i)
+    if (t.dim[i] != 1)
+      order[(*n)++] = i;
+  for (int a = 1; a < *n; ++a)
+    for (int b = a; b > 0 && t.stride[order[b]] > t.stride[order[b - 1]]; --b) {
+      const int o = order[b];
+      order[b] = order[b - 1], order[b - 1] = o;
+    }
   int64_t expect = 1;
-  for (int i = t.rank - 1; i >= 0; --i) {
-    if (t.dim[i] != 1 && t.stride[i] != expect)
+  for (int a = *n - 1; a >= 0; --a) {
+    if (t.stride[order[a]] != expect)
       return false;
-    expect *= t.dim[i];
+    expect *= t.dim[order[a]];
   }
   return true;
 }
@@ -363,20 +373,24 @@ struct PwPlan {
 
 PwPlan make_plan(const fhip_pointwise_desc *d) {
   PwPlan p;
-  const fhip_tensor_desc &o = d->out;
-  if (!float_like(o.dtype) || !dense_row_major(o))
+  // The dims in the output's memory order (channels-last images included), unit
+  // dims left out: the kernel sees flat vectors, rows and columns.
+  const fhip_tensor_desc &out = d->out;
+  int order[FHIP_MAX_RANK], rank = 0;
+  if (!float_like(out.dtype) || !dense_order(out, order, &rank))
     return p;
-  const int64_t total = fhip_desc_volume(o);
+  struct {
+    int rank, dtype;
+    int64_t dim[FHIP_MAX_RANK];
+  } o{rank, out.dtype, {}};
+  int64_t ostride[FHIP_MAX_RANK];
+  for (int i = 0; i < rank; ++i) {
+    o.dim[i] = out.dim[order[i]];
+    ostride[i] = out.stride[order[i]];
+  }
+  const int64_t total = fhip_desc_volume(out);
   if (total <= 0 || total % 8 != 0 || total / 8 >= (1ll << 31))
     return p;
-  int64_t ostride[FHIP_MAX_RANK];
-  {
-    int64_t s = 1;
-    for (int i = o.rank - 1; i >= 0; --i) {
-      ostride[i] = s;
-      s *= o.dim[i];
-    }
-  }
   PwFastArgs &g = p.g;
   g.nvec = total / 8;
   g.o_dt = o.dtype;
@@ -393,9 +407,11 @@ PwPlan make_plan(const fhip_pointwise_desc *d) {
     }
     if (d->in[i].dtype != o.dtype)
       return p;
-    int64_t st[FHIP_MAX_RANK];
-    if (!fhip_broadcast_strides(d->in[i], o.rank, o.dim, st))
+    int64_t full[FHIP_MAX_RANK], st[FHIP_MAX_RANK];
+    if (!fhip_broadcast_strides(d->in[i], out.rank, out.dim, full))
       return p;
+    for (int j = 0; j < rank; ++j)
+      st[j] = full[order[j]];
     // split point k: dims [k, rank) against dims [0, k)
     bool matched = false;
     for (int k = 0; k <= o.rank && !matched; ++k) {
@@ -482,6 +498,7 @@ int fhip_fast_pointwise(fhip_ctx *ctx, const fhip_pointwise_desc *d,
       PW_CASE(2, FHIP_PW_DIV)
       PW_CASE(2, FHIP_PW_MAX_OP)
       PW_CASE(2, FHIP_PW_MIN_OP)
+      PW_CASE(2, FHIP_PW_RELU_BWD)
     default:
       launch_mode<2, -1>(ctx, g);
       break;

@@ -140,3 +140,24 @@ def test_fallbacks_keep_working(ctx):
     t = HT.from_logical(rand(77, 3, [8, 16]), capi.FLOAT, strides=[1, 8])
     out = run(ctx, "ABS", [t], capi.FLOAT, expect_tuned=False)
     assert np.array_equal(out.logical(), np.abs(t.logical()))
+
+
+@pytest.mark.parametrize("dims", [[2, 24, 5, 7], [3, 8, 1, 9], [1, 16, 6, 6]])
+@pytest.mark.parametrize("dtype", [capi.FLOAT, capi.BFLOAT16, capi.HALF])
+def test_channels_last_tensors(ctx, dims, dtype):
+    # dense in another dim order than row-major: flat vectors, and a per-channel
+    # operand is a broadcast row
+    lay = oracle.channels_last_strides
+    a = HT.from_logical(rand(78, 0, dims), dtype, lay(dims))
+    b = HT.from_logical(rand(78, 1, dims), dtype, lay(dims))
+    row = HT.from_logical(rand(78, 2, [1, dims[1], 1, 1]), dtype, lay([1, dims[1], 1, 1]))
+    for mode, other in (("RELU_BWD", b), ("ADD", row)):
+        out = HT.empty(dims, dtype, lay(dims))
+        d = capi.PointwiseDesc()
+        d.mode, d.num_inputs, d.params = capi.PW[mode], 2, capi.PointwiseParams.default()
+        d.in_[0], d.in_[1], d.out = a.desc(), other.desc(), out.desc()
+        assert ctx.lib.fhip_pointwise_supported(d) == 2
+        da, db, do = a.upload(ctx), other.upload(ctx), out.upload(ctx)
+        ctx.pointwise(d, da, db, None, do)
+        ref = oracle.pointwise(capi.PW[mode], [a.logical(), other.logical()])
+        assert_close(out.fetch(ctx, do).logical(), ref, dtype, f"{mode} {dims}")
