@@ -105,6 +105,10 @@ int fhip_norm_long(fhip_ctx *ctx, const fhip_norm_desc *d, int64_t inner,
                    const void *x, const void *scale, const void *bias, void *out,
                    void *mean, void *inv_variance);
 
+// Reduced dims in front of kept ones (channel sums of an image batch, column
+// sums): `handled` false where the kernels do not take the descriptor.
+int fhip_mid_reduce(fhip_ctx *ctx, const fhip_reduce_desc *d, const void *x,
+                    void *y, bool *handled);
 bool fhip_fast_reduce_applicable(const fhip_reduce_desc *d);
 int fhip_fast_reduce(fhip_ctx *ctx, const fhip_reduce_desc *d, const void *x,
                      void *y);

@@ -1987,6 +1987,10 @@ int fhip_reduce(fhip_ctx *ctx, const fhip_reduce_desc *d, const void *x,
   // the row kernel moves 16-byte chunks: an unaligned base takes the generic one
   if (fhip_fast_reduce_applicable(d) && ((uintptr_t)x & 15) == 0)
     return fhip_fast_reduce(ctx, d, x, y);
+  bool handled = false;
+  const int mid_rc = fhip_mid_reduce(ctx, d, x, y, &handled);
+  if (handled)
+    return mid_rc;
   fhip_note_kernel(ctx, "reduce_generic");
   ReduceArgs g{};
   g.y = make_dims(d->y);

@@ -1,5 +1,6 @@
-// Bandwidth-bound keep-dim reductions over the trailing (contiguous) dims of a
-// dense row-major tensor: X viewed as [rows, cols] -> Y[rows].
+// Bandwidth-bound keep-dim reductions of a dense tensor.  Over the trailing dims
+// in memory order: X viewed as [rows, cols] -> Y[rows] (reduce_rows_kernel); with
+// reduced dims in front of kept ones: ReduceMidArgs below.
 //
 // TPR lanes share a row (16, 64 or 256 by row length), each streaming 16-byte
 // non-temporal loads into an f32 accumulator; the map (abs / square / zero->1)
@@ -232,21 +233,210 @@ __global__ __launch_bounds__(256) void reduce_rows_kernel(ReduceRowsArgs g) {
   }
 }
 
-struct ReducePlan {
-  bool ok = false;
-  int64_t rows = 0, cols = 0;
-  int map = M_NONE, comb = C_ADD, post = P_NONE;
+// Reductions that leave dims behind the reduced ones, X[r1][k][r2] -> Y[k]: the
+// bias gradient of a convolution (channels-last: r2 = 1, otherwise r2 = H * W),
+// column sums of a matrix.  The r1 range is cut into slices on workgroups of
+// their own (partial[slice][k], f32), which a second kernel combines in slice
+// order: no atomics.  Bound by reading X once.  N32 56 x 56 K128 bf16 in
+// channels-last (25.7 MB): 104 us on the strided kernel (one workgroup per
+// channel and slice reading one 2-byte element per pixel line) -> 12.7 us
+// (8.8 + 3.9); N100 K32 30 x 30 f32 channels-first (11.5 MB) 31 -> 10.2 us (5.5 +
+// 4.6).
+struct ReduceMidArgs {
+  const char *x;
+  void *y;
+  float *partial; // null: one slice, the result goes to y
+  int64_t r1, per_slice;
+  int32_t k, r2; // r2: in vectors of the kernel's width
+  uint32_t magic_r2;
+  int32_t slices;
+  int32_t y_dt, post;
+  float inv_count;
 };
 
-bool dense_row_major(const fhip_tensor_desc &t) {
-  int64_t expect = 1;
-  for (int i = t.rank - 1; i >= 0; --i) {
-    if (t.dim[i] != 1 && t.stride[i] != expect)
-      return false;
-    expect *= t.dim[i];
-  }
-  return true;
+// NaN-propagating combine of two values (sums and products propagate by
+// themselves)
+template <int COMB> __device__ __forceinline__ float rf_comb_nan(float a, float b) {
+  if constexpr (COMB == C_MIN || COMB == C_MAX)
+    return a != a ? a : (b != b ? b : rf_comb<COMB>(a, b));
+  else
+    return rf_comb<COMB>(a, b);
 }
+
+__device__ __forceinline__ void rf_store(const ReduceMidArgs &g, int64_t i, float v) {
+  if (g.post == P_MEAN)
+    v *= g.inv_count;
+  else if (g.post == P_SQRT)
+    v = sqrtf(v);
+  if (g.y_dt == FHIP_FLOAT)
+    ((RF_AS1 float *)g.y)[i] = v;
+  else if (g.y_dt == FHIP_BFLOAT16)
+    ((RF_AS1 __bf16 *)g.y)[i] = (__bf16)v;
+  else
+    ((RF_AS1 _Float16 *)g.y)[i] = (_Float16)v;
+}
+
+template <typename T, int VEC> struct RfVec {
+  typedef T type __attribute__((ext_vector_type(VEC)));
+};
+template <typename T> struct RfVec<T, 1> {
+  typedef T type;
+};
+template <typename T, int VEC>
+__device__ __forceinline__ void rf_values(typename RfVec<T, VEC>::type v, float (&f)[VEC]) {
+  if constexpr (VEC == 1) {
+    f[0] = (float)v;
+  } else {
+#pragma unroll
+    for (int i = 0; i < VEC; ++i)
+      f[i] = (float)v[i];
+  }
+}
+
+// r2 == 1: TX threads side by side on the columns (VEC each), 256 / TX rows at
+// a time, four rows of loads in flight per thread.
+template <typename T, int MAP, int COMB, int VEC>
+__global__ __launch_bounds__(256) void reduce_cols_kernel(ReduceMidArgs g, int tx_log2) {
+  typedef typename RfVec<T, VEC>::type V;
+  __shared__ float lds[256][VEC + 1];
+  const int tx = 1 << tx_log2, ty = 256 >> tx_log2;
+  const int c = blockIdx.x * tx + (threadIdx.x & (tx - 1)); // column vector
+  const int row0 = threadIdx.x >> tx_log2;
+  const int cols = g.k / VEC;
+  const bool live = c < cols;
+  const int64_t first = (int64_t)blockIdx.y * g.per_slice;
+  const int64_t last = first + g.per_slice < g.r1 ? first + g.per_slice : g.r1;
+  const RF_AS1 V *src = (const RF_AS1 V *)g.x + (live ? c : 0);
+  float acc[VEC];
+#pragma unroll
+  for (int i = 0; i < VEC; ++i)
+    acc[i] = rf_identity<COMB>();
+  auto add = [&](V v) {
+    float f[VEC];
+    rf_values<T, VEC>(v, f);
+#pragma unroll
+    for (int i = 0; i < VEC; ++i)
+      acc[i] = rf_comb_nan<COMB>(acc[i], rf_map<MAP>(f[i]));
+  };
+  int64_t r = first + row0;
+  for (; r + 3 * ty < last; r += 4 * ty) {
+    const V v0 = src[r * cols], v1 = src[(r + ty) * cols];
+    const V v2 = src[(r + 2 * ty) * cols], v3 = src[(r + 3 * ty) * cols];
+    add(v0);
+    add(v1);
+    add(v2);
+    add(v3);
+  }
+  for (; r < last; r += ty)
+    add(src[r * cols]);
+#pragma unroll
+  for (int i = 0; i < VEC; ++i)
+    lds[threadIdx.x][i] = acc[i];
+  for (int s = 128; s >= tx; s >>= 1) {
+    __syncthreads();
+    if ((int)threadIdx.x < s) {
+#pragma unroll
+      for (int i = 0; i < VEC; ++i)
+        lds[threadIdx.x][i] = rf_comb_nan<COMB>(lds[threadIdx.x][i], lds[threadIdx.x + s][i]);
+    }
+  }
+  if ((int)threadIdx.x < tx && live) {
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) {
+      const float v = lds[threadIdx.x][i];
+      if (g.partial)
+        g.partial[(int64_t)blockIdx.y * g.k + (int64_t)c * VEC + i] = v;
+      else
+        rf_store(g, (int64_t)c * VEC + i, v);
+    }
+  }
+}
+
+// r2 > 1: one k and one slice of r1 per workgroup, its runs of r2 as one index.
+template <typename T, int MAP, int COMB, int VEC>
+__global__ __launch_bounds__(256) void reduce_mid_kernel(ReduceMidArgs g) {
+  typedef typename RfVec<T, VEC>::type V;
+  __shared__ float part[4];
+  const int64_t first = (int64_t)blockIdx.y * g.per_slice;
+  const int64_t last = first + g.per_slice < g.r1 ? first + g.per_slice : g.r1;
+  const uint32_t count = (uint32_t)((last - first) * g.r2);
+  const RF_AS1 V *src = (const RF_AS1 V *)g.x + (first * g.k + blockIdx.x) * (int64_t)g.r2;
+  const int64_t pitch = (int64_t)g.k * g.r2;
+  float acc = rf_identity<COMB>();
+  auto at = [&](uint32_t i) {
+    uint32_t q = __umulhi(i, g.magic_r2); // (floor estimate: at most one too small)
+    uint32_t rem = i - q * (uint32_t)g.r2;
+    if (rem >= (uint32_t)g.r2)
+      rem -= (uint32_t)g.r2, ++q;
+    return src[(int64_t)q * pitch + rem];
+  };
+  auto add = [&](V v) {
+    float f[VEC];
+    rf_values<T, VEC>(v, f);
+#pragma unroll
+    for (int i = 0; i < VEC; ++i)
+      acc = rf_comb_nan<COMB>(acc, rf_map<MAP>(f[i]));
+  };
+  uint32_t i = threadIdx.x;
+  for (; i + 768 < count; i += 1024) {
+    const V v0 = at(i), v1 = at(i + 256), v2 = at(i + 512), v3 = at(i + 768);
+    add(v0);
+    add(v1);
+    add(v2);
+    add(v3);
+  }
+  for (; i < count; i += 256)
+    add(at(i));
+#pragma unroll
+  for (int s = 32; s > 0; s >>= 1)
+    acc = rf_comb_nan<COMB>(acc, __shfl_xor(acc, s, 64));
+  if ((threadIdx.x & 63) == 0)
+    part[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const float v = rf_comb_nan<COMB>(rf_comb_nan<COMB>(part[0], part[1]),
+                                      rf_comb_nan<COMB>(part[2], part[3]));
+    if (g.partial)
+      g.partial[(int64_t)blockIdx.y * g.k + blockIdx.x] = v;
+    else
+      rf_store(g, blockIdx.x, v);
+  }
+}
+
+// Combines the slices: 16 columns per workgroup, 16 threads per column.
+template <int COMB>
+__global__ __launch_bounds__(256) void reduce_mid_finish_kernel(ReduceMidArgs g) {
+  __shared__ float lds[16][17];
+  const int cl = threadIdx.x & 15, sl = threadIdx.x >> 4;
+  const int64_t c = (int64_t)blockIdx.x * 16 + cl;
+  float acc = rf_identity<COMB>();
+  if (c < g.k) {
+    const RF_AS1 float *p = (const RF_AS1 float *)g.partial + c;
+    int s = sl;
+    for (; s + 48 < g.slices; s += 64) {
+      const float v0 = p[(int64_t)s * g.k], v1 = p[(int64_t)(s + 16) * g.k];
+      const float v2 = p[(int64_t)(s + 32) * g.k], v3 = p[(int64_t)(s + 48) * g.k];
+      acc = rf_comb_nan<COMB>(rf_comb_nan<COMB>(rf_comb_nan<COMB>(rf_comb_nan<COMB>(acc, v0), v1), v2), v3);
+    }
+    for (; s < g.slices; s += 16)
+      acc = rf_comb_nan<COMB>(acc, p[(int64_t)s * g.k]);
+  }
+  lds[sl][cl] = acc;
+  __syncthreads();
+  if (sl == 0 && c < g.k) {
+    for (int s = 1; s < 16; ++s)
+      acc = rf_comb_nan<COMB>(acc, lds[s][cl]);
+    rf_store(g, c, acc);
+  }
+}
+
+struct ReducePlan {
+  bool ok = false;  // the row kernel takes it
+  bool mid = false; // reduced dims in front of kept ones: the column kernels do
+  int64_t rows = 0, cols = 0;
+  int64_t r1 = 1, k = 1, r2 = 1;
+  int map = M_NONE, comb = C_ADD, post = P_NONE;
+};
 
 ReducePlan make_plan(const fhip_reduce_desc *d) {
   ReducePlan p;
@@ -256,28 +446,45 @@ ReducePlan make_plan(const fhip_reduce_desc *d) {
   };
   if (!f(xdt) || !f(ydt))
     return p;
-  if (!dense_row_major(d->x) || !dense_row_major(d->y))
-    return p;
-  // kept dims first, reduced dims last (unit dims may sit anywhere)
-  p.rows = p.cols = 1;
-  bool in_tail = false;
-  for (int i = 0; i < d->x.rank; ++i) {
-    if (d->x.dim[i] == 1)
-      continue;
-    const bool reduced = d->y.dim[i] == 1;
-    if (reduced) {
-      in_tail = true;
-      p.cols *= d->x.dim[i];
-    } else {
-      if (in_tail)
+  // X's dims in memory order, outermost first (unit dims may sit anywhere);
+  // both tensors dense in that order
+  int order[FHIP_MAX_RANK], n = 0;
+  for (int i = 0; i < d->x.rank; ++i)
+    if (d->x.dim[i] != 1)
+      order[n++] = i;
+  for (int a = 1; a < n; ++a)
+    for (int b = a; b > 0 && d->x.stride[order[b]] > d->x.stride[order[b - 1]]; --b) {
+      const int t = order[b];
+      order[b] = order[b - 1], order[b - 1] = t;
+    }
+  int64_t xs = 1, ys = 1;
+  for (int a = n - 1; a >= 0; --a) {
+    const int i = order[a];
+    if (d->x.stride[i] != xs)
+      return p;
+    xs *= d->x.dim[i];
+    if (d->y.dim[i] != 1) {
+      if (d->y.stride[i] != ys)
         return p;
-      p.rows *= d->x.dim[i];
+      ys *= d->y.dim[i];
     }
   }
-  if (p.cols < 2 || (p.cols * fhip_dtype_size(xdt)) % 16 != 0)
-    return p;
-  if (p.rows >= (1ll << 31) * 16)
-    return p;
+  // runs of reduced (r1), kept (k) and reduced (r2) dims
+  int stage = 0;
+  for (int a = 0; a < n; ++a) {
+    const int64_t dim = d->x.dim[order[a]];
+    const bool reduced = d->y.dim[order[a]] == 1;
+    if (reduced)
+      stage == 0 ? p.r1 *= dim : p.r2 *= dim;
+    else if (p.r2 != 1)
+      return p;
+    else
+      p.k *= dim;
+    if (!reduced)
+      stage = 1;
+  }
+  if (stage == 0) // everything is reduced: one row
+    p.r2 = p.r1, p.r1 = 1;
   switch (d->mode) {
   case FHIP_RED_ADD:
   case FHIP_RED_SUM:
@@ -312,8 +519,69 @@ ReducePlan make_plan(const fhip_reduce_desc *d) {
   default:
     return p;
   }
-  p.ok = true;
+  p.rows = p.k;
+  p.cols = p.r2;
+  p.ok = p.r1 == 1 && p.cols >= 2 && (p.cols * fhip_dtype_size(xdt)) % 16 == 0 &&
+         p.rows < (1ll << 31) * 16;
+  p.mid = !p.ok && p.r1 * p.r2 >= 2 && p.k <= (1 << 24) && p.r2 < (1 << 24);
   return p;
+}
+
+// Slices of r1 and launches of the column kernels (see ReduceMidArgs): about
+// four workgroups per compute unit over all columns, at most 256 slices (the
+// combining kernel reads slices * k values), and at least some 16 rows (r2 = 1)
+// or 2048 elements per workgroup.
+template <typename T, int MAP, int COMB>
+int launch_mid(fhip_ctx *ctx, const ReducePlan &p, ReduceMidArgs g) {
+  constexpr int VEC = 16 / (int)sizeof(T);
+  const bool cols = p.r2 == 1;
+  const bool vec = ((uintptr_t)g.x & 15) == 0 && (cols ? p.k % VEC == 0 : p.r2 % VEC == 0);
+  int tx_log2 = 0;
+  int64_t groups = p.k, most;
+  if (cols) {
+    const int64_t cv = vec ? p.k / VEC : p.k;
+    while ((1ll << tx_log2) < cv && tx_log2 < 8)
+      ++tx_log2;
+    groups = (cv + (1ll << tx_log2) - 1) >> tx_log2;
+    most = p.r1 / ((256 >> tx_log2) * 8);
+  } else {
+    g.r2 = (int32_t)(vec ? p.r2 / VEC : p.r2);
+    g.magic_r2 = g.r2 == 1 ? 0xffffffffu : (uint32_t)((1ull << 32) / (uint32_t)g.r2);
+    most = p.r1 * p.r2 / 2048;
+    most = most < p.r1 ? most : p.r1;
+  }
+  int64_t slices = 4 * (int64_t)(ctx->num_cus > 0 ? ctx->num_cus : 256) / groups;
+  slices = slices < most ? slices : most;
+  slices = slices < 256 ? slices : 256;
+  // (a slice's flat index is 32-bit)
+  const int64_t least = (p.r1 * p.r2) / (1ll << 30) + 1;
+  slices = slices > least ? slices : least;
+  g.per_slice = (p.r1 + slices - 1) / slices;
+  slices = (p.r1 + g.per_slice - 1) / g.per_slice;
+  if (slices > 65535 || g.per_slice * p.r2 >= (1ll << 31))
+    return -1; // (the strided kernel's)
+  g.slices = (int32_t)slices;
+  if (slices > 1) {
+    void *sp = nullptr;
+    if (fhip_ctx_scratch(ctx, (size_t)(slices * p.k) * sizeof(float), &sp) != 0)
+      return 1;
+    g.partial = (float *)sp;
+  }
+  fhip_note_kernel(ctx, cols ? "reduce_cols slices=%d" : "reduce_mid slices=%d", (int)slices);
+  const dim3 grid((unsigned)groups, (unsigned)slices);
+  if (cols && vec)
+    hipLaunchKernelGGL((reduce_cols_kernel<T, MAP, COMB, VEC>), grid, dim3(256), 0, ctx->stream, g, tx_log2);
+  else if (cols)
+    hipLaunchKernelGGL((reduce_cols_kernel<T, MAP, COMB, 1>), grid, dim3(256), 0, ctx->stream, g, tx_log2);
+  else if (vec)
+    hipLaunchKernelGGL((reduce_mid_kernel<T, MAP, COMB, VEC>), grid, dim3(256), 0, ctx->stream, g);
+  else
+    hipLaunchKernelGGL((reduce_mid_kernel<T, MAP, COMB, 1>), grid, dim3(256), 0, ctx->stream, g);
+  if (slices > 1)
+    hipLaunchKernelGGL(reduce_mid_finish_kernel<COMB>, dim3((unsigned)((p.k + 15) / 16)), dim3(256),
+                       0, ctx->stream, g);
+  FHIP_HIP_CHECK(ctx, hipGetLastError());
+  return 0;
 }
 
 template <typename T, int MAP, int COMB>
@@ -337,29 +605,68 @@ int launch_tpr(fhip_ctx *ctx, const ReduceRowsArgs &g) {
 
 // The amax of |x| starts from 0, the others from their combine's identity;
 // only these (map, combine) pairs occur.
+template <typename F> int for_mode(const ReducePlan &p, F &&run) {
+  using std::integral_constant;
+  auto go = [&](auto map, auto comb) { return run(map, comb); };
+  if (p.comb == C_ADD && p.map == M_NONE)
+    return go(integral_constant<int, M_NONE>{}, integral_constant<int, C_ADD>{});
+  if (p.comb == C_ADD && p.map == M_ABS)
+    return go(integral_constant<int, M_ABS>{}, integral_constant<int, C_ADD>{});
+  if (p.comb == C_ADD && p.map == M_SQUARE)
+    return go(integral_constant<int, M_SQUARE>{}, integral_constant<int, C_ADD>{});
+  if (p.comb == C_MUL && p.map == M_NONE)
+    return go(integral_constant<int, M_NONE>{}, integral_constant<int, C_MUL>{});
+  if (p.comb == C_MUL && p.map == M_ZERO_TO_ONE)
+    return go(integral_constant<int, M_ZERO_TO_ONE>{}, integral_constant<int, C_MUL>{});
+  if (p.comb == C_MIN)
+    return go(integral_constant<int, M_NONE>{}, integral_constant<int, C_MIN>{});
+  if (p.comb == C_MAX && p.map == M_ABS)
+    return go(integral_constant<int, M_ABS>{}, integral_constant<int, C_MAX>{});
+  return go(integral_constant<int, M_NONE>{}, integral_constant<int, C_MAX>{});
+}
+
 template <typename T>
 int launch_mode(fhip_ctx *ctx, const ReducePlan &p, const ReduceRowsArgs &g) {
-  if (p.comb == C_ADD && p.map == M_NONE)
-    return launch_tpr<T, M_NONE, C_ADD>(ctx, g);
-  if (p.comb == C_ADD && p.map == M_ABS)
-    return launch_tpr<T, M_ABS, C_ADD>(ctx, g);
-  if (p.comb == C_ADD && p.map == M_SQUARE)
-    return launch_tpr<T, M_SQUARE, C_ADD>(ctx, g);
-  if (p.comb == C_MUL && p.map == M_NONE)
-    return launch_tpr<T, M_NONE, C_MUL>(ctx, g);
-  if (p.comb == C_MUL && p.map == M_ZERO_TO_ONE)
-    return launch_tpr<T, M_ZERO_TO_ONE, C_MUL>(ctx, g);
-  if (p.comb == C_MIN)
-    return launch_tpr<T, M_NONE, C_MIN>(ctx, g);
-  if (p.comb == C_MAX && p.map == M_ABS)
-    return launch_tpr<T, M_ABS, C_MAX>(ctx, g);
-  return launch_tpr<T, M_NONE, C_MAX>(ctx, g);
+  return for_mode(p, [&](auto map, auto comb) {
+    return launch_tpr<T, decltype(map)::value, decltype(comb)::value>(ctx, g);
+  });
+}
+
+template <typename T>
+int launch_mid_mode(fhip_ctx *ctx, const ReducePlan &p, const ReduceMidArgs &g) {
+  return for_mode(p, [&](auto map, auto comb) {
+    return launch_mid<T, decltype(map)::value, decltype(comb)::value>(ctx, p, g);
+  });
 }
 
 } // namespace
 
 bool fhip_fast_reduce_applicable(const fhip_reduce_desc *d) {
   return make_plan(d).ok;
+}
+
+int fhip_mid_reduce(fhip_ctx *ctx, const fhip_reduce_desc *d, const void *x, void *y,
+                    bool *handled) {
+  *handled = false;
+  const ReducePlan p = make_plan(d);
+  if (!p.mid)
+    return 0;
+  ReduceMidArgs g{};
+  g.x = (const char *)x;
+  g.y = y;
+  g.r1 = p.r1;
+  g.k = (int32_t)p.k;
+  g.r2 = (int32_t)p.r2;
+  g.y_dt = d->y.dtype;
+  g.post = p.post;
+  g.inv_count = 1.0f / (float)(p.r1 * p.r2);
+  const int rc = d->x.dtype == FHIP_FLOAT      ? launch_mid_mode<float>(ctx, p, g)
+                 : d->x.dtype == FHIP_BFLOAT16 ? launch_mid_mode<__bf16>(ctx, p, g)
+                                               : launch_mid_mode<_Float16>(ctx, p, g);
+  if (rc < 0)
+    return 0;
+  *handled = true;
+  return rc;
 }
 
 int fhip_fast_reduce(fhip_ctx *ctx, const fhip_reduce_desc *d, const void *x,

@@ -102,3 +102,43 @@ def test_reduce_min_max_propagate_nan_and_inf(ctx, mode, dtype):
     assert np.isnan(out[1]) and not np.isnan(out[[0, 2, 3, 4, 5]]).any()
     assert out[2] == (-np.inf if mode == "MIN" else np.inf if mode == "AMAX" else out[2])
     assert out[3] == (np.inf if mode in ("MAX", "AMAX") else out[3])
+
+
+@pytest.mark.parametrize("mode", MODES)
+@pytest.mark.parametrize("dtype", [capi.FLOAT, capi.BFLOAT16, capi.HALF])
+@pytest.mark.parametrize("dims,odims,channels_last", [
+    ([4, 40, 9, 7], [1, 40, 1, 1], True),    # columns in 16-byte vectors, one slice
+    ([16, 128, 20, 20], [1, 128, 1, 1], True),  # several slices
+    ([3, 13, 11, 5], [1, 13, 1, 1], True),   # odd channel count: element loads
+    ([6000, 70], [1, 70], False),            # column sums of a matrix
+    ([5, 3, 8, 8], [1, 3, 1, 1], False),     # channels first, whole vectors per run
+    ([50, 4, 30, 31], [1, 4, 1, 1], False),  # runs of odd length, several slices
+    ([7, 600, 2], [1, 600, 1], False),       # short runs
+    ([3, 5], [1, 1], False),                 # everything, no whole vector
+])
+def test_reduce_in_front_of_kept_dims_vs_oracle(ctx, mode, dtype, dims, odims, channels_last):
+    x = make_x(66, dims, dtype, mode)
+    y = HT.empty(odims, capi.FLOAT)
+    if channels_last:
+        x = HT.from_logical(x.logical(), dtype, oracle.channels_last_strides(dims))
+        y = HT.empty(odims, capi.FLOAT, oracle.channels_last_strides(odims))
+    d = capi.ReduceDesc()
+    d.x, d.y, d.mode = x.desc(), y.desc(), capi.RED[mode]
+    dx, dy = x.upload(ctx), y.upload(ctx)
+    ctx.reduce(d, dx, dy)
+    assert ctx.last_kernel().startswith(("reduce_cols", "reduce_mid")), ctx.last_kernel()
+    got = y.fetch(ctx, dy).logical()
+    ref = oracle.reduction(x.logical(), odims, capi.RED[mode])
+    rtol = 1e-4 if dtype == capi.FLOAT else 2e-2
+    assert_close(got, ref, capi.FLOAT, f"{mode} {dims}", rtol=rtol)
+
+
+@pytest.mark.parametrize("mode", ["MIN", "MAX", "AMAX"])
+def test_reduce_columns_propagate_nan(ctx, mode):
+    v = rand(67, 0, [700, 24])
+    v[33, 5], v[650, 11], v[2, 17] = np.nan, -np.inf, np.inf
+    out = run(ctx, HT.from_logical(v, capi.BFLOAT16), [1, 24], mode, y_dtype=capi.FLOAT,
+              expect_tuned=False).logical().reshape(-1)
+    assert np.isnan(out[5]) and np.isnan(out).sum() == 1
+    assert out[11] == (-np.inf if mode == "MIN" else np.inf if mode == "AMAX" else out[11])
+    assert out[17] == (np.inf if mode in ("MAX", "AMAX") else out[17])
