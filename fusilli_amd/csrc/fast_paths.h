@@ -17,6 +17,12 @@ int fhip_fast_matmul_outer(fhip_ctx *ctx, const fhip_matmul_desc *d,
                            void *out, int outer, int64_t a_outer,
                            int64_t b_outer, int64_t o_outer);
 
+// Products outside that contract -- few rows or columns, K or row starts that do
+// not fit 128-byte slices, f32 -- on kernels that load MFMA fragments straight
+// from global memory; `handled` false where they do not take the descriptor.
+int fhip_direct_matmul(fhip_ctx *ctx, const fhip_matmul_desc *d, const void *a,
+                       const void *b, const DevEpilogue &epi, void *out, bool *handled);
+
 // `allow_scratch` false: only plans that leave the context's scratch alone
 // (no zero-padded channel copies, no split reduction) -- for the entry point
 // that must not allocate.

@@ -1,0 +1,148 @@
+// Host side of the direct matrix-product kernels (gemm_direct_kernel.h): which
+// descriptors they take, tile, wavefronts and split of K.
+#include "fast_paths.h"
+#include "gemm_direct_kernel.h"
+
+#include <cmath>
+
+namespace {
+
+bool direct_plan(const fhip_matmul_desc *d, DirectPlan *p, DirectArgs *g, int64_t *batch) {
+  const int r = d->a.rank;
+  if ((r != 2 && r != 3) || d->a.dtype != d->b.dtype)
+    return false;
+  switch (d->a.dtype) {
+  case FHIP_BFLOAT16: p->kind = GK_BF16; break;
+  case FHIP_HALF: p->kind = GK_F16; break;
+  case FHIP_INT8: p->kind = GK_I8; break;
+  case FHIP_FP8E4M3: p->kind = GK_FP8E4M3; break;
+  case FHIP_FP8E5M2: p->kind = GK_FP8E5M2; break;
+  case FHIP_FLOAT: p->kind = GK_F32; break;
+  default: return false;
+  }
+  const int elem = fhip_dtype_size(d->a.dtype);
+  auto f = [](int dt) { return dt == FHIP_FLOAT || dt == FHIP_BFLOAT16 || dt == FHIP_HALF; };
+  if (p->kind == GK_I8
+          ? d->c.dtype != FHIP_INT32 || d->out.dtype != FHIP_INT32 || d->epilogue.count != 0
+          : !f(d->c.dtype) || !f(d->out.dtype))
+    return false;
+  const int64_t M = d->a.dim[r - 2], K = d->a.dim[r - 1], N = d->b.dim[r - 1];
+  *batch = r == 3 ? d->c.dim[0] : 1;
+  const int64_t a_sm = d->a.stride[r - 2], a_sk = d->a.stride[r - 1];
+  const int64_t b_sk = d->b.stride[r - 2], b_sn = d->b.stride[r - 1];
+  p->a_kc = a_sk == 1;
+  p->b_kc = b_sk == 1;
+  if ((!p->a_kc && a_sm != 1 && M != 1) || (!p->b_kc && b_sn != 1 && N != 1))
+    return false;
+  const int64_t a_ld = p->a_kc ? a_sm : a_sk, b_ld = p->b_kc ? b_sn : b_sk;
+  // a 16-byte piece of K; 32-bit lane offsets over a tile's rows or a step's
+  // K-rows (at most 128)
+  if (K * elem < 16 || a_ld * elem >= (1 << 24) || b_ld * elem >= (1 << 24) || M >= (1ll << 31) ||
+      N >= (1ll << 31) || K >= (1ll << 31) || *batch > 65535)
+    return false;
+  g->slices = (int)((K * elem + 127) / 128);
+  // Tile, wavefronts and split of K: the shortest of an estimate in
+  // microseconds.  A compute unit pulls some 50 KB of whole lines in one (half
+  // of that in shorter runs), its matrix pipes do 256 (f32) to 8192 (8-bit)
+  // operations a clock, and a split adds the second kernel and the partial
+  // tiles' round trip.
+  static const struct { int mt, nt_kc, nt, waves; } kShapes[] = {
+      {1, 1, 4, 16}, {1, 2, 4, 8}, {2, 2, 4, 8}, {4, 4, 4, 4}};
+  const double ops = p->kind == GK_F32 ? 5.6e5 : elem == 2 ? 4e6 : 8e6; // per us and compute unit
+  double best = 0;
+  for (const auto &c : kShapes) {
+    const int mt = c.mt, nt = p->b_kc ? c.nt_kc : c.nt;
+    // (a run of the interleaved rows lies inside the operand)
+    if ((!p->b_kc && N < nt) || (!p->a_kc && M < mt) || (!p->b_kc && c.nt_kc == 2 && mt == 1))
+      continue;
+    const int most = p->b_kc || mt > 1 ? c.waves : 8;
+    const int64_t tm = (M + 16 * mt - 1) / (16 * mt), tn = (N + 16 * nt - 1) / (16 * nt);
+    const int64_t wgs = tm * tn * *batch;
+    if (tm * tn >= (1ll << 31))
+      continue;
+    // (one thread for every four results, 64 x 64 tiles: sixteen)
+    int waves = g->slices, least = mt * nt == 16 ? 4 : mt * nt;
+    waves = waves > least ? waves : least;
+    waves = waves < 1 ? 1 : waves < most ? waves : most;
+    const double pull_a = 16.0 * mt * K * elem / (p->a_kc || mt * elem >= 8 ? 5e4 : 2.5e4);
+    const double pull_b = 16.0 * nt * K * elem / (p->b_kc || nt * elem >= 8 ? 5e4 : 2.5e4);
+    const double work = 512.0 * mt * nt * (double)K;
+    for (int split = 1; split <= 32; split *= 2) {
+      if (split > 1 && (g->slices < 2 * split * waves || wgs * split > 512))
+        break;
+      // (workgroups that share a compute unit: whole rounds matter below two)
+      const double share = (double)(wgs * split) / 256.0;
+      const double rounds = share <= 1.0 ? 1.0 : fmax(share, mt == 4 ? 1.5 : 1.2);
+      const double us = 2.0 + rounds * fmax(pull_a + pull_b, work / ops) / split +
+                        (split > 1 ? 3.0 + 2.0 * split * wgs * mt * nt * 1024.0 / 4e6 : 0.0);
+      if (best == 0 || us < best) {
+        best = us;
+        p->mt = mt, p->nt = nt, p->waves = waves, g->splits = split;
+        g->tiles_m = (int)tm, g->tiles_n = (int)tn;
+      }
+    }
+  }
+  if (best == 0)
+    return false;
+  g->M = (int)M, g->N = (int)N, g->K = (int)K;
+  g->a_ldb = a_ld * elem, g->b_ldb = b_ld * elem;
+  if (r == 3) {
+    g->a_batch = d->a.dim[0] == 1 ? 0 : d->a.stride[0];
+    g->b_batch = d->b.dim[0] == 1 ? 0 : d->b.stride[0];
+    g->o_batch = d->out.dim[0] == 1 ? 0 : d->out.stride[0];
+  }
+  g->o_sm = d->out.stride[r - 2];
+  g->o_sn = d->out.stride[r - 1];
+  g->c_dt = d->c.dtype;
+  g->o_dt = d->out.dtype;
+  p->ok = true;
+  return true;
+}
+
+} // namespace
+
+int fhip_direct_matmul(fhip_ctx *ctx, const fhip_matmul_desc *d, const void *a, const void *b,
+                       const DevEpilogue &epi, void *out, bool *handled) {
+  *handled = false;
+  DirectPlan p;
+  DirectArgs g{};
+  int64_t batch = 1;
+  if (!direct_plan(d, &p, &g, &batch))
+    return 0;
+  // operands at their own alignment
+  const uintptr_t am = fhip_dtype_size(d->a.dtype) - 1;
+  if ((((uintptr_t)a | (uintptr_t)b) & am) != 0)
+    return 0;
+  *handled = true;
+  g.a = (const char *)a;
+  g.b = (const char *)b;
+  g.out = (char *)out;
+  g.epi = epi;
+  g.epi.rank = 3;
+  const int r = d->a.rank;
+  for (int i = 0; i < epi.count; ++i) {
+    const DevEpiOp &s = epi.op[i];
+    DevEpiOp &o = g.epi.op[i];
+    o.stride[0] = r == 3 ? s.stride[0] : 0;
+    o.stride[1] = s.stride[r - 2];
+    o.stride[2] = s.stride[r - 1];
+  }
+  if (g.splits > 1) {
+    const size_t bytes = (size_t)g.splits * (size_t)batch * g.tiles_m * g.tiles_n * (p.mt * p.nt * 1024);
+    if (fhip_ctx_scratch(ctx, bytes, &g.partial) != 0)
+      return 1;
+  }
+  // (f32 products that split K over the wavefronts of a tile keep that name)
+  if (p.kind == GK_F32)
+    fhip_note_kernel(ctx, "matmul_f32_splitk");
+  else
+    fhip_note_kernel(ctx, "gemm_direct %dx%d waves=%d split=%d", 16 * p.mt, 16 * p.nt, p.waves, g.splits);
+  switch (p.kind) {
+  case GK_BF16: return direct_launch_bf16(ctx, p, g, batch);
+  case GK_F16: return direct_launch_f16(ctx, p, g, batch);
+  case GK_I8: return direct_launch_i8(ctx, p, g, batch);
+  case GK_FP8E4M3: return direct_launch_fp8e4m3(ctx, p, g, batch);
+  case GK_FP8E5M2: return direct_launch_fp8e5m2(ctx, p, g, batch);
+  default: return direct_launch_f32(ctx, p, g, batch);
+  }
+}

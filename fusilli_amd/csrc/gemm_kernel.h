@@ -1461,7 +1461,8 @@ gemm_kernel(GemmArgs g) {
         for (int e = 0; e < nops; ++e) {
           const DevEpiOp &o = g.epi.op[e];
           if (o.kind == FHIP_OPERAND_NONE) {
-            fhip_pw_fast_unary_vec<true, 8>(o.mode, y, o.params.swish_beta);
+            fhip_pw_fast_unary_vec<true, 8>(o.mode, y, o.params.swish_beta,
+                                            o.result_dtype != FHIP_FLOAT);
           } else {
             float other[8];
             if (o.kind == FHIP_OPERAND_SCALAR) {

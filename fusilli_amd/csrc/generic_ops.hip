@@ -1148,6 +1148,10 @@ int fhip_matmul(fhip_ctx *ctx, const fhip_matmul_desc *d, const void *a,
     return 1;
   if (fhip_fast_matmul_applicable(d))
     return fhip_fast_matmul(ctx, d, a, b, epi, out);
+  bool handled = false;
+  const int direct_rc = fhip_direct_matmul(ctx, d, a, b, epi, out, &handled);
+  if (handled)
+    return direct_rc;
   fhip_note_kernel(ctx, "matmul_generic");
 
   MatmulArgs g{};

@@ -164,28 +164,6 @@ __device__ __forceinline__ void store8(void *out, int32_t vec,
   X(FHIP_PW_MIN_OP) X(FHIP_PW_MUL) X(FHIP_PW_RELU_BWD) X(FHIP_PW_SUB)          \
   X(FHIP_PW_SWISH_BWD) X(FHIP_PW_TANH_BWD)
 
-// erf-based GELU for 16-bit outputs: erf by Abramowitz & Stegun 7.1.26
-// (|error| <= 1.5e-7, far below bf16 / f16 resolution) on the hardware's
-// exp2 and reciprocal.  With w = (1 - erf(|x| / sqrt 2)) / 2 = p(t) t e / 2 the
-// result is x (1 - w) for x >= 0 and x w below, i.e. max(x, 0) - |x| w: eleven
-// multiply-adds and the two transcendentals per element, no cancellation on
-// the negative side.
-__device__ __forceinline__ float gelu_erf_16bit(float x) {
-  const float ax = __builtin_fabsf(x);
-  // t = 1 / (1 + 0.3275911 |x| / sqrt 2)
-  const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(0.23164189f, ax, 1.f));
-  // half of the polynomial's coefficients
-  float p = __builtin_fmaf(0.5307027145f, t, -0.7265760135f);
-  p = __builtin_fmaf(p, t, 0.7107068705f);
-  p = __builtin_fmaf(p, t, -0.142248368f);
-  p = __builtin_fmaf(p, t, 0.127414796f);
-  // e = exp(-x^2 / 2) = exp2(-(|x| sqrt(log2(e) / 2))^2)
-  const float u = ax * 0.84932180028801904272f;
-  const float e = __builtin_amdgcn_exp2f(-u * u);
-  const float w = p * t * e;
-  return __builtin_fmaf(-ax, w, __builtin_fmaxf(x, 0.f));
-}
-
 // One lane evaluates 8 elements.  MODE >= 0 fixes the mode at compile time;
 // MODE < 0 branches on the runtime mode once per 8 elements, each arm with the
 // mode folded in (a per-element switch would dominate the kernel).
@@ -201,7 +179,7 @@ __device__ __forceinline__ void evaluate(const PwFastArgs &g,
   } else if constexpr (MODE == FHIP_PW_GELU_FWD && DT != 0) {
 #pragma unroll
     for (int i = 0; i < 8; ++i)
-      r[i] = gelu_erf_16bit(a[i]);
+      r[i] = fhip_gelu_erf_16bit(a[i]);
   } else if constexpr (MODE >= 0) {
 #pragma unroll
     for (int i = 0; i < 8; ++i)

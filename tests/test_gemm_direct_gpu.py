@@ -1,0 +1,96 @@
+"""Direct matrix-product kernels (fragments straight from global memory) vs the
+oracle, at the sizes where they can go wrong: one row, tile edges, K tails of
+every length class, rows that start on odd elements, batches, split K."""
+import numpy as np
+import pytest
+
+from fusilli_amd import capi
+from oracle import oracle
+from helpers import HT, assert_close, rand
+from test_gemm_mfma_gpu import make_operand, ref_matmul
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = [capi.FLOAT, capi.BFLOAT16, capi.HALF, capi.INT8, capi.FP8E4M3, capi.FP8E5M2]
+
+
+def run(ctx, a, b, c_dtype, out_dtype=None, epilogue=(), epi_tensors=()):
+    out_dtype = c_dtype if out_dtype is None else out_dtype
+    cdims = list(np.broadcast_shapes(tuple(a.dims[:-2]), tuple(b.dims[:-2]))) + [a.dims[-2], b.dims[-1]]
+    out = HT.empty(cdims, out_dtype)
+    d = capi.MatmulDesc()
+    d.a, d.b = a.desc(), b.desc()
+    d.c = capi.TensorDesc.make(cdims, out.strides, c_dtype)
+    d.out, d.out_dtype = out.desc(), out_dtype
+    d.epilogue = capi.make_epilogue(list(epilogue))
+    assert ctx.lib.fhip_matmul_supported(d) == 1
+    bufs = [t.upload(ctx) for t in epi_tensors]
+    da, db, do = a.upload(ctx), b.upload(ctx), out.upload(ctx)
+    ctx.matmul(d, da, db, do, epilogue_operands=bufs)
+    name = ctx.last_kernel()
+    assert name == "matmul_f32_splitk" if a.dtype == capi.FLOAT else name.startswith("gemm_direct"), name
+    return out.fetch(ctx, do), name
+
+
+def check(got, ref, dtype):
+    if dtype == capi.INT8:
+        assert np.array_equal(got, ref)
+    else:
+        assert_close(got, ref, capi.FLOAT, rtol=1e-4)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("m,n,k", [
+    (1, 40, 16),      # one row, the shortest K of 8-bit types
+    (16, 16, 128),    # exactly one tile, whole steps
+    (7, 37, 131),     # tails of K and N, odd row pitches
+    (17, 65, 77),     # two row tiles
+    (33, 66, 300),    # four row tiles, a second tile with one row
+    (130, 70, 1029),  # several tiles, K split over four wavefronts
+])
+def test_direct_orientations_and_edges(ctx, dtype, ta, tb, m, n, k):
+    a = make_operand(90, 0, m, k, dtype, ta)
+    b = make_operand(90, 1, k, n, dtype, tb)
+    out, _ = run(ctx, a, b, capi.INT32 if dtype == capi.INT8 else capi.FLOAT)
+    check(out.logical(), ref_matmul(a, b), dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("tb", [False, True])
+@pytest.mark.parametrize("m", [3, 20, 50])
+def test_direct_split_k(ctx, dtype, tb, m):
+    # few tiles over a long K: parts on workgroups of their own, added in order
+    k = (24704 if capi.DTYPE_SIZE[dtype] > 1 else 49408) + 8
+    a = make_operand(91, 0, m, k, dtype, False)
+    b = make_operand(91, 1, k, 34, dtype, tb)
+    out, name = run(ctx, a, b, capi.INT32 if dtype == capi.INT8 else capi.FLOAT)
+    if dtype != capi.FLOAT:
+        assert "split=" in name and not name.endswith("split=1"), name
+    check(out.logical(), ref_matmul(a, b), dtype)
+
+
+@pytest.mark.parametrize("dtype", [capi.FLOAT, capi.HALF, capi.INT8])
+def test_direct_batched(ctx, dtype):
+    a = make_operand(92, 0, 19, 45, dtype, False, batch=3)
+    cdt = capi.INT32 if dtype == capi.INT8 else capi.FLOAT
+    for batch in (3, 1):
+        b = make_operand(92, 1, 45, 33, dtype, False, batch=batch)
+        out, _ = run(ctx, a, b, cdt)
+        check(out.logical(), ref_matmul(a, b), dtype)
+
+
+@pytest.mark.parametrize("dtype", [capi.FLOAT, capi.BFLOAT16, capi.FP8E4M3])
+@pytest.mark.parametrize("m,k", [(5, 90), (60, 90), (5, 49000)])
+def test_direct_epilogue(ctx, dtype, m, k):
+    # a row vector, a full operand and a unary step, also behind a split K
+    a = make_operand(93, 0, m, k, dtype, False)
+    b = make_operand(93, 1, k, 41, dtype, True)
+    bias = HT.from_logical(rand(93, 2, [1, 41]), capi.BFLOAT16)
+    full = HT.from_logical(rand(93, 3, [m, 41]), capi.FLOAT)
+    epi = [capi.epilogue_op(capi.PW["ADD"], capi.FLOAT, operand=bias.desc(), operand_index=0),
+           capi.epilogue_op(capi.PW["MUL"], capi.FLOAT, operand=full.desc(), operand_index=1),
+           capi.epilogue_op(capi.PW["GELU_FWD"], capi.BFLOAT16)]
+    out, _ = run(ctx, a, b, capi.FLOAT, out_dtype=capi.BFLOAT16, epilogue=epi, epi_tensors=[bias, full])
+    ref = (ref_matmul(a, b) + bias.logical()) * full.logical()
+    assert_close(out.logical(), oracle.pointwise(capi.PW["GELU_FWD"], [ref]), capi.BFLOAT16)
