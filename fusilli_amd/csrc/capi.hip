@@ -39,6 +39,8 @@ FhipKnobs parse_knobs() {
     k.conv_rows = atoi(e);
   if (const char *e = getenv("FUSILLI_HIP_WGRAD_DIRECT"))
     k.wgrad_direct = atoi(e);
+  if (const char *e = getenv("FUSILLI_HIP_SDPA_DECODE"))
+    k.sdpa_decode = atoi(e);
   if (const char *e = getenv("FUSILLI_HIP_DGRAD_ROWS"))
     k.dgrad_rf = atoi(e);
   if (const char *e = getenv("FUSILLI_HIP_GEMM_TILE"))

@@ -99,6 +99,12 @@ bool fhip_fast_sdpa_applicable(const fhip_sdpa_desc *d);
 int fhip_fast_sdpa(fhip_ctx *ctx, const fhip_sdpa_desc *d, const void *q,
                    const void *k, const void *v, const void *mask, void *o);
 
+// Few query rows per key / value head (decode): keys split over workgroups.  For
+// descriptors that fhip_fast_sdpa takes; `handled` false where the tiled kernel is
+// the faster one.
+int fhip_decode_sdpa(fhip_ctx *ctx, const fhip_sdpa_desc *d, const void *q,
+                     const void *k, const void *v, void *o, bool *handled);
+
 bool fhip_fast_norm_applicable(const fhip_norm_desc *d);
 int fhip_fast_norm(fhip_ctx *ctx, const fhip_norm_desc *d, const void *x,
                    const void *scale, const void *bias, const DevEpilogue &epi,

@@ -995,6 +995,12 @@ int fhip_fast_sdpa(fhip_ctx *ctx, const fhip_sdpa_desc *d, const void *q,
                (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)o) &
                 15) == 0,
                "sdpa: Q, K, V, O must be 16-byte aligned");
+  {
+    bool handled = false;
+    const int rc = fhip_decode_sdpa(ctx, d, q, k, v, o, &handled);
+    if (handled)
+      return rc;
+  }
   bool staged_mask = false;
   SdpaArgs g{};
   g.q = (const char *)q;

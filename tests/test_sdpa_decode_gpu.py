@@ -1,0 +1,50 @@
+"""Attention with the keys split over workgroups (few query rows per key / value
+head), and the tiled kernel on the same problems, vs the oracle."""
+import pytest
+
+from fusilli_amd import capi
+from oracle import oracle
+from helpers import HT, assert_close, rand
+from test_sdpa_flash_gpu import CASES, bshd_strides, run
+
+pytestmark = pytest.mark.gpu
+
+DECODE = [
+    dict(B=1, Hq=1, Hkv=1, Sq=1, Skv=1, causal=False),       # one key
+    dict(B=2, Hq=4, Hkv=2, Sq=1, Skv=33, causal=False),      # one key past a chunk
+    dict(B=3, Hq=8, Hkv=1, Sq=1, Skv=1000, causal=False),    # grouped heads, splits
+    dict(B=1, Hq=8, Hkv=2, Sq=5, Skv=777, causal=False),     # 20 rows: a second tile
+    dict(B=1, Hq=2, Hkv=1, Sq=8, Skv=515, causal=True),      # exactly one tile, masked
+    dict(B=1, Hq=3, Hkv=3, Sq=90, Skv=300, causal=True),     # wavefronts without a live key
+    dict(B=1, Hq=1, Hkv=1, Sq=40, Skv=7, causal=True),       # fewer keys than queries
+]
+
+
+@pytest.mark.parametrize("case", DECODE + CASES)
+@pytest.mark.parametrize("dtype", [capi.BFLOAT16, capi.HALF])
+@pytest.mark.parametrize("hd", [128, 64])
+@pytest.mark.parametrize("decode", [1, 0])
+def test_both_kernels_vs_oracle(ctx, knobs, case, dtype, hd, decode):
+    knobs(SDPA_DECODE=decode)
+    c = case
+    q = HT.from_logical(rand(56, 0, [c["B"], c["Hq"], c["Sq"], hd], std=2.0), dtype)
+    k = HT.from_logical(rand(56, 1, [c["B"], c["Hkv"], c["Skv"], hd], std=2.0), dtype)
+    v = HT.from_logical(rand(56, 2, [c["B"], c["Hkv"], c["Skv"], hd]), dtype)
+    out = run(ctx, q, k, v, causal=c["causal"])
+    assert ctx.last_kernel().startswith("sdpa_decode" if decode else "sdpa_fwd"), ctx.last_kernel()
+    ref = oracle.sdpa(q.logical(), k.logical(), v.logical(), is_causal=c["causal"])
+    assert_close(out.logical(), ref, dtype, str(case))
+
+
+@pytest.mark.parametrize("hd", [128, 64])
+def test_decode_layout_and_scale(ctx, knobs, hd):
+    # heads interleaved per position, custom scale, several splits
+    knobs(SDPA_DECODE=1)
+    dims_q, dims_k = [2, 6, 3, hd], [2, 2, 900, hd]
+    q = HT.from_logical(rand(57, 0, dims_q), capi.BFLOAT16, bshd_strides(dims_q))
+    k = HT.from_logical(rand(57, 1, dims_k), capi.BFLOAT16, bshd_strides(dims_k))
+    v = HT.from_logical(rand(57, 2, dims_k), capi.BFLOAT16, bshd_strides(dims_k))
+    out = run(ctx, q, k, v, scale=0.31, o_strides=bshd_strides(dims_q))
+    assert "splits=" in ctx.last_kernel() and not ctx.last_kernel().endswith("splits=1"), ctx.last_kernel()
+    assert_close(out.logical(), oracle.sdpa(q.logical(), k.logical(), v.logical(), scale=0.31),
+                 capi.BFLOAT16)
