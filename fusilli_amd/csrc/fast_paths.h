@@ -110,6 +110,12 @@ int fhip_fast_norm(fhip_ctx *ctx, const fhip_norm_desc *d, const void *x,
                    const void *scale, const void *bias, const DevEpilogue &epi,
                    void *out, void *mean, void *inv_variance);
 
+// Dense rows that those kernels do not take (odd lengths, long rows with a fused
+// chain): `handled` false where rows are not dense.
+int fhip_loose_norm(fhip_ctx *ctx, const fhip_norm_desc *d, const void *x,
+                    const void *scale, const void *bias, const DevEpilogue &epi,
+                    void *out, void *mean, void *inv_variance, bool *handled);
+
 // Rows too long for the register-resident kernels (rownorm_long.hip); the
 // layout conditions are the caller's (rownorm.hip).
 bool fhip_norm_long_applicable(const fhip_norm_desc *d);

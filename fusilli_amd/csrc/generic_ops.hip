@@ -1819,6 +1819,10 @@ int fhip_norm_fwd(fhip_ctx *ctx, const fhip_norm_desc *d, const void *x,
     return 1;
   if (fhip_fast_norm_applicable(d))
     return fhip_fast_norm(ctx, d, x, scale, bias, epi, out, mean, inv_variance);
+  bool handled = false;
+  const int rc = fhip_loose_norm(ctx, d, x, scale, bias, epi, out, mean, inv_variance, &handled);
+  if (handled)
+    return rc;
   fhip_note_kernel(ctx, "norm_generic");
 
   NormArgs g{};

@@ -90,9 +90,9 @@ bool pick_shape(int64_t inner, int vec, int *chunks, int *wpr) {
   return false;
 }
 
-} // namespace
-
-bool fhip_fast_norm_applicable(const fhip_norm_desc *d) {
+// The conditions of every kernel here: floating rows dense in memory that X, OUT,
+// scale, bias and the fused operands walk alike, in steps of `vec` elements.
+bool rows_alike(const fhip_norm_desc *d, const InnerLayout &lay, int vec) {
   const fhip_tensor_desc &x = d->x;
   if (!fast_dtype(x.dtype) || d->out.dtype != x.dtype)
     return false;
@@ -101,16 +101,7 @@ bool fhip_fast_norm_applicable(const fhip_norm_desc *d) {
   for (int i = 0; i < d->epilogue.count; ++i)
     if (fhip_pw_is_transcendental(d->epilogue.op[i].mode))
       return false;
-  const InnerLayout lay = inner_layout(x);
-  if (!lay.dense)
-    return false;
-  const int vec = 16 / fhip_dtype_size(x.dtype);
-  if (lay.inner % vec != 0)
-    return false;
-  // rows that do not fit the register-resident kernels go to the long-row
-  // kernels (no fused pointwise chain there)
-  int chunks, wpr;
-  if (!pick_shape(lay.inner, vec, &chunks, &wpr) && !fhip_norm_long_applicable(d))
+  if (!lay.dense || lay.inner % vec != 0)
     return false;
   const int64_t xrs = x.dim[0] > 1 ? x.stride[0] : lay.inner;
   const int64_t ors = d->out.dim[0] > 1 ? d->out.stride[0] : lay.inner;
@@ -145,16 +136,9 @@ bool fhip_fast_norm_applicable(const fhip_norm_desc *d) {
   return true;
 }
 
-int fhip_fast_norm(fhip_ctx *ctx, const fhip_norm_desc *d, const void *x,
-                   const void *scale, const void *bias, const DevEpilogue &epi,
-                   void *out, void *mean, void *inv_variance) {
-  const InnerLayout lay = inner_layout(d->x);
-  const int vec = 16 / fhip_dtype_size(d->x.dtype);
-  int chunks = 1, wpr = 1;
-  if (!pick_shape(lay.inner, vec, &chunks, &wpr))
-    return fhip_norm_long(ctx, d, lay.inner, x, scale, bias, out, mean,
-                          inv_variance);
-  RowNormArgs g{};
+void fill_args(const fhip_norm_desc *d, const InnerLayout &lay, const void *x, const void *scale,
+               const void *bias, const DevEpilogue &epi, void *out, void *mean, void *inv_variance,
+               RowNormArgs &g) {
   g.x = x;
   g.scale = scale;
   g.bias = bias;
@@ -190,6 +174,48 @@ int fhip_fast_norm(fhip_ctx *ctx, const fhip_norm_desc *d, const void *x,
                      ? 1
                      : 0;
   }
+}
+
+} // namespace
+
+bool fhip_fast_norm_applicable(const fhip_norm_desc *d) {
+  if (!fast_dtype(d->x.dtype))
+    return false;
+  const InnerLayout lay = inner_layout(d->x);
+  const int vec = 16 / fhip_dtype_size(d->x.dtype);
+  // rows that do not fit the register-resident kernels go to the long-row
+  // kernels (no fused pointwise chain there)
+  int chunks, wpr;
+  return rows_alike(d, lay, vec) &&
+         (pick_shape(lay.inner, vec, &chunks, &wpr) || fhip_norm_long_applicable(d));
+}
+
+// Dense rows that the kernels above leave: any length, element alignment (down to
+// 2 x 292 the walk beats the generic kernel, 8.6 us against 5.0).
+int fhip_loose_norm(fhip_ctx *ctx, const fhip_norm_desc *d, const void *x, const void *scale,
+                    const void *bias, const DevEpilogue &epi, void *out, void *mean,
+                    void *inv_variance, bool *handled) {
+  const InnerLayout lay = inner_layout(d->x);
+  *handled = fast_dtype(d->x.dtype) && lay.inner > 0 && d->x.dim[0] > 0 && d->x.dim[0] < (1ll << 31) &&
+             rows_alike(d, lay, 1);
+  if (!*handled)
+    return 0;
+  RowNormArgs g{};
+  fill_args(d, lay, x, scale, bias, epi, out, mean, inv_variance, g);
+  return fhip_norm_walk(ctx, d->x.dtype, g);
+}
+
+int fhip_fast_norm(fhip_ctx *ctx, const fhip_norm_desc *d, const void *x,
+                   const void *scale, const void *bias, const DevEpilogue &epi,
+                   void *out, void *mean, void *inv_variance) {
+  const InnerLayout lay = inner_layout(d->x);
+  const int vec = 16 / fhip_dtype_size(d->x.dtype);
+  int chunks = 1, wpr = 1;
+  if (!pick_shape(lay.inner, vec, &chunks, &wpr))
+    return fhip_norm_long(ctx, d, lay.inner, x, scale, bias, out, mean,
+                          inv_variance);
+  RowNormArgs g{};
+  fill_args(d, lay, x, scale, bias, epi, out, mean, inv_variance, g);
   // 16-byte alignment of every vector-accessed base pointer.
   auto aligned = [](const void *p) { return ((uintptr_t)p & 15u) == 0; };
   FHIP_REQUIRE(ctx, aligned(x) && aligned(out) && aligned(scale) &&

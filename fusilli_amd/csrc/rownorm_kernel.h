@@ -32,6 +32,9 @@ struct RowNormArgs {
   FastEpiOp epi[FHIP_MAX_EPILOGUE];
 };
 
+// Rows of any length and alignment (rownorm_walk.hip).
+int fhip_norm_walk(fhip_ctx *ctx, int dtype, const RowNormArgs &n);
+
 // Compile-time specialisations of the per-row work.  Everything a variant
 // fixes is resolved at compile time so the hot loop is straight-line code; the
 // general variant decides the same things with wavefront-uniform branches.

@@ -335,3 +335,29 @@ def test_rownorm_several_row_blocks_per_workgroup(ctx, knobs, rows, cols, kind):
         out = run_norm(ctx, x, s, None, eps=1e-6, y_dtype=capi.FLOAT,
                        epilogue=epi, epi_tensors=ops, expect_path=2)
     assert_close(out.logical(), ref, capi.BFLOAT16, f"{kind} {rows}x{cols}")
+
+
+@pytest.mark.parametrize("dtype", [capi.BFLOAT16, capi.HALF, capi.FLOAT])
+@pytest.mark.parametrize("rows,cols", [
+    # one element, under and just over a vector, both sides of the wavefront / workgroup
+    # line, rows in segments (the last one short), more rows than segments pay for
+    (3, 1), (5, 7), (9, 9), (4, 1023), (7, 1025), (3, 16387), (2, 70001), (600, 16387)])
+@pytest.mark.parametrize("layernorm", [False, True])
+def test_norm_rows_of_any_length_vs_oracle(ctx, dtype, rows, cols, layernorm):
+    x = HT.from_logical(rand(41, 0, [rows, cols], mean=0.5, std=2.0), dtype)
+    s = HT.from_logical(rand(41, 1, [1, cols], mean=1.0, std=0.1), dtype)
+    if layernorm:
+        b = HT.from_logical(rand(41, 2, [1, cols]), dtype)
+        out, mean, rstd = run_norm(ctx, x, s, b, eps=1e-5, layernorm=True, stats=True)
+        y, m, r = oracle.layernorm(x.logical(), s.logical(), b.logical(), 1e-5)
+        assert_close(mean.logical(), m.reshape(-1), capi.FLOAT, "mean")
+        assert_close(rstd.logical(), r.reshape(-1), capi.FLOAT, "rstd")
+    else:
+        mul = HT.from_logical(rand(41, 3, [rows, cols]), dtype)
+        # RMSNorm, ReLU, times a tensor of X's own layout (f32 and 16-bit vectors, tails)
+        out = run_norm(ctx, x, s, None, eps=1e-6, y_dtype=capi.FLOAT, epi_tensors=[mul],
+                       epilogue=[capi.epilogue_op(capi.PW["RELU_FWD"], capi.FLOAT),
+                                 capi.epilogue_op(capi.PW["MUL"], dtype, operand=mul.desc())])
+        y = np.maximum(oracle.rmsnorm(x.logical(), s.logical(), 1e-6), 0) * mul.logical()
+    assert ctx.last_kernel().startswith("rownorm_walk"), ctx.last_kernel()
+    assert_close(out.logical(), y, dtype, f"{rows} x {cols}")
