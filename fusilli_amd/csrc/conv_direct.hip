@@ -934,6 +934,10 @@ int fhip_direct_conv_fprop(fhip_ctx *ctx, const fhip_conv_desc *d,
       return 0;
     }
   }
+  bool handled = false;
+  const int rc = fhip_few_conv_fprop(ctx, d, x, w, epi, out, &handled);
+  if (handled || rc != 0)
+    return rc;
   fhip_note_kernel(ctx, "conv_direct");
   DcArgs g{};
   FHIP_REQUIRE(ctx, make_args(d, g),
@@ -954,6 +958,10 @@ int fhip_direct_conv_fprop(fhip_ctx *ctx, const fhip_conv_desc *d,
 
 int fhip_direct_conv_dgrad(fhip_ctx *ctx, const fhip_conv_desc *d,
                            const void *dy, const void *w, void *dx) {
+  bool handled = false;
+  const int rc = fhip_few_conv_dgrad(ctx, d, dy, w, dx, &handled);
+  if (handled || rc != 0)
+    return rc;
   fhip_note_kernel(ctx, "conv_direct_dgrad");
   DcArgs g{};
   FHIP_REQUIRE(ctx, make_args(d, g),
@@ -974,6 +982,10 @@ int fhip_direct_conv_dgrad(fhip_ctx *ctx, const fhip_conv_desc *d,
 
 int fhip_direct_conv_wgrad(fhip_ctx *ctx, const fhip_conv_desc *d,
                            const void *dy, const void *x, void *dw) {
+  bool handled = false;
+  const int rc = fhip_few_conv_wgrad(ctx, d, dy, x, dw, &handled);
+  if (handled || rc != 0)
+    return rc;
   fhip_note_kernel(ctx, "conv_direct_wgrad");
   DcArgs g{};
   FHIP_REQUIRE(ctx, make_args(d, g),

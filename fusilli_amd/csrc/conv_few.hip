@@ -1,0 +1,762 @@
+// Convolutions over few input channels (the first layer of a network): one group,
+// two spatial dims, channels-first tensors, at most 112 (channel, tap) pairs.
+//
+// Bound by reading and writing the many-channel tensor once; the direct kernels
+// (conv_direct.hip) kept one pixel per thread and fetched every X or DY value from
+// the caches once per tap and channel block.  All arithmetic stays f32: 16-bit
+// tensors are widened when they are staged.
+//   * forward: X of 256 output pixels, padded with zeros, and the filter sit in LDS;
+//     pixels x output channels on 16 x 16 x 4 f32 MFMAs over the (channel, tap) pairs.
+//     A wavefront's four tiles interleave their pixels so that a lane ends up with 16
+//     consecutive pixels of one channel (64-byte stores);
+//   * weight gradient: output channels x pairs on the same MFMAs over the pixels, DY
+//     straight from memory (four consecutive pixels per lane), X from LDS; a
+//     workgroup keeps its sums over many bands of rows, the workgroups' sums meet in
+//     the context's scratch and are added in a fixed order;
+//   * data gradient: one to four input channels leave a matrix tile mostly empty, so a
+//     lane computes 4 x 2 pixels x all channels with vector instructions, the wavefronts
+//     of a workgroup each over a share of the output channels, whose DY rows they
+//     stage for themselves; the shares are added through LDS.
+//
+// One training step (us):
+//   N100 3 -> 32, 32 x 32, 3 x 3, f32: fprop 26.2 -> 15.5, dgrad 60.5 -> 15.0, wgrad 46.1 -> 13.0
+//   N122 1 -> 64, 57 x 57, 5 x 5, bf16: 136 -> 52.6, 701 -> 78.6, 495 -> 45.7
+//
+// Reference semantics: aten.convolution / aten.convolution_backward
+// (reference support/asm_emitter.h:690-701, 868-873, 1030-1035).
+#include "common.h"
+#include "fast_paths.h"
+
+#include <type_traits>
+
+namespace {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kCfThreads = 256;
+constexpr int kCfLds = 64 * 1024;
+constexpr int kCfMaxPairs = 112;
+
+struct CfArgs {
+  int32_t N, C, H, W, K, P, Q, R, S, J; // J = C * R * S
+  int32_t pad_h, pad_w, str_h, str_w, dil_h, dil_w;
+  int64_t xs[4], ws[4], ys[4]; // element strides; ys: Y (gradients) or OUT (forward)
+  int32_t y_dt, o_dt;          // forward: rounding of the sum, type of OUT
+  int32_t lw;                  // columns of the staged X
+  uint32_t lw_magic, rows_magic, q_magic;
+  int32_t xrows;               // most rows of X staged at once
+  int32_t tiles;               // forward: workgroups per image; gradients: bands
+  int32_t band;                // output (data gradient: input) rows per band
+  int32_t quads;               // data gradient: runs of 4 pixels per row
+  DevEpilogue epi;
+};
+
+// e / d for e, d < 2^16 with magic = 2^32 / d + 1 (0 stands for d = 1)
+uint32_t cf_magic(int d) { return d == 1 ? 0u : (uint32_t)((1ull << 32) / (uint32_t)d + 1); }
+__device__ __forceinline__ int cf_div(int e, uint32_t magic) {
+  return magic == 0 ? e : (int)__umulhi((uint32_t)e, magic);
+}
+
+// X rows [row0, row0 + rows) of all channels of an image, zeros outside it, as f32.
+template <typename T>
+__device__ __forceinline__ void cf_stage_x(const CfArgs &g, const T *x, int row0, int rows,
+                                           float *xl) {
+  constexpr int kBatch = 8; // loads in flight per thread
+  const int total = g.C * g.xrows * g.lw;
+  for (int e0 = threadIdx.x; e0 < total; e0 += kBatch * kCfThreads) {
+    float v[kBatch];
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const int e = e0 + i * kCfThreads;
+      const int cr = cf_div(e, g.lw_magic), col = e - cr * g.lw;
+      const int c = cf_div(cr, g.rows_magic), r = cr - c * g.xrows;
+      const int h = row0 + r, w = col - g.pad_w;
+      const bool in = e < total && r < rows && (unsigned)h < (unsigned)g.H && (unsigned)w < (unsigned)g.W;
+      // (the load is issued either way: a branch would wait for every value)
+      const float t = (float)x[in ? c * (int)g.xs[1] + h * (int)g.xs[2] + w * (int)g.xs[3] : 0];
+      v[i] = in ? t : 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i)
+      if (e0 + i * kCfThreads < total)
+        xl[e0 + i * kCfThreads] = v[i];
+  }
+}
+
+// where pair j = (channel, tap) lies in the staged X / in the filter
+__device__ __forceinline__ int cf_pair(const CfArgs &g, int j, int *filter) {
+  const int rs = g.R * g.S;
+  const int c = j / rs, t = j - c * rs;
+  const int r = t / g.S, s = t - r * g.S;
+  *filter = c * (int)g.ws[1] + r * (int)g.ws[2] + s * (int)g.ws[3];
+  return (c * g.xrows + r * g.dil_h) * g.lw + s * g.dil_w;
+}
+
+// ---- forward -------------------------------------------------------------------
+template <typename O>
+__device__ __forceinline__ void cf_store16(void *out, int64_t at, const float (&v)[16]) {
+  constexpr int N = 16 / sizeof(O);
+  typedef O vec __attribute__((ext_vector_type(N), aligned(sizeof(O))));
+#pragma unroll
+  for (int i = 0; i < 16; i += N) {
+    vec t;
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+      t[k] = (O)v[i + k];
+    *(vec *)((O *)out + at + i) = t;
+  }
+}
+
+template <typename T, int KT>
+__global__ __launch_bounds__(kCfThreads) void conv_few_fprop_kernel(CfArgs g, const T *x,
+                                                                    const T *w, void *out) {
+  constexpr int KP = KT * 16 + (KT % 2 ? 0 : 16); // (two rows of pairs in different banks)
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  const int j4 = (g.J + 3) & ~3;
+  float *wl = smem;                 // [pair][output channel]
+  int *tab = (int *)(wl + j4 * KP); // where a pair's X lies, then its filter offset
+  int *woff = tab + j4;
+  float *xl = (float *)(woff + j4);
+  const int tid = threadIdx.x, l = tid & 63, wave = tid >> 6;
+  const int k0 = blockIdx.y * KT * 16;
+  const int n = blockIdx.x / g.tiles, t0 = (blockIdx.x % g.tiles) * kCfThreads;
+  const int pq = g.P * g.Q;
+  const int t1 = t0 + kCfThreads < pq ? t0 + kCfThreads : pq;
+  const int p0 = t0 / g.Q, p1 = (t1 - 1) / g.Q;
+  for (int j = tid; j < j4; j += kCfThreads) {
+    int f = 0, o = 0;
+    if (j < g.J)
+      o = cf_pair(g, j, &f);
+    tab[j] = o, woff[j] = f;
+  }
+  cf_stage_x(g, x + n * g.xs[0], p0 * g.str_h - g.pad_h,
+             (p1 - p0) * g.str_h + (g.R - 1) * g.dil_h + 1, xl);
+  __syncthreads();
+  for (int e0 = tid; e0 < j4 * KT * 16; e0 += 8 * kCfThreads) {
+    float v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int e = e0 + i * kCfThreads, kk = e % (KT * 16);
+      const int j = e / (KT * 16) < j4 ? e / (KT * 16) : 0;
+      const bool in = j < g.J && k0 + kk < g.K;
+      const float t = (float)w[in ? (k0 + kk) * g.ws[0] + woff[j] : 0];
+      v[i] = in ? t : 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int e = e0 + i * kCfThreads;
+      if (e < j4 * KT * 16)
+        wl[e / (KT * 16) * KP + e % (KT * 16)] = v[i];
+    }
+  }
+  __syncthreads();
+  const int first = t0 + wave * 64;
+  if (first >= t1)
+    return;
+  int base[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const int m = l & 15;
+    int px = first + (m >> 2) * 16 + t * 4 + (m & 3);
+    px = px < t1 ? px : t1 - 1;
+    const int p = px / g.Q, q = px - p * g.Q;
+    base[t] = (p - p0) * g.str_h * g.lw + q * g.str_w;
+  }
+  f32x4 acc[4][KT];
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int u = 0; u < KT; ++u)
+      acc[t][u] = f32x4{0, 0, 0, 0};
+  for (int j = l >> 4; j < j4; j += 4) {
+    const int off = tab[j];
+    float xv[4], wv[KT];
+#pragma unroll
+    for (int u = 0; u < KT; ++u)
+      wv[u] = wl[j * KP + u * 16 + (l & 15)];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      xv[t] = xl[base[t] + off];
+      xv[t] = j < g.J ? xv[t] : 0.f; // (0 x infinity)
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int u = 0; u < KT; ++u)
+        acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[t], wv[u], acc[t][u], 0, 0, 0);
+  }
+  // value r of tile t: pixel first + (l / 16) * 16 + t * 4 + r of channel l % 16
+  const int px = first + (l >> 4) * 16;
+  if (px >= t1)
+    return;
+  // (one copy of the chain for all KT tiles: the next tile's sums move to the front)
+#pragma clang loop unroll(disable)
+  for (int u = 0; u < KT; ++u) {
+    const int k = k0 + u * 16 + (l & 15);
+    float v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      v[i] = acc[i >> 2][0][i & 3];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int i = 0; i + 1 < KT; ++i)
+        acc[t][i] = acc[t][i + 1];
+    if (k >= g.K)
+      continue;
+    fhip_round_fast_vec<16>(g.y_dt, v);
+    for (int e = 0; e < g.epi.count; ++e) {
+      const DevEpiOp &o = g.epi.op[e];
+      if (o.kind == FHIP_OPERAND_NONE) {
+        fhip_pw_fast_unary_vec<true, 16>(o.mode, v, o.params.swish_beta,
+                                         o.result_dtype != FHIP_FLOAT);
+      } else {
+        const float s = o.kind == FHIP_OPERAND_SCALAR
+                            ? o.scalar
+                            : fhip_load<float>(o.ptr, o.operand_dtype,
+                                               n * o.stride[0] + k * o.stride[1]);
+        float other[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          other[i] = s;
+        fhip_pw_fast_binary_vec<16>(o.mode, o.acc_is_in1 != 0, v, other);
+      }
+      fhip_round_fast_vec<16>(o.result_dtype, v);
+    }
+    const int64_t at = n * g.ys[0] + k * g.ys[1] + px;
+    if (px + 16 <= t1) {
+      if (g.o_dt == FHIP_FLOAT)
+        cf_store16<float>(out, at, v);
+      else if (g.o_dt == FHIP_BFLOAT16)
+        cf_store16<__bf16>(out, at, v);
+      else
+        cf_store16<_Float16>(out, at, v);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (px + i < t1)
+          fhip_store<float>(out, g.o_dt, at + i, v[i]);
+    }
+  }
+}
+
+// ---- weight gradient -----------------------------------------------------------
+template <typename T, int KT>
+__device__ __forceinline__ void cf_load_dy(const T *const (&dy)[KT], int px, int np,
+                                           float (&a)[KT][4]) {
+  typedef T vec __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+  if (px + 4 <= np) {
+#pragma unroll
+    for (int u = 0; u < KT; ++u) {
+      const vec v = *(const vec *)(dy[u] + px);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        a[u][i] = (float)v[i];
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < KT; ++u)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float t = (float)dy[u][px + i < np ? px + i : 0];
+        a[u][i] = px + i < np ? t : 0.f;
+      }
+  }
+}
+
+// partial[run][k block][KT * JT tiles][4][64]: the fragments as they lie
+template <typename T, int KT, int JT>
+__global__ __launch_bounds__(kCfThreads) void conv_few_wgrad_kernel(CfArgs g, const T *dy,
+                                                                    const T *x, float *partial) {
+  constexpr int kFrag = KT * JT * 256;
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  int *pixtab = (int *)smem; // where a band's pixel lies in the staged X
+  const int slots = (g.band * g.Q + 15) & ~15;
+  float *xl = smem + slots;
+  const int tid = threadIdx.x, l = tid & 63, wave = tid >> 6;
+  const int k0 = blockIdx.y * KT * 16;
+  for (int i = tid; i < slots; i += kCfThreads) {
+    const int p = cf_div(i, g.q_magic), q = i - p * g.Q;
+    pixtab[i] = i < g.band * g.Q ? p * g.str_h * g.lw + q * g.str_w : 0;
+  }
+  int joff[JT];
+#pragma unroll
+  for (int u = 0; u < JT; ++u) {
+    const int j = u * 16 + (l & 15);
+    int f;
+    joff[u] = j < g.J ? cf_pair(g, j, &f) : 0;
+  }
+  f32x4 acc[KT][JT];
+#pragma unroll
+  for (int u = 0; u < KT; ++u)
+#pragma unroll
+    for (int v = 0; v < JT; ++v)
+      acc[u][v] = f32x4{0, 0, 0, 0};
+  const int items = g.N * g.tiles;
+  for (int item = blockIdx.x; item < items; item += gridDim.x) {
+    const int n = item / g.tiles, p0 = (item - n * g.tiles) * g.band;
+    const int rows = g.P - p0 < g.band ? g.P - p0 : g.band;
+    const int np = rows * g.Q;
+    const T *src[KT];
+#pragma unroll
+    for (int u = 0; u < KT; ++u) {
+      const int k = k0 + u * 16 + (l & 15);
+      src[u] = dy + n * g.ys[0] + (k < g.K ? k : g.K - 1) * g.ys[1] + (int64_t)p0 * g.Q;
+    }
+    float a[2][KT][4];
+    const int px0 = wave * 16 + (l >> 4) * 4;
+    cf_load_dy<T, KT>(src, px0, np, a[0]);
+    __syncthreads();
+    cf_stage_x(g, x + n * g.xs[0], p0 * g.str_h - g.pad_h,
+               (rows - 1) * g.str_h + (g.R - 1) * g.dil_h + 1, xl);
+    __syncthreads();
+    auto spend = [&](const float (&b)[KT][4], int px) {
+      const int4 at = *(const int4 *)(pixtab + px);
+      const int off[4] = {at.x, at.y, at.z, at.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float xv[JT];
+#pragma unroll
+        for (int v = 0; v < JT; ++v) {
+          xv[v] = xl[off[i] + joff[v]];
+          xv[v] = px + i < np ? xv[v] : 0.f;
+        }
+#pragma unroll
+        for (int v = 0; v < JT; ++v)
+#pragma unroll
+          for (int u = 0; u < KT; ++u)
+            acc[u][v] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[u][i], xv[v], acc[u][v], 0, 0, 0);
+      }
+    };
+    // (groups of 16 pixels, the wavefronts in turn, the next group's DY in flight)
+    for (int grp = wave * 16; grp < np; grp += 128) {
+      const int px = grp + (l >> 4) * 4;
+      cf_load_dy<T, KT>(src, px + 64, np, a[1]);
+      spend(a[0], px);
+      if (grp + 64 >= np)
+        break;
+      cf_load_dy<T, KT>(src, px + 128, np, a[0]);
+      spend(a[1], px + 64);
+    }
+  }
+  // the wavefronts' sums in a fixed order: 2 -> 0, 3 -> 1, 1 -> 0
+  __syncthreads();
+  auto put = [&](float *to) {
+#pragma unroll
+    for (int u = 0; u < KT; ++u)
+#pragma unroll
+      for (int v = 0; v < JT; ++v)
+        *(f32x4 *)(to + ((u * JT + v) * 64 + l) * 4) = acc[u][v];
+  };
+  auto take = [&](const float *from) {
+#pragma unroll
+    for (int u = 0; u < KT; ++u)
+#pragma unroll
+      for (int v = 0; v < JT; ++v)
+        acc[u][v] += *(const f32x4 *)(from + ((u * JT + v) * 64 + l) * 4);
+  };
+  if (wave >= 2)
+    put(smem + (wave - 2) * kFrag);
+  __syncthreads();
+  if (wave < 2)
+    take(smem + wave * kFrag);
+  __syncthreads();
+  if (wave == 1)
+    put(smem);
+  __syncthreads();
+  if (wave == 0) {
+    take(smem);
+    put(partial + ((int64_t)blockIdx.x * gridDim.y + blockIdx.y) * kFrag);
+  }
+}
+
+// DW = sum of the workgroups' fragments: 16 values per workgroup, 64 slices of the
+// runs, added in a fixed order.
+__global__ __launch_bounds__(256) void conv_few_wgrad_sum_kernel(CfArgs g, const float *partial,
+                                                                 void *dw, int dw_dt, int kt, int jt,
+                                                                 int64_t frags, int runs) {
+  __shared__ float lds[4][16];
+  const int tid = threadIdx.x;
+  const int64_t e0 = (int64_t)blockIdx.x * 16;
+  const float *src = partial + e0 + (tid & 3) * 4;
+  f32x4 s{0, 0, 0, 0};
+#pragma unroll 8
+  for (int r = tid >> 2; r < runs; r += 64)
+    s += *(const f32x4 *)(src + r * frags);
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    for (int o = 4; o < 64; o <<= 1)
+      s[i] += __shfl_xor(s[i], o, 64);
+  if ((tid & 63) < 4)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      lds[tid >> 6][(tid & 3) * 4 + i] = s[i];
+  __syncthreads();
+  if (tid >= 16)
+    return;
+  // value r of lane l of tile (u, v): channel u * 16 + (l / 16) * 4 + r, pair v * 16 + l % 16
+  const int64_t e = e0 + tid;
+  const int r = (int)(e & 3), l = (int)(e >> 2) & 63;
+  const int tile = (int)(e >> 8);
+  const int v = tile % jt, u = tile / jt % kt, kb = tile / (jt * kt);
+  const int k = (kb * kt + u) * 16 + (l >> 4) * 4 + r, j = v * 16 + (l & 15);
+  if (k >= g.K || j >= g.J)
+    return;
+  int f;
+  cf_pair(g, j, &f);
+  fhip_store<float>(dw, dw_dt, k * g.ws[0] + f, (lds[0][tid] + lds[1][tid]) + (lds[2][tid] + lds[3][tid]));
+}
+
+// ---- data gradient (unit stride and dilation) -----------------------------------
+constexpr int kCfStage = 16; // loads per lane of one channel's rows of DY
+constexpr int kCfRows = 2;   // rows of DX per lane: every staged row feeds two of them
+
+template <typename T, int C, int S>
+__global__ __launch_bounds__(512) void conv_few_dgrad_kernel(CfArgs g, const T *dy, const T *w,
+                                                             T *dx) {
+  constexpr int WP = (S * C + 3) & ~3; // a filter row of all channels
+  constexpr int SPAN = (S + 3 + 3) & ~3;
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  const int tid = threadIdx.x, l = tid & 63, wave = tid >> 6;
+  const int threads = blockDim.x, waves = threads >> 6;
+  const int pitch = 4 * g.quads + SPAN - 4, rows = g.band + g.R - 1;
+  float *wl = smem; // [k][r][S][C]
+  float *tile = smem + g.K * g.R * WP + wave * rows * pitch;
+  const int n = blockIdx.x / g.tiles, h0 = (blockIdx.x % g.tiles) * g.band;
+  // the element of every staged row this lane brings in, -1: a zero
+  int at[kCfStage];
+#pragma unroll
+  for (int i = 0; i < kCfStage; ++i) {
+    const int e = l + 64 * i;
+    const int row = cf_div(e, g.lw_magic), col = e - row * pitch;
+    const int p = h0 + g.pad_h - (g.R - 1) + row, q = g.pad_w - (S - 1) + col;
+    at[i] = row < rows && (unsigned)p < (unsigned)g.P && (unsigned)q < (unsigned)g.Q
+                ? p * (int)g.ys[2] + q * (int)g.ys[3]
+                : -1;
+  }
+  const int loads = (rows * pitch + 63) / 64;
+  T ahead[kCfStage];
+  auto fetch = [&](int k) {
+    const T *src = dy + n * g.ys[0] + k * g.ys[1];
+#pragma unroll
+    for (int i = 0; i < kCfStage; ++i)
+      if (i < loads)
+        ahead[i] = src[at[i] >= 0 ? at[i] : 0];
+  };
+  if (wave < g.K)
+    fetch(wave);
+#pragma unroll 4
+  for (int e = tid; e < g.K * g.R * WP; e += threads) {
+    const int kr = e / WP, sc = e % WP < S * C ? e % WP : 0;
+    const int k = kr / g.R, r = kr - k * g.R;
+    wl[e] = (float)w[k * g.ws[0] + (sc % C) * g.ws[1] + r * g.ws[2] + (sc / C) * g.ws[3]];
+  }
+  // (lanes behind the band repeat its last rows)
+  const int hl = l / g.quads * kCfRows, qd = l % g.quads;
+  const float *mine = tile + (hl + kCfRows <= g.band ? hl : g.band - kCfRows) * pitch + qd * 4;
+  float acc[kCfRows][C][4];
+#pragma unroll
+  for (int y = 0; y < kCfRows; ++y)
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        acc[y][c][i] = 0.f;
+  __syncthreads();
+  for (int k = wave; k < g.K; k += waves) {
+    // (a wavefront's LDS operations complete in order: its tile needs no barrier)
+#pragma unroll
+    for (int i = 0; i < kCfStage; ++i)
+      if (i < loads && l + 64 * i < rows * pitch)
+        tile[l + 64 * i] = at[i] >= 0 ? (float)ahead[i] : 0.f;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (k + waves < g.K)
+      fetch(k + waves);
+    // staged row t is tap R - 1 - t of this lane's first row, tap R - t of its second
+    float f[kCfRows][WP];
+    for (int t = 0; t < g.R + kCfRows - 1; ++t) {
+      float v[SPAN];
+#pragma unroll
+      for (int i = 0; i < SPAN; i += 4) {
+        const f32x4 x = *(const f32x4 *)(mine + t * pitch + i);
+        v[i] = x.x, v[i + 1] = x.y, v[i + 2] = x.z, v[i + 3] = x.w;
+      }
+#pragma unroll
+      for (int i = 0; i < WP; ++i)
+        f[1][i] = f[0][i];
+      if (t < g.R) {
+        const float *wr = wl + (k * g.R + g.R - 1 - t) * WP;
+#pragma unroll
+        for (int i = 0; i < WP; i += 4) {
+          const f32x4 x = *(const f32x4 *)(wr + i);
+          f[0][i] = x.x, f[0][i + 1] = x.y, f[0][i + 2] = x.z, f[0][i + 3] = x.w;
+        }
+      }
+      auto add = [&](auto yy) {
+        constexpr int Y = decltype(yy)::value;
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+#pragma unroll
+          for (int c = 0; c < C; ++c)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              acc[Y][c][i] = __builtin_fmaf(v[i + S - 1 - s], f[Y][s * C + c], acc[Y][c][i]);
+      };
+      if (t < g.R)
+        add(std::integral_constant<int, 0>{});
+      if (t > 0)
+        add(std::integral_constant<int, 1>{});
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+  // the wavefronts' sums, added in their order: [wave][row][channel][lane][pixel]
+  __syncthreads();
+#pragma unroll
+  for (int y = 0; y < kCfRows; ++y)
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+      *(f32x4 *)(smem + (((wave * kCfRows + y) * C + c) * 64 + l) * 4) =
+          f32x4{acc[y][c][0], acc[y][c][1], acc[y][c][2], acc[y][c][3]};
+  __syncthreads();
+  const int quad = (tid & 255) >> 2;
+  const int row0 = quad / g.quads * kCfRows, col = (quad % g.quads) * 4 + (tid & 3);
+  if (row0 + kCfRows > g.band || col >= g.W)
+    return;
+  for (int yc = tid >> 8; yc < kCfRows * C; yc += threads >> 8) {
+    const int y = yc / C, c = yc % C;
+    if (h0 + row0 + y >= g.H)
+      continue;
+    const float *s = smem + yc * 256 + (tid & 255);
+    float sum = s[0];
+    for (int i = 1; i < waves; ++i)
+      sum += s[i * kCfRows * C * 256];
+    dx[n * g.xs[0] + c * g.xs[1] + (h0 + row0 + y) * g.xs[2] + col * g.xs[3]] = (T)sum;
+  }
+}
+
+// ---- host side -------------------------------------------------------------------
+bool cf_type(int dt) { return dt == FHIP_FLOAT || dt == FHIP_BFLOAT16 || dt == FHIP_HALF; }
+
+// Everything but the tiling; `y`: OUT (forward) or DY.
+bool cf_args(const fhip_conv_desc *d, const fhip_tensor_desc &y, CfArgs &g) {
+  if (d->spatial_rank != 2 || d->x.rank != 4 || d->w.rank != 4 || y.rank != 4)
+    return false;
+  if (d->w.dim[1] != d->x.dim[1] || d->x.dtype != d->w.dtype || !cf_type(d->x.dtype))
+    return false;
+  const int64_t lim = 1 << 16;
+  for (int i = 0; i < 4; ++i)
+    if (d->x.dim[i] >= lim || d->w.dim[i] >= lim || y.dim[i] >= lim)
+      return false;
+  for (int i = 0; i < 2; ++i)
+    if (d->padding[i] >= lim || d->stride[i] >= lim || d->dilation[i] >= lim)
+      return false;
+  const int64_t J = d->w.dim[1] * d->w.dim[2] * d->w.dim[3];
+  // (fewer output channels than half a tile stay on the kernel of one pixel per thread)
+  if (J > kCfMaxPairs || d->w.dim[0] < 8)
+    return false;
+  g.N = (int32_t)d->x.dim[0], g.C = (int32_t)d->x.dim[1];
+  g.H = (int32_t)d->x.dim[2], g.W = (int32_t)d->x.dim[3];
+  g.K = (int32_t)d->w.dim[0], g.R = (int32_t)d->w.dim[2], g.S = (int32_t)d->w.dim[3];
+  g.P = (int32_t)y.dim[2], g.Q = (int32_t)y.dim[3];
+  g.J = (int32_t)J;
+  g.pad_h = (int32_t)d->padding[0], g.pad_w = (int32_t)d->padding[1];
+  g.str_h = (int32_t)d->stride[0], g.str_w = (int32_t)d->stride[1];
+  g.dil_h = (int32_t)d->dilation[0], g.dil_w = (int32_t)d->dilation[1];
+  auto strides = [](const fhip_tensor_desc &t, int64_t (&s)[4]) {
+    int64_t image = 0;
+    for (int i = 0; i < 4; ++i) {
+      s[i] = t.dim[i] == 1 ? 0 : t.stride[i];
+      if (s[i] >= (1ll << 31))
+        return false;
+      image += i ? (t.dim[i] - 1) * s[i] : 0;
+    }
+    return image < (1ll << 31); // offsets inside one image are 32-bit
+  };
+  if (!strides(d->x, g.xs) || !strides(d->w, g.ws) || !strides(y, g.ys))
+    return false;
+  // X walked along its rows (channels-last tensors have kernels of their own)
+  return g.W == 1 || g.xs[3] == 1;
+}
+
+// pixels of a plane of OUT / DY consecutive
+bool cf_planes(const CfArgs &g) {
+  return (g.Q == 1 || g.ys[3] == 1) && (g.P == 1 || g.ys[2] == g.Q);
+}
+
+// staged X of `span` rows of output; false where LDS does not hold it beside `other` floats
+bool cf_stage(CfArgs &g, int span, int64_t other, size_t *bytes) {
+  const int64_t lw = (int64_t)(g.Q - 1) * g.str_w + (int64_t)(g.S - 1) * g.dil_w + 1;
+  const int64_t rows = (int64_t)(span - 1) * g.str_h + (int64_t)(g.R - 1) * g.dil_h + 1;
+  const int64_t total = lw * rows * g.C;
+  if (lw >= (1 << 16) || rows >= (1 << 16) || total >= (1 << 16) || (total + other) * 4 > kCfLds)
+    return false;
+  g.lw = (int32_t)lw, g.lw_magic = cf_magic(g.lw);
+  g.xrows = (int32_t)rows, g.rows_magic = cf_magic(g.xrows);
+  *bytes = (size_t)(total + other) * 4;
+  return true;
+}
+
+template <typename F> void cf_by_type(int dt, F &&f) {
+  if (dt == FHIP_FLOAT)
+    f(float{});
+  else if (dt == FHIP_BFLOAT16)
+    f(__bf16{});
+  else
+    f(_Float16{});
+}
+
+} // namespace
+
+int fhip_few_conv_fprop(fhip_ctx *ctx, const fhip_conv_desc *d, const void *x, const void *w,
+                        const DevEpilogue &epi, void *out, bool *handled) {
+  *handled = false;
+  CfArgs g{};
+  if (!cf_args(d, d->out, g) || !cf_planes(g) || !cf_type(d->y.dtype) || !cf_type(d->out.dtype) ||
+      !fhip_epilogue_is_fast(d->epilogue))
+    return 0;
+  for (int i = 0; i < epi.count; ++i)
+    if (epi.op[i].kind == FHIP_OPERAND_TENSOR &&
+        ((g.P > 1 && epi.op[i].stride[2] != 0) || (g.Q > 1 && epi.op[i].stride[3] != 0)))
+      return 0; // (operands per channel only)
+  const int kt = g.K > 32 ? 4 : g.K > 16 ? 2 : 1;
+  const int j4 = (g.J + 3) / 4 * 4, kp = kt * 16 + (kt % 2 ? 0 : 16);
+  const int span = (kCfThreads - 1 + g.Q - 1) / g.Q + 1;
+  size_t lds = 0;
+  if (!cf_stage(g, span < g.P ? span : g.P, (int64_t)j4 * (kp + 2), &lds))
+    return 0;
+  g.tiles = (int32_t)(((int64_t)g.P * g.Q + kCfThreads - 1) / kCfThreads);
+  const int64_t blocks = (int64_t)g.N * g.tiles;
+  if ((int64_t)g.P * g.Q >= (1ll << 30) || blocks >= (1ll << 23))
+    return 0;
+  g.y_dt = d->y.dtype, g.o_dt = d->out.dtype;
+  g.epi = epi;
+  *handled = true;
+  fhip_note_kernel(ctx, "conv_few fprop channels=%d", kt * 16);
+  const dim3 grid((unsigned)blocks, (unsigned)((g.K + kt * 16 - 1) / (kt * 16)));
+  cf_by_type(d->x.dtype, [&](auto t) {
+    typedef decltype(t) T;
+    auto kernel = kt == 4   ? conv_few_fprop_kernel<T, 4>
+                  : kt == 2 ? conv_few_fprop_kernel<T, 2>
+                            : conv_few_fprop_kernel<T, 1>;
+    hipLaunchKernelGGL(kernel, grid, dim3(kCfThreads), lds, ctx->stream, g, (const T *)x,
+                       (const T *)w, out);
+  });
+  FHIP_HIP_CHECK(ctx, hipGetLastError());
+  return 0;
+}
+
+int fhip_few_conv_wgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy, const void *x,
+                        void *dw, bool *handled) {
+  *handled = false;
+  CfArgs g{};
+  if (!cf_args(d, d->y, g) || !cf_planes(g) || d->y.dtype != d->x.dtype)
+    return 0;
+  const int kt = g.K > 32 ? 4 : g.K > 16 ? 2 : 1;
+  const int tiles_j = (g.J + 15) / 16;
+  const int jt = tiles_j <= 2 ? 2 : tiles_j <= 3 ? 3 : tiles_j <= 5 ? 5 : 7;
+  // bands of about 256 pixels, of equal height
+  int band = 256 / g.Q;
+  band = band < 1 ? 1 : band < g.P ? band : g.P;
+  g.tiles = (g.P + band - 1) / band;
+  g.band = (g.P + g.tiles - 1) / g.tiles;
+  g.tiles = (g.P + g.band - 1) / g.band;
+  g.q_magic = cf_magic(g.Q);
+  size_t lds = 0;
+  const int64_t slots = ((int64_t)g.band * g.Q + 15) / 16 * 16;
+  if (slots >= (1 << 14) || !cf_stage(g, g.band, slots, &lds))
+    return 0;
+  const size_t meet = (size_t)2 * kt * jt * 256 * sizeof(float);
+  lds = lds < meet ? meet : lds;
+  const int64_t items = (int64_t)g.N * g.tiles;
+  const int kblocks = (g.K + kt * 16 - 1) / (kt * 16);
+  const int64_t frags = (int64_t)kblocks * kt * jt * 256;
+  if (items >= (1ll << 31) || kblocks > 65535)
+    return 0;
+  // two workgroups per compute unit, no more than 8 MB of partial sums
+  const int64_t cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+  int64_t runs = 2 * cus / kblocks, most = (8ll << 20) / (frags * 4);
+  runs = runs < most ? runs : most;
+  runs = runs < items ? runs : items;
+  runs = runs < 1 ? 1 : runs;
+  void *scratch = nullptr;
+  if (fhip_ctx_scratch(ctx, (size_t)(runs * frags) * sizeof(float), &scratch) != 0)
+    return 1;
+  *handled = true;
+  fhip_note_kernel(ctx, "conv_few wgrad tiles=%dx%d", kt, jt);
+  const dim3 grid((unsigned)runs, (unsigned)kblocks);
+  cf_by_type(d->x.dtype, [&](auto t) {
+    typedef decltype(t) T;
+    auto with = [&](auto kk) {
+      constexpr int KT = decltype(kk)::value;
+      auto kernel = jt == 2   ? conv_few_wgrad_kernel<T, KT, 2>
+                    : jt == 3 ? conv_few_wgrad_kernel<T, KT, 3>
+                    : jt == 5 ? conv_few_wgrad_kernel<T, KT, 5>
+                              : conv_few_wgrad_kernel<T, KT, 7>;
+      hipLaunchKernelGGL(kernel, grid, dim3(kCfThreads), lds, ctx->stream, g, (const T *)dy,
+                         (const T *)x, (float *)scratch);
+    };
+    if (kt == 4)
+      with(std::integral_constant<int, 4>{});
+    else if (kt == 2)
+      with(std::integral_constant<int, 2>{});
+    else
+      with(std::integral_constant<int, 1>{});
+  });
+  hipLaunchKernelGGL(conv_few_wgrad_sum_kernel, dim3((unsigned)(frags / 16)), dim3(256), 0,
+                     ctx->stream, g, (const float *)scratch, dw, (int)d->w.dtype, kt, jt, frags,
+                     (int)runs);
+  FHIP_HIP_CHECK(ctx, hipGetLastError());
+  return 0;
+}
+
+int fhip_few_conv_dgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy, const void *w,
+                        void *dx, bool *handled) {
+  *handled = false;
+  CfArgs g{};
+  if (!cf_args(d, d->y, g) || d->y.dtype != d->x.dtype)
+    return 0;
+  if (g.C > 4 || (g.S != 3 && g.S != 5) || g.str_h != 1 || g.str_w != 1 || g.dil_h != 1 ||
+      g.dil_w != 1 || (g.Q > 1 && g.ys[3] != 1) || g.W > 256)
+    return 0;
+  g.quads = (g.W + 3) / 4;
+  // (a multiple of the rows per lane, of equal height)
+  const int pairs = (g.H + kCfRows - 1) / kCfRows, most = 64 / g.quads;
+  g.tiles = (pairs + most - 1) / most;
+  g.band = (pairs + g.tiles - 1) / g.tiles * kCfRows;
+  const int span = (g.S + 6) & ~3, pitch = 4 * g.quads + span - 4, rows = g.band + g.R - 1;
+  const int64_t filter = (int64_t)g.K * g.R * ((g.S * g.C + 3) & ~3);
+  const int64_t blocks = (int64_t)g.N * g.tiles;
+  // a quarter of the output channels per wavefront, an eighth where that leaves
+  // fewer than two wavefronts per SIMD
+  const int64_t cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+  const int waves = blocks * 4 < 8 * cus ? 8 : 4;
+  int64_t floats = filter + (int64_t)waves * rows * pitch;
+  const int64_t meet = (int64_t)waves * kCfRows * 256 * g.C;
+  floats = floats < meet ? meet : floats;
+  if ((int64_t)rows * pitch > 64 * kCfStage || floats * 4 > kCfLds || blocks >= (1ll << 23))
+    return 0;
+  g.lw_magic = cf_magic(pitch);
+  *handled = true;
+  fhip_note_kernel(ctx, "conv_few dgrad channels=%d", g.C);
+  cf_by_type(d->x.dtype, [&](auto t) {
+    typedef decltype(t) T;
+    auto with = [&](auto cc) {
+      constexpr int C = decltype(cc)::value;
+      auto kernel = g.S == 3 ? conv_few_dgrad_kernel<T, C, 3> : conv_few_dgrad_kernel<T, C, 5>;
+      hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(waves * 64), (size_t)floats * 4,
+                         ctx->stream, g, (const T *)dy, (const T *)w, (T *)dx);
+    };
+    if (g.C == 1)
+      with(std::integral_constant<int, 1>{});
+    else if (g.C == 2)
+      with(std::integral_constant<int, 2>{});
+    else if (g.C == 3)
+      with(std::integral_constant<int, 3>{});
+    else
+      with(std::integral_constant<int, 4>{});
+  });
+  FHIP_HIP_CHECK(ctx, hipGetLastError());
+  return 0;
+}

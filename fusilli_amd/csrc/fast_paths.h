@@ -95,6 +95,15 @@ int fhip_direct_conv_dgrad(fhip_ctx *ctx, const fhip_conv_desc *d,
 int fhip_direct_conv_wgrad(fhip_ctx *ctx, const fhip_conv_desc *d,
                            const void *dy, const void *x, void *dw);
 
+// The same convolutions over few input channels (conv_few.hip), tried by the entry
+// points above: `handled` false where they do not take the descriptor.
+int fhip_few_conv_fprop(fhip_ctx *ctx, const fhip_conv_desc *d, const void *x,
+                        const void *w, const DevEpilogue &epi, void *out, bool *handled);
+int fhip_few_conv_dgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy,
+                        const void *w, void *dx, bool *handled);
+int fhip_few_conv_wgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy,
+                        const void *x, void *dw, bool *handled);
+
 bool fhip_fast_sdpa_applicable(const fhip_sdpa_desc *d);
 int fhip_fast_sdpa(fhip_ctx *ctx, const fhip_sdpa_desc *d, const void *q,
                    const void *k, const void *v, const void *mask, void *o);

@@ -1,0 +1,61 @@
+"""Convolutions over few input channels, channels-first (conv_few.hip), through the C
+ABI vs the oracle: forward with bias and ReLU, data gradient, weight gradient."""
+import numpy as np
+import pytest
+
+from fusilli_amd import capi
+from oracle import oracle
+from helpers import HT, assert_close, rand
+from test_generic_ops_gpu import run_conv, run_conv_dgrad, run_conv_wgrad
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # the reference benchmark's shape (reduced batch): tiles of 256 pixels, the last short
+    dict(x=[3, 3, 32, 32], w=[32, 3, 3, 3], pad=[0, 0], s=[1, 1], d=[1, 1]),
+    dict(x=[2, 1, 57, 57], w=[64, 1, 5, 5], pad=[2, 2], s=[1, 1], d=[1, 1]),
+    # 100 pairs; rows of 17 (no multiple of 4 or 16)
+    dict(x=[2, 4, 16, 17], w=[16, 4, 5, 5], pad=[2, 2], s=[1, 1], d=[1, 1]),
+    # fewest output channels, fewer pixels than one wavefront's
+    dict(x=[1, 2, 5, 4], w=[8, 2, 3, 3], pad=[1, 1], s=[1, 1], d=[1, 1]),
+    # two blocks of output channels, stride, dilation (data gradient: direct kernel)
+    dict(x=[2, 3, 20, 33], w=[70, 3, 3, 5], pad=[1, 0], s=[2, 1], d=[1, 2]),
+    # widest rows of the data gradient; single output rows per band
+    dict(x=[1, 3, 5, 252], w=[24, 3, 3, 3], pad=[1, 1], s=[1, 1], d=[1, 1]),
+    # padding beyond the filter, narrow image, many rows
+    dict(x=[1, 1, 150, 3], w=[9, 1, 2, 3], pad=[0, 4], s=[1, 1], d=[1, 1]),
+    # most pairs (112)
+    dict(x=[1, 7, 9, 9], w=[20, 7, 4, 4], pad=[1, 2], s=[1, 1], d=[1, 1]),
+]
+
+
+@pytest.mark.parametrize("case", CASES)
+@pytest.mark.parametrize("dtype", [capi.FLOAT, capi.BFLOAT16, capi.HALF])
+def test_conv_few_channels_vs_oracle(ctx, case, dtype):
+    geom = (case["pad"], case["s"], case["d"])
+    yd = oracle.conv_output_dims(case["x"], case["w"], *geom)
+    x = HT.from_logical(rand(51, 0, case["x"]), dtype)
+    w = HT.from_logical(rand(51, 1, case["w"], std=0.2), dtype)
+    dy = HT.from_logical(rand(51, 2, yd), dtype)
+    bias = HT.from_logical(rand(51, 3, [1, case["w"][0], 1, 1]), dtype)
+    epi = [capi.epilogue_op(capi.PW["ADD"], capi.FLOAT, operand=bias.desc()),
+           capi.epilogue_op(capi.PW["RELU_FWD"], dtype)]
+    y = run_conv(ctx, x, w, *geom, dtype, epilogue=epi, epi_tensors=[bias])
+    assert ctx.last_kernel().startswith("conv_few fprop"), ctx.last_kernel()
+    plain = oracle.conv_fprop(x.logical(), w.logical(), *geom)
+    assert_close(y.logical(), np.maximum(plain + bias.logical(), 0), dtype, f"fprop {case}")
+    # an operand of Y's own size is not one value per channel
+    res = HT.from_logical(rand(51, 4, yd), dtype)
+    y = run_conv(ctx, x, w, *geom, dtype, epi_tensors=[res],
+                 epilogue=[capi.epilogue_op(capi.PW["ADD"], dtype, operand=res.desc())])
+    assert ctx.last_kernel().startswith("conv_direct"), ctx.last_kernel()
+    assert_close(y.logical(), plain + res.logical(), dtype, f"fprop + residual {case}")
+    dx = run_conv_dgrad(ctx, dy, w, case["x"], *geom, dtype, False, tuned=None)
+    few = case["x"][1] <= 4 and case["w"][3] in (3, 5) and case["s"] == case["d"] == [1, 1]
+    assert ctx.last_kernel().startswith("conv_few dgrad" if few else "conv_direct"), ctx.last_kernel()
+    assert_close(dx.logical(), oracle.conv_dgrad(dy.logical(), w.logical(), case["x"], *geom),
+                 dtype, f"dgrad {case}")
+    dw = run_conv_wgrad(ctx, dy, x, case["w"], *geom, dtype, False, tuned=None)
+    assert ctx.last_kernel().startswith("conv_few wgrad"), ctx.last_kernel()
+    assert_close(dw.logical(), oracle.conv_wgrad(dy.logical(), x.logical(), case["w"], *geom),
+                 dtype, f"wgrad {case}")
