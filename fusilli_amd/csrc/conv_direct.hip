@@ -983,7 +983,10 @@ int fhip_direct_conv_dgrad(fhip_ctx *ctx, const fhip_conv_desc *d,
 int fhip_direct_conv_wgrad(fhip_ctx *ctx, const fhip_conv_desc *d,
                            const void *dy, const void *x, void *dw) {
   bool handled = false;
-  const int rc = fhip_few_conv_wgrad(ctx, d, dy, x, dw, &handled);
+  int rc = fhip_few_conv_wgrad(ctx, d, dy, x, dw, &handled);
+  if (handled || rc != 0)
+    return rc;
+  rc = fhip_gather_conv_wgrad(ctx, d, dy, x, dw, &handled);
   if (handled || rc != 0)
     return rc;
   fhip_note_kernel(ctx, "conv_direct_wgrad");

@@ -1,41 +1,287 @@
-// Convolution weight gradient on the MFMA GEMM kernel.
+// Convolution weight gradient for channels-last 16-bit tensors, any filter, stride,
+// padding and dilation (3 x 3 filters at unit stride have conv_wgrad_direct.hip).
 //
-//   DW[k, r, s, c] = sum over n, p, q of DY[n, p, q, k] * X[n, p + r*dil - pad_h, q + s - pad_w, c]
+//   DW[k, (r, s, c)] = sum over output pixels m of
+//                      DY[m, k] * X[pixel of m shifted by (r, s), c]
 //
-// (channels-last tensors, one group, unit dilation along W; written here for
-// unit strides, equal strides in both dims work the same way, see the plan).
-// Both operands are first copied into zero-padded grids of the same geometry,
-// [N][rows = H + 2 pad_h][pitch >= W + 2 pad_w] pixels with pitch a multiple of
-// 64: X shifted by the padding, DY in the top-left corner.  With m the flat
-// pixel index of that grid, tap (r, s) of X is pixel m + r * dil * pitch + s,
-// whatever m: image borders need no case distinction because DY is zero
-// wherever the shifted pixel would leave the image.  For one filter row r the
-// S taps of a pixel are S * C consecutive elements, so
-//   partial[r][n][k][s * C + c] = sum_m DYp[n][m][k] * Xp[n][m + r * dil * pitch][s * C + c]
-// is one batched GEMM per filter row, all rows in one launch (A = DYp, M-contiguous; B = Xp with
-// overlapping rows of S * C elements, row stride C; reduction over the 64-pixel
-// K slices of an image, or of an equal share of it; batch = image x share),
-// and DW is the sum of the partial results over the batch.
+// A matrix product of K rows and J = R * S * C columns whose long reduction runs along
+// both tensors' slow dimension.  Bound by LDS reads (eight transposing reads per four
+// 32 x 32 x 16 MFMAs of a wavefront's 64 x 64 block) and, with few outputs, by the
+// partial sums.  No operand is copied or padded in memory: C is a multiple of 8, so
+// every 16-byte run of a column block lies inside one tap, and a lane fetches it from
+// the shifted pixel, the buffer descriptor's range check giving zeros outside the
+// image, the pixel range and the channel counts.  Where a pixel lies is decided once
+// per chunk of pixels and kept in LDS; loads run three steps of 32 pixels ahead.
+// Workgroups take a tile of outputs and a run of pixels; a second kernel adds the
+// runs' sums in a fixed order.
+//
+// Before, both operands were copied into zero-padded grids for a batched GEMM of 128
+// columns at least: N62 256 -> 48, 39 x 39, 3 x 3, bf16: 248 us -> 76.5; N32 112 ->
+// 384, 26 x 26, f16: 138 -> 40.6; N16 48 -> 48, 48 x 32, f16: 36.7 -> 17.4.
 //
 // Reference semantics: node/conv_node.h:255-426 (ConvWGradNode),
 // aten.convolution_backward, weight gradient.
 #include "common.h"
 #include "fast_paths.h"
 
+#include <type_traits>
+
 namespace {
 
-struct WgradPlan {
-  bool ok = false;
-  int64_t N = 0, H = 0, W = 0, C = 0, K = 0, P = 0, Q = 0, R = 0, S = 0;
-  int64_t Kp = 0; // channels of the padded DY grid: K, or 128 for narrower outputs
-  int64_t pad_h = 0, pad_w = 0, dil_h = 1;
-  int64_t rows = 0, pitch = 0, pix = 0; // padded grid
-  int64_t split = 1; // GEMM batches per image (more workgroups, shorter K)
-  int64_t str = 1;   // convolution stride (same in both dims)
-  int64_t rows_y = 0, pix_y = 0; // DY's grid: rows / str rows of the same pitch
-  size_t xp_bytes = 0, dyp_bytes = 0, part_bytes = 0;
-  fhip_matmul_desc mm; // one filter row
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+#define WG_AS3 __attribute__((address_space(3)))
+
+constexpr int kWgThreads = 256;
+constexpr int kWgStep = 32;    // pixels per step
+constexpr int kWgChunk = 2048; // pixels whose places are in LDS at once
+
+struct WgArgs {
+  const char *x, *dy;
+  float *part; // [run][K][J]
+  int32_t H, W, C, K, P, Q, S, J;
+  int32_t pad_h, pad_w, str_h, str_w, dil_h, dil_w;
+  int32_t jtiles, tiles;
+  int64_t pixels, run; // all, per workgroup (a multiple of the step)
+  int64_t image_bytes;
+  uint32_t chunk_images; // images that a chunk may touch
 };
+
+template <bool BF16> __device__ __forceinline__ f32x16 wg_mfma(const s16x8 &a, const s16x8 &b, const f32x16 &c) {
+  if constexpr (BF16)
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
+                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
+                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+}
+
+// Byte of 16-byte run `chunk` of pixel slot `px` in a stage with rows of ROW bytes.  The
+// 64-byte groups of a row are permuted by the pixel, so that the 8 pixels of a
+// transposing read (64 bytes each) meet every bank twice.
+template <int ROW> __device__ __forceinline__ int wg_swizzle(int px, int group) {
+  if constexpr (ROW >= 256)
+    return group ^ (px & 3);
+  else if constexpr (ROW == 128)
+    return group ^ ((px >> 1) & 1);
+  else
+    return group;
+}
+template <int ROW> __device__ __forceinline__ int wg_place(int px, int chunk) {
+  return px * ROW + (wg_swizzle<ROW>(px, chunk >> 2) << 6) + ((chunk & 3) << 4);
+}
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t wg_rsrc(const char *base, uint32_t bytes) {
+  const uint64_t b = (uint64_t)base;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)b);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
+  return __builtin_amdgcn_make_buffer_rsrc((void *)(((uint64_t)hi << 32) | lo), 0,
+                                           (int)__builtin_amdgcn_readfirstlane(bytes), 0x00020000);
+}
+
+// WK x WJ wavefronts of MT x 2 tiles of 32 x 32 outputs.
+template <bool BF16, int WK, int WJ, int MT>
+__global__ __launch_bounds__(kWgThreads) __attribute__((amdgpu_waves_per_eu(2, 4))) void
+conv_wgrad_gather_kernel(WgArgs g) {
+  constexpr int TK = 32 * MT * WK, TJ = 64 * WJ;
+  constexpr int ROWA = TK * 2, ROWB = TJ * 2;
+  constexpr int CA = TK / 8, CB = TJ / 8; // 16-byte runs per pixel
+  constexpr int NA = (kWgStep * CA + kWgThreads - 1) / kWgThreads, NB = kWgStep * CB / kWgThreads;
+  constexpr int kStage = kWgStep * (ROWA + ROWB);
+  __shared__ __attribute__((aligned(16))) char stage[2 * kStage];
+  __shared__ int2 place[kWgChunk];
+  const int tid = threadIdx.x, l = tid & 63, wave = tid >> 6;
+  const int tile = blockIdx.x % g.tiles;
+  const int64_t m0 = (int64_t)(blockIdx.x / g.tiles) * g.run;
+  const int64_t m1 = m0 + g.run < g.pixels ? m0 + g.run : g.pixels;
+  const int k0 = tile / g.jtiles * TK, j0 = tile % g.jtiles * TJ;
+  // this thread's run of columns: its tap's shift and bytes behind a pixel's place
+  int shift_h, shift_w, jbytes;
+  {
+    const int j = j0 + tid % CB * 8;
+    const int tap = j / g.C, c = j - tap * g.C;
+    const int r = tap / g.S, s = tap - r * g.S;
+    shift_h = j < g.J ? r * g.dil_h : 1 << 20; // (beyond every image)
+    shift_w = s * g.dil_w;
+    jbytes = ((r * g.dil_h * g.W + s * g.dil_w) * g.C + c) * 2;
+  }
+  const int ka = k0 + tid % CA * 8;
+  const bool a_in = ka < g.K && tid / CA < kWgStep;
+  f32x16 acc[MT][2];
+#pragma unroll
+  for (int a = 0; a < MT; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        acc[a][b][i] = 0.f;
+  // transposing reads: 16 lanes address 4 pixels x 16 channels, lane i receives
+  // channel i of the 4 pixels; lanes 32 .. 63 hold the upper 8 pixels of a step of 16
+  const int wk = wave / WJ, wj = wave % WJ;
+  const int lpx = (l >> 5) * 8 + ((l & 15) >> 2), lin = ((l >> 4) & 1) * 32 + (l & 3) * 8;
+  int ra[MT], rb[2];
+#pragma unroll
+  for (int a = 0; a < MT; ++a)
+    ra[a] = lpx * ROWA + (wg_swizzle<ROWA>(lpx, wk * MT + a) << 6) + lin;
+#pragma unroll
+  for (int b = 0; b < 2; ++b)
+    rb[b] = kWgStep * ROWA + lpx * ROWB + (wg_swizzle<ROWB>(lpx, wj * 2 + b) << 6) + lin;
+
+  for (int64_t c0 = m0; c0 < m1; c0 += kWgChunk) {
+    const int count = (int)(m1 - c0 < kWgChunk ? m1 - c0 : kWgChunk);
+    const int steps = (count + kWgStep - 1) / kWgStep;
+    const int pq = g.P * g.Q;
+    const int64_t first_image = c0 / pq;
+    const int in_image = (int)(c0 - first_image * pq);
+    __syncthreads(); // the last chunk's places and stages have been read
+    for (int i = tid; i < steps * kWgStep; i += kWgThreads) {
+      const uint32_t e = (uint32_t)(in_image + i);
+      const uint32_t n = e / (uint32_t)pq, rest = e - n * (uint32_t)pq;
+      const int p = (int)(rest / (uint32_t)g.Q), q = (int)(rest - (uint32_t)p * (uint32_t)g.Q);
+      const int h = p * g.str_h - g.pad_h, w = q * g.str_w - g.pad_w;
+      int2 v;
+      v.x = (int)(n * (uint32_t)g.image_bytes) + (h * g.W + w) * g.C * 2;
+      v.y = i < count ? (int)((uint32_t)(h & 0xffff) | ((uint32_t)w << 16)) : 0x8000; // row -32768
+      place[i] = v;
+    }
+    const int64_t left = (g.pixels + pq - 1) / pq - first_image;
+    const int64_t images = left < g.chunk_images ? left : g.chunk_images;
+    const __amdgpu_buffer_rsrc_t rx =
+        wg_rsrc(g.x + first_image * g.image_bytes, (uint32_t)(images * g.image_bytes));
+    const __amdgpu_buffer_rsrc_t ry = wg_rsrc(g.dy + c0 * g.K * 2, (uint32_t)(count * g.K * 2));
+    __syncthreads();
+    u32x4 va[3][NA], vb[3][NB];
+    auto fetch = [&](auto set, int t) {
+      constexpr int B = decltype(set)::value;
+      if (t >= steps)
+        return;
+#pragma unroll
+      for (int i = 0; i < NA; ++i) {
+        const int px = t * kWgStep + tid / CA + i * (kWgThreads / CA);
+        va[B][i] = __builtin_amdgcn_raw_buffer_load_b128(ry, a_in ? (px * g.K + ka) * 2 : (int)0x80000000, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        const int2 v = place[t * kWgStep + tid / CB + i * (kWgThreads / CB)];
+        const int h = (int)(short)(v.y & 0xffff) + shift_h, w = (v.y >> 16) + shift_w;
+        const bool in = (unsigned)h < (unsigned)g.H && (unsigned)w < (unsigned)g.W;
+        vb[B][i] = __builtin_amdgcn_raw_buffer_load_b128(rx, in ? v.x + jbytes : (int)0x80000000, 0, 0);
+      }
+    };
+    auto step = [&](auto set, int t) {
+      constexpr int B = decltype(set)::value;
+      char *to = stage + (t & 1) * kStage;
+#pragma unroll
+      for (int i = 0; i < NA; ++i)
+        if (NA * kWgThreads == kWgStep * CA || tid < kWgStep * CA)
+          *(u32x4 *)(to + wg_place<ROWA>(tid / CA + i * (kWgThreads / CA), tid % CA)) = va[B][i];
+#pragma unroll
+      for (int i = 0; i < NB; ++i)
+        *(u32x4 *)(to + kWgStep * ROWA + wg_place<ROWB>(tid / CB + i * (kWgThreads / CB), tid % CB)) = vb[B][i];
+      fetch(set, t + 3);
+      // (one barrier per step: a stage is written again two steps later, behind the
+      // barrier that its readers reach after reading)
+      __syncthreads();
+      const WG_AS3 char *from = (const WG_AS3 char *)to;
+#pragma unroll
+      for (int ks = 0; ks < kWgStep / 16; ++ks) {
+        s16x8 fa[MT], fb[2];
+        auto read = [&](int at, int row) {
+          const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((WG_AS3 s16x4 *)(from + at + ks * 16 * row));
+          const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((WG_AS3 s16x4 *)(from + at + (ks * 16 + 4) * row));
+          return s16x8{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+        };
+#pragma unroll
+        for (int a = 0; a < MT; ++a)
+          fa[a] = read(ra[a], ROWA);
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+          fb[b] = read(rb[b], ROWB);
+#pragma unroll
+        for (int a = 0; a < MT; ++a)
+#pragma unroll
+          for (int b = 0; b < 2; ++b)
+            acc[a][b] = wg_mfma<BF16>(fa[a], fb[b], acc[a][b]);
+      }
+    };
+    using S0 = std::integral_constant<int, 0>;
+    using S1 = std::integral_constant<int, 1>;
+    using S2 = std::integral_constant<int, 2>;
+    fetch(S0{}, 0);
+    fetch(S1{}, 1);
+    fetch(S2{}, 2);
+    for (int t = 0; t < steps; t += 3) {
+      step(S0{}, t);
+      if (t + 1 < steps)
+        step(S1{}, t + 1);
+      if (t + 2 < steps)
+        step(S2{}, t + 2);
+    }
+  }
+  // value i of a lane: row 8 * (i / 4) + 4 * (l / 32) + i % 4, column l % 32 of its tile
+  float *out = g.part + (int64_t)(blockIdx.x / g.tiles) * g.K * g.J;
+#pragma unroll
+  for (int a = 0; a < MT; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const int j = j0 + (wj * 2 + b) * 32 + (l & 31);
+      if (j >= g.J)
+        continue;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int k = k0 + (wk * MT + a) * 32 + 8 * (i >> 2) + 4 * (l >> 5) + (i & 3);
+        if (k < g.K)
+          out[(int64_t)k * g.J + j] = acc[a][b][i];
+      }
+    }
+}
+
+struct WgradSumArgs {
+  int32_t runs, J, S, C;
+  int64_t total;          // K * J
+  int64_t sk, sc, sr, ss; // element strides of DW [K, C, R, S]
+  int32_t dt;
+};
+
+// DW = sum of the runs: a workgroup adds SLICES shares of the runs of 1024 / SLICES
+// consecutive values (J is a multiple of 8), the shares in order.
+template <int SLICES>
+__global__ __launch_bounds__(256) void conv_wgrad_sum_kernel(WgradSumArgs a, const float *part,
+                                                             void *dw) {
+  constexpr int kLanes = 256 / SLICES;
+  __shared__ f32x4 meet[SLICES][kLanes];
+  const int o = threadIdx.x % kLanes, z = threadIdx.x / kLanes;
+  const int64_t e = ((int64_t)blockIdx.x * kLanes + o) * 4;
+  f32x4 s{0, 0, 0, 0};
+  if (e < a.total) {
+#pragma unroll 8
+    for (int r = z; r < a.runs; r += SLICES)
+      s += *(const f32x4 *)(part + r * a.total + e);
+  }
+  if constexpr (SLICES > 1) {
+    meet[z][o] = s;
+    __syncthreads();
+    if (z != 0)
+      return;
+#pragma unroll
+    for (int i = 1; i < SLICES; ++i)
+      s += meet[i][o];
+  }
+  if (e >= a.total)
+    return;
+  const int64_t k = e / a.J;
+  const int j = (int)(e - k * a.J), tap = j / a.C, c = j - tap * a.C;
+  const int r = tap / a.S;
+  const int64_t at = k * a.sk + r * a.sr + (tap - r * a.S) * a.ss + c * a.sc;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    fhip_store<float>(dw, a.dt, at + i * a.sc, s[i]);
+}
 
 bool wg_channels_last(const fhip_tensor_desc &t) {
   int64_t expect = 1;
@@ -53,151 +299,137 @@ bool wg_channels_last(const fhip_tensor_desc &t) {
   return true;
 }
 
-size_t wg_align(size_t b) { return (b + 255) / 256 * 256; }
+struct WgradPlan {
+  bool ok = false;
+  WgArgs a{};
+  int tk = 0, tj = 0;
+  int64_t runs = 0;
+  size_t part_bytes = 0;
+};
 
 WgradPlan make_wgrad_plan(const fhip_conv_desc *d) {
   WgradPlan p;
   if (d->spatial_rank != 2)
     return p;
-  const int dt = d->x.dtype;
-  if (dt != FHIP_BFLOAT16 && dt != FHIP_HALF)
+  const int dt = d->x.dtype, wdt = d->w.dtype;
+  if ((dt != FHIP_BFLOAT16 && dt != FHIP_HALF) || d->y.dtype != dt)
     return p;
-  if (d->y.dtype != dt)
-    return p;
-  const int wdt = d->w.dtype;
   if (wdt != FHIP_BFLOAT16 && wdt != FHIP_HALF && wdt != FHIP_FLOAT)
     return p;
   if (d->w.dim[1] != d->x.dim[1]) // groups
     return p;
-  if (d->stride[0] != d->stride[1] || d->dilation[1] != 1)
-    return p;
-  p.str = d->stride[0];
   if (!wg_channels_last(d->x) || !wg_channels_last(d->y))
     return p;
-  p.N = d->x.dim[0], p.C = d->x.dim[1], p.H = d->x.dim[2], p.W = d->x.dim[3];
-  p.K = d->w.dim[0], p.R = d->w.dim[2], p.S = d->w.dim[3];
-  // the padding copies move whole 16-byte chunks of a pixel's channels
-  if (p.C % 8 != 0 || p.K % 8 != 0)
+  const int64_t N = d->x.dim[0], C = d->x.dim[1], H = d->x.dim[2], W = d->x.dim[3];
+  const int64_t K = d->w.dim[0], R = d->w.dim[2], S = d->w.dim[3];
+  const int64_t P = d->y.dim[2], Q = d->y.dim[3];
+  if (C % 8 != 0 || K % 8 != 0) // whole 16-byte runs of a pixel's channels
     return p;
-  // the GEMM's tiles want at least 128 rows: narrower gradients are zero-padded
-  p.Kp = p.K < 128 ? 128 : p.K;
-  p.P = d->y.dim[2], p.Q = d->y.dim[3];
-  p.pad_h = d->padding[0], p.pad_w = d->padding[1], p.dil_h = d->dilation[0];
-  // Strides: output pixel (p, q) reads input pixel (p * str + r * dil, q * str
-  // + s); with DY on a grid of the SAME pitch and rows / str rows, DY pixel m
-  // pairs with X pixel str * m + shift: B's row stride becomes str * C.
-  p.rows = (p.H + 2 * p.pad_h + p.str - 1) / p.str * p.str;
-  p.pitch = (p.W + 2 * p.pad_w + 63) / 64 * 64;
-  p.pix = p.rows * p.pitch;
-  p.rows_y = p.rows / p.str;
-  p.pix_y = p.rows_y * p.pitch;
-  if (p.P > p.rows_y || (p.Q - 1) * p.str + p.S > p.pitch)
+  // places of pixels are 16-bit signed pairs, -32768 marks none
+  for (int i = 0; i < 2; ++i)
+    if (d->x.dim[2 + i] >= 32768 || d->padding[i] >= 16384 || d->stride[i] >= 16384 ||
+        d->dilation[i] >= 16384 || d->dilation[i] * (d->w.dim[2 + i] - 1) >= 16384 ||
+        (d->y.dim[2 + i] - 1) * d->stride[i] - d->padding[i] >= 32768)
+      return p;
+  const int64_t J = R * S * C, pixels = N * P * Q, image = H * W * C * 2;
+  const int64_t chunk_images = (kWgChunk + P * Q - 2) / (P * Q) + 1;
+  // 32-bit offsets inside a chunk, taps in the padding included (they wrap)
+  if (P * Q >= (1ll << 30) || K >= (1 << 18) || J >= (1ll << 30) || pixels >= (1ll << 40) ||
+      (chunk_images + 1) * image >= (1ll << 31))
     return p;
-  // guard behind the last image: the furthest tap of the last pixel
-  const int64_t guard = (p.R - 1) * p.dil_h * p.pitch * p.C + p.S * p.C;
-  p.xp_bytes = wg_align((size_t)(p.N * p.pix * p.C + guard) * 2);
-  p.dyp_bytes = wg_align((size_t)(p.N * p.pix_y * p.Kp) * 2);
-  // An image's pixels are cut into `split` equal runs of whole 64-pixel
-  // slices, each a batch entry of its own: the largest cut that keeps at
-  // least 8 slices per run and at most ~1024 workgroups per launch.
-  {
-    const int64_t slices = p.pix_y / 64;
-    const int64_t col_tiles = (p.S * p.C + 127) / 128, row_tiles = (p.K + 127) / 128;
-    for (int64_t f = 1; f <= slices; ++f)
-      if (slices % f == 0 && slices / f >= 8 &&
-          p.N * f * col_tiles * row_tiles <= 1024)
-        p.split = f;
+  WgArgs &a = p.a;
+  a.H = (int32_t)H, a.W = (int32_t)W, a.C = (int32_t)C, a.K = (int32_t)K;
+  a.P = (int32_t)P, a.Q = (int32_t)Q, a.S = (int32_t)S, a.J = (int32_t)J;
+  a.pad_h = (int32_t)d->padding[0], a.pad_w = (int32_t)d->padding[1];
+  a.str_h = (int32_t)d->stride[0], a.str_w = (int32_t)d->stride[1];
+  a.dil_h = (int32_t)d->dilation[0], a.dil_w = (int32_t)d->dilation[1];
+  a.pixels = pixels, a.image_bytes = image, a.chunk_images = (uint32_t)chunk_images;
+  // the tile with the least padding; equal ones: the squarest (fewest bytes per product)
+  static const int shapes[4][2] = {{128, 128}, {64, 256}, {256, 64}, {32, 256}};
+  int64_t best = 0;
+  for (const auto &s : shapes) {
+    const int64_t area = ((K + s[0] - 1) / s[0]) * ((J + s[1] - 1) / s[1]) * s[0] * s[1];
+    if (p.tk == 0 || area < best)
+      best = area, p.tk = s[0], p.tj = s[1];
   }
-  p.part_bytes = wg_align((size_t)(p.R * p.N * p.split * p.Kp * p.S * p.C) * 4);
-  if (p.xp_bytes >= (1ull << 32) || p.dyp_bytes >= (1ull << 32))
+  a.jtiles = (int32_t)((J + p.tj - 1) / p.tj);
+  const int64_t tiles = ((K + p.tk - 1) / p.tk) * a.jtiles;
+  if (tiles >= (1 << 20))
     return p;
-  fhip_matmul_desc &m = p.mm;
-  std::memset(&m, 0, sizeof(m));
-  auto set = [](fhip_tensor_desc &t, int dtype, int64_t d0, int64_t d1, int64_t d2,
-                int64_t s0, int64_t s1, int64_t s2) {
-    t.rank = 3;
-    t.dtype = dtype;
-    t.dim[0] = d0, t.dim[1] = d1, t.dim[2] = d2;
-    t.stride[0] = s0, t.stride[1] = s1, t.stride[2] = s2;
-  };
-  const int64_t nb = p.N * p.split, run = p.pix_y / p.split;
-  set(m.a, dt, nb, p.Kp, run, run * p.Kp, 1, p.Kp);
-  set(m.b, dt, nb, run, p.S * p.C, p.str * run * p.C, p.str * p.C, 1);
-  set(m.c, FHIP_FLOAT, nb, p.Kp, p.S * p.C, p.Kp * p.S * p.C, p.S * p.C, 1);
-  m.out = m.c;
-  m.out_dtype = FHIP_FLOAT;
-  if (!fhip_fast_matmul_applicable(&m))
-    return p;
-  p.ok = true;
+  a.tiles = (int32_t)tiles;
+  // runs of pixels: two workgroups per compute unit where each then has 16 steps, else
+  // one, of 4 steps at least (planned for 256 units whatever the device: the workspace
+  // size is answered without one)
+  const int64_t steps = (pixels + kWgStep - 1) / kWgStep;
+  int64_t runs = (steps * tiles >= 512 * 16 ? 512 : 256) / tiles;
+  runs = runs < steps / 4 ? runs : steps / 4;
+  runs = runs < 1 ? 1 : runs;
+  a.run = (steps + runs - 1) / runs * kWgStep;
+  p.runs = (pixels + a.run - 1) / a.run;
+  // (a line more than the sums: the size tells this plan from the 3 x 3 kernel's whole blocks)
+  p.part_bytes = (size_t)(p.runs * K * J) * sizeof(float) + 256;
+  p.ok = p.runs * tiles < (1ll << 23);
   return p;
 }
 
-struct PadArgs {
-  int64_t N, rows, pitch, ch;  // destination grid, channels per pixel
-  int64_t src_ch;              // channels per source pixel (<= ch: the rest is zero)
-  int64_t h, w;                // source extent
-  int64_t off_h, off_w;        // destination position of source pixel (0, 0)
-  int64_t total;               // 16-byte chunks of the destination
-};
-
-// dst[n][row][col][:] = src[n][row - off_h][col - off_w][:] inside the source,
-// zeros elsewhere; one 16-byte chunk (8 channels) per thread.
-__global__ void conv_pad_grid_kernel(PadArgs a, const uint4 *src, uint4 *dst) {
-  const int64_t lin = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (lin >= a.total)
-    return;
-  const int64_t cpp = a.ch / 8; // chunks per pixel
-  const int64_t chunk = lin % cpp;
-  int64_t pixel = lin / cpp;
-  const int64_t col = pixel % a.pitch;
-  pixel /= a.pitch;
-  const int64_t row = pixel % a.rows;
-  const int64_t n = pixel / a.rows;
-  const int64_t sr = row - a.off_h, sc = col - a.off_w;
-  uint4 v = make_uint4(0, 0, 0, 0);
-  const int64_t scpp = a.src_ch / 8;
-  if (n < a.N && sr >= 0 && sr < a.h && sc >= 0 && sc < a.w && chunk < scpp)
-    v = src[((n * a.h + sr) * a.w + sc) * scpp + chunk];
-  dst[lin] = v;
-}
-
-struct WgradSumArgs {
-  int64_t N, K, R, S, C;
-  int64_t Kp; // rows of a partial result (K, or 128 for narrower gradients)
-  int64_t sk, sc, sr, ss; // element strides of DW [K, C, R, S]
-  int32_t dt;
-};
-
-// DW[k][c][r][s] = sum over the N batch entries of partial[r][n][k][s * C + c]
-__global__ void conv_wgrad_sum_kernel(WgradSumArgs a, const float *part,
-                                      void *dw, int64_t total) {
-  const int64_t lin = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (lin >= total)
-    return;
-  const int64_t sc = a.S * a.C;
-  const int64_t j = lin % sc; // s * C + c
-  int64_t rem = lin / sc;
-  const int64_t k = rem % a.K;
-  const int64_t r = rem / a.K;
-  const float *src = part + (r * a.N * a.Kp + k) * sc + j;
-  float acc = 0.f;
-#pragma unroll 8 // independent loads: several in flight
-  for (int64_t n = 0; n < a.N; ++n)
-    acc += src[n * a.Kp * sc];
-  const int64_t s = j / a.C, c = j - s * a.C;
-  fhip_store<float>(dw, a.dt, k * a.sk + c * a.sc + r * a.sr + s * a.ss, acc);
+int wg_run(fhip_ctx *ctx, const fhip_conv_desc *d, const WgradPlan &p, const void *dy,
+           const void *x, void *dw, void *part) {
+  WgArgs a = p.a;
+  a.x = (const char *)x, a.dy = (const char *)dy, a.part = (float *)part;
+  auto go = [&](auto bf) {
+    constexpr bool B = decltype(bf)::value;
+    auto kernel = p.tk == 32    ? conv_wgrad_gather_kernel<B, 1, 4, 1>
+                  : p.tk == 64  ? conv_wgrad_gather_kernel<B, 1, 4, 2>
+                  : p.tk == 128 ? conv_wgrad_gather_kernel<B, 2, 2, 2>
+                                : conv_wgrad_gather_kernel<B, 4, 1, 2>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(p.runs * a.tiles)), dim3(kWgThreads), 0, ctx->stream, a);
+  };
+  if (d->x.dtype == FHIP_BFLOAT16)
+    go(std::true_type{});
+  else
+    go(std::false_type{});
+  FHIP_HIP_CHECK(ctx, hipGetLastError());
+  WgradSumArgs s;
+  s.runs = (int32_t)p.runs, s.J = a.J, s.S = a.S, s.C = a.C;
+  s.total = (int64_t)a.K * a.J;
+  s.sk = d->w.dim[0] == 1 ? 0 : d->w.stride[0];
+  s.sc = d->w.dim[1] == 1 ? 0 : d->w.stride[1];
+  s.sr = d->w.dim[2] == 1 ? 0 : d->w.stride[2];
+  s.ss = d->w.dim[3] == 1 ? 0 : d->w.stride[3];
+  s.dt = d->w.dtype;
+  auto sum = [&](auto zz) {
+    constexpr int Z = decltype(zz)::value;
+    const int64_t per = 1024 / Z;
+    hipLaunchKernelGGL(conv_wgrad_sum_kernel<Z>, dim3((unsigned)((s.total + per - 1) / per)), dim3(256),
+                       0, ctx->stream, s, (const float *)part, dw);
+  };
+  // (eight loads in flight per thread: more shares where there are more runs)
+  if (s.runs > 32)
+    sum(std::integral_constant<int, 16>{});
+  else if (s.runs > 8)
+    sum(std::integral_constant<int, 4>{});
+  else
+    sum(std::integral_constant<int, 1>{});
+  FHIP_HIP_CHECK(ctx, hipGetLastError());
+  fhip_note_kernel(ctx, "conv_wgrad_gather %dx%d runs=%d", p.tk, p.tj, (int)p.runs);
+  return 0;
 }
 
 } // namespace
 
+// Descriptors whose partial sums go to the caller's workspace; the others that the
+// kernel takes (fewer than 128 columns per filter row, unequal strides, dilation along
+// W) keep them in the context's scratch.
 bool fhip_fast_conv_wgrad_applicable(const fhip_conv_desc *d,
                                      size_t *workspace_bytes) {
   if (fhip_fast_conv_wgrad_direct_applicable(d, workspace_bytes))
     return true;
   const WgradPlan p = make_wgrad_plan(d);
+  const bool ok = p.ok && d->stride[0] == d->stride[1] && d->dilation[1] == 1 &&
+                  d->w.dim[3] * d->w.dim[1] >= 128;
   if (workspace_bytes)
-    *workspace_bytes = p.ok ? p.xp_bytes + p.dyp_bytes + p.part_bytes : 0;
-  return p.ok;
+    *workspace_bytes = ok ? p.part_bytes : 0;
+  return ok;
 }
 
 int fhip_fast_conv_wgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy,
@@ -209,40 +441,18 @@ int fhip_fast_conv_wgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy,
   FHIP_REQUIRE(ctx, ((uintptr_t)workspace & 255) == 0 && ((uintptr_t)x & 15) == 0 &&
                         ((uintptr_t)dy & 15) == 0,
                "conv wgrad: workspace must be 256-byte and tensors 16-byte aligned");
-  char *xp = (char *)workspace;
-  char *dyp = xp + p.xp_bytes;
-  float *part = (float *)(dyp + p.dyp_bytes);
-  // X into its padded grid (the guard behind the last image included: the
-  // grid is extended by whole zero images' worth of chunks up to the buffer's
-  // end), DY into the top-left corner of the same grid
-  PadArgs ax{p.N, p.rows, p.pitch, p.C, p.C, p.H, p.W, p.pad_h, p.pad_w,
-             (int64_t)(p.xp_bytes / 16)};
-  hipLaunchKernelGGL(conv_pad_grid_kernel, dim3((unsigned)((ax.total + 255) / 256)),
-                     dim3(256), 0, ctx->stream, ax, (const uint4 *)x, (uint4 *)xp);
-  PadArgs ay{p.N, p.rows_y, p.pitch, p.Kp, p.K, p.P, p.Q, 0, 0,
-             (int64_t)(p.N * p.pix_y * p.Kp * 2 / 16)};
-  hipLaunchKernelGGL(conv_pad_grid_kernel, dim3((unsigned)((ay.total + 255) / 256)),
-                     dim3(256), 0, ctx->stream, ay, (const uint4 *)dy, (uint4 *)dyp);
-  FHIP_HIP_CHECK(ctx, hipGetLastError());
-  DevEpilogue epi{};
-  // all filter rows in one launch: the outer batch dim steps B by one filter
-  // row of pixels and the output by one block of partial results
-  if (fhip_fast_matmul_outer(ctx, &p.mm, dyp, xp, epi, part, (int)p.R, 0,
-                             p.dil_h * p.pitch * p.C,
-                             p.N * p.split * p.Kp * p.S * p.C) != 0)
+  return wg_run(ctx, d, p, dy, x, dw, workspace);
+}
+
+int fhip_gather_conv_wgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy, const void *x,
+                           void *dw, bool *handled) {
+  *handled = false;
+  const WgradPlan p = make_wgrad_plan(d);
+  if (!p.ok || (((uintptr_t)x | (uintptr_t)dy) & 15) != 0)
+    return 0;
+  void *scratch = nullptr;
+  if (fhip_ctx_scratch(ctx, p.part_bytes, &scratch) != 0)
     return 1;
-  WgradSumArgs as;
-  as.N = p.N * p.split, as.K = p.K, as.R = p.R, as.S = p.S, as.C = p.C;
-  as.Kp = p.Kp;
-  as.sk = d->w.dim[0] == 1 ? 0 : d->w.stride[0];
-  as.sc = d->w.dim[1] == 1 ? 0 : d->w.stride[1];
-  as.sr = d->w.dim[2] == 1 ? 0 : d->w.stride[2];
-  as.ss = d->w.dim[3] == 1 ? 0 : d->w.stride[3];
-  as.dt = d->w.dtype;
-  const int64_t total = p.R * p.K * p.S * p.C;
-  hipLaunchKernelGGL(conv_wgrad_sum_kernel, dim3((unsigned)((total + 255) / 256)),
-                     dim3(256), 0, ctx->stream, as, part, dw, total);
-  FHIP_HIP_CHECK(ctx, hipGetLastError());
-  fhip_note_kernel(ctx, "conv_wgrad batched gemm");
-  return 0;
+  *handled = true;
+  return wg_run(ctx, d, p, dy, x, dw, scratch);
 }

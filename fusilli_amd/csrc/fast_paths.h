@@ -10,13 +10,6 @@ bool fhip_fast_matmul_applicable(const fhip_matmul_desc *d);
 int fhip_fast_matmul(fhip_ctx *ctx, const fhip_matmul_desc *d, const void *a,
                      const void *b, const DevEpilogue &epi, void *out);
 
-// The same with an outer batch dim of `outer` entries around the descriptor's
-// own (element strides per operand, 16-byte multiples; empty epilogue).
-int fhip_fast_matmul_outer(fhip_ctx *ctx, const fhip_matmul_desc *d,
-                           const void *a, const void *b, const DevEpilogue &epi,
-                           void *out, int outer, int64_t a_outer,
-                           int64_t b_outer, int64_t o_outer);
-
 // Products outside that contract -- few rows or columns, K or row starts that do
 // not fit 128-byte slices, f32 -- on kernels that load MFMA fragments straight
 // from global memory; `handled` false where they do not take the descriptor.
@@ -63,13 +56,16 @@ int fhip_fast_conv_dgrad_rf(fhip_ctx *ctx, const fhip_conv_desc *d,
 // fhip_conv_dgrad_static into the context (device current, creation lock held).
 int fhip_conv_dgrad_static_setup(fhip_ctx *ctx);
 
-// Weight gradient as batched GEMMs over zero-padded copies of X and DY
-// (channels-last 16-bit tensors, equal strides, one group); needs
-// `*workspace_bytes` of 256-byte aligned workspace.
+// Weight gradient of channels-last 16-bit tensors (channel counts multiples of 8, one
+// group) straight from X and DY on gathered MFMA tiles; needs `*workspace_bytes` of
+// 256-byte aligned workspace.  fhip_gather_conv_wgrad takes further descriptors, with
+// the context's scratch.
 bool fhip_fast_conv_wgrad_applicable(const fhip_conv_desc *d,
                                      size_t *workspace_bytes);
 int fhip_fast_conv_wgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy,
                          const void *x, void *dw, void *workspace);
+int fhip_gather_conv_wgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy,
+                           const void *x, void *dw, bool *handled);
 
 // Weight gradient of 3 x 3, padding-1, unit-stride convolutions straight from
 // X and DY (no operand copies): one MFMA kernel plus the sum of its partial
