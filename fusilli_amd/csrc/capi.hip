@@ -35,6 +35,8 @@ FhipKnobs parse_knobs() {
     k.conv_halo = atoi(e);
   if (const char *e = getenv("FUSILLI_HIP_CONV_BN"))
     k.conv_bn = atoi(e);
+  if (const char *e = getenv("FUSILLI_HIP_CONV_GATHER"))
+    k.conv_gather = atoi(e);
   if (const char *e = getenv("FUSILLI_HIP_CONV_ROWS"))
     k.conv_rows = atoi(e);
   if (const char *e = getenv("FUSILLI_HIP_WGRAD_DIRECT"))

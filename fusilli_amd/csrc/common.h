@@ -58,6 +58,7 @@ struct FhipKnobs {
   int conv_tile_bm = 0, conv_tile_bn = 0; // FUSILLI_HIP_CONV_TILE "bm,bn"
   int conv_halo = -1;               // FUSILLI_HIP_CONV_HALO (-1: unset)
   int conv_bn = 0;                  // FUSILLI_HIP_CONV_BN
+  int conv_gather = -1;             // FUSILLI_HIP_CONV_GATHER (-1: unset, 0: off, 1: wherever it can run)
   int conv_rows = -1;               // FUSILLI_HIP_CONV_ROWS (-1: unset)
   int gemm_tile_bm = 0, gemm_tile_bn = 0; // FUSILLI_HIP_GEMM_TILE "bm,bn"
   bool conv_depthwise_strips = true; // FUSILLI_HIP_CONV_DEPTHWISE_STRIPS=0: the general small-group kernel

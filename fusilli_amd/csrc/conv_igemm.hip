@@ -11,6 +11,7 @@
 // Reference semantics: aten.convolution, groups = 1 here (reference
 // support/asm_emitter.h:690-701, node/conv_node.h:38-56).
 #include "common.h"
+#include "conv_gather.h"
 #include "fast_paths.h"
 #include "gemm_kernel.h"
 
@@ -333,7 +334,31 @@ struct ConvResolved {
   bool padded = false; // X and W are first copied into the context's scratch
   int64_t C = 0, Cp = 0, x_pixels = 0, w_pixels = 0;
   size_t x_bytes = 0, w_bytes = 0;
+  // runs on the gathered tiles of conv_gather.hip instead (unpadded operands)
+  ConvGatherPlan gather{0};
 };
+
+// The gathered tiles for a problem that make_plan accepted (`C` its true channels).
+void choose_gather(ConvResolved &r, int64_t C) {
+  const ConvPlan &p = r.plan;
+  const FhipKnobs &knobs = fhip_knobs();
+  if (knobs.conv_gather == 0 || p.groups != 1 || C % 8 != 0 || knobs.conv_tile_bm || knobs.conv_halo >= 0 ||
+      knobs.conv_bn)
+    return;
+  const int64_t J = (int64_t)p.geom.R * p.geom.S * C;
+  // Channels that need padding copies first (16.9 -> 9 us at N16 48 -> 48, 48 x 32); else
+  // few tiles of several taps, whose chain of K slices leaves compute units idle (N32 256 ->
+  // 256, 14 x 14, 98 tiles: halo 31.4, here 25.4 us; N20 320 -> 320, 20 x 20, 189 tiles: 39.0,
+  // 41.0; N64 128 -> 64, 28 x 28, 392 tiles: 19.2, 24.7), and gathered tiles over outputs of
+  // less than half their width (N62 256 -> 48, 39 x 39: 69 us, here 50).
+  const int64_t tiles = ((p.M + p.bm - 1) / p.bm) * ((p.N + p.bn - 1) / p.bn);
+  const bool few = p.ksplit == 1 && tiles < 160 && p.geom.R * p.geom.S > 1;
+  const bool narrow = !p.halo && p.ksplit == 1 && p.N < 64;
+  const bool want = r.padded || knobs.conv_gather > 0 || few || narrow;
+  // (whole slices: no parts -- the entry point without scratch gives the same bits)
+  if (want)
+    r.gather = conv_gather_plan(p.M, p.N, J, r.padded && p.N % 4 == 0);
+}
 
 ConvResolved resolve(const fhip_conv_desc *d, bool allow_scratch = true) {
   ConvResolved r;
@@ -341,6 +366,8 @@ ConvResolved resolve(const fhip_conv_desc *d, bool allow_scratch = true) {
   const fhip_conv_desc *g = fold_3d(d, &folded) ? &folded : d;
   r.run = *g;
   r.plan = make_plan(g, d, allow_scratch);
+  if (r.plan.ok)
+    choose_gather(r, g->x.dim[1]);
   if (r.plan.ok || !allow_scratch)
     return r;
   // channel padding: 16-bit channels-last tensors, whole 16-byte chunks
@@ -379,6 +406,7 @@ ConvResolved resolve(const fhip_conv_desc *d, bool allow_scratch = true) {
   r.w_pixels = fhip_desc_volume(g->w) / C;
   r.x_bytes = ((size_t)(r.x_pixels * Cp * 2) + 255) / 256 * 256;
   r.w_bytes = ((size_t)(r.w_pixels * Cp * 2) + 255) / 256 * 256;
+  choose_gather(r, C);
   return r;
 }
 
@@ -486,12 +514,13 @@ int fhip_fast_conv(fhip_ctx *ctx, const fhip_conv_desc *d, const void *x,
                "conv: X and W must be 16-byte aligned");
   // the context's scratch: zero-padded copies of X and W, then the parts of a
   // split reduction
-  const size_t pad_bytes = res.padded ? res.x_bytes + res.w_bytes : 0;
+  const bool gather = res.gather.parts != 0;
+  const size_t pad_bytes = res.padded && !gather ? res.x_bytes + res.w_bytes : 0;
   // (rows of the parts are padded to whole column tiles, which are stored
   // whole: every cache line of the parts is written by one workgroup)
-  const int64_t part_pitch = (p.N + p.bn - 1) / p.bn * p.bn;
-  const size_t part_bytes =
-      p.ksplit > 1 ? (size_t)p.ksplit * (size_t)(p.M * part_pitch) * sizeof(float) : 0;
+  const int64_t part_pitch = gather ? p.N : (p.N + p.bn - 1) / p.bn * p.bn;
+  const int parts = gather ? res.gather.parts : p.ksplit;
+  const size_t part_bytes = parts > 1 ? (size_t)parts * (size_t)(p.M * part_pitch) * sizeof(float) : 0;
   char *scratch = nullptr;
   if (pad_bytes + part_bytes > 0) {
     void *sp = nullptr;
@@ -499,7 +528,7 @@ int fhip_fast_conv(fhip_ctx *ctx, const fhip_conv_desc *d, const void *x,
       return 1;
     scratch = (char *)sp;
   }
-  if (res.padded) {
+  if (res.padded && !gather) {
     // channel counts that are no multiple of 64: zero-padded copies of X and W
     char *xp = scratch, *wp = xp + res.x_bytes;
     const int32_t c8 = (int32_t)(res.C / 8), cp8 = (int32_t)(res.Cp / 8);
@@ -554,6 +583,44 @@ int fhip_fast_conv(fhip_ctx *ctx, const fhip_conv_desc *d, const void *x,
     o.stride[0] = 0;
     o.stride[1] = sm;          // per-pixel step (0 for channel vectors)
     o.stride[2] = s.stride[1]; // per-channel step
+  }
+  auto add_parts = [&](const float *part, const DevEpilogue &by_pixel) {
+    SplitSumArgs a{};
+    a.part = part;
+    a.out = out;
+    a.part_stride = p.M * part_pitch;
+    a.pitch = (int32_t)part_pitch;
+    a.mn4 = p.M * p.N / 4;
+    a.N = (int32_t)p.N;
+    a.parts = parts;
+    a.y_dt = d->y.dtype;
+    a.o_dt = d->out.dtype;
+    a.epi = by_pixel;
+    hipLaunchKernelGGL(conv_splitk_sum_kernel, dim3((unsigned)((a.mn4 + 255) / 256)),
+                       dim3(256), 0, ctx->stream, a);
+    FHIP_HIP_CHECK(ctx, hipGetLastError());
+    return 0;
+  };
+  if (gather) {
+    const ConvGeom &cg = p.geom;
+    ConvGatherArgs a{};
+    a.x = (const char *)x, a.w = (const char *)w, a.out = out;
+    a.part = parts > 1 ? (float *)scratch : nullptr;
+    a.M = p.M, a.N = (int32_t)p.N;
+    a.H = cg.H, a.W = cg.W, a.C = (int32_t)(res.padded ? res.C : cg.C), a.P = cg.P, a.Q = cg.Q, a.S = cg.S;
+    a.J = cg.R * cg.S * a.C;
+    a.pad_h = cg.pad_h, a.pad_w = cg.pad_w, a.str_h = cg.str_h, a.str_w = cg.str_w;
+    a.dil_h = cg.dil_h, a.dil_w = cg.dil_w;
+    a.x_bytes = (uint32_t)(p.M / ((int64_t)cg.P * cg.Q) * cg.H * cg.W * a.C * 2);
+    a.y_dt = d->y.dtype, a.o_dt = d->out.dtype;
+    a.epi = g.epi;
+    if (conv_gather_launch(ctx, p.kind == GK_BF16, res.gather, a) != 0)
+      return 1;
+    if (parts > 1 && add_parts((const float *)scratch, g.epi) != 0)
+      return 1;
+    fhip_note_kernel(ctx, "conv_igemm unpadded %dx%d split=%d", kConvGatherTile, kConvGatherTile,
+                     parts);
+    return 0;
   }
   // A single tap at unit stride without padding is the matrix product
   // X[pixels][C] . W[K][C]^T of dense operands: the GEMM entry takes them as
@@ -612,20 +679,8 @@ int fhip_fast_conv(fhip_ctx *ctx, const fhip_conv_desc *d, const void *x,
                                      : conv_launch_f16(ctx, p.bm, p.bn, g);
     if (rc != 0)
       return rc;
-    SplitSumArgs a{};
-    a.part = part;
-    a.out = out;
-    a.part_stride = p.M * part_pitch;
-    a.pitch = (int32_t)part_pitch;
-    a.mn4 = p.M * p.N / 4;
-    a.N = (int32_t)p.N;
-    a.parts = p.ksplit;
-    a.y_dt = d->y.dtype;
-    a.o_dt = d->out.dtype;
-    a.epi = by_pixel;
-    hipLaunchKernelGGL(conv_splitk_sum_kernel, dim3((unsigned)((a.mn4 + 255) / 256)),
-                       dim3(256), 0, ctx->stream, a);
-    FHIP_HIP_CHECK(ctx, hipGetLastError());
+    if (add_parts(part, by_pixel) != 0)
+      return 1;
     fhip_note_kernel(ctx, "conv_igemm gather %dx%d split=%d padded=%d groups=%d", p.bm, p.bn,
                      p.ksplit, (int)res.padded, (int)p.groups);
     return 0;

@@ -96,8 +96,15 @@ conv_wgrad_gather_kernel(WgArgs g) {
   __shared__ __attribute__((aligned(16))) char stage[2 * kStage];
   __shared__ int2 place[kWgChunk];
   const int tid = threadIdx.x, l = tid & 63, wave = tid >> 6;
-  const int tile = blockIdx.x % g.tiles;
-  const int64_t m0 = (int64_t)(blockIdx.x / g.tiles) * g.run;
+  // (workgroups go to the eight L2 slices in turn: the tiles of a run of pixels share one)
+  uint32_t id = blockIdx.x;
+  {
+    const uint32_t per = gridDim.x / 8, rest = gridDim.x % 8, slice = id % 8;
+    id = slice * per + (slice < rest ? slice : rest) + id / 8;
+  }
+  const int tile = (int)(id % (uint32_t)g.tiles);
+  const uint32_t which = id / (uint32_t)g.tiles; // run of pixels
+  const int64_t m0 = (int64_t)which * g.run;
   const int64_t m1 = m0 + g.run < g.pixels ? m0 + g.run : g.pixels;
   const int k0 = tile / g.jtiles * TK, j0 = tile % g.jtiles * TJ;
   // this thread's run of columns: its tap's shift and bytes behind a pixel's place
@@ -224,7 +231,7 @@ conv_wgrad_gather_kernel(WgArgs g) {
     }
   }
   // value i of a lane: row 8 * (i / 4) + 4 * (l / 32) + i % 4, column l % 32 of its tile
-  float *out = g.part + (int64_t)(blockIdx.x / g.tiles) * g.K * g.J;
+  float *out = g.part + (int64_t)which * g.K * g.J;
 #pragma unroll
   for (int a = 0; a < MT; ++a)
 #pragma unroll
@@ -304,8 +311,34 @@ struct WgradPlan {
   WgArgs a{};
   int tk = 0, tj = 0;
   int64_t runs = 0;
-  size_t part_bytes = 0;
+  size_t part_bytes = 0, contract = 0;
 };
+
+// The workspace that callers bring, 0 for descriptors that ask for none.  Sizes are kept
+// in callers' saved plans, so they stay what they were when X and DY were copied into
+// zero-padded grids (rows and columns padded, 64-pixel pitch, DY of 128 channels at
+// least) in front of the sums of every image's share; the sums of the runs fit in it.
+size_t wgrad_contract(const fhip_conv_desc *d) {
+  const int64_t N = d->x.dim[0], C = d->x.dim[1], K = d->w.dim[0], R = d->w.dim[2], S = d->w.dim[3];
+  const int64_t P = d->y.dim[2], Q = d->y.dim[3], str = d->stride[0];
+  if (str != d->stride[1] || d->dilation[1] != 1 || S * C < 128)
+    return 0;
+  const int64_t rows = (d->x.dim[2] + 2 * d->padding[0] + str - 1) / str * str, rows_y = rows / str;
+  const int64_t pitch = (d->x.dim[3] + 2 * d->padding[1] + 63) / 64 * 64;
+  if (P > rows_y || (Q - 1) * str + S > pitch)
+    return 0;
+  const int64_t Kp = K < 128 ? 128 : K, slices = rows_y * pitch / 64;
+  auto line = [](int64_t bytes) { return (size_t)(bytes + 255) / 256 * 256; };
+  int64_t split = 1;
+  for (int64_t f = 1; f <= slices; ++f)
+    if (slices % f == 0 && slices / f >= 8 && N * f * ((S * C + 127) / 128) * ((K + 127) / 128) <= 1024)
+      split = f;
+  const size_t x = line((N * rows * pitch * C + (R - 1) * d->dilation[0] * pitch * C + S * C) * 2);
+  const size_t dy = line(N * rows_y * pitch * Kp * 2);
+  if (x >= (1ull << 32) || dy >= (1ull << 32) || N * split > 65535)
+    return 0;
+  return x + dy + line(R * N * split * Kp * S * C * 4);
+}
 
 WgradPlan make_wgrad_plan(const fhip_conv_desc *d) {
   WgradPlan p;
@@ -362,12 +395,14 @@ WgradPlan make_wgrad_plan(const fhip_conv_desc *d) {
   // size is answered without one)
   const int64_t steps = (pixels + kWgStep - 1) / kWgStep;
   int64_t runs = (steps * tiles >= 512 * 16 ? 512 : 256) / tiles;
+  p.contract = wgrad_contract(d);
+  if (p.contract && runs > (int64_t)p.contract / (K * J * 4))
+    runs = (int64_t)p.contract / (K * J * 4);
   runs = runs < steps / 4 ? runs : steps / 4;
   runs = runs < 1 ? 1 : runs;
   a.run = (steps + runs - 1) / runs * kWgStep;
   p.runs = (pixels + a.run - 1) / a.run;
-  // (a line more than the sums: the size tells this plan from the 3 x 3 kernel's whole blocks)
-  p.part_bytes = (size_t)(p.runs * K * J) * sizeof(float) + 256;
+  p.part_bytes = (size_t)(p.runs * K * J) * sizeof(float);
   p.ok = p.runs * tiles < (1ll << 23);
   return p;
 }
@@ -425,10 +460,9 @@ bool fhip_fast_conv_wgrad_applicable(const fhip_conv_desc *d,
   if (fhip_fast_conv_wgrad_direct_applicable(d, workspace_bytes))
     return true;
   const WgradPlan p = make_wgrad_plan(d);
-  const bool ok = p.ok && d->stride[0] == d->stride[1] && d->dilation[1] == 1 &&
-                  d->w.dim[3] * d->w.dim[1] >= 128;
+  const bool ok = p.ok && p.contract != 0;
   if (workspace_bytes)
-    *workspace_bytes = ok ? p.part_bytes : 0;
+    *workspace_bytes = ok ? p.contract : 0;
   return ok;
 }
 
