@@ -87,6 +87,14 @@ int fhip_fail(fhip_ctx *ctx, const char *fmt, ...) {
   return 1;
 }
 
+bool fhip_ctx_scratch_ready(fhip_ctx *ctx, size_t bytes) {
+  if (bytes <= ctx->scratch_bytes)
+    return true;
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(ctx->stream, &status) == hipSuccess &&
+         status == hipStreamCaptureStatusNone;
+}
+
 int fhip_ctx_scratch(fhip_ctx *ctx, size_t bytes, void **out) {
   if (bytes > ctx->scratch_bytes) {
     FHIP_HIP_CHECK(ctx, hipSetDevice(ctx->device));

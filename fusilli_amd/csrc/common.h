@@ -46,6 +46,9 @@ inline void fhip_note_kernel(fhip_ctx *ctx, const char *fmt, ...) {
 // At least `bytes` of 256-byte aligned scratch in *out.  Growing it allocates
 // (after the stream has drained): not for callers under graph capture.
 int fhip_ctx_scratch(fhip_ctx *ctx, size_t bytes, void **out);
+// False where that would have to allocate while the context's stream is being captured;
+// paths that can do without scratch then do.
+bool fhip_ctx_scratch_ready(fhip_ctx *ctx, size_t bytes);
 
 // Tuning / test knobs from the environment, parsed once per process (and again
 // on fhip_tuning_reload) instead of on every launch.

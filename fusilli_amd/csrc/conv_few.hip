@@ -680,8 +680,11 @@ int fhip_few_conv_wgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy, 
   runs = runs < most ? runs : most;
   runs = runs < items ? runs : items;
   runs = runs < 1 ? 1 : runs;
+  const size_t bytes = (size_t)(runs * frags) * sizeof(float);
   void *scratch = nullptr;
-  if (fhip_ctx_scratch(ctx, (size_t)(runs * frags) * sizeof(float), &scratch) != 0)
+  if (!fhip_ctx_scratch_ready(ctx, bytes))
+    return 0;
+  if (fhip_ctx_scratch(ctx, bytes, &scratch) != 0)
     return 1;
   *handled = true;
   fhip_note_kernel(ctx, "conv_few wgrad tiles=%dx%d", kt, jt);

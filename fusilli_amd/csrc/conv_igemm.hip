@@ -354,7 +354,10 @@ void choose_gather(ConvResolved &r, int64_t C) {
   const int64_t tiles = ((p.M + p.bm - 1) / p.bm) * ((p.N + p.bn - 1) / p.bn);
   const bool few = p.ksplit == 1 && tiles < 160 && p.geom.R * p.geom.S > 1;
   const bool narrow = !p.halo && p.ksplit == 1 && p.N < 64;
-  const bool want = r.padded || knobs.conv_gather > 0 || few || narrow;
+  // (copies that add a seventh at most pay over many tiles: N32 112 -> 384, 26 x 26, 507
+  // tiles: step with the copies 152.7, without 157.0 us; N10 496 -> 128, 45 x 45, 159: 182, 177)
+  const bool copies = r.padded && !((r.Cp - r.C) * 7 <= r.C && tiles >= 400);
+  const bool want = copies || knobs.conv_gather > 0 || few || narrow;
   // (whole slices: no parts -- the entry point without scratch gives the same bits)
   if (want)
     r.gather = conv_gather_plan(p.M, p.N, J, r.padded && p.N % 4 == 0);
@@ -519,8 +522,11 @@ int fhip_fast_conv(fhip_ctx *ctx, const fhip_conv_desc *d, const void *x,
   // (rows of the parts are padded to whole column tiles, which are stored
   // whole: every cache line of the parts is written by one workgroup)
   const int64_t part_pitch = gather ? p.N : (p.N + p.bn - 1) / p.bn * p.bn;
-  const int parts = gather ? res.gather.parts : p.ksplit;
-  const size_t part_bytes = parts > 1 ? (size_t)parts * (size_t)(p.M * part_pitch) * sizeof(float) : 0;
+  ConvGatherPlan gather_plan = res.gather;
+  int parts = gather ? gather_plan.parts : p.ksplit;
+  size_t part_bytes = parts > 1 ? (size_t)parts * (size_t)(p.M * part_pitch) * sizeof(float) : 0;
+  if (gather && parts > 1 && !fhip_ctx_scratch_ready(ctx, part_bytes))
+    gather_plan.parts = parts = 1, part_bytes = 0;
   char *scratch = nullptr;
   if (pad_bytes + part_bytes > 0) {
     void *sp = nullptr;
@@ -614,7 +620,7 @@ int fhip_fast_conv(fhip_ctx *ctx, const fhip_conv_desc *d, const void *x,
     a.x_bytes = (uint32_t)(p.M / ((int64_t)cg.P * cg.Q) * cg.H * cg.W * a.C * 2);
     a.y_dt = d->y.dtype, a.o_dt = d->out.dtype;
     a.epi = g.epi;
-    if (conv_gather_launch(ctx, p.kind == GK_BF16, res.gather, a) != 0)
+    if (conv_gather_launch(ctx, p.kind == GK_BF16, gather_plan, a) != 0)
       return 1;
     if (parts > 1 && add_parts((const float *)scratch, g.epi) != 0)
       return 1;

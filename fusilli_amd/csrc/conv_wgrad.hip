@@ -482,7 +482,7 @@ int fhip_gather_conv_wgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *d
                            void *dw, bool *handled) {
   *handled = false;
   const WgradPlan p = make_wgrad_plan(d);
-  if (!p.ok || (((uintptr_t)x | (uintptr_t)dy) & 15) != 0)
+  if (!p.ok || (((uintptr_t)x | (uintptr_t)dy) & 15) != 0 || !fhip_ctx_scratch_ready(ctx, p.part_bytes))
     return 0;
   void *scratch = nullptr;
   if (fhip_ctx_scratch(ctx, p.part_bytes, &scratch) != 0)

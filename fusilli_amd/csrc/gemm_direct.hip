@@ -129,7 +129,9 @@ int fhip_direct_matmul(fhip_ctx *ctx, const fhip_matmul_desc *d, const void *a, 
   }
   if (g.splits > 1) {
     const size_t bytes = (size_t)g.splits * (size_t)batch * g.tiles_m * g.tiles_n * (p.mt * p.nt * 1024);
-    if (fhip_ctx_scratch(ctx, bytes, &g.partial) != 0)
+    if (!fhip_ctx_scratch_ready(ctx, bytes))
+      g.splits = 1;
+    else if (fhip_ctx_scratch(ctx, bytes, &g.partial) != 0)
       return 1;
   }
   // (f32 products that split K over the wavefronts of a tile keep that name)

@@ -562,8 +562,11 @@ int launch_mid(fhip_ctx *ctx, const ReducePlan &p, ReduceMidArgs g) {
     return -1; // (the strided kernel's)
   g.slices = (int32_t)slices;
   if (slices > 1) {
+    const size_t bytes = (size_t)(slices * p.k) * sizeof(float);
     void *sp = nullptr;
-    if (fhip_ctx_scratch(ctx, (size_t)(slices * p.k) * sizeof(float), &sp) != 0)
+    if (!fhip_ctx_scratch_ready(ctx, bytes))
+      return -1;
+    if (fhip_ctx_scratch(ctx, bytes, &sp) != 0)
       return 1;
     g.partial = (float *)sp;
   }

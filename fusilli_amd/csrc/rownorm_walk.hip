@@ -269,12 +269,14 @@ int fhip_norm_walk(fhip_ctx *ctx, int dtype, const RowNormArgs &n) {
   splits = splits < most ? splits : most;
   splits = splits < kRwThreads ? splits : kRwThreads;
   RowWalkArgs g{};
-  const bool cut = n.inner > 4 * kRwThreads * vec && n.rows < 2 * cus && splits > 1;
+  const size_t sums = (size_t)(2 * n.rows * (splits > 0 ? splits : 0)) * sizeof(float);
+  const bool cut = n.inner > 4 * kRwThreads * vec && n.rows < 2 * cus && splits > 1 &&
+                   fhip_ctx_scratch_ready(ctx, sums);
   if (cut) {
     g.seg = ((n.inner + splits - 1) / splits + vec - 1) / vec * vec;
     g.splits = (int32_t)((n.inner + g.seg - 1) / g.seg);
     void *scratch = nullptr;
-    if (fhip_ctx_scratch(ctx, (size_t)(2 * n.rows * g.splits) * sizeof(float), &scratch) != 0)
+    if (fhip_ctx_scratch(ctx, sums, &scratch) != 0)
       return 1;
     g.partial = (float *)scratch;
     g.n = n;

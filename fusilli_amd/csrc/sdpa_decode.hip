@@ -164,6 +164,12 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void sdpa_decode_kernel(DecodeArgs g)
   float m = kNegBig, sum = 0.f; // of query lq: max over all lanes, sum over this lane's keys
   auto spend = [&](auto buf, int c) {
     constexpr int B = decltype(buf)::value;
+    // (keys past the last are copies of it with probability 0; its values may be infinite)
+    if ((c + 1) * kChunk > g.Skv)
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (c * kChunk + (i >> 2) * 16 + lg * 4 + (i & 3) >= g.Skv)
+          vf[B][i] = VRow{};
     float s[8];
     uint32_t live = 0;
     float top = kNegBig;
@@ -340,6 +346,10 @@ int fhip_decode_sdpa(fhip_ctx *ctx, const fhip_sdpa_desc *d, const void *q, cons
   g.splits = (int32_t)(splits < 1 ? 1 : splits < 64 ? splits : 64);
   if (tiles * g.splits >= (1ll << 31))
     return 0;
+  const size_t rows16 = (size_t)g.splits * (size_t)tiles * 16;
+  const size_t part_bytes = rows16 * (size_t)(HD + 2) * sizeof(float);
+  if (g.splits > 1 && !fhip_ctx_scratch_ready(ctx, part_bytes))
+    g.splits = 1;
   *handled = true;
   g.q = (const char *)q, g.k = (const char *)k, g.v = (const char *)v, g.o = (char *)o;
   auto st = [](const fhip_tensor_desc &t, int i) { return t.dim[i] > 1 ? t.stride[i] : 0; };
@@ -351,9 +361,8 @@ int fhip_decode_sdpa(fhip_ctx *ctx, const fhip_sdpa_desc *d, const void *q, cons
   const float scale = d->has_scale ? d->scale : 1.0f / sqrtf((float)HD);
   g.scale_log2e = scale * 1.4426950408889634f;
   if (g.splits > 1) {
-    const size_t rows16 = (size_t)g.splits * (size_t)tiles * 16;
     void *sp = nullptr;
-    if (fhip_ctx_scratch(ctx, rows16 * (size_t)(HD + 2) * sizeof(float), &sp) != 0)
+    if (fhip_ctx_scratch(ctx, part_bytes, &sp) != 0)
       return 1;
     g.part = (float *)sp;
     g.part_ml = g.part + rows16 * HD;

@@ -1,0 +1,69 @@
+"""Calls recorded into a graph on a context that has never run one: paths that would
+have to grow the context's scratch do without it.  Every replay is compared with the
+eager result of a second context."""
+import pytest
+
+from fusilli_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+
+def _norm(torch):
+    x = torch.randn(2, 70001, device="cuda")
+    out = torch.empty_like(x)
+    d = capi.NormDesc()
+    d.x = d.y = d.out = capi.TensorDesc.make([2, 70001], [70001, 1], capi.FLOAT)
+    d.out_dtype, d.epsilon = capi.FLOAT, 1e-6
+    d.epilogue = capi.make_epilogue([capi.epilogue_op(capi.PW["MUL"], capi.FLOAT, scalar=0.5)])
+    return x, out, lambda c: c.norm_fwd(d, x.data_ptr(), None, None, out.data_ptr()), 1e-5
+
+
+def _sdpa(torch):
+    q, k, v = (torch.randn(1, 2, s, 64, device="cuda", dtype=torch.bfloat16) for s in (1, 2000, 2000))
+    out = torch.empty_like(q)
+    d = capi.SdpaDesc()
+    for f, t in (("q", q), ("k", k), ("v", v), ("o", out)):
+        setattr(d, f, capi.TensorDesc.make(list(t.shape), list(t.stride()), capi.BFLOAT16))
+    return q, out, lambda c: c.sdpa_fwd(d, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr()), 2e-2
+
+
+def _matmul(torch):
+    a = torch.randn(16, 4096, device="cuda", dtype=torch.bfloat16)
+    b = torch.randn(4096, 128, device="cuda", dtype=torch.bfloat16)
+    out = torch.empty(16, 128, device="cuda", dtype=torch.bfloat16)
+    d = capi.MatmulDesc()
+    d.a = capi.TensorDesc.make([16, 4096], [4096, 1], capi.BFLOAT16)
+    d.b = capi.TensorDesc.make([4096, 128], [128, 1], capi.BFLOAT16)
+    d.c = capi.TensorDesc.make([16, 128], [128, 1], capi.FLOAT)
+    d.out = capi.TensorDesc.make([16, 128], [128, 1], capi.BFLOAT16)
+    d.out_dtype = capi.BFLOAT16
+    d.epilogue = capi.make_epilogue([])
+    return a, out, lambda c: c.matmul(d, a.data_ptr(), b.data_ptr(), out.data_ptr()), 2e-2
+
+
+@pytest.mark.parametrize("make", [_norm, _sdpa, _matmul])
+def test_first_call_under_capture(make):
+    import torch
+    torch.manual_seed(1)
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        x, out, call, tol = make(torch)
+        cold = capi.Context(torch.cuda.current_device(), stream.cuda_stream)
+        warm = capi.Context(torch.cuda.current_device(), stream.cuda_stream)
+        graph = torch.cuda.CUDAGraph()
+        stream.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            call(cold)
+        for i in range(3):
+            x.copy_(torch.randn_like(x))
+            call(warm)
+            want = out.float().clone()
+            out.zero_()
+            graph.replay()
+            stream.synchronize()
+            got = out.float()
+            err = (got - want).norm() / want.norm()
+            assert err <= tol, (i, float(err))
+        del graph
+        cold.close()
+        warm.close()
