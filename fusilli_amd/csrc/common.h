@@ -551,7 +551,9 @@ __device__ __forceinline__ float fhip_gelu_erf_16bit(float x) {
   const float u = ax * 0.84932180028801904272f;
   const float e = __builtin_amdgcn_exp2f(-u * u);
   const float w = p * t * e;
-  return __builtin_fmaf(-ax, w, __builtin_fmaxf(x, 0.f));
+  // (w is 0 at +infinity: a finite factor keeps the product 0 there)
+  const float af = __builtin_fabsf(__builtin_fminf(x, __FLT_MAX__));
+  return __builtin_fmaf(-af, w, __builtin_fmaxf(x, 0.f));
 }
 
 // Vector forms: one uniform branch per call, straight-line code per case.

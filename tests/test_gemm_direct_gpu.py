@@ -94,3 +94,18 @@ def test_direct_epilogue(ctx, dtype, m, k):
     out, _ = run(ctx, a, b, capi.FLOAT, out_dtype=capi.BFLOAT16, epilogue=epi, epi_tensors=[bias, full])
     ref = (ref_matmul(a, b) + bias.logical()) * full.logical()
     assert_close(out.logical(), oracle.pointwise(capi.PW["GELU_FWD"], [ref]), capi.BFLOAT16)
+
+
+@pytest.mark.parametrize("dtype", [capi.BFLOAT16, capi.HALF])
+def test_direct_gelu_of_infinities(ctx, dtype):
+    a = make_operand(94, 0, 20, 64, dtype, False)
+    b = make_operand(94, 1, 64, 40, dtype, True)
+    v = np.zeros([1, 40], np.float32)
+    v[0, 3], v[0, 9] = np.inf, np.nan
+    bias = HT.from_logical(v, dtype)
+    epi = [capi.epilogue_op(capi.PW["ADD"], capi.FLOAT, operand=bias.desc(), operand_index=0),
+           capi.epilogue_op(capi.PW["GELU_FWD"], dtype)]
+    out, _ = run(ctx, a, b, capi.FLOAT, out_dtype=dtype, epilogue=epi, epi_tensors=[bias])
+    got = out.logical()
+    assert (got[:, 3] == np.inf).all() and np.isnan(got[:, 9]).all()
+    assert np.isfinite(np.delete(got, [3, 9], axis=1)).all()
