@@ -142,3 +142,16 @@ def test_reduce_columns_propagate_nan(ctx, mode):
     assert np.isnan(out[5]) and np.isnan(out).sum() == 1
     assert out[11] == (-np.inf if mode == "MIN" else np.inf if mode == "AMAX" else out[11])
     assert out[17] == (np.inf if mode in ("MAX", "AMAX") else out[17])
+
+
+@pytest.mark.parametrize("dtype", [capi.FLOAT, capi.BFLOAT16])
+@pytest.mark.parametrize("dims,odims", [([40000, 64], [1, 64]), ([200, 24, 20, 20], [1, 24, 1, 1])])
+def test_column_sums_round_about_once(ctx, dtype, dims, odims):
+    # Running sums in f64 over f32 sums of four: what is left is the rounding of the
+    # slices' sums and of the result, 2^-24 of a value each at most.  As a 2-norm both
+    # stay below one such step (the strided kernel this replaced: 4.5e-8 to 6.9e-8).
+    x = HT.from_logical(rand(68, 0, dims), dtype)
+    got = run(ctx, x, odims, "SUM", y_dtype=capi.FLOAT, expect_tuned=False).logical().astype(np.float64)
+    axes = tuple(i for i, n in enumerate(odims) if n == 1)
+    ref = x.logical().astype(np.float64).sum(axis=axes, keepdims=True)
+    assert np.linalg.norm(got - ref) <= 2.0 ** -24 * np.linalg.norm(ref)
