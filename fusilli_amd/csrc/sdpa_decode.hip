@@ -50,6 +50,7 @@ struct DecodeArgs {
   float *part_ml;
   int32_t Sq, Skv, group, Hkv;
   int32_t heads;     // B * Hkv
+  int32_t pitch;     // packed rows per query head: Sq, or Sq rounded up to whole tiles
   int32_t qtiles;    // tiles of 16 rows per key / value head
   int32_t splits, chunks, causal;
   float scale_log2e;
@@ -82,11 +83,12 @@ template <bool BF16> __device__ __forceinline__ void dec_store(char *o, int64_t 
     ((SD_AS1 _Float16 *)o)[at] = (_Float16)v;
 }
 
-// Offset of packed row `r` (grouped head r / Sq, position r % Sq) in Q or O.
+// Offset of packed row `r` (grouped head r / pitch, position r % pitch; positions past
+// the last stand for it) in Q or O.
 __device__ __forceinline__ int64_t dec_row(const DecodeArgs &g, int b, int hk, int r, int64_t sb,
                                            int64_t sh, int64_t ss) {
-  const int hg = r / g.Sq;
-  return b * sb + (int64_t)(hk * g.group + hg) * sh + (int64_t)(r - hg * g.Sq) * ss;
+  const int hg = r / g.pitch, p = r - hg * g.pitch;
+  return b * sb + (int64_t)(hk * g.group + hg) * sh + (int64_t)(p < g.Sq ? p : g.Sq - 1) * ss;
 }
 
 template <bool BF16, int HD>
@@ -105,10 +107,10 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void sdpa_decode_kernel(DecodeArgs g)
   const int qt = blockIdx.x / per, rest = blockIdx.x % per;
   const int head = rest / g.splits, split = rest % g.splits;
   const int b = head / g.Hkv, hk = head % g.Hkv;
-  const int rows = g.group * g.Sq;
+  const int rows = g.group * g.pitch;
   const int row = qt * 16 + lq;
   const int rowc = row < rows ? row : rows - 1;
-  const int pos = rowc % g.Sq; // query position, for the causal mask
+  const int pos = rowc % g.pitch; // query position, for the causal mask
 
   uint32_t qf[KD][4];
   {
@@ -127,7 +129,8 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void sdpa_decode_kernel(DecodeArgs g)
   int chunks = g.chunks;
   if (g.causal) {
     const int first = qt * 16, last = first + 15 < rows - 1 ? first + 15 : rows - 1;
-    const int top = first / g.Sq == last / g.Sq ? last % g.Sq : g.Sq - 1;
+    int top = first / g.pitch == last / g.pitch ? last % g.pitch : g.Sq - 1;
+    top = top < g.Sq ? top : g.Sq - 1;
     const int need = top / kChunk + 1;
     chunks = need < chunks ? need : chunks;
   }
@@ -253,6 +256,8 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void sdpa_decode_kernel(DecodeArgs g)
   const int64_t tiles = (int64_t)g.heads * g.qtiles;
   const int d = threadIdx.x % HD;
   for (int q = threadIdx.x / HD; q < 16 && qt * 16 + q < rows; q += kWaves * 64 / HD) {
+    if ((qt * 16 + q) % g.pitch >= g.Sq)
+      continue;
     float top = ml[0][0][q];
 #pragma unroll
     for (int w = 1; w < kWaves; ++w)
@@ -278,12 +283,14 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void sdpa_decode_kernel(DecodeArgs g)
 // Combines the splits of one packed query row per HD threads.
 template <bool BF16, int HD>
 __global__ __launch_bounds__(256) void sdpa_decode_combine_kernel(DecodeArgs g) {
-  const int rows = g.group * g.Sq;
+  const int rows = g.group * g.pitch;
   const int64_t lin = (int64_t)blockIdx.x * (256 / HD) + threadIdx.x / HD; // (head, row)
   const int d = threadIdx.x % HD;
   if (lin >= (int64_t)g.heads * rows)
     return;
   const int head = (int)(lin / rows), row = (int)(lin % rows);
+  if (row % g.pitch >= g.Sq)
+    return;
   const int64_t tiles = (int64_t)g.heads * g.qtiles;
   const int64_t at = (int64_t)(head * g.qtiles + row / 16) * 16 + row % 16;
   const SD_AS1 float *ml = (const SD_AS1 float *)g.part_ml;
@@ -317,10 +324,15 @@ int fhip_decode_sdpa(fhip_ctx *ctx, const fhip_sdpa_desc *d, const void *q, cons
   g.Skv = (int32_t)d->k.dim[2];
   g.group = (int32_t)(Hq / Hkv);
   g.Hkv = (int32_t)Hkv;
-  if (B * Hkv >= (1 << 24) || (int64_t)g.group * g.Sq >= (1 << 24))
+  if (B * Hkv >= (1 << 24) || (int64_t)g.group * (g.Sq + 15) >= (1 << 24))
     return 0;
   g.heads = (int32_t)(B * Hkv);
-  const int rows = g.group * g.Sq;
+  // Under a causal mask a tile walks the keys up to its last position.  With the end of
+  // one head's positions and the start of the next in one tile, the first positions would
+  // be multiplied (by zero) with values up to the last key, infinite or NaN ones included,
+  // where the tiled kernel stops at their own 64 keys: there a head starts a tile.
+  g.pitch = d->is_causal && g.Sq > 64 ? (g.Sq + 15) / 16 * 16 : g.Sq;
+  const int rows = g.group * g.pitch;
   g.qtiles = (rows + 15) / 16;
   int kv = g.Skv; // keys that any row sees
   if (d->is_causal && g.Sq < kv)

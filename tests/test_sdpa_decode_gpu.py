@@ -1,5 +1,6 @@
 """Attention with the keys split over workgroups (few query rows per key / value
 head), and the tiled kernel on the same problems, vs the oracle."""
+import numpy as np
 import pytest
 
 from fusilli_amd import capi
@@ -48,3 +49,25 @@ def test_decode_layout_and_scale(ctx, knobs, hd):
     assert "splits=" in ctx.last_kernel() and not ctx.last_kernel().endswith("splits=1"), ctx.last_kernel()
     assert_close(out.logical(), oracle.sdpa(q.logical(), k.logical(), v.logical(), scale=0.31),
                  capi.BFLOAT16)
+
+
+@pytest.mark.parametrize("hd", [128, 64])
+@pytest.mark.parametrize("decode", [1, 0])
+@pytest.mark.parametrize("sq,group,first", [
+    (100, 4, 64),   # a tile of 16 packed rows holds the end of one head and the start of the next
+    (100, 1, 64),
+    (20, 3, None),  # one tile of 64 keys: the tiled kernel multiplies masked values there as well
+])
+def test_causal_rows_do_not_meet_late_values(ctx, knobs, hd, decode, sq, group, first):
+    # the last key's value is infinite: only the rows whose 64 keys hold it may show that
+    knobs(SDPA_DECODE=decode)
+    q = HT.from_logical(rand(58, 0, [1, 2 * group, sq, hd]), capi.BFLOAT16)
+    k = HT.from_logical(rand(58, 1, [1, 2, sq, hd]), capi.BFLOAT16)
+    v = rand(58, 2, [1, 2, sq, hd])
+    ref = oracle.sdpa(q.logical(), k.logical(), HT.from_logical(v, capi.BFLOAT16).logical(), is_causal=True)
+    v[:, :, -1, :] = np.inf
+    out = run(ctx, q, k, HT.from_logical(v, capi.BFLOAT16), causal=True).logical()
+    assert ctx.last_kernel().startswith("sdpa_decode" if decode else "sdpa_fwd"), ctx.last_kernel()
+    assert not np.isfinite(out[:, :, -1]).any()
+    if first is not None:
+        assert_close(out[:, :, :first], ref[:, :, :first], capi.BFLOAT16)
