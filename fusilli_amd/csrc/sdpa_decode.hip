@@ -339,17 +339,23 @@ int fhip_decode_sdpa(fhip_ctx *ctx, const fhip_sdpa_desc *d, const void *q, cons
     kv = g.Sq;
   g.chunks = (kv + kChunk - 1) / kChunk;
   const int64_t tiles = (int64_t)g.heads * g.qtiles;
-  // Estimates in microseconds.  Here: K and V of a head once per tile of rows at
-  // 6.5 TB/s (B4, 32 heads, 256 x 256, D128: 36.5), half of that under a causal
-  // mask.  The tiled kernel: 1.7 per 64 keys and round of 256 workgroups of 256
-  // rows, a long and a short tile per workgroup under a causal mask (the same
-  // 12.2; B2, 16 heads, 512 x 512 causal 27.7, here 20).
-  const double half = d->is_causal && g.Sq > 16 ? 0.5 + 8.0 / g.Sq : 1.0;
-  const double here = 4.0 + (double)tiles * kv * HD * 4.0 / 6.5e6 * half;
+  // Estimates in microseconds, fitted to both kernels' times on 700 problems (1 to 2500
+  // queries, 32 to 4096 keys, 1 to 64 heads, batches to 32).  Here: the tiles' reads of K
+  // and V, whole rounds of the four wavefronts' 32 keys, half of them under a causal mask,
+  // at 10.7 TB/s from the caches; a tile's fixed part; the heads' own K and V from memory.
+  // The tiled kernel: 1.45 (D 64: 0.97) per 64 keys and round of 256 workgroups of 256
+  // rows, a long and a short tile per workgroup under a causal mask.  (B21, 64 heads on 8,
+  // 68 x 68 causal, D128, 5880 tiles: tiled 48.5, here 62.2; B4, 8 heads on 1, 320 x 3456,
+  // D64: 56.3, 60.1; B2, 16 heads on 4, 128 x 128 causal, D64: 6.4, 5.1.)
+  const double keys = kv <= kChunk ? 64.0 // (one wavefront works)
+                                   : ceil(kv * (d->is_causal && g.Sq > 16 ? 0.5 + 8.0 / g.Sq : 1.0) / 128.0) * 128.0;
+  const double here = 4.64 + (double)tiles * keys * HD * 4.0 * 0.093e-6 + (double)tiles * HD * 2e-5 +
+                      (double)g.heads * kv * HD * 4.0 * 0.074e-6;
   const int64_t big = (g.Sq + 255) / 256, kvt = (kv + 63) / 64;
   const bool pairs = d->is_causal && big > 1;
-  const double there = 4.0 + ceil((double)(B * Hq * (pairs ? (big + 1) / 2 : big)) / 256.0) *
-                                 (pairs ? 3.0 + 1.7 * (double)(kvt * (big + 1)) / (double)big : 1.7 * (double)kvt);
+  const double per = HD == 128 ? 1.45 : 0.97;
+  const double there = 0.43 + ceil((double)(B * Hq * (pairs ? (big + 1) / 2 : big)) / 256.0) *
+                                  (pairs ? 8.2 + per * (double)(kvt * (big + 1)) / (double)big : 4.1 + per * (double)kvt);
   if (here >= there && forced != 1)
     return 0;
   // two workgroups per compute unit, two chunks per wavefront at least

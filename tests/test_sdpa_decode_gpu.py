@@ -71,3 +71,50 @@ def test_causal_rows_do_not_meet_late_values(ctx, knobs, hd, decode, sq, group, 
     assert not np.isfinite(out[:, :, -1]).any()
     if first is not None:
         assert_close(out[:, :, :first], ref[:, :, :first], capi.BFLOAT16)
+
+
+@pytest.mark.parametrize("case", [
+    dict(B=8, Hq=32, Hkv=8, Sq=1, Skv=4000, hd=128, causal=False),
+    dict(B=2, Hq=16, Hkv=4, Sq=128, Skv=128, hd=64, causal=True),
+    dict(B=2, Hq=8, Hkv=2, Sq=16, Skv=2000, hd=64, causal=False),
+])
+@pytest.mark.parametrize("dtype", [capi.BFLOAT16, capi.HALF])
+@pytest.mark.parametrize("std", [1.0, 3.0])
+def test_split_keys_lose_no_precision(ctx, knobs, case, dtype, std):
+    # Both kernels round the probabilities to 16 bits, against different reference points;
+    # the error against 64 bits may not grow by it.  (The two errors are sums over at least
+    # 32 000 independent roundings: their ratio moves by a percent or so.)
+    c = case
+    q = HT.from_logical(rand(59, 0, [c["B"], c["Hq"], c["Sq"], c["hd"]], std=std), dtype)
+    k = HT.from_logical(rand(59, 1, [c["B"], c["Hkv"], c["Skv"], c["hd"]]), dtype)
+    v = HT.from_logical(rand(59, 2, [c["B"], c["Hkv"], c["Skv"], c["hd"]]), dtype)
+    group = c["Hq"] // c["Hkv"]
+    ql, kl, vl = (t.logical().astype(np.float64) for t in (q, k, v))
+    ref = np.empty(q.dims, np.float64)
+    for b in range(c["B"]):
+        for h in range(c["Hq"]):
+            s = ql[b, h] @ kl[b, h // group].T / np.sqrt(c["hd"])
+            if c["causal"]:
+                s[np.triu_indices(c["Sq"], 1)] = -np.inf
+            p = np.exp(s - s.max(1, keepdims=True))
+            ref[b, h] = p @ vl[b, h // group] / p.sum(1, keepdims=True)
+    err = []
+    for decode in (0, 1):
+        knobs(SDPA_DECODE=decode)
+        out = run(ctx, q, k, v, causal=c["causal"])
+        assert ctx.last_kernel().startswith("sdpa_decode" if decode else "sdpa_fwd"), ctx.last_kernel()
+        err.append(np.linalg.norm(out.logical() - ref) / np.linalg.norm(ref))
+    assert err[1] <= 1.02 * err[0], err
+
+
+def test_route_of_short_products_and_many_tiles(ctx):
+    # the kernel that measured faster on each side of the rule
+    def name(b, hq, hkv, sq, skv, hd, causal):
+        q = HT.from_logical(rand(60, 0, [b, hq, sq, hd]), capi.BFLOAT16)
+        k = HT.from_logical(rand(60, 1, [b, hkv, skv, hd]), capi.BFLOAT16)
+        run(ctx, q, k, k, causal=causal)
+        return ctx.last_kernel().split()[0]
+    assert name(1, 8, 2, 1, 2000, 128, False) == "sdpa_decode"
+    assert name(2, 16, 4, 128, 128, 64, True) == "sdpa_decode"
+    assert name(4, 64, 8, 68, 68, 128, True) == "sdpa_fwd"
+    assert name(5, 32, 32, 266, 266, 64, True) == "sdpa_fwd"
