@@ -87,28 +87,41 @@ int fhip_fail(fhip_ctx *ctx, const char *fmt, ...) {
   return 1;
 }
 
-bool fhip_ctx_scratch_ready(fhip_ctx *ctx, size_t bytes) {
-  if (bytes <= ctx->scratch_bytes)
-    return true;
+// (an error stands for a capture: the legacy stream beside another stream's)
+static bool stream_is_captured(fhip_ctx *ctx) {
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(ctx->stream, &status) == hipSuccess &&
-         status == hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(ctx->stream, &status) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return status != hipStreamCaptureStatusNone;
+}
+
+bool fhip_ctx_scratch_ready(fhip_ctx *ctx, size_t bytes) {
+  return bytes <= ctx->scratch.bytes || !stream_is_captured(ctx);
 }
 
 int fhip_ctx_scratch(fhip_ctx *ctx, size_t bytes, void **out) {
-  if (bytes > ctx->scratch_bytes) {
+  if (bytes > ctx->scratch.bytes) {
     FHIP_HIP_CHECK(ctx, hipSetDevice(ctx->device));
-    if (ctx->scratch) {
+    if (ctx->scratch.block)
       FHIP_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
-      FHIP_HIP_CHECK(ctx, hipFree(ctx->scratch));
-      ctx->scratch = nullptr;
-      ctx->scratch_bytes = 0;
-    }
-    const size_t want = bytes < (64u << 10) ? (64u << 10) : bytes;
-    FHIP_HIP_CHECK(ctx, hipMalloc(&ctx->scratch, want));
-    ctx->scratch_bytes = want;
+    hipError_t status = hipErrorOutOfMemory;
+    const bool grown = ctx->scratch.grow(
+        bytes,
+        [&](size_t size) {
+          void *p = nullptr;
+          status = hipMalloc(&p, size);
+          if (status != hipSuccess)
+            (void)hipGetLastError();
+          return status == hipSuccess ? p : nullptr;
+        },
+        [&](void *p) { (void)hipFree(p); });
+    FHIP_REQUIRE(ctx, grown, "scratch of %zu bytes: %s", bytes, hipGetErrorString(status));
   }
-  *out = ctx->scratch;
+  if (!ctx->scratch.recorded && stream_is_captured(ctx))
+    ctx->scratch.recorded = true;
+  *out = ctx->scratch.block;
   return 0;
 }
 
@@ -274,8 +287,7 @@ int fhip_ctx_destroy(fhip_ctx *ctx) {
     (void)hipStreamSynchronize(ctx->stream);
     (void)hipStreamDestroy(ctx->stream);
   }
-  if (ctx->scratch)
-    (void)hipFree(ctx->scratch);
+  ctx->scratch.release_all([](void *p) { (void)hipFree(p); });
   delete ctx;
   return 0;
 }

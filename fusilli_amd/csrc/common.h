@@ -13,6 +13,7 @@
 #include <string>
 
 #include "../../include/fusilli_hip.h"
+#include "scratch_blocks.h"
 
 // ---------------------------------------------------------------------------
 // Context
@@ -26,8 +27,7 @@ struct fhip_ctx {
   void *dgrad_static_scratch = nullptr;
   // device memory for kernels' partial results, owned by the context (one
   // stream: its users are ordered); grown on demand, freed with the context
-  void *scratch = nullptr;
-  size_t scratch_bytes = 0;
+  FhipScratchBlocks scratch;
   std::string err;
   // name and shape parameters of the kernel variant that the last operator
   // call on this context chose (fhip_last_kernel)
@@ -44,7 +44,8 @@ inline void fhip_note_kernel(fhip_ctx *ctx, const char *fmt, ...) {
   va_end(ap);
 }
 // At least `bytes` of 256-byte aligned scratch in *out.  Growing it allocates
-// (after the stream has drained): not for callers under graph capture.
+// (after the stream has drained): not for callers under graph capture.  Memory handed
+// out while the stream is being captured stays where it is until the context goes.
 int fhip_ctx_scratch(fhip_ctx *ctx, size_t bytes, void **out);
 // False where that would have to allocate while the context's stream is being captured;
 // paths that can do without scratch then do.

@@ -22,6 +22,9 @@
  *     the op's fixed logical order (NCHW / KCRS / [B,H,S,D] / [..,M,K]) plus
  *     element strides that define the physical layout
  *     (reference: attributes/tensor_attributes.h:374-809);
+ *   - calls may be recorded into a HIP graph; replays are ordered with the
+ *     context's stream like its calls (they share its scratch memory, which
+ *     stays allocated until fhip_ctx_destroy) and end before the context does;
  *   - a context is not thread-safe; creating contexts concurrently is
  *     (reference: tests/test_handle.cpp:47-85).
  */

@@ -1,6 +1,7 @@
-"""Calls recorded into a graph on a context that has never run one: paths that would
-have to grow the context's scratch do without it.  Every replay is compared with the
-eager result of a second context."""
+"""Calls recorded into a graph: on a context that has never run one, paths that would
+have to grow the context's scratch do without it; on one that has, the scratch that the
+graph names outlives later growth.  Every replay is compared with the eager result of a
+second context."""
 import pytest
 
 from fusilli_amd import capi
@@ -39,6 +40,51 @@ def _matmul(torch):
     d.out_dtype = capi.BFLOAT16
     d.epilogue = capi.make_epilogue([])
     return a, out, lambda c: c.matmul(d, a.data_ptr(), b.data_ptr(), out.data_ptr()), 2e-2
+
+
+@pytest.mark.parametrize("make", [_norm, _sdpa, _matmul])
+def test_replay_after_scratch_has_grown(make):
+    import torch
+    torch.manual_seed(2)
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        x, out, call, tol = make(torch)
+        big = capi.ConvDesc()  # 4 MB of partial sums
+        xs = torch.randn(8, 32, 32, 64, device="cuda", dtype=torch.bfloat16)
+        dy = torch.randn(8, 32, 32, 256, device="cuda", dtype=torch.bfloat16)
+        dw = torch.empty(256, 1, 1, 64, device="cuda")
+        cl = lambda n, c, h, w: capi.TensorDesc.make([n, c, h, w], [c * h * w, 1, c * w, c], capi.BFLOAT16)  # noqa: E731
+        big.x, big.y = cl(8, 64, 32, 32), cl(8, 256, 32, 32)
+        big.w = capi.TensorDesc.make([256, 64, 1, 1], [64, 1, 64, 64], capi.FLOAT)
+        big.spatial_rank = 2
+        for i in range(2):
+            big.stride[i] = big.dilation[i] = 1
+        big.epilogue = capi.make_epilogue([])
+        warm = capi.Context(torch.cuda.current_device(), stream.cuda_stream)
+        other = capi.Context(torch.cuda.current_device(), stream.cuda_stream)
+        call(warm)
+        graph = torch.cuda.CUDAGraph()
+        stream.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            call(warm)
+        for i in range(4):
+            if i == 1:
+                warm.conv_wgrad(big, dy.data_ptr(), xs.data_ptr(), dw.data_ptr())
+                assert warm.last_kernel() == "conv_wgrad_gather 256x64 runs=64"
+            x.copy_(torch.randn_like(x))
+            call(other)
+            want = out.clone()
+            out.zero_()
+            # memory that went back to the device would be handed out again here
+            fill = [torch.full((1 << 18,), 7.0, device="cuda") for _ in range(8)]
+            graph.replay()
+            stream.synchronize()
+            assert torch.equal(out, want), i
+            assert all(bool((f == 7.0).all()) for f in fill), i
+            del fill
+        del graph
+        warm.close()
+        other.close()
 
 
 @pytest.mark.parametrize("make", [_norm, _sdpa, _matmul])

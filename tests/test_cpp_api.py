@@ -41,6 +41,12 @@ def test_cpp_node_validation():
     assert "cases, 0 failed" in out
 
 
+def test_cpp_scratch_blocks():
+    """Which scratch blocks live and go: memory that a recorded graph names is kept."""
+    out = _run("test_scratch_blocks", 60)
+    assert "cases, 0 failed" in out
+
+
 @pytest.mark.gpu
 def test_cpp_device_api():
     _run("test_device_api", 300)
