@@ -172,7 +172,7 @@ struct ReduceRowsArgs {
   int64_t rows;
   int64_t chunks; // 16-byte chunks per row
   int32_t y_dt, post;
-  float inv_count;
+  float count; // reduced values behind a result (mean: a division, exact for equal values)
 };
 
 template <typename T, int MAP, int COMB, int TPR>
@@ -221,7 +221,7 @@ __global__ __launch_bounds__(256) void reduce_rows_kernel(ReduceRowsArgs g) {
   float acc = rf_finish<T, MAP, COMB>(a);
   if (lane == 0 && live) {
     if (g.post == P_MEAN)
-      acc *= g.inv_count;
+      acc /= g.count;
     else if (g.post == P_SQRT)
       acc = sqrtf(acc);
     if (g.y_dt == FHIP_FLOAT)
@@ -251,7 +251,7 @@ struct ReduceMidArgs {
   uint32_t magic_r2;
   int32_t slices;
   int32_t y_dt, post;
-  float inv_count;
+  float count; // reduced values behind a result (mean: a division, exact for equal values)
 };
 
 // NaN-propagating combine of two values (sums and products propagate by
@@ -283,7 +283,7 @@ template <int COMB, typename A> __device__ __forceinline__ A rf_run_comb(A a, A 
 
 __device__ __forceinline__ void rf_store(const ReduceMidArgs &g, int64_t i, float v) {
   if (g.post == P_MEAN)
-    v *= g.inv_count;
+    v /= g.count;
   else if (g.post == P_SQRT)
     v = sqrtf(v);
   if (g.y_dt == FHIP_FLOAT)
@@ -710,7 +710,7 @@ int fhip_mid_reduce(fhip_ctx *ctx, const fhip_reduce_desc *d, const void *x, voi
   g.r2 = (int32_t)p.r2;
   g.y_dt = d->y.dtype;
   g.post = p.post;
-  g.inv_count = 1.0f / (float)(p.r1 * p.r2);
+  g.count = (float)(p.r1 * p.r2);
   const int rc = d->x.dtype == FHIP_FLOAT      ? launch_mid_mode<float>(ctx, p, g)
                  : d->x.dtype == FHIP_BFLOAT16 ? launch_mid_mode<__bf16>(ctx, p, g)
                                                : launch_mid_mode<_Float16>(ctx, p, g);
@@ -732,7 +732,7 @@ int fhip_fast_reduce(fhip_ctx *ctx, const fhip_reduce_desc *d, const void *x,
   g.chunks = p.cols * fhip_dtype_size(d->x.dtype) / 16;
   g.y_dt = d->y.dtype;
   g.post = p.post;
-  g.inv_count = 1.0f / (float)p.cols;
+  g.count = (float)p.cols;
   fhip_note_kernel(ctx, "reduce_rows");
   switch (d->x.dtype) {
   case FHIP_FLOAT:

@@ -155,3 +155,17 @@ def test_column_sums_round_about_once(ctx, dtype, dims, odims):
     axes = tuple(i for i, n in enumerate(odims) if n == 1)
     ref = x.logical().astype(np.float64).sum(axis=axes, keepdims=True)
     assert np.linalg.norm(got - ref) <= 2.0 ** -24 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("dtype", [capi.FLOAT, capi.HALF])
+@pytest.mark.parametrize("kernel", ["reduce_cols", "reduce_mid", "reduce_rows"])
+@pytest.mark.parametrize("n", [41, 47, 55, 82, 83, 94, 97])
+def test_mean_of_equal_values_is_that_value(ctx, dtype, kernel, n):
+    # (n times the f32 nearest to 1 / n is not 1 for these n)
+    assert np.float32(n) * (np.float32(1) / np.float32(n)) != 1
+    dims, odims = {"reduce_cols": ([n, 5], [1, 5]), "reduce_mid": ([2, 3, n, 2], [1, 3, 1, 1]),
+                   "reduce_rows": ([3, 8 * n], [3, 1])}[kernel]
+    x = HT.from_logical(np.ones(dims), dtype)
+    out = run(ctx, x, odims, "AVG", y_dtype=capi.FLOAT, expect_tuned=kernel == "reduce_rows").logical()
+    assert ctx.last_kernel().startswith(kernel), ctx.last_kernel()
+    assert (out == 1).all()
