@@ -235,8 +235,8 @@ __global__ __launch_bounds__(256) void reduce_rows_kernel(ReduceRowsArgs g) {
 
 // Reductions that leave dims behind the reduced ones, X[r1][k][r2] -> Y[k]: the
 // bias gradient of a convolution (channels-last: r2 = 1, otherwise r2 = H * W),
-// column sums of a matrix.  The r1 range is cut into slices on workgroups of
-// their own (partial[slice][k], f32), which a second kernel combines in slice
+// column sums of a matrix.  The range of r1 (of r1 * r2 where r2 > 1) is cut into
+// slices on workgroups of their own (partial[slice][k], f32), which a second kernel combines in slice
 // order: no atomics.  Bound by reading X once.  N32 56 x 56 K128 bf16 in
 // channels-last (25.7 MB): 104 us on the strided kernel (one workgroup per
 // channel and slice reading one 2-byte element per pixel line) -> 12.7 us
@@ -246,8 +246,8 @@ struct ReduceMidArgs {
   const char *x;
   void *y;
   float *partial; // null: one slice, the result goes to y
-  int64_t r1, per_slice;
-  int32_t k, r2; // r2: in vectors of the kernel's width
+  int64_t r1, per_slice; // of a slice: rows (r2 == 1), vectors of the r1 * r2 range otherwise
+  int32_t k, r2;         // r2: in vectors of the kernel's width
   uint32_t magic_r2;
   int32_t slices;
   int32_t y_dt, post;
@@ -255,10 +255,13 @@ struct ReduceMidArgs {
 };
 
 // NaN-propagating combine of two values (sums and products propagate by
-// themselves)
+// themselves; the others are one instruction each: bf16 [8, 7, 7] x 512 channels-last
+// maxima 10.9 us with compares and selects)
 template <int COMB> __device__ __forceinline__ float rf_comb_nan(float a, float b) {
-  if constexpr (COMB == C_MIN || COMB == C_MAX)
-    return a != a ? a : (b != b ? b : rf_comb<COMB>(a, b));
+  if constexpr (COMB == C_MIN)
+    return __builtin_elementwise_minimum(a, b);
+  else if constexpr (COMB == C_MAX)
+    return __builtin_elementwise_maximum(a, b);
   else
     return rf_comb<COMB>(a, b);
 }
@@ -385,19 +388,28 @@ __global__ __launch_bounds__(256) void reduce_cols_kernel(ReduceMidArgs g, int t
   }
 }
 
-// r2 > 1: one k and one slice of r1 per workgroup, its runs of r2 as one index.
-template <typename T, int MAP, int COMB, int VEC>
+// r2 > 1: one k and one slice of the r1 * r2 range per workgroup, the range's runs of r2
+// as one index.  (Without SLICED the range is whole: a million rows of 3 values are
+// bound by what a workgroup does before its loop, 556 us against 616.)
+template <typename T, int MAP, int COMB, int VEC, bool SLICED>
 __global__ __launch_bounds__(256) void reduce_mid_kernel(ReduceMidArgs g) {
   typedef typename RfVec<T, VEC>::type V;
   typedef typename RfRun<COMB>::type A;
   __shared__ A part[4];
-  const int64_t first = (int64_t)blockIdx.y * g.per_slice;
-  const int64_t last = first + g.per_slice < g.r1 ? first + g.per_slice : g.r1;
-  const uint32_t count = (uint32_t)((last - first) * g.r2);
-  const RF_AS1 V *src = (const RF_AS1 V *)g.x + (first * g.k + blockIdx.x) * (int64_t)g.r2;
+  uint32_t count = (uint32_t)g.per_slice, begin = 0; // < 2^31, < 2^24
+  const RF_AS1 V *src = (const RF_AS1 V *)g.x + blockIdx.x * (int64_t)g.r2;
+  if constexpr (SLICED) {
+    const int64_t total = g.r1 * g.r2, first = (int64_t)blockIdx.y * g.per_slice;
+    count = (uint32_t)(first + g.per_slice < total ? g.per_slice : total - first);
+    const int64_t run0 = first / g.r2;
+    begin = (uint32_t)(first - run0 * g.r2);
+    src += run0 * g.k * g.r2;
+  }
   const int64_t pitch = (int64_t)g.k * g.r2;
   A acc = rf_identity<COMB>();
   auto at = [&](uint32_t i) {
+    if constexpr (SLICED)
+      i += begin;
     uint32_t q = __umulhi(i, g.magic_r2); // (floor estimate: at most one too small)
     uint32_t rem = i - q * (uint32_t)g.r2;
     if (rem >= (uint32_t)g.r2)
@@ -423,13 +435,16 @@ __global__ __launch_bounds__(256) void reduce_mid_kernel(ReduceMidArgs g) {
         acc = rf_comb_nan<COMB>(acc, rf_map<MAP>(f[i]));
     }
   };
+  constexpr uint32_t U = SLICED && VEC == 1 ? 8 : 4; // loads in flight per thread
   uint32_t i = threadIdx.x;
-  for (; i + 768 < count; i += 1024) {
-    const V v0 = at(i), v1 = at(i + 256), v2 = at(i + 512), v3 = at(i + 768);
-    add(v0);
-    add(v1);
-    add(v2);
-    add(v3);
+  for (; i + (U - 1) * 256 < count; i += U * 256) {
+    V v[U];
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u)
+      v[u] = at(i + u * 256);
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u)
+      add(v[u]);
   }
   for (; i < count; i += 256)
     add(at(i));
@@ -442,40 +457,43 @@ __global__ __launch_bounds__(256) void reduce_mid_kernel(ReduceMidArgs g) {
   if (threadIdx.x == 0) {
     const float v = (float)rf_run_comb<COMB, A>(rf_run_comb<COMB, A>(part[0], part[1]),
                                                 rf_run_comb<COMB, A>(part[2], part[3]));
-    if (g.partial)
+    if constexpr (SLICED)
       g.partial[(int64_t)blockIdx.y * g.k + blockIdx.x] = v;
     else
       rf_store(g, blockIdx.x, v);
   }
 }
 
-// Combines the slices: 16 columns per workgroup, 16 threads per column.
+// Combines the slices: 2^cols_log2 columns per workgroup, the other threads of a column
+// over its slices.
 template <int COMB>
-__global__ __launch_bounds__(256) void reduce_mid_finish_kernel(ReduceMidArgs g) {
+__global__ __launch_bounds__(256) void reduce_mid_finish_kernel(ReduceMidArgs g, int cols_log2) {
   typedef typename RfRun<COMB>::type A;
-  __shared__ A lds[16][17];
-  const int cl = threadIdx.x & 15, sl = threadIdx.x >> 4;
-  const int64_t c = (int64_t)blockIdx.x * 16 + cl;
+  __shared__ A lds[256];
+  const int cols = 1 << cols_log2, per = 256 >> cols_log2;
+  const int cl = threadIdx.x & (cols - 1), sl = threadIdx.x >> cols_log2;
+  const int64_t c = (int64_t)blockIdx.x * cols + cl;
   A acc = rf_identity<COMB>();
   if (c < g.k) {
     const RF_AS1 float *p = (const RF_AS1 float *)g.partial + c;
     int s = sl;
-    for (; s + 48 < g.slices; s += 64) {
-      const float v0 = p[(int64_t)s * g.k], v1 = p[(int64_t)(s + 16) * g.k];
-      const float v2 = p[(int64_t)(s + 32) * g.k], v3 = p[(int64_t)(s + 48) * g.k];
+    for (; s + 3 * per < g.slices; s += 4 * per) {
+      const float v0 = p[(int64_t)s * g.k], v1 = p[(int64_t)(s + per) * g.k];
+      const float v2 = p[(int64_t)(s + 2 * per) * g.k], v3 = p[(int64_t)(s + 3 * per) * g.k];
       acc = rf_run_comb<COMB, A>(
           rf_run_comb<COMB, A>(rf_run_comb<COMB, A>(rf_run_comb<COMB, A>(acc, v0), v1), v2), v3);
     }
-    for (; s < g.slices; s += 16)
+    for (; s < g.slices; s += per)
       acc = rf_run_comb<COMB, A>(acc, p[(int64_t)s * g.k]);
   }
-  lds[sl][cl] = acc;
-  __syncthreads();
-  if (sl == 0 && c < g.k) {
-    for (int s = 1; s < 16; ++s)
-      acc = rf_run_comb<COMB, A>(acc, lds[s][cl]);
-    rf_store(g, c, (float)acc);
+  lds[threadIdx.x] = acc;
+  for (int s = 128; s >= cols; s >>= 1) {
+    __syncthreads();
+    if ((int)threadIdx.x < s)
+      lds[threadIdx.x] = rf_run_comb<COMB, A>(lds[threadIdx.x], lds[threadIdx.x + s]);
   }
+  if (sl == 0 && c < g.k)
+    rf_store(g, c, (float)lds[threadIdx.x]);
 }
 
 struct ReducePlan {
@@ -575,38 +593,52 @@ ReducePlan make_plan(const fhip_reduce_desc *d) {
   return p;
 }
 
-// Slices of r1 and launches of the column kernels (see ReduceMidArgs): about
-// four workgroups per compute unit over all columns, at most 256 slices (the
-// combining kernel reads slices * k values), and at least some 16 rows (r2 = 1)
-// or 2048 elements per workgroup.
+// Slices of the reduced range and launches of the column kernels (see ReduceMidArgs):
+// about four workgroups per compute unit over all columns, at least 2048 elements or
+// eight rounds of rows (r2 == 1) each, at most 1024 (256 of more than 16 results: the
+// combining kernel reads slices * k values).
+//
+// Slices of r1 alone left [2, 3, 1024, 1024] f32 -> 3 sums to six workgroups (59.5 us on
+// the strided kernel, 74 so) and a sum of 10 000 001 values to one (88 -> 3670 us).
 template <typename T, int MAP, int COMB>
 int launch_mid(fhip_ctx *ctx, const ReducePlan &p, ReduceMidArgs g) {
   constexpr int VEC = 16 / (int)sizeof(T);
   const bool cols = p.r2 == 1;
   const bool vec = ((uintptr_t)g.x & 15) == 0 && (cols ? p.k % VEC == 0 : p.r2 % VEC == 0);
   int tx_log2 = 0;
-  int64_t groups = p.k, most;
+  int64_t groups = p.k, most, range = p.r1;
   if (cols) {
     const int64_t cv = vec ? p.k / VEC : p.k;
     while ((1ll << tx_log2) < cv && tx_log2 < 8)
       ++tx_log2;
-    groups = (cv + (1ll << tx_log2) - 1) >> tx_log2;
     most = p.r1 / ((256 >> tx_log2) * 8);
+    // Few rows: one slice, and one launch, on narrow workgroups (eight vectors at least,
+    // four rows per thread) unless there are 512 wide ones ([64, 2048] bf16 maxima: strided
+    // 6.7 us, eight slices 8.4; [8, 7, 7] x 512 sums 6.7, so 4.4).
+    if (p.r1 <= 1024) {
+      while (tx_log2 > 3 && (cv >> tx_log2) < 512 && (512 >> tx_log2) * 4 <= p.r1)
+        --tx_log2;
+      most = 1;
+    }
+    groups = (cv + (1ll << tx_log2) - 1) >> tx_log2;
   } else {
     g.r2 = (int32_t)(vec ? p.r2 / VEC : p.r2);
     g.magic_r2 = g.r2 == 1 ? 0xffffffffu : (uint32_t)((1ull << 32) / (uint32_t)g.r2);
     most = p.r1 * p.r2 / 2048;
-    most = most < p.r1 ? most : p.r1;
+    range = p.r1 * g.r2;
   }
   int64_t slices = 4 * (int64_t)(ctx->num_cus > 0 ? ctx->num_cus : 256) / groups;
   slices = slices < most ? slices : most;
-  slices = slices < 256 ? slices : 256;
+  const int64_t cap = p.k <= 16 ? 1024 : 256;
+  slices = slices < cap ? slices : cap;
   // (a slice's flat index is 32-bit)
-  const int64_t least = (p.r1 * p.r2) / (1ll << 30) + 1;
+  const int64_t least = range / (1ll << 30) + 1;
   slices = slices > least ? slices : least;
-  g.per_slice = (p.r1 + slices - 1) / slices;
-  slices = (p.r1 + g.per_slice - 1) / g.per_slice;
-  if (slices > 65535 || g.per_slice * p.r2 >= (1ll << 31))
+  if (slices > 1 && !fhip_ctx_scratch_ready(ctx, (size_t)(slices * p.k) * sizeof(float)))
+    slices = least; // (usually one: no scratch)
+  g.per_slice = (range + slices - 1) / slices;
+  slices = (range + g.per_slice - 1) / g.per_slice;
+  if (slices > 65535 || g.per_slice >= (1ll << 31))
     return -1; // (the strided kernel's)
   g.slices = (int32_t)slices;
   if (slices > 1) {
@@ -624,13 +656,21 @@ int launch_mid(fhip_ctx *ctx, const ReducePlan &p, ReduceMidArgs g) {
     hipLaunchKernelGGL((reduce_cols_kernel<T, MAP, COMB, VEC>), grid, dim3(256), 0, ctx->stream, g, tx_log2);
   else if (cols)
     hipLaunchKernelGGL((reduce_cols_kernel<T, MAP, COMB, 1>), grid, dim3(256), 0, ctx->stream, g, tx_log2);
-  else if (vec)
-    hipLaunchKernelGGL((reduce_mid_kernel<T, MAP, COMB, VEC>), grid, dim3(256), 0, ctx->stream, g);
-  else
-    hipLaunchKernelGGL((reduce_mid_kernel<T, MAP, COMB, 1>), grid, dim3(256), 0, ctx->stream, g);
-  if (slices > 1)
-    hipLaunchKernelGGL(reduce_mid_finish_kernel<COMB>, dim3((unsigned)((p.k + 15) / 16)), dim3(256),
-                       0, ctx->stream, g);
+  else {
+    auto kernel = slices > 1 ? (vec ? reduce_mid_kernel<T, MAP, COMB, VEC, true>
+                                    : reduce_mid_kernel<T, MAP, COMB, 1, true>)
+                             : (vec ? reduce_mid_kernel<T, MAP, COMB, VEC, false>
+                                    : reduce_mid_kernel<T, MAP, COMB, 1, false>);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, ctx->stream, g);
+  }
+  if (slices > 1) {
+    int cols_log2 = 0;
+    while ((1 << cols_log2) < p.k && cols_log2 < 4)
+      ++cols_log2;
+    hipLaunchKernelGGL(reduce_mid_finish_kernel<COMB>,
+                       dim3((unsigned)((p.k + (1ll << cols_log2) - 1) >> cols_log2)), dim3(256), 0,
+                       ctx->stream, g, cols_log2);
+  }
   FHIP_HIP_CHECK(ctx, hipGetLastError());
   return 0;
 }

@@ -42,6 +42,27 @@ def _matmul(torch):
     return a, out, lambda c: c.matmul(d, a.data_ptr(), b.data_ptr(), out.data_ptr()), 2e-2
 
 
+def _reduce(torch, channels_last):
+    dims = [8, 24, 50, 50]
+    x = torch.randn(dims, device="cuda")
+    if channels_last:
+        x = x.contiguous(memory_format=torch.channels_last)
+    out = torch.empty(24, device="cuda")
+    d = capi.ReduceDesc()
+    d.x = capi.TensorDesc.make(dims, list(x.stride()), capi.FLOAT)
+    d.y = capi.TensorDesc.make([1, 24, 1, 1], [24, 1, 1, 1], capi.FLOAT)
+    d.mode = capi.RED["AVG"]
+    return x, out, lambda c: c.reduce(d, x.data_ptr(), out.data_ptr()), 1e-5
+
+
+def _bias_gradient(torch):
+    return _reduce(torch, True)
+
+
+def _channel_means(torch):
+    return _reduce(torch, False)
+
+
 @pytest.mark.parametrize("make", [_norm, _sdpa, _matmul])
 def test_replay_after_scratch_has_grown(make):
     import torch
@@ -87,7 +108,7 @@ def test_replay_after_scratch_has_grown(make):
         other.close()
 
 
-@pytest.mark.parametrize("make", [_norm, _sdpa, _matmul])
+@pytest.mark.parametrize("make", [_norm, _sdpa, _matmul, _bias_gradient, _channel_means])
 def test_first_call_under_capture(make):
     import torch
     torch.manual_seed(1)

@@ -169,3 +169,32 @@ def test_mean_of_equal_values_is_that_value(ctx, dtype, kernel, n):
     out = run(ctx, x, odims, "AVG", y_dtype=capi.FLOAT, expect_tuned=kernel == "reduce_rows").logical()
     assert ctx.last_kernel().startswith(kernel), ctx.last_kernel()
     assert (out == 1).all()
+
+
+@pytest.mark.parametrize("mode", ["SUM", "AVG", "MAX", "AMAX", "MUL"])
+@pytest.mark.parametrize("dtype", [capi.FLOAT, capi.BFLOAT16])
+@pytest.mark.parametrize("dims,odims,least", [
+    ([2, 3, 256, 256], [1, 3, 1, 1], 60),  # two long runs per result: slices end inside them
+    ([1, 3, 129, 131], [1, 3, 1, 1], 8),   # one run of odd length per result
+    ([1, 100003], [1, 1], 48),             # everything, one run
+    ([3, 5, 4099], [1, 5, 1], 6),          # slices that start at odd elements of a run
+    ([4, 20, 2050], [1, 20, 1], 4),
+])
+def test_reduce_slices_of_few_long_runs(ctx, mode, dtype, dims, odims, least):
+    x = make_x(69, dims, dtype, mode)
+    if mode == "MUL":  # ((1 + 0.02 r)^100000 is out of range)
+        x = HT.from_logical(1 + 2e-3 * rand(69, 0, dims), dtype)
+    out = run(ctx, x, odims, mode, y_dtype=capi.FLOAT, expect_tuned=False)
+    kernel, slices = ctx.last_kernel().split(" slices=")
+    assert kernel == "reduce_mid" and int(slices) >= least, ctx.last_kernel()
+    ref = oracle.reduction(x.logical(), odims, capi.RED[mode])
+    assert_close(out.logical(), ref, capi.FLOAT, f"{mode} {dims}", rtol=1e-4 if dtype == capi.FLOAT else 2e-2)
+
+
+@pytest.mark.parametrize("mode", ["SUM", "MAX"])
+@pytest.mark.parametrize("dims", [[2, 8], [1024, 40], [1025, 40], [64, 2048], [700, 16392], [33, 4101]])
+def test_reduce_few_rows_in_one_launch(ctx, mode, dims):
+    x = make_x(70, dims, capi.BFLOAT16, mode)
+    out = run(ctx, x, [1, dims[1]], mode, y_dtype=capi.FLOAT, expect_tuned=False)
+    assert (ctx.last_kernel() == "reduce_cols slices=1") == (dims[0] <= 1024), ctx.last_kernel()
+    assert_close(out.logical(), oracle.reduction(x.logical(), [1, dims[1]], capi.RED[mode]), capi.FLOAT, rtol=2e-2)
