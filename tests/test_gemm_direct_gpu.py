@@ -1,6 +1,8 @@
 """Direct matrix-product kernels (fragments straight from global memory) vs the
 oracle, at the sizes where they can go wrong: one row, tile edges, K tails of
 every length class, rows that start on odd elements, batches, split K."""
+import math
+
 import numpy as np
 import pytest
 
@@ -109,3 +111,37 @@ def test_direct_gelu_of_infinities(ctx, dtype):
     got = out.logical()
     assert (got[:, 3] == np.inf).all() and np.isnan(got[:, 9]).all()
     assert np.isfinite(np.delete(got, [3, 9], axis=1)).all()
+
+
+@pytest.mark.parametrize("dtype", [capi.BFLOAT16, capi.HALF])
+@pytest.mark.parametrize("fused", [True, False])
+def test_gelu_rounds_once(ctx, dtype, fused):
+    # every value of the type from -13 to 13, as the bias of an empty product or as the input
+    # of the pointwise operation: half a unit in the last place is the result's own rounding,
+    # 0.01 what the function and the hardware's exp2 and reciprocal add (measured 0.003)
+    bits = np.arange(1 << 16, dtype=np.uint16)
+    v = oracle.dequantize(bits.view(oracle.storage_dtype(dtype)), dtype)
+    x = v[np.isfinite(v) & (np.abs(v) <= 13)]
+    x = x[:len(x) // 8 * 8].astype(np.float64).reshape(1, -1)
+    t = HT.from_logical(x, dtype)
+    if fused:
+        a = make_operand(95, 0, 1, 16, dtype, False)
+        b = HT.from_logical(np.zeros([16, x.size]), dtype)
+        epi = [capi.epilogue_op(capi.PW["ADD"], capi.FLOAT, operand=t.desc(), operand_index=0),
+               capi.epilogue_op(capi.PW["GELU_FWD"], dtype)]
+        got = run(ctx, a, b, capi.FLOAT, out_dtype=dtype, epilogue=epi, epi_tensors=[t])[0].logical()
+    else:
+        out = HT.empty([1, x.size], dtype)
+        d = capi.PointwiseDesc()
+        d.mode, d.num_inputs, d.params = capi.PW["GELU_FWD"], 1, capi.PointwiseParams.default()
+        d.in_[0], d.out = t.desc(), out.desc()
+        bi, bo = t.upload(ctx), out.upload(ctx)
+        ctx.pointwise(d, bi, None, None, bo)
+        assert ctx.last_kernel().startswith("pointwise_fast"), ctx.last_kernel()
+        got = out.fetch(ctx, bo).logical()
+    exact = np.array([0.5 * e * math.erfc(-e / math.sqrt(2)) for e in x.ravel()]).reshape(x.shape)
+    digits, least = (10, -14) if dtype == capi.HALF else (7, -126)
+    size = np.where(exact == 0, 1e-300, np.abs(exact))
+    ulp = np.exp2(np.maximum(np.floor(np.log2(size)), least) - digits)
+    worst = np.abs(got - exact) / ulp
+    assert worst.max() <= 0.51, (float(worst.max()), float(x.ravel()[worst.argmax()]))
