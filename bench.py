@@ -60,7 +60,7 @@ TRAFFIC = {
 # target), the kernel variant that must have run (prefix of fhip_last_kernel),
 # and the driver command that times the same problem through Graph::execute.
 CONFIGS = {
-    "C1": ("matmul_f32_1x256x512x256", None, "matmul_f32_splitk",
+    "C1": ("matmul_f32_1x256x512x256", None, "gemm_direct ",
            "matmul -M 256 -N 256 -K 512 --a_type f32 --b_type f32 --out_type f32"),
     "C2": (None, 0.70, "rownorm chunks=",
            "rmsnorm -X 8192x4096 -t bf16 -e 1e-6 --mul 0.5"),

@@ -134,11 +134,7 @@ int fhip_direct_matmul(fhip_ctx *ctx, const fhip_matmul_desc *d, const void *a, 
     else if (fhip_ctx_scratch(ctx, bytes, &g.partial) != 0)
       return 1;
   }
-  // (f32 products that split K over the wavefronts of a tile keep that name)
-  if (p.kind == GK_F32)
-    fhip_note_kernel(ctx, "matmul_f32_splitk");
-  else
-    fhip_note_kernel(ctx, "gemm_direct %dx%d waves=%d split=%d", 16 * p.mt, 16 * p.nt, p.waves, g.splits);
+  fhip_note_kernel(ctx, "gemm_direct %dx%d waves=%d split=%d", 16 * p.mt, 16 * p.nt, p.waves, g.splits);
   switch (p.kind) {
   case GK_BF16: return direct_launch_bf16(ctx, p, g, batch);
   case GK_F16: return direct_launch_f16(ctx, p, g, batch);

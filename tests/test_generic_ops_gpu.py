@@ -36,9 +36,8 @@ def test_matmul_config1_f32(ctx):
     b = HT.from_logical(rand(1, 1, [1, 512, 256], "uniform"), capi.FLOAT)
     out = run_matmul(ctx, a, b, capi.FLOAT)
     assert_close(out.logical(), oracle.matmul(a.logical(), b.logical()), capi.FLOAT)
-    # 16 tiles of 64 x 64: the f32 matrix-instruction kernel that splits K
-    # over the wavefronts of a 32 x 32 tile
-    assert ctx.last_kernel() == "matmul_f32_splitk", ctx.last_kernel()
+    # few tiles: the direct kernel, whose wavefronts split K
+    assert ctx.last_kernel().startswith("gemm_direct "), ctx.last_kernel()
 
 
 @pytest.mark.parametrize("transpose_b", [False, True])
@@ -91,6 +90,30 @@ def test_matmul_f32_mfma_tiles(ctx, m, n, k, layout):
     out = run_matmul(ctx, a, b, capi.FLOAT, epilogue=epi, epi_tensors=[bias])
     ref = np.maximum(oracle.matmul(a.logical(), b.logical()) + bias.logical(), 0.0)
     assert_close(out.logical(), ref, capi.FLOAT, f"{m}x{n}x{k} {layout}")
+
+
+@pytest.mark.parametrize("m,n,k,kernel", [
+    (45, 70, 200, "matmul_f32_splitk"), (33, 31, 129, "matmul_f32_splitk"),
+    (64, 64, 1000, "matmul_f32_splitk"), (300, 500, 136, "matmul_f32_splitk"),
+    (45, 70, 40, "matmul_f32_tiled"), (130, 260, 64, "matmul_f32_tiled"),
+    (700, 900, 136, "matmul_f32_tiled"),
+])
+@pytest.mark.parametrize("form", ["mixed types", "no contiguous dim", "rank 4"])
+def test_matmul_f32_tiles_of_general_operands(ctx, m, n, k, kernel, form):
+    # what the direct kernel does not take: K split over the wavefronts of 32 x 32 tiles
+    # where 64 x 64 ones are few, those otherwise
+    lead = [1, 1] if form == "rank 4" else []
+    b_st = [2 * n + 3, 2] if form == "no contiguous dim" else None
+    b_dt = capi.BFLOAT16 if form == "mixed types" else capi.FLOAT
+    a = HT.from_logical(rand(9, 0, lead + [m, k]), capi.FLOAT)
+    b = HT.from_logical(rand(9, 1, lead + [k, n]), b_dt, b_st)
+    bias = HT.from_logical(rand(9, 2, lead + [1, n]), capi.FLOAT)
+    epi = [capi.epilogue_op(capi.PW["ADD"], capi.FLOAT, operand=bias.desc()),
+           capi.epilogue_op(capi.PW["RELU_FWD"], capi.FLOAT)]
+    out = run_matmul(ctx, a, b, capi.FLOAT, epilogue=epi, epi_tensors=[bias])
+    assert ctx.last_kernel() == kernel, ctx.last_kernel()
+    ref = np.maximum(oracle.matmul(a.logical(), b.logical()) + bias.logical(), 0.0)
+    assert_close(out.logical(), ref, capi.FLOAT, f"{m}x{n}x{k} {form}")
 
 
 def test_matmul_strided_operands_and_output(ctx):
