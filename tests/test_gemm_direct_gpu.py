@@ -71,6 +71,32 @@ def test_direct_split_k(ctx, dtype, tb, m):
     check(out.logical(), ref_matmul(a, b), dtype)
 
 
+@pytest.mark.parametrize("dtype,ta,tb,m,n,batch,line", [
+    (capi.FLOAT, False, False, 600, 1100, 1, 150),  # 180 tiles
+    (capi.FLOAT, True, False, 33, 65, 100, 150),    # 200, a second one for a row and a column
+    (capi.FLOAT, False, True, 1500, 1450, 1, 185),  # 552, both K-contiguous
+    (capi.HALF, False, False, 1100, 1200, 1, 24),
+    (capi.BFLOAT16, True, True, 1100, 1200, 1, 50),
+    (capi.HALF, False, True, 600, 1100, 1, 34),
+])
+def test_short_k_takes_the_f32_tiles(ctx, dtype, ta, tb, m, n, batch, line):
+    # both sides of the rule's line; K odd to its slices on either
+    for k, direct in ((9, False), (line - 1, False), (line, True)):
+        a = make_operand(96, 0, m, k, dtype, ta, batch=batch if batch > 1 else None)
+        b = make_operand(96, 1, k, n, dtype, tb)
+        if batch > 1:
+            b = make_operand(96, 1, k, n, dtype, tb, batch=1)
+        out = HT.empty(([batch] if batch > 1 else []) + [m, n], capi.FLOAT)
+        d = capi.MatmulDesc()
+        d.a, d.b, d.c, d.out, d.out_dtype = a.desc(), b.desc(), out.desc(), out.desc(), capi.FLOAT
+        d.epilogue = capi.make_epilogue([])
+        da, db, do = a.upload(ctx), b.upload(ctx), out.upload(ctx)
+        ctx.matmul(d, da, db, do)
+        name = ctx.last_kernel()
+        assert name.startswith("gemm_direct" if direct else "matmul_f32_tiled"), (k, name)
+        check(out.fetch(ctx, do).logical(), ref_matmul(a, b), dtype)
+
+
 @pytest.mark.parametrize("dtype", [capi.FLOAT, capi.HALF, capi.INT8])
 def test_direct_batched(ctx, dtype):
     a = make_operand(92, 0, 19, 45, dtype, False, batch=3)
