@@ -313,19 +313,41 @@ __global__ __launch_bounds__(kCfThreads) void conv_few_wgrad_kernel(CfArgs g, co
     auto spend = [&](const float (&b)[KT][4], int px) {
       const int4 at = *(const int4 *)(pixtab + px);
       const int off[4] = {at.x, at.y, at.z, at.w};
+      float xv[JT][4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float xv[JT];
+      for (int v = 0; v < JT; ++v)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          xv[v][i] = xl[off[i] + joff[v]];
+          xv[v][i] = px + i < np ? xv[v][i] : 0.f;
+        }
+      if constexpr (sizeof(T) == 4) {
+        // The 16 products of a group from zero, then one addition to the running sum: a
+        // chain of roundings as many groups long as this wavefront sees, not as many
+        // pixels.  (In one chain N64 3 -> 32, 128 x 128, 3 x 3 was 4.1e-7 from the exact
+        // gradient, 1.6e-7 so, the kernel of one pixel per thread 2.4e-7; 49.4 -> 51.3 us.
+        // A gradient rounded to 16 bits does not show either.)
 #pragma unroll
         for (int v = 0; v < JT; ++v) {
-          xv[v] = xl[off[i] + joff[v]];
-          xv[v] = px + i < np ? xv[v] : 0.f;
-        }
+          f32x4 part[KT];
 #pragma unroll
-        for (int v = 0; v < JT; ++v)
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int u = 0; u < KT; ++u)
+              part[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                  b[u][i], xv[v][i], i == 0 ? f32x4{0, 0, 0, 0} : part[u], 0, 0, 0);
 #pragma unroll
           for (int u = 0; u < KT; ++u)
-            acc[u][v] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[u][i], xv[v], acc[u][v], 0, 0, 0);
+            acc[u][v] += part[u];
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int v = 0; v < JT; ++v)
+#pragma unroll
+            for (int u = 0; u < KT; ++u)
+              acc[u][v] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[u][i], xv[v][i], acc[u][v], 0, 0, 0);
       }
     };
     // (groups of 16 pixels, the wavefronts in turn, the next group's DY in flight)

@@ -59,3 +59,27 @@ def test_conv_few_channels_vs_oracle(ctx, case, dtype):
     assert ctx.last_kernel().startswith("conv_few wgrad"), ctx.last_kernel()
     assert_close(dw.logical(), oracle.conv_wgrad(dy.logical(), x.logical(), case["w"], *geom),
                  dtype, f"wgrad {case}")
+
+
+@pytest.mark.parametrize("x,w,pad", [
+    ([64, 3, 64, 64], [32, 3, 3, 3], [1, 1]),   # many bands per workgroup
+    ([8, 1, 28, 28], [16, 1, 5, 5], [2, 2]),    # one
+    ([4, 12, 16, 16], [64, 12, 3, 3], [1, 1]),  # the widest tiles
+])
+def test_weight_gradient_rounds_in_short_chains(ctx, x, w, pad):
+    # Groups of 16 pixels, a wavefront's groups and the workgroups' sums are chains of
+    # their own, at most 64 roundings each; a chain of n adds about sqrt(n) / 3 * 2^-24 of
+    # a random sum's size (one chain of all a workgroup's pixels reached 4e-7)
+    geom = (pad, [1, 1], [1, 1])
+    xs = HT.from_logical(rand(52, 0, x), capi.FLOAT)
+    dy = HT.from_logical(rand(52, 1, oracle.conv_output_dims(x, w, *geom)), capi.FLOAT)
+    dw = run_conv_wgrad(ctx, dy, xs, w, *geom, capi.FLOAT, False, tuned=None).logical()
+    assert ctx.last_kernel().startswith("conv_few wgrad"), ctx.last_kernel()
+    xp = np.pad(xs.logical().astype(np.float64), [(0, 0), (0, 0), (pad[0],) * 2, (pad[1],) * 2])
+    g = dy.logical().astype(np.float64)
+    p, q = g.shape[2:]
+    ref = np.empty(w)
+    for r in range(w[2]):
+        for s in range(w[3]):
+            ref[:, :, r, s] = np.einsum("nkpq,ncpq->kc", g, xp[:, :, r:r + p, s:s + q], optimize=True)
+    assert np.linalg.norm(dw - ref) <= 8 / 3 * 2.0 ** -24 * np.linalg.norm(ref)
