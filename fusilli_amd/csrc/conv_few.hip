@@ -43,7 +43,7 @@ struct CfArgs {
   int64_t xs[4], ws[4], ys[4]; // element strides; ys: Y (gradients) or OUT (forward)
   int32_t y_dt, o_dt;          // forward: rounding of the sum, type of OUT
   int32_t lw;                  // columns of the staged X
-  uint32_t lw_magic, rows_magic, q_magic;
+  uint32_t lw_magic, rows_magic, q_magic, rs_magic, s_magic;
   int32_t xrows;               // most rows of X staged at once
   int32_t tiles;               // forward: workgroups per image; gradients: bands
   int32_t band;                // output (data gradient: input) rows per band
@@ -85,9 +85,8 @@ __device__ __forceinline__ void cf_stage_x(const CfArgs &g, const T *x, int row0
 
 // where pair j = (channel, tap) lies in the staged X / in the filter
 __device__ __forceinline__ int cf_pair(const CfArgs &g, int j, int *filter) {
-  const int rs = g.R * g.S;
-  const int c = j / rs, t = j - c * rs;
-  const int r = t / g.S, s = t - r * g.S;
+  const int c = cf_div(j, g.rs_magic), t = j - c * g.R * g.S;
+  const int r = cf_div(t, g.s_magic), s = t - r * g.S;
   *filter = c * (int)g.ws[1] + r * (int)g.ws[2] + s * (int)g.ws[3];
   return (c * g.xrows + r * g.dil_h) * g.lw + s * g.dil_w;
 }
@@ -111,44 +110,73 @@ template <typename T, int KT>
 __global__ __launch_bounds__(kCfThreads) void conv_few_fprop_kernel(CfArgs g, const T *x,
                                                                     const T *w, void *out) {
   constexpr int KP = KT * 16 + (KT % 2 ? 0 : 16); // (two rows of pairs in different banks)
+  constexpr int K16 = KT * 16;
   extern __shared__ __attribute__((aligned(16))) float smem[];
   const int j4 = (g.J + 3) & ~3;
-  float *wl = smem;                 // [pair][output channel]
-  int *tab = (int *)(wl + j4 * KP); // where a pair's X lies, then its filter offset
-  int *woff = tab + j4;
-  float *xl = (float *)(woff + j4);
+  float *wl = smem;                            // [pair][output channel]
+  float *ops = wl + j4 * KP;                   // [fused operation][output channel]
+  int *tab = (int *)(ops + FHIP_MAX_EPILOGUE * K16); // where a pair's X lies
+  float *xl = (float *)(tab + j4);
   const int tid = threadIdx.x, l = tid & 63, wave = tid >> 6;
-  const int k0 = blockIdx.y * KT * 16;
+  const int k0 = blockIdx.y * K16;
   const int n = blockIdx.x / g.tiles, t0 = (blockIdx.x % g.tiles) * kCfThreads;
   const int pq = g.P * g.Q;
   const int t1 = t0 + kCfThreads < pq ? t0 + kCfThreads : pq;
   const int p0 = t0 / g.Q, p1 = (t1 - 1) / g.Q;
+  // Everything a workgroup reads is requested before the first wait: the filter, the fused
+  // operations' values per channel, X (one after another: 0.2 to 0.5 us more).
+  constexpr int kBatch = 8;
+  const int kk = tid % K16, jt = tid / K16; // this thread's channel, its first pair
+  const bool k_in = k0 + kk < g.K;
+  auto weights = [&](int j0, float (&v)[kBatch]) {
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const int j = j0 + i * (kCfThreads / K16);
+      const bool in = j < g.J && k_in;
+      int f;
+      cf_pair(g, in ? j : 0, &f);
+      // (the load is issued either way: a branch would wait for every value)
+      const float t = (float)w[in ? (k0 + kk) * g.ws[0] + f : 0];
+      v[i] = in ? t : 0.f;
+    }
+  };
+  auto put_weights = [&](int j0, const float (&v)[kBatch]) {
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const int j = j0 + i * (kCfThreads / K16);
+      if (j < j4)
+        wl[j * KP + kk] = v[i];
+    }
+  };
+  float wv0[kBatch], op[FHIP_MAX_EPILOGUE];
+  weights(jt, wv0);
+#pragma unroll
+  for (int e = 0; e < FHIP_MAX_EPILOGUE; ++e) {
+    op[e] = 0.f;
+    if (e < g.epi.count && g.epi.op[e].kind != FHIP_OPERAND_NONE) { // (uniform)
+      const DevEpiOp &o = g.epi.op[e];
+      op[e] = o.kind == FHIP_OPERAND_SCALAR
+                  ? o.scalar
+                  : fhip_load<float>(o.ptr, o.operand_dtype,
+                                     n * o.stride[0] + (k_in ? k0 + kk : g.K - 1) * o.stride[1]);
+    }
+  }
   for (int j = tid; j < j4; j += kCfThreads) {
-    int f = 0, o = 0;
-    if (j < g.J)
-      o = cf_pair(g, j, &f);
-    tab[j] = o, woff[j] = f;
+    int f;
+    tab[j] = j < g.J ? cf_pair(g, j, &f) : 0;
   }
   cf_stage_x(g, x + n * g.xs[0], p0 * g.str_h - g.pad_h,
              (p1 - p0) * g.str_h + (g.R - 1) * g.dil_h + 1, xl);
-  __syncthreads();
-  for (int e0 = tid; e0 < j4 * KT * 16; e0 += 8 * kCfThreads) {
-    float v[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int e = e0 + i * kCfThreads, kk = e % (KT * 16);
-      const int j = e / (KT * 16) < j4 ? e / (KT * 16) : 0;
-      const bool in = j < g.J && k0 + kk < g.K;
-      const float t = (float)w[in ? (k0 + kk) * g.ws[0] + woff[j] : 0];
-      v[i] = in ? t : 0.f;
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int e = e0 + i * kCfThreads;
-      if (e < j4 * KT * 16)
-        wl[e / (KT * 16) * KP + e % (KT * 16)] = v[i];
-    }
+  put_weights(jt, wv0);
+  for (int j0 = jt + kBatch * (kCfThreads / K16); j0 < j4; j0 += kBatch * (kCfThreads / K16)) {
+    float v[kBatch];
+    weights(j0, v);
+    put_weights(j0, v);
   }
+  if (tid < K16)
+#pragma unroll
+    for (int e = 0; e < FHIP_MAX_EPILOGUE; ++e)
+      ops[e * K16 + tid] = op[e];
   __syncthreads();
   const int first = t0 + wave * 64;
   if (first >= t1)
@@ -168,8 +196,10 @@ __global__ __launch_bounds__(kCfThreads) void conv_few_fprop_kernel(CfArgs g, co
 #pragma unroll
     for (int u = 0; u < KT; ++u)
       acc[t][u] = f32x4{0, 0, 0, 0};
+  int next = tab[l >> 4];
   for (int j = l >> 4; j < j4; j += 4) {
-    const int off = tab[j];
+    const int off = next;
+    next = tab[j + 4 < j4 ? j + 4 : j];
     float xv[4], wv[KT];
 #pragma unroll
     for (int u = 0; u < KT; ++u)
@@ -211,10 +241,7 @@ __global__ __launch_bounds__(kCfThreads) void conv_few_fprop_kernel(CfArgs g, co
         fhip_pw_fast_unary_vec<true, 16>(o.mode, v, o.params.swish_beta,
                                          o.result_dtype != FHIP_FLOAT);
       } else {
-        const float s = o.kind == FHIP_OPERAND_SCALAR
-                            ? o.scalar
-                            : fhip_load<float>(o.ptr, o.operand_dtype,
-                                               n * o.stride[0] + k * o.stride[1]);
+        const float s = ops[e * K16 + u * 16 + (l & 15)];
         float other[16];
 #pragma unroll
         for (int i = 0; i < 16; ++i)
@@ -583,6 +610,7 @@ bool cf_args(const fhip_conv_desc *d, const fhip_tensor_desc &y, CfArgs &g) {
   g.K = (int32_t)d->w.dim[0], g.R = (int32_t)d->w.dim[2], g.S = (int32_t)d->w.dim[3];
   g.P = (int32_t)y.dim[2], g.Q = (int32_t)y.dim[3];
   g.J = (int32_t)J;
+  g.rs_magic = cf_magic(g.R * g.S), g.s_magic = cf_magic(g.S);
   g.pad_h = (int32_t)d->padding[0], g.pad_w = (int32_t)d->padding[1];
   g.str_h = (int32_t)d->stride[0], g.str_w = (int32_t)d->stride[1];
   g.dil_h = (int32_t)d->dilation[0], g.dil_w = (int32_t)d->dilation[1];
@@ -642,15 +670,28 @@ int fhip_few_conv_fprop(fhip_ctx *ctx, const fhip_conv_desc *d, const void *x, c
     if (epi.op[i].kind == FHIP_OPERAND_TENSOR &&
         ((g.P > 1 && epi.op[i].stride[2] != 0) || (g.Q > 1 && epi.op[i].stride[3] != 0)))
       return 0; // (operands per channel only)
-  const int kt = g.K > 32 ? 4 : g.K > 16 ? 2 : 1;
-  const int j4 = (g.J + 3) / 4 * 4, kp = kt * 16 + (kt % 2 ? 0 : 16);
-  const int span = (kCfThreads - 1 + g.Q - 1) / g.Q + 1;
-  size_t lds = 0;
-  if (!cf_stage(g, span < g.P ? span : g.P, (int64_t)j4 * (kp + 2), &lds))
-    return 0;
   g.tiles = (int32_t)(((int64_t)g.P * g.Q + kCfThreads - 1) / kCfThreads);
   const int64_t blocks = (int64_t)g.N * g.tiles;
   if ((int64_t)g.P * g.Q >= (1ll << 30) || blocks >= (1ll << 23))
+    return 0;
+  const int j4 = (g.J + 3) / 4 * 4;
+  const int span = (kCfThreads - 1 + g.Q - 1) / g.Q + 1;
+  size_t lds = 0;
+  int kt = g.K > 32 ? 4 : g.K > 16 ? 2 : 1;
+  auto fits = [&]() {
+    const int kp = kt * 16 + (kt % 2 ? 0 : 16);
+    return cf_stage(g, span < g.P ? span : g.P, (int64_t)j4 * (kp + 1) + FHIP_MAX_EPILOGUE * kt * 16, &lds);
+  };
+  if (!fits())
+    return 0;
+  const int64_t cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+  // (few tiles: a workgroup of 64 channels is a long chain of its own, mostly scalar loads
+  // of the fused operations, so fewer channels each until there are two workgroups per
+  // compute unit: N16 3 -> 64, 20 x 20, 3 x 3 f32 64 channels 14.9 us, 16 of them 8.8, the
+  // kernel of one pixel per thread 11.2)
+  while (kt > 1 && blocks * ((g.K + kt * 16 - 1) / (kt * 16)) < 2 * cus)
+    kt /= 2;
+  if (!fits())
     return 0;
   g.y_dt = d->y.dtype, g.o_dt = d->out.dtype;
   g.epi = epi;
@@ -675,7 +716,7 @@ int fhip_few_conv_wgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy, 
   CfArgs g{};
   if (!cf_args(d, d->y, g) || !cf_planes(g) || d->y.dtype != d->x.dtype)
     return 0;
-  const int kt = g.K > 32 ? 4 : g.K > 16 ? 2 : 1;
+  int kt = g.K > 32 ? 4 : g.K > 16 ? 2 : 1;
   const int tiles_j = (g.J + 15) / 16;
   const int jt = tiles_j <= 2 ? 2 : tiles_j <= 3 ? 3 : tiles_j <= 5 ? 5 : 7;
   // bands of about 256 pixels, of equal height
@@ -689,15 +730,19 @@ int fhip_few_conv_wgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy, 
   const int64_t slots = ((int64_t)g.band * g.Q + 15) / 16 * 16;
   if (slots >= (1 << 14) || !cf_stage(g, g.band, slots, &lds))
     return 0;
+  const int64_t items = (int64_t)g.N * g.tiles;
+  const int64_t cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+  // (few bands: their products are a workgroup's longest part, so fewer output channels
+  // each; N4 12 -> 64, 16 x 16, 3 x 3 f32: 20.8 us with 64)
+  while (kt > 1 && items * ((g.K + kt * 16 - 1) / (kt * 16)) < cus)
+    kt /= 2;
   const size_t meet = (size_t)2 * kt * jt * 256 * sizeof(float);
   lds = lds < meet ? meet : lds;
-  const int64_t items = (int64_t)g.N * g.tiles;
   const int kblocks = (g.K + kt * 16 - 1) / (kt * 16);
   const int64_t frags = (int64_t)kblocks * kt * jt * 256;
   if (items >= (1ll << 31) || kblocks > 65535)
     return 0;
   // two workgroups per compute unit, no more than 8 MB of partial sums
-  const int64_t cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
   int64_t runs = 2 * cus / kblocks, most = (8ll << 20) / (frags * 4);
   runs = runs < most ? runs : most;
   runs = runs < items ? runs : items;

@@ -83,3 +83,28 @@ def test_weight_gradient_rounds_in_short_chains(ctx, x, w, pad):
         for s in range(w[3]):
             ref[:, :, r, s] = np.einsum("nkpq,ncpq->kc", g, xp[:, :, r:r + p, s:s + q], optimize=True)
     assert np.linalg.norm(dw - ref) <= 8 / 3 * 2.0 ** -24 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("n,forward,gradient", [(2, 16, 1), (160, 32, 4), (400, 64, 4)])
+def test_few_tiles_take_fewer_channels_each(ctx, n, forward, gradient):
+    # blocks of channels by the number of tiles; operands per channel and per image
+    x = HT.from_logical(np.resize(rand(53, 0, [2, 3, 20, 20]), [n, 3, 20, 20]), capi.FLOAT)
+    w = HT.from_logical(rand(53, 1, [64, 3, 3, 3], std=0.2), capi.FLOAT)
+    bias = HT.from_logical(rand(53, 2, [1, 64, 1, 1]), capi.BFLOAT16)
+    full = np.zeros([n, 64, 1, 1])
+    full[1] = rand(53, 3, [64, 1, 1])
+    image = HT.from_logical(full, capi.FLOAT)  # a value per image and channel
+    epi = [capi.epilogue_op(capi.PW["ADD"], capi.FLOAT, operand=bias.desc(), operand_index=0),
+           capi.epilogue_op(capi.PW["MUL"], capi.FLOAT, scalar=0.5),
+           capi.epilogue_op(capi.PW["ADD"], capi.FLOAT, operand=image.desc(), operand_index=1),
+           capi.epilogue_op(capi.PW["GELU_FWD"], capi.FLOAT)]
+    geom = ([0, 0], [1, 1], [1, 1])
+    y = run_conv(ctx, x, w, *geom, capi.FLOAT, epilogue=epi, epi_tensors=[bias, image])
+    assert ctx.last_kernel() == f"conv_few fprop channels={forward}", ctx.last_kernel()
+    ref = oracle.conv_fprop(x.logical()[:2], w.logical(), *geom) + bias.logical()
+    ref = oracle.pointwise(capi.PW["GELU_FWD"], [ref * 0.5 + full[:2]])
+    assert_close(y.logical()[:2], ref, capi.FLOAT)
+    dy = HT.from_logical(rand(53, 4, [n, 64, 18, 18]), capi.FLOAT)
+    dw = run_conv_wgrad(ctx, dy, x, [64, 3, 3, 3], *geom, capi.FLOAT, False, tuned=None)
+    assert ctx.last_kernel() == f"conv_few wgrad tiles={gradient}x2", ctx.last_kernel()
+    assert_close(dw.logical(), oracle.conv_wgrad(dy.logical(), x.logical(), [64, 3, 3, 3], *geom), capi.FLOAT)
