@@ -352,11 +352,33 @@ void choose_gather(ConvResolved &r, int64_t C) {
   // 41.0; N64 128 -> 64, 28 x 28, 392 tiles: 19.2, 24.7), and gathered tiles over outputs of
   // less than half their width (N62 256 -> 48, 39 x 39: 69 us, here 50).
   const int64_t tiles = ((p.M + p.bm - 1) / p.bm) * ((p.N + p.bn - 1) / p.bn);
-  const bool few = p.ksplit == 1 && tiles < 160 && p.geom.R * p.geom.S > 1;
+  // (the narrow halo tile keeps up sooner: N6 64 -> 16, 54 x 54, 137 tiles 9.6 us, here 10.6)
+  const bool few = p.ksplit == 1 && tiles < (p.halo && p.bn == 64 ? 128 : 160) && p.geom.R * p.geom.S > 1;
   const bool narrow = !p.halo && p.ksplit == 1 && p.N < 64;
-  // (copies that add a seventh at most pay over many tiles: N32 112 -> 384, 26 x 26, 507
-  // tiles: step with the copies 152.7, without 157.0 us; N10 496 -> 128, 45 x 45, 159: 182, 177)
-  const bool copies = r.padded && !((r.Cp - r.C) * 7 <= r.C && tiles >= 400);
+  // Where the copies pay (us, copies and product / here; both kernels on 589 problems):
+  auto copies_pay = [&]() {
+    const double mn = (double)p.M * (double)p.N, more = (double)(r.Cp - r.C) / (double)r.C;
+    // * tiles of 256 rows over reductions of some length, or over very many results: N8 240 ->
+    //   256, 60 x 60 55 / 76; N44 80 -> 256, 1 x 1, 58 x 58 51 / 67 (N11 16 -> 560, 64 x 64 at
+    //   stride 2: 24.7 / 19.0);
+    //   and columns that fill the tiles (N18 224 -> 144, 46 x 46: 100 / 57)
+    const int64_t columns = (p.N + p.bn - 1) / p.bn * p.bn;
+    if (p.bm == 256 && p.bn >= 128 && p.N * 4 >= columns * 3 && (J >= 200 || mn >= 1.6e7))
+      return true;
+    // * many tiles, a seventh of padding at most: N32 112 -> 384, 26 x 26, 507 tiles, step
+    //   153 / 157; N10 496 -> 128, 45 x 45, 159 tiles 182 / 177
+    if (more * 7 <= 1 && tiles >= 400)
+      return true;
+    // * the halo's largest products: N39 216 -> 352, 30 x 18 64.7 / 73.2 (N32 240 -> 256,
+    //   28 x 28 even; N32 136 -> 256 54 / 44)
+    if (p.halo && p.bm == 128 && p.bn == 128 && mn * (double)J >= 1.4e10 && more * 5 <= 1)
+      return true;
+    // * long reductions that fill one round of units with whole tiles: N8 472 -> 128, 60 x 60
+    //   70.8 / 76.4 (N8 312 -> 128 even, 248 -> 128 47 / 45)
+    return !p.halo && p.bm == 128 && p.N % 128 == 0 && tiles >= 190 && tiles <= 256 && J >= 3300 &&
+           more * 11 <= 1;
+  };
+  const bool copies = r.padded && !copies_pay();
   const bool want = copies || knobs.conv_gather > 0 || few || narrow;
   // (whole slices: no parts -- the entry point without scratch gives the same bits)
   if (want)

@@ -59,3 +59,28 @@ def test_conv_gather_vs_oracle(ctx, case, dtype, forced, knobs):
         dx = run_conv_dgrad(ctx, dy, w, case["x"], *geom, dtype, tuned=None)
         assert_close(dx.logical(), oracle.conv_dgrad(dy.logical(), w.logical(), case["x"], *geom),
                      dtype, f"dgrad {case} {ctx.last_kernel()}")
+
+
+@pytest.mark.parametrize("x,w,pad,gathered", [
+    ([8, 200, 60, 60], [256, 200, 3, 3], 1, False),  # tiles of 256 rows, a long reduction
+    ([44, 80, 58, 58], [256, 80, 1, 1], 0, False),   # over very many results
+    ([18, 224, 46, 46], [144, 224, 3, 3], 1, True),  # the same tiles half empty
+    ([11, 16, 64, 64], [560, 16, 3, 3], 1, True),    # a short reduction
+    ([39, 216, 30, 18], [352, 216, 3, 3], 1, False),  # the halo's largest products
+    ([32, 136, 28, 28], [256, 136, 3, 3], 1, True),
+    ([11, 472, 48, 48], [128, 472, 3, 3], 1, False),  # one round of whole tiles
+    ([11, 248, 48, 48], [128, 248, 3, 3], 1, True),
+])
+def test_padded_copies_where_they_pay(ctx, knobs, x, w, pad, gathered):
+    # both sides of the rule, and the same sums (of whole numbers: exact in f32) on either route
+    stride = 2 if x[1] == 16 else 1
+    lay = oracle.channels_last_strides
+    xs = HT.from_logical(np.resize(rand(72, 0, [4099], "int", lo=-3, hi=4), x), capi.BFLOAT16, lay(x))
+    ws = HT.from_logical(np.resize(rand(72, 1, [4093], "int", lo=-3, hi=4), w), capi.BFLOAT16, lay(w))
+    geom = ([pad, pad], [stride, stride], [1, 1])
+    y = run_conv(ctx, xs, ws, *geom, capi.FLOAT, channels_last_out=True).logical()
+    assert ("unpadded" in ctx.last_kernel()) == gathered, ctx.last_kernel()
+    knobs(CONV_GATHER=0 if gathered else 1)
+    z = run_conv(ctx, xs, ws, *geom, capi.FLOAT, channels_last_out=True).logical()
+    assert ("unpadded" in ctx.last_kernel()) != gathered, ctx.last_kernel()
+    assert np.array_equal(y, z)
