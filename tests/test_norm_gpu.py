@@ -361,3 +361,20 @@ def test_norm_rows_of_any_length_vs_oracle(ctx, dtype, rows, cols, layernorm):
         y = np.maximum(oracle.rmsnorm(x.logical(), s.logical(), 1e-6), 0) * mul.logical()
     assert ctx.last_kernel().startswith("rownorm_walk"), ctx.last_kernel()
     assert_close(out.logical(), y, dtype, f"{rows} x {cols}")
+
+
+@pytest.mark.parametrize("dtype", [capi.HALF, capi.FLOAT])
+@pytest.mark.parametrize("rows,cols", [(3000, 65), (2000, 1003), (1000, 3001), (300, 16387)])
+def test_means_of_walked_rows_are_rounded_once(ctx, dtype, rows, cols):
+    # One rounding of a mean is 2^-24 of it at most, 0.43 of that as a 2-norm.  f32 sums in
+    # pairs in front of the 64-bit ones: exact or nearly so for 16-bit values; n f32 ones of
+    # variance 1 in fours round n / 4 times three sums of rms 1.4, 1.4 and 2 by 2^-24 / sqrt(12)
+    # of about their size, 0.41 sqrt(n) 2^-24 against a sum of sqrt(n): up to 0.7 with both,
+    # 0.83 measured.  (A tree of f32 additions: 0.8 to 1.4 and 1.3 to 2.)
+    x = HT.from_logical(rand(42, 0, [rows, cols]), dtype)
+    s = HT.from_logical(rand(42, 1, [1, cols], mean=1.0, std=0.1), dtype)
+    _, mean, _ = run_norm(ctx, x, s, s, eps=1e-5, layernorm=True, stats=True)
+    assert ctx.last_kernel().startswith("rownorm_walk"), ctx.last_kernel()
+    ref = x.logical().astype(np.float64).mean(1)
+    most = 0.6 if dtype == capi.HALF else 1.0
+    assert np.linalg.norm(mean.logical() - ref) <= most * 2.0 ** -24 * np.linalg.norm(ref)
