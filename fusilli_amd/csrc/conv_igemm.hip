@@ -336,7 +336,21 @@ struct ConvResolved {
   size_t x_bytes = 0, w_bytes = 0;
   // runs on the gathered tiles of conv_gather.hip instead (unpadded operands)
   ConvGatherPlan gather{0};
+
+  // parts of a split reduction and their rows' pitch (padded to whole column tiles, which
+  // are stored whole: every cache line of the parts is written by one workgroup)
+  int parts() const { return gather.parts ? gather.parts : plan.ksplit; }
+  int64_t part_pitch() const {
+    return gather.parts ? plan.N : (plan.N + plan.bn - 1) / plan.bn * plan.bn;
+  }
+  size_t pad_bytes() const { return padded && !gather.parts ? x_bytes + w_bytes : 0; }
 };
+
+// The context's scratch: zero-padded copies of X and W, then the parts of a split reduction.
+size_t scratch_bytes(const ConvResolved &r) {
+  const size_t sums = r.parts() > 1 ? (size_t)r.parts() * (size_t)(r.plan.M * r.part_pitch()) * sizeof(float) : 0;
+  return r.pad_bytes() + sums;
+}
 
 // The gathered tiles for a problem that make_plan accepted (`C` its true channels).
 void choose_gather(ConvResolved &r, int64_t C) {
@@ -513,6 +527,17 @@ int conv_launch_f16(fhip_ctx *ctx, int bm, int bn, const GemmArgs &g) {
   return conv_launch_kind<GK_F16>(ctx, bm, bn, g);
 }
 
+// Where scratch cannot be had: reductions in one part, and gathered tiles, which read X and
+// W in place, instead of padded copies.
+static void do_without_scratch(const fhip_conv_desc *d, ConvResolved &r) {
+  if (!r.padded && r.gather.parts == 0)
+    r = resolve(d, false);
+  else if (r.gather.parts == 0)
+    r.gather = conv_gather_plan(r.plan.M, r.plan.N, (int64_t)r.plan.geom.R * r.plan.geom.S * r.C, false);
+  if (r.gather.parts)
+    r.gather.parts = 1;
+}
+
 bool fhip_fast_conv_applicable(const fhip_conv_desc *d, bool allow_scratch) {
   return fhip_fast_conv_rf_applicable(d) || resolve(d, allow_scratch).plan.ok;
 }
@@ -527,7 +552,9 @@ int fhip_fast_conv(fhip_ctx *ctx, const fhip_conv_desc *d, const void *x,
     return 1;
   if (taken)
     return 0;
-  const ConvResolved res = resolve(d, allow_scratch);
+  ConvResolved res = resolve(d, allow_scratch);
+  if (res.plan.ok && !fhip_ctx_scratch_ready(ctx, scratch_bytes(res)))
+    do_without_scratch(d, res);
   const ConvPlan &p = res.plan;
   if (handled) {
     *handled = p.ok;
@@ -537,22 +564,13 @@ int fhip_fast_conv(fhip_ctx *ctx, const fhip_conv_desc *d, const void *x,
   FHIP_REQUIRE(ctx, p.ok, "conv: descriptor not supported by the MFMA kernel");
   FHIP_REQUIRE(ctx, ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0,
                "conv: X and W must be 16-byte aligned");
-  // the context's scratch: zero-padded copies of X and W, then the parts of a
-  // split reduction
   const bool gather = res.gather.parts != 0;
-  const size_t pad_bytes = res.padded && !gather ? res.x_bytes + res.w_bytes : 0;
-  // (rows of the parts are padded to whole column tiles, which are stored
-  // whole: every cache line of the parts is written by one workgroup)
-  const int64_t part_pitch = gather ? p.N : (p.N + p.bn - 1) / p.bn * p.bn;
-  ConvGatherPlan gather_plan = res.gather;
-  int parts = gather ? gather_plan.parts : p.ksplit;
-  size_t part_bytes = parts > 1 ? (size_t)parts * (size_t)(p.M * part_pitch) * sizeof(float) : 0;
-  if (gather && parts > 1 && !fhip_ctx_scratch_ready(ctx, part_bytes))
-    gather_plan.parts = parts = 1, part_bytes = 0;
+  const int64_t part_pitch = res.part_pitch();
+  const int parts = res.parts();
   char *scratch = nullptr;
-  if (pad_bytes + part_bytes > 0) {
+  if (scratch_bytes(res) > 0) {
     void *sp = nullptr;
-    if (fhip_ctx_scratch(ctx, pad_bytes + part_bytes, &sp) != 0)
+    if (fhip_ctx_scratch(ctx, scratch_bytes(res), &sp) != 0)
       return 1;
     scratch = (char *)sp;
   }
@@ -642,7 +660,7 @@ int fhip_fast_conv(fhip_ctx *ctx, const fhip_conv_desc *d, const void *x,
     a.x_bytes = (uint32_t)(p.M / ((int64_t)cg.P * cg.Q) * cg.H * cg.W * a.C * 2);
     a.y_dt = d->y.dtype, a.o_dt = d->out.dtype;
     a.epi = g.epi;
-    if (conv_gather_launch(ctx, p.kind == GK_BF16, gather_plan, a) != 0)
+    if (conv_gather_launch(ctx, p.kind == GK_BF16, res.gather, a) != 0)
       return 1;
     if (parts > 1 && add_parts((const float *)scratch, g.epi) != 0)
       return 1;
@@ -691,7 +709,7 @@ int fhip_fast_conv(fhip_ctx *ctx, const fhip_conv_desc *d, const void *x,
     // every part writes plain f32 sums; rounding and the fused operations
     // follow in the kernel that adds them
     const DevEpilogue by_pixel = g.epi; // the remapped (0, pixel, channel) strides
-    float *part = (float *)(scratch + pad_bytes);
+    float *part = (float *)(scratch + res.pad_bytes());
     g.out = (char *)part;
     g.c_dt = g.o_dt = FHIP_FLOAT;
     g.o_sm = part_pitch;

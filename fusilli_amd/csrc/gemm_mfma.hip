@@ -276,8 +276,12 @@ bool fhip_fast_matmul_applicable(const fhip_matmul_desc *d) {
 
 int fhip_fast_matmul(fhip_ctx *ctx, const fhip_matmul_desc *d, const void *a,
                      const void *b, const DevEpilogue &epi, void *out) {
-  const GemmPlan p = make_plan(d);
+  GemmPlan p = make_plan(d);
   FHIP_REQUIRE(ctx, p.ok, "gemm: descriptor not supported by the MFMA kernel");
+  const int64_t pitch = (p.N + p.bn - 1) / p.bn * p.bn; // of the parts of a split reduction
+  const size_t part_bytes = (size_t)p.ksplit * (size_t)(p.M * pitch) * sizeof(float);
+  if (p.ksplit > 1 && !fhip_ctx_scratch_ready(ctx, part_bytes))
+    p.ksplit = 1;
   FHIP_REQUIRE(ctx, ((uintptr_t)a & 15) == 0 && ((uintptr_t)b & 15) == 0,
                "gemm: A and B must be 16-byte aligned");
   GemmArgs g{};
@@ -340,8 +344,7 @@ int fhip_fast_matmul(fhip_ctx *ctx, const fhip_matmul_desc *d, const void *a,
     // stored whole: every cache line of the parts is written by one workgroup,
     // with full 16-byte stores)
     void *sp = nullptr;
-    const int64_t pitch = (int64_t)g.tiles_n * p.bn;
-    if (fhip_ctx_scratch(ctx, (size_t)p.ksplit * (size_t)(p.M * pitch) * sizeof(float), &sp) != 0)
+    if (fhip_ctx_scratch(ctx, part_bytes, &sp) != 0)
       return 1;
     g.out = (char *)sp;
     g.c_dt = g.o_dt = p.kind == GK_I8 ? FHIP_INT32 : FHIP_FLOAT;

@@ -42,6 +42,44 @@ def _matmul(torch):
     return a, out, lambda c: c.matmul(d, a.data_ptr(), b.data_ptr(), out.data_ptr()), 2e-2
 
 
+def _matmul_tiled(torch):
+    a = torch.randn(512, 8192, device="cuda", dtype=torch.bfloat16)
+    b = torch.randn(256, 8192, device="cuda", dtype=torch.bfloat16)
+    out = torch.empty(512, 256, device="cuda", dtype=torch.bfloat16)
+    d = capi.MatmulDesc()
+    d.a = capi.TensorDesc.make([512, 8192], [8192, 1], capi.BFLOAT16)
+    d.b = capi.TensorDesc.make([8192, 256], [1, 8192], capi.BFLOAT16)
+    d.c = capi.TensorDesc.make([512, 256], [256, 1], capi.FLOAT)
+    d.out = capi.TensorDesc.make([512, 256], [256, 1], capi.BFLOAT16)
+    d.out_dtype = capi.BFLOAT16
+    d.epilogue = capi.make_epilogue([])
+    return a, out, lambda c: c.matmul(d, a.data_ptr(), b.data_ptr(), out.data_ptr()), 2.0 ** -8
+
+
+def _conv(torch, n, c, k, hw, pad=1):
+    cl = lambda n, c, h, w: capi.TensorDesc.make([n, c, h, w], [c * h * w, 1, c * w, c], capi.BFLOAT16)  # noqa: E731
+    x = torch.randn(n, hw, hw, c, device="cuda", dtype=torch.bfloat16)
+    w = torch.randn(k, 1 + 2 * pad, 1 + 2 * pad, c, device="cuda", dtype=torch.bfloat16)
+    out = torch.empty(n, hw, hw, k, device="cuda", dtype=torch.bfloat16)
+    d = capi.ConvDesc()
+    d.x, d.w = cl(n, c, hw, hw), cl(k, c, 1 + 2 * pad, 1 + 2 * pad)
+    d.y = d.out = cl(n, k, hw, hw)
+    d.out_dtype, d.spatial_rank = capi.BFLOAT16, 2
+    for i in range(2):
+        d.stride[i] = d.dilation[i] = 1
+        d.padding[i] = pad
+    d.epilogue = capi.make_epilogue([])
+    return x, out, lambda c: c.conv_fprop(d, x.data_ptr(), w.data_ptr(), out.data_ptr()), 2.0 ** -8  # two roundings to bf16
+
+
+def _conv_padded(torch):
+    return _conv(torch, 44, 80, 256, 58, pad=0)
+
+
+def _conv_split(torch):
+    return _conv(torch, 4, 512, 128, 7)
+
+
 def _reduce(torch, channels_last):
     dims = [8, 24, 50, 50]
     x = torch.randn(dims, device="cuda")
@@ -61,6 +99,12 @@ def _bias_gradient(torch):
 
 def _channel_means(torch):
     return _reduce(torch, False)
+
+
+# what runs where there is scratch
+ROUTES = {_matmul_tiled: "gemm_mfma bf16 128x128 waves=8 split=16",
+          _conv_padded: "conv_igemm gather 256x256 split=1 padded=1 groups=1",
+          _conv_split: "conv_igemm gather 128x128 split=8 padded=0 groups=1"}
 
 
 @pytest.mark.parametrize("make", [_norm, _sdpa, _matmul])
@@ -108,7 +152,8 @@ def test_replay_after_scratch_has_grown(make):
         other.close()
 
 
-@pytest.mark.parametrize("make", [_norm, _sdpa, _matmul, _bias_gradient, _channel_means])
+@pytest.mark.parametrize("make", [_norm, _sdpa, _matmul, _matmul_tiled, _conv_padded, _conv_split, _bias_gradient,
+                                  _channel_means])
 def test_first_call_under_capture(make):
     import torch
     torch.manual_seed(1)
@@ -121,9 +166,11 @@ def test_first_call_under_capture(make):
         stream.synchronize()
         with torch.cuda.graph(graph, stream=stream):
             call(cold)
+        assert "split=1" in cold.last_kernel() or "split=" not in cold.last_kernel()
         for i in range(3):
             x.copy_(torch.randn_like(x))
             call(warm)
+            assert warm.last_kernel() == ROUTES.get(make, warm.last_kernel())
             want = out.float().clone()
             out.zero_()
             graph.replay()
