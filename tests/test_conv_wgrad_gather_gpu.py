@@ -1,6 +1,7 @@
 """Weight gradient on gathered MFMA tiles (conv_wgrad.hip), through the C ABI vs the
 oracle: channel counts off the tiles, tap runs across column tiles, strides, dilation,
 padding beyond the image, pixel counts off the steps, several chunks of pixels."""
+import numpy as np
 import pytest
 
 from fusilli_amd import capi
@@ -51,3 +52,32 @@ def test_conv_wgrad_gather_vs_oracle(ctx, case, dtype, f32_out):
         assert_close(dw.logical(), oracle.conv_wgrad(dy.logical(), x.logical(), case["w"], *geom),
                      dtype, f"wgrad {case}")
     assert ctx.last_kernel().startswith("conv_wgrad_gather"), ctx.last_kernel()
+
+
+@pytest.mark.parametrize("dtype", [capi.BFLOAT16, capi.HALF])
+@pytest.mark.parametrize("x,w,stride,tile", [
+    ([4, 256, 48, 60], [256, 256, 5, 5], 1, "128x128"),
+    ([6, 512, 24, 24], [192, 512, 5, 5], 1, "64x256"),
+    ([6, 512, 24, 24], [96, 512, 5, 5], 1, "32x256"),
+    ([8, 320, 64, 60], [2560, 320, 1, 1], 2, "256x64"),
+])
+def test_f32_weight_gradient_rounds_in_short_chains(ctx, dtype, x, w, stride, tile):
+    # Few runs of many pixels: 30 additions of 16 products each, at most seven such groups per
+    # run, at most ten runs are chains of their own.  A chain of n adds about sqrt(n) / 3 *
+    # 2^-24 of a random sum's size: 2.4 together (one chain of a run's 770 to 2900 pixels: 2.4
+    # to 4.6).
+    pad = w[2] // 2
+    geom = ([pad, pad], [stride, stride], [1, 1])
+    lay = oracle.channels_last_strides
+    yd = oracle.conv_output_dims(x, w, *geom)
+    xs = HT.from_logical(rand(62, 0, x), dtype, lay(x))
+    dy = HT.from_logical(rand(62, 1, yd), dtype, lay(yd))
+    dw = run_conv_wgrad(ctx, dy, xs, w, *geom, dtype, tuned=None, w_dtype=capi.FLOAT).logical()
+    assert ctx.last_kernel().startswith(f"conv_wgrad_gather {tile} "), ctx.last_kernel()
+    xp = np.pad(xs.logical().astype(np.float64), [(0, 0), (0, 0), (pad, pad), (pad, pad)])
+    for r, s in ((0, 0), (w[2] - 1, w[3] // 2)):
+        shifted = xp[:, :, r:r + stride * (yd[2] - 1) + 1:stride, s:s + stride * (yd[3] - 1) + 1:stride]
+        ref = (dy.logical().astype(np.float64).transpose(1, 0, 2, 3).reshape(w[0], -1)
+               @ shifted.transpose(0, 2, 3, 1).reshape(-1, w[1]))
+        err = np.linalg.norm(dw[:, :, r, s] - ref) / np.linalg.norm(ref)
+        assert err <= 2.6 * 2.0 ** -24, (ctx.last_kernel(), err * 2.0 ** 24)
