@@ -234,16 +234,18 @@ conv_wgrad_gather_kernel(WgArgs g) {
     fetch(S0{}, 0);
     fetch(S1{}, 1);
     fetch(S2{}, 2);
-    for (int t0 = 0; t0 < steps; t0 += SHORT ? kWgGroup : kWgChunk) {
-      const int end = SHORT && t0 + kWgGroup < steps ? t0 + kWgGroup : steps;
-      for (int t = t0; t < end; t += 3) {
+    auto walk = [&](int from, int to) {
+      for (int t = from; t < to; t += 3) {
         step(S0{}, t);
-        if (t + 1 < end)
+        if (t + 1 < to)
           step(S1{}, t + 1);
-        if (t + 2 < end)
+        if (t + 2 < to)
           step(S2{}, t + 2);
       }
-      if constexpr (SHORT) {
+    };
+    if constexpr (SHORT) {
+      for (int t = 0; t < steps; t += kWgGroup) {
+        walk(t, t + kWgGroup < steps ? t + kWgGroup : steps);
 #pragma unroll
         for (int a = 0; a < MT; ++a)
 #pragma unroll
@@ -251,6 +253,8 @@ conv_wgrad_gather_kernel(WgArgs g) {
             sum[a][b] += acc[a][b];
         clear(acc);
       }
+    } else {
+      walk(0, steps);
     }
   }
   auto &result = SHORT ? sum : acc;
