@@ -16,8 +16,8 @@
 // runs' sums in a fixed order.
 //
 // Before, both operands were copied into zero-padded grids for a batched GEMM of 128
-// columns at least: N62 256 -> 48, 39 x 39, 3 x 3, bf16: 248 us -> 76.5; N32 112 ->
-// 384, 26 x 26, f16: 138 -> 40.6; N16 48 -> 48, 48 x 32, f16: 36.7 -> 17.4.
+// columns at least: N62 256 -> 48, 39 x 39, 3 x 3, bf16: 248 us -> 48.7; N32 112 ->
+// 384, 26 x 26: 138 -> 34.4; N16 48 -> 48, 48 x 32: 36.7 -> 15.5.
 //
 // Reference semantics: node/conv_node.h:255-426 (ConvWGradNode),
 // aten.convolution_backward, weight gradient.
@@ -342,8 +342,9 @@ struct WgradPlan {
   size_t part_bytes = 0, contract = 0;
 };
 
-// The workspace that callers bring, 0 for descriptors that ask for none.  Sizes are kept
-// in callers' saved plans, so they stay what they were when X and DY were copied into
+// The workspace that callers bring, 0 for descriptors that ask for none.  Saved plans hold
+// its size and are taken only where they equal the plan of today byte for byte
+// (Graph::loadFromArtifact), so it stays what it was when X and DY were copied into
 // zero-padded grids (rows and columns padded, 64-pixel pitch, DY of 128 channels at
 // least) in front of the sums of every image's share; the sums of the runs fit in it.
 size_t wgrad_contract(const fhip_conv_desc *d) {

@@ -239,8 +239,8 @@ __global__ __launch_bounds__(256) void reduce_rows_kernel(ReduceRowsArgs g) {
 // slices on workgroups of their own (partial[slice][k], f32), which a second kernel combines in slice
 // order: no atomics.  Bound by reading X once.  N32 56 x 56 K128 bf16 in
 // channels-last (25.7 MB): 104 us on the strided kernel (one workgroup per
-// channel and slice reading one 2-byte element per pixel line) -> 12.7 us
-// (8.8 + 3.9); N100 K32 30 x 30 f32 channels-first (11.5 MB) 31 -> 10.2 us (5.5 +
+// channel and slice reading one 2-byte element per pixel line) -> 8.4 us
+// (both launches); N100 K32 30 x 30 f32 channels-first (11.5 MB) 31 -> 10.2 us (5.5 +
 // 4.6).
 struct ReduceMidArgs {
   const char *x;

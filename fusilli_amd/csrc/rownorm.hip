@@ -190,8 +190,8 @@ bool fhip_fast_norm_applicable(const fhip_norm_desc *d) {
          (pick_shape(lay.inner, vec, &chunks, &wpr) || fhip_norm_long_applicable(d));
 }
 
-// Dense rows that the kernels above leave: any length, element alignment (down to
-// 2 x 292 the walk beats the generic kernel, 8.6 us against 5.0).
+// Dense rows that the kernels above leave: any length, element alignment (the
+// generic kernel / the walk: 2 x 292 f16 7.9 / 4.2 us, 1000 x 1003 19.6 / 5.0).
 int fhip_loose_norm(fhip_ctx *ctx, const fhip_norm_desc *d, const void *x, const void *scale,
                     const void *bias, const DevEpilogue &epi, void *out, void *mean,
                     void *inv_variance, bool *handled) {

@@ -238,7 +238,8 @@ typedef struct {
 } fhip_matmul_desc;
 
 int fhip_matmul_workspace_size(const fhip_matmul_desc *d, size_t *bytes);
-/* 0 = unsupported, 1 = generic strided kernel, 2 = MFMA fast path */
+/* 0 = unsupported, 1 = another kernel (direct, or generic for any strides),
+ * 2 = tiled MFMA kernel */
 int fhip_matmul_supported(const fhip_matmul_desc *d);
 int fhip_matmul(fhip_ctx *ctx, const fhip_matmul_desc *d, const void *a,
                 const void *b, const void *const *epilogue_operands, void *out,
@@ -276,11 +277,14 @@ int fhip_conv_fprop(fhip_ctx *ctx, const fhip_conv_desc *d, const void *x,
  *      kernel takes the problem (16-bit channels-last tensors, one group):
  *      it then needs fhip_conv_dgrad_workspace_size bytes of 256-byte aligned
  *      workspace (a mirrored copy of the filter; with strides above one also
- *      DY spread over a zero grid) and fails without them.  fhip_conv_wgrad_supported returns 2 for 16-bit
- *      channels-last X and DY with equal strides, one group, K >= 128 and
- *      S * C >= 128 (batched MFMA GEMMs over zero-padded copies of both
- *      operands; 256-byte aligned workspace of
- *      fhip_conv_wgrad_workspace_size bytes). ----------------------------- */
+ *      DY spread over a zero grid) and fails without them.
+ *      fhip_conv_wgrad_supported returns 2 for 16-bit channels-last X and DY
+ *      of one group with C and K multiples of 8, equal strides, no dilation
+ *      along W and S * C >= 128 (MFMA tiles gathered from X and DY as they
+ *      lie; partial sums in 256-byte aligned workspace of
+ *      fhip_conv_wgrad_workspace_size bytes, without which it fails), and for
+ *      1 x 1 filters at unit stride that run as a matrix product (no
+ *      workspace). ----------------------------- */
 int fhip_conv_dgrad_workspace_size(const fhip_conv_desc *d, size_t *bytes);
 int fhip_conv_dgrad_supported(const fhip_conv_desc *d);
 int fhip_conv_dgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy,

@@ -74,9 +74,9 @@ def test_gradient_and_batchnorm_queries_need_no_gpu():
         d.stride[i] = 2
     d.y = capi.TensorDesc.make([32, 128, 28, 28], cl([32, 128, 28, 28]), capi.BFLOAT16)
     assert lib.fhip_conv_dgrad_supported(d) == 2  # DY spread over a zero grid
-    assert lib.fhip_conv_wgrad_supported(d) == 2  # batched GEMMs, B rows two pixels apart
+    assert lib.fhip_conv_wgrad_supported(d) == 2  # gathered tiles
     assert lib.fhip_conv_wgrad_workspace_size(d, ctypes.byref(n)) == 0
-    assert n.value > 32 * 58 * 64 * 64 * 2  # zero-padded copies of X and DY
+    assert n.value > 32 * 58 * 64 * 64 * 2  # (what callers' saved plans carry; the partial sums take less)
     d.y = capi.TensorDesc.make([32, 128, 28, 27], cl([32, 128, 28, 27]), capi.BFLOAT16)
     assert lib.fhip_conv_dgrad_supported(d) == 0  # DY extent disagrees
 

@@ -627,8 +627,7 @@ def test_conv_wgrad_direct_kernel_vs_oracle(ctx, case, dtype, knobs):
     # the workspace is only the partial sums: one 36 KB block per workgroup
     d = conv_bwd_desc(x, HT.empty(wd, dtype, cl(wd)), dy, [1, 1], [1, 1], [1, 1])
     assert ctx.conv_wgrad_workspace(d) % (9 * 16 * 64 * 4) == 0
-    # switched off, the same descriptor runs on the batched-GEMM path or the
-    # generic kernel and agrees
+    # switched off, the same descriptor runs on the gathered tiles and agrees
     knobs(WGRAD_DIRECT="0")
     assert ctx.conv_wgrad_workspace(d) % (9 * 16 * 64 * 4) != 0 or \
         ctx.conv_wgrad_workspace(d) == 0
