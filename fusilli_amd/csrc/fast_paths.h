@@ -12,9 +12,10 @@ int fhip_fast_matmul(fhip_ctx *ctx, const fhip_matmul_desc *d, const void *a,
 
 // Products outside that contract -- few rows or columns, K or row starts that do
 // not fit 128-byte slices, f32 -- on kernels that load MFMA fragments straight
-// from global memory; `handled` false where they do not take the descriptor.
-int fhip_direct_matmul(fhip_ctx *ctx, const fhip_matmul_desc *d, const void *a,
-                       const void *b, const DevEpilogue &epi, void *out, bool *handled);
+// from global memory; `handled` false where they do not take the descriptor, `short_k` true
+// where that is for the speed of the general path's f32 tiles over a short K.
+int fhip_direct_matmul(fhip_ctx *ctx, const fhip_matmul_desc *d, const void *a, const void *b,
+                       const DevEpilogue &epi, void *out, bool *handled, bool *short_k);
 
 // `allow_scratch` false: only plans that leave the context's scratch alone
 // (no zero-padded channel copies, no split reduction) -- for the entry point

@@ -11,36 +11,42 @@ namespace {
 // workgroup does once, and the general path's 64 x 64 f32 tiles (generic_ops.hip), one
 // slice of 16 K at a time and whole rows stored, finish them sooner.  `p`: the plan for the
 // direct kernel; `tiles`: 64 x 64 tiles of all batches.  Where the line lies was measured
-// at 25 values of K, 24 shapes of 25 to 4096 tiles and 16 batched ones in all four
-// orientations; it lies anew for every round of slices that a tile's wavefronts take, higher
-// where both operands are K-contiguous, and for 16 bits (whose general path widens them) at
-// 12 to 58.  us, f32 tiles / here: f32 1000 x 1000 K16 4.8 / 8.5, K104 8.8 / 8.9, K200
-// 12.8 / 11.3; 2048 x 2048 K40 13.7 / 19.5, K136 24.3 / 26.9, K232 35.3 / 30.6; 1600 x
-// 1600, both K-contiguous, K264 32.9 / 35.9, K520 57 / 59, K776 82 / 80; 200 batches of
-// 64 x 64 K40 6.4 / 11.3; f16 2048 x 2048, neither, K24 13.2 / 20.7, K68 22.3 / 19.4;
-// both, K16 10.8 / 14.0, K44 16.2 / 14.1.
+// at 32 values of K, 17 shapes of 64 to 4096 tiles and 11 batched ones in all four
+// orientations (3380 f32 products, 0.2 % of the better kernel's time left on average); it
+// lies anew for every round of slices that a tile's wavefronts take, lower where K is whole
+// slices, and for 16 bits (whose general path widens them) at 12 to 58.  us, f32 tiles /
+// here: f32 1000 x 1000 K16 4.8 / 8.5, K88 8.7 / 9.0, K128 10.2 / 8.3; 2048 x 2048 K40 14.0
+// / 18.6, K136 25.6 / 27.5, K160 27.5 / 24.4; both K-contiguous, 1600 x 1600 K128 20.7 /
+// 15.8, K264 35.8 / 36.1; 200 batches of 64 x 64 K40 6.5 / 11.1; f16 2048 x 2048, neither,
+// K24 13.2 / 20.7, K68 22.3 / 19.4; both, K16 10.8 / 14.0, K44 16.2 / 14.1.
 bool short_k(const DirectPlan &p, const DirectArgs &g, int64_t M, int64_t N, int64_t K, int64_t batch) {
   if (p.kind != GK_F32 && p.kind != GK_BF16 && p.kind != GK_F16)
     return false; // (8-bit products have no such path)
   const int64_t tiles = (M + 63) / 64 * ((N + 63) / 64) * batch;
   if (p.mt == 1 || tiles < 64 || (tiles < 128 && K >= 128))
     return false;
-  if (p.mt != 4 && p.b_kc)
-    return false; // (32 x 32 tiles keep up)
+  const bool whole = g.slices * 32 == K; // (f32: no slice is cut)
+  // (smaller tiles that are no more than the rows or columns ask for)
+  const bool halves = p.mt != 4 && 2 * (int64_t)g.tiles_m * g.tiles_n * batch > 3 * tiles;
+  if (p.mt != 4 && p.b_kc) // (32 x 32 tiles keep up)
+    return p.kind == GK_F32 && halves && tiles >= 110 && K < 17;
   const int rounds = (g.slices + p.waves - 1) / p.waves;
   if (p.kind == GK_F32) {
     if (tiles < 130)
       return !p.b_kc && K <= 40;
-    if (p.mt != 4) { // (32 x 64: half of a 64 x 64 tile each, unless there are no more rows)
-      const bool halves = 2 * (int64_t)g.tiles_m * g.tiles_n * batch > 3 * tiles;
-      return K < (!halves ? 110 : tiles <= 256 ? 150 : p.a_kc && rounds == 2 ? 275 : 190);
+    if (p.mt != 4) { // (32 x 64)
+      if (!halves)
+        return K < (tiles <= 256 ? 20 : whole ? 65 : p.a_kc ? 113 : 60);
+      if (tiles <= 256)
+        return K < (p.a_kc && !whole ? 150 : 130);
+      return K < (rounds == 1 ? 205 : 300);
     }
+    if (whole)
+      return K < (!p.b_kc ? (tiles > 256 && tiles <= 512 ? 97 : 65) : p.a_kc && tiles > 512 ? 65 : 33);
     if (rounds == 1)
-      return K < (p.a_kc ? 110 : 96) || (p.a_kc && p.b_kc && tiles > 512);
-    if (rounds == 2)
-      return K < (!p.a_kc ? 150 : !p.b_kc || tiles <= 512 ? 160 : 185);
-    // (both K-contiguous: a last round of workgroups that is not full)
-    return p.a_kc && p.b_kc && tiles > 512 && tiles % 512 != 0 && K < (rounds == 3 ? 300 : 400);
+      return K < (p.b_kc ? (tiles > 256 ? (p.a_kc ? 113 : 81) : p.a_kc ? 81 : 57)
+                         : !p.a_kc ? 85 : tiles > 256 ? 113 : 89);
+    return rounds == 2 && p.a_kc && K < (p.b_kc && tiles > 512 ? 153 : 145);
   }
   if (tiles < 130)
     return !p.a_kc && p.b_kc && K < 20;
@@ -51,7 +57,7 @@ bool short_k(const DirectPlan &p, const DirectArgs &g, int64_t M, int64_t N, int
   return K < (tiles <= 256 ? (p.b_kc ? 20 : 12) : (p.b_kc ? 50 : 40) + (tiles >= 1024 ? 8 : 0));
 }
 
-bool direct_plan(const fhip_matmul_desc *d, DirectPlan *p, DirectArgs *g, int64_t *batch) {
+bool direct_plan(const fhip_matmul_desc *d, DirectPlan *p, DirectArgs *g, int64_t *batch, bool *too_short) {
   const int r = d->a.rank;
   if ((r != 2 && r != 3) || d->a.dtype != d->b.dtype)
     return false;
@@ -126,7 +132,13 @@ bool direct_plan(const fhip_matmul_desc *d, DirectPlan *p, DirectArgs *g, int64_
       }
     }
   }
-  if (best == 0 || short_k(*p, *g, M, N, K, *batch))
+  if (best == 0)
+    return false;
+  // (16-bit operands into f32: the f32 tiles would be further from the exact sums, f16 K24
+  // 1.3 units of 2^-24 against 0.7)
+  const bool f32_of_16 = p->kind != GK_F32 && d->c.dtype == FHIP_FLOAT && d->out.dtype == FHIP_FLOAT;
+  *too_short = !f32_of_16 && short_k(*p, *g, M, N, K, *batch);
+  if (*too_short)
     return false;
   g->M = (int)M, g->N = (int)N, g->K = (int)K;
   g->a_ldb = a_ld * elem, g->b_ldb = b_ld * elem;
@@ -146,12 +158,12 @@ bool direct_plan(const fhip_matmul_desc *d, DirectPlan *p, DirectArgs *g, int64_
 } // namespace
 
 int fhip_direct_matmul(fhip_ctx *ctx, const fhip_matmul_desc *d, const void *a, const void *b,
-                       const DevEpilogue &epi, void *out, bool *handled) {
-  *handled = false;
+                       const DevEpilogue &epi, void *out, bool *handled, bool *short_k) {
+  *handled = *short_k = false;
   DirectPlan p;
   DirectArgs g{};
   int64_t batch = 1;
-  if (!direct_plan(d, &p, &g, &batch))
+  if (!direct_plan(d, &p, &g, &batch, short_k))
     return 0;
   // operands at their own alignment
   const uintptr_t am = fhip_dtype_size(d->a.dtype) - 1;

@@ -71,30 +71,47 @@ def test_direct_split_k(ctx, dtype, tb, m):
     check(out.logical(), ref_matmul(a, b), dtype)
 
 
-@pytest.mark.parametrize("dtype,ta,tb,m,n,batch,line", [
-    (capi.FLOAT, False, False, 600, 1100, 1, 150),  # 180 tiles
-    (capi.FLOAT, True, False, 33, 65, 100, 150),    # 200, a second one for a row and a column
-    (capi.FLOAT, False, True, 1500, 1450, 1, 185),  # 552, both K-contiguous
-    (capi.HALF, False, False, 1100, 1200, 1, 24),
-    (capi.BFLOAT16, True, True, 1100, 1200, 1, 50),
-    (capi.HALF, False, True, 600, 1100, 1, 34),
+@pytest.mark.parametrize("dtype,ta,tb,m,n,batch,tiled,direct", [
+    (capi.FLOAT, False, False, 600, 1100, 1, [9, 128, 149], [150]),   # 180 tiles
+    (capi.FLOAT, True, False, 33, 65, 100, [9, 64, 129], [130, 160]),  # 200, a second one for a row and a column
+    (capi.FLOAT, False, True, 1500, 1450, 1, [9, 64, 112, 152], [96, 113, 153]),  # 552, both K-contiguous
+    (capi.FLOAT, True, False, 1500, 1450, 1, [64, 84], [85, 96, 129]),
+    (capi.FLOAT, False, True, 700, 900, 1, [9, 16], [17]),
+    (capi.HALF, False, False, 1100, 1200, 1, [9, 23], [24]),
+    (capi.BFLOAT16, True, True, 1100, 1200, 1, [9, 49], [50]),
+    (capi.HALF, False, True, 600, 1100, 1, [9, 33], [34]),
 ])
-def test_short_k_takes_the_f32_tiles(ctx, dtype, ta, tb, m, n, batch, line):
-    # both sides of the rule's line; K odd to its slices on either
-    for k, direct in ((9, False), (line - 1, False), (line, True)):
+def test_short_k_takes_the_f32_tiles(ctx, dtype, ta, tb, m, n, batch, tiled, direct):
+    # both sides of the rule's lines, whole slices of 32 and cut ones
+    for k in tiled + direct:
         a = make_operand(96, 0, m, k, dtype, ta, batch=batch if batch > 1 else None)
-        b = make_operand(96, 1, k, n, dtype, tb)
-        if batch > 1:
-            b = make_operand(96, 1, k, n, dtype, tb, batch=1)
-        out = HT.empty(([batch] if batch > 1 else []) + [m, n], capi.FLOAT)
+        b = make_operand(96, 1, k, n, dtype, tb, batch=1 if batch > 1 else None)
+        out = HT.empty(([batch] if batch > 1 else []) + [m, n], dtype)
         d = capi.MatmulDesc()
-        d.a, d.b, d.c, d.out, d.out_dtype = a.desc(), b.desc(), out.desc(), out.desc(), capi.FLOAT
+        d.a, d.b, d.c, d.out, d.out_dtype = a.desc(), b.desc(), out.desc(), out.desc(), dtype
+        d.c.dtype = capi.FLOAT
         d.epilogue = capi.make_epilogue([])
         da, db, do = a.upload(ctx), b.upload(ctx), out.upload(ctx)
         ctx.matmul(d, da, db, do)
         name = ctx.last_kernel()
-        assert name.startswith("gemm_direct" if direct else "matmul_f32_tiled"), (k, name)
-        check(out.fetch(ctx, do).logical(), ref_matmul(a, b), dtype)
+        assert name.startswith("gemm_direct" if k in direct else "matmul_f32_tiled"), (k, name)
+        got, ref = out.fetch(ctx, do).logical(), ref_matmul(a, b)
+        check(got, ref, dtype) if dtype == capi.FLOAT else assert_close(got, ref, dtype)
+        if dtype == capi.FLOAT:
+            # Steps of 16 products and their sums are chains of their own: n additions round n
+            # times sums of half the result's size on average by 2^-24 / sqrt(12) of it, 0.41
+            # sqrt(n) 2^-24 together; 16 + 10 here (one chain of 152: 3.7 measured)
+            exact = a.logical().astype(np.float64) @ b.logical().astype(np.float64)
+            assert np.linalg.norm(got - exact) <= 0.41 * 26 ** 0.5 * 2.0 ** -24 * np.linalg.norm(exact), k
+
+
+@pytest.mark.parametrize("dtype", [capi.HALF, capi.BFLOAT16])
+def test_16_bit_operands_into_f32_keep_the_direct_kernel(ctx, dtype):
+    # (the f32 tiles' chains would show in the result)
+    a, b = make_operand(97, 0, 1100, 17, dtype, True), make_operand(97, 1, 17, 1200, dtype, True)
+    out, _ = run(ctx, a, b, capi.FLOAT)
+    exact = a.logical().astype(np.float64) @ b.logical().astype(np.float64)
+    assert np.linalg.norm(out.logical() - exact) <= 2.0 ** -24 * np.linalg.norm(exact)
 
 
 @pytest.mark.parametrize("dtype", [capi.FLOAT, capi.HALF, capi.INT8])
