@@ -688,8 +688,10 @@ int fhip_few_conv_fprop(fhip_ctx *ctx, const fhip_conv_desc *d, const void *x, c
   // (few tiles: a workgroup of 64 channels is a long chain of its own, mostly scalar loads
   // of the fused operations, so fewer channels each until there are two workgroups per
   // compute unit: N16 3 -> 64, 20 x 20, 3 x 3 f32 64 channels 14.9 us, 16 of them 8.8, the
-  // kernel of one pixel per thread 11.2)
-  while (kt > 1 && blocks * ((g.K + kt * 16 - 1) / (kt * 16)) < 2 * cus)
+  // kernel of one pixel per thread 11.2; shorter ones until there are 1.6: bf16 N71 4 -> 32,
+  // 40 x 40, 497 tiles 10.5, with 16 channels each 11.5)
+  const int64_t enough = g.K > 32 ? 2 * cus : 8 * cus / 5;
+  while (kt > 1 && blocks * ((g.K + kt * 16 - 1) / (kt * 16)) < enough)
     kt /= 2;
   if (!fits())
     return 0;
