@@ -615,8 +615,10 @@ int launch_mid(fhip_ctx *ctx, const ReducePlan &p, ReduceMidArgs g) {
     most = p.r1 / ((256 >> tx_log2) * 8);
     // Few rows: one slice, and one launch, on narrow workgroups (eight vectors at least,
     // four rows per thread) unless there are 512 wide ones ([64, 2048] bf16 maxima: strided
-    // 6.7 us, eight slices 8.4; [8, 7, 7] x 512 sums 6.7, so 4.4).
-    if (p.r1 <= 1024) {
+    // 6.7 us, eight slices 8.4; [8, 7, 7] x 512 sums 6.7, so 4.4).  Beyond 512 rows the few
+    // workgroups wait for memory where X is not in a cache: 1024 x 80 in a training step
+    // that takes 31.0 us with slices, 33.2 in one; 950 x 256, 55.7 and 57.2.
+    if (p.r1 <= 512) {
       while (tx_log2 > 3 && (cv >> tx_log2) < 512 && (512 >> tx_log2) * 4 <= p.r1)
         --tx_log2;
       most = 1;

@@ -192,9 +192,9 @@ def test_reduce_slices_of_few_long_runs(ctx, mode, dtype, dims, odims, least):
 
 
 @pytest.mark.parametrize("mode", ["SUM", "MAX"])
-@pytest.mark.parametrize("dims", [[2, 8], [1024, 40], [1025, 40], [64, 2048], [700, 16392], [33, 4101]])
+@pytest.mark.parametrize("dims", [[2, 8], [512, 40], [513, 40], [64, 2048], [300, 16392], [33, 4101]])
 def test_reduce_few_rows_in_one_launch(ctx, mode, dims):
     x = make_x(70, dims, capi.BFLOAT16, mode)
     out = run(ctx, x, [1, dims[1]], mode, y_dtype=capi.FLOAT, expect_tuned=False)
-    assert (ctx.last_kernel() == "reduce_cols slices=1") == (dims[0] <= 1024), ctx.last_kernel()
+    assert (ctx.last_kernel() == "reduce_cols slices=1") == (dims[0] <= 512), ctx.last_kernel()
     assert_close(out.logical(), oracle.reduction(x.logical(), [1, dims[1]], capi.RED[mode]), capi.FLOAT, rtol=2e-2)
