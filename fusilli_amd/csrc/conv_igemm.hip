@@ -352,8 +352,50 @@ size_t scratch_bytes(const ConvResolved &r) {
   return r.pad_bytes() + sums;
 }
 
+// Whether zero-padded copies of X and W and the product over whole slices beat the gathered
+// 64 x 64 tiles (`J`: the reduction, `fused`: operations behind the sum).  Both routes on 1373
+// problems without fused operations and as many with bias and ReLU, which cost the gathered
+// tiles more (8 us per 10^7 results, the others 2): the slower route is taken for 0.1 and
+// 0.5 % more time on average.  us, copies and product / here, plain, then with bias and ReLU.
+bool copies_pay(const ConvResolved &r, int64_t J, bool fused) {
+  const ConvPlan &p = r.plan;
+  const ConvGeom &g = p.geom;
+  // (N54 328 -> 256, 56 x 56, 1 x 1 at stride 2: 59 / 22, 63 / 32)
+  if (g.str_h != 1 || g.str_w != 1 || p.bn < 128)
+    return false;
+  const int64_t columns = (p.N + p.bn - 1) / p.bn, tiles = (p.M + p.bm - 1) / p.bm * columns;
+  const int64_t slots = p.halo || p.bm == 128 ? 512 : 256, rounds = (tiles + slots - 1) / slots;
+  const double fill = (double)p.N / (double)(columns * p.bn), full = (double)tiles / (double)(rounds * slots);
+  const double mn = (double)p.M * (double)p.N;
+  const bool seventh = (r.Cp - r.C) * 7 <= r.C;
+  // split reductions of 128 x 128 tiles (N11 472 -> 128, 48 x 48: 60 / 71, 63 / 74; N5 376 ->
+  // 128, 46 x 46, 5 x 5: 50 / 62, 53 / 65; N17 368 -> 128, 28 x 28: 0.73 of the time here)
+  if (p.ksplit > 1)
+    return seventh && fill >= 0.8 && ((J >= 5500 && tiles >= 80) || (J >= 3300 && tiles >= 190));
+  if (g.R * g.S == 1) // (N44 80 -> 256, 58 x 58: 45 / 34, 51 / 67)
+    return fused && (p.halo ? mn >= 4.5e6 : p.bn == 256 && fill >= 0.75 && (fill >= 0.85 || mn >= 2e7));
+  if (p.halo && p.bm == 256) // (N10 56 -> 256: 28.7 / 34.6, 30.7 / 47.1; 24 -> 384, 37 x 37: 28.8 / 22.4)
+    return fused ? J >= 480 || (J >= 280 && full >= 0.68 && fill >= 0.75) || (mn >= 2.4e7 && full >= 0.85)
+                 : J >= 480 && seventh && full >= 0.7 && fill >= 0.8;
+  if (p.halo) // (N39 216 -> 352, 30 x 18: 61 / 69, 63 / 73; N32 136 -> 256, 28 x 28: 51 / 39, 54 / 44)
+    return ((seventh || ((r.Cp - r.C) * 5 <= r.C && mn * (double)J >= 1.4e10)) && J >= 1000 && fill >= 0.8 &&
+            full >= (fused ? 0.75 : 0.8)) ||
+           (fused && J >= 400 && J <= 600 && tiles >= 300 && (r.Cp - r.C) * 3 <= r.C);
+  if (p.bn == 256) // (N8 240 -> 256, 60 x 60: 53 / 74, 54 / 78)
+    return J >= 1000 && fill >= (fused ? 0.85 : 0.9);
+  if (p.bm == 256) // (N18 224 -> 144, 46 x 46: 86 / 53, 90 / 58)
+    return J >= 1000 && fill >= 0.9 && full >= 0.7;
+  // 128 x 128 (120 -> 128, 102400 pixels: 60 / 69, 63 / 76), in one round long reductions only
+  // (N8 432 -> 256, 13832 pixels: 57 / 64, 57 / 68)
+  if (!seventh || J < 1000)
+    return false;
+  if (tiles >= 190 && tiles <= 256 && p.N % 128 == 0 && J >= (p.N >= 256 ? 2600 : 3300))
+    return true;
+  return fused ? p.N % 128 == 0 && tiles >= 500 : tiles >= 360 && fill >= 0.8 && full >= 0.7;
+}
+
 // The gathered tiles for a problem that make_plan accepted (`C` its true channels).
-void choose_gather(ConvResolved &r, int64_t C) {
+void choose_gather(ConvResolved &r, int64_t C, bool fused) {
   const ConvPlan &p = r.plan;
   const FhipKnobs &knobs = fhip_knobs();
   if (knobs.conv_gather == 0 || p.groups != 1 || C % 8 != 0 || knobs.conv_tile_bm || knobs.conv_halo >= 0 ||
@@ -366,34 +408,13 @@ void choose_gather(ConvResolved &r, int64_t C) {
   // 41.0; N64 128 -> 64, 28 x 28, 392 tiles: 19.2, 24.7), and gathered tiles over outputs of
   // less than half their width (N62 256 -> 48, 39 x 39: 69 us, here 50).
   const int64_t tiles = ((p.M + p.bm - 1) / p.bm) * ((p.N + p.bn - 1) / p.bn);
-  // (the narrow halo tile keeps up sooner: N6 64 -> 16, 54 x 54, 137 tiles 9.6 us, here 10.6)
-  const bool few = p.ksplit == 1 && tiles < (p.halo && p.bn == 64 ? 128 : 160) && p.geom.R * p.geom.S > 1;
+  // (the narrow halo tile, on 666 problems of 80 to 190 tiles: here 5 to 20 % faster up to the
+  // last without fused operations; with them even below 128 and 5 to 12 % slower from there)
+  const int64_t line = !p.halo || p.bn != 64 ? 160 : fused ? 128 : 192;
+  const bool few = p.ksplit == 1 && tiles < line && p.geom.R * p.geom.S > 1;
   const bool narrow = !p.halo && p.ksplit == 1 && p.N < 64;
-  // Where the copies pay (us, copies and product / here; both kernels on 589 problems):
-  auto copies_pay = [&]() {
-    const double mn = (double)p.M * (double)p.N, more = (double)(r.Cp - r.C) / (double)r.C;
-    // * tiles of 256 rows over reductions of some length, or over very many results: N8 240 ->
-    //   256, 60 x 60 55 / 76; N44 80 -> 256, 1 x 1, 58 x 58 51 / 67 (N11 16 -> 560, 64 x 64 at
-    //   stride 2: 24.7 / 19.0);
-    //   and columns that fill the tiles (N18 224 -> 144, 46 x 46: 100 / 57)
-    const int64_t columns = (p.N + p.bn - 1) / p.bn * p.bn;
-    if (p.bm == 256 && p.bn >= 128 && p.N * 4 >= columns * 3 && (J >= 200 || mn >= 1.6e7))
-      return true;
-    // * many tiles, a seventh of padding at most: N32 112 -> 384, 26 x 26, 507 tiles, step
-    //   153 / 157; N10 496 -> 128, 45 x 45, 159 tiles 182 / 177
-    if (more * 7 <= 1 && tiles >= 400)
-      return true;
-    // * the halo's largest products: N39 216 -> 352, 30 x 18 64.7 / 73.2 (N32 240 -> 256,
-    //   28 x 28 even; N32 136 -> 256 54 / 44)
-    if (p.halo && p.bm == 128 && p.bn == 128 && mn * (double)J >= 1.4e10 && more * 5 <= 1)
-      return true;
-    // * long reductions that fill one round of units with whole tiles: N8 472 -> 128, 60 x 60
-    //   70.8 / 76.4 (N8 312 -> 128 even, 248 -> 128 47 / 45)
-    return !p.halo && p.bm == 128 && p.N % 128 == 0 && tiles >= 190 && tiles <= 256 && J >= 3300 &&
-           more * 11 <= 1;
-  };
-  const bool copies = r.padded && !copies_pay();
-  const bool want = copies || knobs.conv_gather > 0 || few || narrow;
+  const bool copies = r.padded && copies_pay(r, J, fused);
+  const bool want = (r.padded && !copies) || knobs.conv_gather > 0 || few || narrow;
   // (whole slices: no parts -- the entry point without scratch gives the same bits)
   if (want)
     r.gather = conv_gather_plan(p.M, p.N, J, r.padded && p.N % 4 == 0);
@@ -406,7 +427,7 @@ ConvResolved resolve(const fhip_conv_desc *d, bool allow_scratch = true) {
   r.run = *g;
   r.plan = make_plan(g, d, allow_scratch);
   if (r.plan.ok)
-    choose_gather(r, g->x.dim[1]);
+    choose_gather(r, g->x.dim[1], d->epilogue.count > 0);
   if (r.plan.ok || !allow_scratch)
     return r;
   // channel padding: 16-bit channels-last tensors, whole 16-byte chunks
@@ -445,7 +466,7 @@ ConvResolved resolve(const fhip_conv_desc *d, bool allow_scratch = true) {
   r.w_pixels = fhip_desc_volume(g->w) / C;
   r.x_bytes = ((size_t)(r.x_pixels * Cp * 2) + 255) / 256 * 256;
   r.w_bytes = ((size_t)(r.w_pixels * Cp * 2) + 255) / 256 * 256;
-  choose_gather(r, C);
+  choose_gather(r, C, d->epilogue.count > 0);
   return r;
 }
 

@@ -73,7 +73,7 @@ def _conv(torch, n, c, k, hw, pad=1):
 
 
 def _conv_padded(torch):
-    return _conv(torch, 44, 80, 256, 58, pad=0)
+    return _conv(torch, 8, 200, 256, 60)
 
 
 def _conv_split(torch):
@@ -103,7 +103,7 @@ def _channel_means(torch):
 
 # what runs where there is scratch
 ROUTES = {_matmul_tiled: "gemm_mfma bf16 128x128 waves=8 split=16",
-          _conv_padded: "conv_igemm gather 256x256 split=1 padded=1 groups=1",
+          _conv_padded: "conv_igemm gather 256x128 split=1 padded=1 groups=1",
           _conv_split: "conv_igemm gather 128x128 split=8 padded=0 groups=1"}
 
 

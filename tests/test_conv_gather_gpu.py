@@ -61,26 +61,47 @@ def test_conv_gather_vs_oracle(ctx, case, dtype, forced, knobs):
                      dtype, f"dgrad {case} {ctx.last_kernel()}")
 
 
-@pytest.mark.parametrize("x,w,pad,gathered", [
-    ([8, 200, 60, 60], [256, 200, 3, 3], 1, False),  # tiles of 256 rows, a long reduction
-    ([44, 80, 58, 58], [256, 80, 1, 1], 0, False),   # over very many results
-    ([18, 224, 46, 46], [144, 224, 3, 3], 1, True),  # the same tiles half empty
-    ([11, 16, 64, 64], [560, 16, 3, 3], 1, True),    # a short reduction
-    ([39, 216, 30, 18], [352, 216, 3, 3], 1, False),  # the halo's largest products
-    ([32, 136, 28, 28], [256, 136, 3, 3], 1, True),
-    ([11, 472, 48, 48], [128, 472, 3, 3], 1, False),  # one round of whole tiles
-    ([11, 248, 48, 48], [128, 248, 3, 3], 1, True),
+@pytest.mark.parametrize("x,w,pad,stride,plain,fused", [  # whether gathered
+    ([8, 200, 60, 60], [256, 200, 3, 3], 1, 1, False, False),  # tiles of 256 rows, a long reduction
+    ([44, 80, 58, 58], [256, 80, 1, 1], 0, 1, True, False),    # 1 x 1 over very many results
+    ([12, 328, 56, 56], [256, 328, 1, 1], 0, 2, True, True),   # strided
+    ([18, 224, 46, 46], [144, 224, 3, 3], 1, 1, True, True),   # tiles half empty
+    ([11, 16, 64, 64], [560, 16, 3, 3], 1, 2, True, True),     # a short reduction
+    ([39, 216, 30, 18], [352, 216, 3, 3], 1, 1, False, False),  # halo tiles, full rounds
+    ([32, 136, 28, 28], [256, 136, 3, 3], 1, 1, True, True),
+    ([22, 56, 48, 48], [256, 56, 3, 3], 1, 1, False, False),   # halo tiles of 256 rows
+    ([27, 40, 36, 36], [384, 40, 3, 3], 1, 1, True, False),    # much padding
+    ([11, 472, 48, 48], [128, 472, 3, 3], 1, 1, False, False),  # a split reduction
+    ([11, 248, 48, 48], [128, 248, 3, 3], 1, 1, True, True),
 ])
-def test_padded_copies_where_they_pay(ctx, knobs, x, w, pad, gathered):
+@pytest.mark.parametrize("relu", [False, True])
+def test_padded_copies_where_they_pay(ctx, knobs, x, w, pad, stride, plain, fused, relu):
     # both sides of the rule, and the same sums (of whole numbers: exact in f32) on either route
-    stride = 2 if x[1] == 16 else 1
+    gathered = fused if relu else plain
     lay = oracle.channels_last_strides
     xs = HT.from_logical(np.resize(rand(72, 0, [4099], "int", lo=-3, hi=4), x), capi.BFLOAT16, lay(x))
     ws = HT.from_logical(np.resize(rand(72, 1, [4093], "int", lo=-3, hi=4), w), capi.BFLOAT16, lay(w))
     geom = ([pad, pad], [stride, stride], [1, 1])
-    y = run_conv(ctx, xs, ws, *geom, capi.FLOAT, channels_last_out=True).logical()
+    epi = [capi.epilogue_op(capi.PW["RELU_FWD"], capi.FLOAT)] if relu else []
+    y = run_conv(ctx, xs, ws, *geom, capi.FLOAT, epilogue=epi, channels_last_out=True).logical()
     assert ("unpadded" in ctx.last_kernel()) == gathered, ctx.last_kernel()
     knobs(CONV_GATHER=0 if gathered else 1)
-    z = run_conv(ctx, xs, ws, *geom, capi.FLOAT, channels_last_out=True).logical()
+    z = run_conv(ctx, xs, ws, *geom, capi.FLOAT, epilogue=epi, channels_last_out=True).logical()
     assert ("unpadded" in ctx.last_kernel()) != gathered, ctx.last_kernel()
     assert np.array_equal(y, z)
+
+
+@pytest.mark.parametrize("relu", [False, True])
+def test_narrow_layers_by_tiles_and_fused_operations(ctx, relu):
+    # 64 output channels at most: gathered below 128 tiles of 128 rows, without fused
+    # operations below 192
+    for n, gathered in ((12, True), (16, not relu), (25, False)):  # 96, 128, 200 tiles
+        x = HT.from_logical(np.resize(rand(73, 0, [4099]), [n, 64, 32, 32]), capi.BFLOAT16,
+                            oracle.channels_last_strides([n, 64, 32, 32]))
+        w = HT.from_logical(rand(73, 1, [32, 64, 3, 3], std=0.05), capi.BFLOAT16,
+                            oracle.channels_last_strides([32, 64, 3, 3]))
+        epi = [capi.epilogue_op(capi.PW["RELU_FWD"], capi.BFLOAT16)] if relu else []
+        y = run_conv(ctx, x, w, [1, 1], [1, 1], [1, 1], capi.BFLOAT16, epilogue=epi, channels_last_out=True).logical()
+        assert ("unpadded" in ctx.last_kernel()) == gathered, (n, ctx.last_kernel())
+        ref = oracle.conv_fprop(x.logical()[:1], w.logical(), [1, 1], [1, 1], [1, 1])
+        assert_close(y[:1], np.maximum(ref, 0) if relu else ref, capi.BFLOAT16)
