@@ -355,29 +355,32 @@ int fhip_decode_sdpa(fhip_ctx *ctx, const fhip_sdpa_desc *d, const void *q, cons
     kv = g.Sq;
   g.chunks = (kv + kChunk - 1) / kChunk;
   const int64_t tiles = (int64_t)g.heads * g.qtiles;
-  // Estimates in microseconds, fitted to both kernels' times on 700 problems (1 to 2500
-  // queries, 32 to 4096 keys, 1 to 64 heads, batches to 32).  Here: the tiles' reads of K
-  // and V, whole rounds of the four wavefronts' 32 keys, half of them under a causal mask,
-  // at 10.7 TB/s from the caches; a tile's fixed part; the heads' own K and V from memory.
-  // The tiled kernel: 1.45 (D 64: 0.97) per 64 keys and round of 256 workgroups of 256
-  // rows, a long and a short tile per workgroup under a causal mask.  (B21, 64 heads on 8,
-  // 68 x 68 causal, D128, 5880 tiles: tiled 48.5, here 62.2; B4, 8 heads on 1, 320 x 3456,
-  // D64: 56.3, 60.1; B2, 16 heads on 4, 128 x 128 causal, D64: 6.4, 5.1.)
-  const double keys = kv <= kChunk ? 64.0 // (one wavefront works)
-                                   : ceil(kv * (d->is_causal && g.Sq > 16 ? 0.5 + 8.0 / g.Sq : 1.0) / 128.0) * 128.0;
-  const double here = 4.64 + (double)tiles * keys * HD * 4.0 * 0.093e-6 + (double)tiles * HD * 2e-5 +
-                      (double)g.heads * kv * HD * 4.0 * 0.074e-6;
-  const int64_t big = (g.Sq + 255) / 256, kvt = (kv + 63) / 64;
-  const bool pairs = d->is_causal && big > 1;
-  const double per = HD == 128 ? 1.45 : 0.97;
-  const double there = 0.43 + ceil((double)(B * Hq * (pairs ? (big + 1) / 2 : big)) / 256.0) *
-                                  (pairs ? 8.2 + per * (double)(kvt * (big + 1)) / (double)big : 4.1 + per * (double)kvt);
-  if (here >= there && forced != 1)
-    return 0;
   // two workgroups per compute unit, two chunks per wavefront at least
   int64_t splits = 512 / tiles, deep = g.chunks / (2 * kWaves);
   splits = splits < deep ? splits : deep;
   g.splits = (int32_t)(splits < 1 ? 1 : splits < 64 ? splits : 64);
+  // Estimates in microseconds, fitted to both kernels' times on 1098 problems (1 to 1500
+  // queries, 32 to 4096 keys, 1 to 64 heads, batches to 32), of which the slower kernel costs
+  // 0.6 % on average.  Here: a wavefront's rounds of 32 keys, half of them under a causal
+  // mask; the tiles' reads of K and V at 14.7 TB/s from the caches; a tile's rows; the second
+  // launch.  The tiled kernel: 1.45 (D 64: 1.06) per 64 keys and round of 256 workgroups of
+  // 256 rows, a long and a short tile per workgroup under a causal mask.  (Tiled / here: B21,
+  // 64 heads on 8, 68 x 68 causal, D128, 5880 tiles 48.5 / 62.2; B4, 8 heads on 1, 320 x 3456,
+  // D64 56.3 / 60.1; B2, 32 heads, 65 x 65 causal, D128 8.6 / 6.2; B7, 32 heads, 1 x 175, D128
+  // 9.1 / 5.9.)
+  const double half = d->is_causal && g.Sq > 16 ? 0.5 + 8.0 / g.Sq : 1.0;
+  const double iters = ceil(g.chunks * half / (kWaves * g.splits)), keys = ceil(kv * half / kChunk) * kChunk;
+  const double valid = fmin(1.0, (double)g.group * g.Sq / (16.0 * g.qtiles));
+  const double here = (HD == 128 ? 4.2 + 0.99 * iters : 3.4 + 0.81 * iters) + (double)tiles * keys * HD * 4.0 * 0.068e-6 +
+                      (double)tiles * HD * 1e-5 * fmax(0.0, 7.8 * valid - 2.7) + (g.splits > 1 ? 4.8 : 0.0);
+  const int64_t big = (g.Sq + 255) / 256, kvt = (kv + 63) / 64;
+  const bool pairs = d->is_causal && big > 1;
+  const double per = HD == 128 ? 1.45 : 1.063, first = pairs ? 7.9 : HD == 128 ? 4.32 : 3.34;
+  const double there = (d->is_causal ? 1.36 : 0.16) +
+                       ceil((double)(B * Hq * (pairs ? (big + 1) / 2 : big)) / 256.0) *
+                           (first + per * (pairs ? (double)(kvt * (big + 1)) / (double)big : (double)kvt));
+  if (here >= there && forced != 1)
+    return 0;
   if (tiles * g.splits >= (1ll << 31))
     return 0;
   const size_t rows16 = (size_t)g.splits * (size_t)tiles * 16;

@@ -118,3 +118,6 @@ def test_route_of_short_products_and_many_tiles(ctx):
     assert name(2, 16, 4, 128, 128, 64, True) == "sdpa_decode"
     assert name(4, 64, 8, 68, 68, 128, True) == "sdpa_fwd"
     assert name(5, 32, 32, 266, 266, 64, True) == "sdpa_fwd"
+    assert name(2, 32, 32, 65, 65, 128, True) == "sdpa_decode"
+    assert name(7, 32, 32, 1, 175, 128, False) == "sdpa_decode"
+    assert name(5, 32, 32, 1, 64, 128, False) == "sdpa_decode"
