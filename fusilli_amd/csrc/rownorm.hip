@@ -59,6 +59,24 @@ bool zero_inner_strides(const fhip_tensor_desc &x, const int64_t *strides) {
   return true;
 }
 
+// Whether a row that sixteen wavefronts could hold in sixteen vectors per lane is better cut
+// into segments (rownorm_walk.hip).  One workgroup to a row leaves the chip idle under few
+// rows, and sixteen vectors with their scale and bias leave a lane no registers for loads in
+// flight: whole / cut, us, bf16 4 x 131072 LayerNorm 31.4 / 6.9, 256 x 65544 37 / 26, 2500 x
+// 70000 320 / 237, RMSNorm 337 / 225 (f16 4096 x 65544 RMSNorm 335 / 339).  f32 vectors hold
+// half as many values to finish, and RMSNorm has no bias to hold: LayerNorm 4 x 32772 12.1 /
+// 6.9, 128 x 32772 15.9 / 13.8, 256 x 32772 21.1 / 22.5, 511 x 65536 73 / 62; RMSNorm 4 x
+// 32772 5.9 / 6.9, 10 x 45000 8.1 / 6.9, 64 x 65536 12.2 / 12.0, 128 x 65536 13.0 / 19.8.
+bool cut_pays(const fhip_norm_desc *d, int64_t rows, int64_t inner, int chunks, fhip_ctx *ctx) {
+  if (chunks != 16 || fhip_knobs().rownorm_shape_w)
+    return false;
+  const bool layer = d->is_layernorm != 0;
+  const bool pays = d->x.dtype != FHIP_FLOAT ? rows < 4096
+                    : layer                 ? rows <= 128 || inner >= 49152
+                                            : rows <= 64 && inner >= 45056;
+  return pays && fhip_norm_walk_splits(ctx, d->x.dtype, rows, inner, true) > 1;
+}
+
 bool fast_dtype(int dt) {
   return dt == FHIP_BFLOAT16 || dt == FHIP_HALF || dt == FHIP_FLOAT;
 }
@@ -183,11 +201,12 @@ bool fhip_fast_norm_applicable(const fhip_norm_desc *d) {
     return false;
   const InnerLayout lay = inner_layout(d->x);
   const int vec = 16 / fhip_dtype_size(d->x.dtype);
-  // rows that do not fit the register-resident kernels go to the long-row
-  // kernels (no fused pointwise chain there)
+  // rows that do not fit the register-resident kernels are walked (reported as a tuned
+  // path without a fused pointwise chain only)
   int chunks, wpr;
   return rows_alike(d, lay, vec) &&
-         (pick_shape(lay.inner, vec, &chunks, &wpr) || fhip_norm_long_applicable(d));
+         (pick_shape(lay.inner, vec, &chunks, &wpr) ||
+          (d->epilogue.count == 0 && d->x.dim[0] <= 65535));
 }
 
 // Dense rows that the kernels above leave: any length, element alignment (the
@@ -202,7 +221,7 @@ int fhip_loose_norm(fhip_ctx *ctx, const fhip_norm_desc *d, const void *x, const
     return 0;
   RowNormArgs g{};
   fill_args(d, lay, x, scale, bias, epi, out, mean, inv_variance, g);
-  return fhip_norm_walk(ctx, d->x.dtype, g);
+  return fhip_norm_walk(ctx, d->x.dtype, g, false);
 }
 
 int fhip_fast_norm(fhip_ctx *ctx, const fhip_norm_desc *d, const void *x,
@@ -211,19 +230,19 @@ int fhip_fast_norm(fhip_ctx *ctx, const fhip_norm_desc *d, const void *x,
   const InnerLayout lay = inner_layout(d->x);
   const int vec = 16 / fhip_dtype_size(d->x.dtype);
   int chunks = 1, wpr = 1;
-  if (!pick_shape(lay.inner, vec, &chunks, &wpr))
-    return fhip_norm_long(ctx, d, lay.inner, x, scale, bias, out, mean,
-                          inv_variance);
+  const bool held = pick_shape(lay.inner, vec, &chunks, &wpr);
   RowNormArgs g{};
   fill_args(d, lay, x, scale, bias, epi, out, mean, inv_variance, g);
   // 16-byte alignment of every vector-accessed base pointer.
   auto aligned = [](const void *p) { return ((uintptr_t)p & 15u) == 0; };
-  FHIP_REQUIRE(ctx, aligned(x) && aligned(out) && aligned(scale) &&
-                        aligned(bias),
+  FHIP_REQUIRE(ctx, aligned(x) && aligned(out) && (!held || (aligned(scale) && aligned(bias))),
                "rownorm: tensor base pointers must be 16-byte aligned");
   for (int i = 0; i < epi.count; ++i)
-    FHIP_REQUIRE(ctx, g.epi[i].col_unit == 0 || aligned(g.epi[i].ptr),
+    FHIP_REQUIRE(ctx, !held || g.epi[i].col_unit == 0 || aligned(g.epi[i].ptr),
                  "rownorm: epilogue operand must be 16-byte aligned");
+  const bool cut = held && cut_pays(d, g.rows, g.inner, chunks, ctx);
+  if (!held || cut)
+    return fhip_norm_walk(ctx, d->x.dtype, g, cut);
   // Choose the compile-time specialisation that matches this call exactly.
   int variant = RN_GENERAL;
   const bool scale_same = scale && d->scale.dtype == d->x.dtype;

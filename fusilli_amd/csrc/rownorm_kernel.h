@@ -33,7 +33,9 @@ struct RowNormArgs {
 };
 
 // Rows of any length and alignment (rownorm_walk.hip).
-int fhip_norm_walk(fhip_ctx *ctx, int dtype, const RowNormArgs &n);
+// `cut_pays`: segments are the better choice up to 16 rows per compute unit.
+int fhip_norm_walk(fhip_ctx *ctx, int dtype, const RowNormArgs &n, bool cut_pays);
+int fhip_norm_walk_splits(fhip_ctx *ctx, int dtype, int64_t rows, int64_t inner, bool many_pay);
 
 // Compile-time specialisations of the per-row work.  Everything a variant
 // fixes is resolved at compile time so the hot loop is straight-line code; the

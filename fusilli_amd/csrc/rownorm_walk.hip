@@ -1,21 +1,24 @@
-// RMSNorm / LayerNorm forward for the dense rows that neither the
-// register-resident nor the long-row kernels take: lengths and row strides that
-// are no multiple of a 16-byte vector, long rows with a fused pointwise chain.
+// RMSNorm / LayerNorm forward for the dense rows that the register-resident kernels do not
+// take or leave: lengths and row strides that are no multiple of a 16-byte vector, rows too
+// long for registers, few long ones.
 //
-// Bound by memory (long rows) or by the latency of one launch (short ones); the
-// generic kernel they ran on moves one element per thread with 64-bit index
-// arithmetic, one workgroup per row whatever the row count.  Here a row's storage
+// Bound by memory (long rows) or by the latency of the launches (short ones); the
+// generic kernel moves one element per thread with 64-bit index arithmetic, one
+// workgroup per row whatever the row count.  Here a row's storage
 // is walked linearly with 16-byte loads at element alignment (a misaligned vector
-// costs one more cache line per wavefront, not one per lane) and the statistics are
-// taken as before: the mean first, then the second moment around it.
+// costs one more cache line per wavefront, not one per lane) and the second moment is
+// taken around a mean.
 //   * short rows: one wavefront each (four rows per workgroup), longer ones a
 //     workgroup each; the second and third walk hit the caches;
-//   * few long rows: segments of a row on workgroups of their own, sums through
-//     the context's scratch, added in a fixed order (one launch per walk).
+//   * few long rows: segments of a row on workgroups of their own, in two launches,
+//     sums through the context's scratch, added in a fixed order.
 //
-// bf16 RMSNorm + MUL 2 x 239616: 2465 us -> 8.6; f32 9 x 97280: 997 -> 8.7; bf16
-// 16000 x 1003: 207 -> 20.3 (3.2 TB/s); f16 LayerNorm 9000 x 3001: 442 -> 49 (2.2 TB/s).
-// (Unrolling the walk four times is slower: 49 -> 55.6.)
+// bf16 16000 x 1003 RMSNorm + MUL: 207 us (generic) -> 20.3 (3.2 TB/s); f16 LayerNorm 9000 x
+// 3001: 442 -> 49 (2.2 TB/s).  (Unrolling the walk four times is slower: 49 -> 55.6.)
+// Segments: bf16 LayerNorm 16 x 262144 9.6 us, of which two launches that do next to nothing
+// take 7; 600 x 300000 329 -> 237 (a pivot in place of the segments' means, segments of
+// eight vectors per thread walked, scale and bias fetched after the sums); a launch per sum
+// and whole rows, bf16 LayerNorm 204 x 9335 13.3 -> 9.4.
 //
 // Reference semantics: aten.rms_norm / aten.layer_norm over all dims except
 // dim 0 (reference support/asm_emitter.h:1592-1626, 1427-1503;
@@ -27,10 +30,12 @@
 namespace {
 
 constexpr int kRwThreads = 256;
+constexpr int kRwWaves = kRwThreads / 64;
+constexpr int64_t kRwResident = 16384; // vectors of the longest rows that rownorm_kernel.h holds
 
 struct RowWalkArgs {
   RowNormArgs n;
-  double *partial; // [2][rows][splits]: sums of x, centred second moments
+  double *partial; // [rows][splits][2]: sums of x, second moments around the segment's mean
   double inv;      // 1 / elements per row
   int64_t seg;     // elements per segment, a multiple of the vector width
   int32_t splits;
@@ -63,6 +68,23 @@ template <typename T> struct RwVec {
     for (int k = 0; k < kN; ++k)
       if (k < live)
         p[k] = (T)v[k];
+  }
+  // the same, kept in the row's type
+  static __device__ __forceinline__ loose load_raw(const T *p, int live) {
+    loose t;
+    if (live == kN) {
+      t = *(const loose *)p;
+    } else {
+#pragma unroll
+      for (int k = 0; k < kN; ++k)
+        t[k] = k < live ? p[k] : (T)0.f;
+    }
+    return t;
+  }
+  static __device__ __forceinline__ void widen(const loose &t, float (&v)[kN]) {
+#pragma unroll
+    for (int k = 0; k < kN; ++k)
+      v[k] = (float)t[k];
   }
   // an operand of the row's type or f32
   static __device__ __forceinline__ void load_as(const void *p, int dt, int64_t at, int live,
@@ -126,38 +148,92 @@ template <int WAVES> __device__ __forceinline__ double rw_sum(double v, double *
   return v;
 }
 
+// Sum of the first `live` x (MOMENT 1) or (x - mean)^2 (MOMENT 2) of a vector.
+template <typename T, int MOMENT>
+__device__ __forceinline__ double rw_tree(const float (&v)[RwVec<T>::kN], float mean, int live) {
+  constexpr int N = RwVec<T>::kN;
+  float t[N];
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    const float d = v[k] - mean;
+    t[k] = k < live ? (MOMENT == 1 ? v[k] : d * d) : 0.f;
+  }
+#pragma unroll
+  for (int n = N / 2; n > 0; n >>= 1)
+#pragma unroll
+    for (int k = 0; k < n; ++k)
+      t[k] += t[k + n];
+  return (double)t[0];
+}
+
 // This lane's part of sum x (MOMENT 1) or sum (x - mean)^2 (MOMENT 2) of [lo, hi).
 template <typename T, int MOMENT>
 __device__ __forceinline__ double rw_walk(const T *xr, float mean, int64_t lo, int64_t hi, int lane,
                                           int lanes) {
   using V = RwVec<T>;
   double s = 0.;
-  auto add = [&](const float (&v)[V::kN], int live) {
-    float t[V::kN];
-#pragma unroll
-    for (int k = 0; k < V::kN; ++k) {
-      const float d = v[k] - mean;
-      t[k] = k < live ? (MOMENT == 1 ? v[k] : d * d) : 0.f;
-    }
-#pragma unroll
-    for (int n = V::kN / 2; n > 0; n >>= 1)
-#pragma unroll
-      for (int k = 0; k < n; ++k)
-        t[k] += t[k + n];
-    s += (double)t[0];
-  };
   int64_t i = lo + (int64_t)lane * V::kN;
   for (; i + V::kN <= hi; i += (int64_t)lanes * V::kN) {
     float v[V::kN];
     V::load(xr + i, v);
-    add(v, V::kN);
+    s += rw_tree<T, MOMENT>(v, mean, V::kN);
   }
   if (i < hi) {
     float v[V::kN];
     V::load_some(xr + i, (int)(hi - i), v);
-    add(v, (int)(hi - i));
+    s += rw_tree<T, MOMENT>(v, mean, (int)(hi - i));
   }
   return s;
+}
+
+// Normalises, finishes and stores the `live` elements from `i` of a row, whose X, scale and
+// bias (where there are any) are in x, sc and bi.
+template <typename T>
+__device__ __forceinline__ void rw_finish(const RowNormArgs &g, int64_t row, float mean, float rstd,
+                                          int64_t i, int live, const float (&x)[RwVec<T>::kN],
+                                          const float (&sc)[RwVec<T>::kN], const float (&bi)[RwVec<T>::kN]) {
+  using V = RwVec<T>;
+  constexpr int N = V::kN;
+  float y[N], t[N];
+#pragma unroll
+  for (int k = 0; k < N; ++k)
+    y[k] = (x[k] - mean) * rstd;
+  if (g.scale) {
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+      y[k] *= sc[k];
+  }
+  if (g.bias) {
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+      y[k] += bi[k];
+  }
+  fhip_round_fast_vec<N>(g.y_dt, y);
+  for (int e = 0; e < g.epi_count; ++e) {
+    const FastEpiOp &o = g.epi[e];
+    if (o.kind == FHIP_OPERAND_NONE) {
+      fhip_pw_fast_unary_vec<false, N>(o.mode, y, o.params.swish_beta);
+    } else {
+      if (o.kind == FHIP_OPERAND_TENSOR && o.col_unit) {
+        V::load_as(o.ptr, o.operand_dtype, row * o.row_stride + i, live, t);
+      } else {
+        const float s = o.kind == FHIP_OPERAND_SCALAR ? o.scalar
+                        : o.operand_dtype == DtypeOf<T>::value
+                            ? (float)((const T *)o.ptr)[row * o.row_stride]
+                            : ((const float *)o.ptr)[row * o.row_stride];
+#pragma unroll
+        for (int k = 0; k < N; ++k)
+          t[k] = s;
+      }
+      fhip_pw_fast_binary_vec<N>(o.mode, o.acc_is_in1 != 0, y, t);
+    }
+    fhip_round_fast_vec<N>(o.result_dtype, y);
+  }
+  T *orow = (T *)g.out + row * g.out_row_stride;
+  if (live == N)
+    V::store(orow + i, y);
+  else
+    V::store_some(orow + i, live, y);
 }
 
 template <typename T>
@@ -166,51 +242,15 @@ __device__ __forceinline__ void rw_apply(const RowNormArgs &g, int64_t row, floa
   using V = RwVec<T>;
   constexpr int N = V::kN;
   const T *xr = (const T *)g.x + row * g.x_row_stride;
-  T *orow = (T *)g.out + row * g.out_row_stride;
   for (int64_t i = lo + (int64_t)lane * N; i < hi; i += (int64_t)lanes * N) {
     const int live = hi - i < N ? (int)(hi - i) : N;
-    float y[N], t[N];
-    V::load_as(xr, DtypeOf<T>::value, i, live, y);
-#pragma unroll
-    for (int k = 0; k < N; ++k)
-      y[k] = (y[k] - mean) * rstd;
-    if (g.scale) {
-      V::load_as(g.scale, g.scale_dt, i, live, t);
-#pragma unroll
-      for (int k = 0; k < N; ++k)
-        y[k] *= t[k];
-    }
-    if (g.bias) {
-      V::load_as(g.bias, g.bias_dt, i, live, t);
-#pragma unroll
-      for (int k = 0; k < N; ++k)
-        y[k] += t[k];
-    }
-    fhip_round_fast_vec<N>(g.y_dt, y);
-    for (int e = 0; e < g.epi_count; ++e) {
-      const FastEpiOp &o = g.epi[e];
-      if (o.kind == FHIP_OPERAND_NONE) {
-        fhip_pw_fast_unary_vec<false, N>(o.mode, y, o.params.swish_beta);
-      } else {
-        if (o.kind == FHIP_OPERAND_TENSOR && o.col_unit) {
-          V::load_as(o.ptr, o.operand_dtype, row * o.row_stride + i, live, t);
-        } else {
-          const float s = o.kind == FHIP_OPERAND_SCALAR ? o.scalar
-                          : o.operand_dtype == DtypeOf<T>::value
-                              ? (float)((const T *)o.ptr)[row * o.row_stride]
-                              : ((const float *)o.ptr)[row * o.row_stride];
-#pragma unroll
-          for (int k = 0; k < N; ++k)
-            t[k] = s;
-        }
-        fhip_pw_fast_binary_vec<N>(o.mode, o.acc_is_in1 != 0, y, t);
-      }
-      fhip_round_fast_vec<N>(o.result_dtype, y);
-    }
-    if (live == N)
-      V::store(orow + i, y);
-    else
-      V::store_some(orow + i, live, y);
+    float x[N], sc[N], bi[N];
+    V::load_as(xr, DtypeOf<T>::value, i, live, x);
+    if (g.scale)
+      V::load_as(g.scale, g.scale_dt, i, live, sc);
+    if (g.bias)
+      V::load_as(g.bias, g.bias_dt, i, live, bi);
+    rw_finish<T>(g, row, mean, rstd, i, live, x, sc, bi);
   }
 }
 
@@ -238,44 +278,151 @@ __global__ __launch_bounds__(kRwThreads) void rownorm_walk_kernel(RowNormArgs g,
   rw_apply<T>(g, row, mean, rstd, 0, g.inner, lane, kLanes);
 }
 
-// The sum of a row's parts (at most one per thread).
-__device__ __forceinline__ double rw_parts(const RowWalkArgs &g, int moment, int64_t row, double *lds) {
-  const double *p = g.partial + ((moment - 1) * g.n.rows + row) * g.splits;
-  return rw_sum<kRwThreads / 64>((int)threadIdx.x < g.splits ? p[threadIdx.x] : 0., lds);
-}
+// Few long rows: a segment of a row per workgroup, two launches.  The first leaves every
+// segment's sum and its second moment around the segment's own mean (RMSNorm: around zero);
+// the second adds a row's pairs up, moved to the first segment's mean, and applies.  NV > 0:
+// a thread's NV vectors of the segment stay in registers between the two sums, and come with
+// their scale and bias while the pairs are on their way; 0: segments of any length are walked.
+// (A segment per wavefront, no barrier in the first launch, but four times the pairs: bf16
+// 4 x 65544 7.5 -> 7.9 us, f32 32 x 524288 34.8 -> 40.6.)
+typedef double rw_pair __attribute__((ext_vector_type(2)));
 
-template <typename T, int MOMENT>
+template <typename T, int NV>
 __global__ __launch_bounds__(kRwThreads) void rownorm_walk_sums_kernel(RowWalkArgs g) {
-  __shared__ double lds[kRwThreads / 64];
+  using V = RwVec<T>;
+  constexpr int N = V::kN;
+  __shared__ double lds[kRwWaves];
   const int64_t row = blockIdx.y, lo = blockIdx.x * g.seg;
   const int64_t hi = lo + g.seg < g.n.inner ? lo + g.seg : g.n.inner;
-  float mean = 0.f;
-  if (MOMENT == 2 && g.n.is_layernorm)
-    mean = (float)(rw_parts(g, 1, row, lds) * g.inv);
   const T *xr = (const T *)g.n.x + row * g.n.x_row_stride;
-  const double s = rw_sum<kRwThreads / 64>(rw_walk<T, MOMENT>(xr, mean, lo, hi, threadIdx.x, kRwThreads), lds);
+  double s1 = 0., s2 = 0.;
+  float mean = 0.f;
+  if constexpr (NV > 0) {
+    typename V::loose raw[NV];
+    int live[NV];
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const int64_t i = lo + (int64_t)(threadIdx.x + j * kRwThreads) * N;
+      live[j] = hi - i >= N ? N : hi > i ? (int)(hi - i) : 0;
+      raw[j] = V::load_raw(xr + i, live[j]);
+    }
+    if (g.n.is_layernorm) {
+#pragma unroll
+      for (int j = 0; j < NV; ++j) {
+        float v[N];
+        V::widen(raw[j], v);
+        s1 += rw_tree<T, 1>(v, 0.f, live[j]);
+      }
+      s1 = rw_sum<kRwWaves>(s1, lds);
+      mean = (float)(s1 / (double)(hi - lo));
+    }
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      float v[N];
+      V::widen(raw[j], v);
+      s2 += rw_tree<T, 2>(v, mean, live[j]);
+    }
+  } else {
+    if (g.n.is_layernorm) {
+      s1 = rw_sum<kRwWaves>(rw_walk<T, 1>(xr, 0.f, lo, hi, threadIdx.x, kRwThreads), lds);
+      mean = (float)(s1 / (double)(hi - lo));
+    }
+    s2 = rw_walk<T, 2>(xr, mean, lo, hi, threadIdx.x, kRwThreads);
+  }
+  s2 = rw_sum<kRwWaves>(s2, lds);
   if (threadIdx.x == 0)
-    g.partial[((MOMENT - 1) * g.n.rows + row) * g.splits + blockIdx.x] = s;
+    ((rw_pair *)g.partial)[row * g.splits + blockIdx.x] = rw_pair{s1, s2};
 }
 
-template <typename T>
+template <typename T, int NV>
 __global__ __launch_bounds__(kRwThreads) void rownorm_walk_apply_kernel(RowWalkArgs g) {
-  __shared__ double lds[kRwThreads / 64];
+  using V = RwVec<T>;
+  constexpr int N = V::kN;
+  __shared__ rw_pair lds[kRwWaves];
   const int64_t row = blockIdx.y, lo = blockIdx.x * g.seg;
   const int64_t hi = lo + g.seg < g.n.inner ? lo + g.seg : g.n.inner;
-  const float mean = g.n.is_layernorm ? (float)(rw_parts(g, 1, row, lds) * g.inv) : 0.f;
-  const float rstd = 1.0f / sqrtf((float)(rw_parts(g, 2, row, lds) * g.inv) + g.n.eps);
+  // the pairs first: loads return in order
+  const rw_pair *p = (const rw_pair *)g.partial + row * g.splits;
+  const double first = p[0].x;
+  const bool in = threadIdx.x < (unsigned)g.splits; // (at most one per thread)
+  const rw_pair mine = p[in ? threadIdx.x : 0];
+  typename V::loose rx[NV > 0 ? NV : 1], rs[NV > 0 ? NV : 1], rb[NV > 0 ? NV : 1];
+  const bool own_s = g.n.scale && g.n.scale_dt == DtypeOf<T>::value;
+  const bool own_b = g.n.bias && g.n.bias_dt == DtypeOf<T>::value;
+  if constexpr (NV > 0) {
+    const T *xr = (const T *)g.n.x + row * g.n.x_row_stride;
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const int64_t i = lo + (int64_t)(threadIdx.x + j * kRwThreads) * N;
+      const int live = hi - i >= N ? N : hi > i ? (int)(hi - i) : 0;
+      rx[j] = V::load_raw(xr + i, live);
+      if (own_s)
+        rs[j] = V::load_raw((const T *)g.n.scale + i, live);
+      if (own_b)
+        rb[j] = V::load_raw((const T *)g.n.bias + i, live);
+    }
+  }
+  // sum (x - c0)^2 = sum (x - c)^2 + 2 d (sum x - n c) + n d^2 of a segment whose second
+  // moment lies around c, d = c - c0 (RMSNorm: all zero)
+  const double n0 = (double)(g.seg < g.n.inner ? g.seg : g.n.inner);
+  const double c0 = g.n.is_layernorm ? (double)(float)(first / n0) : 0.;
+  const int64_t left = g.n.inner - (in ? threadIdx.x : 0) * g.seg;
+  const double n = (double)(left < g.seg ? left : g.seg);
+  const double c = g.n.is_layernorm ? (double)(float)(mine.x / n) : 0., d = c - c0;
+  double s = rw_wave_sum(in ? mine.x : 0.);
+  double q = rw_wave_sum(in ? mine.y + 2. * d * (mine.x - n * c) + n * d * d : 0.);
+  if ((threadIdx.x & 63) == 0)
+    lds[threadIdx.x >> 6] = rw_pair{s, q};
+  __syncthreads();
+  s = q = 0.;
+#pragma unroll
+  for (int i = 0; i < kRwWaves; ++i) {
+    s += lds[i].x;
+    q += lds[i].y;
+  }
+  s *= g.inv;
+  q *= g.inv;
+  const float mean = (float)s;
+  const double e = (double)mean - c0, around = q - 2. * e * (s - c0) + e * e;
+  const float var = g.n.is_layernorm ? (around < 0. ? 0.f : (float)around) : (float)q;
+  const float rstd = 1.0f / sqrtf(var + g.n.eps);
   if (g.n.emit_stats && blockIdx.x == 0 && threadIdx.x == 0)
     rw_stats(g.n, row, mean, rstd);
-  rw_apply<T>(g.n, row, mean, rstd, lo, hi, threadIdx.x, kRwThreads);
+  if constexpr (NV > 0) {
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const int64_t i = lo + (int64_t)(threadIdx.x + j * kRwThreads) * N;
+      if (i >= hi)
+        break;
+      const int live = hi - i < N ? (int)(hi - i) : N;
+      float v[N], sc[N], bi[N];
+      V::widen(rx[j], v);
+      if (own_s)
+        V::widen(rs[j], sc);
+      else if (g.n.scale)
+        V::load_as(g.n.scale, g.n.scale_dt, i, live, sc);
+      if (own_b)
+        V::widen(rb[j], bi);
+      else if (g.n.bias)
+        V::load_as(g.n.bias, g.n.bias_dt, i, live, bi);
+      rw_finish<T>(g.n, row, mean, rstd, i, live, v, sc, bi);
+    }
+  } else {
+    rw_apply<T>(g.n, row, mean, rstd, lo, hi, threadIdx.x, kRwThreads);
+  }
 }
 
 template <typename T> void rw_launch_split(hipStream_t stream, const RowWalkArgs &g) {
   const dim3 grid((unsigned)g.splits, (unsigned)g.n.rows), wg(kRwThreads);
-  if (g.n.is_layernorm)
-    hipLaunchKernelGGL((rownorm_walk_sums_kernel<T, 1>), grid, wg, 0, stream, g);
-  hipLaunchKernelGGL((rownorm_walk_sums_kernel<T, 2>), grid, wg, 0, stream, g);
-  hipLaunchKernelGGL(rownorm_walk_apply_kernel<T>, grid, wg, 0, stream, g);
+  auto go = [&](auto nv) {
+    constexpr int NV = decltype(nv)::value;
+    hipLaunchKernelGGL((rownorm_walk_sums_kernel<T, NV>), grid, wg, 0, stream, g);
+    hipLaunchKernelGGL((rownorm_walk_apply_kernel<T, NV>), grid, wg, 0, stream, g);
+  };
+  if (g.seg <= 2 * kRwThreads * RwVec<T>::kN)
+    go(std::integral_constant<int, 2>{});
+  else
+    go(std::integral_constant<int, 0>{});
 }
 
 template <typename T> void rw_launch_rows(hipStream_t stream, const RowNormArgs &g, int waves) {
@@ -288,31 +435,41 @@ template <typename T> void rw_launch_rows(hipStream_t stream, const RowNormArgs 
 
 } // namespace
 
+// Segments that a row is cut into, 1: none.  Rows of more than four vectors per thread of a
+// workgroup are cut into segments of two vectors per thread, 256 at most (a pair per thread of
+// the second launch), unless there are so many rows that whole ones, which take one launch and
+// read X from memory once, keep up (bf16 8000 x 16387 LayerNorm 196 us whole / 204 in
+// segments, f16 1500 x 40001 80 / 71; RMSNorm, which walks a row twice and not three times,
+// bf16 600 x 16387 19.4 / 17.4, f32 700 x 60001 134 / 87, 1200 x 30001 74 / 71, bf16 3000 x
+// 20001 63 / 65).  Segments' sums need the context's scratch.
+int fhip_norm_walk_splits(fhip_ctx *ctx, int dtype, int64_t rows, int64_t inner, bool many_pay) {
+  const int64_t vec = 16 / (int64_t)fhip_dtype_size(dtype);
+  const int64_t cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+  const int64_t unit = 2 * kRwThreads * vec;
+  int64_t splits = (inner + unit - 1) / unit;
+  splits = splits < kRwThreads ? splits : kRwThreads;
+  const bool many = rows >= (many_pay ? 16 : 4) * cus && inner <= kRwResident * vec;
+  if (inner <= 2 * unit || many || rows > 65535 ||
+      !fhip_ctx_scratch_ready(ctx, (size_t)(2 * rows * splits) * sizeof(double)))
+    return 1;
+  return (int)splits;
+}
+
 // The caller (rownorm.hip) has checked that rows are dense and that X, OUT, scale,
 // bias and the fused operands walk a row alike.
-int fhip_norm_walk(fhip_ctx *ctx, int dtype, const RowNormArgs &n) {
+int fhip_norm_walk(fhip_ctx *ctx, int dtype, const RowNormArgs &n, bool cut_pays) {
   // A wavefront per row up to four vectors per lane, where the rows then still
   // fill half of the chip's wavefront slots or are shorter than two vectors per lane.
   const int64_t vec = 16 / (int64_t)fhip_dtype_size(dtype);
   const int waves = n.inner <= 128 * vec || (n.inner <= 256 * vec && n.rows >= 4096) ? 1 : 4;
-  // Rows of more than four vectors per thread of a workgroup are cut where there are
-  // fewer of them than two per compute unit, into about eight workgroups per unit and
-  // segments of two vectors per thread at least (one launch more than whole rows).
-  const int64_t cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
-  const int64_t min_seg = kRwThreads * vec * 2;
-  int64_t splits = (8 * cus + n.rows - 1) / n.rows;
-  const int64_t most = (n.inner + min_seg - 1) / min_seg;
-  splits = splits < most ? splits : most;
-  splits = splits < kRwThreads ? splits : kRwThreads;
+  const int64_t splits = fhip_norm_walk_splits(ctx, dtype, n.rows, n.inner, cut_pays || n.is_layernorm);
+  const bool cut = splits > 1;
   RowWalkArgs g{};
-  const size_t sums = (size_t)(2 * n.rows * (splits > 0 ? splits : 0)) * sizeof(double);
-  const bool cut = n.inner > 4 * kRwThreads * vec && n.rows < 2 * cus && splits > 1 &&
-                   fhip_ctx_scratch_ready(ctx, sums);
   if (cut) {
     g.seg = ((n.inner + splits - 1) / splits + vec - 1) / vec * vec;
     g.splits = (int32_t)((n.inner + g.seg - 1) / g.seg);
     void *scratch = nullptr;
-    if (fhip_ctx_scratch(ctx, sums, &scratch) != 0)
+    if (fhip_ctx_scratch(ctx, (size_t)(2 * n.rows * splits) * sizeof(double), &scratch) != 0)
       return 1;
     g.partial = (double *)scratch;
     g.inv = 1.0 / (double)n.inner;

@@ -378,3 +378,43 @@ def test_means_of_walked_rows_are_rounded_once(ctx, dtype, rows, cols):
     ref = x.logical().astype(np.float64).mean(1)
     most = 0.6 if dtype == capi.HALF else 1.0
     assert np.linalg.norm(mean.logical() - ref) <= most * 2.0 ** -24 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("dtype,rows,cols", [
+    # the shortest and the longest rows that a workgroup could hold, a last segment of one
+    # vector, more pairs than a thread each (segments longer than registers hold)
+    (capi.BFLOAT16, 3, 65544), (capi.HALF, 2, 131072), (capi.BFLOAT16, 1, 16 * 4096 + 8),
+    (capi.FLOAT, 2, 49152), (capi.FLOAT, 1, 256 * 2048 + 4), (capi.HALF, 1, 256 * 4096 + 8)])
+@pytest.mark.parametrize("kind", ["layernorm", "rmsnorm", "rmsnorm in place"])
+def test_norm_rows_in_segments_vs_64_bits(ctx, dtype, rows, cols, kind):
+    # segments of unlike means, the largest far from the first element's
+    x = rand(43, 0, [rows, cols], std=1.0)
+    x += np.linspace(0.0, 8.0, cols, dtype=np.float32)
+    x[:, 0] = 200.0
+    x = HT.from_logical(x, dtype)
+    s = HT.from_logical(rand(43, 1, [1, cols], mean=1.0, std=0.1), dtype)
+    v = x.logical().astype(np.float64)
+    if kind == "layernorm":
+        b = HT.from_logical(rand(43, 2, [1, cols]), dtype)
+        out, mean, rstd = run_norm(ctx, x, s, b, eps=1e-5, layernorm=True, stats=True)
+        m, r = v.mean(1), 1.0 / np.sqrt(v.var(1) + 1e-5)
+        y = (v - m[:, None]) * r[:, None] * s.logical() + b.logical()
+        # sums of 64 bits over f32 ones of a vector: the statistics' own rounding, twice
+        assert np.all(np.abs(mean.logical() - m) <= 2.0 ** -23 * np.abs(m))
+        assert np.all(np.abs(rstd.logical() - r) <= 2.0 ** -22 * r)
+    else:
+        mul = [capi.epilogue_op(capi.PW["MUL"], dtype, scalar=0.5)]
+        y = v / np.sqrt((v * v).mean(1) + 1e-6)[:, None] * s.logical() * 0.5
+        if kind == "rmsnorm":
+            out = run_norm(ctx, x, s, None, eps=1e-6, y_dtype=capi.FLOAT, epilogue=mul)
+        else:
+            d = capi.NormDesc()
+            d.x, d.scale, d.out, d.out_dtype = x.desc(), s.desc(), x.desc(), dtype
+            d.y = capi.TensorDesc.make(x.dims, x.strides, capi.FLOAT)
+            d.epsilon, d.epilogue = 1e-6, capi.make_epilogue(mul)
+            dx, ds = x.upload(ctx), s.upload(ctx)
+            ctx.norm_fwd(d, dx, ds, None, dx)
+            out = HT.empty(x.dims, dtype, x.strides)
+            out.fetch(ctx, dx)
+    assert ctx.last_kernel().startswith("rownorm_walk segments="), ctx.last_kernel()
+    assert_close(out.logical(), y, dtype, f"{kind} {rows} x {cols}")
