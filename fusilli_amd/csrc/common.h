@@ -955,6 +955,12 @@ inline bool fhip_epilogue_is_fast(const fhip_epilogue &e) {
   }
   return true;
 }
+inline bool fhip_epilogue_is_transcendental(const fhip_epilogue &e) {
+  for (int i = 0; i < e.count; ++i)
+    if (fhip_pw_is_transcendental(e.op[i].mode))
+      return true;
+  return false;
+}
 // Right-aligned broadcast of `operand` against an output of out_rank/out_dims;
 // writes per-output-dim strides (0 where broadcast).  Returns false when the
 // shapes are not broadcast-compatible.

@@ -10,12 +10,19 @@ bool fhip_fast_matmul_applicable(const fhip_matmul_desc *d);
 int fhip_fast_matmul(fhip_ctx *ctx, const fhip_matmul_desc *d, const void *a,
                      const void *b, const DevEpilogue &epi, void *out);
 
-// Products outside that contract -- few rows or columns, K or row starts that do
-// not fit 128-byte slices, f32 -- on kernels that load MFMA fragments straight
-// from global memory; `handled` false where they do not take the descriptor, `short_k` true
-// where that is for the speed of the general path's f32 tiles over a short K.
+// Whichever tuned kernel an estimate prefers: those of that contract, also where K ends inside
+// a 128-byte slice, or those below.  `handled` false where none takes the descriptor, `short_k`
+// true where that is for the speed of the general path's f32 tiles over a short K.
+int fhip_tuned_matmul(fhip_ctx *ctx, const fhip_matmul_desc *d, const void *a, const void *b,
+                      const DevEpilogue &epi, void *out, bool *handled, bool *short_k);
+
+// Few rows or columns, K or row starts that do not fit that contract, f32, and few tiles, on
+// kernels that load MFMA fragments straight from global memory or stage tiles through
+// registers; `handled` false where they do not take the descriptor or would take longer than
+// `other_us` (0: there is no other).  `whole`: the contract holds.
 int fhip_direct_matmul(fhip_ctx *ctx, const fhip_matmul_desc *d, const void *a, const void *b,
-                       const DevEpilogue &epi, void *out, bool *handled, bool *short_k);
+                       const DevEpilogue &epi, void *out, double other_us, bool whole, bool *handled,
+                       bool *short_k);
 
 // `allow_scratch` false: only plans that leave the context's scratch alone
 // (no zero-padded channel copies, no split reduction) -- for the entry point

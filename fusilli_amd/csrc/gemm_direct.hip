@@ -1,7 +1,8 @@
-// Host side of the direct matrix-product kernels (gemm_direct_kernel.h): which
-// descriptors they take, tile, wavefronts and split of K.
+// Host side of the direct matrix-product kernels (gemm_direct_kernel.h) and of the
+// register-staged tiles (gemm_tile_kernel.h): which descriptors they take, tile, wavefronts
+// and split of K, and the choice between them and the tiled GEMM.
 #include "fast_paths.h"
-#include "gemm_direct_kernel.h"
+#include "gemm_tile_kernel.h"
 
 #include <cmath>
 
@@ -57,7 +58,8 @@ bool short_k(const DirectPlan &p, const DirectArgs &g, int64_t M, int64_t N, int
   return K < (tiles <= 256 ? (p.b_kc ? 20 : 12) : (p.b_kc ? 50 : 40) + (tiles >= 1024 ? 8 : 0));
 }
 
-bool direct_plan(const fhip_matmul_desc *d, DirectPlan *p, DirectArgs *g, int64_t *batch, bool *too_short) {
+bool direct_plan(const fhip_matmul_desc *d, DirectPlan *p, DirectArgs *g, int64_t *batch, double *us,
+                 bool *too_short) {
   const int r = d->a.rank;
   if ((r != 2 && r != 3) || d->a.dtype != d->b.dtype)
     return false;
@@ -134,6 +136,7 @@ bool direct_plan(const fhip_matmul_desc *d, DirectPlan *p, DirectArgs *g, int64_
   }
   if (best == 0)
     return false;
+  *us = best;
   // (16-bit operands into f32: the f32 tiles would be further from the exact sums, f16 K24
   // 1.3 units of 2^-24 against 0.7)
   const bool f32_of_16 = p->kind != GK_F32 && d->c.dtype == FHIP_FLOAT && d->out.dtype == FHIP_FLOAT;
@@ -155,21 +158,118 @@ bool direct_plan(const fhip_matmul_desc *d, DirectPlan *p, DirectArgs *g, int64_
   return true;
 }
 
+// What the planners' estimates leave out, fitted to 400 random products (16 and 8 bits, M from
+// 1 to 4096) that all three families ran: us = once + scale * estimate, more where operands'
+// rows start off 16 bytes, lie along M or N, or the chain ends in GELU.  With them the family
+// chosen is 1.5 % slower than the best one on average; over 400 others 12 % faster than the tiled
+// GEMM where its contract held and the direct kernels elsewhere, up to 4 times.
+struct ProductTimes {
+  struct Line {
+    double once, scale, gelu_once, loose, rows;
+  };
+  int loose, rows; // operands whose rows start off 16 bytes / lie along M or N
+  bool gelu, wide; // 64 x 64 tiles
+  bool few, byte;  // 16 rows; 8-bit operands
+  ProductTimes(const DirectPlan &p, const DirectArgs &g, const fhip_matmul_desc *d, int elem, const void *a,
+               const void *b)
+      : loose(((g.a_ldb | (int64_t)(uintptr_t)a) % 16 != 0) + ((g.b_ldb | (int64_t)(uintptr_t)b) % 16 != 0)),
+        rows(!p.a_kc + !p.b_kc), gelu(fhip_epilogue_is_transcendental(d->epilogue)), wide(p.mt == 4),
+        few(p.mt == 1), byte(elem == 1) {}
+  double of(const Line &l, double us) const {
+    return us > 0 ? l.once + us * (l.scale + l.loose * loose + l.rows * rows) + (gelu ? l.gelu_once : 0.0) : 0.0;
+  }
+  double direct(double us, const DirectArgs &g, int64_t batch) const {
+    static const Line k16[2] = {{2.55, 0.75, 1.12, 0.09, 0.11}, {2.29, 0.89, 1.37, 0.19, 0.11}};
+    static const Line k8[2] = {{2.50, 0.61, 0.54, 0, -0.10}, {1.97, 0.99, 0.47, 0, -0.16}};
+    if (!wide)
+      return of((byte ? k8 : k16)[few ? 0 : 1], us);
+    // 64 x 64 tiles (229 of them): a wavefront's slices at a pace, alone or with another
+    // workgroup, as for the tiles below
+    const double load = (double)((int64_t)g.tiles_m * g.tiles_n * batch * g.splits) / 256.0;
+    const int run = (g.slices + 4 * g.splits - 1) / (4 * g.splits);
+    const double alone = byte ? 0.87 : 1.27, shared = byte ? 2.03 : 2.19;
+    const double pace = (load <= 1.0 ? alone : shared * (load <= 2.0 ? 1.0 : 0.25 * load + 0.5 * ceil(0.5 * load))) *
+                        (byte ? 1.0 + 0.70 * rows : 1.0 + 0.12 * loose + 0.06 * rows);
+    return (byte ? 4.55 : 2.94) + run * pace +
+           fmax(1.0, load) * (byte ? 1.5 + 1.3 * gelu : 2.4 + 1.5 * gelu) +
+           (g.splits > 1 ? 0.3 + (byte ? 0.67 : 0.85) * g.splits * (double)g.tiles_m * g.tiles_n * batch * 4096 * 4e-6
+                         : 0.0);
+  }
+  double tile(double us) const {
+    static const Line k16 = {-0.39, 1.01, 0.34, 0.07, 0.06}, k8 = {-0.91, 1.11, 0.98, 0, 0.06};
+    return of(byte ? k8 : k16, us);
+  }
+};
+
+// The shortest estimate of the LDS-tiled kernels (gemm_tile_kernel.h) for the product that `p`
+// and `g` describe; us, 0: none applies.  A workgroup's time is its slices at a pace (alone on
+// its compute unit, or two to one: they share its LDS) plus what it does once; with a split,
+// the parts' round trip and the second kernel.  Fitted to 453 + 624 times (16 and 8 bits) of
+// random products of 17 to 4096 rows, 256 to 8192 columns and K, in all orientations, on one
+// chip, 10 to 13 % rms; the choice between these tiles loses 2 % against the best of them.
+double tile_plan(const DirectPlan &dp, const DirectArgs &g, int elem, bool gelu, int64_t batch, DirectPlan *p, int *tiles_m,
+                 int *tiles_n, int *splits) {
+  struct Fit {
+    int mt, nt, waves;
+    double once, alone, shared, round, sum, part, gelu;
+  };
+  static const Fit k16[] = {{4, 4, 4, 4.33, 0.253, 0.483, 1.75, 1.77, 0.34, 0.81},
+                             {4, 4, 8, 2.06, 0.444, 1.155, 3.42, 2.36, 0.40, 0.95},
+                             {4, 8, 4, 5.54, 0.412, 0.700, 2.50, 0.00, 0.44, 1.65},
+                             {8, 4, 4, 5.49, 0.402, 0.702, 2.53, 0.57, 0.41, 0.97},
+                             {8, 8, 4, 3.69, 0.662, 1.080, 5.12, 0.00, 0.39, 1.78}};
+  static const Fit k8[] = {{4, 4, 4, 3.76, 0.188, 0.497, 1.35, 1.90, 0.45, 1.00},
+                             {4, 4, 8, 2.84, 0.334, 1.354, 2.05, 2.16, 0.55, 1.00},
+                             {4, 8, 4, 4.24, 0.303, 0.680, 2.39, 0.97, 0.57, 1.00},
+                             {8, 4, 4, 3.61, 0.297, 0.681, 2.45, 1.66, 0.48, 1.00},
+                             {8, 8, 4, 2.11, 0.470, 1.002, 5.22, 0.81, 0.52, 1.00}};
+  const int pe = 16 / elem;
+  if ((!dp.a_kc && g.M < pe) || (!dp.b_kc && g.N < pe)) // (whole chunks of the other operand)
+    return 0;
+  double best = 0;
+  for (const Fit &f : elem == 2 ? k16 : k8) {
+    const int bm = 16 * f.mt, bn = 16 * f.nt;
+    const int64_t tm = (g.M + bm - 1) / bm, tn = (g.N + bn - 1) / bn;
+    if (tm * tn >= (1ll << 31))
+      continue;
+    for (int split = 1; split <= 16; ++split) {
+      const int run = (g.slices + split - 1) / split;
+      if (split > 1 && (run < 3 || tm * tn * batch * split > 2048))
+        break;
+      const double load = (double)(tm * tn * batch * split) / 256.0;
+      const double pace = load <= 1.0 ? f.alone
+                                      : f.shared * (load <= 2.0 ? 1.0 : 0.25 * load + 0.5 * ceil(0.5 * load));
+      const int teams = f.waves / 4;
+      double us = f.once + (double)((run + teams - 1) / teams) * pace + fmax(1.0, load) * (f.round + (gelu ? f.gelu : 0.0));
+      if (split > 1)
+        us += f.sum + f.part * split * (double)(tm * tn * batch * bm * bn) * 4e-6;
+      if (best == 0 || us < best) {
+        best = us;
+        *p = dp;
+        p->tile = true, p->mt = f.mt, p->nt = f.nt, p->waves = f.waves;
+        *tiles_m = (int)tm, *tiles_n = (int)tn, *splits = split;
+      }
+    }
+  }
+  return best;
+}
+
 } // namespace
 
 int fhip_direct_matmul(fhip_ctx *ctx, const fhip_matmul_desc *d, const void *a, const void *b,
-                       const DevEpilogue &epi, void *out, bool *handled, bool *short_k) {
+                       const DevEpilogue &epi, void *out, double other_us, bool whole, bool *handled,
+                       bool *short_k) {
   *handled = *short_k = false;
   DirectPlan p;
   DirectArgs g{};
   int64_t batch = 1;
-  if (!direct_plan(d, &p, &g, &batch, short_k))
+  double us = 0;
+  if (!direct_plan(d, &p, &g, &batch, &us, short_k))
     return 0;
   // operands at their own alignment
   const uintptr_t am = fhip_dtype_size(d->a.dtype) - 1;
   if ((((uintptr_t)a | (uintptr_t)b) & am) != 0)
     return 0;
-  *handled = true;
   g.a = (const char *)a;
   g.b = (const char *)b;
   g.out = (char *)out;
@@ -183,12 +283,59 @@ int fhip_direct_matmul(fhip_ctx *ctx, const fhip_matmul_desc *d, const void *a, 
     o.stride[1] = s.stride[r - 2];
     o.stride[2] = s.stride[r - 1];
   }
+  g.lean = fhip_epilogue_is_fast(d->epilogue), g.lean_op = -1;
+  for (int i = 0; i < epi.count; ++i) {
+    const DevEpiOp &o = g.epi.op[i];
+    if (o.kind == FHIP_OPERAND_TENSOR) {
+      const bool typed = o.operand_dtype == FHIP_FLOAT || o.operand_dtype == FHIP_BFLOAT16 || o.operand_dtype == FHIP_HALF;
+      if (o.stride[0] != 0 || o.stride[1] != 0 || !typed || g.lean_op >= 0)
+        g.lean = 0;
+      g.lean_op = i;
+    }
+  }
+  // f32 results of 16-bit or fp8 operands keep the kernel they had: the length of the chains
+  // that the sums are taken in shows there.
+  const bool f32_out = p.kind != GK_I8 && d->c.dtype == FHIP_FLOAT && d->out.dtype == FHIP_FLOAT;
+  // Split products over a long K stay on the tiled GEMM, those over less than a slice here.
+  if (whole && (f32_out || g.slices >= 128))
+    return 0;
+  if (p.kind != GK_F32 && !f32_out && g.slices > 1) {
+    DirectPlan t;
+    int tm = 0, tn = 0, splits = 1;
+    const int elem = fhip_dtype_size(d->a.dtype);
+    const ProductTimes times(p, g, d, elem, a, b);
+    // the kernel that took the product before there were tiles of every size, or the tiled
+    // GEMM where K fills no slice; the tiles where they clearly outrun it
+    const double direct_us = times.direct(us, g, batch);
+    const bool other = other_us > 0 && (whole || other_us * 1.08 < direct_us);
+    const double known_us = other ? other_us : direct_us;
+    // (tiles that are at least half full; none takes less than 6 us)
+    const bool fills = g.M > 32 && g.N > 32 && (int64_t)g.M * g.N >= 2048 && known_us > 6.0;
+    const double tile_us =
+        fills ? times.tile(tile_plan(p, g, elem, times.gelu, batch, &t, &tm, &tn, &splits)) : 0;
+    if (tile_us > 0 && tile_us * (other ? 1.08 : 1.04) < known_us)
+      p = t, g.tiles_m = tm, g.tiles_n = tn, g.splits = splits;
+    else if (other)
+      return 0;
+  }
+  *handled = true;
   if (g.splits > 1) {
     const size_t bytes = (size_t)g.splits * (size_t)batch * g.tiles_m * g.tiles_n * (p.mt * p.nt * 1024);
     if (!fhip_ctx_scratch_ready(ctx, bytes))
       g.splits = 1;
     else if (fhip_ctx_scratch(ctx, bytes, &g.partial) != 0)
       return 1;
+  }
+  if (p.tile) {
+    static const char *const kKindName[] = {"bf16", "f16", "i8", "fp8e4m3", "fp8e5m2"};
+    fhip_note_kernel(ctx, "gemm_mfma %s %dx%d waves=%d split=%d", kKindName[p.kind], 16 * p.mt, 16 * p.nt, p.waves, g.splits);
+    switch (p.kind) {
+    case GK_BF16: return tile_launch_bf16(ctx, p, g, batch);
+    case GK_F16: return tile_launch_f16(ctx, p, g, batch);
+    case GK_I8: return tile_launch_i8(ctx, p, g, batch);
+    case GK_FP8E4M3: return tile_launch_fp8e4m3(ctx, p, g, batch);
+    default: return tile_launch_fp8e5m2(ctx, p, g, batch);
+    }
   }
   fhip_note_kernel(ctx, "gemm_direct %dx%d waves=%d split=%d", 16 * p.mt, 16 * p.nt, p.waves, g.splits);
   switch (p.kind) {

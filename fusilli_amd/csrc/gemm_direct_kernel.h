@@ -48,6 +48,9 @@ struct DirectArgs {
   int32_t tiles_m, tiles_n;
   int32_t slices, splits; // of K; workgroups that share a tile's
   int32_t c_dt, o_dt;
+  // fused chain of fast modes whose operands are scalars but for one at most (`lean_op`, -1:
+  // none), which depends on the column alone
+  int32_t lean, lean_op;
   DevEpilogue epi; // strides over (batch, m, n)
 };
 
@@ -514,6 +517,7 @@ struct DirectPlan {
   int kind = 0;
   bool a_kc = true, b_kc = true;
   int mt = 1, nt = 1, waves = 1;
+  bool tile = false; // gemm_tile_kernel.h
 };
 
 template <int KIND, bool A_KC, bool B_KC, int MT, int NT, int U, int MAXW>

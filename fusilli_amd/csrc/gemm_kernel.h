@@ -315,6 +315,24 @@ dma_setup(int group0, int64_t ld_bytes, int64_t row0, int64_t rows_total,
   }
 }
 
+// The same offsets for a slice that ends after `rest` bytes of K: loads of what lies
+// behind them (whole 16-byte chunks of a K-contiguous row, whole K-rows) read past
+// 2^31, where the caller's descriptor ends, and bring zeros.
+template <int ROWS, int ELEM, bool KCONTIG, int NW, int STEP, int J0, int J1>
+__device__ __forceinline__ void dma_cut(int group0, int rest,
+                                        const uint32_t (&off)[SliceGeom<ROWS, ELEM, KCONTIG, NW>::kLoads],
+                                        uint32_t (&cut)[SliceGeom<ROWS, ELEM, KCONTIG, NW>::kLoads]) {
+  using G = SliceGeom<ROWS, ELEM, KCONTIG, NW>;
+  const int l = threadIdx.x & 63;
+#pragma unroll
+  for (int j = J0; j < J1; ++j) {
+    const int group = group0 + j * STEP;
+    const int at = KCONTIG ? ((l & 7) ^ kc_swz(group * 8 + (l >> 3))) * 16
+                           : (group * G::kRowsPerLoad + l / G::kCPR) * ELEM;
+    cut[j] = at < rest ? off[j] : 0x80000000u;
+  }
+}
+
 // This wavefront's loads of one K slice of one operand, global -> LDS (its first
 // group to `lds_dst`, the others STEP KB apart): each wavefront instruction moves
 // 64 x 16 bytes to 1024 consecutive LDS bytes.  Buffer addressing (uniform
@@ -629,7 +647,9 @@ template <int BM, int BN, int NSTAGE, int NW, bool HALO = false> struct GemmLds 
 
 // Halo kernels are laid out for two workgroups per compute unit (two
 // wavefronts per SIMD): at most 256 registers per lane.
-template <int KIND, int BM, int BN, int A_MODE, bool B_KC, int NSTAGE, int NW>
+// CUT: K ends inside its last slice (matrix products; a variant of its own, because the test
+// for that slice costs the others 0.5 us of 8 and 1 to 3 % of large products).
+template <int KIND, int BM, int BN, int A_MODE, bool B_KC, int NSTAGE, int NW, bool CUT = false>
 __global__ __launch_bounds__(NW * 64)
 __attribute__((amdgpu_waves_per_eu(A_MODE == A_HALO ? 2 : 1, 8))) void
 gemm_kernel(GemmArgs g) {
@@ -698,9 +718,16 @@ gemm_kernel(GemmArgs g) {
   // first row past this tile's share of the output
   const int64_t m_end = m0 + tile_rows < g.M ? m0 + tile_rows : g.M;
   const int64_t a_ldb = g.a_ld * ELEM, b_ldb = g.b_ld * ELEM;
-  const int kt_count =
-      !HALO && g.kt_split > 0 ? g.kt_split : (int)(g.K * ELEM / kTileKBytes);
+  static_assert(!CUT || A_MODE == A_KCONTIG || A_MODE == A_MCONTIG, "matrix products");
+  const int kt_total = (int)((g.K * ELEM + (CUT ? kTileKBytes - 1 : 0)) / kTileKBytes);
   const int kt_base = !HALO && g.kt_split > 0 ? (int)outer * g.kt_split : 0;
+  // (the last part of a split may be shorter)
+  const int kt_count =
+      !HALO && g.kt_split > 0 && kt_base + g.kt_split < kt_total ? g.kt_split : kt_total - kt_base;
+  // bytes of K in its last slice, and the slice (of this part) whose loads leave the rest
+  // out, -1: none here
+  const int kt_rest = (int)(g.K * ELEM - (int64_t)(kt_total - 1) * kTileKBytes);
+  const int kt_cut = CUT && kt_base + kt_count == kt_total ? kt_count - 1 : -1;
 
   const int wave = threadIdx.x >> 6;
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
@@ -845,6 +872,10 @@ gemm_kernel(GemmArgs g) {
         off[j] = (cv_mask[HALVES ? j / 2 : j] & need_j) == need_j ? off_a[j] + at : 0x80000000u;
       }
       dma_issue<LSTEP, GA::kLoads, A0, A1>(a_base, g.conv.x_bytes & lim, off, dst);
+    } else if (CUT && kt == kt_cut) {
+      uint32_t off[GA::kLoads];
+      dma_cut<BM, ELEM, A_KC, LW, LSTEP, A0, A1>(group_a, kt_rest, off_a, off);
+      dma_issue<LSTEP, GA::kLoads, A0, A1>(a_base + kt * a_step, 0x80000000u, off, dst);
     } else {
       dma_issue<LSTEP, GA::kLoads, A0, A1>(a_base + kt * a_step, lim, off_a, dst);
     }
@@ -857,7 +888,13 @@ gemm_kernel(GemmArgs g) {
     constexpr int B0 = PART * GB::kLoads / PARTS, B1 = (PART + 1) * GB::kLoads / PARTS;
     const uint32_t dst =
         (HALVES ? stage_half(team, st) + GA::kBytes / 2 : stage_b(st)) + (uint32_t)w_load * 1024u;
-    dma_issue<LSTEP, GB::kLoads, B0, B1>(b_base + kt * b_step, 0xffffffffu, off_b, dst);
+    if (CUT && kt == kt_cut) {
+      uint32_t off[GB::kLoads];
+      dma_cut<BN, ELEM, B_KC, LW, LSTEP, B0, B1>(group_b, kt_rest, off_b, off);
+      dma_issue<LSTEP, GB::kLoads, B0, B1>(b_base + kt * b_step, 0x80000000u, off, dst);
+    } else {
+      dma_issue<LSTEP, GB::kLoads, B0, B1>(b_base + kt * b_step, 0xffffffffu, off_b, dst);
+    }
   };
   auto issue = [&](int kt, int st, auto part_c, auto parts_c) {
     issue_a(kt, st, part_c, parts_c);
@@ -1599,6 +1636,7 @@ struct GemmPlan {
   // parts the reduction is cut into (f32 partial results in the context's
   // scratch, added by a second kernel); 1: none
   int ksplit = 1;
+  double us = 0; // estimated
 };
 
 // Stage count per tile: as many as fit the 160 KB LDS, at most 4.
@@ -1615,12 +1653,12 @@ template <int BM, int BN> struct GemmWaves {
   static constexpr int value = BM == 256 && BN == 128 ? 8 : GemmLayout<BM, BN>::kWaves;
 };
 
-template <int KIND, int BM, int BN, int A_MODE, bool B_KC, int STAGES = 0, int WAVES = 0>
+template <int KIND, int BM, int BN, int A_MODE, bool B_KC, int STAGES = 0, int WAVES = 0, bool CUT = false>
 int launch(fhip_ctx *ctx, const GemmArgs &g, int64_t batch) {
   constexpr int NSTAGE = STAGES ? STAGES : GemmStages<BM, BN>::value;
   constexpr int NW = WAVES ? WAVES : GemmWaves<BM, BN>::value;
   constexpr int lds = GemmLds<BM, BN, NSTAGE, NW>::kBytes;
-  auto kernel = gemm_kernel<KIND, BM, BN, A_MODE, B_KC, NSTAGE, NW>;
+  auto kernel = gemm_kernel<KIND, BM, BN, A_MODE, B_KC, NSTAGE, NW, CUT>;
   static FhipOncePerDevice configured;
   if (!configured.done(ctx->device)) {
     FHIP_HIP_CHECK(ctx, hipFuncSetAttribute(
@@ -1635,26 +1673,32 @@ int launch(fhip_ctx *ctx, const GemmArgs &g, int64_t batch) {
   return 0;
 }
 
-template <int KIND, int BM, int BN, int STAGES = 0, int WAVES = 0>
+template <int KIND, int BM, int BN, bool CUT, int STAGES = 0, int WAVES = 0>
 int launch_orient(fhip_ctx *ctx, const GemmPlan &p, const GemmArgs &g) {
   if (p.a_kc && p.b_kc)
-    return launch<KIND, BM, BN, A_KCONTIG, true, STAGES, WAVES>(ctx, g, p.batch);
+    return launch<KIND, BM, BN, A_KCONTIG, true, STAGES, WAVES, CUT>(ctx, g, p.batch);
   if (p.a_kc && !p.b_kc)
-    return launch<KIND, BM, BN, A_KCONTIG, false, STAGES, WAVES>(ctx, g, p.batch);
+    return launch<KIND, BM, BN, A_KCONTIG, false, STAGES, WAVES, CUT>(ctx, g, p.batch);
   if (!p.a_kc && p.b_kc)
-    return launch<KIND, BM, BN, A_MCONTIG, true, STAGES, WAVES>(ctx, g, p.batch);
-  return launch<KIND, BM, BN, A_MCONTIG, false, STAGES, WAVES>(ctx, g, p.batch);
+    return launch<KIND, BM, BN, A_MCONTIG, true, STAGES, WAVES, CUT>(ctx, g, p.batch);
+  return launch<KIND, BM, BN, A_MCONTIG, false, STAGES, WAVES, CUT>(ctx, g, p.batch);
+}
+
+template <int KIND, bool CUT>
+int gemm_launch_cut(fhip_ctx *ctx, const GemmPlan &p, const GemmArgs &g) {
+  if (p.bm == 256 && p.bn == 256)
+    return launch_orient<KIND, 256, 256, CUT>(ctx, p, g);
+  if (p.bm == 256 && p.bn == 128)
+    return launch_orient<KIND, 256, 128, CUT>(ctx, p, g);
+  // (eight wavefronts of 64 x 32 in two phases, two stages: two workgroups per
+  // compute unit at 116-118 registers a lane)
+  return launch_orient<KIND, 128, 128, CUT, 2, 8>(ctx, p, g);
 }
 
 template <int KIND>
 int gemm_launch_kind(fhip_ctx *ctx, const GemmPlan &p, const GemmArgs &g) {
-  if (p.bm == 256 && p.bn == 256)
-    return launch_orient<KIND, 256, 256>(ctx, p, g);
-  if (p.bm == 256 && p.bn == 128)
-    return launch_orient<KIND, 256, 128>(ctx, p, g);
-  // (eight wavefronts of 64 x 32 in two phases, two stages: two workgroups per
-  // compute unit at 116-118 registers a lane)
-  return launch_orient<KIND, 128, 128, 2, 8>(ctx, p, g);
+  return g.K * KindTraits<KIND>::kElemBytes % kTileKBytes != 0 ? gemm_launch_cut<KIND, true>(ctx, p, g)
+                                                               : gemm_launch_cut<KIND, false>(ctx, p, g);
 }
 
 // Implicit-GEMM convolution launchers (A gathered, B = filter, K-contiguous).

@@ -8,6 +8,10 @@
 //     K-contiguous tiles are read from LDS with 16-byte loads, the other kind
 //     with the gfx950 transposing LDS reads (ds_read_b64_tr_b16 / _tr_b8), so
 //     no operand is ever transposed in registers or in HBM;
+//   * K may end inside a 128-byte slice (in whole 16-byte chunks where an operand lies along
+//     it): a variant of the kernel masks the last slice's loads (bf16 4000 x 4000 x 4008
+//     419 us on the direct kernels -> 104, fp8 3702 x 3584 x 6640 292 -> 77); the parts of a
+//     split reduction may differ in length (323 x 688 x 5952 in 12 parts instead of 3, 28.8 -> 21.7);
 //   * 256 threads = 2 x 2 wavefronts per workgroup, each wavefront owning a
 //     (BM/2) x (BN/2) block of 32x32 MFMA tiles; K advances in 128-byte slices
 //     through double-buffered, bank-conflict-padded LDS with the next slice's
@@ -50,7 +54,8 @@ bool kind_for(int a_dt, int b_dt, int *kind) {
   }
 }
 
-GemmPlan make_plan(const fhip_matmul_desc *d) {
+// `ragged`: K may end inside a 128-byte slice.
+GemmPlan make_plan(const fhip_matmul_desc *d, bool ragged) {
   GemmPlan p;
   const int r = d->a.rank;
   if (r != 2 && r != 3)
@@ -83,9 +88,9 @@ GemmPlan make_plan(const fhip_matmul_desc *d) {
   } else {
     return p;
   }
-  // whole 128-byte K slices; 16-byte aligned rows; tiles no larger than the
-  // matrix so edge clamping stays in bounds
-  if ((p.K * elem) % kTileKBytes != 0)
+  // 16-byte aligned rows, whole 16-byte chunks of K along them (the last slice may
+  // be part of one); tiles no larger than the matrix so edge clamping stays in bounds
+  if (ragged ? (p.a_kc || p.b_kc) && (p.K * elem) % 16 != 0 : (p.K * elem) % kTileKBytes != 0)
     return p;
   if ((p.a_ld * elem) % 16 != 0 || (p.b_ld * elem) % 16 != 0)
     return p;
@@ -143,7 +148,7 @@ GemmPlan make_plan(const fhip_matmul_desc *d) {
   // (fitted: 0.65 + 0.35 x the busy share).  Microseconds on this chip, from
   // 2048^3 ... 8192 x 8192 x 1024 problems of each type.
   const bool k16 = p.kind == GK_BF16 || p.kind == GK_F16;
-  const int64_t slices = p.K * elem / kTileKBytes;
+  const int64_t slices = (p.K * elem + kTileKBytes - 1) / kTileKBytes;
   auto tiles = [&](int bm, int bn) {
     return (double)(((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn) * p.batch);
   };
@@ -159,12 +164,13 @@ GemmPlan make_plan(const fhip_matmul_desc *d) {
     const double full = floor(t / 256.0), rest = t - 256.0 * full;
     const double rounds = full + (rest > 0 ? 1 : 0);
     const double work = full + (rest > 0 ? 0.65 + 0.35 * rest / 256.0 : 0.0);
-    double us = (double)(slices / sk) * pace * work +
+    const double run = (double)((slices + sk - 1) / sk); // slices of a part
+    double us = run * pace * work +
                 (shape != 2 ? fixed * rounds
                  : p.kind == GK_I8 ? fixed * (1.0 + 0.5 * (rounds - 1)) // (int32 stores)
                                    // (a partner with under 4.25 us of K slices does not cover it:
                                    // fp8 4096 x 4096 x 512 18.9 us against 16.1 on 256 x 256)
-                                   : fixed + (rounds - 1) * fmax(0.0, 4.25 - (double)(slices / sk) * pace));
+                                   : fixed + (rounds - 1) * fmax(0.0, 4.25 - run * pace));
     if (sk > 1) // the parts' f32 stores and the kernel that adds them (~5 TB/s each way)
       us += 2.0 * sk * (double)p.M * (double)p.N * 4.0 / 5.0e6 + 2.5;
     return us;
@@ -172,6 +178,11 @@ GemmPlan make_plan(const fhip_matmul_desc *d) {
   const int forced = fhip_knobs().gemm_split; // (1: never split)
   const bool may_split = p.batch == 1 && p.N % 4 == 0 && p.o_sn == 1 &&
                          forced != 1;
+  // parts of ceil(slices / sk) slices, at least 8, the last one maybe shorter but not empty
+  auto splits = [&](int sk) {
+    const int64_t run = (slices + sk - 1) / sk;
+    return run >= 8 && (sk - 1) * run < slices;
+  };
   double best = 0;
   p.bm = p.bn = 0;
   static const int shapes[3][2] = {{128, 128}, {256, 128}, {256, 256}};
@@ -180,10 +191,12 @@ GemmPlan make_plan(const fhip_matmul_desc *d) {
     if (i > 0 && (p.M < bm || p.N < bn))
       continue;
     for (int sk = 1; sk <= 128; ++sk) {
-      if (sk > 1 && (!may_split || slices % sk != 0 || slices / sk < 8))
+      if (sk > 1 && (!may_split || (slices + sk - 1) / sk < 8))
+        break;
+      if (sk > 1 && !splits(sk))
         continue;
-      // (a forced count must still divide the slices into runs of at least 8)
-      if (forced > 1 && may_split && slices % forced == 0 && slices / forced >= 8 && sk != forced)
+      // (a forced count must still cut the slices into runs of at least 8)
+      if (forced > 1 && may_split && splits(forced) && sk != forced)
         continue;
       // a split must pay clearly; ties go to the larger tile (compute units
       // run faster while others idle)
@@ -202,9 +215,9 @@ GemmPlan make_plan(const fhip_matmul_desc *d) {
       p.bm = bm, p.bn = bn, p.ksplit = 1;
       best = estimate(bm, bn, 1);
       for (int sk = 2; sk <= 128 && may_split; ++sk) {
-        if (slices % sk != 0 || slices / sk < 8)
+        if (!splits(sk))
           continue;
-        if (forced > 1 && slices % forced == 0 && slices / forced >= 8 && sk != forced)
+        if (forced > 1 && splits(forced) && sk != forced)
           continue;
         const double us = estimate(bm, bn, sk) * 1.1;
         if (us < best || sk == forced)
@@ -212,6 +225,7 @@ GemmPlan make_plan(const fhip_matmul_desc *d) {
       }
     }
   }
+  p.us = best;
   p.ok = true;
   return p;
 }
@@ -270,14 +284,48 @@ __global__ void gemm_splitk_sum_kernel(GemmSumArgs a) {
 
 } // namespace
 
+static int run_plan(fhip_ctx *ctx, GemmPlan p, const fhip_matmul_desc *d, const void *a,
+                    const void *b, const DevEpilogue &epi, void *out);
+
 bool fhip_fast_matmul_applicable(const fhip_matmul_desc *d) {
-  return make_plan(d).ok;
+  return make_plan(d, false).ok;
 }
 
 int fhip_fast_matmul(fhip_ctx *ctx, const fhip_matmul_desc *d, const void *a,
                      const void *b, const DevEpilogue &epi, void *out) {
-  GemmPlan p = make_plan(d);
+  const GemmPlan p = make_plan(d, false);
   FHIP_REQUIRE(ctx, p.ok, "gemm: descriptor not supported by the MFMA kernel");
+  return run_plan(ctx, p, d, a, b, epi, out);
+}
+
+int fhip_tuned_matmul(fhip_ctx *ctx, const fhip_matmul_desc *d, const void *a,
+                      const void *b, const DevEpilogue &epi, void *out, bool *handled, bool *short_k) {
+  *handled = true;
+  *short_k = false;
+  const GemmPlan p = make_plan(d, true);
+  const bool whole = p.ok && p.K * fhip_dtype_size(d->a.dtype) % kTileKBytes == 0;
+  const bool aligned = (((uintptr_t)a | (uintptr_t)b) & 15) == 0;
+  if (whole && (!aligned || fhip_knobs().gemm_tile_bm || fhip_knobs().gemm_split))
+    return run_plan(ctx, p, d, a, b, epi, out); // (misaligned operands of the contract are refused)
+  double us = 0;
+  if (p.ok && aligned) {
+    // (the planner's estimate against 154 products of 128 to 4096 rows and 256 to 8192 columns:
+    // 14 % rms for 16 bits, 5 for fp8, 11 for int8; GELU over whole 128-wide tiles 6 us)
+    const bool gelu = fhip_epilogue_is_transcendental(d->epilogue);
+    us = p.kind == GK_I8 ? 0.95 * p.us - 1.0
+         : p.kind == GK_BF16 || p.kind == GK_F16 ? 1.1 * p.us - 1.0 + (gelu ? 6.0 : 0.0)
+                                                 : 1.05 * p.us + 1.6 + (gelu ? 6.0 : 0.0);
+    us = us > 1.0 ? us : 1.0;
+  }
+  const int rc = fhip_direct_matmul(ctx, d, a, b, epi, out, us, whole, handled, short_k);
+  if (*handled || us == 0 || *short_k)
+    return rc;
+  *handled = true;
+  return run_plan(ctx, p, d, a, b, epi, out);
+}
+
+static int run_plan(fhip_ctx *ctx, GemmPlan p, const fhip_matmul_desc *d, const void *a,
+                    const void *b, const DevEpilogue &epi, void *out) {
   const int64_t pitch = (p.N + p.bn - 1) / p.bn * p.bn; // of the parts of a split reduction
   const size_t part_bytes = (size_t)p.ksplit * (size_t)(p.M * pitch) * sizeof(float);
   if (p.ksplit > 1 && !fhip_ctx_scratch_ready(ctx, part_bytes))
@@ -356,7 +404,10 @@ int fhip_fast_matmul(fhip_ctx *ctx, const fhip_matmul_desc *d, const void *a,
     g.epi.rank = 3;
     g.outer = p.ksplit;
     g.o_outer = p.M * pitch;
-    g.kt_split = (int32_t)(p.K * fhip_dtype_size(d->a.dtype) / kTileKBytes / p.ksplit);
+    {
+      const int64_t slices = (p.K * fhip_dtype_size(d->a.dtype) + kTileKBytes - 1) / kTileKBytes;
+      g.kt_split = (int32_t)((slices + p.ksplit - 1) / p.ksplit);
+    }
     gemm_fill_linear(fhip_epilogue{}, g);
     const int rc = launch();
     if (rc != 0)

@@ -1,0 +1,6 @@
+// Matrix products on register-staged LDS tiles, f16 operands.
+#include "gemm_tile_kernel.h"
+
+int tile_launch_f16(fhip_ctx *ctx, const DirectPlan &p, const DirectArgs &g, int64_t batch) {
+  return tile_launch_kind<GK_F16>(ctx, p, g, batch);
+}

@@ -1155,12 +1155,10 @@ int fhip_matmul(fhip_ctx *ctx, const fhip_matmul_desc *d, const void *a,
   if (fhip_build_epilogue(ctx, d->epilogue, r, d->c.dim, epilogue_operands,
                           &epi) != 0)
     return 1;
-  if (fhip_fast_matmul_applicable(d))
-    return fhip_fast_matmul(ctx, d, a, b, epi, out);
   bool handled = false, short_k = false;
-  const int direct_rc = fhip_direct_matmul(ctx, d, a, b, epi, out, &handled, &short_k);
+  const int tuned_rc = fhip_tuned_matmul(ctx, d, a, b, epi, out, &handled, &short_k);
   if (handled)
-    return direct_rc;
+    return tuned_rc;
   fhip_note_kernel(ctx, "matmul_generic");
 
   MatmulArgs g{};

@@ -1,0 +1,94 @@
+"""Products whose K ends inside a 128-byte slice, whose rows start on any element or whose tiles
+are few: the register-staged LDS tiles (gemm_tile_kernel.h) and the tiled GEMM's cut slices,
+against the oracle."""
+import numpy as np
+import pytest
+
+from fusilli_amd import capi
+from helpers import HT, assert_close, rand
+from oracle import oracle
+from test_gemm_mfma_gpu import make_operand, ref_matmul
+
+pytestmark = pytest.mark.gpu
+BYTES = [capi.INT8, capi.FP8E4M3, capi.FP8E5M2]
+DTYPES = [capi.BFLOAT16, capi.HALF] + BYTES
+
+
+def run(ctx, a, b, epilogue=(), epi_tensors=()):
+    i8 = a.dtype == capi.INT8
+    cdt, odt = (capi.INT32, capi.INT32) if i8 else (capi.FLOAT, capi.HALF if a.dtype == capi.HALF else capi.BFLOAT16)
+    dims = a.dims[:-2] + [a.dims[-2], b.dims[-1]]
+    out = HT.empty(dims, odt)
+    d = capi.MatmulDesc()
+    d.a, d.b, d.out, d.out_dtype = a.desc(), b.desc(), out.desc(), odt
+    d.c = capi.TensorDesc.make(dims, out.strides, cdt)
+    d.epilogue = capi.make_epilogue(list(epilogue))
+    bufs = [t.upload(ctx) for t in epi_tensors]
+    da, db, do = a.upload(ctx), b.upload(ctx), out.upload(ctx)
+    ctx.matmul(d, da, db, do, epilogue_operands=bufs)
+    return out.fetch(ctx, do).logical(), ctx.last_kernel(), odt
+
+
+def check(got, ref, odt, what):
+    if odt == capi.INT32:
+        assert np.array_equal(got, ref), what
+    else:
+        # one rounding to the result's type over f32 sums: half a unit in the last place, and as
+        # much again where the sum's own error crosses a rounding boundary
+        ulp = 2.0 ** -8 if odt == capi.BFLOAT16 else 2.0 ** -11
+        rms = np.sqrt(np.mean(np.square(ref)))
+        assert np.all(np.abs(got - ref) <= 1.01 * ulp * np.abs(ref) + 1e-4 * rms), what
+
+
+# tile rows and columns, remainders on either side, one slice and a cut one, K odd
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("m,n,k", [(640, 1089, 2051), (705, 705, 3001), (1153, 641, 1999), (1025, 1027, 1033)])
+def test_tiles_of_64(ctx, dtype, ta, tb, m, n, k):
+    a, b = make_operand(81, 0, m, k, dtype, ta), make_operand(81, 1, k, n, dtype, tb)
+    got, name, odt = run(ctx, a, b)
+    check(got, ref_matmul(a, b), odt, name)
+    assert name.startswith("gemm_mfma") and "x64 " in name, name
+
+
+@pytest.mark.parametrize("dtype", [capi.BFLOAT16, capi.FP8E4M3, capi.INT8])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("m,n,k", [(1299, 1930, 777), (2049, 1282, 1001)])
+def test_wide_tiles(ctx, dtype, ta, tb, m, n, k):
+    a, b = make_operand(82, 0, m, k, dtype, ta), make_operand(82, 1, k, n, dtype, tb)
+    got, name, odt = run(ctx, a, b)
+    check(got, ref_matmul(a, b), odt, name)
+    assert name.startswith("gemm_mfma") and "128x128 waves=4" in name, name
+
+
+# whole 16-byte chunks of K, and any K where neither operand lies along it: the tiled GEMM
+@pytest.mark.parametrize("dtype,k16", [(capi.BFLOAT16, 8), (capi.HALF, 8), (capi.INT8, 16), (capi.FP8E5M2, 16)])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("m,n,slices,rest", [(3072, 2064, 8, 1), (2064, 2064, 7, 7), (2576, 2592, 3, 3), (256, 4096, 33, 5)])
+def test_cut_slices(ctx, dtype, k16, ta, tb, m, n, slices, rest):
+    k = slices * 8 * k16 + rest * k16 + (3 if ta and not tb else 0)
+    a, b = make_operand(83, 0, m, k, dtype, ta), make_operand(83, 1, k, n, dtype, tb)
+    got, name, odt = run(ctx, a, b)
+    assert name.startswith("gemm_mfma"), name
+    check(got, ref_matmul(a, b), odt, name)
+
+
+@pytest.mark.parametrize("dtype", [capi.BFLOAT16, capi.HALF])
+@pytest.mark.parametrize("m,n,k,batch", [(130, 250, 1003, 1), (140, 140, 6001, 1), (90, 200, 700, 5), (700, 1300, 1500, 1)])
+def test_fused_chains(ctx, dtype, m, n, k, batch):
+    # a column operand alone (requested early), and with a full one; also behind a split K
+    lead = [batch] if batch > 1 else []
+    a = make_operand(84, 0, m, k, dtype, False, batch=batch if batch > 1 else None)
+    b = make_operand(84, 1, k, n, dtype, True, batch=batch if batch > 1 else None)
+    bias = HT.from_logical(rand(84, 2, [1] * (len(lead) + 1) + [n]), dtype)
+    full = HT.from_logical(rand(84, 3, lead + [m, n]), capi.FLOAT)
+    product = ref_matmul(a, b)
+    add = capi.epilogue_op(capi.PW["ADD"], capi.FLOAT, operand=bias.desc(), operand_index=0)
+    mul = capi.epilogue_op(capi.PW["MUL"], dtype, operand=full.desc(), operand_index=1)
+    scale = capi.epilogue_op(capi.PW["MUL"], capi.FLOAT, scalar=0.25)
+    gelu = capi.epilogue_op(capi.PW["GELU_FWD"], dtype)
+    for ops, tensors, ref in (
+            ([add, gelu], [bias], oracle.pointwise(capi.PW["GELU_FWD"], [product + bias.logical()])),
+            ([scale, add, mul], [bias, full], (0.25 * product + bias.logical()) * full.logical())):
+        got, name, odt = run(ctx, a, b, ops, tensors)
+        assert_close(got, ref, dtype, name)
