@@ -14,7 +14,8 @@
 // Stages of 64 values sit in LDS twice; loads run two steps ahead in registers.  The
 // result goes through LDS so that a lane finishes and stores 8 channels of a pixel.
 //
-// N16 48 -> 48, 48 x 32, 3 x 3, f16: copy + product 16.9 us -> 9.
+// N16 48 -> 48, 48 x 32, 3 x 3, f16: copy + product 16.9 us -> 9.  Long reductions and few
+// tiles: conv_tile_kernel.h.
 // (128 x 128, 256 x 64, 128 x 64 and 128 x 32 tiles of the same kernel are slower.)
 //
 // Reference semantics: aten.convolution (reference support/asm_emitter.h:690-701).

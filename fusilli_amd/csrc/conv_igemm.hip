@@ -12,6 +12,7 @@
 // support/asm_emitter.h:690-701, node/conv_node.h:38-56).
 #include "common.h"
 #include "conv_gather.h"
+#include "conv_tile.h"
 #include "fast_paths.h"
 #include "gemm_kernel.h"
 
@@ -334,20 +335,26 @@ struct ConvResolved {
   bool padded = false; // X and W are first copied into the context's scratch
   int64_t C = 0, Cp = 0, x_pixels = 0, w_pixels = 0;
   size_t x_bytes = 0, w_bytes = 0;
-  // runs on the gathered tiles of conv_gather.hip instead (unpadded operands)
+  // runs on gathered tiles instead (unpadded operands): those of conv_gather.hip, or, with a
+  // plan in `tile`, of conv_tile.hip
   ConvGatherPlan gather{0};
+  ConvTilePlan tile;
+  ConvTileArgs args{}; // of either, while one of them runs or was weighed
 
+  bool unpadded() const { return gather.parts != 0 || tile.bm != 0; }
   // parts of a split reduction and their rows' pitch (padded to whole column tiles, which
   // are stored whole: every cache line of the parts is written by one workgroup)
   int parts() const { return gather.parts ? gather.parts : plan.ksplit; }
   int64_t part_pitch() const {
     return gather.parts ? plan.N : (plan.N + plan.bn - 1) / plan.bn * plan.bn;
   }
-  size_t pad_bytes() const { return padded && !gather.parts ? x_bytes + w_bytes : 0; }
+  size_t pad_bytes() const { return padded && !unpadded() ? x_bytes + w_bytes : 0; }
 };
 
 // The context's scratch: zero-padded copies of X and W, then the parts of a split reduction.
 size_t scratch_bytes(const ConvResolved &r) {
+  if (r.tile.bm)
+    return conv_tile_scratch(r.tile, r.args);
   const size_t sums = r.parts() > 1 ? (size_t)r.parts() * (size_t)(r.plan.M * r.part_pitch()) * sizeof(float) : 0;
   return r.pad_bytes() + sums;
 }
@@ -394,8 +401,46 @@ bool copies_pay(const ConvResolved &r, int64_t J, bool fused) {
   return fused ? p.N % 128 == 0 && tiles >= 500 : tiles >= 360 && fill >= 0.8 && full >= 0.7;
 }
 
+// Scratch that the parts of a reduction over gathered tiles may take.
+constexpr size_t kTileRoom = 64u << 20;
+
+// The arguments of the gathered tiles for the problem of `p` over `C` channels.
+void tile_args(const ConvPlan &p, int64_t C, ConvTileArgs &a) {
+  const ConvGeom &g = p.geom;
+  a.parts = 1;
+  ConvTilePart &t = a.part[0];
+  t.M = (int32_t)p.M, t.P = g.P, t.Q = g.Q;
+  t.J = (int32_t)(g.R * g.S * C), t.S = g.S;
+  t.off_h = -g.pad_h, t.off_w = -g.pad_w;
+  a.d.M = t.M, a.d.N = (int32_t)p.N, a.d.K = t.J;
+  a.H = g.H, a.W = g.W, a.C = (int32_t)C;
+  a.str_h = g.str_h, a.str_w = g.str_w, a.dil_h = g.dil_h, a.dil_w = g.dil_w;
+  a.x_bytes = (uint32_t)(p.M / ((int64_t)g.P * g.Q) * g.H * g.W * C * 2);
+  a.d.o_sm = p.N, a.d.o_sn = 1;
+}
+
+// What the kernel that `r` names takes, 0: not known.  Fitted as the tiles' times are (6 to 7 %
+// rms, the halo tiles 11) to 1319 layers on conv_gather.hip, 365 on the GEMM's gather and 143
+// gradients on halo tiles; a gradient's times hold the mirrored filter.
+double igemm_us(const ConvResolved &r, bool dgrad, bool fused) {
+  static const ConvTileTimes kGather = {64, 64, 1, 3, 3.146, 0.385, 0.251, 0.437, 2.203, 0.378, 2.271, 0.541};
+  static const ConvTileTimes kWide[] = {{128, 128, 1, 2, 3.075, 0.689, 0.520, 2.265, 3.791, 0.303, 1.350, 0},
+                                        {128, 128, 1, 2, 5.536, 0.709, 0.534, 2.323, 7.404, 0.270, 0, 0}};
+  static const ConvTileTimes kHalo[] = {{128, 128, 1, 2, 6.773, 0.790, 0.779, 0, 0, 0, 0, 0},
+                                        {128, 64, 1, 2, 7.289, 0.622, 0.470, 0, 0, 0, 0, 0}};
+  const ConvPlan &p = r.plan;
+  if (r.gather.parts)
+    return conv_tile_us(kGather, r.args, r.gather.parts, fused) + (dgrad ? 2.6 : 0.0);
+  if (r.padded || p.groups != 1 || p.bm != 128)
+    return 0;
+  if (p.halo)
+    return dgrad ? conv_tile_us(kHalo[p.bn == 64], r.args, 1, false) : 0;
+  return p.bn == 128 ? conv_tile_us(kWide[dgrad], r.args, p.ksplit > 1 ? p.ksplit : 1, fused) : 0;
+}
+
 // The gathered tiles for a problem that make_plan accepted (`C` its true channels).
-void choose_gather(ConvResolved &r, int64_t C, bool fused) {
+// `split`: whether the reduction may be cut where C is a multiple of 64.
+void choose_gather(ConvResolved &r, int64_t C, bool fused, bool split) {
   const ConvPlan &p = r.plan;
   const FhipKnobs &knobs = fhip_knobs();
   if (knobs.conv_gather == 0 || p.groups != 1 || C % 8 != 0 || knobs.conv_tile_bm || knobs.conv_halo >= 0 ||
@@ -415,19 +460,41 @@ void choose_gather(ConvResolved &r, int64_t C, bool fused) {
   const bool narrow = !p.halo && p.ksplit == 1 && p.N < 64;
   const bool copies = r.padded && copies_pay(r, J, fused);
   const bool want = (r.padded && !copies) || knobs.conv_gather > 0 || few || narrow;
+  // 128 x 128 tiles of the tiled GEMM's gather, which the smaller ones outrun where they are few,
+  // narrow or short (N9 128 -> 128, 12 x 12, 5 x 5 23.4 -> 11.9 us, N11 448 -> 64, 63 x 10 at
+  // stride 2 17.4 -> 13.2; on 49 random layers that ran there 21 % in the mean, none slower;
+  // 1 x 1 at stride 2 over 5600 pixels, 128 -> 224 7.0 -> 4.6)
+  const bool single = p.geom.R * p.geom.S == 1 && p.geom.str_h == 1 && p.geom.str_w == 1;
+  // (not where they fill the chip, whole or in eight parts: N32 512 -> 512, 7 x 7 26.0, here 26.1)
+  const bool wide =
+      !p.halo && !r.padded && p.bm == 128 && p.bn == 128 && p.ksplit < 8 && tiles < 512 && !single;
+  if (!want && !wide)
+    return;
+  tile_args(p, C, r.args);
+  const ConvTilePlan t = conv_tile_plan(r.args, false, fused, r.padded || split ? kTileRoom : 0);
+  const double known = want ? 0 : igemm_us(r, false, fused);
   // (whole slices: no parts -- the entry point without scratch gives the same bits)
-  if (want)
-    r.gather = conv_gather_plan(p.M, p.N, J, r.padded && p.N % 4 == 0);
+  r.gather = conv_gather_plan(p.M, p.N, J, r.padded && p.N % 4 == 0);
+  // Its loop is the shortest to start (N16 48 -> 48, 48 x 32: 7.4 us, on the tiles 8.5) and
+  // the slowest in a long reduction (N31 192 -> 192, 11 x 11, 5 x 5: 36.0, on the tiles 24.5;
+  // over 179 random layers that ran there the choice takes 0.93 of its time).
+  const double here = igemm_us(r, false, fused);
+  if (t.bm && t.us < 0.95 * here)
+    r.gather.parts = 0, r.tile = t;
+  if (!want && (t.us < here ? t.us : here) > 0.95 * known)
+    r.gather.parts = 0, r.tile = ConvTilePlan{};
 }
 
-ConvResolved resolve(const fhip_conv_desc *d, bool allow_scratch = true) {
+// `split`: see choose_gather; the data gradient's entry point without scratch gives the bits of
+// the one with it.  `choose` false: only whether a plan exists.
+ConvResolved resolve(const fhip_conv_desc *d, bool allow_scratch = true, bool split = true, bool choose = true) {
   ConvResolved r;
   fhip_conv_desc folded;
   const fhip_conv_desc *g = fold_3d(d, &folded) ? &folded : d;
   r.run = *g;
   r.plan = make_plan(g, d, allow_scratch);
-  if (r.plan.ok)
-    choose_gather(r, g->x.dim[1], d->epilogue.count > 0);
+  if (r.plan.ok && choose)
+    choose_gather(r, g->x.dim[1], d->epilogue.count > 0, allow_scratch && split);
   if (r.plan.ok || !allow_scratch)
     return r;
   // channel padding: 16-bit channels-last tensors, whole 16-byte chunks
@@ -466,7 +533,8 @@ ConvResolved resolve(const fhip_conv_desc *d, bool allow_scratch = true) {
   r.w_pixels = fhip_desc_volume(g->w) / C;
   r.x_bytes = ((size_t)(r.x_pixels * Cp * 2) + 255) / 256 * 256;
   r.w_bytes = ((size_t)(r.w_pixels * Cp * 2) + 255) / 256 * 256;
-  choose_gather(r, C, d->epilogue.count > 0);
+  if (choose)
+    choose_gather(r, C, d->epilogue.count > 0, true);
   return r;
 }
 
@@ -551,21 +619,23 @@ int conv_launch_f16(fhip_ctx *ctx, int bm, int bn, const GemmArgs &g) {
 // Where scratch cannot be had: reductions in one part, and gathered tiles, which read X and
 // W in place, instead of padded copies.
 static void do_without_scratch(const fhip_conv_desc *d, ConvResolved &r) {
-  if (!r.padded && r.gather.parts == 0)
+  if (!r.padded && !r.unpadded())
     r = resolve(d, false);
-  else if (r.gather.parts == 0)
+  else if (!r.unpadded())
     r.gather = conv_gather_plan(r.plan.M, r.plan.N, (int64_t)r.plan.geom.R * r.plan.geom.S * r.C, false);
   if (r.gather.parts)
     r.gather.parts = 1;
+  if (r.tile.bm)
+    r.tile = conv_tile_plan(r.args, false, d->epilogue.count > 0, 0);
 }
 
 bool fhip_fast_conv_applicable(const fhip_conv_desc *d, bool allow_scratch) {
-  return fhip_fast_conv_rf_applicable(d) || resolve(d, allow_scratch).plan.ok;
+  return fhip_fast_conv_rf_applicable(d) || resolve(d, allow_scratch, true, false).plan.ok;
 }
 
 int fhip_fast_conv(fhip_ctx *ctx, const fhip_conv_desc *d, const void *x,
                    const void *w, const DevEpilogue &epi, void *out,
-                   bool *handled, bool allow_scratch) {
+                   bool *handled, bool allow_scratch, bool split) {
   if (handled)
     *handled = true;
   bool taken = false;
@@ -573,7 +643,7 @@ int fhip_fast_conv(fhip_ctx *ctx, const fhip_conv_desc *d, const void *x,
     return 1;
   if (taken)
     return 0;
-  ConvResolved res = resolve(d, allow_scratch);
+  ConvResolved res = resolve(d, allow_scratch, split);
   if (res.plan.ok && !fhip_ctx_scratch_ready(ctx, scratch_bytes(res)))
     do_without_scratch(d, res);
   const ConvPlan &p = res.plan;
@@ -585,7 +655,6 @@ int fhip_fast_conv(fhip_ctx *ctx, const fhip_conv_desc *d, const void *x,
   FHIP_REQUIRE(ctx, p.ok, "conv: descriptor not supported by the MFMA kernel");
   FHIP_REQUIRE(ctx, ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0,
                "conv: X and W must be 16-byte aligned");
-  const bool gather = res.gather.parts != 0;
   const int64_t part_pitch = res.part_pitch();
   const int parts = res.parts();
   char *scratch = nullptr;
@@ -595,7 +664,7 @@ int fhip_fast_conv(fhip_ctx *ctx, const fhip_conv_desc *d, const void *x,
       return 1;
     scratch = (char *)sp;
   }
-  if (res.padded && !gather) {
+  if (res.padded && !res.unpadded()) {
     // channel counts that are no multiple of 64: zero-padded copies of X and W
     char *xp = scratch, *wp = xp + res.x_bytes;
     const int32_t c8 = (int32_t)(res.C / 8), cp8 = (int32_t)(res.Cp / 8);
@@ -668,7 +737,7 @@ int fhip_fast_conv(fhip_ctx *ctx, const fhip_conv_desc *d, const void *x,
     FHIP_HIP_CHECK(ctx, hipGetLastError());
     return 0;
   };
-  if (gather) {
+  if (res.gather.parts) {
     const ConvGeom &cg = p.geom;
     ConvGatherArgs a{};
     a.x = (const char *)x, a.w = (const char *)w, a.out = out;
@@ -688,6 +757,15 @@ int fhip_fast_conv(fhip_ctx *ctx, const fhip_conv_desc *d, const void *x,
     fhip_note_kernel(ctx, "conv_igemm unpadded %dx%d split=%d", kConvGatherTile, kConvGatherTile,
                      parts);
     return 0;
+  }
+  if (res.tile.bm) {
+    DirectArgs &a = res.args.d;
+    a.a = (const char *)x, a.b = (const char *)w, a.out = (char *)out;
+    a.c_dt = d->y.dtype, a.o_dt = d->out.dtype;
+    a.epi = g.epi;
+    conv_tile_lean(d->epilogue, res.args);
+    fhip_note_kernel(ctx, "conv_igemm unpadded %dx%d split=%d", res.tile.bm, res.tile.bn, res.tile.splits);
+    return conv_tile_launch(ctx, p.kind == GK_BF16, false, res.tile, res.args, scratch);
   }
   // A single tap at unit stride without padding is the matrix product
   // X[pixels][C] . W[K][C]^T of dense operands: the GEMM entry takes them as
@@ -770,9 +848,12 @@ int fhip_fast_conv(fhip_ctx *ctx, const fhip_conv_desc *d, const void *x,
 //   W'[c, k, f'] = W[k, c, F - 1 - f']   (taps mirrored, channel roles swapped)
 // under padding' = dil * (F - 1) - pad.  W' is small (the filter's size); it is
 // rebuilt in the caller's workspace on every call, channels-last, by a
-// transposing copy, and the forward kernel does the rest.  Strides above one:
-// DY is spread over a zero grid first (DY(p, q) at (p * stride, q * stride)),
-// which is the unit-stride case again at stride^2 times the MFMA work.
+// transposing copy, and the forward kernel does the rest.  Gathered tiles
+// (conv_tile_kernel.h) take strides above one, and unit strides where they are
+// faster, from DY and W as they lie.  What strides they leave (groups, channels
+// off 8, more than 16 remainders): DY is spread over a zero grid first (DY(p, q)
+// at (p * stride, q * stride)), which is the unit-stride case again at stride^2
+// times the MFMA work.
 // (Reference node/conv_node.h:428-598; aten.convolution_backward, input
 // gradient.)
 // ---------------------------------------------------------------------------
@@ -949,6 +1030,135 @@ bool fhip_fast_conv_dgrad_applicable(const fhip_conv_desc *d,
   return p.ok;
 }
 
+// The gradient on gathered tiles (conv_tile_kernel.h), which read DY and W in place: strides
+// above one, and unit strides where the forward problem would run on them.
+struct DgradTiles {
+  bool ok = false;
+  bool copy = false; // W is first laid out channels-last in the workspace
+  ConvTileArgs args{};
+  ConvTilePlan plan;
+};
+
+// One spatial dim of a gradient: output rows of remainder `a` by the stride.
+struct DgradRows {
+  int64_t rows, taps, last, off; // rows of DX, taps, the largest one, its place under row 0 of DY
+  DgradRows(int64_t extent, int64_t filter, int64_t stride, int64_t dil, int64_t pad, int64_t a)
+      : rows(a < extent ? (extent - a + stride - 1) / stride : 0), taps(0), last(0), off(0) {
+    for (int64_t r = 0; r < filter; ++r)
+      if ((a + pad - r * dil) % stride == 0)
+        ++taps, last = r, off = (a + pad - r * dil) / stride;
+  }
+};
+
+static DgradTiles make_dgrad_tiles(const fhip_conv_desc *d, const DgradPlan &p, const void *dy, const void *w,
+                                   bool allow_scratch) {
+  DgradTiles t;
+  const int sp = d->spatial_rank;
+  const int64_t K = d->w.dim[0], C = d->w.dim[1];
+  if (fhip_knobs().conv_gather == 0 || C != d->x.dim[1] || C % 8 != 0 || K % 8 != 0 ||
+      (((uintptr_t)dy | (uintptr_t)w) & 15) != 0 || !is_channels_last(d->y) || !is_channels_last(d->x))
+    return t;
+  double other = 0; // of the forward kernel on the mirrored filter
+  if (!p.spread) {
+    if (fhip_fast_conv_rf_applicable(&p.fwd))
+      return t;
+    ConvResolved r = resolve(&p.fwd, allow_scratch, false);
+    if (!r.unpadded())
+      tile_args(r.plan, K, r.args);
+    other = r.tile.bm ? r.tile.us + 2.6 : igemm_us(r, true, false);
+    // (128 x 128 halo tiles are the least well known)
+    other *= !r.unpadded() && r.plan.halo && r.plan.bn == 128 ? 0.9 : 0.95;
+    // (a single tap at unit stride is a matrix product)
+    if (other == 0 || (!r.unpadded() && r.plan.geom.R * r.plan.geom.S == 1))
+      return t;
+  }
+  t.copy = !is_channels_last(d->w);
+  auto dim = [&](const int64_t *v, int i, int64_t none) { return sp == 2 ? v[i] : i == 1 ? v[0] : none; };
+  const int64_t H = sp == 2 ? d->x.dim[2] : 1, W = d->x.dim[1 + sp];
+  const int64_t R = sp == 2 ? d->w.dim[2] : 1, S = d->w.dim[1 + sp];
+  const int64_t P = sp == 2 ? d->y.dim[2] : 1, Q = d->y.dim[1 + sp], N = d->y.dim[0];
+  const int64_t sh = dim(d->stride, 0, 1), sw = dim(d->stride, 1, 1);
+  const int64_t dh = dim(d->dilation, 0, 1), dw = dim(d->dilation, 1, 1);
+  const int64_t ph = dim(d->padding, 0, 0), pw = dim(d->padding, 1, 0);
+  if (sh * sw > kConvTileParts || N * P * Q * K * 2 >= (1ll << 31) || K * R * S * C * 2 >= (1ll << 30) ||
+      N * H * W >= (1ll << 31) || K * R * S >= (1ll << 30))
+    return t;
+  auto gcd = [](int64_t a, int64_t b) {
+    while (b != 0) {
+      const int64_t r = a % b;
+      a = b, b = r;
+    }
+    return a;
+  };
+  // taps of one remainder are `step` apart in the filter, `near` rows of DY
+  const int64_t step_h = sh / gcd(sh, dh), step_w = sw / gcd(sw, dw);
+  ConvTileArgs &g = t.args;
+  for (int64_t a = 0; a < sh; ++a)
+    for (int64_t b = 0; b < sw; ++b) {
+      const DgradRows h(H, R, sh, dh, ph, a), v(W, S, sw, dw, pw, b);
+      if (h.rows * v.rows == 0)
+        continue;
+      ConvTilePart q{};
+      q.M = (int32_t)(N * h.rows * v.rows), q.P = (int32_t)h.rows, q.Q = (int32_t)v.rows;
+      q.J = (int32_t)(h.taps * v.taps * K), q.S = (int32_t)(v.taps > 0 ? v.taps : 1);
+      q.off_h = (int32_t)h.off, q.off_w = (int32_t)v.off;
+      q.h = (int32_t)a, q.w = (int32_t)b;
+      q.w_first = (int32_t)((h.last * S + v.last) * C * 2);
+      q.w_row = (int32_t)(-step_h * S * C * 2), q.w_tap = (int32_t)(-step_w * C * 2);
+      int at = g.parts++; // longest reduction first
+      for (; at > 0 && g.part[at - 1].J < q.J; --at)
+        g.part[at] = g.part[at - 1];
+      g.part[at] = q;
+    }
+  g.d.M = g.part[0].M, g.d.N = (int32_t)C, g.d.K = g.part[0].J;
+  g.H = (int32_t)P, g.W = (int32_t)Q, g.C = (int32_t)K;
+  g.str_h = g.str_w = 1;
+  g.dil_h = (int32_t)(dh / gcd(sh, dh)), g.dil_w = (int32_t)(dw / gcd(sw, dw));
+  g.x_bytes = (uint32_t)(N * P * Q * K * 2), g.w_bytes = (uint32_t)(K * R * S * C * 2);
+  g.w_pitch = (int32_t)(R * S * C * 2);
+  g.out_h = (int32_t)H, g.out_w = (int32_t)W, g.step_h = (int32_t)sh, g.step_w = (int32_t)sw;
+  g.d.o_sm = C, g.d.o_sn = 1;
+  g.d.c_dt = g.d.o_dt = d->x.dtype;
+  // (parts of the reduction: what the entry point without scratch has room for)
+  const size_t copy = t.copy ? p.filter_bytes : 0;
+  t.plan = conv_tile_plan(g, true, false, copy < FHIP_CONV_DGRAD_STATIC_MAX_BYTES ? FHIP_CONV_DGRAD_STATIC_MAX_BYTES - copy : 0);
+  // Strides above one: always (N32 288 -> 176, 38 x 38, 5 x 5 at stride 2 264 -> 85 us; over 74
+  // random layers 0.48 of the time of DY spread over a zero grid, 0.85 at worst).
+  t.ok = t.plan.bm != 0 && (p.spread || t.plan.us + (t.copy ? 2.6 : 0.0) < other);
+  return t;
+}
+
+static int run_dgrad_tiles(fhip_ctx *ctx, const fhip_conv_desc *d, const DgradPlan &p, DgradTiles &t, const void *dy,
+                           const void *w, void *dx, void *workspace, bool allow_scratch) {
+  const int sp = d->spatial_rank;
+  void *partial = nullptr;
+  if (allow_scratch) {
+    size_t bytes = conv_tile_scratch(t.plan, t.args);
+    if (bytes > 0 && !fhip_ctx_scratch_ready(ctx, bytes))
+      t.plan = conv_tile_plan(t.args, true, false, bytes = 0);
+    if (bytes > 0 && fhip_ctx_scratch(ctx, bytes, &partial) != 0)
+      return 1;
+  } else {
+    partial = (char *)workspace + (t.copy ? p.filter_bytes : 0);
+  }
+  if (t.copy) { // [K][R][S][C]: the mirroring copy's roles changed, its taps counted from the other end
+    FlipArgs a;
+    a.K = d->w.dim[1], a.C = d->w.dim[0];
+    a.R = sp == 2 ? d->w.dim[2] : 1, a.S = d->w.dim[1 + sp];
+    a.sk = d->w.dim[1] == 1 ? 0 : d->w.stride[1], a.sc = d->w.dim[0] == 1 ? 0 : d->w.stride[0];
+    a.sr = sp == 2 ? -d->w.stride[2] : 0, a.ss = -d->w.stride[1 + sp];
+    const int64_t total = a.K * a.C * a.R * a.S;
+    hipLaunchKernelGGL(conv_flip_filter_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, ctx->stream, a,
+                       (const uint16_t *)w - (a.R - 1) * a.sr - (a.S - 1) * a.ss, (uint16_t *)workspace, total);
+    FHIP_HIP_CHECK(ctx, hipGetLastError());
+    w = workspace;
+  }
+  t.args.d.a = (const char *)dy, t.args.d.b = (const char *)w, t.args.d.out = (char *)dx;
+  fhip_note_kernel(ctx, "dgrad conv_igemm unpadded %dx%d split=%d parts=%d", t.plan.bm, t.plan.bn, t.plan.splits,
+                   t.args.parts);
+  return conv_tile_launch(ctx, d->y.dtype == FHIP_BFLOAT16, true, t.plan, t.args, partial);
+}
+
 int fhip_fast_conv_dgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy,
                          const void *w, void *dx, void *workspace, bool allow_scratch) {
   const DgradPlan p = make_dgrad_plan(d, allow_scratch);
@@ -959,6 +1169,9 @@ int fhip_fast_conv_dgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy,
     return fhip_fast_conv_dgrad_rf(ctx, d, dy, w, dx);
   FHIP_REQUIRE(ctx, ((uintptr_t)workspace & 15) == 0,
                "conv dgrad: workspace must be 16-byte aligned");
+  DgradTiles tiles = make_dgrad_tiles(d, p, dy, w, allow_scratch);
+  if (tiles.ok)
+    return run_dgrad_tiles(ctx, d, p, tiles, dy, w, dx, workspace, allow_scratch);
   const int sp = d->spatial_rank;
   FlipArgs a;
   const int64_t groups = d->x.dim[1] / d->w.dim[1];
@@ -993,11 +1206,11 @@ int fhip_fast_conv_dgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy,
                        dim3((unsigned)((sa.total + 255) / 256)), dim3(256), 0,
                        ctx->stream, sa, (const uint4 *)dy, (uint4 *)grid);
     FHIP_HIP_CHECK(ctx, hipGetLastError());
-    const int rc = fhip_fast_conv(ctx, &p.fwd, grid, workspace, epi, dx, nullptr, allow_scratch);
+    const int rc = fhip_fast_conv(ctx, &p.fwd, grid, workspace, epi, dx, nullptr, allow_scratch, false);
     dgrad_note(ctx, "dgrad spread + ");
     return rc;
   }
-  const int rc = fhip_fast_conv(ctx, &p.fwd, dy, workspace, epi, dx, nullptr, allow_scratch);
+  const int rc = fhip_fast_conv(ctx, &p.fwd, dy, workspace, epi, dx, nullptr, allow_scratch, false);
   dgrad_note(ctx, "dgrad ");
   return rc;
 }

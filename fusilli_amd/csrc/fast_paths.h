@@ -29,10 +29,11 @@ int fhip_direct_matmul(fhip_ctx *ctx, const fhip_matmul_desc *d, const void *a, 
 // that must not allocate.
 bool fhip_fast_conv_applicable(const fhip_conv_desc *d, bool allow_scratch = true);
 // With `handled` the call plans once and reports whether a tuned kernel was
-// launched; a descriptor that none takes is then no error.
+// launched; a descriptor that none takes is then no error.  `split` false: reductions over
+// whole slices are not cut where the plan without scratch would not cut them.
 int fhip_fast_conv(fhip_ctx *ctx, const fhip_conv_desc *d, const void *x,
                    const void *w, const DevEpilogue &epi, void *out,
-                   bool *handled = nullptr, bool allow_scratch = true);
+                   bool *handled = nullptr, bool allow_scratch = true, bool split = true);
 
 // The same problem on the register-filter kernel (unit stride and dilation,
 // 3 x 3 x 64 filters, K a multiple of 128, 16-bit output, linear epilogue that

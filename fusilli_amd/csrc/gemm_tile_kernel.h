@@ -73,7 +73,6 @@ template <int KIND, bool KC, int ROWS, int T, int STEPS> struct TileOperand {
   // `t`: thread of the team; `lds`: the team's first stage of this operand.
   __device__ __forceinline__ void setup(const char *p, int64_t ld_bytes, int row0, int rows, int t, int tile0, int step0,
                                         uint32_t lds) {
-    const int l = t & 63;
     ldb = (uint32_t)ld_bytes;
     const int r = t / CPR, c = t % CPR;
     if constexpr (KC) {
@@ -86,15 +85,6 @@ template <int KIND, bool KC, int ROWS, int T, int STEPS> struct TileOperand {
         row = (row < rows ? row : rows - 1) - row0;
         off[j] = (uint32_t)row * ldb + (uint32_t)(c * 16);
       }
-      // (STEP is a multiple of 16: the permutation is the same in every load)
-      static_assert(!KC || STEP % 16 == 0, "rows between a thread's chunks");
-      wr = lds + (uint32_t)(r * 128 + ((c ^ kc_swz(r)) << 4));
-      const int fr = tile0 * 32 + (l & 31), sw = kc_swz(l & 31);
-#pragma unroll
-      for (int s = 0; s < STEPS; ++s)
-#pragma unroll
-        for (int i = 0; i < CHH; ++i)
-          rd[s * CHH + i] = lds + (uint32_t)(fr * 128 + ((((step0 + s) * CH + (l >> 5) * CHH + i) ^ sw) << 4));
     } else {
       // (rows >= PE; a chunk that starts early may start in front of the tile)
       const int first = row0 < PE ? 0 : row0 - PE;
@@ -105,6 +95,25 @@ template <int KIND, bool KC, int ROWS, int T, int STEPS> struct TileOperand {
       ragged = row0 + ROWS > rows;
       k0 = r;
       off[0] = (uint32_t)(ee - first) * ELEM + (uint32_t)r * ldb;
+    }
+    place(t, tile0, step0, lds);
+  }
+
+  // Where this thread's chunks go in LDS and its fragments come from.
+  __device__ __forceinline__ void place(int t, int tile0, int step0, uint32_t lds) {
+    const int l = t & 63;
+    const int r = t / CPR, c = t % CPR;
+    if constexpr (KC) {
+      // (STEP is a multiple of 16: the permutation is the same in every load)
+      static_assert(!KC || STEP % 16 == 0, "rows between a thread's chunks");
+      wr = lds + (uint32_t)(r * 128 + ((c ^ kc_swz(r)) << 4));
+      const int fr = tile0 * 32 + (l & 31), sw = kc_swz(l & 31);
+#pragma unroll
+      for (int s = 0; s < STEPS; ++s)
+#pragma unroll
+        for (int i = 0; i < CHH; ++i)
+          rd[s * CHH + i] = lds + (uint32_t)(fr * 128 + ((((step0 + s) * CH + (l >> 5) * CHH + i) ^ sw) << 4));
+    } else {
       static_assert(KC || STEP % 8 == 0, "the permutation is the same in every load");
       wr = lds + (uint32_t)(r * RB + tile_pos<ELEM, RB>(r, c) * 16);
       const int L = l & 15, h = (l >> 4) & 1;
@@ -229,14 +238,15 @@ template <int V> struct TileColumns {
   }
 };
 
-// Finishes and stores the V values of columns n .. of row m.
-template <typename Acc, int V>
-__device__ __forceinline__ void tile_store(const DirectArgs &g, int64_t batch, int m, int n, const Acc (&acc)[V],
-                                           const TileColumns<V> *lean = nullptr) {
-  if (m >= g.M || n >= g.N)
+// Finishes and stores the V values of columns n .. of row m, which starts at element `row` of
+// OUT (-1: there is no such row).
+template <typename Acc, int V, bool PLAIN = false>
+__device__ __forceinline__ void tile_store(const DirectArgs &g, int64_t batch, int m, int64_t row, int n,
+                                           const Acc (&acc)[V], const TileColumns<V> *lean = nullptr) {
+  if (row < 0 || n >= g.N)
     return;
   const int live = g.N - n < V ? g.N - n : V;
-  const int64_t at = batch * g.o_batch + (int64_t)m * g.o_sm + (int64_t)n * g.o_sn;
+  const int64_t at = row + (int64_t)n * g.o_sn;
   if constexpr (std::is_same<Acc, int>::value) {
     typedef int loose __attribute__((ext_vector_type(4), aligned(4)));
     GEMM_AS1 int32_t *out = (GEMM_AS1 int32_t *)g.out + at;
@@ -256,7 +266,8 @@ __device__ __forceinline__ void tile_store(const DirectArgs &g, int64_t batch, i
     for (int i = 0; i < V; ++i)
       v[i] = acc[i];
     fhip_round_fast_vec<V>(g.c_dt, v);
-    if (lean && g.lean) {
+    if (PLAIN) { // (no fused chain)
+    } else if (lean && g.lean) {
       for (int i = 0; i < g.epi.count; ++i) {
         const DevEpiOp &o = g.epi.op[i];
         if (o.kind == FHIP_OPERAND_NONE) {
@@ -316,9 +327,9 @@ __device__ __forceinline__ void tile_store(const DirectArgs &g, int64_t batch, i
 
 // Adds a tile's SUMS shares of K in LDS, finishes and stores it, or stores the plain sums of
 // a split product.
-template <typename Acc, int V, int BM, int BN, int SUMS, int PITCH, int SUM, int THREADS>
+template <typename Acc, int V, int BM, int BN, int SUMS, int PITCH, int SUM, int THREADS, bool PLAIN, class Row>
 __device__ __forceinline__ void tile_finish(const DirectArgs &g, uint32_t lds, uint32_t id, int64_t batch, int m0, int n0,
-                                            const TileColumns<V> &columns) {
+                                            const TileColumns<V> &columns, const Row &at_row) {
   typedef Acc Acc4 __attribute__((ext_vector_type(4)));
   constexpr int RUNS = BN / V; // runs of V columns in a row
 #pragma clang loop unroll(disable)
@@ -341,7 +352,7 @@ __device__ __forceinline__ void tile_finish(const DirectArgs &g, uint32_t lds, u
       for (int q = 0; q < V; q += 4)
         to[q / 4] = Acc4{v[q], v[q + 1], v[q + 2], v[q + 3]};
     } else {
-      tile_store<Acc, V>(g, batch, m0 + row, n0 + col, v, &columns);
+      tile_store<Acc, V, PLAIN>(g, batch, m0 + row, at_row(m0 + row), n0 + col, v, &columns);
     }
   }
 }
@@ -349,10 +360,12 @@ __device__ __forceinline__ void tile_finish(const DirectArgs &g, uint32_t lds, u
 // Wavefronts of a team own 64 x 64 outputs each and share the slice's K-steps where the tile
 // is smaller than four of those, so that few bytes of a stage are read twice (fp8 has two
 // K-steps only: 64 x 64 tiles, 64 x 32 outputs each).
-template <int KIND, int MT, int NT, int TEAMS> struct TileShape {
-  static constexpr int BM = 64 * MT, BN = 64 * NT;
-  static constexpr int WK = KindTraits<KIND>::kStepBytes == 64 && MT * NT == 1 ? 2 : 4 / (MT * NT);
-  static constexpr int WM = MT, WN = 4 / WK / WM;
+// SHORT (64 x 64 tiles): a quarter of the tile each, every byte read twice, for reductions that
+// are over before it shows: no shares to add, and half the registers.
+template <int KIND, int MT, int NT, int TEAMS_, bool SHORT = false> struct TileShape {
+  static constexpr int BM = 64 * MT, BN = 64 * NT, TEAMS = TEAMS_;
+  static constexpr int WK = SHORT ? 1 : KindTraits<KIND>::kStepBytes == 64 && MT * NT == 1 ? 2 : 4 / (MT * NT);
+  static constexpr int WM = SHORT ? 2 : MT, WN = 4 / WK / WM;
   static constexpr int TM = BM / WM / 32, TN = BN / WN / 32;
   static constexpr int STEPS = 128 / KindTraits<KIND>::kStepBytes / WK;
   static constexpr int kStage = (BM + BN) * 128;    // a slice of both operands
@@ -363,44 +376,46 @@ template <int KIND, int MT, int NT, int TEAMS> struct TileShape {
   static constexpr int V = BM * BN / (256 * TEAMS) >= 8 ? 8 : 4; // columns that a thread finishes
 };
 
-template <int KIND, bool A_KC, bool B_KC, int MT, int NT, int TEAMS, int U>
-__global__ __launch_bounds__(256 * TEAMS)
-__attribute__((amdgpu_waves_per_eu(2, 8))) void gemm_tile_kernel(DirectArgs g) {
-  using D = DirectKind<KIND>;
-  using Acc = typename D::Acc;
-  using S = TileShape<KIND, MT, NT, TEAMS>;
-  constexpr int BM = S::BM, BN = S::BN, TM = S::TM, TN = S::TN;
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int team = wave >> 2, w = wave & 3;
-  const int wk = w % S::WK, wn = w / S::WK % S::WN, wm = w / (S::WK * S::WN);
-  const int t = threadIdx.x & 255, l = threadIdx.x & 63;
-  // (workgroups go to the eight L2 slices in turn: each slice gets a run of neighbouring
-  // tiles, column after column)
-  uint32_t id = blockIdx.x;
-  {
-    const uint32_t per = gridDim.x / 8, rest = gridDim.x % 8, slice = id % 8;
-    id = slice * per + (slice < rest ? slice : rest) + id / 8;
+// The share of K of a team: its whole slices, and how many the longest team of the workgroup
+// has; where K ends inside a slice, the last team of the last part takes that one first.
+struct TilePart {
+  int whole, krem, s0, count, longest;
+  bool cut, cut_mine; // (`cut`: uniform over the workgroup)
+  __device__ __forceinline__ TilePart(int whole_, int krem_, int splits, int teams, int team) : whole(whole_), krem(krem_) {
+    const int parts = splits * teams, part = blockIdx.y * teams + team;
+    s0 = (int)((int64_t)whole * part / parts);
+    count = (int)((int64_t)whole * (part + 1) / parts) - s0;
+    longest = (whole + parts - 1) / parts;
+    cut = krem > 0 && (int)blockIdx.y == splits - 1;
+    cut_mine = cut && team == teams - 1;
   }
-  const int tile_m = id % (uint32_t)g.tiles_m, tile_n = id / (uint32_t)g.tiles_m;
-  const int64_t batch = blockIdx.z;
-  const int m0 = tile_m * BM, n0 = tile_n * BN;
-  // this team's whole slices, and how many the longest team of the workgroup has; where K
-  // ends inside a slice, the last team of the last part takes that one first
-  const int whole = g.K / D::SK, krem = g.K - whole * D::SK;
-  const int parts = g.splits * TEAMS, part = blockIdx.y * TEAMS + team;
-  const int s0 = (int)((int64_t)whole * part / parts);
-  const int count = (int)((int64_t)whole * (part + 1) / parts) - s0;
-  const int longest = (whole + parts - 1) / parts;
-  const bool cut = krem > 0 && (int)blockIdx.y == g.splits - 1; // (uniform over the workgroup)
-  const bool cut_mine = cut && team == TEAMS - 1;
-  using OA = TileOperand<KIND, A_KC, BM, TM, S::STEPS>;
-  using OB = TileOperand<KIND, B_KC, BN, TN, S::STEPS>;
-  const uint32_t lds = (uint32_t)(uintptr_t)smem + (uint32_t)(team * 2 * S::kStage);
-  OA oa;
-  OB ob;
-  oa.setup(g.a + batch * g.a_batch * D::ELEM, g.a_ldb, m0, g.M, t, wm * TM, wk * S::STEPS, lds);
-  ob.setup(g.b + batch * g.b_batch * D::ELEM, g.b_ldb, n0, g.N, t, wn * TN, wk * S::STEPS, lds + OA::BYTES);
+};
+
+// A team's wavefront: which share of a slice's K-steps, rows and columns it has.
+template <class S> struct TileWave {
+  int team, wk, wn, wm;
+  __device__ __forceinline__ TileWave() {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), w = wave & 3;
+    team = wave >> 2;
+    wk = w % S::WK, wn = w / S::WK % S::WN, wm = w / (S::WK * S::WN);
+  }
+};
+
+// (workgroups go to the eight L2 slices in turn: each slice gets a run of neighbouring tiles)
+__device__ __forceinline__ uint32_t tile_id() {
+  const uint32_t id = blockIdx.x, per = gridDim.x / 8, rest = gridDim.x % 8, slice = id % 8;
+  return slice * per + (slice < rest ? slice : rest) + id / 8;
+}
+
+// The tile at (m0, n0) whose operands are set up; `at_row(m)`: where row m of OUT starts, -1
+// behind the last.  PLAIN: no fused chain.
+template <int KIND, class S, int U, bool CUT, bool PLAIN, class OA, class OB, class Row>
+__device__ __forceinline__ void tile_run(const DirectArgs &g, uint32_t smem, const TilePart &p, const TileWave<S> &at, OA &oa,
+                                         OB &ob, uint32_t id, int64_t batch, int m0, int n0, const Row &at_row) {
+  using Acc = typename DirectKind<KIND>::Acc;
+  constexpr int BM = S::BM, BN = S::BN, TM = S::TM, TN = S::TN, TEAMS = S::TEAMS;
+  const int team = at.team, wk = at.wk, wn = at.wn, wm = at.wm, l = threadIdx.x & 63;
+  const int s0 = p.s0, count = p.count, longest = p.longest;
   typename KindTraits<KIND>::AccVec acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
@@ -432,9 +447,11 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void gemm_tile_kernel(DirectArgs g) {
   };
   typename OA::Raw ca;
   typename OB::Raw cb;
-  if (cut_mine) {
-    oa.template fetch<true>(whole, krem, ca);
-    ob.template fetch<true>(whole, krem, cb);
+  if constexpr (CUT) {
+    if (p.cut_mine) {
+      oa.template fetch<true>(p.whole, p.krem, ca);
+      ob.template fetch<true>(p.whole, p.krem, cb);
+    }
   }
   // Loads of whole slices stand outside every branch: where control flow joins, the compiler
   // can only wait for all loads in flight, and the slices ahead would be waited for with the
@@ -443,7 +460,7 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void gemm_tile_kernel(DirectArgs g) {
     const int last = s0 + (count > 0 ? count - 1 : 0);
     int at = s0 + s;
     at = at < last ? at : last;
-    at = at < whole ? at : whole - 1;
+    at = at < p.whole ? at : p.whole - 1;
     oa.template fetch<false>(at, 0, va);
     ob.template fetch<false>(at, 0, vb);
   };
@@ -459,18 +476,22 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void gemm_tile_kernel(DirectArgs g) {
     ob.put(rb[0], 0);
     fetch(U, ra[0], rb[0]);
   }
-  if (cut_mine) {
-    oa.template put<true>(ca, S::kStage, krem);
-    ob.template put<true>(cb, S::kStage, krem);
+  if constexpr (CUT) {
+    if (p.cut_mine) {
+      oa.template put<true>(ca, S::kStage, p.krem);
+      ob.template put<true>(cb, S::kStage, p.krem);
+    }
   }
   meet();
-  if (cut) {
-    if (cut_mine)
-      gemm_static_for<S::STEPS>([&](auto kc) {
-        read(kc, S::kStage, C0{});
-        product(C0{});
-      });
-    meet(); // (the second stage is free again)
+  if constexpr (CUT) {
+    if (p.cut) {
+      if (p.cut_mine)
+        gemm_static_for<S::STEPS>([&](auto kc) {
+          read(kc, S::kStage, C0{});
+          product(C0{});
+        });
+      meet(); // (the second stage is free again)
+    }
   }
   // One barrier per slice.  In front of it the last fragments of slice s are read and the
   // products but the last step's are under way; behind it the first fragments of slice s + 1
@@ -508,7 +529,7 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void gemm_tile_kernel(DirectArgs g) {
   // (a thread finishes the same columns of several rows)
   static_assert(256 * TEAMS % (BN / S::V) == 0, "columns of a thread");
   TileColumns<S::V> columns;
-  if (g.lean && g.lean_op >= 0 && !g.partial)
+  if (!PLAIN && g.lean && g.lean_op >= 0 && !g.partial)
     columns.request(g, n0 + (int)(threadIdx.x % (BN / S::V)) * S::V);
   gemm_static_for<U>([&](auto uc) {
     constexpr int u = decltype(uc)::value, n = (u + 2) % U;
@@ -531,7 +552,7 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void gemm_tile_kernel(DirectArgs g) {
   // 4 (l / 32) + r % 4 of its 32 x 32 tile, column l % 32
   __syncthreads();
   {
-    GEMM_AS3 Acc *mine = (GEMM_AS3 Acc *)(uintptr_t)((uint32_t)(uintptr_t)smem + (uint32_t)((team * S::WK + wk) * S::kSum));
+    GEMM_AS3 Acc *mine = (GEMM_AS3 Acc *)(uintptr_t)(smem + (uint32_t)((team * S::WK + wk) * S::kSum));
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -542,15 +563,43 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void gemm_tile_kernel(DirectArgs g) {
                (l & 31)] = acc[i][j][r];
   }
   __syncthreads();
-  tile_finish<Acc, S::V, BM, BN, S::kSums, S::kPitch, S::kSum, 256 * TEAMS>(g, (uint32_t)(uintptr_t)smem, id, batch, m0,
-                                                                           n0, columns);
+  tile_finish<Acc, S::V, BM, BN, S::kSums, S::kPitch, S::kSum, 256 * TEAMS, PLAIN>(g, smem, id, batch, m0, n0, columns,
+                                                                                  at_row);
+}
+
+template <int KIND, bool A_KC, bool B_KC, int MT, int NT, int TEAMS, int U>
+__global__ __launch_bounds__(256 * TEAMS)
+__attribute__((amdgpu_waves_per_eu(2, 8))) void gemm_tile_kernel(DirectArgs g) {
+  using D = DirectKind<KIND>;
+  using S = TileShape<KIND, MT, NT, TEAMS>;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const TileWave<S> at;
+  const int t = threadIdx.x & 255;
+  const uint32_t id = tile_id(); // (column after column)
+  const int tile_m = id % (uint32_t)g.tiles_m, tile_n = id / (uint32_t)g.tiles_m;
+  const int64_t batch = blockIdx.z;
+  const int m0 = tile_m * S::BM, n0 = tile_n * S::BN;
+  const int whole = g.K / D::SK;
+  const TilePart p(whole, g.K - whole * D::SK, g.splits, TEAMS, at.team);
+  using OA = TileOperand<KIND, A_KC, S::BM, S::TM, S::STEPS>;
+  using OB = TileOperand<KIND, B_KC, S::BN, S::TN, S::STEPS>;
+  const uint32_t lds = (uint32_t)(uintptr_t)smem + (uint32_t)(at.team * 2 * S::kStage);
+  OA oa;
+  OB ob;
+  oa.setup(g.a + batch * g.a_batch * D::ELEM, g.a_ldb, m0, g.M, t, at.wm * S::TM, at.wk * S::STEPS, lds);
+  ob.setup(g.b + batch * g.b_batch * D::ELEM, g.b_ldb, n0, g.N, t, at.wn * S::TN, at.wk * S::STEPS, lds + OA::BYTES);
+  tile_run<KIND, S, U, true, false>(
+      g, (uint32_t)(uintptr_t)smem, p, at, oa, ob, id, batch, m0, n0,
+      [&](int m) { return m < g.M ? batch * g.o_batch + (int64_t)m * g.o_sm : (int64_t)-1; });
 }
 
 // Adds the split parts of every tile in order and finishes as above: four columns a thread.
-template <typename Acc, int BM, int BN>
+template <typename Acc, int BM, int BN, bool BY_ROWS = false>
 __global__ __launch_bounds__(256) void gemm_tile_finish_kernel(DirectArgs g) {
   typedef Acc Acc4 __attribute__((ext_vector_type(4)));
-  const int tile_m = blockIdx.x % (uint32_t)g.tiles_m, tile_n = blockIdx.x / (uint32_t)g.tiles_m;
+  const uint32_t run = (uint32_t)(BY_ROWS ? g.tiles_n : g.tiles_m); // tiles one after another, row by row or down a column
+  const int along = blockIdx.x % run, over = blockIdx.x / run;
+  const int tile_m = BY_ROWS ? over : along, tile_n = BY_ROWS ? along : over;
   const int64_t batch = blockIdx.z;
   const int q = blockIdx.y * 256 + threadIdx.x;
   const GEMM_AS1 Acc4 *p = (const GEMM_AS1 Acc4 *)g.partial + (batch * gridDim.x + blockIdx.x) * (BM * BN / 4) + q;
@@ -560,7 +609,8 @@ __global__ __launch_bounds__(256) void gemm_tile_finish_kernel(DirectArgs g) {
   for (int s = 1; s < g.splits; ++s)
     x += p[s * stride];
   const Acc v[4] = {x.x, x.y, x.z, x.w};
-  tile_store<Acc, 4>(g, batch, tile_m * BM + q / (BN / 4), tile_n * BN + q % (BN / 4) * 4, v);
+  const int m = tile_m * BM + q / (BN / 4);
+  tile_store<Acc, 4>(g, batch, m, m < g.M ? batch * g.o_batch + (int64_t)m * g.o_sm : -1, tile_n * BN + q % (BN / 4) * 4, v);
 }
 
 template <int KIND, bool A_KC, bool B_KC, int MT, int NT, int TEAMS, int U>
