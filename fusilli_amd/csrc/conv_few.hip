@@ -3,8 +3,8 @@
 //
 // Bound by reading and writing the many-channel tensor once; the direct kernels
 // (conv_direct.hip) kept one pixel per thread and fetched every X or DY value from
-// the caches once per tap and channel block.  All arithmetic stays f32: 16-bit
-// tensors are widened when they are staged.
+// the caches once per tap and channel block.  All sums are f32; 16-bit tensors are widened when
+// they are staged, but in the products of the data gradient, where the MFMA does that.
 //   * forward: X of 256 output pixels, padded with zeros, and the filter sit in LDS;
 //     pixels x output channels on 16 x 16 x 4 f32 MFMAs over the (channel, tap) pairs.
 //     A wavefront's four tiles interleave their pixels so that a lane ends up with 16
@@ -13,14 +13,16 @@
 //     straight from memory (four consecutive pixels per lane), X from LDS; a
 //     workgroup keeps its sums over many bands of rows, the workgroups' sums meet in
 //     the context's scratch and are added in a fixed order;
-//   * data gradient: one to four input channels leave a matrix tile mostly empty, so a
-//     lane computes 4 x 2 pixels x all channels with vector instructions, the wavefronts
-//     of a workgroup each over a share of the output channels, whose DY rows they
-//     stage for themselves; the shares are added through LDS.
+//   * data gradient: products first (pairs x pixels of DY on the MFMAs, summed over the
+//     output channels), then the taps of a DX pixel are added in LDS.  Where that takes
+//     several passes over the input channels and does not pay, a lane computes 4 x 2 pixels x
+//     all channels with vector instructions, the wavefronts of a workgroup each over a
+//     share of the output channels, whose DY rows they stage for themselves; the shares are
+//     added through LDS.
 //
 // One training step (us):
-//   N100 3 -> 32, 32 x 32, 3 x 3, f32: fprop 26.2 -> 15.5, dgrad 60.5 -> 15.0, wgrad 46.1 -> 13.0
-//   N122 1 -> 64, 57 x 57, 5 x 5, bf16: 136 -> 52.6, 701 -> 78.6, 495 -> 45.7
+//   N100 3 -> 32, 32 x 32, 3 x 3, f32: fprop 26.2 -> 15.5, dgrad 60.5 -> 15.0 -> 11.1, wgrad 46.1 -> 13.0
+//   N122 1 -> 64, 57 x 57, 5 x 5, bf16: 136 -> 52.6, 701 -> 78.6 -> 33.0, 495 -> 45.7
 //
 // Reference semantics: aten.convolution / aten.convolution_backward
 // (reference support/asm_emitter.h:690-701, 868-873, 1030-1035).
@@ -35,6 +37,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kCfThreads = 256;
 constexpr int kCfLds = 64 * 1024;
+constexpr int kCfDgradLds = 160 * 1024;
 constexpr int kCfMaxPairs = 112;
 
 struct CfArgs {
@@ -47,14 +50,18 @@ struct CfArgs {
   int32_t xrows;               // most rows of X staged at once
   int32_t tiles;               // forward: workgroups per image; gradients: bands
   int32_t band;                // output (data gradient: input) rows per band
-  int32_t quads;               // data gradient: runs of 4 pixels per row
+  int32_t quads;               // data gradient: runs of 4 pixels per row,
+  int32_t wt;                  // products: columns per band,
+  int32_t cb, wpitch, gat, gpitch; // channels per pass, pitch of the filter, where G starts, pitch of a row in G
+  int32_t packed;              // W without gaps, in this order
+  uint32_t w_magic, quads_magic;
   DevEpilogue epi;
 };
 
 // e / d for e, d < 2^16 with magic = 2^32 / d + 1 (0 stands for d = 1)
 uint32_t cf_magic(int d) { return d == 1 ? 0u : (uint32_t)((1ull << 32) / (uint32_t)d + 1); }
 __device__ __forceinline__ int cf_div(int e, uint32_t magic) {
-  return magic == 0 ? e : (int)__umulhi((uint32_t)e, magic);
+  return (int)__umulhi((uint32_t)e, magic) + (magic == 0 ? e : 0);
 }
 
 // X rows [row0, row0 + rows) of all channels of an image, zeros outside it, as f32.
@@ -585,6 +592,270 @@ __global__ __launch_bounds__(512) void conv_few_dgrad_kernel(CfArgs g, const T *
   }
 }
 
+// ---- data gradient, products first ----------------------------------------------
+// G[pair][pixel of DY] = sum over the output channels on the matrix cores, into LDS; a DX
+// pixel then adds the R * S values of G that fall on it.  Bound by latency: a wavefront requests
+// its 64 pixels of all channels at once, straight from memory, 4 consecutive pixels of a channel
+// per load, and the filter behind them.  f32 N100 3 -> 32, 32 x 32, 3 x 3 (medians): 2.2 us to the
+// last request, 1.6 for the data, 2.1 products, 2.8 taps; the lanes that keep 4 x 2 pixels take 7.3
+// us for their loop of dependent rounds.  Where three tiles of pairs do not hold all input channels,
+// passes of `cb` channels follow each other on the same registers or, while that fits two workgroups
+// per compute unit, lie side by side.
+//
+// us, before -> now: f32 N100 3 -> 32, 32 x 32, 3 x 3 12.9 -> 11.1, N110 1 -> 32, 20 x 20 9.6 -> 5.6, N67
+// 4 -> 32, 62 x 62 28.5 -> 25.7; bf16 N122 1 -> 64, 57 x 57, 5 x 5 77.0 -> 33.0, N118 3 -> 64, 39 x 39,
+// 3 x 3 36.8 -> 15.1, N49 4 -> 64, 24 x 24 23.1 -> 7.2.
+template <typename T> struct CfDgrad {
+  static constexpr bool WIDE = sizeof(T) == 4; // f32: 16 x 16 x 4 products, else 16 x 16 x 32
+  static constexpr int STEP = WIDE ? 4 : 32;   // channels of a product
+  static constexpr int ROWS = WIDE ? 1 : 8;    // of them in a lane
+  typedef T Quad __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+  typedef T Eight __attribute__((ext_vector_type(8)));
+};
+
+// (a 16-bit product of eight channels per lane; never called with f32)
+template <typename T, typename V> __device__ __forceinline__ f32x4 cf_mfma(V a, V b, f32x4 c) {
+  if constexpr (std::is_same<T, __bf16>::value)
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+
+// KB: output channels in registers at once; PT: tiles of 16 pairs.
+template <typename T, int S, int PT, int KB>
+__global__ __launch_bounds__(1024) void conv_few_dgrad_products_kernel(CfArgs g, const T *dy, const T *w,
+                                                             T *dx) {
+  typedef CfDgrad<T> D;
+  typedef typename D::Quad Quad;
+  constexpr int STEPS = KB / D::STEP;
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  const int tid = threadIdx.x, l = tid & 63, threads = blockDim.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = threads >> 6;
+  const int n = blockIdx.x / g.tiles, h0 = (blockIdx.x - n * g.tiles) * g.band;
+  const int w0 = blockIdx.y * g.wt;
+  const int rows = g.H - h0 < g.band ? g.H - h0 : g.band, cols = g.W - w0 < g.wt ? g.W - w0 : g.wt;
+  // Rows and columns of DY that reach this band (whole rows unless bands are cut).  A row is
+  // whole quads, in G followed by the zeros that the taps beside the image meet.
+  int p0 = h0 + g.pad_h - (g.R - 1), p1 = h0 + rows - 1 + g.pad_h;
+  p0 = p0 < 0 ? 0 : p0;
+  p1 = p1 < g.P ? p1 : g.P - 1;
+  const int np = p1 >= p0 ? p1 - p0 + 1 : 0;
+  int q0 = 0, q1 = g.Q - 1;
+  if (gridDim.y > 1) {
+    q0 = w0 + g.pad_w - (S - 1), q1 = w0 + cols - 1 + g.pad_w;
+    q0 = q0 < 0 ? 0 : q0 < g.Q ? q0 : g.Q - 1;
+    q1 = q1 < q0 ? q0 : q1 < g.Q ? q1 : g.Q - 1;
+  }
+  const int nq = q1 - q0 + 1, per_row = (nq + 3) >> 2, pitch = g.gpitch;
+  const int quads = np * per_row, units = (quads + 15) >> 4;
+  // A row's last quad may reach behind it (its values are not used) wherever DY goes on there.
+  const bool whole = (nq & 3) == 0 ||
+                     (g.Q >= 4 && ((p1 + 1 < g.P && g.ys[2] >= 4) || (n + 1 < g.N && g.ys[0] >= 4)));
+  // (then a row's address is a uniform one plus 32 bits per lane)
+  const bool fast = whole && (D::WIDE || (g.K & 7) == 0) && g.ys[1] < (1 << 24) && g.ys[2] < (1 << 16);
+  const T *src = dy + n * g.ys[0] + (int64_t)p0 * g.ys[2] + q0;
+  auto quad_row = [&](int i) { return gridDim.y > 1 ? i / per_row : cf_div(i, g.quads_magic); };
+  Quad raw[STEPS][D::ROWS];
+  auto fetch = [&](int unit, int k0) {
+    asm volatile("" : "+s"(k0)); // (row addresses are not kept from one call to the next)
+    int i = unit * 16 + (l & 15);
+    i = i < quads ? i : quads - 1;
+    const int row = quad_row(i), col = (i - row * per_row) * 4;
+    if (fast) {
+      const uint32_t at = (uint32_t)(row * (int)g.ys[2] + col);
+      const uint32_t part = (uint32_t)((l >> 4) * D::ROWS), ks = (uint32_t)g.ys[1];
+#pragma unroll
+      for (int s = 0; s < STEPS; ++s) {
+        // (channels behind the last one stand for channels in front of it)
+        const int k = k0 + s * D::STEP, left = g.K - k;
+        const uint32_t last = left >= D::STEP ? D::STEP : left > 0 ? (uint32_t)left - D::ROWS : 0u;
+        const uint32_t off = (at + (part < last ? part : last) * ks) * (uint32_t)sizeof(T);
+#pragma unroll
+        for (int r = 0; r < D::ROWS; ++r) {
+          const T *base = src + (k + r < g.K ? k + r : g.K - 1) * g.ys[1];
+          raw[s][r] = *(const Quad *)((const char *)base + off);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int s = 0; s < STEPS; ++s)
+#pragma unroll
+        for (int r = 0; r < D::ROWS; ++r) {
+          int k = k0 + s * D::STEP + (l >> 4) * D::ROWS + r;
+          k = k < g.K ? k : g.K - 1;
+          const T *q = src + ((int64_t)row * g.ys[2] + k * g.ys[1]);
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            raw[s][r][j] = q[col + j < nq ? col + j : nq - 1];
+          __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+  };
+  // the filter: f32 [channel][pair], else [pair][channel], zeros behind the last channel
+  T *wl = (T *)smem;
+  const int kpad = (g.K + D::STEP - 1) / D::STEP * D::STEP;
+  auto stage = [&](auto packed) {
+    constexpr int kBatch = 8; // (loads in flight; in branches of their own they would wait for each other)
+    const int total = g.K * g.J;
+    for (int e0 = tid; e0 < total; e0 += kBatch * threads) {
+      T v[kBatch];
+      int to[kBatch];
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) {
+        int e = e0 + i * threads;
+        e = e < total ? e : total - 1;
+        const int k = cf_div(e, g.q_magic), j = e - k * g.J;
+        to[i] = D::WIDE ? k * g.wpitch + j : j * g.wpitch + k;
+        if constexpr (decltype(packed)::value) {
+          v[i] = w[e];
+        } else {
+          const int c = cf_div(j, g.rs_magic), t = j - c * g.R * S, r = cf_div(t, g.s_magic);
+          v[i] = w[k * g.ws[0] + c * (int)g.ws[1] + r * (int)g.ws[2] + (t - r * S) * (int)g.ws[3]];
+        }
+      }
+      // (the last one may be written several times)
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i)
+        wl[to[i]] = v[i];
+    }
+    for (int e = tid; e < (kpad - g.K) * g.J; e += threads) {
+      const int k = cf_div(e, g.q_magic), j = e - k * g.J;
+      wl[D::WIDE ? (g.K + k) * g.wpitch + j : j * g.wpitch + g.K + k] = (T)0.f;
+    }
+  };
+  float *gl = smem + g.gat + 4; // G, [pair][row][column], zeros in front of it
+  const int gp = np * pitch, rs = g.R * S;
+  const bool held = units <= waves && g.K <= KB;
+  bool first = true;
+  for (int c0 = blockIdx.z * g.cb; c0 < g.C; c0 += gridDim.z * g.cb) {
+    const int cs = g.C - c0 < g.cb ? g.C - c0 : g.cb, pairs = cs * rs;
+    // (every wavefront takes part in every round: the first one holds a barrier)
+    for (int unit = wave; unit - wave < units; unit += waves) {
+      f32x4 acc[PT][4];
+#pragma unroll
+      for (int u = 0; u < PT; ++u)
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          acc[u][t] = f32x4{0, 0, 0, 0};
+      for (int k0 = 0; k0 < g.K; k0 += KB) {
+        if (first || !held)
+          fetch(unit, k0);
+        if (first) {
+          if (g.packed)
+            stage(std::true_type{});
+          else
+            stage(std::false_type{});
+          if (tid < 4)
+            gl[tid - 4] = 0.f;
+          if (pitch > 4 * per_row)
+            for (int i = tid; i < g.cb * rs * np; i += threads)
+              for (int j = 4 * per_row; j < pitch; j += 4)
+                *(f32x4 *)(gl + i * pitch + j) = f32x4{0, 0, 0, 0};
+          __syncthreads();
+          first = false;
+        }
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) {
+          const int k = k0 + s * D::STEP;
+          if (k >= g.K)
+            continue;
+          if (k + D::STEP > g.K) // (0 x infinity)
+#pragma unroll
+            for (int r = 0; r < D::ROWS; ++r)
+              if (k + (l >> 4) * D::ROWS + r >= g.K)
+                raw[s][r] = Quad{};
+          if constexpr (D::WIDE) {
+            const float *wr = (const float *)wl + (k + (l >> 4)) * g.wpitch + c0 * rs + (l & 15);
+#pragma unroll
+            for (int u = 0; u < PT; ++u) {
+              const float a = wr[u * 16];
+#pragma unroll
+              for (int t = 0; t < 4; ++t)
+                acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, (float)raw[s][0][t], acc[u][t], 0, 0, 0);
+            }
+          } else {
+            typename D::Eight b[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+              for (int r = 0; r < 8; ++r)
+                b[t][r] = raw[s][r % D::ROWS][t];
+#pragma unroll
+            for (int u = 0; u < PT; ++u) {
+              const auto a = *(const typename D::Eight *)(wl + (c0 * rs + u * 16 + (l & 15)) * g.wpitch + k +
+                                                          (l >> 4) * 8);
+#pragma unroll
+              for (int t = 0; t < 4; ++t)
+                acc[u][t] = cf_mfma<T>(a, b[t], acc[u][t]);
+            }
+          }
+        }
+      }
+      // value r of tile (u, t): pair u * 16 + (l / 16) * 4 + r, pixel t of quad l % 16
+      const int i = unit * 16 + (l & 15);
+      if (i < quads) {
+        const int row = quad_row(i), col = (i - row * per_row) * 4;
+        float *to = gl + (l >> 4) * 4 * gp + row * pitch + col;
+        if (col + 4 > nq)
+#pragma unroll
+          for (int t = 1; t < 4; ++t)
+            if (col + t >= nq)
+#pragma unroll
+              for (int u = 0; u < PT; ++u)
+                acc[u][t] = f32x4{0, 0, 0, 0};
+#pragma unroll
+        for (int u = 0; u < PT; ++u)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (u * 16 + (l >> 4) * 4 + r < pairs)
+              *(f32x4 *)(to + (u * 16 + r) * gp) = f32x4{acc[u][0][r], acc[u][1][r], acc[u][2][r], acc[u][3][r]};
+      }
+    }
+    __syncthreads();
+    // runs of four pixels of DX
+    const int per = (cols + 3) >> 2, plane = rows * per;
+    for (int e = tid; e < cs * plane; e += threads) {
+      int c = 0, i = e;
+      for (; i >= plane; i -= plane)
+        ++c;
+      const int hh = cols == g.wt ? cf_div(i, g.w_magic) : i / per, wc = (i - hh * per) * 4;
+      // tap (r, s) of a pixel: row p - r, column q - s of DY
+      const int p = h0 + hh + g.pad_h, q = w0 + wc + g.pad_w - q0;
+      const float *from = gl + c * rs * gp;
+      typedef float Four __attribute__((ext_vector_type(4), aligned(4)));
+      f32x4 sum{0, 0, 0, 0};
+#pragma unroll 3
+      for (int r = 0; r < g.R; ++r) {
+        const bool in = p - r >= p0 && p - r <= p1;
+        const float *row = from + r * S * gp + (in ? (p - r - p0) * pitch + q : 0);
+        f32x4 v[S];
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+          v[s] = *(const Four *)(row + s * gp - s);
+#pragma unroll
+        for (int s = 1; s < S; ++s)
+          v[0] += v[s];
+        sum += in ? v[0] : f32x4{0, 0, 0, 0};
+      }
+      T *to = dx + (n * g.xs[0] + (c0 + c) * g.xs[1] + (h0 + hh) * g.xs[2] + w0 + wc);
+      if (wc + 4 <= cols) {
+        Quad t;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          t[j] = (T)sum[j];
+        *(Quad *)to = t;
+      } else {
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+          if (wc + j < cols)
+            to[j] = (T)sum[j];
+      }
+    }
+    if (c0 + (int)gridDim.z * g.cb < g.C)
+      __syncthreads();
+  }
+}
+
 // ---- host side -------------------------------------------------------------------
 bool cf_type(int dt) { return dt == FHIP_FLOAT || dt == FHIP_BFLOAT16 || dt == FHIP_HALF; }
 
@@ -783,6 +1054,129 @@ int fhip_few_conv_wgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy, 
   return 0;
 }
 
+static int cf_allow_lds(fhip_ctx *ctx, const void *kernel, FhipOncePerDevice &configured) {
+  if (configured.done(ctx->device))
+    return 0;
+  FHIP_HIP_CHECK(ctx, hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kCfDgradLds));
+  configured.mark(ctx->device);
+  return 0;
+}
+
+static int cf_dgrad_products(fhip_ctx *ctx, const fhip_conv_desc *d, CfArgs g, const void *dy, const void *w,
+                             void *dx, bool *handled) {
+  const int rs = g.R * g.S;
+  if (rs > 48)
+    return 0;
+  // (three tiles of pairs at most)
+  const int most = 48 / rs < g.C ? 48 / rs : g.C, passes = (g.C + most - 1) / most;
+  g.cb = (g.C + passes - 1) / passes;
+  const int pt = (g.cb * rs + 15) / 16;
+  // The filter in LDS: f32 [channel][pair], the four rows of a product in different banks;
+  // 16 bits [pair][channel], whole 16-byte runs.  Tiles read behind the last pair.
+  const bool wide = d->x.dtype == FHIP_FLOAT;
+  const int seen = (passes - 1) * g.cb * rs + pt * 16;
+  const int64_t kpad = wide ? (g.K + 3) / 4 * 4 : (g.K + 31) / 32 * 32;
+  g.wpitch = wide ? (seen + 15) / 32 * 32 + 16 : (int32_t)kpad + 8;
+  const int64_t filter = (wide ? kpad * g.wpitch : (int64_t)seen * g.wpitch / 2 + 1) + 16;
+  if (kpad * g.J >= (1 << 16))
+    return 0;
+  g.gat = (int32_t)((filter + 3) / 4 * 4);
+  g.q_magic = cf_magic(g.J);
+  g.packed = (g.S == 1 || g.ws[3] == 1) && (g.R == 1 || g.ws[2] == g.S) && (g.C == 1 || g.ws[1] == rs) && g.ws[0] == g.J;
+  const int64_t tiles_w = (g.W + 127) / 128;
+  g.wt = (int32_t)((g.W + tiles_w - 1) / tiles_w);
+  g.w_magic = cf_magic((g.wt + 3) / 4), g.quads_magic = cf_magic((g.Q + 3) / 4);
+  const int64_t nq = tiles_w == 1 || g.wt + g.S - 1 > g.Q ? g.Q : g.wt + g.S - 1;
+  const int beside = g.S - 1 > g.pad_w ? g.S - 1 - g.pad_w : 0; // columns that taps reach beside DY
+  const int64_t row = (nq + beside + 3) / 4 * 4;
+  g.gpitch = (int32_t)row;
+  auto rows_dy = [&](int64_t band) { return band + g.R - 1 < g.P ? band + g.R - 1 : (int64_t)g.P; };
+  auto units_of = [&](int64_t band) { return (rows_dy(band) * ((nq + 3) / 4) + 15) / 16; };
+  // Rows of DX per band: G in `lds` bytes, a wavefront's 64 pixels once.
+  auto band_of = [&](int64_t lds, int64_t waves) {
+    int64_t fit = (lds / 4 - g.gat - 16) / (g.cb * rs * row), unit = waves * 16 / ((nq + 3) / 4);
+    fit = fit < unit ? fit : unit;
+    const int64_t band = fit >= g.P ? (int64_t)g.H : fit - (g.R - 1);
+    return band < g.H ? band : (int64_t)g.H;
+  };
+  int64_t band = band_of(kCfDgradLds / 2, 8), alone = band_of(kCfDgradLds, 16);
+  // (rows read per row written: f32 N128 4 -> 64, 64 x 64, 5 x 5 in half of LDS 304 us, in all of it
+  // 174; N113 3 -> 16, 47 x 47, 3 x 3, where the difference is a tenth, 15.6 and 17.2)
+  auto halo = [&](int64_t b) { return b < 1 ? 1e9 : b == g.H ? 1.0 : (double)(b + g.R - 1) / (double)b; };
+  if (halo(alone) < 0.75 * halo(band))
+    band = alone;
+  if (band < 1)
+    return 0;
+  band = band * g.wt < (1 << 16) ? band : ((1 << 16) - 1) / g.wt;
+  // Lower bands where that spreads the pixels better: rounds of workgroups over the compute units,
+  // each a start and its wavefronts' products.  (f32 N100 3 -> 32, 32 x 32, 3 x 3: 300 workgroups
+  // 13.5 us, 400 11.1; bf16 N22 1 -> 64, 54 x 54, 5 x 5: 308 8.9, 242 6.9.)
+  const int64_t cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+  double best = 1e30;
+  for (int64_t t = (g.H + band - 1) / band; t <= g.H; ++t) {
+    const int64_t b = (g.H + t - 1) / t, wgs = (int64_t)g.N * ((g.H + b - 1) / b) * tiles_w;
+    const double cost = (double)((wgs + cus - 1) / cus) * ((double)units_of(b) + 2.0);
+    if (cost < best)
+      best = cost, g.band = (int32_t)b;
+    if (wgs > 4 * cus || b < g.R)
+      break;
+  }
+  g.tiles = (g.H + g.band - 1) / g.band;
+  const int64_t blocks = (int64_t)g.N * g.tiles;
+  if (blocks >= (1ll << 23))
+    return 0;
+  const size_t lds = (size_t)(g.gat + 16 + rows_dy(g.band) * row * g.cb * rs) * 4;
+  const int64_t units = units_of(g.band);
+  const int waves = (int)(units < 2 ? 2 : units < 16 ? units : 16);
+  const unsigned parts = passes > 1 && blocks * tiles_w * passes <= 2 * cus ? (unsigned)passes : 1u;
+  // Passes on one workgroup pay where the taps' multiplications of conv_few_dgrad_kernel are many:
+  // 16-bit tensors from 32 output channels on (us there / here, 5 x 5: bf16 N64 4 -> 64, 36 x 36 36.9 /
+  // 16.6, 4 -> 32 21.8 / 14.9, 4 -> 16 13.3 / 15.5), f32 where the pixels are few besides (N64 3 -> 32,
+  // 20 x 20 17.2 / 13.5, 36 x 36 18.1 / 18.1, N120, 50 x 50 46.7 / 53.2).
+  if (passes > 1 && parts == 1 &&
+      (g.K < 32 || (wide && (int64_t)g.N * g.H * g.W > 110 * cus)))
+    return 0;
+  *handled = true;
+  fhip_note_kernel(ctx, "conv_few dgrad products channels=%d", g.C);
+  int status = 0;
+  cf_by_type(d->x.dtype, [&](auto t) {
+    typedef decltype(t) T;
+    auto with = [&](auto ss, auto tiles, auto block) {
+      constexpr int S = decltype(ss)::value, PT = decltype(tiles)::value, KB = decltype(block)::value;
+      constexpr bool held = sizeof(T) == 2 || PT < 3; // (see channels)
+      auto kernel = conv_few_dgrad_products_kernel<T, S, PT, held ? KB : 32>;
+      static FhipOncePerDevice configured;
+      status = cf_allow_lds(ctx, reinterpret_cast<const void *>(kernel), configured);
+      if (status == 0)
+        hipLaunchKernelGGL(kernel, dim3((unsigned)blocks, (unsigned)tiles_w, parts), dim3(waves * 64), lds, ctx->stream, g,
+                           (const T *)dy, (const T *)w, (T *)dx);
+    };
+    auto pairs = [&](auto ss, auto block) {
+      if (pt == 1)
+        with(ss, std::integral_constant<int, 1>{}, block);
+      else if (pt == 2)
+        with(ss, std::integral_constant<int, 2>{}, block);
+      else
+        with(ss, std::integral_constant<int, 3>{}, block);
+    };
+    auto channels = [&](auto ss) {
+      // (128 registers: f32 channels beside three tiles of pairs in two blocks)
+      if (g.K <= 32 || (wide && pt == 3))
+        pairs(ss, std::integral_constant<int, 32>{});
+      else
+        pairs(ss, std::integral_constant<int, 64>{});
+    };
+    if (g.S == 3)
+      channels(std::integral_constant<int, 3>{});
+    else
+      channels(std::integral_constant<int, 5>{});
+  });
+  if (status != 0)
+    return status;
+  FHIP_HIP_CHECK(ctx, hipGetLastError());
+  return 0;
+}
+
 int fhip_few_conv_dgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy, const void *w,
                         void *dx, bool *handled) {
   *handled = false;
@@ -792,6 +1186,9 @@ int fhip_few_conv_dgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy, 
   if (g.C > 4 || (g.S != 3 && g.S != 5) || g.str_h != 1 || g.str_w != 1 || g.dil_h != 1 ||
       g.dil_w != 1 || (g.Q > 1 && g.ys[3] != 1) || g.W > 256)
     return 0;
+  const int status = cf_dgrad_products(ctx, d, g, dy, w, dx, handled);
+  if (status != 0 || *handled)
+    return status;
   g.quads = (g.W + 3) / 4;
   // (a multiple of the rows per lane, of equal height)
   const int pairs = (g.H + kCfRows - 1) / kCfRows, most = 64 / g.quads;

@@ -108,3 +108,47 @@ def test_few_tiles_take_fewer_channels_each(ctx, n, forward, gradient):
     dw = run_conv_wgrad(ctx, dy, x, [64, 3, 3, 3], *geom, capi.FLOAT, False, tuned=None)
     assert ctx.last_kernel() == f"conv_few wgrad tiles={gradient}x2", ctx.last_kernel()
     assert_close(dw.logical(), oracle.conv_wgrad(dy.logical(), x.logical(), [64, 3, 3, 3], *geom), capi.FLOAT)
+
+
+@pytest.mark.parametrize("dtype", [capi.FLOAT, capi.BFLOAT16, capi.HALF])
+@pytest.mark.parametrize("x,w,pad,dense,kind", [
+    ([3, 3, 32, 32], [32, 3, 3, 3], [0, 0], True, "products"),
+    ([2, 2, 21, 30], [32, 2, 3, 3], [1, 1], True, "products"),    # rows of 30: the last quad reaches behind
+    ([1, 1, 6, 4], [9, 1, 3, 3], [0, 0], True, "products"),       # rows of two, odd channels
+    ([2, 4, 40, 9], [37, 4, 3, 3], [2, 2], True, "products"),     # three tiles of pairs, channels in two blocks
+    ([2, 3, 20, 24], [65, 3, 5, 5], [2, 2], True, "products"),    # passes side by side, 65 channels
+    ([300, 2, 12, 12], [40, 2, 5, 5], [2, 2], True, None),        # passes one after the other (16 bits)
+    ([300, 3, 12, 12], [16, 3, 5, 5], [2, 2], True, "channels"),  # few output channels: vector instructions
+    ([1, 1, 30, 200], [24, 1, 5, 5], [0, 1], True, "products"),   # bands cut in columns
+    ([2, 1, 3, 250], [8, 1, 2, 3], [3, 3], True, "products"),     # DY beside the image
+    ([2, 3, 20, 18], [16, 3, 3, 3], [1, 1], False, "products"),   # rows of DY with gaps
+])
+def test_data_gradient_products_first(ctx, x, w, pad, dense, kind, dtype):
+    geom = (pad, [1, 1], [1, 1])
+    yd = oracle.conv_output_dims(x, w, *geom)
+    wt = HT.from_logical(rand(54, 0, w, std=0.2), dtype)
+    if dense:
+        dy = HT.from_logical(rand(54, 1, yd), dtype)
+    else:
+        pitch = yd[3] + 3
+        st = [yd[1] * yd[2] * pitch, yd[2] * pitch, pitch, 1]
+        dy = HT.from_logical(rand(54, 1, yd), dtype, strides=st)
+    dx = run_conv_dgrad(ctx, dy, wt, x, *geom, dtype, False, tuned=None)
+    if kind is None:
+        kind = "channels" if dtype == capi.FLOAT else "products"
+    assert ctx.last_kernel().startswith(f"conv_few dgrad {kind}"), ctx.last_kernel()
+    assert_close(dx.logical(), oracle.conv_dgrad(dy.logical(), wt.logical(), x, *geom), dtype, f"{x} {w}")
+
+
+def test_data_gradient_keeps_infinities_where_they_fall(ctx):
+    # one infinite value of DY reaches the pixels under its filter and no others
+    geom = ([1, 1], [1, 1], [1, 1])
+    g = rand(55, 0, [2, 12, 10, 11])
+    g[0, 11, 4, 10] = np.inf  # last column, last channel
+    wt = HT.from_logical(np.abs(rand(55, 1, [12, 3, 3, 3])) + 0.1, capi.FLOAT)
+    dx = run_conv_dgrad(ctx, HT.from_logical(g, capi.FLOAT), wt, [2, 3, 10, 11], *geom, capi.FLOAT, False,
+                        tuned=None).logical()
+    assert ctx.last_kernel().startswith("conv_few dgrad products"), ctx.last_kernel()
+    hit = np.zeros(dx.shape, bool)
+    hit[0, :, 3:6, 9:11] = True
+    assert np.isposinf(dx[hit]).all() and np.isfinite(dx[~hit]).all()
