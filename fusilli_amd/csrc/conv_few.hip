@@ -21,7 +21,7 @@
 //     added through LDS.
 //
 // One training step (us):
-//   N100 3 -> 32, 32 x 32, 3 x 3, f32: fprop 26.2 -> 15.5, dgrad 60.5 -> 15.0 -> 11.1, wgrad 46.1 -> 13.0
+//   N100 3 -> 32, 32 x 32, 3 x 3, f32: fprop 26.2 -> 13.6 -> 12.0, dgrad 60.5 -> 15.0 -> 11.1, wgrad 46.1 -> 13.0
 //   N122 1 -> 64, 57 x 57, 5 x 5, bf16: 136 -> 52.6, 701 -> 78.6 -> 33.0, 495 -> 45.7
 //
 // Reference semantics: aten.convolution / aten.convolution_backward
@@ -64,14 +64,15 @@ __device__ __forceinline__ int cf_div(int e, uint32_t magic) {
   return (int)__umulhi((uint32_t)e, magic) + (magic == 0 ? e : 0);
 }
 
-// X rows [row0, row0 + rows) of all channels of an image, zeros outside it, as f32.
-template <typename T>
-__device__ __forceinline__ void cf_stage_x(const CfArgs &g, const T *x, int row0, int rows,
-                                           float *xl) {
-  constexpr int kBatch = 8; // loads in flight per thread
-  const int total = g.C * g.xrows * g.lw;
-  for (int e0 = threadIdx.x; e0 < total; e0 += kBatch * kCfThreads) {
-    float v[kBatch];
+// X rows [row0, row0 + rows) of all channels of an image, zeros outside it, as f32, in batches:
+// request() issues a batch's loads, put() waits for them.
+template <typename T> struct CfStageX {
+  static constexpr int kBatch = 8; // loads in flight per thread
+  T v[kBatch];
+  uint32_t live;
+  __device__ __forceinline__ void request(const CfArgs &g, const T *x, int row0, int rows, int e0) {
+    const int total = g.C * g.xrows * g.lw;
+    live = 0;
 #pragma unroll
     for (int i = 0; i < kBatch; ++i) {
       const int e = e0 + i * kCfThreads;
@@ -80,15 +81,26 @@ __device__ __forceinline__ void cf_stage_x(const CfArgs &g, const T *x, int row0
       const int h = row0 + r, w = col - g.pad_w;
       const bool in = e < total && r < rows && (unsigned)h < (unsigned)g.H && (unsigned)w < (unsigned)g.W;
       // (the load is issued either way: a branch would wait for every value)
-      const float t = (float)x[in ? c * (int)g.xs[1] + h * (int)g.xs[2] + w * (int)g.xs[3] : 0];
-      v[i] = in ? t : 0.f;
+      v[i] = x[in ? c * (int)g.xs[1] + h * (int)g.xs[2] + w * (int)g.xs[3] : 0];
+      live |= (uint32_t)in << i;
     }
+  }
+  __device__ __forceinline__ void put(const CfArgs &g, int e0, float *xl) const {
+    const int total = g.C * g.xrows * g.lw;
 #pragma unroll
     for (int i = 0; i < kBatch; ++i)
       if (e0 + i * kCfThreads < total)
-        xl[e0 + i * kCfThreads] = v[i];
+        xl[e0 + i * kCfThreads] = (live >> i) & 1 ? (float)v[i] : 0.f;
   }
-}
+  // all batches from `e0` on
+  static __device__ __forceinline__ void stage(const CfArgs &g, const T *x, int row0, int rows, int e0, float *xl) {
+    for (; e0 < g.C * g.xrows * g.lw; e0 += kBatch * kCfThreads) {
+      CfStageX b;
+      b.request(g, x, row0, rows, e0);
+      b.put(g, e0, xl);
+    }
+  }
+};
 
 // where pair j = (channel, tap) lies in the staged X / in the filter
 __device__ __forceinline__ int cf_pair(const CfArgs &g, int j, int *filter) {
@@ -99,7 +111,8 @@ __device__ __forceinline__ int cf_pair(const CfArgs &g, int j, int *filter) {
 }
 
 // ---- forward -------------------------------------------------------------------
-template <typename O>
+// 16 values, four at a time TS elements apart
+template <typename O, int TS>
 __device__ __forceinline__ void cf_store16(void *out, int64_t at, const float (&v)[16]) {
   constexpr int N = 16 / sizeof(O);
   typedef O vec __attribute__((ext_vector_type(N), aligned(sizeof(O))));
@@ -109,7 +122,7 @@ __device__ __forceinline__ void cf_store16(void *out, int64_t at, const float (&
 #pragma unroll
     for (int k = 0; k < N; ++k)
       t[k] = (O)v[i + k];
-    *(vec *)((O *)out + at + i) = t;
+    *(vec *)((O *)out + at + (i >> 2) * TS) = t;
   }
 }
 
@@ -130,32 +143,35 @@ __global__ __launch_bounds__(kCfThreads) void conv_few_fprop_kernel(CfArgs g, co
   const int pq = g.P * g.Q;
   const int t1 = t0 + kCfThreads < pq ? t0 + kCfThreads : pq;
   const int p0 = t0 / g.Q, p1 = (t1 - 1) / g.Q;
-  // Everything a workgroup reads is requested before the first wait: the filter, the fused
-  // operations' values per channel, X (one after another: 0.2 to 0.5 us more).
+  // Everything a workgroup reads is requested before the first wait: X, the filter, then the
+  // fused operations' values per channel.  Nothing looks at a loaded value before that, not
+  // even a select (f32 N22 1 -> 16, 28 x 28, 3 x 3 7.3 -> 6.8 us, bf16 N71 1 -> 32, 17 x 17, 5 x 5 9.1 -> 8.3).
+  const int row0 = p0 * g.str_h - g.pad_h, xrows = (p1 - p0) * g.str_h + (g.R - 1) * g.dil_h + 1;
+  CfStageX<T> xv0;
+  xv0.request(g, x + n * g.xs[0], row0, xrows, tid);
   constexpr int kBatch = 8;
   const int kk = tid % K16, jt = tid / K16; // this thread's channel, its first pair
   const bool k_in = k0 + kk < g.K;
-  auto weights = [&](int j0, float (&v)[kBatch]) {
+  auto weights = [&](int j0, T (&v)[kBatch]) {
 #pragma unroll
     for (int i = 0; i < kBatch; ++i) {
       const int j = j0 + i * (kCfThreads / K16);
       const bool in = j < g.J && k_in;
       int f;
       cf_pair(g, in ? j : 0, &f);
-      // (the load is issued either way: a branch would wait for every value)
-      const float t = (float)w[in ? (k0 + kk) * g.ws[0] + f : 0];
-      v[i] = in ? t : 0.f;
+      v[i] = w[in ? (k0 + kk) * g.ws[0] + f : 0];
     }
   };
-  auto put_weights = [&](int j0, const float (&v)[kBatch]) {
+  auto put_weights = [&](int j0, const T (&v)[kBatch]) {
 #pragma unroll
     for (int i = 0; i < kBatch; ++i) {
       const int j = j0 + i * (kCfThreads / K16);
       if (j < j4)
-        wl[j * KP + kk] = v[i];
+        wl[j * KP + kk] = j < g.J && k_in ? (float)v[i] : 0.f;
     }
   };
-  float wv0[kBatch], op[FHIP_MAX_EPILOGUE];
+  T wv0[kBatch];
+  float op[FHIP_MAX_EPILOGUE];
   weights(jt, wv0);
 #pragma unroll
   for (int e = 0; e < FHIP_MAX_EPILOGUE; ++e) {
@@ -172,11 +188,11 @@ __global__ __launch_bounds__(kCfThreads) void conv_few_fprop_kernel(CfArgs g, co
     int f;
     tab[j] = j < g.J ? cf_pair(g, j, &f) : 0;
   }
-  cf_stage_x(g, x + n * g.xs[0], p0 * g.str_h - g.pad_h,
-             (p1 - p0) * g.str_h + (g.R - 1) * g.dil_h + 1, xl);
+  xv0.put(g, tid, xl);
+  CfStageX<T>::stage(g, x + n * g.xs[0], row0, xrows, tid + CfStageX<T>::kBatch * kCfThreads, xl);
   put_weights(jt, wv0);
   for (int j0 = jt + kBatch * (kCfThreads / K16); j0 < j4; j0 += kBatch * (kCfThreads / K16)) {
-    float v[kBatch];
+    T v[kBatch];
     weights(j0, v);
     put_weights(j0, v);
   }
@@ -188,11 +204,16 @@ __global__ __launch_bounds__(kCfThreads) void conv_few_fprop_kernel(CfArgs g, co
   const int first = t0 + wave * 64;
   if (first >= t1)
     return;
+  // Pixels of the four tiles: a lane ends up with 16 in a row where OUT has 16-bit elements
+  // (two whole stores), else with runs of 4 that its neighbours continue (64 bytes a channel
+  // and store, not 16 bytes each on 32 cache lines: N67 4 -> 32, 62 x 62, 3 x 3 27.2 -> 23.0 us, N60 1 -> 64, 40 x 40
+  // 15.8 -> 13.1).
+  const int ts = g.o_dt == FHIP_FLOAT ? 16 : 4, gs = 20 - ts;
   int base[4];
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
     const int m = l & 15;
-    int px = first + (m >> 2) * 16 + t * 4 + (m & 3);
+    int px = first + (m >> 2) * gs + t * ts + (m & 3);
     px = px < t1 ? px : t1 - 1;
     const int p = px / g.Q, q = px - p * g.Q;
     base[t] = (p - p0) * g.str_h * g.lw + q * g.str_w;
@@ -222,8 +243,8 @@ __global__ __launch_bounds__(kCfThreads) void conv_few_fprop_kernel(CfArgs g, co
       for (int u = 0; u < KT; ++u)
         acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[t], wv[u], acc[t][u], 0, 0, 0);
   }
-  // value r of tile t: pixel first + (l / 16) * 16 + t * 4 + r of channel l % 16
-  const int px = first + (l >> 4) * 16;
+  // value r of tile t: pixel first + (l / 16) * gs + t * ts + r of channel l % 16
+  const int px = first + (l >> 4) * gs;
   if (px >= t1)
     return;
   // (one copy of the chain for all KT tiles: the next tile's sums move to the front)
@@ -258,13 +279,28 @@ __global__ __launch_bounds__(kCfThreads) void conv_few_fprop_kernel(CfArgs g, co
       fhip_round_fast_vec<16>(o.result_dtype, v);
     }
     const int64_t at = n * g.ys[0] + k * g.ys[1] + px;
-    if (px + 16 <= t1) {
+    if (px + 3 * ts + 4 <= t1) {
       if (g.o_dt == FHIP_FLOAT)
-        cf_store16<float>(out, at, v);
+        cf_store16<float, 16>(out, at, v);
       else if (g.o_dt == FHIP_BFLOAT16)
-        cf_store16<__bf16>(out, at, v);
+        cf_store16<__bf16, 4>(out, at, v);
       else
-        cf_store16<_Float16>(out, at, v);
+        cf_store16<_Float16, 4>(out, at, v);
+    } else if (g.o_dt == FHIP_FLOAT) {
+      typedef float Four __attribute__((ext_vector_type(4), aligned(4)));
+#pragma unroll
+      for (int i = 0; i < 16; i += 4) {
+        float *to = (float *)out + at + 4 * i;
+        const int left = t1 - (px + 4 * i);
+        if (left >= 4) {
+          *(Four *)to = Four{v[i], v[i + 1], v[i + 2], v[i + 3]};
+        } else {
+#pragma unroll
+          for (int j = 0; j < 3; ++j)
+            if (j < left)
+              to[j] = v[i + j];
+        }
+      }
     } else {
 #pragma unroll
       for (int i = 0; i < 16; ++i)
@@ -341,8 +377,8 @@ __global__ __launch_bounds__(kCfThreads) void conv_few_wgrad_kernel(CfArgs g, co
     const int px0 = wave * 16 + (l >> 4) * 4;
     cf_load_dy<T, KT>(src, px0, np, a[0]);
     __syncthreads();
-    cf_stage_x(g, x + n * g.xs[0], p0 * g.str_h - g.pad_h,
-               (rows - 1) * g.str_h + (g.R - 1) * g.dil_h + 1, xl);
+    CfStageX<T>::stage(g, x + n * g.xs[0], p0 * g.str_h - g.pad_h,
+                       (rows - 1) * g.str_h + (g.R - 1) * g.dil_h + 1, tid, xl);
     __syncthreads();
     auto spend = [&](const float (&b)[KT][4], int px) {
       const int4 at = *(const int4 *)(pixtab + px);
