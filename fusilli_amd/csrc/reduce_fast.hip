@@ -239,7 +239,7 @@ __global__ __launch_bounds__(256) void reduce_rows_kernel(ReduceRowsArgs g) {
 // slices on workgroups of their own (partial[slice][k], f32), which a second kernel combines in slice
 // order: no atomics.  Bound by reading X once.  N32 56 x 56 K128 bf16 in
 // channels-last (25.7 MB): 104 us on the strided kernel (one workgroup per
-// channel and slice reading one 2-byte element per pixel line) -> 8.4 us
+// channel and slice reading one 2-byte element per pixel line) -> 8.4 -> 7.0 us
 // (both launches); N100 K32 30 x 30 f32 channels-first (11.5 MB) 31 -> 10.2 us (5.5 +
 // 4.6).
 struct ReduceMidArgs {
@@ -315,7 +315,9 @@ __device__ __forceinline__ void rf_values(typename RfVec<T, VEC>::type v, float 
 }
 
 // r2 == 1: TX threads side by side on the columns (VEC each), 256 / TX rows at
-// a time, four rows of loads in flight per thread.
+// a time, for sums eight rows of loads in flight per thread: a workgroup per compute unit is
+// bound by their latency (N32 56 x 56 K128 bf16, four rows 8.2 us, eight 6.9; more slices
+// cost the combining launch what they save here: 512 of them 1.3 us more in all).
 template <typename T, int MAP, int COMB, int VEC>
 __global__ __launch_bounds__(256) void reduce_cols_kernel(ReduceMidArgs g, int tx_log2) {
   typedef typename RfVec<T, VEC>::type V;
@@ -351,6 +353,15 @@ __global__ __launch_bounds__(256) void reduce_cols_kernel(ReduceMidArgs g, int t
                                     rf_comb_nan<COMB>(rf_map<MAP>(f[2][i]), rf_map<MAP>(f[3][i]))));
   };
   int64_t r = first + row0;
+  if constexpr (COMB == C_ADD)
+    for (; r + 7 * ty < last; r += 8 * ty) {
+      V v[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        v[i] = src[(r + i * ty) * cols];
+      add4(v[0], v[1], v[2], v[3]);
+      add4(v[4], v[5], v[6], v[7]);
+    }
   for (; r + 3 * ty < last; r += 4 * ty) {
     const V v0 = src[r * cols], v1 = src[(r + ty) * cols];
     const V v2 = src[(r + 2 * ty) * cols], v3 = src[(r + 3 * ty) * cols];
