@@ -250,15 +250,16 @@ __device__ __forceinline__ void tile_store(const DirectArgs &g, int64_t batch, i
   if constexpr (std::is_same<Acc, int>::value) {
     typedef int loose __attribute__((ext_vector_type(4), aligned(4)));
     GEMM_AS1 int32_t *out = (GEMM_AS1 int32_t *)g.out + at;
-    if (live == V && g.o_sn == 1) {
 #pragma unroll
-      for (int i = 0; i < V; i += 4)
+    for (int i = 0; i < V; i += 4) {
+      if (live >= i + 4 && g.o_sn == 1) {
         *(GEMM_AS1 loose *)(out + i) = loose{acc[i], acc[i + 1], acc[i + 2], acc[i + 3]};
-    } else {
+      } else {
 #pragma unroll
-      for (int i = 0; i < V; ++i)
-        if (i < live)
-          out[i * g.o_sn] = acc[i];
+        for (int k = i; k < i + 4; ++k)
+          if (k < live)
+            out[k * g.o_sn] = acc[k];
+      }
     }
   } else {
     float v[V];
@@ -293,40 +294,46 @@ __device__ __forceinline__ void tile_store(const DirectArgs &g, int64_t batch, i
         cols[i] = n + (i < live ? i : 0);
       fhip_apply_epilogue_many<float, V>(g.epi, v, coord, 2, cols);
     }
-    const bool whole = live == V && g.o_sn == 1;
+    // (whole runs of 16 bytes, or of the V columns, single values where the last one ends)
     if (g.o_dt == FHIP_FLOAT) {
       typedef float loose __attribute__((ext_vector_type(4), aligned(4)));
       GEMM_AS1 float *out = (GEMM_AS1 float *)g.out + at;
 #pragma unroll
-      for (int i = 0; i < V; i += 4)
-        if (whole)
+      for (int i = 0; i < V; i += 4) {
+        if (live >= i + 4 && g.o_sn == 1) {
           *(GEMM_AS1 loose *)(out + i) = loose{v[i], v[i + 1], v[i + 2], v[i + 3]};
+        } else {
 #pragma unroll
-      for (int i = 0; i < V; ++i)
-        if (!whole && i < live)
-          out[i * g.o_sn] = v[i];
+          for (int k = i; k < i + 4; ++k)
+            if (k < live)
+              out[k * g.o_sn] = v[k];
+        }
+      }
     } else {
-      typedef uint16_t loose __attribute__((ext_vector_type(V), aligned(2)));
+      constexpr int H = V < 8 ? V : 8;
+      typedef uint16_t loose __attribute__((ext_vector_type(H), aligned(2)));
       GEMM_AS1 uint16_t *out = (GEMM_AS1 uint16_t *)g.out + at;
-      loose h;
 #pragma unroll
-      for (int i = 0; i < V; ++i)
-        h[i] = g.o_dt == FHIP_BFLOAT16 ? __builtin_bit_cast(uint16_t, (__bf16)v[i])
-                                       : __builtin_bit_cast(uint16_t, (_Float16)v[i]);
-      if (whole) {
-        *(GEMM_AS1 loose *)out = h;
-      } else {
+      for (int i = 0; i < V; i += H) {
+        loose h;
 #pragma unroll
-        for (int i = 0; i < V; ++i)
-          if (i < live)
-            out[i * g.o_sn] = h[i];
+        for (int k = 0; k < H; ++k)
+          h[k] = g.o_dt == FHIP_BFLOAT16 ? __builtin_bit_cast(uint16_t, (__bf16)v[i + k])
+                                         : __builtin_bit_cast(uint16_t, (_Float16)v[i + k]);
+        if (live >= i + H && g.o_sn == 1) {
+          *(GEMM_AS1 loose *)(out + i) = h;
+        } else {
+#pragma unroll
+          for (int k = 0; k < H; ++k)
+            if (i + k < live)
+              out[(i + k) * g.o_sn] = h[k];
+        }
       }
     }
   }
 }
 
-// Adds a tile's SUMS shares of K in LDS, finishes and stores it, or stores the plain sums of
-// a split product.
+// Adds a tile's SUMS shares of K in LDS, finishes and stores it.
 template <typename Acc, int V, int BM, int BN, int SUMS, int PITCH, int SUM, int THREADS, bool PLAIN, class Row>
 __device__ __forceinline__ void tile_finish(const DirectArgs &g, uint32_t lds, uint32_t id, int64_t batch, int m0, int n0,
                                             const TileColumns<V> &columns, const Row &at_row) {
@@ -345,15 +352,26 @@ __device__ __forceinline__ void tile_finish(const DirectArgs &g, uint32_t lds, u
         x += p[h * (SUM / 16)];
       v[q] = x.x, v[q + 1] = x.y, v[q + 2] = x.z, v[q + 3] = x.w;
     }
-    if (g.partial) {
-      GEMM_AS1 Acc4 *to = (GEMM_AS1 Acc4 *)g.partial +
-                          ((((int64_t)blockIdx.y * gridDim.z + batch) * gridDim.x + id) * (BM * BN) + row * BN + col) / 4;
+    tile_store<Acc, V, PLAIN>(g, batch, m0 + row, at_row(m0 + row), n0 + col, v, &columns);
+  }
+}
+
+// The plain sums of a split product's tile: 16 bytes a lane, side by side (in runs of eight columns
+// f16 605 x 296 x 3456 in five parts 10.8 us, so 10.4; of sixteen 11.3).
+template <typename Acc, int BM, int BN, int SUMS, int PITCH, int SUM, int THREADS>
+__device__ __forceinline__ void tile_part(const DirectArgs &g, uint32_t lds, uint32_t id, int64_t batch) {
+  typedef Acc Acc4 __attribute__((ext_vector_type(4)));
+  GEMM_AS1 Acc4 *to = (GEMM_AS1 Acc4 *)g.partial +
+                      (((int64_t)blockIdx.y * gridDim.z + batch) * gridDim.x + id) * (BM * BN / 4);
+#pragma unroll 4
+  for (int e = threadIdx.x; e < BM * BN / 4; e += THREADS) {
+    const GEMM_AS3 Acc4 *p =
+        (const GEMM_AS3 Acc4 *)(uintptr_t)(lds + (uint32_t)((e / (BN / 4) * PITCH + e % (BN / 4) * 4) * 4));
+    Acc4 x = *p;
 #pragma unroll
-      for (int q = 0; q < V; q += 4)
-        to[q / 4] = Acc4{v[q], v[q + 1], v[q + 2], v[q + 3]};
-    } else {
-      tile_store<Acc, V, PLAIN>(g, batch, m0 + row, at_row(m0 + row), n0 + col, v, &columns);
-    }
+    for (int h = 1; h < SUMS; ++h)
+      x += p[h * (SUM / 16)];
+    to[e] = x;
   }
 }
 
@@ -373,7 +391,16 @@ template <int KIND, int MT, int NT, int TEAMS_, bool SHORT = false> struct TileS
   static constexpr int kSum = BM * kPitch * 4;      // the accumulators of wavefronts with one share of K
   static constexpr int kSums = WK * TEAMS;
   static constexpr int kLds = TEAMS * 2 * kStage > kSums * kSum ? TEAMS * 2 * kStage : kSums * kSum;
-  static constexpr int V = BM * BN / (256 * TEAMS) >= 8 ? 8 : 4; // columns that a thread finishes
+  // Columns of a row that a thread finishes at once: the chain's loads and branches take a
+  // wavefront on its own 0.8 us a run, 0.15 more a column (bias and GELU on 64 x 64 tiles of four
+  // wavefronts: four runs of four 5.4 us, two of eight 3.9), so one run of sixteen where there are
+  // as many: bf16 3050 x 512 x 384 11.1 -> 10.2 us, fp8 1536 x 2560 x 6192 41.1 -> 39.2.
+  // Whole numbers have no chain, and 16 of them are 64 bytes a lane: i8 896 x 1792 x 1408 on 128 x 64
+  // tiles 10.4 us, with eight 9.2, with four 9.35; 128 x 7552 x 1280 on 64 x 64 ones with eight 8.05, with four 7.75.
+  static constexpr int V = KIND == GK_I8 ? (BM * BN / (256 * TEAMS) >= 32 ? 8 : 4)
+                           : BM * BN / (256 * TEAMS) >= 16 ? 16
+                           : BM * BN / (256 * TEAMS) >= 8  ? 8
+                                                           : 4;
 };
 
 // The share of K of a team: its whole slices, and how many the longest team of the workgroup
@@ -563,6 +590,10 @@ __device__ __forceinline__ void tile_run(const DirectArgs &g, uint32_t smem, con
                (l & 31)] = acc[i][j][r];
   }
   __syncthreads();
+  if (g.partial) {
+    tile_part<Acc, BM, BN, S::kSums, S::kPitch, S::kSum, 256 * TEAMS>(g, smem, id, batch);
+    return;
+  }
   tile_finish<Acc, S::V, BM, BN, S::kSums, S::kPitch, S::kSum, 256 * TEAMS, PLAIN>(g, smem, id, batch, m0, n0, columns,
                                                                                   at_row);
 }
@@ -602,6 +633,9 @@ __global__ __launch_bounds__(256) void gemm_tile_finish_kernel(DirectArgs g) {
   const int tile_m = BY_ROWS ? over : along, tile_n = BY_ROWS ? along : over;
   const int64_t batch = blockIdx.z;
   const int q = blockIdx.y * 256 + threadIdx.x;
+  TileColumns<4> columns;
+  if (g.lean && g.lean_op >= 0)
+    columns.request(g, tile_n * BN + q % (BN / 4) * 4);
   const GEMM_AS1 Acc4 *p = (const GEMM_AS1 Acc4 *)g.partial + (batch * gridDim.x + blockIdx.x) * (BM * BN / 4) + q;
   const int64_t stride = (int64_t)gridDim.z * gridDim.x * (BM * BN / 4);
   Acc4 x = p[0];
@@ -610,7 +644,8 @@ __global__ __launch_bounds__(256) void gemm_tile_finish_kernel(DirectArgs g) {
     x += p[s * stride];
   const Acc v[4] = {x.x, x.y, x.z, x.w};
   const int m = tile_m * BM + q / (BN / 4);
-  tile_store<Acc, 4>(g, batch, m, m < g.M ? batch * g.o_batch + (int64_t)m * g.o_sm : -1, tile_n * BN + q % (BN / 4) * 4, v);
+  tile_store<Acc, 4>(g, batch, m, m < g.M ? batch * g.o_batch + (int64_t)m * g.o_sm : -1, tile_n * BN + q % (BN / 4) * 4, v,
+                   &columns);
 }
 
 template <int KIND, bool A_KC, bool B_KC, int MT, int NT, int TEAMS, int U>

@@ -92,3 +92,28 @@ def test_fused_chains(ctx, dtype, m, n, k, batch):
             ([scale, add, mul], [bias, full], (0.25 * product + bias.logical()) * full.logical())):
         got, name, odt = run(ctx, a, b, ops, tensors)
         assert_close(got, ref, dtype, name)
+
+
+@pytest.mark.parametrize("dtype", [capi.BFLOAT16, capi.HALF])
+@pytest.mark.parametrize("m,n,k", [
+    (777, 1400, 1000),  # sixteen columns a thread, the last run of eight
+    (700, 1301, 1500),  # ... of five
+    (520, 520, 4001),   # split: four columns
+    (1299, 1930, 777),  # wide tiles
+])
+def test_chains_of_four(ctx, dtype, m, n, k):
+    # 2 - (swish_0.7(0.25 x) - bias): a scalar in front, a unary with a parameter, the accumulator
+    # as the second operand of a scalar and the first of a column's, roundings between
+    a, b = make_operand(85, 0, m, k, dtype, False), make_operand(85, 1, k, n, dtype, True)
+    bias = HT.from_logical(rand(85, 2, [1, n]), capi.FLOAT)
+    swish = capi.PointwiseParams.default()
+    swish.swish_beta = 0.7
+    ops = [capi.epilogue_op(capi.PW["MUL"], capi.FLOAT, scalar=0.25),
+           capi.epilogue_op(capi.PW["SWISH_FWD"], dtype, params=swish),
+           capi.epilogue_op(capi.PW["SUB"], capi.FLOAT, operand=bias.desc()),
+           capi.epilogue_op(capi.PW["SUB"], dtype, scalar=2.0, acc_is_in1=True)]
+    got, name, odt = run(ctx, a, b, ops, [bias])
+    assert name.startswith("gemm_mfma") and "waves=" in name, name
+    x = 0.25 * ref_matmul(a, b)
+    act = oracle.pointwise(capi.PW["SWISH_FWD"], [x], swish_beta=0.7)
+    assert_close(got, 2.0 - (act - bias.logical()), dtype, name)
