@@ -8,7 +8,7 @@
 //   * forward: X of 256 output pixels, padded with zeros, and the filter sit in LDS;
 //     pixels x output channels on 16 x 16 x 4 f32 MFMAs over the (channel, tap) pairs.
 //     A wavefront's four tiles interleave their pixels so that a lane ends up with 16
-//     consecutive pixels of one channel (64-byte stores);
+//     consecutive pixels of one channel (16-bit OUT) or four runs that its neighbours continue;
 //   * weight gradient: output channels x pairs on the same MFMAs over the pixels, DY
 //     straight from memory (four consecutive pixels per lane), X from LDS; a
 //     workgroup keeps its sums over many bands of rows, the workgroups' sums meet in

@@ -152,3 +152,15 @@ def test_data_gradient_keeps_infinities_where_they_fall(ctx):
     hit = np.zeros(dx.shape, bool)
     hit[0, :, 3:6, 9:11] = True
     assert np.isposinf(dx[hit]).all() and np.isfinite(dx[~hit]).all()
+
+
+@pytest.mark.parametrize("dtype,tiny", [(capi.HALF, 2.0 ** -22), (capi.BFLOAT16, 2.0 ** -130)])
+def test_data_gradient_keeps_subnormal_values(ctx, dtype, tiny):
+    # 16-bit DY below the normal range times whole numbers: exact sums of 12 * 9 values at most
+    dy = HT.from_logical(np.full([1, 12, 8, 8], tiny), dtype)
+    wt = HT.from_logical(np.full([12, 3, 3, 3], 64.0 if dtype == capi.HALF else 4.0), dtype)
+    dx = run_conv_dgrad(ctx, dy, wt, [1, 3, 8, 8], [1, 1], [1, 1], [1, 1], dtype, False, tuned=None).logical()
+    assert ctx.last_kernel().startswith("conv_few dgrad products"), ctx.last_kernel()
+    scale = 12 * wt.logical().flat[0] * tiny
+    assert np.array_equal(dx[0, 0, 1:-1, 1:-1], np.full([6, 6], 9 * scale)), dx[0, 0]
+    assert np.array_equal(dx[0, :, 0, 0], np.full([3], 4 * scale))
