@@ -364,13 +364,17 @@ __global__ __launch_bounds__(kRwThreads) void rownorm_walk_apply_kernel(RowWalkA
   }
   // sum (x - c0)^2 = sum (x - c)^2 + 2 d (sum x - n c) + n d^2 of a segment whose second
   // moment lies around c, d = c - c0 (RMSNorm: all zero)
-  const double n0 = (double)(g.seg < g.n.inner ? g.seg : g.n.inner);
-  const double c0 = g.n.is_layernorm ? (double)(float)(first / n0) : 0.;
-  const int64_t left = g.n.inner - (in ? threadIdx.x : 0) * g.seg;
-  const double n = (double)(left < g.seg ? left : g.seg);
-  const double c = g.n.is_layernorm ? (double)(float)(mine.x / n) : 0., d = c - c0;
-  double s = rw_wave_sum(in ? mine.x : 0.);
-  double q = rw_wave_sum(in ? mine.y + 2. * d * (mine.x - n * c) + n * d * d : 0.);
+  double c0 = 0., s = 0., q = in ? mine.y : 0.;
+  if (g.n.is_layernorm) { // (two divisions in 64 bits: RMSNorm passes them by)
+    const double n0 = (double)(g.seg < g.n.inner ? g.seg : g.n.inner);
+    c0 = (double)(float)(first / n0);
+    const int64_t left = g.n.inner - (in ? threadIdx.x : 0) * g.seg;
+    const double n = (double)(left < g.seg ? left : g.seg);
+    const double c = (double)(float)(mine.x / n), d = c - c0;
+    s = rw_wave_sum(in ? mine.x : 0.);
+    q = in ? mine.y + 2. * d * (mine.x - n * c) + n * d * d : 0.;
+  }
+  q = rw_wave_sum(q);
   if ((threadIdx.x & 63) == 0)
     lds[threadIdx.x >> 6] = rw_pair{s, q};
   __syncthreads();
@@ -412,14 +416,18 @@ __global__ __launch_bounds__(kRwThreads) void rownorm_walk_apply_kernel(RowWalkA
   }
 }
 
-template <typename T> void rw_launch_split(hipStream_t stream, const RowWalkArgs &g) {
+template <typename T> void rw_launch_split(hipStream_t stream, const RowWalkArgs &g, int64_t cus) {
   const dim3 grid((unsigned)g.splits, (unsigned)g.n.rows), wg(kRwThreads);
   auto go = [&](auto nv) {
     constexpr int NV = decltype(nv)::value;
     hipLaunchKernelGGL((rownorm_walk_sums_kernel<T, NV>), grid, wg, 0, stream, g);
     hipLaunchKernelGGL((rownorm_walk_apply_kernel<T, NV>), grid, wg, 0, stream, g);
   };
-  if (g.seg <= 2 * kRwThreads * RwVec<T>::kN)
+  // (RMSNorm needs one sum and has no bias to fetch ahead: there walked segments are 2 to 8 %
+  // faster, f16 28 x 229376 12.4 us against 13.0, f32 22 x 195584 14.1 / 14.7; so are those of
+  // LayerNorm beyond four workgroups per compute unit, which cover each other's waits: f16
+  // 12 x 400384 11.9 / 12.3, 28 x 229376 13.4 / 13.7, but 20 x 200704 10.5 / 10.3, 5 x 310272 8.0 / 7.9)
+  if (g.seg <= 2 * kRwThreads * RwVec<T>::kN && g.n.is_layernorm && g.n.rows * g.splits <= 4 * cus)
     go(std::integral_constant<int, 2>{});
   else
     go(std::integral_constant<int, 0>{});
@@ -480,7 +488,7 @@ int fhip_norm_walk(fhip_ctx *ctx, int dtype, const RowNormArgs &n, bool cut_pays
   }
   auto go = [&](auto t) {
     typedef decltype(t) T;
-    cut ? rw_launch_split<T>(ctx->stream, g) : rw_launch_rows<T>(ctx->stream, n, waves);
+    cut ? rw_launch_split<T>(ctx->stream, g, ctx->num_cus > 0 ? ctx->num_cus : 256) : rw_launch_rows<T>(ctx->stream, n, waves);
   };
   if (dtype == FHIP_BFLOAT16)
     go(__bf16{});
