@@ -384,7 +384,8 @@ def test_means_of_walked_rows_are_rounded_once(ctx, dtype, rows, cols):
     # the shortest and the longest rows that a workgroup could hold, a last segment of one
     # vector, more pairs than a thread each (segments longer than registers hold)
     (capi.BFLOAT16, 3, 65544), (capi.HALF, 2, 131072), (capi.BFLOAT16, 1, 16 * 4096 + 8),
-    (capi.FLOAT, 2, 49152), (capi.FLOAT, 1, 256 * 2048 + 4), (capi.HALF, 1, 256 * 4096 + 8)])
+    (capi.FLOAT, 2, 49152), (capi.FLOAT, 1, 256 * 2048 + 4), (capi.HALF, 1, 256 * 4096 + 8),
+    (capi.HALF, 40, 110600)])  # more segments than four per compute unit
 @pytest.mark.parametrize("kind", ["layernorm", "rmsnorm", "rmsnorm in place"])
 def test_norm_rows_in_segments_vs_64_bits(ctx, dtype, rows, cols, kind):
     # segments of unlike means, the largest far from the first element's
