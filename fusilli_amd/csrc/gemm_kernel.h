@@ -315,22 +315,33 @@ dma_setup(int group0, int64_t ld_bytes, int64_t row0, int64_t rows_total,
   }
 }
 
-// The same offsets for a slice that ends after `rest` bytes of K: loads of what lies
-// behind them (whole 16-byte chunks of a K-contiguous row, whole K-rows) read past
-// 2^31, where the caller's descriptor ends, and bring zeros.
-template <int ROWS, int ELEM, bool KCONTIG, int NW, int STEP, int J0, int J1>
-__device__ __forceinline__ void dma_cut(int group0, int rest,
-                                        const uint32_t (&off)[SliceGeom<ROWS, ELEM, KCONTIG, NW>::kLoads],
-                                        uint32_t (&cut)[SliceGeom<ROWS, ELEM, KCONTIG, NW>::kLoads]) {
+// A slice that ends after `rest` bytes of K (whole 16-byte chunks where the operand lies along
+// K).  dma_cut: the same offsets, but those behind the end repeat the row's last chunk, or the
+// last K-row, so that every load is a real one.  dma_blank: once they have landed, zeros over
+// what they brought (of both operands: 0 x infinity), by the lanes that requested it.
+template <int ROWS, int ELEM, bool KCONTIG, int NW>
+__device__ __forceinline__ int dma_k(int group) { // byte of K in the slice where this lane's load starts
   using G = SliceGeom<ROWS, ELEM, KCONTIG, NW>;
   const int l = threadIdx.x & 63;
+  return KCONTIG ? ((l & 7) ^ kc_swz(group * 8 + (l >> 3))) * 16 : (group * G::kRowsPerLoad + l / G::kCPR) * ELEM;
+}
+template <int ROWS, int ELEM, bool KCONTIG, int NW, int STEP>
+__device__ __forceinline__ void dma_cut(int group0, int rest, int64_t ld_bytes,
+                                        const uint32_t (&off)[SliceGeom<ROWS, ELEM, KCONTIG, NW>::kLoads],
+                                        uint32_t (&cut)[SliceGeom<ROWS, ELEM, KCONTIG, NW>::kLoads]) {
 #pragma unroll
-  for (int j = J0; j < J1; ++j) {
-    const int group = group0 + j * STEP;
-    const int at = KCONTIG ? ((l & 7) ^ kc_swz(group * 8 + (l >> 3))) * 16
-                           : (group * G::kRowsPerLoad + l / G::kCPR) * ELEM;
-    cut[j] = at < rest ? off[j] : 0x80000000u;
+  for (int j = 0; j < SliceGeom<ROWS, ELEM, KCONTIG, NW>::kLoads; ++j) {
+    const int behind = dma_k<ROWS, ELEM, KCONTIG, NW>(group0 + j * STEP) - (rest - (KCONTIG ? 16 : ELEM));
+    cut[j] = off[j] - (behind > 0 ? KCONTIG ? (uint32_t)behind : (uint32_t)(behind / ELEM) * (uint32_t)ld_bytes : 0u);
   }
+}
+template <int ROWS, int ELEM, bool KCONTIG, int NW, int STEP>
+__device__ __forceinline__ void dma_blank(int group0, int rest, uint32_t lds_dst) {
+#pragma unroll
+  for (int j = 0; j < SliceGeom<ROWS, ELEM, KCONTIG, NW>::kLoads; ++j)
+    if (dma_k<ROWS, ELEM, KCONTIG, NW>(group0 + j * STEP) >= rest)
+      *(GEMM_AS3 u32x4 *)(uintptr_t)(lds_dst + (uint32_t)(j * STEP) * 1024u + (threadIdx.x & 63) * 16u) =
+          u32x4{0, 0, 0, 0};
 }
 
 // This wavefront's loads of one K slice of one operand, global -> LDS (its first
@@ -647,8 +658,10 @@ template <int BM, int BN, int NSTAGE, int NW, bool HALO = false> struct GemmLds 
 
 // Halo kernels are laid out for two workgroups per compute unit (two
 // wavefronts per SIMD): at most 256 registers per lane.
-// CUT: K ends inside its last slice (matrix products; a variant of its own, because the test
-// for that slice costs the others 0.5 us of 8 and 1 to 3 % of large products).
+// CUT: K ends inside its last slice (matrix products).  With the cut slice as the loop's last, a
+// test in every iteration and offsets of its own, the 256 x 256 variants had no registers left
+// (up to 45 spilled, some in the loop): bf16 4096 x 4096 x 4088, A along M and B along N, 371 us,
+// taken first 110; 4000 x 4000 x 4008 with B along K 120 / 105, 6936 x 2240 x 592 26.8 / 25.2.
 template <int KIND, int BM, int BN, int A_MODE, bool B_KC, int NSTAGE, int NW, bool CUT = false>
 __global__ __launch_bounds__(NW * 64)
 __attribute__((amdgpu_waves_per_eu(A_MODE == A_HALO ? 2 : 1, 8))) void
@@ -724,10 +737,10 @@ gemm_kernel(GemmArgs g) {
   // (the last part of a split may be shorter)
   const int kt_count =
       !HALO && g.kt_split > 0 && kt_base + g.kt_split < kt_total ? g.kt_split : kt_total - kt_base;
-  // bytes of K in its last slice, and the slice (of this part) whose loads leave the rest
-  // out, -1: none here
+  // A part that ends inside a slice takes that one first, ahead of the loop, which is the
+  // other variants' own; kt_rest: bytes of K in it.
+  const bool kt_cut = CUT && kt_base + kt_count == kt_total;
   const int kt_rest = (int)(g.K * ELEM - (int64_t)(kt_total - 1) * kTileKBytes);
-  const int kt_cut = CUT && kt_base + kt_count == kt_total ? kt_count - 1 : -1;
 
   const int wave = threadIdx.x >> 6;
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
@@ -840,9 +853,12 @@ gemm_kernel(GemmArgs g) {
   // Slices past the end of K are not loaded at all; the loops' waits by count
   // become waits for everything where a batch is missing.  (They used to be
   // "loaded" through zero-sized buffers, which kept every iteration identical;
-  // but such a load counts as complete before its zeros are written to LDS:
-  // on tiles whose real loads return quickly the zeros of the last batch
-  // could land in the epilogue's bands, after the final wait and barrier.)
+  // without those loads a split reduction that was wrong now and then no longer
+  // is.  That such a load counts as complete before its zeros are in LDS was the
+  // suspicion, and has not been seen: of 13 million wavefront loads from zero-sized
+  // buffers, as many behind a buffer's end and as many with half of the lanes there, every
+  // one had its zeros in LDS when vmcnt said so, and wrote nothing later.  Masked taps of
+  // the gather rest on that; a slice that K cuts does not, see dma_cut.)
   auto issue_a = [&](int kt, int st, auto part_c, auto parts_c) {
     if (kt >= kt_count)
       return;
@@ -872,10 +888,6 @@ gemm_kernel(GemmArgs g) {
         off[j] = (cv_mask[HALVES ? j / 2 : j] & need_j) == need_j ? off_a[j] + at : 0x80000000u;
       }
       dma_issue<LSTEP, GA::kLoads, A0, A1>(a_base, g.conv.x_bytes & lim, off, dst);
-    } else if (CUT && kt == kt_cut) {
-      uint32_t off[GA::kLoads];
-      dma_cut<BM, ELEM, A_KC, LW, LSTEP, A0, A1>(group_a, kt_rest, off_a, off);
-      dma_issue<LSTEP, GA::kLoads, A0, A1>(a_base + kt * a_step, 0x80000000u, off, dst);
     } else {
       dma_issue<LSTEP, GA::kLoads, A0, A1>(a_base + kt * a_step, lim, off_a, dst);
     }
@@ -888,13 +900,7 @@ gemm_kernel(GemmArgs g) {
     constexpr int B0 = PART * GB::kLoads / PARTS, B1 = (PART + 1) * GB::kLoads / PARTS;
     const uint32_t dst =
         (HALVES ? stage_half(team, st) + GA::kBytes / 2 : stage_b(st)) + (uint32_t)w_load * 1024u;
-    if (CUT && kt == kt_cut) {
-      uint32_t off[GB::kLoads];
-      dma_cut<BN, ELEM, B_KC, LW, LSTEP, B0, B1>(group_b, kt_rest, off_b, off);
-      dma_issue<LSTEP, GB::kLoads, B0, B1>(b_base + kt * b_step, 0x80000000u, off, dst);
-    } else {
-      dma_issue<LSTEP, GB::kLoads, B0, B1>(b_base + kt * b_step, 0xffffffffu, off_b, dst);
-    }
+    dma_issue<LSTEP, GB::kLoads, B0, B1>(b_base + kt * b_step, 0xffffffffu, off_b, dst);
   };
   auto issue = [&](int kt, int st, auto part_c, auto parts_c) {
     issue_a(kt, st, part_c, parts_c);
@@ -944,6 +950,19 @@ gemm_kernel(GemmArgs g) {
       issue(0, 0, Zero{}, One{});
       if (team)
         issue(1, 1, Zero{}, One{}); // (nothing when there is one slice)
+    } else if (CUT && kt_cut) {
+      if (team) {
+        uint32_t off[GB::kLoads];
+        dma_cut<BN, ELEM, B_KC, LW, LSTEP>(group_b, kt_rest, b_ldb, off_b, off);
+        dma_issue<LSTEP>(b_base + (kt_count - 1) * b_step, 0xffffffffu, off, stage_b(0) + (uint32_t)w_load * 1024u);
+        b_base -= b_step; // (of the slice behind it)
+        issue_b(1, 1, Zero{}, One{});
+      } else {
+        uint32_t off[GA::kLoads];
+        dma_cut<BM, ELEM, A_KC, LW, LSTEP>(group_a, kt_rest, a_ldb, off_a, off);
+        dma_issue<LSTEP>(a_base + (kt_count - 1) * a_step, 0xffffffffu, off, stage_a(0) + (uint32_t)w_load * 1024u);
+        a_base -= a_step;
+      }
     } else if (team) {
       issue_b(0, 0, Zero{}, One{});
       issue_b(1, 1, Zero{}, One{});
@@ -1018,6 +1037,16 @@ gemm_kernel(GemmArgs g) {
       __builtin_amdgcn_s_waitcnt(gemm_wait_imm(HALVES ? LPS : GB::kLoads));
     else
       __builtin_amdgcn_s_waitcnt(gemm_wait_imm(0));
+    static_assert(!CUT || TEAMS, "a wavefront loads one operand");
+    if constexpr (CUT) {
+      if (kt_cut) {
+        if (team)
+          dma_blank<BN, ELEM, B_KC, LW, LSTEP>(group_b, kt_rest, stage_b(0) + (uint32_t)w_load * 1024u);
+        else
+          dma_blank<BM, ELEM, A_KC, LW, LSTEP>(group_a, kt_rest, stage_a(0) + (uint32_t)w_load * 1024u);
+        __builtin_amdgcn_s_waitcnt(gemm_wait_imm(63));
+      }
+    }
     gemm_barrier();
   } else {
     __builtin_amdgcn_s_waitcnt(gemm_wait_imm(0));

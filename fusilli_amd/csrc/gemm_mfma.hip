@@ -9,9 +9,10 @@
 //     with the gfx950 transposing LDS reads (ds_read_b64_tr_b16 / _tr_b8), so
 //     no operand is ever transposed in registers or in HBM;
 //   * K may end inside a 128-byte slice (in whole 16-byte chunks where an operand lies along
-//     it): a variant of the kernel masks the last slice's loads (bf16 4000 x 4000 x 4008
-//     419 us on the direct kernels -> 104, fp8 3702 x 3584 x 6640 292 -> 77); the parts of a
-//     split reduction may differ in length (323 x 688 x 5952 in 12 parts instead of 3, 28.8 -> 21.7);
+//     it): a variant of the kernel takes that slice first and blanks what lies behind K (bf16
+//     4000 x 4000 x 4008 419 us on the direct kernels -> 101, fp8 3702 x 3584 x 6640 292 -> 80); the
+//     parts of a split reduction may differ in length (bf16 232 x 2232 x 5664, both transposed, in six
+//     parts 41.7 -> 23.3);
 //   * 256 threads = 2 x 2 wavefronts per workgroup, each wavefront owning a
 //     (BM/2) x (BN/2) block of 32x32 MFMA tiles; K advances in 128-byte slices
 //     through double-buffered, bank-conflict-padded LDS with the next slice's

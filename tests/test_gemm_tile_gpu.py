@@ -73,6 +73,52 @@ def test_cut_slices(ctx, dtype, k16, ta, tb, m, n, slices, rest):
     check(got, ref_matmul(a, b), odt, name)
 
 
+# every tile of the tiled GEMM, operands along M / N (whole K-rows are masked) and along K, split
+# reductions whose last part is the shorter one, a slice of a few values
+CUT = [
+    (capi.HALF, 601, 4736, 808, False, False, "128x128 waves=8 split=1"),
+    (capi.BFLOAT16, 4104, 4104, 75, True, False, "128x128 waves=8 split=1"),
+    (capi.FP8E4M3, 2576, 2592, 4000, True, True, "256x128 waves=8 split=1"),
+    (capi.BFLOAT16, 4096, 4096, 72, True, False, "256x256 waves=8 split=1"),
+    (capi.HALF, 6936, 2240, 592, True, True, "256x256 waves=8 split=1"),
+    (capi.FP8E4M3, 4096, 4096, 131, True, False, "256x256 waves=8 split=1"),
+    (capi.FP8E4M3, 6936, 2240, 1168, False, False, "256x256 waves=8 split=1"),
+    (capi.INT8, 6936, 2240, 1168, False, True, "256x256 waves=8 split=1"),
+    (capi.BFLOAT16, 232, 2232, 5664, True, True, "128x128 waves=8 split=6"),
+    (capi.BFLOAT16, 1059, 1152, 5744, False, False, "128x128 waves=8 split=3"),
+    (capi.INT8, 1248, 800, 8752, True, True, "128x128 waves=8 split=3"),
+]
+
+
+@pytest.mark.parametrize("dtype,m,n,k,ta,tb,route", CUT)
+def test_cut_slice_after_garbage(ctx, dtype, m, n, k, ta, tb, route):
+    # What a masked part of the last slice holds in LDS must not reach the sums: the same product
+    # of NaNs (127 in int8) has just left its operands there.
+    a, b = make_operand(87, 0, m, k, dtype, ta), make_operand(87, 1, k, n, dtype, tb)
+    full = 127 if dtype == capi.INT8 else np.nan
+    fill = [HT.from_logical(np.full(t.dims, full), dtype, t.strides) for t in (a, b)]
+    run(ctx, *fill)
+    got, name, odt = run(ctx, a, b)
+    assert name.endswith(route), name
+    check(got, ref_matmul(a, b), odt, name)
+
+
+@pytest.mark.parametrize("m,n,k,ta,tb", [(4096, 4096, 72, True, False), (601, 4736, 808, False, False)])
+def test_infinities_in_front_of_a_cut(ctx, m, n, k, ta, tb):
+    # the last row of K is fetched again in place of those behind it: neither operand's may count
+    a, b = make_operand(88, 0, m, k, capi.BFLOAT16, ta), make_operand(88, 1, k, n, capi.BFLOAT16, tb)
+    av, bv = a.logical(), b.logical()
+    av[5, k - 1], bv[k - 1, 7] = np.inf, -np.inf
+    a = HT.from_logical(av, capi.BFLOAT16, a.strides)
+    b = HT.from_logical(bv, capi.BFLOAT16, b.strides)
+    got, name, _ = run(ctx, a, b)
+    ref = ref_matmul(a, b)
+    assert "waves=8 split=1" in name, name
+    assert np.array_equal(np.isposinf(got), np.isposinf(ref)) and np.array_equal(np.isneginf(got), np.isneginf(ref)), name
+    finite = np.isfinite(ref)
+    assert_close(got[finite], ref[finite], capi.BFLOAT16, name)
+
+
 @pytest.mark.parametrize("dtype", [capi.BFLOAT16, capi.HALF])
 @pytest.mark.parametrize("m,n,k,batch", [(130, 250, 1003, 1), (140, 140, 6001, 1), (90, 200, 700, 5), (700, 1300, 1500, 1)])
 def test_fused_chains(ctx, dtype, m, n, k, batch):
