@@ -309,7 +309,10 @@ int fhip_tuned_matmul(fhip_ctx *ctx, const fhip_matmul_desc *d, const void *a,
   if (whole && (!aligned || fhip_knobs().gemm_tile_bm || fhip_knobs().gemm_split))
     return run_plan(ctx, p, d, a, b, epi, out); // (misaligned operands of the contract are refused)
   double us = 0;
-  if (p.ok && aligned) {
+  // (f32 results of a K inside one 16-byte chunk, which the direct kernels leave to the general
+  // path, stay there: an fp8 MFMA aligns its products to the largest, 5e-6 of the result at K 13)
+  const bool f32_out = p.kind != GK_I8 && d->c.dtype == FHIP_FLOAT && d->out.dtype == FHIP_FLOAT;
+  if (p.ok && aligned && (whole || !f32_out)) {
     // (the planner's estimate against 154 products of 128 to 4096 rows and 256 to 8192 columns:
     // 14 % rms for 16 bits, 5 for fp8, 11 for int8; GELU over whole 128-wide tiles 6 us)
     const bool gelu = fhip_epilogue_is_transcendental(d->epilogue);

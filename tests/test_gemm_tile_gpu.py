@@ -103,6 +103,22 @@ def test_cut_slice_after_garbage(ctx, dtype, m, n, k, ta, tb, route):
     check(got, ref_matmul(a, b), odt, name)
 
 
+@pytest.mark.parametrize("dtype,m,n,k", [
+    (capi.FP8E5M2, 1024, 512, 13), (capi.FP8E4M3, 256, 272, 15), (capi.BFLOAT16, 512, 512, 7), (capi.HALF, 264, 1040, 3)])
+def test_few_values_of_k_into_f32(ctx, dtype, m, n, k):
+    # exact products and an f32 sum: each addition may be off by half a unit of its partial sum
+    a, b = make_operand(89, 0, m, k, dtype, True), make_operand(89, 1, k, n, dtype, False)
+    out = HT.empty([m, n], capi.FLOAT)
+    d = capi.MatmulDesc()
+    d.a, d.b, d.out, d.out_dtype = a.desc(), b.desc(), out.desc(), capi.FLOAT
+    d.c = capi.TensorDesc.make([m, n], out.strides, capi.FLOAT)
+    d.epilogue = capi.make_epilogue([])
+    da, db, do = a.upload(ctx), b.upload(ctx), out.upload(ctx)
+    ctx.matmul(d, da, db, do)
+    got, size = out.fetch(ctx, do).logical(), np.abs(a.logical()) @ np.abs(b.logical())
+    assert np.all(np.abs(got - ref_matmul(a, b)) <= k * 2.0 ** -24 * size), ctx.last_kernel()
+
+
 @pytest.mark.parametrize("m,n,k,ta,tb", [(4096, 4096, 72, True, False), (601, 4736, 808, False, False)])
 def test_infinities_in_front_of_a_cut(ctx, m, n, k, ta, tb):
     # the last row of K is fetched again in place of those behind it: neither operand's may count
