@@ -15,10 +15,9 @@
 //
 // bf16 16000 x 1003 RMSNorm + MUL: 207 us (generic) -> 20.3 (3.2 TB/s); f16 LayerNorm 9000 x
 // 3001: 442 -> 49 (2.2 TB/s).  (Unrolling the walk four times is slower: 49 -> 55.6.)
-// Segments: bf16 LayerNorm 16 x 262144 9.6 us, of which two launches that do next to nothing
-// take 7; 600 x 300000 329 -> 237 (a pivot in place of the segments' means, segments of
-// eight vectors per thread walked, scale and bias fetched after the sums); a launch per sum
-// and whole rows, bf16 LayerNorm 204 x 9335 13.3 -> 9.4.
+// Segments: bf16 LayerNorm 16 x 262144 9.0 us, of which two launches that do next to nothing
+// take 7; 600 x 300000 329 -> 242 (segments of eight vectors per thread); whole rows, bf16
+// LayerNorm 204 x 9335 14.8 -> 9.0.
 //
 // Reference semantics: aten.rms_norm / aten.layer_norm over all dims except
 // dim 0 (reference support/asm_emitter.h:1592-1626, 1427-1503;
@@ -36,7 +35,8 @@ constexpr int64_t kRwResident = 16384; // vectors of the longest rows that rowno
 struct RowWalkArgs {
   RowNormArgs n;
   double *partial; // [rows][splits][2]: sums of x, second moments around the segment's mean
-  double inv;      // 1 / elements per row
+  double inv;      // 1 / elements per row,
+  double inv_seg, inv_last; // per segment, of the last one
   int64_t seg;     // elements per segment, a multiple of the vector width
   int32_t splits;
 };
@@ -280,60 +280,85 @@ __global__ __launch_bounds__(kRwThreads) void rownorm_walk_kernel(RowNormArgs g,
 
 // Few long rows: a segment of a row per workgroup, two launches.  The first leaves every
 // segment's sum and its second moment around the segment's own mean (RMSNorm: around zero);
-// the second adds a row's pairs up, moved to the first segment's mean, and applies.  NV > 0:
-// a thread's NV vectors of the segment stay in registers between the two sums, and come with
-// their scale and bias while the pairs are on their way; 0: segments of any length are walked.
+// the second adds a row's pairs up, moved to the first segment's mean, and applies.
 // (A segment per wavefront, no barrier in the first launch, but four times the pairs: bf16
 // 4 x 65544 7.5 -> 7.9 us, f32 32 x 524288 34.8 -> 40.6.)
 typedef double rw_pair __attribute__((ext_vector_type(2)));
 
-template <typename T, int NV>
+// The mean of segment `i`, rounded: both launches have the same from a segment's sum.
+__device__ __forceinline__ double rw_centre(const RowWalkArgs &g, int i, double sum) {
+  return (double)(float)(sum * (i + 1 < g.splits ? g.inv_seg : g.inv_last));
+}
+
+// A segment is read once and reduced once.  A vector's deviations are taken in f32 from the
+// vector's own mean (as f32 has it: their sum makes up for the difference) and moved in f64
+// to `pivot`, an element of the segment, so that the second moment there is at most `elements`
+// times the one around the segment's mean, to which it goes last: no digit that f32 holds is lost.
+// (Sums first, then moments, of vectors kept or walked again: 0.2 to 0.6 us more.)
+template <typename T>
+__device__ __forceinline__ void rw_moments(const float (&v)[RwVec<T>::kN], int live, double pivot, double &s1,
+                                           double &s2) {
+  constexpr int N = RwVec<T>::kN;
+  const float sum = (float)rw_tree<T, 1>(v, 0.f, live), mean = live == N ? sum * (1.f / N) : sum / (float)live;
+  float d[N];
+#pragma unroll
+  for (int k = 0; k < N; ++k)
+    d[k] = v[k] - mean;
+  const double e = (double)mean - pivot, n = (double)live, rest = rw_tree<T, 1>(d, 0.f, live);
+  s1 += n * (double)mean + rest;
+  s2 += rw_tree<T, 2>(d, 0.f, live) + e * (n * e + 2. * rest);
+}
+
+template <typename T, bool LAYER>
 __global__ __launch_bounds__(kRwThreads) void rownorm_walk_sums_kernel(RowWalkArgs g) {
   using V = RwVec<T>;
-  constexpr int N = V::kN;
-  __shared__ double lds[kRwWaves];
+  constexpr int N = V::kN, kStep = kRwThreads * N;
+  __shared__ rw_pair lds[kRwWaves];
   const int64_t row = blockIdx.y, lo = blockIdx.x * g.seg;
   const int64_t hi = lo + g.seg < g.n.inner ? lo + g.seg : g.n.inner;
   const T *xr = (const T *)g.n.x + row * g.n.x_row_stride;
+  const double pivot = LAYER ? (double)(float)xr[lo] : 0.;
   double s1 = 0., s2 = 0.;
-  float mean = 0.f;
-  if constexpr (NV > 0) {
-    typename V::loose raw[NV];
-    int live[NV];
-#pragma unroll
-    for (int j = 0; j < NV; ++j) {
-      const int64_t i = lo + (int64_t)(threadIdx.x + j * kRwThreads) * N;
-      live[j] = hi - i >= N ? N : hi > i ? (int)(hi - i) : 0;
-      raw[j] = V::load_raw(xr + i, live[j]);
-    }
-    if (g.n.is_layernorm) {
-#pragma unroll
-      for (int j = 0; j < NV; ++j) {
-        float v[N];
-        V::widen(raw[j], v);
-        s1 += rw_tree<T, 1>(v, 0.f, live[j]);
-      }
-      s1 = rw_sum<kRwWaves>(s1, lds);
-      mean = (float)(s1 / (double)(hi - lo));
-    }
-#pragma unroll
-    for (int j = 0; j < NV; ++j) {
-      float v[N];
-      V::widen(raw[j], v);
-      s2 += rw_tree<T, 2>(v, mean, live[j]);
-    }
-  } else {
-    if (g.n.is_layernorm) {
-      s1 = rw_sum<kRwWaves>(rw_walk<T, 1>(xr, 0.f, lo, hi, threadIdx.x, kRwThreads), lds);
-      mean = (float)(s1 / (double)(hi - lo));
-    }
-    s2 = rw_walk<T, 2>(xr, mean, lo, hi, threadIdx.x, kRwThreads);
+  auto add = [&](const typename V::loose &raw, int live) {
+    float v[N];
+    V::widen(raw, v);
+    if constexpr (LAYER)
+      rw_moments<T>(v, live, pivot, s1, s2);
+    else
+      s2 += rw_tree<T, 2>(v, 0.f, live);
+  };
+  int64_t i = lo + (int64_t)threadIdx.x * N;
+  for (; i + kStep + N <= hi; i += 2 * kStep) { // (two loads in flight)
+    const typename V::loose a = V::load_raw(xr + i, N), b = V::load_raw(xr + i + kStep, N);
+    add(a, N);
+    add(b, N);
   }
-  s2 = rw_sum<kRwWaves>(s2, lds);
-  if (threadIdx.x == 0)
+  for (; i < hi; i += kStep) {
+    const int live = hi - i < N ? (int)(hi - i) : N;
+    add(V::load_raw(xr + i, live), live);
+  }
+  s1 = LAYER ? rw_wave_sum(s1) : 0.;
+  s2 = rw_wave_sum(s2);
+  if ((threadIdx.x & 63) == 0)
+    lds[threadIdx.x >> 6] = rw_pair{s1, s2};
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    s1 = s2 = 0.;
+#pragma unroll
+    for (int w = 0; w < kRwWaves; ++w) {
+      s1 += lds[w].x;
+      s2 += lds[w].y;
+    }
+    if constexpr (LAYER) {
+      const double n = (double)(hi - lo), d = rw_centre(g, (int)blockIdx.x, s1) - pivot;
+      s2 += d * (n * d - 2. * (s1 - n * pivot));
+    }
     ((rw_pair *)g.partial)[row * g.splits + blockIdx.x] = rw_pair{s1, s2};
+  }
 }
 
+// NV > 0 (LayerNorm): a thread's NV vectors of X come with their scale and bias while the pairs are
+// on their way; 0: segments of any length are walked.
 template <typename T, int NV>
 __global__ __launch_bounds__(kRwThreads) void rownorm_walk_apply_kernel(RowWalkArgs g) {
   using V = RwVec<T>;
@@ -365,12 +390,12 @@ __global__ __launch_bounds__(kRwThreads) void rownorm_walk_apply_kernel(RowWalkA
   // sum (x - c0)^2 = sum (x - c)^2 + 2 d (sum x - n c) + n d^2 of a segment whose second
   // moment lies around c, d = c - c0 (RMSNorm: all zero)
   double c0 = 0., s = 0., q = in ? mine.y : 0.;
-  if (g.n.is_layernorm) { // (two divisions in 64 bits: RMSNorm passes them by)
-    const double n0 = (double)(g.seg < g.n.inner ? g.seg : g.n.inner);
-    c0 = (double)(float)(first / n0);
+  const bool layer = NV > 0 || g.n.is_layernorm != 0;
+  if (layer) {
+    c0 = rw_centre(g, 0, first);
     const int64_t left = g.n.inner - (in ? threadIdx.x : 0) * g.seg;
     const double n = (double)(left < g.seg ? left : g.seg);
-    const double c = (double)(float)(mine.x / n), d = c - c0;
+    const double c = rw_centre(g, in ? (int)threadIdx.x : 0, mine.x), d = c - c0;
     s = rw_wave_sum(in ? mine.x : 0.);
     q = in ? mine.y + 2. * d * (mine.x - n * c) + n * d * d : 0.;
   }
@@ -388,7 +413,7 @@ __global__ __launch_bounds__(kRwThreads) void rownorm_walk_apply_kernel(RowWalkA
   q *= g.inv;
   const float mean = (float)s;
   const double e = (double)mean - c0, around = q - 2. * e * (s - c0) + e * e;
-  const float var = g.n.is_layernorm ? (around < 0. ? 0.f : (float)around) : (float)q;
+  const float var = layer ? (around < 0. ? 0.f : (float)around) : (float)q;
   const float rstd = 1.0f / sqrtf(var + g.n.eps);
   if (g.n.emit_stats && blockIdx.x == 0 && threadIdx.x == 0)
     rw_stats(g.n, row, mean, rstd);
@@ -418,19 +443,18 @@ __global__ __launch_bounds__(kRwThreads) void rownorm_walk_apply_kernel(RowWalkA
 
 template <typename T> void rw_launch_split(hipStream_t stream, const RowWalkArgs &g, int64_t cus) {
   const dim3 grid((unsigned)g.splits, (unsigned)g.n.rows), wg(kRwThreads);
-  auto go = [&](auto nv) {
-    constexpr int NV = decltype(nv)::value;
-    hipLaunchKernelGGL((rownorm_walk_sums_kernel<T, NV>), grid, wg, 0, stream, g);
-    hipLaunchKernelGGL((rownorm_walk_apply_kernel<T, NV>), grid, wg, 0, stream, g);
-  };
-  // (RMSNorm needs one sum and has no bias to fetch ahead: there walked segments are 2 to 8 %
-  // faster, f16 28 x 229376 12.4 us against 13.0, f32 22 x 195584 14.1 / 14.7; so are those of
-  // LayerNorm beyond four workgroups per compute unit, which cover each other's waits: f16
-  // 12 x 400384 11.9 / 12.3, 28 x 229376 13.4 / 13.7, but 20 x 200704 10.5 / 10.3, 5 x 310272 8.0 / 7.9)
-  if (g.seg <= 2 * kRwThreads * RwVec<T>::kN && g.n.is_layernorm && g.n.rows * g.splits <= 4 * cus)
-    go(std::integral_constant<int, 2>{});
+  if (g.n.is_layernorm)
+    hipLaunchKernelGGL((rownorm_walk_sums_kernel<T, true>), grid, wg, 0, stream, g);
   else
-    go(std::integral_constant<int, 0>{});
+    hipLaunchKernelGGL((rownorm_walk_sums_kernel<T, false>), grid, wg, 0, stream, g);
+  // (RMSNorm has no bias to fetch ahead: walked segments are 2 to 8 % faster there, f16 28 x 229376
+  // 12.4 us against 13.0, f32 22 x 195584 14.1 / 14.7; so are those of LayerNorm beyond four workgroups
+  // per compute unit, which cover each other's waits: bf16 18 x 412672 13.9 / 15.8, 30 x 140288 10.4 / 11.1,
+  // but f32 32 x 524288 35.4 / 34.3)
+  if (g.seg <= 2 * kRwThreads * RwVec<T>::kN && g.n.is_layernorm && g.n.rows * g.splits <= 4 * cus)
+    hipLaunchKernelGGL((rownorm_walk_apply_kernel<T, 2>), grid, wg, 0, stream, g);
+  else
+    hipLaunchKernelGGL((rownorm_walk_apply_kernel<T, 0>), grid, wg, 0, stream, g);
 }
 
 template <typename T> void rw_launch_rows(hipStream_t stream, const RowNormArgs &g, int waves) {
@@ -481,6 +505,8 @@ int fhip_norm_walk(fhip_ctx *ctx, int dtype, const RowNormArgs &n, bool cut_pays
       return 1;
     g.partial = (double *)scratch;
     g.inv = 1.0 / (double)n.inner;
+    g.inv_seg = 1.0 / (double)g.seg;
+    g.inv_last = 1.0 / (double)(n.inner - (g.splits - 1) * g.seg);
     g.n = n;
     fhip_note_kernel(ctx, "rownorm_walk segments=%d", g.splits);
   } else {

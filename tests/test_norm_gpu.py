@@ -419,3 +419,26 @@ def test_norm_rows_in_segments_vs_64_bits(ctx, dtype, rows, cols, kind):
             out.fetch(ctx, dx)
     assert ctx.last_kernel().startswith("rownorm_walk segments="), ctx.last_kernel()
     assert_close(out.logical(), y, dtype, f"{kind} {rows} x {cols}")
+
+
+@pytest.mark.parametrize("dtype,rows,cols,at", [
+    (capi.FLOAT, 2, 65541, 3000.0), (capi.FLOAT, 40, 60003, -5.0e5), (capi.HALF, 3, 131079, 100.0),
+    (capi.BFLOAT16, 1, 256 * 4096 + 3, -60.0), (capi.FLOAT, 1, 2049 * 4 + 1, 7.0)])
+def test_segments_far_from_zero(ctx, dtype, rows, cols, at):
+    # means of many deviations, the first element of some segments far from the others, a last
+    # vector of a few elements
+    x = rand(44, 0, [rows, cols], std=1.0) + np.float32(at)
+    x[:, ::4096] += 90.0
+    x = HT.from_logical(x, dtype)
+    s = HT.from_logical(rand(44, 1, [1, cols], mean=1.0, std=0.1), dtype)
+    b = HT.from_logical(rand(44, 2, [1, cols]), dtype)
+    out, mean, rstd = run_norm(ctx, x, s, b, eps=1e-5, layernorm=True, stats=True)
+    assert ctx.last_kernel().startswith("rownorm_walk segments="), ctx.last_kernel()
+    # the statistics' own rounding, twice; the second moment is the one around the rounded mean
+    v, m = x.logical().astype(np.float64), mean.logical().astype(np.float64)
+    assert np.all(np.abs(m - v.mean(1)) <= 2.0 ** -23 * np.abs(m))
+    r = 1.0 / np.sqrt(np.square(v - m[:, None]).mean(1) + 1e-5)
+    assert np.all(np.abs(rstd.logical() - r) <= 2.0 ** -22 * r)
+    # f32 arithmetic on deviations, one rounding to the result's type
+    y = (v - m[:, None]) * r[:, None] * s.logical() + b.logical()
+    assert np.all(np.abs(out.logical() - y) <= 2.0 ** {capi.FLOAT: -20, capi.HALF: -10, capi.BFLOAT16: -7}[dtype] * (1 + np.abs(y)))
