@@ -633,6 +633,9 @@ bool fhip_fast_conv_applicable(const fhip_conv_desc *d, bool allow_scratch) {
   return fhip_fast_conv_rf_applicable(d) || resolve(d, allow_scratch, true, false).plan.ok;
 }
 
+static int run_resolved(fhip_ctx *ctx, const fhip_conv_desc *d, ConvResolved &res, const void *x, const void *w,
+                        const DevEpilogue &epi, void *out, bool *handled, bool allow_scratch);
+
 int fhip_fast_conv(fhip_ctx *ctx, const fhip_conv_desc *d, const void *x,
                    const void *w, const DevEpilogue &epi, void *out,
                    bool *handled, bool allow_scratch, bool split) {
@@ -644,6 +647,12 @@ int fhip_fast_conv(fhip_ctx *ctx, const fhip_conv_desc *d, const void *x,
   if (taken)
     return 0;
   ConvResolved res = resolve(d, allow_scratch, split);
+  return run_resolved(ctx, d, res, x, w, epi, out, handled, allow_scratch);
+}
+
+// `d` as `res` has it, on what is left of the kernels here.
+static int run_resolved(fhip_ctx *ctx, const fhip_conv_desc *d, ConvResolved &res, const void *x, const void *w,
+                        const DevEpilogue &epi, void *out, bool *handled, bool allow_scratch) {
   if (res.plan.ok && !fhip_ctx_scratch_ready(ctx, scratch_bytes(res)))
     do_without_scratch(d, res);
   const ConvPlan &p = res.plan;
@@ -862,6 +871,7 @@ namespace {
 struct DgradPlan {
   bool ok = false;
   fhip_conv_desc fwd; // the equivalent forward problem
+  bool rf = false;    // which the register-filter kernel takes (its plan costs the host 3 us)
   size_t filter_bytes = 0;
   // strides above one: DY is first spread over a zero grid of the unit-stride
   // output extent (element (p, q) at (p * stride, q * stride)), in workspace
@@ -930,7 +940,8 @@ DgradPlan make_dgrad_plan(const fhip_conv_desc *d, bool allow_scratch = true) {
     st *= f.w.dim[2 + i];
   }
   f.w.stride[0] = st;
-  if (!fhip_fast_conv_applicable(&f, allow_scratch))
+  p.rf = fhip_fast_conv_rf_applicable(&f);
+  if (!p.rf && !resolve(&f, allow_scratch, true, false).plan.ok)
     return p;
   p.filter_bytes =
       ((size_t)(st * f.w.dim[0]) * fhip_dtype_size(f.w.dtype) + 255) / 256 * 256;
@@ -1037,6 +1048,8 @@ struct DgradTiles {
   bool copy = false; // W is first laid out channels-last in the workspace
   ConvTileArgs args{};
   ConvTilePlan plan;
+  bool resolved = false; // unit strides: what runs the forward problem instead is in `fwd`
+  ConvResolved fwd;
 };
 
 // One spatial dim of a gradient: output rows of remainder `a` by the stride.
@@ -1060,9 +1073,11 @@ static DgradTiles make_dgrad_tiles(const fhip_conv_desc *d, const DgradPlan &p, 
     return t;
   double other = 0; // of the forward kernel on the mirrored filter
   if (!p.spread) {
-    if (fhip_fast_conv_rf_applicable(&p.fwd))
+    if (p.rf)
       return t;
-    ConvResolved r = resolve(&p.fwd, allow_scratch, false);
+    ConvResolved &r = t.fwd;
+    r = resolve(&p.fwd, allow_scratch, false);
+    t.resolved = true;
     if (!r.unpadded())
       tile_args(r.plan, K, r.args);
     other = r.tile.bm ? r.tile.us + 2.6 : igemm_us(r, true, false);
@@ -1210,7 +1225,9 @@ int fhip_fast_conv_dgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy,
     dgrad_note(ctx, "dgrad spread + ");
     return rc;
   }
-  const int rc = fhip_fast_conv(ctx, &p.fwd, dy, workspace, epi, dx, nullptr, allow_scratch, false);
+  const int rc = tiles.resolved
+                     ? run_resolved(ctx, &p.fwd, tiles.fwd, dy, workspace, epi, dx, nullptr, allow_scratch)
+                     : fhip_fast_conv(ctx, &p.fwd, dy, workspace, epi, dx, nullptr, allow_scratch, false);
   dgrad_note(ctx, "dgrad ");
   return rc;
 }

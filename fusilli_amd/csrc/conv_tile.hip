@@ -68,9 +68,15 @@ ConvTilePlan conv_tile_plan(const ConvTileArgs &g, bool dgrad, bool fused, size_
     const TileLoad l(f, g);
     if (l.most >= (1ll << 23))
       continue;
+    // (a split leaves the tiles' work as it is and adds to all else: nothing shorter comes
+    // behind one whose work and rounds alone take longer than the best so far)
+    const double load = (double)l.tiles / 256.0, teams = f.teams > 1 ? f.teams : 1;
+    const double least = f.once + f.sum + l.longest * load * std::max(f.alone / f.occ, f.shared) / teams;
+    const double each = f.round * load + f.part * (double)(l.tiles * f.bm * f.bn) * 4e-6;
     for (int split = 1; split <= 12; ++split) {
       if (split > 1 && (g.parts > 1 || l.longest / split < 2 || l.most * split > 1500 ||
-                        (size_t)split * (size_t)(l.most * f.bm * f.bn) * sizeof(float) > room))
+                        (size_t)split * (size_t)(l.most * f.bm * f.bn) * sizeof(float) > room ||
+                        least + split * each >= best.us))
         break;
       const double us = tile_us(f, l, g.parts == 1, split, fused);
       if (best.bm == 0 || us < best.us)
