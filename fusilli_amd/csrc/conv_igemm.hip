@@ -773,7 +773,8 @@ static int run_resolved(fhip_ctx *ctx, const fhip_conv_desc *d, ConvResolved &re
     a.c_dt = d->y.dtype, a.o_dt = d->out.dtype;
     a.epi = g.epi;
     conv_tile_lean(d->epilogue, res.args);
-    fhip_note_kernel(ctx, "conv_igemm unpadded %dx%d split=%d", res.tile.bm, res.tile.bn, res.tile.splits);
+    fhip_note_kernel(ctx, "conv_igemm unpadded %dx%d split=%d teams=%d", res.tile.bm, res.tile.bn, res.tile.splits,
+                     res.tile.teams);
     return conv_tile_launch(ctx, p.kind == GK_BF16, false, res.tile, res.args, scratch);
   }
   // A single tap at unit stride without padding is the matrix product
@@ -1169,8 +1170,8 @@ static int run_dgrad_tiles(fhip_ctx *ctx, const fhip_conv_desc *d, const DgradPl
     w = workspace;
   }
   t.args.d.a = (const char *)dy, t.args.d.b = (const char *)w, t.args.d.out = (char *)dx;
-  fhip_note_kernel(ctx, "dgrad conv_igemm unpadded %dx%d split=%d parts=%d", t.plan.bm, t.plan.bn, t.plan.splits,
-                   t.args.parts);
+  fhip_note_kernel(ctx, "dgrad conv_igemm unpadded %dx%d split=%d parts=%d teams=%d", t.plan.bm, t.plan.bn, t.plan.splits,
+                   t.args.parts, t.plan.teams);
   return conv_tile_launch(ctx, d->y.dtype == FHIP_BFLOAT16, true, t.plan, t.args, partial);
 }
 

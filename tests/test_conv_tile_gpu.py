@@ -67,12 +67,11 @@ def test_data_gradient(ctx, x, w, pad, st, dil, parts, dtype, flat):
     ([9, 128, 12, 12], [128, 128, 5, 5], 2, 1),    # few tiles, a long reduction
     ([31, 192, 11, 11], [180, 192, 5, 5], 2, 1),   # columns off a tile
     ([7, 456, 13, 14], [61, 456, 3, 3], 1, 2),     # odd columns, channels off a slice
-    ([40, 264, 30, 30], [260, 264, 3, 3], 1, 1),   # wide tiles
+    ([40, 264, 30, 30], [260, 264, 3, 3], 1, 1),   # wide tiles; with a chain conv_gather.hip
     ([2, 520, 6, 6], [64, 520, 5, 5], 2, 1),
 ])
 @pytest.mark.parametrize("chain", [False, True])
-def test_forward(ctx, x, w, pad, st, chain):
-    dtype = capi.BFLOAT16
+def test_forward(ctx, x, w, pad, st, chain, dtype=capi.BFLOAT16, route=""):
     geom = ([pad, pad], [st, st], [1, 1])
     yd = oracle.conv_output_dims(x, w, *geom)
     xs, wt = _whole(82, 0, x, 3, dtype), _whole(82, 1, w, 2, dtype)
@@ -83,8 +82,30 @@ def test_forward(ctx, x, w, pad, st, chain):
            capi.epilogue_op(capi.PW["RELU_FWD"], dtype)] if chain else []
     y = run_conv(ctx, xs, wt, *geom, capi.FLOAT, out_dtype=dtype if chain else capi.FLOAT, epilogue=epi,
                  epi_tensors=[bias, res] if chain else [], channels_last_out=True)
-    assert ctx.last_kernel().startswith("conv_igemm unpadded"), ctx.last_kernel()
+    assert ctx.last_kernel().startswith(f"conv_igemm unpadded {route}"), ctx.last_kernel()
     ref = torch.nn.functional.conv2d(torch.from_numpy(xs.logical()), torch.from_numpy(wt.logical()), None, st, pad)
     if chain:
         ref = (ref + torch.from_numpy(bias.logical()) + torch.from_numpy(res.logical())).clamp(min=0)
     _equal(y.logical(), ref, dtype if chain else capi.FLOAT)
+
+
+# every tile of the forward kernel, whole and in parts (teams=0: the kernel for short reductions)
+@pytest.mark.parametrize("x,w,pad,st,chain,route", [
+    ([33, 120, 22, 38], [200, 120, 3, 3], 1, 1, False, "128x128 split=1 teams=1"),
+    ([13, 120, 36, 33], [196, 120, 3, 3], 1, 1, True, "128x128 split=1 teams=1"),
+    ([27, 296, 36, 9], [76, 296, 3, 3], 1, 1, False, "128x128 split=3 teams=1"),
+    ([10, 416, 24, 36], [68, 416, 3, 3], 1, 1, True, "128x128 split=3 teams=1"),
+    ([33, 184, 17, 34], [144, 184, 3, 3], 1, 1, True, "128x64 split=1 teams=1"),
+    ([31, 288, 27, 7], [140, 288, 5, 5], 2, 1, False, "128x64 split=3 teams=1"),
+    ([30, 112, 39, 25], [104, 112, 3, 3], 1, 1, False, "64x128 split=1 teams=1"),
+    ([13, 56, 25, 38], [216, 56, 5, 5], 2, 1, True, "64x128 split=1 teams=1"),
+    ([11, 216, 19, 14], [72, 216, 5, 5], 2, 1, False, "64x128 split=5 teams=1"),
+    ([8, 184, 24, 26], [72, 184, 5, 5], 2, 1, True, "64x128 split=3 teams=1"),
+    ([9, 176, 25, 15], [264, 176, 3, 3], 1, 1, True, "64x64 split=1 teams=0"),
+    ([2, 104, 5, 8], [92, 104, 3, 3], 1, 1, True, "64x64 split=5 teams=0"),
+    ([12, 128, 10, 27], [200, 128, 3, 3], 1, 2, False, "64x64 split=1 teams=2"),
+    ([1, 216, 28, 18], [37, 216, 5, 5], 2, 2, False, "64x64 split=11 teams=2"),
+])
+@pytest.mark.parametrize("dtype", [capi.BFLOAT16, capi.HALF])
+def test_forward_tiles(ctx, x, w, pad, st, chain, route, dtype):
+    test_forward(ctx, x, w, pad, st, chain, dtype, route)

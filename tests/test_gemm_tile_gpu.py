@@ -61,7 +61,37 @@ def test_wide_tiles(ctx, dtype, ta, tb, m, n, k):
     assert name.startswith("gemm_mfma") and "128x128 waves=4" in name, name
 
 
-# whole 16-byte chunks of K, and any K where neither operand lies along it: the tiled GEMM
+# 64 x 128 and 128 x 64 tiles, whole and in parts
+HALF_WIDE = [
+    (capi.BFLOAT16, 1059, 1928, 623, False, False, "64x128 waves=4 split=1"),
+    (capi.HALF, 1944, 1098, 692, False, True, "64x128 waves=4 split=1"),
+    (capi.BFLOAT16, 1581, 1217, 258, True, False, "64x128 waves=4 split=1"),
+    (capi.HALF, 1311, 1705, 264, True, True, "64x128 waves=4 split=1"),
+    (capi.BFLOAT16, 910, 352, 4928, False, False, "64x128 waves=4 split=5"),
+    (capi.BFLOAT16, 225, 2051, 4303, True, False, "64x128 waves=4 split=3"),
+    (capi.HALF, 193, 2252, 4521, True, True, "64x128 waves=4 split=3"),
+    (capi.FP8E4M3, 816, 2320, 1248, True, True, "64x128 waves=4 split=1"),
+    (capi.FP8E5M2, 1155, 1623, 426, False, True, "64x128 waves=4 split=1"),
+    (capi.INT8, 824, 2329, 285, True, False, "64x128 waves=4 split=1"),
+    (capi.BFLOAT16, 1399, 1572, 273, True, True, "128x64 waves=4 split=1"),
+    (capi.HALF, 1626, 300, 4271, True, False, "128x64 waves=4 split=3"),
+    (capi.BFLOAT16, 464, 1072, 4368, False, True, "128x64 waves=4 split=3"),
+    (capi.FP8E4M3, 847, 1534, 350, False, False, "128x64 waves=4 split=1"),
+    (capi.INT8, 466, 2978, 208, True, True, "128x64 waves=4 split=1"),
+]
+
+
+@pytest.mark.parametrize("dtype,m,n,k,ta,tb,route", HALF_WIDE)
+def test_half_wide_tiles(ctx, dtype, m, n, k, ta, tb, route):
+    a, b = make_operand(86, 0, m, k, dtype, ta), make_operand(86, 1, k, n, dtype, tb)
+    got, name, odt = run(ctx, a, b)
+    assert name.endswith(route), name
+    check(got, ref_matmul(a, b), odt, name)
+
+
+# whole 16-byte chunks of K, and any K where neither operand lies along it: the tiled GEMM (its
+# other tiles and split reductions: test_cut_slice_after_garbage), but for the last row, whose few
+# tiles are staged
 @pytest.mark.parametrize("dtype,k16", [(capi.BFLOAT16, 8), (capi.HALF, 8), (capi.INT8, 16), (capi.FP8E5M2, 16)])
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("m,n,slices,rest", [(3072, 2064, 8, 1), (2064, 2064, 7, 7), (2576, 2592, 3, 3), (256, 4096, 33, 5)])
@@ -69,7 +99,7 @@ def test_cut_slices(ctx, dtype, k16, ta, tb, m, n, slices, rest):
     k = slices * 8 * k16 + rest * k16 + (3 if ta and not tb else 0)
     a, b = make_operand(83, 0, m, k, dtype, ta), make_operand(83, 1, k, n, dtype, tb)
     got, name, odt = run(ctx, a, b)
-    assert name.startswith("gemm_mfma"), name
+    assert name.endswith("256x128 waves=8 split=1" if m > 256 else "64x64 waves=8 split=1"), name
     check(got, ref_matmul(a, b), odt, name)
 
 
@@ -136,9 +166,18 @@ def test_infinities_in_front_of_a_cut(ctx, m, n, k, ta, tb):
 
 
 @pytest.mark.parametrize("dtype", [capi.BFLOAT16, capi.HALF])
-@pytest.mark.parametrize("m,n,k,batch", [(130, 250, 1003, 1), (140, 140, 6001, 1), (90, 200, 700, 5), (700, 1300, 1500, 1)])
-def test_fused_chains(ctx, dtype, m, n, k, batch):
-    # a column operand alone (requested early), and with a full one; also behind a split K
+@pytest.mark.parametrize("m,n,k,batch,route", [
+    # the direct kernels
+    (130, 250, 1003, 1, "gemm_direct 16x16"), (140, 140, 6001, 1, "split=4"), (90, 200, 700, 5, "gemm_direct"),
+    # staged tiles of every size, whole, in parts, of a batch
+    (700, 1300, 1500, 1, "64x64 waves=8 split=1"), (576, 2402, 263, 1, "64x64 waves=4 split=1"),
+    (205, 216, 3456, 1, "64x64 waves=4 split=11"), (1368, 69, 4977, 1, "64x64 waves=8 split=5"),
+    (354, 589, 273, 3, "64x64 waves=8 split=1"), (77, 400, 5771, 3, "64x64 waves=8 split=6"),
+    (778, 2381, 446, 1, "64x128 waves=4 split=1"), (267, 610, 4957, 3, "64x128 waves=4 split=3"),
+    (330, 1138, 339, 5, "128x64 waves=4 split=1"), (207, 1430, 5666, 1, "128x64 waves=4 split=5"),
+    (1212, 883, 241, 3, "128x128 waves=4 split=1"), (866, 1248, 2483, 1, "128x128 waves=4 split=3")])
+def test_fused_chains(ctx, dtype, m, n, k, batch, route):
+    # a column operand alone (requested early), and with a full one
     lead = [batch] if batch > 1 else []
     a = make_operand(84, 0, m, k, dtype, False, batch=batch if batch > 1 else None)
     b = make_operand(84, 1, k, n, dtype, True, batch=batch if batch > 1 else None)
@@ -153,6 +192,7 @@ def test_fused_chains(ctx, dtype, m, n, k, batch):
             ([add, gelu], [bias], oracle.pointwise(capi.PW["GELU_FWD"], [product + bias.logical()])),
             ([scale, add, mul], [bias, full], (0.25 * product + bias.logical()) * full.logical())):
         got, name, odt = run(ctx, a, b, ops, tensors)
+        assert route in name, name
         assert_close(got, ref, dtype, name)
 
 
