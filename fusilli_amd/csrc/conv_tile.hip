@@ -51,14 +51,12 @@ double conv_tile_us(const ConvTileTimes &f, const ConvTileArgs &g, int split, bo
 ConvTilePlan conv_tile_plan(const ConvTileArgs &g, bool dgrad, bool fused, size_t room) {
   static const ConvTileTimes kForward[] = {
       {64, 64, 0, 3, 3.854, 0.348, 0.245, 1.219, 1.743, 0.413, 1.579, 0.466},
-      {64, 64, 1, 2, 3.783, 0.339, 0.243, 2.364, 1.934, 0.328, 1.123, 0.973},
       {64, 64, 2, 2, 0.944, 0.154, 0.489, 4.558, 1.887, 0.627, 0.226, 1.490},
       {64, 128, 1, 2, 4.688, 0.422, 0.354, 2.733, 0, 0.558, 0.568, 2.349},
       {128, 64, 1, 2, 4.363, 0.573, 0.396, 3.187, 0.070, 0.618, 0.762, 2.043},
       {128, 128, 1, 1, 5.704, 0.529, 0.771, 3.527, 0, 0.237, 0, 3.915}};
   static const ConvTileTimes kGradient[] = {
       {64, 64, 0, 3, 4.279, 0.381, 0.257, 0.901, 1.513, 0.529, 0, 0},
-      {64, 64, 1, 2, 3.689, 0.377, 0.272, 2.216, 2.291, 0.344, 0, 0},
       {64, 64, 2, 2, 1.312, 0.568, 0.568, 4.618, 1.438, 0.745, 0, 0},
       {64, 128, 1, 2, 4.091, 0.540, 0.417, 2.946, 0.771, 0.648, 0, 0},
       {128, 64, 1, 2, 3.843, 0.619, 0.431, 2.948, 1.101, 0.608, 0, 0},

@@ -245,9 +245,7 @@ int conv_tile_shape(fhip_ctx *ctx, const ConvTilePlan &p, const ConvTileArgsOf<P
     return conv_tile_go<KIND, DGRAD, PARTS, 4, 1, 2, 1>(ctx, g);
   if (p.teams == 2)
     return conv_tile_go<KIND, DGRAD, PARTS, 2, 1, 1, 2>(ctx, g);
-  if (p.teams == 0)
-    return conv_tile_go<KIND, DGRAD, PARTS, 2, 1, 1, 1, true>(ctx, g);
-  return conv_tile_go<KIND, DGRAD, PARTS, 4, 1, 1, 1>(ctx, g);
+  return conv_tile_go<KIND, DGRAD, PARTS, 2, 1, 1, 1, true>(ctx, g);
 }
 
 template <int KIND> int conv_tile_kind(fhip_ctx *ctx, bool dgrad, const ConvTilePlan &p, const ConvTileArgs &g) {
