@@ -103,6 +103,19 @@ def test_cut_slices(ctx, dtype, k16, ta, tb, m, n, slices, rest):
     check(got, ref_matmul(a, b), odt, name)
 
 
+# one whole slice of K: the tiled GEMM, also in batches (the direct kernels take up to seven times as long)
+@pytest.mark.parametrize("dtype,m,n,k,batch", [
+    (capi.BFLOAT16, 1536, 448, 64, 4), (capi.HALF, 2048, 1160, 64, 1), (capi.FP8E4M3, 640, 2240, 128, 1),
+    (capi.INT8, 256, 400, 128, 3)])
+@pytest.mark.parametrize("ta,tb", [(False, True), (True, False)])
+def test_one_whole_slice(ctx, dtype, m, n, k, batch, ta, tb):
+    of = batch if batch > 1 else None
+    a, b = make_operand(90, 0, m, k, dtype, ta, batch=of), make_operand(90, 1, k, n, dtype, tb, batch=of)
+    got, name, odt = run(ctx, a, b)
+    assert name.startswith("gemm_mfma") and name.endswith("waves=8 split=1"), name
+    check(got, ref_matmul(a, b), odt, name)
+
+
 # every tile of the tiled GEMM, operands along M / N (whole K-rows are masked) and along K, split
 # reductions whose last part is the shorter one, a slice of a few values
 CUT = [
