@@ -305,7 +305,8 @@ __device__ __forceinline__ void rw_moments(const float (&v)[RwVec<T>::kN], int l
   for (int k = 0; k < N; ++k)
     d[k] = v[k] - mean;
   const double e = (double)mean - pivot, n = (double)live, rest = rw_tree<T, 1>(d, 0.f, live);
-  s1 += n * (double)mean + rest;
+  // (around an infinite mean `rest` is NaN, where the row's mean is that infinity)
+  s1 += __builtin_isfinite(sum) ? n * (double)mean + rest : (double)sum;
   s2 += rw_tree<T, 2>(d, 0.f, live) + e * (n * e + 2. * rest);
 }
 

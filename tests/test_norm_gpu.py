@@ -442,3 +442,22 @@ def test_segments_far_from_zero(ctx, dtype, rows, cols, at):
     # f32 arithmetic on deviations, one rounding to the result's type
     y = (v - m[:, None]) * r[:, None] * s.logical() + b.logical()
     assert np.all(np.abs(out.logical() - y) <= 2.0 ** {capi.FLOAT: -20, capi.HALF: -10, capi.BFLOAT16: -7}[dtype] * (1 + np.abs(y)))
+
+
+@pytest.mark.parametrize("dtype", [capi.HALF, capi.BFLOAT16, capi.FLOAT])
+def test_segments_with_infinities(ctx, dtype):
+    # a row's mean is its infinity wherever that lies (first element, inside a vector, in the
+    # last one, which is not whole), NaN with both of them; other rows are not touched
+    cols = 65541
+    x = rand(45, 0, [6, cols], mean=0.5)
+    x[0, 0], x[1, 30003], x[2, -1], x[3, 5], x[3, 40000], x[4, 777] = np.inf, -np.inf, np.inf, np.inf, -np.inf, np.nan
+    x = HT.from_logical(x, dtype)
+    s = HT.from_logical(rand(45, 1, [1, cols], mean=1.0, std=0.1), dtype)
+    b = HT.from_logical(rand(45, 2, [1, cols]), dtype)
+    out, mean, rstd = run_norm(ctx, x, s, b, eps=1e-5, layernorm=True, stats=True)
+    assert ctx.last_kernel().startswith("rownorm_walk segments="), ctx.last_kernel()
+    assert np.array_equal(mean.logical()[:5], np.float32([np.inf, -np.inf, np.inf, np.nan, np.nan]), equal_nan=True)
+    assert np.all(np.isnan(rstd.logical()[:5])) and np.all(np.isnan(out.logical()[:5]))
+    y, m, r = oracle.layernorm(x.logical()[5:], s.logical(), b.logical(), 1e-5)
+    assert_close(mean.logical()[5:], m.reshape(-1), capi.FLOAT, "mean")
+    assert_close(out.logical()[5:], y, dtype, "the row without")
