@@ -318,25 +318,26 @@ __global__ __launch_bounds__(kRwThreads) void rownorm_walk_sums_kernel(RowWalkAr
   const int64_t row = blockIdx.y, lo = blockIdx.x * g.seg;
   const int64_t hi = lo + g.seg < g.n.inner ? lo + g.seg : g.n.inner;
   const T *xr = (const T *)g.n.x + row * g.n.x_row_stride;
-  const double pivot = LAYER ? (double)(float)xr[lo] : 0.;
   double s1 = 0., s2 = 0.;
-  auto add = [&](const typename V::loose &raw, int live) {
-    float v[N];
-    V::widen(raw, v);
-    if constexpr (LAYER)
+  if constexpr (LAYER) {
+    const double pivot = (double)(float)xr[lo];
+    auto add = [&](const typename V::loose &raw, int live) {
+      float v[N];
+      V::widen(raw, v);
       rw_moments<T>(v, live, pivot, s1, s2);
-    else
-      s2 += rw_tree<T, 2>(v, 0.f, live);
-  };
-  int64_t i = lo + (int64_t)threadIdx.x * N;
-  for (; i + kStep + N <= hi; i += 2 * kStep) { // (two loads in flight)
-    const typename V::loose a = V::load_raw(xr + i, N), b = V::load_raw(xr + i + kStep, N);
-    add(a, N);
-    add(b, N);
-  }
-  for (; i < hi; i += kStep) {
-    const int live = hi - i < N ? (int)(hi - i) : N;
-    add(V::load_raw(xr + i, live), live);
+    };
+    int64_t i = lo + (int64_t)threadIdx.x * N;
+    for (; i + kStep + N <= hi; i += 2 * kStep) { // (two loads in flight)
+      const typename V::loose a = V::load_raw(xr + i, N), b = V::load_raw(xr + i + kStep, N);
+      add(a, N);
+      add(b, N);
+    }
+    for (; i < hi; i += kStep) {
+      const int live = hi - i < N ? (int)(hi - i) : N;
+      add(V::load_raw(xr + i, live), live);
+    }
+  } else {
+    s2 = rw_walk<T, 2>(xr, 0.f, lo, hi, threadIdx.x, kRwThreads);
   }
   s1 = LAYER ? rw_wave_sum(s1) : 0.;
   s2 = rw_wave_sum(s2);
@@ -351,7 +352,8 @@ __global__ __launch_bounds__(kRwThreads) void rownorm_walk_sums_kernel(RowWalkAr
       s2 += lds[w].y;
     }
     if constexpr (LAYER) {
-      const double n = (double)(hi - lo), d = rw_centre(g, (int)blockIdx.x, s1) - pivot;
+      const double pivot = (double)(float)xr[lo], n = (double)(hi - lo);
+      const double d = rw_centre(g, (int)blockIdx.x, s1) - pivot;
       s2 += d * (n * d - 2. * (s1 - n * pivot));
     }
     ((rw_pair *)g.partial)[row * g.splits + blockIdx.x] = rw_pair{s1, s2};
