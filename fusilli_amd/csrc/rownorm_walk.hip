@@ -472,11 +472,19 @@ template <typename T> void rw_launch_rows(hipStream_t stream, const RowNormArgs 
 
 // Segments that a row is cut into, 1: none.  Rows of more than four vectors per thread of a
 // workgroup are cut into segments of two vectors per thread, 256 at most (a pair per thread of
-// the second launch), unless there are so many rows that whole ones, which take one launch and
-// read X from memory once, keep up (bf16 8000 x 16387 LayerNorm 196 us whole / 204 in
-// segments, f16 1500 x 40001 80 / 71; RMSNorm, which walks a row twice and not three times,
-// bf16 600 x 16387 19.4 / 17.4, f32 700 x 60001 134 / 87, 1200 x 30001 74 / 71, bf16 3000 x
-// 20001 63 / 65).  Segments' sums need the context's scratch.
+// the second launch), unless whole ones, which take one launch and read X from memory once,
+// keep up (us, whole / cut):
+//   * more than sixteen rows (RMSNorm, which walks a row twice and not three times: four) per
+//     compute unit: bf16 8000 x 16387 LayerNorm 196 / 204; RMSNorm bf16 3000 x 20001 63 / 65, f32
+//     1200 x 30001 74 / 71, where many more walk as fast cut;
+//   * LayerNorm in three segments, from 1.4 rows per unit on: f16 387 x 8818 10.6 / 11.7, bf16
+//     1428 x 9324 19.1 / 24.7, f32 801 x 4463 9.9 / 13.4 (16 bits, 330 x 8510 11.5 / 10.2); in four, as
+//     long as all rows run at once, eight workgroups to a unit: bf16 463 x 15564 15.7 / 14.8, 608 x 14156
+//     16.3 / 17.3, 1381 x 12394 24.4 / 29.1, f32 1122 x 6187 17.7 / 21.2, 2234 x 6733 40.6 / 37.2; in five
+//     854 x 17783 29.9 / 26.7;
+//   * RMSNorm with more rows than two thirds of a unit's per segment: f32 671 x 4578 9.7 / 11.1, bf16
+//     979 x 11162 15.9 / 17.6, 789 x 12434 16.3 / 17.4; but 543 x 13412 14.8 / 14.2, 713 x 19630 22.7 / 20.6.
+// Segments' sums need the context's scratch.
 int fhip_norm_walk_splits(fhip_ctx *ctx, int dtype, int64_t rows, int64_t inner, bool many_pay) {
   const int64_t vec = 16 / (int64_t)fhip_dtype_size(dtype);
   const int64_t cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
@@ -484,7 +492,10 @@ int fhip_norm_walk_splits(fhip_ctx *ctx, int dtype, int64_t rows, int64_t inner,
   int64_t splits = (inner + unit - 1) / unit;
   splits = splits < kRwThreads ? splits : kRwThreads;
   const bool many = rows >= (many_pay ? 16 : 4) * cus && inner <= kRwResident * vec;
-  if (inner <= 2 * unit || many || rows > 65535 ||
+  const bool few = many_pay ? (splits == 3 && 10 * rows >= 14 * cus) ||
+                                  (splits == 4 && 10 * rows >= 21 * cus && rows <= 8 * cus)
+                            : 3 * rows >= 2 * cus * splits;
+  if (inner <= 2 * unit || many || few || rows > 65535 ||
       !fhip_ctx_scratch_ready(ctx, (size_t)(2 * rows * splits) * sizeof(double)))
     return 1;
   return (int)splits;

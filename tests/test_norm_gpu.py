@@ -363,6 +363,29 @@ def test_norm_rows_of_any_length_vs_oracle(ctx, dtype, rows, cols, layernorm):
     assert_close(out.logical(), y, dtype, f"{rows} x {cols}")
 
 
+@pytest.mark.parametrize("layernorm,rows,segments,cut", [
+    # both sides of every line between whole rows and segments
+    (True, 358, 3, True), (True, 359, 3, False), (True, 537, 4, True), (True, 538, 4, False),
+    (True, 2048, 4, False), (True, 2049, 4, True), (True, 900, 5, True),
+    (False, 511, 3, True), (False, 512, 3, False), (False, 853, 5, True), (False, 854, 5, False)])
+@pytest.mark.parametrize("dtype", [capi.BFLOAT16, capi.FLOAT])
+def test_norm_rows_whole_or_in_segments(ctx, dtype, layernorm, rows, segments, cut):
+    cols = (segments - 1) * 512 * (4 if dtype == capi.FLOAT else 8) + 9
+    x = HT.from_logical(rand(46, 0, [rows, cols], mean=0.5, std=2.0), dtype)
+    s = HT.from_logical(rand(46, 1, [1, cols], mean=1.0, std=0.1), dtype)
+    if layernorm:
+        b = HT.from_logical(rand(46, 2, [1, cols]), dtype)
+        out, mean, rstd = run_norm(ctx, x, s, b, eps=1e-5, layernorm=True, stats=True)
+        y, m, r = oracle.layernorm(x.logical(), s.logical(), b.logical(), 1e-5)
+        assert_close(mean.logical(), m.reshape(-1), capi.FLOAT, "mean")
+        assert_close(rstd.logical(), r.reshape(-1), capi.FLOAT, "rstd")
+    else:
+        out = run_norm(ctx, x, s, None, eps=1e-6)
+        y = oracle.rmsnorm(x.logical(), s.logical(), 1e-6)
+    assert ctx.last_kernel() == f"rownorm_walk {f'segments={segments}' if cut else 'waves_per_row=4'}", ctx.last_kernel()
+    assert_close(out.logical(), y, dtype, f"{rows} x {cols}")
+
+
 @pytest.mark.parametrize("dtype", [capi.HALF, capi.FLOAT])
 @pytest.mark.parametrize("rows,cols", [(3000, 65), (2000, 1003), (1000, 3001), (300, 16387)])
 def test_means_of_walked_rows_are_rounded_once(ctx, dtype, rows, cols):
