@@ -1098,6 +1098,34 @@ static int cf_allow_lds(fhip_ctx *ctx, const void *kernel, FhipOncePerDevice &co
   return 0;
 }
 
+// conv_few_dgrad_kernel: bands of DX rows (a multiple of the rows per lane, of equal height) in `g`,
+// workgroups, their wavefronts and LDS; `ok` false where it does not take the problem.
+struct CfLanes {
+  bool ok = false;
+  int64_t blocks = 0, floats = 0;
+  int waves = 0, pitch = 0;
+};
+static CfLanes cf_dgrad_lanes(fhip_ctx *ctx, CfArgs &g) {
+  CfLanes p;
+  g.quads = (g.W + 3) / 4;
+  const int pairs = (g.H + kCfRows - 1) / kCfRows, most = 64 / g.quads;
+  g.tiles = (pairs + most - 1) / most;
+  g.band = (pairs + g.tiles - 1) / g.tiles * kCfRows;
+  const int span = (g.S + 6) & ~3, rows = g.band + g.R - 1;
+  p.pitch = 4 * g.quads + span - 4;
+  const int64_t filter = (int64_t)g.K * g.R * ((g.S * g.C + 3) & ~3);
+  p.blocks = (int64_t)g.N * g.tiles;
+  // a quarter of the output channels per wavefront, an eighth where that leaves
+  // fewer than two wavefronts per SIMD
+  const int64_t cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
+  p.waves = p.blocks * 4 < 8 * cus ? 8 : 4;
+  p.floats = filter + (int64_t)p.waves * rows * p.pitch;
+  const int64_t meet = (int64_t)p.waves * kCfRows * 256 * g.C;
+  p.floats = p.floats < meet ? meet : p.floats;
+  p.ok = (int64_t)rows * p.pitch <= 64 * kCfStage && p.floats * 4 <= kCfLds && p.blocks < (1ll << 23);
+  return p;
+}
+
 static int cf_dgrad_products(fhip_ctx *ctx, const fhip_conv_desc *d, CfArgs g, const void *dy, const void *w,
                              void *dx, bool *handled) {
   const int rs = g.R * g.S;
@@ -1172,6 +1200,24 @@ static int cf_dgrad_products(fhip_ctx *ctx, const fhip_conv_desc *d, CfArgs g, c
   if (passes > 1 && parts == 1 &&
       (g.K < 32 || (wide && (int64_t)g.N * g.H * g.W > 110 * cus)))
     return 0;
+  // In f32 conv_few_dgrad_kernel takes over where a compute unit has much work here (rounds of
+  // workgroups times wavefronts of each): its bands do not overlap, and up to two workgroups of eight
+  // wavefronts to a unit it takes one round.  us, there / here, 5 x 5 over one channel: N22, 24 x 24 -> 16
+  // 7.6 / 6.2, N69, 33 x 33 8.2 / 10.1, N101, 62 x 62 16.9 / 28.5; N67, 48 x 48 -> 32 without pad 15.9 / 12.8,
+  // N120, 39 x 39 16.5 / 19.6; N50, 33 x 33 -> 64 18.4 / 15.8, N78, 45 x 45 25.8 / 31.1, N68, 55 x 55 27.8 /
+  // 42.8.  3 x 3: N62 3 -> 64, 62 x 62 29.4 / 44.3, N62 4 -> 16, 60 x 60 13.8 / 17.8, N106 3 -> 16, 61 x 61 18.8 /
+  // 24.3, N113 3 -> 64, 60 x 60 51.8 / 61.2, but N104 4 -> 16, 38 x 38 13.7 / 13.4, N120 3 -> 32, 49 x 49 29.9 / 24.5.
+  // (16 bits: 3 x 3 always faster here, 5 x 5 from 32 channels on 1.4 to 3.9 times, -> 16 as often up to a
+  // fifth slower as faster.)
+  if (wide && passes == 1) {
+    const int64_t work = (blocks * tiles_w + cus - 1) / cus * units;
+    CfArgs other = g;
+    const CfLanes lanes = cf_dgrad_lanes(ctx, other);
+    const bool lead = g.K > 16 && g.K <= 32; // (32 channels are one block of registers here)
+    const int64_t most = g.S == 5 ? (lead ? 16 : 8) : lanes.waves == 8 ? 16 : lead ? 36 : 24;
+    if (lanes.ok && work > most)
+      return 0;
+  }
   *handled = true;
   fhip_note_kernel(ctx, "conv_few dgrad products channels=%d", g.C);
   int status = 0;
@@ -1225,24 +1271,10 @@ int fhip_few_conv_dgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy, 
   const int status = cf_dgrad_products(ctx, d, g, dy, w, dx, handled);
   if (status != 0 || *handled)
     return status;
-  g.quads = (g.W + 3) / 4;
-  // (a multiple of the rows per lane, of equal height)
-  const int pairs = (g.H + kCfRows - 1) / kCfRows, most = 64 / g.quads;
-  g.tiles = (pairs + most - 1) / most;
-  g.band = (pairs + g.tiles - 1) / g.tiles * kCfRows;
-  const int span = (g.S + 6) & ~3, pitch = 4 * g.quads + span - 4, rows = g.band + g.R - 1;
-  const int64_t filter = (int64_t)g.K * g.R * ((g.S * g.C + 3) & ~3);
-  const int64_t blocks = (int64_t)g.N * g.tiles;
-  // a quarter of the output channels per wavefront, an eighth where that leaves
-  // fewer than two wavefronts per SIMD
-  const int64_t cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
-  const int waves = blocks * 4 < 8 * cus ? 8 : 4;
-  int64_t floats = filter + (int64_t)waves * rows * pitch;
-  const int64_t meet = (int64_t)waves * kCfRows * 256 * g.C;
-  floats = floats < meet ? meet : floats;
-  if ((int64_t)rows * pitch > 64 * kCfStage || floats * 4 > kCfLds || blocks >= (1ll << 23))
+  const CfLanes lanes = cf_dgrad_lanes(ctx, g);
+  if (!lanes.ok)
     return 0;
-  g.lw_magic = cf_magic(pitch);
+  g.lw_magic = cf_magic(lanes.pitch);
   *handled = true;
   fhip_note_kernel(ctx, "conv_few dgrad channels=%d", g.C);
   cf_by_type(d->x.dtype, [&](auto t) {
@@ -1250,7 +1282,7 @@ int fhip_few_conv_dgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy, 
     auto with = [&](auto cc) {
       constexpr int C = decltype(cc)::value;
       auto kernel = g.S == 3 ? conv_few_dgrad_kernel<T, C, 3> : conv_few_dgrad_kernel<T, C, 5>;
-      hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(waves * 64), (size_t)floats * 4,
+      hipLaunchKernelGGL(kernel, dim3((unsigned)lanes.blocks), dim3(lanes.waves * 64), (size_t)lanes.floats * 4,
                          ctx->stream, g, (const T *)dy, (const T *)w, (T *)dx);
     };
     if (g.C == 1)

@@ -122,6 +122,14 @@ def test_few_tiles_take_fewer_channels_each(ctx, n, forward, gradient):
     ([1, 1, 30, 200], [24, 1, 5, 5], [0, 1], True, "products"),   # bands cut in columns
     ([2, 1, 3, 250], [8, 1, 2, 3], [3, 3], True, "products"),     # DY beside the image
     ([2, 3, 20, 18], [16, 3, 3, 3], [1, 1], False, "products"),   # rows of DY with gaps
+    # both sides of the line for much work per compute unit: vector instructions (f32)
+    ([69, 1, 33, 33], [16, 1, 5, 5], [2, 2], True, None),
+    ([67, 1, 48, 48], [32, 1, 5, 5], [0, 0], True, "products"),
+    ([120, 1, 39, 39], [32, 1, 5, 5], [2, 2], True, None),
+    ([50, 1, 63, 63], [16, 1, 3, 3], [1, 1], True, None),
+    ([104, 4, 38, 38], [16, 4, 3, 3], [1, 1], True, "products"),
+    ([106, 3, 61, 61], [16, 3, 3, 3], [1, 1], True, None),
+    ([69, 1, 33, 33], [460, 1, 5, 5], [2, 2], True, "products"),  # a filter that LDS does not hold there
 ])
 def test_data_gradient_products_first(ctx, x, w, pad, dense, kind, dtype):
     geom = (pad, [1, 1], [1, 1])
