@@ -1001,8 +1001,8 @@ __global__ void conv_flip_filter_kernel(FlipArgs a, const uint16_t *src,
 } // namespace
 
 // Scratch of the entry point that allocates nothing (fhip_conv_dgrad_static):
-// the mirrored filter and, with strides above one, DY spread over its zero
-// grid live here instead of in caller workspace.  Every device that loads the
+// the mirrored filter, DY spread over its zero grid and the partial sums of gathered
+// tiles live here instead of in caller workspace.  Every device that loads the
 // library holds its own copy at its own address until the process ends; the
 // address is resolved once per device by fhip_conv_dgrad_static_setup and kept
 // in the context.  In host code the array's name is only a handle for that
@@ -1037,6 +1037,7 @@ static void dgrad_note(fhip_ctx *ctx, const char *prefix) {
 bool fhip_fast_conv_dgrad_applicable(const fhip_conv_desc *d,
                                      size_t *workspace_bytes, bool allow_scratch) {
   const DgradPlan p = make_dgrad_plan(d, allow_scratch);
+  // (the zero grid also where gathered tiles would do without: pointers off 16 bytes need it)
   if (workspace_bytes)
     *workspace_bytes = p.ok ? p.filter_bytes + p.spread_bytes : 0;
   return p.ok;

@@ -276,8 +276,11 @@ int fhip_conv_fprop(fhip_ctx *ctx, const fhip_conv_desc *d, const void *x,
  *      gradient's dtype.  fhip_conv_dgrad_supported returns 2 where the MFMA
  *      kernel takes the problem (16-bit channels-last tensors, one group):
  *      it then needs fhip_conv_dgrad_workspace_size bytes of 256-byte aligned
- *      workspace (a mirrored copy of the filter; with strides above one also
- *      DY spread over a zero grid) and fails without them.
+ *      workspace and fails without them: room for a mirrored copy of the
+ *      filter and, with strides above one, for DY spread over a zero grid.
+ *      The size follows from the descriptor alone; the kernels that read DY
+ *      and W as they lie (most strided gradients with channels in multiples
+ *      of 8 and 16-byte aligned tensors) leave that room untouched.
  *      fhip_conv_wgrad_supported returns 2 for 16-bit channels-last X and DY
  *      of one group with C and K multiples of 8, equal strides, no dilation
  *      along W and S * C >= 128 (MFMA tiles gathered from X and DY as they
@@ -293,13 +296,14 @@ int fhip_conv_dgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy,
 /* fhip_conv_dgrad without any allocation and without caller workspace.  It has
  * no counterpart in the reference; it exists for callers that cannot allocate
  * device memory around the call (code under HIP graph capture, tight serving
- * loops, harnesses that forbid hipMalloc).  The mirrored filter (and DY's zero
- * grid for strides above one) live in a per-device static array of
+ * loops, harnesses that forbid hipMalloc).  What fhip_conv_dgrad keeps in its
+ * workspace, and the partial sums of split reductions over tiles gathered
+ * from DY and W as they lie, live in a per-device static array of
  * FHIP_CONV_DGRAD_STATIC_MAX_BYTES inside the library; descriptors whose
  * fhip_conv_dgrad_workspace_size exceeds that fail with a message.  It plans
  * without the context's growable scratch: descriptors that fhip_conv_dgrad
- * runs on zero-padded channel copies or with a split reduction take the
- * direct (slower) kernels here, 1 x 1 filters at unit stride (which
+ * runs on zero-padded channel copies, or with a split reduction over the
+ * mirrored filter, take other (slower) kernels here, 1 x 1 filters at unit stride (which
  * fhip_conv_dgrad hands to the matrix-product kernels, whose planner may use
  * the scratch) stay on the convolution kernel, and the results of both may
  * differ from fhip_conv_dgrad's in the last bit (another summation order);
