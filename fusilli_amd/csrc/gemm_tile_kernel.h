@@ -17,10 +17,10 @@
 // behind K, M or N is masked there.  (Fragments straight from memory, no LDS, every wavefront
 // with slices of its own, are no faster on aligned rows and 3 to 10 times slower on odd ones.)
 //
-// us, before -> now: bf16 1024^3 13.1 -> 7.9 (tiled GEMM), with bias and GELU 19.9 -> 10.2; f16 777
-// x 1400 x 1000 with both 18.8 -> 16.8 (direct kernel); bf16 132 x 2632 x 3392 43 -> 16; odd
-// rows, bf16 4095 x 8191 x 2001 390 -> 233 (128 x 128 tiles, 575 TFLOP/s), 1177 x 2223 x 2160
-// 54.7 -> 26.6.
+// us, before -> now: bf16 1024^3 11.8 -> 8.0 (tiled GEMM), with bias and GELU 18.8 -> 9.8; f16 777
+// x 1400 x 1000 with both 18.9 -> 16.2 (direct kernel); bf16 132 x 2632 x 3392 35.8 -> 14.6; odd
+// rows, bf16 4095 x 8191 x 2001 344 -> 228 (128 x 128 tiles, 589 TFLOP/s), 1177 x 2223 x 2160
+// 44.2 -> 35.1, with B along K 55.1 -> 33.7.
 //
 //   K-contiguous operand: rows of 128 bytes, 16 bytes a lane, chunks permuted as in
 //   gemm_kernel.h.  In the last slice a chunk ends at K and is shifted down, so zeros

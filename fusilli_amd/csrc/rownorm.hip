@@ -62,11 +62,11 @@ bool zero_inner_strides(const fhip_tensor_desc &x, const int64_t *strides) {
 // Whether a row that sixteen wavefronts could hold in sixteen vectors per lane is better cut
 // into segments (rownorm_walk.hip).  One workgroup to a row leaves the chip idle under few
 // rows, and sixteen vectors with their scale and bias leave a lane no registers for loads in
-// flight: whole / cut, us, bf16 4 x 131072 LayerNorm 31.4 / 6.9, 256 x 65544 37 / 26, 2500 x
-// 70000 320 / 237, RMSNorm 337 / 225 (f16 4096 x 65544 RMSNorm 335 / 339).  f32 vectors hold
+// flight: whole / cut, us, bf16 4 x 131072 LayerNorm 30.3 / 6.1, 256 x 65544 37 / 25, 2500 x
+// 70000 321 / 244, RMSNorm 337 / 222 (f16 4096 x 65544 RMSNorm 335 / 339).  f32 vectors hold
 // half as many values to finish, and RMSNorm has no bias to hold: LayerNorm 4 x 32772 12.1 /
-// 6.9, 128 x 32772 15.9 / 13.8, 256 x 32772 21.1 / 22.5, 511 x 65536 73 / 62; RMSNorm 4 x
-// 32772 5.9 / 6.9, 10 x 45000 8.1 / 6.9, 64 x 65536 12.2 / 12.0, 128 x 65536 13.0 / 19.8.
+// 6.2, 128 x 32772 15.9 / 13.2, 256 x 32772 21.1 / 22.5, 511 x 65536 74 / 65; RMSNorm 4 x
+// 32772 5.9 / 6.9, 10 x 45000 8.1 / 6.9, 64 x 65536 12.2 / 11.0, 128 x 65536 13.0 / 19.8.
 bool cut_pays(const fhip_norm_desc *d, int64_t rows, int64_t inner, int chunks, fhip_ctx *ctx) {
   if (chunks != 16 || fhip_knobs().rownorm_shape_w)
     return false;

@@ -15,9 +15,9 @@
 //
 // bf16 16000 x 1003 RMSNorm + MUL: 207 us (generic) -> 20.3 (3.2 TB/s); f16 LayerNorm 9000 x
 // 3001: 442 -> 49 (2.2 TB/s).  (Unrolling the walk four times is slower: 49 -> 55.6.)
-// Segments: bf16 LayerNorm 16 x 262144 9.0 us, of which two launches that do next to nothing
-// take 7; 600 x 300000 329 -> 242 (segments of eight vectors per thread); whole rows, bf16
-// LayerNorm 204 x 9335 14.8 -> 9.0.
+// Segments (recorded into a graph): bf16 LayerNorm 16 x 262144 9.8 -> 9.1 us, of which two launches
+// that do next to nothing take 7; 600 x 300000 330 -> 246 (segments of eight vectors per thread),
+// 204 x 9335 12.9 -> 9.0.
 //
 // Reference semantics: aten.rms_norm / aten.layer_norm over all dims except
 // dim 0 (reference support/asm_emitter.h:1592-1626, 1427-1503;
