@@ -137,20 +137,35 @@ __global__ __launch_bounds__(kBnThreads) void bn_stats_kernel(BnFastArgs g) {
 // sums w, w + 64, ... and meet through a fixed tree (lanes of a wavefront by
 // cross-lane moves, the four wavefronts in LDS), the same for every run.
 constexpr int kBnFinCh = 4;
+// (the other types' code out of the way: the launch is a few workgroups that wait for theirs)
+__device__ __forceinline__ float bn_load(const void *p, int dt, int c) {
+  return __builtin_expect(dt == FHIP_FLOAT, 1) ? ((const float *)p)[c] : fhip_load<float>(p, dt, c);
+}
 template <typename T>
 __global__ __launch_bounds__(kBnThreads) void bn_finalize_kernel(BnFastArgs g) {
   __shared__ float red[kBnThreads / 64][kBnFinCh][2];
   const int ci = threadIdx.x % kBnFinCh, wl = threadIdx.x / kBnFinCh;
   const int c = blockIdx.x * kBnFinCh + ci;
   const bool live = c < g.C;
-  float s1 = 0.f, s2 = 0.f;
+  float s1 = 0.f, s2 = 0.f, pivot = 0.f, sc = 1.f, bi = 0.f;
+  if (wl == 0 && live) { // (requested with the sums)
+    if (g.training)
+      pivot = (float)((const T *)g.x)[c];
+    if (g.scale)
+      sc = bn_load(g.scale, g.scale_dt, c);
+    if (g.bias)
+      bi = bn_load(g.bias, g.bias_dt, c);
+  }
   if (g.training) {
     if (live) {
-#pragma unroll 8
-      for (int w = wl; w < g.nwg; w += kBnThreads / kBnFinCh) {
-        s1 += g.partial[(int64_t)w * 2 * g.C + c];
-        s2 += g.partial[(int64_t)w * 2 * g.C + g.C + c];
-      }
+      const float *p = g.partial + c;
+      fhip_for_parts<8>(
+          wl, kBnThreads / kBnFinCh, g.nwg,
+          [&](int w) { return make_float2(p[(int64_t)w * 2 * g.C], p[(int64_t)w * 2 * g.C + g.C]); },
+          [&](float2 v, bool in) {
+            s1 = in ? s1 + v.x : s1;
+            s2 = in ? s2 + v.y : s2;
+          });
     }
     // lanes l, l ^ 4, l ^ 8, ... hold the same channel
 #pragma unroll
@@ -176,19 +191,22 @@ __global__ __launch_bounds__(kBnThreads) void bn_finalize_kernel(BnFastArgs g) {
     }
     const float n = (float)g.rows;
     const float m1 = s1 / n;
-    const float pivot = (float)((const T *)g.x)[c];
     mean = pivot + m1;
     float var = s2 / n - m1 * m1;
     var = var > 0.f ? var : 0.f;
     inv = 1.0f / sqrtf(var + g.eps);
-    fhip_store<float>(g.saved_mean, g.stats_dt, c, mean);
-    fhip_store<float>(g.saved_inv, g.stats_dt, c, inv);
+    if (__builtin_expect(g.stats_dt == FHIP_FLOAT, 1)) {
+      ((float *)g.saved_mean)[c] = mean;
+      ((float *)g.saved_inv)[c] = inv;
+    } else {
+#pragma clang loop unroll(disable)
+      for (int i = 0; i < 2; ++i)
+        fhip_store<float>(i ? g.saved_inv : g.saved_mean, g.stats_dt, c, i ? inv : mean);
+    }
   } else {
-    mean = fhip_load<float>(g.mean, g.running_dt, c);
-    inv = 1.0f / sqrtf(fhip_load<float>(g.var, g.running_dt, c) + g.eps);
+    mean = bn_load(g.mean, g.running_dt, c);
+    inv = 1.0f / sqrtf(bn_load(g.var, g.running_dt, c) + g.eps);
   }
-  const float sc = g.scale ? fhip_load<float>(g.scale, g.scale_dt, c) : 1.f;
-  const float bi = g.bias ? fhip_load<float>(g.bias, g.bias_dt, c) : 0.f;
   float *ab = g.partial + (int64_t)g.nwg * 2 * g.C;
   ab[c] = inv * sc;
   ab[g.C + c] = mean;

@@ -251,6 +251,44 @@ __host__ __device__ inline uint8_t fhip_float_to_fp8(float f, int ebits) {
 
 #if defined(__HIPCC__)
 
+// Parts first, first + step, ... below `count`, in order, the loads of U of them in flight
+// at a time.  A launch that adds a few dozen partial results takes as long as its dependent
+// rounds of loads (about 0.8 us each, the parts come from the other dies' workgroups), and
+// what a loop of unknown length leaves of its unrolled rounds it loads one by one.  Places past
+// the end load the last part again and are left out by `take(value, live)`.
+template <int U, typename Load, typename Take>
+__device__ __forceinline__ void fhip_for_parts(int first, int step, int count, Load load, Take take) {
+  for (int i = first; i < count; i += U * step) {
+    decltype(load(0)) v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int at = i + u * step;
+      v[u] = load(at < count ? at : count - 1);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      take(v[u], i + u * step < count);
+  }
+}
+
+// The same where `first` and `count` are the whole wavefront's: places past the end load nothing.
+template <int U, typename Load, typename Take>
+__device__ __forceinline__ void fhip_for_uniform_parts(int first, int step, int count, Load load, Take take) {
+  for (int i = first; i < count; i += U * step) {
+    decltype(load(0)) v[U];
+    v[0] = load(i);
+#pragma unroll
+    for (int u = 1; u < U; ++u)
+      if (i + u * step < count)
+        v[u] = load(i + u * step);
+    take(v[0]);
+#pragma unroll
+    for (int u = 1; u < U; ++u)
+      if (i + u * step < count)
+        take(v[u]);
+  }
+}
+
 // Load element `idx` of a tensor of runtime dtype as CT (float or double).
 template <typename CT>
 __device__ __forceinline__ CT fhip_load(const void *p, int dt, int64_t idx) {
@@ -281,6 +319,26 @@ __device__ __forceinline__ CT fhip_load(const void *p, int dt, int64_t idx) {
     return (CT)fhip_fp8_to_float(((const uint8_t *)p)[idx], 4);
   default:
     return (CT)0;
+  }
+}
+
+// N values `step` apart in a tensor of f32, bf16 or f16: one choice for all.  A launch of a few
+// workgroups waits for its code as it does for its data; four calls of fhip_store
+// are 7 KB, of which each executes a line of its own.
+template <int N>
+__device__ __forceinline__ void fhip_store_float(void *p, int dt, int64_t at, int64_t step, const float (&v)[N]) {
+  if (dt == FHIP_FLOAT) {
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+      ((float *)p)[at + n * step] = v[n];
+  } else if (dt == FHIP_BFLOAT16) {
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+      ((__bf16 *)p)[at + n * step] = (__bf16)v[n];
+  } else {
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+      ((_Float16 *)p)[at + n * step] = (_Float16)v[n];
   }
 }
 

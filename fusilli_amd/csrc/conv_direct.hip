@@ -748,9 +748,8 @@ __global__ __launch_bounds__(256) void direct_conv_wgrad_sum_kernel(
   if (lin >= elems)
     return;
   float sum = 0.f;
-#pragma unroll 8
-  for (int r = 0; r < runs; ++r)
-    sum += partial[(int64_t)r * elems + lin];
+  fhip_for_uniform_parts<8>(
+      0, 1, runs, [&](int r) { return partial[(int64_t)r * elems + lin]; }, [&](float v) { sum += v; });
   const int fvol = g.fd[0] * g.fd[1] * g.fd[2];
   const int64_t npairs = (int64_t)g.fC * fvol;
   const int64_t k = lin / npairs;

@@ -472,9 +472,9 @@ __global__ __launch_bounds__(256) void conv_few_wgrad_sum_kernel(CfArgs g, const
   const int64_t e0 = (int64_t)blockIdx.x * 16;
   const float *src = partial + e0 + (tid & 3) * 4;
   f32x4 s{0, 0, 0, 0};
-#pragma unroll 8
-  for (int r = tid >> 2; r < runs; r += 64)
-    s += *(const f32x4 *)(src + r * frags);
+  fhip_for_parts<4>(
+      tid >> 2, 64, runs, [&](int r) { return *(const f32x4 *)(src + r * frags); },
+      [&](f32x4 v, bool in) { s = in ? s + v : s; });
 #pragma unroll
   for (int i = 0; i < 4; ++i)
     for (int o = 4; o < 64; o <<= 1)
@@ -496,7 +496,8 @@ __global__ __launch_bounds__(256) void conv_few_wgrad_sum_kernel(CfArgs g, const
     return;
   int f;
   cf_pair(g, j, &f);
-  fhip_store<float>(dw, dw_dt, k * g.ws[0] + f, (lds[0][tid] + lds[1][tid]) + (lds[2][tid] + lds[3][tid]));
+  const float sum[1] = {(lds[0][tid] + lds[1][tid]) + (lds[2][tid] + lds[3][tid])};
+  fhip_store_float(dw, dw_dt, k * g.ws[0] + f, 0, sum);
 }
 
 // ---- data gradient (unit stride and dilation) -----------------------------------

@@ -578,10 +578,9 @@ __global__ void conv_splitk_sum_kernel(SplitSumArgs a) {
   const int n0 = (int)(e - m * a.N);
   const float *src = a.part + m * a.pitch + n0;
   float4 acc = *(const float4 *)src;
-  for (int z = 1; z < a.parts; ++z) {
-    const float4 v = *(const float4 *)(src + (int64_t)z * a.part_stride);
-    acc.x += v.x, acc.y += v.y, acc.z += v.z, acc.w += v.w;
-  }
+  fhip_for_uniform_parts<4>(
+      1, 1, a.parts, [&](int z) { return *(const float4 *)(src + (int64_t)z * a.part_stride); },
+      [&](float4 v) { acc.x += v.x, acc.y += v.y, acc.z += v.z, acc.w += v.w; });
   // fused operands are addressed as base + m * pixel step + n * channel step,
   // whatever the rank of the convolution (a folded 3-D problem included)
   int64_t coord[FHIP_MAX_RANK] = {};
@@ -594,9 +593,8 @@ __global__ void conv_splitk_sum_kernel(SplitSumArgs a) {
     v[i] = fhip_round_through<float>(a.y_dt, v[i]);
   }
   fhip_apply_epilogue_many<float, 4>(a.epi, v, coord, 2, cols);
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    fhip_store<float>(a.out, a.o_dt, e + i, v[i]);
+  const int64_t at[4] = {e + 0, e + 1, e + 2, e + 3};
+  fhip_store_many<float, 4>(a.out, a.o_dt, at, v, 15);
 }
 
 } // namespace

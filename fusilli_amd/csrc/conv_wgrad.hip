@@ -294,9 +294,11 @@ __global__ __launch_bounds__(256) void conv_wgrad_sum_kernel(WgradSumArgs a, con
   const int64_t e = ((int64_t)blockIdx.x * kLanes + o) * 4;
   f32x4 s{0, 0, 0, 0};
   if (e < a.total) {
-#pragma unroll 8
-    for (int r = z; r < a.runs; r += SLICES)
-      s += *(const f32x4 *)(part + r * a.total + e);
+    const auto run = [&](int r) { return *(const f32x4 *)(part + r * a.total + e); };
+    if constexpr (kLanes < 64)
+      fhip_for_parts<4>(z, SLICES, a.runs, run, [&](f32x4 v, bool in) { s = in ? s + v : s; });
+    else
+      fhip_for_uniform_parts<8>(__builtin_amdgcn_readfirstlane(z), SLICES, a.runs, run, [&](f32x4 v) { s += v; });
   }
   if constexpr (SLICES > 1) {
     meet[z][o] = s;
@@ -309,13 +311,12 @@ __global__ __launch_bounds__(256) void conv_wgrad_sum_kernel(WgradSumArgs a, con
   }
   if (e >= a.total)
     return;
-  const int64_t k = e / a.J;
+  const int64_t k = __builtin_expect(a.total >> 32 != 0, 0) ? e / a.J : (uint32_t)e / (uint32_t)a.J;
   const int j = (int)(e - k * a.J), tap = j / a.C, c = j - tap * a.C;
   const int r = tap / a.S;
   const int64_t at = k * a.sk + r * a.sr + (tap - r * a.S) * a.ss + c * a.sc;
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    fhip_store<float>(dw, a.dt, at + i * a.sc, s[i]);
+  const float v[4] = {s[0], s[1], s[2], s[3]};
+  fhip_store_float(dw, a.dt, at, a.sc, v);
 }
 
 bool wg_channels_last(const fhip_tensor_desc &t) {

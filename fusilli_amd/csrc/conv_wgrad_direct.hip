@@ -423,9 +423,9 @@ conv_wgrad_direct_sum_kernel(WgDirectSumArgs a, const float *part, void *dw) {
   const int within = (int)(lin - (int64_t)type * kWdBlock);
   const float *src = part + (int64_t)type * a.nparts * kWdBlock + within;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
-  for (int p = j; p < a.nparts; p += 4)
-    acc += *(const f32x4 *)(src + (int64_t)p * kWdBlock);
+  fhip_for_uniform_parts<8>(
+      __builtin_amdgcn_readfirstlane(j), 4, a.nparts,
+      [&](int p) { return *(const f32x4 *)(src + (int64_t)p * kWdBlock); }, [&](f32x4 v) { acc += v; });
   red[j][o] = acc;
   __syncthreads();
   if (j != 0)
@@ -437,12 +437,9 @@ conv_wgrad_direct_sum_kernel(WgDirectSumArgs a, const float *part, void *dw) {
   const int kb = type / a.ctypes, cb = type - kb * a.ctypes;
   const int64_t c = cb * 32 + (lane & 31);
   const int r = tap / 3, sx = tap - r * 3;
-#pragma unroll
-  for (int comp = 0; comp < 4; ++comp) {
-    const int i = 4 * (e & 3) + comp;
-    const int64_t k = kb * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
-    fhip_store<float>(dw, a.dt, k * a.sk + c * a.sc + r * a.sr + sx * a.ss, acc[comp]);
-  }
+  const int64_t k = kb * 32 + 8 * (e & 3) + 4 * (lane >> 5);
+  const float v[4] = {acc[0], acc[1], acc[2], acc[3]};
+  fhip_store_float(dw, a.dt, k * a.sk + c * a.sc + r * a.sr + sx * a.ss, a.sk, v);
 }
 
 struct WgDirectPlan {

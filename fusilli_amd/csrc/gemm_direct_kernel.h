@@ -500,9 +500,7 @@ __global__ __launch_bounds__(64) void gemm_direct_finish_kernel(DirectArgs g) {
   const GEMM_AS1 Acc4 *p = (const GEMM_AS1 Acc4 *)g.partial + (batch * gridDim.x + blockIdx.x) * Q + q;
   const int64_t stride = (int64_t)gridDim.z * gridDim.x * Q;
   Acc4 v = p[0];
-#pragma unroll 4
-  for (int s = 1; s < g.splits; ++s)
-    v += p[s * stride];
+  fhip_for_uniform_parts<4>(1, 1, g.splits, [&](int s) { return p[s * stride]; }, [&](Acc4 x) { v += x; });
   int m, dm, n;
   direct_coord<A_KC, B_KC, MT, NT>(q, &m, &dm, &n);
   m += tile_m * 16 * MT;

@@ -254,19 +254,17 @@ __global__ void gemm_splitk_sum_kernel(GemmSumArgs a) {
   const float *src = a.part + m * a.pitch + n0;
   if (a.ints) {
     uint4 sum = *(const uint4 *)src; // (unsigned: wraps like the kernel's int32 accumulators)
-    for (int z = 1; z < a.parts; ++z) {
-      const uint4 v = *(const uint4 *)(src + (int64_t)z * a.part_stride);
-      sum.x += v.x, sum.y += v.y, sum.z += v.z, sum.w += v.w;
-    }
+    fhip_for_uniform_parts<4>(
+        1, 1, a.parts, [&](int z) { return *(const uint4 *)(src + (int64_t)z * a.part_stride); },
+        [&](uint4 v) { sum.x += v.x, sum.y += v.y, sum.z += v.z, sum.w += v.w; });
     uint32_t *o = (uint32_t *)a.out + m * a.o_sm + n0;
     o[0] = sum.x, o[1] = sum.y, o[2] = sum.z, o[3] = sum.w;
     return;
   }
   float4 acc = *(const float4 *)src;
-  for (int z = 1; z < a.parts; ++z) {
-    const float4 v = *(const float4 *)(src + (int64_t)z * a.part_stride);
-    acc.x += v.x, acc.y += v.y, acc.z += v.z, acc.w += v.w;
-  }
+  fhip_for_uniform_parts<4>(
+      1, 1, a.parts, [&](int z) { return *(const float4 *)(src + (int64_t)z * a.part_stride); },
+      [&](float4 v) { acc.x += v.x, acc.y += v.y, acc.z += v.z, acc.w += v.w; });
   int64_t coord[FHIP_MAX_RANK];
   coord[0] = 0;
   coord[a.rank - 2] = m;
@@ -278,9 +276,8 @@ __global__ void gemm_splitk_sum_kernel(GemmSumArgs a) {
     v[i] = fhip_round_through<float>(a.c_dt, v[i]);
   }
   fhip_apply_epilogue_many<float, 4>(a.epi, v, coord, a.rank - 1, cols);
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    fhip_store<float>(a.out, a.o_dt, m * a.o_sm + n0 + i, v[i]);
+  const int64_t at[4] = {m * a.o_sm + n0 + 0, m * a.o_sm + n0 + 1, m * a.o_sm + n0 + 2, m * a.o_sm + n0 + 3};
+  fhip_store_many<float, 4>(a.out, a.o_dt, at, v, 15);
 }
 
 } // namespace

@@ -639,9 +639,7 @@ __global__ __launch_bounds__(256) void gemm_tile_finish_kernel(DirectArgs g) {
   const GEMM_AS1 Acc4 *p = (const GEMM_AS1 Acc4 *)g.partial + (batch * gridDim.x + blockIdx.x) * (BM * BN / 4) + q;
   const int64_t stride = (int64_t)gridDim.z * gridDim.x * (BM * BN / 4);
   Acc4 x = p[0];
-#pragma unroll 4
-  for (int s = 1; s < g.splits; ++s)
-    x += p[s * stride];
+  fhip_for_uniform_parts<4>(1, 1, g.splits, [&](int s) { return p[s * stride]; }, [&](Acc4 v) { x += v; });
   const Acc v[4] = {x.x, x.y, x.z, x.w};
   const int m = tile_m * BM + q / (BN / 4);
   tile_store<Acc, 4>(g, batch, m, m < g.M ? batch * g.o_batch + (int64_t)m * g.o_sm : -1, tile_n * BN + q % (BN / 4) * 4, v,

@@ -487,15 +487,9 @@ __global__ __launch_bounds__(256) void reduce_mid_finish_kernel(ReduceMidArgs g,
   A acc = rf_identity<COMB>();
   if (c < g.k) {
     const RF_AS1 float *p = (const RF_AS1 float *)g.partial + c;
-    int s = sl;
-    for (; s + 3 * per < g.slices; s += 4 * per) {
-      const float v0 = p[(int64_t)s * g.k], v1 = p[(int64_t)(s + per) * g.k];
-      const float v2 = p[(int64_t)(s + 2 * per) * g.k], v3 = p[(int64_t)(s + 3 * per) * g.k];
-      acc = rf_run_comb<COMB, A>(
-          rf_run_comb<COMB, A>(rf_run_comb<COMB, A>(rf_run_comb<COMB, A>(acc, v0), v1), v2), v3);
-    }
-    for (; s < g.slices; s += per)
-      acc = rf_run_comb<COMB, A>(acc, p[(int64_t)s * g.k]);
+    fhip_for_parts<4>(
+        sl, per, g.slices, [&](int s) { return p[(int64_t)s * g.k]; },
+        [&](float v, bool in) { acc = in ? rf_run_comb<COMB, A>(acc, v) : acc; });
   }
   // (inside the wavefronts first: a barrier for every halving was 0.4 us slower)
   for (int s = 32; s >= cols; s >>= 1)

@@ -296,10 +296,10 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void sdpa_decode_kernel(DecodeArgs g)
 // Combines the splits of one packed query row per HD threads.
 template <bool BF16, int HD>
 __global__ __launch_bounds__(256) void sdpa_decode_combine_kernel(DecodeArgs g) {
-  const int rows = g.group * g.pitch;
-  const int64_t lin = (int64_t)blockIdx.x * (256 / HD) + threadIdx.x / HD; // (head, row)
+  const uint32_t rows = (uint32_t)(g.group * g.pitch);
+  const uint32_t lin = blockIdx.x * (256 / HD) + threadIdx.x / HD; // (head, row; their parts fit the device)
   const int d = threadIdx.x % HD;
-  if (lin >= (int64_t)g.heads * rows)
+  if (lin >= (uint32_t)g.heads * rows)
     return;
   const int head = (int)(lin / rows), row = (int)(lin % rows);
   const int hg = row / g.pitch;
@@ -310,18 +310,38 @@ __global__ __launch_bounds__(256) void sdpa_decode_combine_kernel(DecodeArgs g) 
   const int64_t at = (int64_t)(head * g.qtiles + row / 16) * 16 + row % 16;
   const SD_AS1 float *ml = (const SD_AS1 float *)g.part_ml;
   const SD_AS1 float *p = (const SD_AS1 float *)g.part;
-  float top = kNegBig;
-#pragma unroll 4
-  for (int s = 0; s < g.splits; ++s)
-    top = fmaxf(top, ml[(s * tiles * 16 + at) * 2]);
-  float acc = 0.f, den = 0.f;
-#pragma unroll 4
-  for (int s = 0; s < g.splits; ++s) {
+  struct Part {
+    float m, l, o;
+  };
+  const auto load = [&](int s) {
     const int64_t i = s * tiles * 16 + at;
-    const float f = __builtin_amdgcn_exp2f(ml[i * 2] - top);
-    den += ml[i * 2 + 1] * f;
-    acc += p[i * HD + d] * f;
-  }
+    return Part{ml[i * 2], ml[i * 2 + 1], p[i * HD + d]};
+  };
+  // the first parts whole, so that up to eight splits cost one round of loads
+  constexpr int U = 8;
+  Part v[U];
+#pragma unroll
+  for (int s = 0; s < U; ++s)
+    if (s < g.splits)
+      v[s] = load(s);
+  __builtin_amdgcn_sched_barrier(0);
+  float top = kNegBig, acc = 0.f, den = 0.f;
+#pragma unroll
+  for (int s = 0; s < U; ++s)
+    if (s < g.splits)
+      top = fmaxf(top, v[s].m);
+  fhip_for_uniform_parts<U>(
+      U, 1, g.splits, [&](int s) { return ml[(s * tiles * 16 + at) * 2]; }, [&](float m) { top = fmaxf(top, m); });
+  const auto add = [&](const Part &x) {
+    const float f = __builtin_amdgcn_exp2f(x.m - top);
+    den += x.l * f;
+    acc += x.o * f;
+  };
+#pragma unroll
+  for (int s = 0; s < U; ++s)
+    if (s < g.splits)
+      add(v[s]);
+  fhip_for_uniform_parts<U>(U, 1, g.splits, load, add);
   dec_store<BF16>(g.o, dec_offset(g, head / g.Hkv, head % g.Hkv, r, g.o_sb, g.o_sh, g.o_ss) + d, acc / den);
 }
 

@@ -1,0 +1,40 @@
+"""Launches that add partial results, at part counts on both sides of their rounds of loads:
+small whole numbers, so that every sum is exact in f32 whatever its order."""
+import numpy as np
+import pytest
+
+from fusilli_amd import capi
+from oracle import oracle
+from helpers import HT
+from test_generic_ops_gpu import run_batchnorm, run_conv_wgrad
+
+pytestmark = pytest.mark.gpu
+
+
+def whole(seed, dims, dtype, span):
+    v = np.random.default_rng(seed).integers(-span, span + 1, size=dims).astype(np.float64)
+    return HT.from_logical(v, dtype, oracle.channels_last_strides(dims))
+
+
+# 64 rows of 32 channels per workgroup, 64 lanes per channel that take eight parts a round
+@pytest.mark.parametrize("parts", [1, 2, 63, 64, 65, 449, 511, 512])
+@pytest.mark.parametrize("affine", [capi.FLOAT, capi.HALF])
+def test_batchnorm_parts(ctx, parts, affine):
+    x = whole(parts, [parts, 32, 8, 8], capi.BFLOAT16, 3)
+    one = HT.from_logical(np.ones(32), affine)
+    _, m, _ = run_batchnorm(ctx, x, training=True, eps=1e-3, scale=one, bias=one)
+    assert f"workgroups={parts}" in ctx.last_kernel(), ctx.last_kernel()
+    # (one division and one addition to the pivot, each rounded once)
+    np.testing.assert_allclose(m, x.logical().mean(axis=(0, 2, 3)), rtol=0, atol=3 * 2.0 ** -23)
+
+
+# gathered tiles: runs of 32-pixel steps, added one by one, four and sixteen at a time
+@pytest.mark.parametrize("n", [2, 3, 5, 8, 9, 17, 33, 36, 39, 65, 130])
+@pytest.mark.parametrize("dtype", [capi.BFLOAT16, capi.FLOAT])
+def test_weight_gradient_parts(ctx, n, dtype):
+    x, dy = whole(n, [n, 8, 16, 16], capi.BFLOAT16, 2), whole(n + 1, [n, 24, 16, 16], capi.BFLOAT16, 1)
+    dw = run_conv_wgrad(ctx, dy, x, [24, 8, 1, 3], [0, 1], [1, 1], [1, 1], capi.BFLOAT16, tuned=None,
+                        w_dtype=capi.FLOAT if dtype == capi.FLOAT else None)
+    assert ctx.last_kernel().startswith("conv_wgrad_gather"), ctx.last_kernel()
+    ref = oracle.conv_wgrad(dy.logical(), x.logical(), [24, 8, 1, 3], [0, 1], [1, 1], [1, 1])
+    np.testing.assert_array_equal(dw.logical(), HT.from_logical(ref, dtype).logical())
