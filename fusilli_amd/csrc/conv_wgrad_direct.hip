@@ -8,17 +8,21 @@
 // the reduction runs along the tensors' slow dimension.  The kernel therefore
 //
 //  * gives a workgroup one 32 x 32 block of (k, c) for all nine taps -- 144
-//    accumulator registers per lane -- and lets its eight wavefronts reduce
-//    different image rows; their results are summed through LDS at the end, so
-//    a workgroup leaves 36 KB of partial sums, not 288 KB;
+//    accumulator registers per lane -- and an equal share of the batch's rows,
+//    of which its eight wavefronts reduce equal shares; their results are summed
+//    through LDS at the end, so a workgroup leaves 36 KB of partial sums, not 288 KB;
 //  * streams image rows through small per-wavefront LDS rings by LDS-DMA (a
 //    pixel's 32 channels of this block are 64 contiguous bytes) and takes the
 //    MFMA operands out of them with transposing reads: 16 consecutive pixels of
-//    a row are the K extent of one 32 x 32 x 16 MFMA;
+//    a row are the K extent of one 32 x 32 x 16 MFMA, and a row takes as many
+//    as it has (NKS), not the four of the widest;
 //  * walks the rows of X: row rho pairs with the DY rows rho + 1, rho, rho - 1
 //    (filter rows 0, 1, 2), whose fragments stay in registers for the three
 //    visits, and the three column taps are the same LDS row read one pixel
 //    apart -- six fragment reads feed nine MFMAs;
+//  * runs from one image into the next: the loads of a step are always the same
+//    number (rows that do not exist are fetched from nowhere), kD steps ahead of it, so the
+//    waits count and nothing drains between images;
 //  * needs no barrier in the main loop: a wavefront only waits for its own DMA.
 //
 // A second, small kernel sums the workgroups' partial results in a fixed
@@ -31,27 +35,22 @@
 #include "fast_paths.h"
 #include "gemm_kernel.h"
 
-#ifndef WD_EXP
-#define WD_EXP 0 // timing experiments: 1 no MFMA, 2 no loads in the loop, 4 no LDS sum, 8 no fragment reads
-#endif
-
-#ifdef WD_PROFILE // experiment builds: cycle stamps of workgroup 0 replace its results
-#define WD_STAMP(i) st[i] = __builtin_amdgcn_s_memtime()
-#else
-#define WD_STAMP(i)                                                            \
-  do {                                                                         \
-  } while (0)
-#endif
-
 namespace {
 
 constexpr int kWdWaves = 8;
 constexpr int kWdThreads = kWdWaves * 64;
-constexpr int kWdRow = 4096;   // LDS bytes of a row slice: 64 pixel slots x 64 bytes
-constexpr int kWdXSlots = 3;   // X rows in flight per wavefront
-constexpr int kWdYSlots = 2;   // DY rows in flight per wavefront
-constexpr int kWdWaveLds = (kWdXSlots + kWdYSlots) * kWdRow;
+constexpr int kWdWaveLds = 20480;
 constexpr int kWdLds = kWdWaves * kWdWaveLds; // 160 KB
+
+// Rows of up to 16 NKS pixels (56 for NKS 4): LDS-DMA instructions of 16 pixels (1 KB) per row of
+// X (one pixel of padding on each side) and of DY, and the steps that loads run ahead: as
+// many as a wavefront's 20 KB hold (kD rows of DY, kD + 1 of X).
+template <int NKS> struct WdRows {
+  static constexpr int kX = NKS < 4 ? NKS + 1 : 4, kY = NKS;
+  static constexpr int kD = NKS == 1 ? 6 : NKS == 2 ? 3 : 2;
+  static constexpr uint32_t kXBytes = kX * 1024, kYBytes = kY * 1024, kYBase = (kD + 1) * kXBytes;
+  static_assert(kYBase + kD * kYBytes <= kWdWaveLds && (kD - 1) * (kX + kY) < 64, "LDS, vmcnt");
+};
 constexpr int kWdMaxW = 56;
 constexpr int kWdBlock = 9 * 16 * 64; // partial sums of one workgroup (floats)
 
@@ -61,16 +60,17 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 struct WgDirectArgs {
   const char *x, *dy;
   float *part;
-  int32_t N, H, W, C, K;
-  int32_t rpw;    // image rows per pair of wavefronts (w, w + 4) that share a SIMD
-  int32_t rfirst; // of which wavefront w takes the first rfirst, w + 4 the rest
-  int32_t chunks; // row chunks (4 * rpw rows) per image
-  int32_t ipw;    // images per workgroup
+  int32_t H, W, C, K;
+  int32_t rows;   // of the batch: N * H
   int32_t nparts; // workgroups per (k, c) block
-  int32_t ctypes; // C / 32
-  uint32_t magic_ctypes;
+  int32_t types, ctypes; // blocks, C / 32
+  int32_t total, per_xcd; // types * nparts, an eighth of it rounded up
+  uint32_t magic_types, magic_ctypes, magic_h;
   uint32_t x_bytes, dy_bytes;
 };
+
+// rows [first, last) of share `i` of `n`
+__device__ __forceinline__ int wd_share(int rows, int i, int n) { return (int)((int64_t)rows * i / n); }
 
 template <int KIND>
 __device__ __forceinline__ f32x16 wd_mfma(const u32x2 &a0, const u32x2 &a1,
@@ -78,11 +78,6 @@ __device__ __forceinline__ f32x16 wd_mfma(const u32x2 &a0, const u32x2 &a1,
                                           const f32x16 &c) {
   const u32x4 a = {a0.x, a0.y, a1.x, a1.y};
   const u32x4 b = {b0.x, b0.y, b1.x, b1.y};
-  if (WD_EXP & 1) {
-    f32x16 r = c;
-    asm volatile("" : "+v"(r) : "v"(a), "v"(b));
-    return r;
-  }
   if constexpr (KIND == GK_BF16)
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(
         __builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
@@ -99,10 +94,6 @@ __device__ __forceinline__ f32x16 wd_mfma(const u32x2 &a0, const u32x2 &a1,
 template <int OFFSET>
 __device__ __forceinline__ void wd_read_tr(u32x2 &dst, uint32_t addr) {
   static_assert(OFFSET >= 0 && OFFSET < 65536, "16-bit offset field");
-  if (WD_EXP & 8) {
-    asm volatile("" : "=v"(dst) : "v"(addr));
-    return;
-  }
   asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2"
                : "=v"(dst)
                : "v"(addr), "n"(OFFSET));
@@ -125,67 +116,73 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t wd_rsrc(const void *base,
       (int)__builtin_amdgcn_readfirstlane(bytes), 0x00020000);
 }
 
-template <int KIND>
+template <int KIND, int NKS>
 __global__ __launch_bounds__(kWdThreads)
 __attribute__((amdgpu_waves_per_eu(2, 2))) void
 conv_wgrad_direct_kernel(WgDirectArgs g) {
+  using R = WdRows<NKS>;
   extern __shared__ __attribute__((aligned(16))) char smem[];
-#ifdef WD_PROFILE
-  uint64_t st[8] = {};
-#endif
-  WD_STAMP(0);
   const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int l = threadIdx.x & 63;
-  const int a_H = g.H, a_W = g.W, a_C = g.C, a_K = g.K, a_N = g.N;
-  const int a_rpw = g.rpw, a_ipw = g.ipw;
+  const int a_H = g.H, a_W = g.W;
 
-  // workgroup (x, y, z) -> row chunk, image group, (k block, c block)
-  const int chunk = (int)blockIdx.x, igroup = (int)blockIdx.y, type = (int)blockIdx.z;
+  // Workgroup -> (part, block): a die's workgroups (every eighth) take the blocks of a part one
+  // after another, which read the same rows of X and DY.
+  const int lin = (int)(blockIdx.x & 7) * g.per_xcd + (int)(blockIdx.x >> 3);
+  if (lin >= g.total)
+    return;
+  const int part = conv_div(lin, g.types, g.magic_types), type = lin - part * g.types;
   const int kb = conv_div(type, g.ctypes, g.magic_ctypes), cb = type - kb * g.ctypes;
-  const int n0 = igroup * a_ipw;
-  const int n1 = n0 + a_ipw < a_N ? n0 + a_ipw : a_N;
-  // rows: the pair (w, w + 4) of a SIMD shares a_rpw rows; the first of the
-  // pair, which the SIMD serves first, takes the larger part
-  const int second = wave >> 2;
-  const int p0 = (chunk * 4 + (wave & 3)) * a_rpw + (second ? g.rfirst : 0);
-  const int share = second ? a_rpw - g.rfirst : g.rfirst;
-  int nrows = a_H - p0;
-  nrows = nrows < share ? nrows : share;
-  nrows = nrows > 0 ? nrows : 0;
-  // Step t of a wavefront's walk brings DY row p0 - 1 + t into registers and,
-  // from t = 2 on, multiplies X row p0 + t - 2 with the three DY rows held:
-  // the newest is filter row 0, the oldest filter row 2.
-  const int n_st = nrows > 0 ? nrows + 2 : 0;
+  const int row0 = wd_share(g.rows, part, g.nparts), row1 = wd_share(g.rows, part + 1, g.nparts);
+  const int first = row0 + (((row1 - row0) * wave) >> 3);
+  const int last = row0 + (((row1 - row0) * (wave + 1)) >> 3);
+
+  // A walk over rows [first, last) of the batch, cut into the images' runs.  Step t of a run
+  // that starts at row p0 of its image brings DY row p0 - 1 + t into registers and, from
+  // t = 2 on, multiplies X row p0 + t - 2 with the three DY rows held: the newest is
+  // filter row 0, the oldest filter row 2.
+  struct Walk {
+    int row, p0, n, t; // the run's first row in the batch and in its image, its rows, the step
+  };
+  const int img0 = conv_div(first, a_H, g.magic_h);
+  auto begin = [&](int row, int p0) __attribute__((always_inline)) {
+    const int in_image = a_H - p0, left = last - row;
+    return Walk{row, p0, left < in_image ? left : in_image, 0};
+  };
+  auto step = [&](Walk &w) __attribute__((always_inline)) {
+    if (++w.t == w.n + 2)
+      w = begin(w.row + w.n, 0);
+  };
 
   // ---- LDS-DMA lane offsets (relative to a row's first byte) --------------------
   // instruction j fills pixel slots 16 j .. 16 j + 15 of a row slice: lane d
   // carries 16 bytes (8 channels) d % 4 of slot 16 j + d / 4.  X slot t holds
   // image column t - 1 (slot 0 and the slots past the image are the zero
   // padding), DY slot t holds column t (zeros past the image).
-  uint32_t xrel[4], yrel[4];
+  uint32_t xrel[R::kX], yrel[R::kY];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
+  for (int j = 0; j < R::kX; ++j) {
     const int slot = 16 * j + (l >> 2);
     const int q = slot - 1;
     xrel[j] = (unsigned)q < (unsigned)a_W
-                  ? (uint32_t)(q * a_C * 2 + cb * 64 + (l & 3) * 16)
+                  ? (uint32_t)(q * g.C * 2 + cb * 64 + (l & 3) * 16)
                   : 0x80000000u;
-    yrel[j] = slot < a_W ? (uint32_t)(slot * a_K * 2 + kb * 64 + (l & 3) * 16)
-                         : 0x80000000u;
+    if (j < R::kY)
+      yrel[j < R::kY ? j : 0] = slot < a_W ? (uint32_t)(slot * g.K * 2 + kb * 64 + (l & 3) * 16)
+                                           : 0x80000000u;
   }
   const __amdgpu_buffer_rsrc_t rx = wd_rsrc(g.x, g.x_bytes);
   const __amdgpu_buffer_rsrc_t ry = wd_rsrc(g.dy, g.dy_bytes);
   const __amdgpu_buffer_rsrc_t rnone = wd_rsrc(g.x, 0); // every lane reads zero
+  const int x_pitch = a_W * g.C * 2, y_pitch = a_W * g.K * 2;
 
   const uint32_t wbase = lds0 + (uint32_t)wave * kWdWaveLds;
   // fragment read address inside a row slice: lane l is MFMA row / column
   // l % 32 and K half l / 32 (pixels 8 h .. 8 h + 7 of the K-step)
   const uint32_t tbase = (uint32_t)(((l >> 5) * 8 + ((l & 15) >> 2)) * 64 +
                                     ((l >> 4) & 1) * 32 + (l & 3) * 8);
-  const uint32_t xbase = wbase + tbase;
-  const uint32_t ybase = wbase + kWdXSlots * kWdRow + tbase;
-  const bool upper = l >= 32;
+  [[maybe_unused]] const bool upper = l >= 32;
 
   f32x16 acc[9];
 #pragma unroll
@@ -194,78 +191,70 @@ conv_wgrad_direct_kernel(WgDirectArgs g) {
     for (int i = 0; i < 16; ++i)
       acc[t][i] = 0.f;
 
-  for (int n = n0; n < n1 && n_st > 0; ++n) {
-    // Loads of step t: four instructions each, so that the waits can count.
-    // Rows outside the image arrive as zeros (DY rows of the neighbouring
-    // wavefronts' shares are real: they are this share's halo).
-    auto issue_y = [&](int t) __attribute__((always_inline)) {
-      const int row = p0 - 1 + t;
-      const bool ok = t < n_st && (unsigned)row < (unsigned)a_H;
-      const __amdgpu_buffer_rsrc_t rs = ok ? ry : rnone;
-      const int off = ok ? ((n * a_H + row) * a_W) * a_K * 2 : 0;
-      const uint32_t dst = wbase + (uint32_t)(kWdXSlots + (t & 1)) * kWdRow;
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            rs, (GEMM_AS3 char *)__builtin_amdgcn_readfirstlane(dst + j * 1024u),
-            16, (int)yrel[j], off, 0, 0);
+  if (first < last) {
+    Walk ahead = begin(first, first - img0 * a_H), now = ahead;
+    // ring slots of the next loads and the next reads
+    uint32_t put_x = 0, put_y = R::kYBase, get_x = 0, get_y = R::kYBase;
+    auto turn = [](uint32_t &at, uint32_t by, uint32_t from, uint32_t to) __attribute__((always_inline)) {
+      at = at + by == to ? from : at + by;
     };
-    auto issue_x = [&](int t, int xs) __attribute__((always_inline)) {
-      const int row = p0 + t - 2;
-      const bool ok = t < n_st;
-      const __amdgpu_buffer_rsrc_t rs = ok ? rx : rnone;
-      const int off = ok ? ((n * a_H + row) * a_W) * a_C * 2 : 0;
-      const uint32_t dst = wbase + (uint32_t)xs * kWdRow;
+    // the loads of a step, always kX + kY of them; rows outside the image, and all past the walk's
+    // end, come from nowhere (DY rows of the neighbouring shares are real: they are this
+    // share's halo)
+    auto issue = [&]() __attribute__((always_inline)) {
+      const bool live = ahead.n > 0;
+      const bool y_ok = live && (unsigned)(ahead.p0 - 1 + ahead.t) < (unsigned)a_H, x_ok = live && ahead.t >= 2;
+      const __amdgpu_buffer_rsrc_t ys = y_ok ? ry : rnone, xs = x_ok ? rx : rnone;
+      const int y_off = y_ok ? (ahead.row - 1 + ahead.t) * y_pitch : 0;
+      const int x_off = x_ok ? (ahead.row + ahead.t - 2) * x_pitch : 0;
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < R::kX; ++j)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            rs, (GEMM_AS3 char *)__builtin_amdgcn_readfirstlane(dst + j * 1024u),
-            16, (int)xrel[j], off, 0, 0);
+            xs, (GEMM_AS3 char *)__builtin_amdgcn_readfirstlane(wbase + put_x + j * 1024u), 16, (int)xrel[j], x_off,
+            0, 0);
+#pragma unroll
+      for (int j = 0; j < R::kY; ++j)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            ys, (GEMM_AS3 char *)__builtin_amdgcn_readfirstlane(wbase + put_y + j * 1024u), 16, (int)yrel[j], y_off,
+            0, 0);
+      turn(put_x, R::kXBytes, 0, R::kYBase);
+      turn(put_y, R::kYBytes, R::kYBase, R::kYBase + R::kD * R::kYBytes);
+      if (live)
+        step(ahead);
     };
+#pragma unroll
+    for (int i = 0; i < R::kD; ++i)
+      issue();
 
-    // DY fragments of three rows: dyf[j] holds the row of step t, t % 3 == j
-    u32x2 dyf[3][4][2];
-
-    WD_STAMP(1);
-    issue_y(0);
-    issue_y(1);
-    issue_x(2, 0);
-    WD_STAMP(2);
-
-    auto read_y = [&](auto jc, int t) __attribute__((always_inline)) {
+    // DY fragments of three rows: dyf[j] holds the row of a run's steps that are j modulo 3
+    u32x2 dyf[3][NKS][2];
+    auto read_y = [&](auto jc) __attribute__((always_inline)) {
       constexpr int J = decltype(jc)::value;
-      const uint32_t ya = ybase + (uint32_t)(t & 1) * kWdRow;
-      gemm_static_for<4>([&](auto kc) {
+      const uint32_t ya = wbase + get_y + tbase;
+      gemm_static_for<NKS>([&](auto kc) {
         constexpr int ks = decltype(kc)::value;
         wd_read_tr<ks * 1024>(dyf[J][ks][0], ya);
         wd_read_tr<ks * 1024 + 256>(dyf[J][ks][1], ya);
       });
     };
-    // steps 0 and 1: a DY row into registers, its slot refilled.  The order of
-    // all loads is Y0 Y1 X2 | Y2 X3 | Y3 | X4 Y4 | X5 Y5 ...: from step 2 on a
-    // step finds exactly eight loads issued after the ones it needs.
-    auto light = [&](auto jc, auto vmc, int t) __attribute__((always_inline)) {
-      if (!(WD_EXP & 2))
-        __builtin_amdgcn_s_waitcnt(gemm_wait_imm(decltype(vmc)::value));
-      read_y(jc, t);
+    // A step: its loads have landed when only those of the kD - 1 steps issued after it are
+    // out.  Its DY row's slot, and the X slot of the step before, are free once the DY row
+    // is in registers.
+    auto light = [&](auto jc) __attribute__((always_inline)) {
+      __builtin_amdgcn_s_waitcnt(gemm_wait_imm((R::kD - 1) * (R::kX + R::kY)));
+      read_y(jc);
+      turn(get_x, R::kXBytes, 0, R::kYBase);
+      turn(get_y, R::kYBytes, R::kYBase, R::kYBase + R::kD * R::kYBytes);
       wd_wait_lgkm<0>();
-      if (!(WD_EXP & 2)) {
-        issue_y(t + 2);
-        if (t == 0)
-          issue_x(3, 1);
-      }
+      issue();
     };
-    // step t >= 2 (t % 3 == J): X row p0 + t - 2 against the three DY rows
-    auto full = [&](auto jc, auto vmc, int t) __attribute__((always_inline)) {
-      constexpr int J = decltype(jc)::value;
-      constexpr int J1 = (J + 2) % 3, J2 = (J + 1) % 3;
-      constexpr int XS = (J + 1) % 3; // (t - 2) % 3
-      // the loads of this step have landed when only the eight issued after
-      // them are out
-      if (!(WD_EXP & 2))
-        __builtin_amdgcn_s_waitcnt(gemm_wait_imm(decltype(vmc)::value));
-      read_y(jc, t);
-      const uint32_t xa = xbase + (uint32_t)XS * kWdRow;
+    auto full = [&](auto jc) __attribute__((always_inline)) {
+      constexpr int J = decltype(jc)::value, J1 = (J + 2) % 3, J2 = (J + 1) % 3;
+      __builtin_amdgcn_s_waitcnt(gemm_wait_imm((R::kD - 1) * (R::kX + R::kY)));
+      read_y(jc);
+      const uint32_t xa = wbase + get_x + tbase;
+      turn(get_x, R::kXBytes, 0, R::kYBase);
+      turn(get_y, R::kYBytes, R::kYBase, R::kYBase + R::kD * R::kYBytes);
       u32x2 xf[2][3][2];
       auto read_x = [&](auto kc) __attribute__((always_inline)) {
         constexpr int ks = decltype(kc)::value;
@@ -276,16 +265,11 @@ conv_wgrad_direct_kernel(WgDirectArgs g) {
         });
       };
       read_x(std::integral_constant<int, 0>{});
-      // the DY row is in registers: its slot, and the X slot read in the
-      // step before, can be refilled
       wd_wait_lgkm<6>();
-      if (!(WD_EXP & 2)) {
-        issue_x(t + 2, J);
-        issue_y(t + 2);
-      }
-      gemm_static_for<4>([&](auto kc) {
+      issue();
+      gemm_static_for<NKS>([&](auto kc) {
         constexpr int ks = decltype(kc)::value;
-        if constexpr (ks + 1 < 4) {
+        if constexpr (ks + 1 < NKS) {
           read_x(std::integral_constant<int, ks + 1>{});
           wd_wait_lgkm<6>();
         } else {
@@ -327,46 +311,30 @@ conv_wgrad_direct_kernel(WgDirectArgs g) {
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
     using I2 = std::integral_constant<int, 2>;
-    using V8 = std::integral_constant<int, 8>;
-    using V12 = std::integral_constant<int, 12>;
-    light(I0{}, V8{}, 0);
-    light(I1{}, V12{}, 1);
-    int t = 2;
-    while (true) {
-      if (t >= n_st)
-        break;
-      full(I2{}, V8{}, t);
-      ++t;
-      if (t >= n_st)
-        break;
-      full(I0{}, V8{}, t);
-      ++t;
-      if (t >= n_st)
-        break;
-      full(I1{}, V8{}, t);
-      ++t;
+    // (run by run, the products in a loop of their own: under a branch of one loop over all steps
+    // the compiler copies the accumulators about and spills 440 to 880 registers)
+    for (; now.n > 0; now = begin(now.row + now.n, 0)) {
+      light(I0{});
+      light(I1{});
+      for (int left = now.n;;) {
+        full(I2{});
+        if (--left == 0)
+          break;
+        full(I0{});
+        if (--left == 0)
+          break;
+        full(I1{});
+        if (--left == 0)
+          break;
+      }
     }
-    // the loads still in flight land before the next image reuses the slots
-    __builtin_amdgcn_s_waitcnt(gemm_wait_imm(0));
   }
 
   // ---- sum of the eight wavefronts through LDS, half of the block at a time ---
-  WD_STAMP(4);
+  // (the loads still in flight land before their slots hold sums)
   __builtin_amdgcn_s_waitcnt(gemm_wait_imm(0));
   __syncthreads();
-  WD_STAMP(5);
-  const unsigned wg = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-  f32x4 *dst4 = (f32x4 *)(g.part + (size_t)wg * kWdBlock);
-  if (WD_EXP & 4) {
-    float v = 0.f;
-#pragma unroll
-    for (int t = 0; t < 9; ++t)
-#pragma unroll
-      for (int i = 0; i < 16; ++i)
-        v += acc[t][i];
-    ((float *)dst4)[wave * 64 + l] = v;
-    return;
-  }
+  f32x4 *dst4 = (f32x4 *)(g.part + ((size_t)type * g.nparts + part) * kWdBlock);
   // entry e = 4 * tap + j is registers 4 j .. 4 j + 3 of a tap's accumulator:
   // one 16-byte LDS access per lane
   f32x4 *scr4 = (f32x4 *)smem; // [wavefront][18 entries][64 lanes]
@@ -392,13 +360,6 @@ conv_wgrad_direct_kernel(WgDirectArgs g) {
     }
     __syncthreads();
   });
-#ifdef WD_PROFILE
-  __builtin_amdgcn_s_waitcnt(gemm_wait_imm(0));
-  WD_STAMP(6);
-  if (wg == 0 && l == 0)
-    for (int i = 0; i < 8; ++i)
-      ((uint64_t *)dst4)[wave * 8 + i] = st[i];
-#endif
 }
 
 struct WgDirectSumArgs {
@@ -444,10 +405,9 @@ conv_wgrad_direct_sum_kernel(WgDirectSumArgs a, const float *part, void *dw) {
 
 struct WgDirectPlan {
   bool ok = false;
-  int kind = GK_BF16;
+  int kind = GK_BF16, nks = 4;
   WgDirectArgs a{};
-  dim3 grid;
-  size_t part_bytes = 0;
+  size_t contract = 0; // bytes of the caller's workspace
 };
 
 bool wd_channels_last(const fhip_tensor_desc &t) {
@@ -505,9 +465,10 @@ WgDirectPlan make_wd_plan(const fhip_conv_desc *d, int num_cus) {
   const int64_t types = (C / 32) * (K / 32);
   if (types > 4096)
     return p;
-  // One workgroup per (block, image group, row chunk): as few partial results
-  // as fill the machine once.  Small batches cut the image into row chunks,
-  // large ones give a workgroup several images.
+  // The caller's workspace: the partial sums of workgroups that take whole images, or row chunks
+  // of one, a round of them and no fewer.  Saved plans hold its size and are taken only where they equal
+  // the plan of today byte for byte (Graph::loadFromArtifact); parts beyond it lie in
+  // the context's scratch.
   int64_t chunks = 1, ipw = 1;
   if (types * N < cus) {
     chunks = (cus + types * N - 1) / (types * N);
@@ -517,31 +478,53 @@ WgDirectPlan make_wd_plan(const fhip_conv_desc *d, int num_cus) {
     ipw = types * N / cus;
     ipw = ipw < 1 ? 1 : ipw;
   }
-  // rows per pair of wavefronts
   const int64_t rpw = (H + 4 * chunks - 1) / (4 * chunks);
   chunks = (H + 4 * rpw - 1) / (4 * rpw);
-  const int64_t rfirst = (rpw + 1) / 2;
   const int64_t igroups = (N + ipw - 1) / ipw;
-  const int64_t nparts = igroups * chunks;
-  if (types * nparts >= (1ll << 31) / kWdBlock)
+  const int64_t whole = igroups * chunks;
+  if (types * whole >= (1ll << 31) / kWdBlock || chunks > 65535 || igroups > 65535)
     return p;
+  p.contract = (size_t)(types * whole) * kWdBlock * sizeof(float);
   WgDirectArgs &a = p.a;
-  a.N = (int32_t)N, a.H = (int32_t)H, a.W = (int32_t)W, a.C = (int32_t)C, a.K = (int32_t)K;
-  a.rpw = (int32_t)rpw, a.rfirst = (int32_t)rfirst;
-  a.chunks = (int32_t)chunks, a.ipw = (int32_t)ipw;
-  a.nparts = (int32_t)nparts, a.ctypes = (int32_t)(C / 32);
-  a.magic_ctypes = conv_magic(a.ctypes);
+  a.H = (int32_t)H, a.W = (int32_t)W, a.C = (int32_t)C, a.K = (int32_t)K;
+  a.rows = (int32_t)(N * H);
+  a.types = (int32_t)types, a.ctypes = (int32_t)(C / 32);
+  a.magic_types = conv_magic(a.types), a.magic_ctypes = conv_magic(a.ctypes), a.magic_h = conv_magic(a.H);
   a.x_bytes = (uint32_t)x_bytes, a.dy_bytes = (uint32_t)dy_bytes;
-  if (chunks > 65535 || igroups > 65535 || types > 65535)
-    return p;
-  p.grid = dim3((unsigned)chunks, (unsigned)igroups, (unsigned)types);
-  p.part_bytes = (size_t)(types * nparts) * kWdBlock * sizeof(float);
+  p.nks = (int)((W + 15) / 16);
   p.ok = true;
   return p;
 }
 
-template <int KIND> int wd_launch(fhip_ctx *ctx, const WgDirectPlan &p) {
-  auto kernel = conv_wgrad_direct_kernel<KIND>;
+// Workgroups per (k, c) block, `most` at most.  A compute unit holds one workgroup, so what
+// counts is rounds times a round: 7.5 us of start and sums, 0.4 to 0.9 per row of a
+// wavefront, and 15 ns a partial result (36 KB written and read).  Fitted to 17 layers with 2 to
+// 1280 parts: 14 images of 24 x 24, 320 -> 480 (150 blocks) 43.9 us in one part, 41.4 in three,
+// 54.0 in six; 14 x 14 x 14, 64 -> 192 (12) 11.6 in ten, 13.6 in 21, 21.8 in 42; 56 x 56 x 32, 64 -> 128
+// (8) 28.1 in 16, 25.0 in 32, 35.0 in 64.  Shares of whole images took a round and a little
+// more wherever the blocks do not divide 256 (those layers: 86.8, 22.3 and 24.9).
+int wd_parts(const WgDirectArgs &a, int nks, int64_t most) {
+  constexpr int64_t kCus = 256;
+  const double row = nks == 1 ? 0.4 : nks == 2 ? 0.75 : nks == 3 ? 0.85 : 0.9;
+  int64_t best = 1;
+  double least = 0;
+  for (const int quarters : {1, 2, 3, 4, 8, 12}) {
+    int64_t parts = quarters * kCus / (4 * a.types);
+    const int64_t useful = (a.rows + kWdWaves - 1) / kWdWaves;
+    parts = parts < useful ? parts : useful;
+    parts = parts < most ? parts : most;
+    parts = parts < 1 ? 1 : parts;
+    const int64_t deep = (a.rows + kWdWaves * parts - 1) / (kWdWaves * parts);
+    const double us = (double)((parts * a.types + kCus - 1) / kCus) * (7.5 + row * (double)deep) +
+                      0.015 * (double)(parts * a.types);
+    if (quarters == 1 || us < least)
+      least = us, best = parts;
+  }
+  return (int)best;
+}
+
+template <int KIND, int NKS> int wd_launch(fhip_ctx *ctx, const WgDirectArgs &a) {
+  auto kernel = conv_wgrad_direct_kernel<KIND, NKS>;
   static FhipOncePerDevice configured;
   if (!configured.done(ctx->device)) {
     FHIP_HIP_CHECK(ctx, hipFuncSetAttribute(
@@ -549,9 +532,16 @@ template <int KIND> int wd_launch(fhip_ctx *ctx, const WgDirectPlan &p) {
                             hipFuncAttributeMaxDynamicSharedMemorySize, kWdLds));
     configured.mark(ctx->device);
   }
-  hipLaunchKernelGGL(kernel, p.grid, dim3(kWdThreads), kWdLds, ctx->stream, p.a);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)a.per_xcd * 8), dim3(kWdThreads), kWdLds, ctx->stream, a);
   FHIP_HIP_CHECK(ctx, hipGetLastError());
   return 0;
+}
+
+template <int KIND> int wd_launch(fhip_ctx *ctx, const WgDirectPlan &p) {
+  return p.nks == 1   ? wd_launch<KIND, 1>(ctx, p.a)
+         : p.nks == 2 ? wd_launch<KIND, 2>(ctx, p.a)
+         : p.nks == 3 ? wd_launch<KIND, 3>(ctx, p.a)
+                      : wd_launch<KIND, 4>(ctx, p.a);
 }
 
 } // namespace
@@ -560,7 +550,7 @@ bool fhip_fast_conv_wgrad_direct_applicable(const fhip_conv_desc *d,
                                             size_t *workspace_bytes) {
   const WgDirectPlan p = make_wd_plan(d, 256);
   if (workspace_bytes)
-    *workspace_bytes = p.ok ? p.part_bytes : 0;
+    *workspace_bytes = p.ok ? p.contract : 0;
   return p.ok;
 }
 
@@ -574,9 +564,22 @@ int fhip_fast_conv_wgrad_direct(fhip_ctx *ctx, const fhip_conv_desc *d,
   FHIP_REQUIRE(ctx, ((uintptr_t)workspace & 255) == 0 && ((uintptr_t)x & 15) == 0 &&
                         ((uintptr_t)dy & 15) == 0,
                "conv wgrad: workspace must be 256-byte and tensors 16-byte aligned");
+  constexpr size_t kBytes = kWdBlock * sizeof(float);
+  const int64_t held = (int64_t)(p.contract / kBytes) / p.a.types;
+  p.a.nparts = wd_parts(p.a, p.nks, (1ll << 31) / kWdBlock / p.a.types);
+  void *part = workspace;
+  if (p.a.nparts > held) {
+    const size_t bytes = (size_t)p.a.types * p.a.nparts * kBytes;
+    if (!fhip_ctx_scratch_ready(ctx, bytes))
+      p.a.nparts = wd_parts(p.a, p.nks, held);
+    else if (fhip_ctx_scratch(ctx, bytes, &part) != 0)
+      return 1;
+  }
+  p.a.total = p.a.types * p.a.nparts;
+  p.a.per_xcd = (p.a.total + 7) / 8;
   p.a.x = (const char *)x;
   p.a.dy = (const char *)dy;
-  p.a.part = (float *)workspace;
+  p.a.part = (float *)part;
   if ((p.kind == GK_BF16 ? wd_launch<GK_BF16>(ctx, p) : wd_launch<GK_F16>(ctx, p)) != 0)
     return 1;
   WgDirectSumArgs s;
@@ -590,6 +593,6 @@ int fhip_fast_conv_wgrad_direct(fhip_ctx *ctx, const fhip_conv_desc *d,
   hipLaunchKernelGGL(conv_wgrad_direct_sum_kernel, dim3((unsigned)(total / 256)),
                      dim3(256), 0, ctx->stream, s, (const float *)p.a.part, dw);
   FHIP_HIP_CHECK(ctx, hipGetLastError());
-  fhip_note_kernel(ctx, "conv_wgrad_direct");
+  fhip_note_kernel(ctx, "conv_wgrad_direct steps=%d parts=%d", p.nks, p.a.nparts);
   return 0;
 }

@@ -38,3 +38,23 @@ def test_weight_gradient_parts(ctx, n, dtype):
     assert ctx.last_kernel().startswith("conv_wgrad_gather"), ctx.last_kernel()
     ref = oracle.conv_wgrad(dy.logical(), x.logical(), [24, 8, 1, 3], [0, 1], [1, 1], [1, 1])
     np.testing.assert_array_equal(dw.logical(), HT.from_logical(ref, dtype).logical())
+
+
+# 3 x 3 filters at unit stride: rows of one to four 16-pixel steps, shares of the batch's rows that
+# start and end inside images, cross several, or are empty
+@pytest.mark.parametrize("x,k,steps", [
+    ([1, 32, 3, 1], 32, 1), ([21, 32, 5, 15], 64, 1), ([300, 32, 1, 16], 32, 1), ([40, 96, 14, 16], 64, 1),
+    ([9, 64, 13, 17], 32, 2), ([14, 320, 24, 24], 480, 2), ([3, 32, 50, 32], 160, 2),
+    ([5, 32, 19, 33], 96, 3), ([4, 64, 48, 48], 192, 3), ([2, 96, 7, 49], 32, 4), ([11, 32, 56, 56], 64, 4),
+])
+def test_direct_weight_gradient_shares(ctx, x, k, steps):
+    xt, dy = whole(k, x, capi.BFLOAT16, 2), whole(k + 1, [x[0], k] + x[2:], capi.BFLOAT16, 1)
+    w = [k, x[1], 3, 3]
+    dw = run_conv_wgrad(ctx, dy, xt, w, [1, 1], [1, 1], [1, 1], capi.BFLOAT16, tuned=True, w_dtype=capi.FLOAT)
+    assert ctx.last_kernel().startswith(f"conv_wgrad_direct steps={steps}"), ctx.last_kernel()
+    got = dw.logical()
+    if k > 300:  # (some blocks of a large one)
+        xt, dy = xt.logical()[:, 256:], dy.logical()[:, 416:]
+        np.testing.assert_array_equal(got[416:, 256:], oracle.conv_wgrad(dy, xt, [64, 64, 3, 3], [1, 1], [1, 1], [1, 1]))
+    else:
+        np.testing.assert_array_equal(got, oracle.conv_wgrad(dy.logical(), xt.logical(), w, [1, 1], [1, 1], [1, 1]))
