@@ -43,6 +43,8 @@ FhipKnobs parse_knobs() {
     k.wgrad_direct = atoi(e);
   if (const char *e = getenv("FUSILLI_HIP_SDPA_DECODE"))
     k.sdpa_decode = atoi(e);
+  if (const char *e = getenv("FUSILLI_HIP_SDPA_SPLIT"))
+    k.sdpa_split = atoi(e);
   if (const char *e = getenv("FUSILLI_HIP_DGRAD_ROWS"))
     k.dgrad_rf = atoi(e);
   if (const char *e = getenv("FUSILLI_HIP_GEMM_TILE"))

@@ -92,6 +92,7 @@ struct FhipKnobs {
   int conv_slices = 0;              // FUSILLI_HIP_CONV_SLICES (channel slices per workgroup of the register-filter kernel: 2 or 4; 0: planner)
   int wgrad_direct = -1;            // FUSILLI_HIP_WGRAD_DIRECT (-1: unset, 0: off)
   int sdpa_decode = -1;             // FUSILLI_HIP_SDPA_DECODE (-1: unset, 0: off, 1: wherever it can run)
+  int sdpa_split = -1;              // FUSILLI_HIP_SDPA_SPLIT, of the tiled kernel (the same)
   int dgrad_rf = -1;                // FUSILLI_HIP_DGRAD_ROWS (-1: unset, 0: off, n: rows per
                                     // tile, + 100 x column tiles per row of tiles)
 };

@@ -396,9 +396,13 @@ int fhip_decode_sdpa(fhip_ctx *ctx, const fhip_sdpa_desc *d, const void *q, cons
   const int64_t big = (g.Sq + 255) / 256, kvt = (kv + 63) / 64;
   const bool pairs = d->is_causal && big > 1;
   const double per = HD == 128 ? 1.45 : 1.063, first = pairs ? 7.9 : HD == 128 ? 4.32 : 3.34;
-  const double there = (d->is_causal ? 1.36 : 0.16) +
-                       ceil((double)(B * Hq * (pairs ? (big + 1) / 2 : big)) / 256.0) *
-                           (first + per * (pairs ? (double)(kvt * (big + 1)) / (double)big : (double)kvt));
+  double there = (d->is_causal ? 1.36 : 0.16) +
+                 ceil((double)(B * Hq * (pairs ? (big + 1) / 2 : big)) / 256.0) *
+                     (first + per * (pairs ? (double)(kvt * (big + 1)) / (double)big : (double)kvt));
+  // grouped heads folded, keys split between teams (never below 6)
+  const double cut = here > 6.0 && here < there ? fhip_flash_sdpa_us(d) : -1;
+  if (cut > 0 && cut < there)
+    there = cut;
   if (here >= there && forced != 1)
     return 0;
   if (tiles * g.splits >= (1ll << 31))

@@ -31,6 +31,12 @@
 //
 // Head dim 64 or 128 (template parameter); bf16 or f16.
 //
+// Where workgroups of 256 rows are few, or fill a round and a little more (SPLIT): 128 rows
+// per workgroup, of which both teams of four wavefronts own the same rows and take every
+// other key tile.  A team has rings of its own (two stages: a round of lead) and loads its own
+// tiles; in the end the teams exchange halves of O^T with their reference points and sums.  A
+// round is a little longer (twice the LDS-DMA) and there are half as many.
+//
 // Reference semantics: aten.scaled_dot_product_attention (reference
 // support/asm_emitter.h:2409-2468, node/sdpa_node.h:36-236), GQA by head
 // repetition, causal mask aligned top-left; mask tensors as in
@@ -38,6 +44,7 @@
 #include "common.h"
 #include "fast_paths.h"
 
+#include <cstdlib>
 #include <type_traits>
 
 namespace {
@@ -75,6 +82,15 @@ template <int HD> struct SdShape {
   // kernels that stage the mask: 8 KB per wavefront behind the rings
   static constexpr int kMaskB = 8192;
   static constexpr int kLdsMaskB = kLdsB + kWaves * kMaskB;
+  // SPLIT: rings per team, three stages each for head dim 64, otherwise what fits: two of V, and
+  // of K three, with a mask two.  The mask's elements are 16 bits at most.  Exchange:
+  // half of a wavefront's O^T, (m, l) of its lanes, its rows of half the features.
+  static constexpr int split_k(bool mask) { return HD == 64 || !mask ? 3 : 2; }
+  static constexpr int split_lds(bool mask) { return 2 * (split_k(mask) + (HD == 64 ? 3 : 2)) * kTileB; }
+  static constexpr int kSplitMaskB = 4096;
+  static constexpr int kSplitSend = HD * 64;
+  static constexpr int kSplitPitch = kRowB / 2 + 16;
+  static_assert(kWaves * (kSplitSend + 512 + 32 * kSplitPitch) <= split_lds(true), "LDS of the exchange");
 };
 
 struct SdpaArgs {
@@ -95,6 +111,7 @@ struct SdpaArgs {
   // the key stride is 1
   const char *mask;
   int64_t m_sb, m_sh, m_sq;
+  int32_t m_rows;   // rows of the mask: row r of a folded group reads row r % m_rows
   uint32_t m_bytes; // bytes of one (batch, head) slab
   int32_t m_dt;     // FHIP_BOOLEAN / FHIP_FLOAT / FHIP_BFLOAT16 / FHIP_HALF
 };
@@ -242,19 +259,26 @@ __device__ __forceinline__ void sd_barrier() {
 }
 
 // MASK: 0 no mask tensor, 1 mask read into registers, 2 mask staged in LDS
-template <bool BF16, bool CAUSAL, int HD, int MASK>
+template <bool BF16, bool CAUSAL, int HD, int MASK, bool SPLIT = false>
 __global__ __launch_bounds__(kWaves * 64) void sdpa_fwd_kernel(SdpaArgs g) {
   static_assert(!(CAUSAL && MASK), "a mask tensor excludes the causal flag");
+  static_assert(!(SPLIT && MASK == 1), "split keys stage their mask");
   using C = SdShape<HD>;
   constexpr int kD = HD;
   constexpr int kRowB = C::kRowB, kTileB = C::kTileB;
-  constexpr int kLoadsPerTile = C::kLoadsPerTile, kOutPitch = C::kOutPitch;
+  constexpr int kLoaders = SPLIT ? kWaves / 2 : kWaves; // wavefronts that bring a tile in
+  constexpr int kLoadsPerTile = kTileB / 1024 / kLoaders, kOutPitch = C::kOutPitch;
+  constexpr int kRows = SPLIT ? kBQ / 2 : kBQ;
+  constexpr bool kTight = SPLIT && HD == 128; // two stages of V
+  constexpr int kStagesK = kTight ? C::split_k(MASK != 0) : kStages;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
   // wave index as a scalar: everything derived from it stays in SGPRs
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l = threadIdx.x & 63;
   const int half = l >> 5, lq = l & 31;
+  const int team = __builtin_amdgcn_readfirstlane(wave >> 2);
+  const int loader = SPLIT ? wave & 3 : wave;
   // Causal masks: a workgroup runs query tile (last - z) and then tile z, a
   // long and a short one, so all workgroups do the same work (tiles of one
   // head need 1 .. n key-tile rows).  Otherwise one tile per workgroup.
@@ -270,15 +294,15 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_fwd_kernel(SdpaArgs g) {
     h = head % g.xcd_heads;
     b = head / g.xcd_heads;
   }
-  const int n_qtiles = (g.Sq + kBQ - 1) / kBQ;
+  const int n_qtiles = (g.Sq + kRows - 1) / kRows;
   const int passes = CAUSAL && n_qtiles - 1 - z != z ? 2 : 1;
   for (int pass = 0; pass < passes; ++pass) {
   const int qtile = CAUSAL && pass == 0 ? n_qtiles - 1 - z : z;
   if (pass) // the first tile's output staging has been read
     __builtin_amdgcn_s_barrier();
   const int hk = h / g.group;
-  const int q0 = qtile * kBQ;
-  const int qw0 = q0 + wave * 32; // first query row of this wavefront
+  const int q0 = qtile * kRows;
+  const int qw0 = q0 + loader * 32; // first query row of this wavefront
   const int qrow = qw0 + lq;      // query this lane's scores belong to
 
   const char *qp = g.q + (b * g.q_sb + h * g.q_sh) * 2;
@@ -291,10 +315,13 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_fwd_kernel(SdpaArgs g) {
   // number of key tiles this workgroup visits
   int kv_end = g.Skv;
   if (CAUSAL) {
-    const int last_q = q0 + kBQ - 1 < g.Sq - 1 ? q0 + kBQ - 1 : g.Sq - 1;
+    const int last_q = q0 + kRows - 1 < g.Sq - 1 ? q0 + kRows - 1 : g.Sq - 1;
     kv_end = last_q + 1 < g.Skv ? last_q + 1 : g.Skv;
   }
   const int tiles = (kv_end + kBKV - 1) / kBKV;
+  // the rounds they take, and the tile of this wavefront in round t
+  const int rounds = SPLIT ? (tiles + 1) / 2 : tiles;
+  auto tile_of = [&](int t) { return SPLIT ? 2 * t + team : t; };
 
   // ---- Q fragments (B operand of S^T = K Q^T): row lq, 8 d per register quad
   uint32_t qf[kD / 16][4];
@@ -315,7 +342,7 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_fwd_kernel(SdpaArgs g) {
   uint32_t koff[kLoadsPerTile], voff[kLoadsPerTile];
 #pragma unroll
   for (int j = 0; j < kLoadsPerTile; ++j) {
-    const int row = (j * kWaves + wave) * C::kRowsPerLoad + l / C::kChunks;
+    const int row = (j * kLoaders + loader) * C::kRowsPerLoad + l / C::kChunks;
     const int p = l % C::kChunks;
     koff[j] = (uint32_t)(row * k_rowb + ((p ^ sd_kswz<HD>(row)) << 4));
     voff[j] = (uint32_t)(row * v_rowb + (sd_vchunk<HD>(row, p) << 4));
@@ -343,10 +370,12 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_fwd_kernel(SdpaArgs g) {
   __amdgpu_buffer_rsrc_t m_rsrc = k_rsrc;
   if constexpr (MASK != 0)
     m_rsrc = slab_rsrc(g.mask + ((b * g.m_sb + h * g.m_sh) << m_esh), g.m_bytes);
+  // (eight divisions are 0.3 us of a short kernel: folded groups only)
+  auto m_row = [&](int r) { return g.m_rows != g.Sq ? r % g.m_rows : r; };
   // MASK == 1: one register load per run, issued at the top of a round
   uint32_t m_off = 0;
   if constexpr (MASK == 1) {
-    const int qr = qrow < g.Sq ? qrow : g.Sq - 1;
+    const int qr = m_row(qrow < g.Sq ? qrow : g.Sq - 1);
     m_off = (uint32_t)(((int64_t)qr * g.m_sq + half * 4) << m_esh);
   }
   u32x4 mreg[MASK == 1 ? 8 : 1];
@@ -370,7 +399,8 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_fwd_kernel(SdpaArgs g) {
   // region by LDS-DMA, 1 KB (16 / 8 / 4 whole rows) per instruction; chunk c of
   // row r sits at position c ^ ((r / 2) % chunks-per-row), which spreads the
   // runs that the lanes of a read touch over the banks.
-  const uint32_t m_lds = lds0 + (uint32_t)C::kLdsB + (uint32_t)wave * C::kMaskB;
+  const uint32_t m_lds = lds0 + (uint32_t)(SPLIT ? C::split_lds(true) : C::kLdsB) +
+                         (uint32_t)wave * (SPLIT ? C::kSplitMaskB : C::kMaskB);
   uint32_t m_dma[MASK == 2 ? 8 : 1]; // lane offsets of the DMA instructions
   uint32_t m_rd[MASK == 2 ? 8 : 1];  // LDS address of this lane's run i
   if constexpr (MASK == 2) {
@@ -380,7 +410,7 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_fwd_kernel(SdpaArgs g) {
     for (int j = 0; j < 8; ++j) {
       const int row = j * rows_per + l / cpr;
       const int c = (l % cpr) ^ ((row >> 1) & (cpr - 1));
-      const int qr = qw0 + row < g.Sq ? qw0 + row : g.Sq - 1;
+      const int qr = m_row(qw0 + row < g.Sq ? qw0 + row : g.Sq - 1);
       m_dma[j] = (uint32_t)((((int64_t)qr * g.m_sq) << m_esh) + c * 16);
     }
 #pragma unroll
@@ -391,10 +421,10 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_fwd_kernel(SdpaArgs g) {
     }
   }
   auto issue_mask = [&](int t) {
-    const int so = t < tiles ? (t * kBKV) << m_esh : 0;
+    const int so = tile_of(t) < tiles ? (tile_of(t) * kBKV) << m_esh : 0;
     const int n = 2 << m_esh; // instructions per tile
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
+    for (int j = 0; j < (SPLIT ? 4 : 8); ++j)
       if (j < n)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
             m_rsrc,
@@ -412,22 +442,35 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_fwd_kernel(SdpaArgs g) {
     else
       __builtin_amdgcn_s_waitcnt(sd_wait_imm(2 * kLoadsPerTile + 8));
   };
+  // kTight: only the next tile's mask, or (three stages, wavefronts 0..3) the K tile behind
+  // the next may be out
+  auto wait_tight = [&]() {
+    if (MASK != 2 && kStagesK == 3 && !team)
+      __builtin_amdgcn_s_waitcnt(sd_wait_imm(kLoadsPerTile));
+    else if (MASK != 2)
+      __builtin_amdgcn_s_waitcnt(sd_wait_imm(0));
+    else if (m_esh == 0)
+      __builtin_amdgcn_s_waitcnt(sd_wait_imm(2));
+    else
+      __builtin_amdgcn_s_waitcnt(sd_wait_imm(4));
+  };
   auto issue_kv = [&](const __amdgpu_buffer_rsrc_t &r, uint32_t tile_bytes,
                       const uint32_t (&off)[kLoadsPerTile], int t,
                       uint32_t stage) {
-    const uint32_t toff = t < tiles ? (uint32_t)t * tile_bytes : 0x80000000u;
+    const uint32_t toff = tile_of(t) < tiles ? (uint32_t)tile_of(t) * tile_bytes : 0x80000000u;
 #pragma unroll
     for (int j = 0; j < kLoadsPerTile; ++j) {
-      const uint32_t dst = stage + (uint32_t)(j * kWaves + wave) * 1024u;
+      const uint32_t dst = stage + (uint32_t)(j * kLoaders + loader) * 1024u;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           r, (SD_AS3 char *)(uintptr_t)__builtin_amdgcn_readfirstlane(dst), 16,
           (int)(off[j] + toff), 0, 0, 0);
     }
   };
   // ring slot (0 .. kStages - 1) -> LDS address
-  auto k_stage = [&](int slot) { return lds0 + (uint32_t)slot * kTileB; };
+  const uint32_t ring = lds0 + (SPLIT ? (uint32_t)team * (uint32_t)(C::split_lds(MASK != 0) / 2) : 0u);
+  auto k_stage = [&](int slot) { return ring + (uint32_t)slot * kTileB; };
   auto v_stage = [&](int slot) {
-    return lds0 + (uint32_t)(kStages + slot) * kTileB;
+    return ring + (uint32_t)(kStagesK + slot) * kTileB;
   };
   auto issue_k = [&](int t, int slot) {
     issue_kv(k_rsrc, (uint32_t)(kBKV * k_rowb), koff, t, k_stage(slot));
@@ -477,7 +520,10 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_fwd_kernel(SdpaArgs g) {
   // barrier t + 1 only K tile t + 1 and V tile t are read; the loads issued at
   // the top of round t (K tile t + 2, V tile t + 1) reuse the stages of K tile
   // t - 1 and V tile t - 2 and have to land by barrier t + 1.
-  const int team = __builtin_amdgcn_readfirstlane(wave >> 2);
+  // kTight: between barriers t and t + 1 a team reads its own tiles' K (t + 1) and V (t) only, and
+  // the stages of K (t) and V (t - 1) are free: wavefronts 4..7 refill them behind their
+  // barrier (K (t + 2), V (t + 1)), wavefronts 0..3 in front of the next MFMA phase (V (t + 1), and
+  // K (t + 2), or with three stages K (t + 3)).
   constexpr bool kLoadsInValuPhase = MASK == 0 && HD == 128;
 #ifndef SD_FUSE_PLAIN
 #define SD_FUSE_PLAIN 0
@@ -486,19 +532,29 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_fwd_kernel(SdpaArgs g) {
   if constexpr (MASK == 2)
     issue_mask(0); // older than every K / V load: landed by the first wait
   issue_k(0, 0);
-  issue_v(0, 0);
-  issue_k(1, 1);
-  // K tile 0 has landed
-  __builtin_amdgcn_s_waitcnt(sd_wait_imm(2 * kLoadsPerTile));
+  if (!kTight || team) {
+    issue_v(0, 0);
+    issue_k(1, 1);
+    // K tile 0 has landed
+    __builtin_amdgcn_s_waitcnt(sd_wait_imm(2 * kLoadsPerTile));
+  } else if (kStagesK == 3) {
+    issue_k(1, 1);
+    __builtin_amdgcn_s_waitcnt(sd_wait_imm(kLoadsPerTile));
+  } else {
+    __builtin_amdgcn_s_waitcnt(sd_wait_imm(0));
+  }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 
   uint32_t pf[4][4]; // probabilities as B-operand fragments, 16 keys each
   // a wavefront whose rows all lie above a tile has nothing to add
-  auto active = [&](int t) { return !(CAUSAL && t * kBKV > qw0 + 31); };
-  // ring slots of tile t - 1, t, t + 1, t + 2 (slot of t + 2 == slot of t - 1)
-  int sl_prev = kStages - 1, sl_cur = 0, sl_next = 1;
+  auto active = [&](int t) {
+    return !(CAUSAL && tile_of(t) * kBKV > qw0 + 31) && (!SPLIT || tile_of(t) < tiles);
+  };
+  // ring slots of tile t - 1, t, t + 1, t + 2 (slot of t + 2 == slot of t - 1, with two stages of t)
+  int sl_prev = kStagesK - 1, sl_cur = 0, sl_next = 1;
+  auto v_slot = [&](int t, int slot) { return kTight ? t & 1 : slot; };
   // One round.  The first (tile 0: no O^T update, and the softmax always takes
   // its full route) and the last (t == tiles: only the O^T update of the last
   // tile) are peeled off the loop as straight-line code, so that the loop holds
@@ -516,7 +572,15 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_fwd_kernel(SdpaArgs g) {
     // tens of clocks.  They go in front of the shorter of a round's two phases:
     // the MFMA phase with a mask tensor or head dim 64, the vector-ALU phase
     // otherwise (the SIMD's other wavefront feeds the matrix pipe meanwhile).
-    if constexpr (!kLoadsInValuPhase) {
+    if constexpr (kTight) {
+      if (!LAST && !team) {
+        issue_v(t, t & 1);
+        if constexpr (kStagesK == 3)
+          issue_k(t + 2, sl_prev);
+        else
+          issue_k(t + 1, sl_next);
+      }
+    } else if constexpr (!kLoadsInValuPhase) {
       issue_k(t + 2, sl_prev);
       issue_v(t + 1, sl_next);
     }
@@ -539,7 +603,7 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_fwd_kernel(SdpaArgs g) {
                   "groups do not straddle the two products");
     auto mfma_range = [&](auto first_c, auto last_c) __attribute__((always_inline)) {
       constexpr int M0 = decltype(first_c)::value, M1 = decltype(last_c)::value;
-      const uint32_t sk = k_stage(sl_cur) + kaddr0, sv = v_stage(sl_prev) + vaddr0;
+      const uint32_t sk = k_stage(sl_cur) + kaddr0, sv = v_stage(v_slot(t - 1, sl_prev)) + vaddr0;
       u32x4 kr[NS];
       u32x2 vr[NP][2];
       auto read = [&](auto mc) __attribute__((always_inline)) {
@@ -623,12 +687,21 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_fwd_kernel(SdpaArgs g) {
     // round has landed (which, in the vector-ALU phase, have not been issued
     // yet)
     if (team) {
-      __builtin_amdgcn_s_waitcnt(sd_wait_imm(kLoadsInValuPhase ? 0 : 2 * kLoadsPerTile));
+      if constexpr (kTight)
+        wait_tight();
+      else
+        __builtin_amdgcn_s_waitcnt(sd_wait_imm(kLoadsInValuPhase ? 0 : 2 * kLoadsPerTile));
       sd_barrier();
     }
     if constexpr (LAST)
       return;
-    if constexpr (kLoadsInValuPhase) {
+    if constexpr (kTight) {
+      if (team) {
+        issue_k(t + 2, kStagesK == 3 ? sl_prev : sl_cur);
+        issue_v(t + 1, (t + 1) & 1);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    } else if constexpr (kLoadsInValuPhase) {
       issue_k(t + 2, sl_prev);
       issue_v(t + 1, sl_next);
       __builtin_amdgcn_sched_barrier(0);
@@ -636,7 +709,7 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_fwd_kernel(SdpaArgs g) {
 
     // ---- vector-ALU phase -------------------------------------------------------
     if (active(t)) {
-      const int kv0 = t * kBKV;
+      const int kv0 = tile_of(t) * kBKV;
       // with a mask the scores are scaled here, with the mask folded in, and
       // the softmax below converts them to log2 units
       const float sl2 = MASK ? 1.4426950408889634f : g.scale_log2e;
@@ -852,18 +925,21 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_fwd_kernel(SdpaArgs g) {
     }
     // wavefronts 0..3 end their round here
     if (!team) {
-      wait_all_but_round();
+      if constexpr (kTight)
+        wait_tight();
+      else
+        wait_all_but_round();
       sd_barrier();
     }
     sl_prev = sl_cur;
     sl_cur = sl_next;
-    sl_next = next_slot(sl_next);
+    sl_next = kStagesK == 2 ? sl_prev : next_slot(sl_next);
   };
   round(0, std::integral_constant<int, 0>{});
 #pragma clang loop unroll(disable)
-  for (int t = 1; t < tiles; ++t)
+  for (int t = 1; t < rounds; ++t)
     round(t, std::integral_constant<int, 1>{});
-  round(tiles, std::integral_constant<int, 2>{});
+  round(rounds, std::integral_constant<int, 2>{});
   if (!team) // pairs with the last barrier of wavefronts 4..7
     __builtin_amdgcn_s_barrier();
 
@@ -872,6 +948,61 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_fwd_kernel(SdpaArgs g) {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  char *op = g.o + (b * g.o_sb + h * g.o_sh) * 2;
+  if constexpr (SPLIT) {
+    // A wavefront keeps half of the features, its team's, and sends the others to the wavefront
+    // that owns the same rows in the other team.
+    constexpr int H = kD / 64; // blocks of 32 features
+    const float sl2 = MASK ? 1.4426950408889634f : g.scale_log2e;
+    const uint32_t send = lds0 + (uint32_t)wave * C::kSplitSend, recv = lds0 + (uint32_t)(wave ^ 4) * C::kSplitSend;
+    const uint32_t ml0 = lds0 + (uint32_t)kWaves * C::kSplitSend;
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int i = 0; i < H; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; r += 4) {
+        f32x4 x;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float first = o[i][r + e], second = o[i + H][r + e];
+          x[e] = team ? first : second;
+          o[i][r + e] = team ? second : first;
+        }
+        *(SD_AS3 f32x4 *)(uintptr_t)(send + (uint32_t)((i * 4 + r / 4) * 1024 + l * 16)) = x;
+      }
+    *(SD_AS3 f32x2 *)(uintptr_t)(ml0 + (uint32_t)(wave * 64 + l) * 8) = f32x2{m_run, l_run};
+    __syncthreads();
+    const f32x2 other = *(const SD_AS3 f32x2 *)(uintptr_t)(ml0 + (uint32_t)((wave ^ 4) * 64 + l) * 8);
+    const float top = fmaxf(m_run, other.x);
+    const float mine = __builtin_amdgcn_exp2f((m_run - top) * sl2), theirs = __builtin_amdgcn_exp2f((other.x - top) * sl2);
+    const float inv = 1.0f / sd_half_sum(l_run * mine + other.y * theirs);
+    const uint32_t band = lds0 + (uint32_t)kWaves * (C::kSplitSend + 512) + (uint32_t)wave * (32 * C::kSplitPitch);
+#pragma unroll
+    for (int i = 0; i < H; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; r += 4) {
+        const f32x4 x = *(const SD_AS3 f32x4 *)(uintptr_t)(recv + (uint32_t)((i * 4 + r / 4) * 1024 + l * 16));
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          v[e] = (o[i][r + e] * mine + x[e] * theirs) * inv;
+        u32x2 w2;
+        w2.x = sd_pack<BF16>(v[0], v[1]);
+        w2.y = sd_pack<BF16>(v[2], v[3]);
+        *(SD_AS3 u32x2 *)(uintptr_t)(band + lq * C::kSplitPitch + (i * 32 + r * 2 + half * 4) * 2) = w2;
+      }
+    constexpr int kHalf = C::kChunks / 2; // lanes that cover half an output row
+#pragma unroll
+    for (int rows = 0; rows < 32; rows += 64 / kHalf) {
+      const int row = rows + l / kHalf;
+      const int cb = (l % kHalf) * 16;
+      const u32x4 v = *(const SD_AS3 u32x4 *)(uintptr_t)(band + row * C::kSplitPitch + cb);
+      const int qr = qw0 + row;
+      if (qr < g.Sq)
+        *(SD_AS1 u32x4 *)(op + (int64_t)qr * g.o_ss * 2 + team * (kRowB / 2) + cb) = v;
+    }
+  } else {
   const float inv = 1.0f / sd_half_sum(l_run);
   const uint32_t band = lds0 + (uint32_t)wave * (32 * kOutPitch);
   // lane holds query lq, features 32*dt + 8*(r/4) + 4*half + r%4
@@ -885,7 +1016,6 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_fwd_kernel(SdpaArgs g) {
       *(SD_AS3 u32x2 *)(uintptr_t)(band + lq * kOutPitch +
                                    (dt * 32 + r4 * 8 + half * 4) * 2) = w2;
     }
-  char *op = g.o + (b * g.o_sb + h * g.o_sh) * 2;
   // kChunks lanes cover one output row; 4 or 8 rows per pass
 #pragma unroll
   for (int rows = 0; rows < 32; rows += C::kRowsPerLoad) {
@@ -896,6 +1026,7 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_fwd_kernel(SdpaArgs g) {
     const int qr = qw0 + row;
     if (qr < g.Sq)
       *(SD_AS1 u32x4 *)(op + (int64_t)qr * g.o_ss * 2 + cb) = v;
+  }
   }
   } // pass
 }
@@ -981,10 +1112,96 @@ SdpaPlan make_plan(const fhip_sdpa_desc *d) {
   return p;
 }
 
+// How a problem is cut: rows of a (folded) head, heads, teams on the same rows.
+struct SdpaChoice {
+  int64_t rows, heads;
+  int fold = 0; // a group's rows are one matrix: 1 head after head, 2 position after position
+  bool split = false;
+  double us = 0;
+};
+
+// Microseconds of the kernel, fitted to its times on 400 problems (16 to 4096 queries and keys, 1 to
+// 128 heads, batches to 8; 6 to 13 % off): start, one pass over a workgroup's rows, one key tile
+// (SPLIT: a tile for each team), times rounds of 256 workgroups.
+double sdpa_us(const fhip_sdpa_desc *d, int64_t rows, int64_t heads, bool split) {
+  static const double fits[2][3][2][3] = {
+      // no mask, causal, mask tensor; whole, split
+      {{{0.02, 4.52, 1.000}, {0.90, 3.84, 1.062}}, {{1.38, 3.74, 1.036}, {1.99, 3.52, 1.178}}, {{0.0, 4.75, 1.404}, {0.81, 4.30, 1.561}}},
+      {{{0.0, 6.33, 1.338}, {0.0, 6.27, 1.628}}, {{0.0, 6.22, 1.439}, {1.30, 5.60, 1.755}}, {{0.0, 6.70, 1.814}, {0.0, 6.63, 2.201}}}};
+  const double *f = fits[d->q.dim[3] == 128][d->mask.rank ? 2 : d->is_causal ? 1 : 0][split];
+  const int64_t bq = split ? kBQ / 2 : kBQ, big = (rows + bq - 1) / bq, Skv = d->k.dim[2];
+  int64_t groups = big, iters = 0;
+  auto walk = [&](int64_t keys) {
+    const int64_t tiles = (keys + kBKV - 1) / kBKV;
+    return split ? (tiles + 1) / 2 : tiles;
+  };
+  if (d->is_causal) {
+    groups = (big + 1) / 2;
+    auto upto = [&](int64_t i) {
+      const int64_t last = (i + 1) * bq < rows ? (i + 1) * bq : rows;
+      return walk(last < Skv ? last : Skv);
+    };
+    // (a pair's keys: most in the first pair, or, where all keys lie in front, in the last)
+    for (const int64_t z : {(int64_t)0, groups - 1}) {
+      const int64_t n = upto(big - 1 - z) + (big - 1 - z != z ? upto(z) : 0);
+      iters = n > iters ? n : iters;
+    }
+  } else {
+    iters = walk(Skv);
+  }
+  const int64_t wgs = d->q.dim[0] * heads * groups;
+  return f[0] + (double)((wgs + 255) / 256) * (f[1] * (d->is_causal && big > 1 ? 2.0 : 1.0) + f[2] * (double)iters);
+}
+
+// `may_split`: the mask tensor, if any, can be staged beside the teams' rings.
+SdpaChoice choose(const fhip_sdpa_desc *d, bool may_split) {
+  const int64_t Sq = d->q.dim[2], Hq = d->q.dim[1], Hkv = d->k.dim[1], group = Hq / Hkv, Skv = d->k.dim[2];
+  SdpaChoice best{Sq, Hq};
+  const int forced = fhip_knobs().sdpa_split;
+  const bool only_split = forced == 1 && may_split;
+  best.us = only_split ? 1e30 : sdpa_us(d, Sq, Hq, false);
+  auto consider = [&](int64_t rows, int64_t heads, int fold, bool split, double us) {
+    if (us < best.us)
+      best = SdpaChoice{rows, heads, fold, split, us};
+  };
+  // Split keys: half the work per workgroup, for rounds that are not full: B1, 16 heads, 2200 causal,
+  // D128, 80 workgroups 65 us, so 46; B3, 8 heads, 2624 under a mask, 264 workgroups 155 / 120; full
+  // rounds are 7 to 20 % slower so.  Two key tiles and fewer are over before it shows.
+  const bool split_pays = only_split || (may_split && forced != 0 && Skv > 2 * kBKV && Sq <= 65535ll * (kBQ / 2));
+  if (split_pays)
+    consider(Sq, Hq, 0, true, 1.05 * sdpa_us(d, Sq, Hq, true));
+  // Grouped heads read the same keys: where no causal mask tells their rows apart, and the mask tensor
+  // is the same for all of them, they are the rows of one head (B3, 128 heads on 16, 64 x 3052, D128
+  // 150 us, folded 67, folded and split 48).  As many rounds: 3 to 10 % faster with long
+  // keys, whose tiles more workgroups side by side share; short ones lose 0.5 us.
+  const fhip_tensor_desc &m = d->mask;
+  const bool same_mask = m.rank == 0 || m.dim[1] == 1 || m.stride[1] == 0;
+  if (group > 1 && !d->is_causal && same_mask && Sq * group <= 65535ll * (kBQ / 2)) {
+    auto runs = [&](const fhip_tensor_desc &t) { return t.stride[1] == Sq * t.stride[2]; };
+    auto turns = [&](const fhip_tensor_desc &t) { return Sq == 1 || t.stride[2] == group * t.stride[1]; };
+    const int fold = Sq > 1 && runs(d->q) && runs(d->o)                            ? 1
+                     : m.rank == 0 && Hkv == 1 && turns(d->q) && turns(d->o) ? 2
+                                                                             : 0;
+    if (fold) {
+      auto of = [&](double us) { return Skv >= (m.rank ? 1024 : 512) ? 0.97 * us : us + 0.5; };
+      if (!only_split)
+        consider(Sq * group, Hkv, fold, false, of(sdpa_us(d, Sq * group, Hkv, false)));
+      if (split_pays)
+        consider(Sq * group, Hkv, fold, true, of(1.05 * sdpa_us(d, Sq * group, Hkv, true)));
+    }
+  }
+  return best;
+}
+
 } // namespace
 
 bool fhip_fast_sdpa_applicable(const fhip_sdpa_desc *d) {
   return make_plan(d).ok;
+}
+
+double fhip_flash_sdpa_us(const fhip_sdpa_desc *d) {
+  const SdpaChoice c = choose(d, true);
+  return c.split || c.fold ? c.us : -1;
 }
 
 int fhip_fast_sdpa(fhip_ctx *ctx, const fhip_sdpa_desc *d, const void *q,
@@ -1002,6 +1219,14 @@ int fhip_fast_sdpa(fhip_ctx *ctx, const fhip_sdpa_desc *d, const void *q,
       return rc;
   }
   bool staged_mask = false;
+  if (p.mask) {
+    FHIP_REQUIRE(ctx, mask != nullptr, "sdpa: mask descriptor without a mask");
+    FHIP_REQUIRE(ctx,
+                 ((uintptr_t)mask & (4 * fhip_dtype_size(d->mask.dtype) - 1)) == 0,
+                 "sdpa: the mask must be aligned to four of its elements");
+    staged_mask = p.mask_rows16 && ((uintptr_t)mask & 15) == 0;
+  }
+  const SdpaChoice c = choose(d, !p.mask || (staged_mask && fhip_dtype_size(d->mask.dtype) <= 2));
   SdpaArgs g{};
   g.q = (const char *)q;
   g.k = (const char *)k;
@@ -1014,18 +1239,18 @@ int fhip_fast_sdpa(fhip_ctx *ctx, const fhip_sdpa_desc *d, const void *q,
   g.k_sb = st(d->k, 0), g.k_sh = st(d->k, 1), g.k_ss = st(d->k, 2);
   g.v_sb = st(d->v, 0), g.v_sh = st(d->v, 1), g.v_ss = st(d->v, 2);
   g.o_sb = st(d->o, 0), g.o_sh = st(d->o, 1), g.o_ss = st(d->o, 2);
-  g.Sq = (int32_t)d->q.dim[2];
+  g.Sq = (int32_t)c.rows;
   g.Skv = (int32_t)d->k.dim[2];
-  g.group = (int32_t)(d->q.dim[1] / d->k.dim[1]);
+  g.group = (int32_t)(c.heads / d->k.dim[1]);
+  if (c.fold == 1) // a group's rows, head after head
+    g.q_sh *= d->q.dim[1] / d->k.dim[1], g.o_sh *= d->q.dim[1] / d->k.dim[1];
+  else if (c.fold == 2) // position after position
+    g.q_ss = g.q_sh, g.q_sh = 0, g.o_ss = g.o_sh, g.o_sh = 0;
   g.causal = d->is_causal;
   if (p.mask) {
-    FHIP_REQUIRE(ctx, mask != nullptr, "sdpa: mask descriptor without a mask");
-    FHIP_REQUIRE(ctx,
-                 ((uintptr_t)mask & (4 * fhip_dtype_size(d->mask.dtype) - 1)) == 0,
-                 "sdpa: the mask must be aligned to four of its elements");
-    staged_mask = p.mask_rows16 && ((uintptr_t)mask & 15) == 0;
     g.mask = (const char *)mask;
     g.m_sb = p.m_st[0], g.m_sh = p.m_st[1], g.m_sq = p.m_st[2];
+    g.m_rows = (int32_t)d->q.dim[2];
     g.m_bytes = p.m_bytes;
     g.m_dt = d->mask.dtype;
   }
@@ -1033,13 +1258,15 @@ int fhip_fast_sdpa(fhip_ctx *ctx, const fhip_sdpa_desc *d, const void *q,
       d->has_scale ? d->scale : 1.0f / sqrtf((float)d->q.dim[3]);
   g.scale_log2e = scale * 1.4426950408889634f;
   g.scale = scale;
-  const int n_qtiles = (g.Sq + kBQ - 1) / kBQ;
+  const bool split = c.split;
+  const int rows = split ? kBQ / 2 : kBQ;
+  const int n_qtiles = (g.Sq + rows - 1) / rows;
   const int64_t groups = d->is_causal ? (n_qtiles + 1) / 2 : n_qtiles;
-  const int64_t heads = d->q.dim[1] * d->q.dim[0];
-  dim3 grid((unsigned)d->q.dim[1], (unsigned)d->q.dim[0], (unsigned)groups);
+  const int64_t heads = c.heads * d->q.dim[0];
+  dim3 grid((unsigned)c.heads, (unsigned)d->q.dim[0], (unsigned)groups);
   if (heads % 8 == 0 && groups > 1 && heads * groups < (1ll << 31) &&
       std::getenv("FUSILLI_HIP_SDPA_GRID") == nullptr) {
-    g.xcd_heads = (int32_t)d->q.dim[1];
+    g.xcd_heads = (int32_t)c.heads;
     g.xcd_groups = (int32_t)groups;
     grid = dim3((unsigned)(heads * groups));
   }
@@ -1057,30 +1284,26 @@ int fhip_fast_sdpa(fhip_ctx *ctx, const fhip_sdpa_desc *d, const void *q,
     return 0;
   };
   // one flag per kernel instance: [head dim][type][plain / causal / mask in
-  // registers / mask staged in LDS]
-  static FhipOncePerDevice configured[2][2][4];
-  fhip_note_kernel(ctx, "sdpa_fwd d=%d causal=%d mask=%d", p.hd, (int)(d->is_causal != 0),
-                   p.mask ? (staged_mask ? 2 : 1) : 0);
-  auto pick = [&](auto hd) {
+  // registers / mask staged in LDS, the first two and the last again with split keys]
+  static FhipOncePerDevice configured[2][2][8];
+  fhip_note_kernel(ctx, "sdpa_fwd d=%d causal=%d mask=%d%s%s", p.hd, (int)(d->is_causal != 0),
+                   p.mask ? (staged_mask ? 2 : 1) : 0, c.fold ? " folded" : "", split ? " split" : "");
+  auto pick = [&](auto hd, auto bf) {
     constexpr int HD = decltype(hd)::value;
-    FhipOncePerDevice(&cfg)[2][4] = configured[HD == 128];
-    constexpr int lds = SdShape<HD>::kLdsB;
-    constexpr int lds_mask = SdShape<HD>::kLdsMaskB;
-    if (p.mask && staged_mask)
-      return p.bf16
-                 ? launch(sdpa_fwd_kernel<true, false, HD, 2>, lds_mask, cfg[1][3])
-                 : launch(sdpa_fwd_kernel<false, false, HD, 2>, lds_mask, cfg[0][3]);
+    constexpr bool BF = decltype(bf)::value;
+    using C = SdShape<HD>;
+    FhipOncePerDevice(&cfg)[8] = configured[HD == 128][BF];
+    if (split)
+      return p.mask           ? launch(sdpa_fwd_kernel<BF, false, HD, 2, true>, C::split_lds(true) + kWaves * C::kSplitMaskB, cfg[7])
+             : d->is_causal ? launch(sdpa_fwd_kernel<BF, true, HD, 0, true>, C::split_lds(false), cfg[5])
+                            : launch(sdpa_fwd_kernel<BF, false, HD, 0, true>, C::split_lds(false), cfg[4]);
     if (p.mask)
-      return p.bf16 ? launch(sdpa_fwd_kernel<true, false, HD, 1>, lds, cfg[1][2])
-                    : launch(sdpa_fwd_kernel<false, false, HD, 1>, lds, cfg[0][2]);
-    if (p.bf16)
-      return d->is_causal
-                 ? launch(sdpa_fwd_kernel<true, true, HD, 0>, lds, cfg[1][1])
-                 : launch(sdpa_fwd_kernel<true, false, HD, 0>, lds, cfg[1][0]);
-    return d->is_causal
-               ? launch(sdpa_fwd_kernel<false, true, HD, 0>, lds, cfg[0][1])
-               : launch(sdpa_fwd_kernel<false, false, HD, 0>, lds, cfg[0][0]);
+      return staged_mask ? launch(sdpa_fwd_kernel<BF, false, HD, 2>, C::kLdsMaskB, cfg[3])
+                         : launch(sdpa_fwd_kernel<BF, false, HD, 1>, C::kLdsB, cfg[2]);
+    return d->is_causal ? launch(sdpa_fwd_kernel<BF, true, HD, 0>, C::kLdsB, cfg[1])
+                        : launch(sdpa_fwd_kernel<BF, false, HD, 0>, C::kLdsB, cfg[0]);
   };
-  return p.hd == 128 ? pick(std::integral_constant<int, 128>{})
-                     : pick(std::integral_constant<int, 64>{});
+  auto typed = [&](auto hd) { return p.bf16 ? pick(hd, std::true_type{}) : pick(hd, std::false_type{}); };
+  return p.hd == 128 ? typed(std::integral_constant<int, 128>{})
+                     : typed(std::integral_constant<int, 64>{});
 }

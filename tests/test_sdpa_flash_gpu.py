@@ -277,3 +277,129 @@ def test_flash_head_dim_64_many_tiles(ctx):
     vl = v.logical()[0, 1]
     assert_close(out[0, 1], np.cumsum(vl, axis=0) / np.arange(1, S + 1)[:, None],
                  capi.BFLOAT16, "uniform head")
+
+
+# Keys split between the two teams of a workgroup of 128 rows: odd tile counts (one team has a tile
+# less, or none), rows and keys off the tiles, wavefronts and whole teams above a causal diagonal.
+SPLIT_CASES = CASES + [
+    dict(B=1, Hq=2, Hkv=2, Sq=129, Skv=64, causal=False),
+    dict(B=1, Hq=1, Hkv=1, Sq=128, Skv=449, causal=False),
+    dict(B=1, Hq=2, Hkv=1, Sq=700, Skv=700, causal=True),
+    dict(B=1, Hq=1, Hkv=1, Sq=400, Skv=130, causal=True),
+]
+
+
+@pytest.mark.parametrize("case", SPLIT_CASES)
+@pytest.mark.parametrize("dtype", [capi.BFLOAT16, capi.HALF])
+@pytest.mark.parametrize("hd", [128, 64])
+def test_flash_split_keys_vs_oracle(ctx, knobs, case, dtype, hd):
+    knobs(SDPA_DECODE=0, SDPA_SPLIT=1)
+    c = case
+    # (scores far apart: the teams' reference points differ)
+    q = HT.from_logical(rand(61, 0, [c["B"], c["Hq"], c["Sq"], hd], std=3.0), dtype)
+    k = HT.from_logical(rand(61, 1, [c["B"], c["Hkv"], c["Skv"], hd], std=2.0), dtype)
+    v = HT.from_logical(rand(61, 2, [c["B"], c["Hkv"], c["Skv"], hd]), dtype)
+    out = run(ctx, q, k, v, causal=c["causal"])
+    assert ctx.last_kernel().endswith("split"), ctx.last_kernel()
+    ref = oracle.sdpa(q.logical(), k.logical(), v.logical(), is_causal=c["causal"])
+    assert_close(out.logical(), ref, dtype, str(case))
+
+
+@pytest.mark.parametrize("case", MASK_CASES + [dict(B=2, Hq=6, Hkv=2, Sq=100, Skv=328, mdims="b1qk")])
+@pytest.mark.parametrize("mdt", [capi.BOOLEAN, capi.BFLOAT16, capi.HALF, capi.FLOAT])
+@pytest.mark.parametrize("hd", [128, 64])
+def test_flash_split_keys_mask_tensor(ctx, knobs, case, mdt, hd):
+    knobs(SDPA_SPLIT=1)
+    c = case
+    q = HT.from_logical(rand(62, 0, [c["B"], c["Hq"], c["Sq"], hd]), capi.BFLOAT16)
+    k = HT.from_logical(rand(62, 1, [c["B"], c["Hkv"], c["Skv"], hd]), capi.BFLOAT16)
+    v = HT.from_logical(rand(62, 2, [c["B"], c["Hkv"], c["Skv"], hd]), capi.BFLOAT16)
+    dims = mask_dims(c)
+    if mdt == capi.BOOLEAN:
+        m = (rand(62, 3, dims) > -0.5).astype(np.float64)
+        m[..., -1] = 1  # (no row without a key)
+    else:
+        m = rand(62, 3, dims)
+    mask = HT.from_logical(m, mdt)
+    out = run(ctx, q, k, v, mask=mask)
+    es = {capi.BOOLEAN: 1, capi.FLOAT: 4}.get(mdt, 2)
+    # staged masks of 16 bits and less; the others run whole
+    assert ctx.last_kernel().endswith("split") == (c["Skv"] * es % 16 == 0 and es <= 2), ctx.last_kernel()
+    ml = mask.logical()
+    ref = oracle.sdpa(q.logical(), k.logical(), v.logical(), mask=ml.astype(bool) if mdt == capi.BOOLEAN else ml)
+    assert_close(out.logical(), ref, capi.BFLOAT16, str(case))
+
+
+@pytest.mark.parametrize("layout", ["bhsd", "bshd"])
+@pytest.mark.parametrize("hkv", [1, 2])
+@pytest.mark.parametrize("split", [0, 1])
+@pytest.mark.parametrize("sq", [1, 70])
+def test_flash_folded_groups(ctx, knobs, layout, hkv, split, sq):
+    # a group's heads as the rows of one head: one after another, or position after position (one key head)
+    knobs(SDPA_DECODE=0, SDPA_SPLIT=split)
+    dims = [3, 8 * hkv, sq, 128]
+    kd = [3, hkv, 1030, 128]
+    st = bshd_strides(dims) if layout == "bshd" else None
+    q = HT.from_logical(rand(63, 0, dims, std=2.0), capi.BFLOAT16, st)
+    k, v = (HT.from_logical(rand(63, i, kd), capi.BFLOAT16) for i in (1, 2))
+    out = run(ctx, q, k, v, o_strides=st)
+    folds = sq > 1 and (layout == "bhsd" or hkv == 1) or sq == 1 and hkv == 1
+    assert ("folded" in ctx.last_kernel()) == folds, ctx.last_kernel()
+    assert_close(out.logical(), oracle.sdpa(q.logical(), k.logical(), v.logical()), capi.BFLOAT16)
+
+
+@pytest.mark.parametrize("causal,masked,hd", [(False, False, 128), (True, False, 128), (False, True, 64)])
+def test_flash_split_keys_lose_no_precision(ctx, knobs, causal, masked, hd):
+    # Probabilities are rounded against each team's reference point: the error against 64 bits may not
+    # grow (sums over 100 000 independent roundings; the ratio moves by a percent or so).
+    dims = [1, 4, 400, hd]
+    q, k, v = (HT.from_logical(rand(64, i, dims, std=1.5), capi.BFLOAT16) for i in range(3))
+    m = HT.from_logical(rand(64, 3, [1, 1, 400, 400]), capi.BFLOAT16) if masked else None
+    s = np.einsum("bhqd,bhkd->bhqk", q.logical().astype(np.float64), k.logical()) / np.sqrt(hd)
+    if masked:
+        s += m.logical()
+    if causal:
+        s[..., np.triu(np.ones((400, 400), bool), 1)] = -np.inf
+    p = np.exp(s - s.max(-1, keepdims=True))
+    ref = np.einsum("bhqk,bhkd->bhqd", p / p.sum(-1, keepdims=True), v.logical().astype(np.float64))
+    err = []
+    for split in (0, 1):
+        knobs(SDPA_DECODE=0, SDPA_SPLIT=split)
+        out = run(ctx, q, k, v, causal=causal, mask=m)
+        assert ctx.last_kernel().endswith("split") == bool(split), ctx.last_kernel()
+        err.append(np.linalg.norm(out.logical() - ref) / np.linalg.norm(ref))
+    assert err[1] <= 1.02 * err[0], err
+
+
+def test_flash_route_of_split_and_folded_problems(ctx):
+    # both sides of the rule, as measured
+    def name(b, hq, hkv, sq, skv, hd, causal=False):
+        q = HT.from_logical(rand(65, 0, [b, hq, sq, hd]), capi.BFLOAT16)
+        k = HT.from_logical(rand(65, 1, [b, hkv, skv, hd]), capi.BFLOAT16)
+        run(ctx, q, k, k, causal=causal)
+        return ctx.last_kernel()
+    assert name(1, 16, 16, 2200, 2200, 128, True).endswith("split")
+    assert name(1, 64, 8, 64, 3052, 128).endswith("folded split")
+    assert name(3, 32, 4, 623, 623, 128).endswith("folded")
+    assert name(2, 32, 32, 1664, 1664, 64).endswith("mask=0")
+    assert name(4, 32, 32, 669, 669, 128, True).endswith("mask=0")
+
+
+@pytest.mark.parametrize("hd", [128, 64])
+def test_flash_split_keys_dead_rows(ctx, knobs, hd):
+    # rows whose keys are all dead, and rows whose keys are dead in one team's tiles only
+    knobs(SDPA_SPLIT=1)
+    q, k, v = (HT.from_logical(rand(66, i, [1, 2, 96, hd]), capi.HALF) for i in range(3))
+    k, v = (HT.from_logical(rand(66, i, [1, 2, 320, hd]), capi.HALF) for i in (1, 2))
+    m = rand(66, 3, [1, 1, 96, 320]).astype(np.float32)
+    m[0, 0, 17] = -np.inf
+    even = np.arange(320) // 64 % 2 == 0
+    m[0, 0, 20, even] = -np.inf
+    m[0, 0, 40, ~even] = -np.inf
+    mask = HT.from_logical(m, capi.HALF)
+    out = run(ctx, q, k, v, mask=mask).logical()
+    assert ctx.last_kernel().endswith("split"), ctx.last_kernel()
+    assert np.all(np.isnan(out[:, :, 17]))
+    rows = np.arange(96) != 17
+    ref = oracle.sdpa(q.logical(), k.logical(), v.logical(), mask=mask.logical())
+    assert_close(out[:, :, rows], ref[:, :, rows], capi.HALF)
