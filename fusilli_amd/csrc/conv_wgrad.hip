@@ -1,5 +1,5 @@
 // Convolution weight gradient for channels-last 16-bit tensors, any filter, stride,
-// padding and dilation (3 x 3 filters at unit stride have conv_wgrad_direct.hip).
+// padding and dilation (most 3 x 3 filters at unit stride have conv_wgrad_direct.hip).
 //
 //   DW[k, (r, s, c)] = sum over output pixels m of
 //                      DY[m, k] * X[pixel of m shifted by (r, s), c]
@@ -499,9 +499,13 @@ bool fhip_fast_conv_wgrad_applicable(const fhip_conv_desc *d,
 }
 
 int fhip_fast_conv_wgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy,
-                         const void *x, void *dw, void *workspace) {
-  if (fhip_fast_conv_wgrad_direct_applicable(d, nullptr))
-    return fhip_fast_conv_wgrad_direct(ctx, d, dy, x, dw, workspace);
+                         const void *x, void *dw, void *workspace, size_t workspace_bytes) {
+  {
+    bool handled = false;
+    const int rc = fhip_fast_conv_wgrad_direct(ctx, d, dy, x, dw, workspace, workspace_bytes, &handled);
+    if (handled || rc != 0)
+      return rc;
+  }
   const WgradPlan p = make_wgrad_plan(d);
   FHIP_REQUIRE(ctx, p.ok, "conv wgrad: descriptor not supported by the MFMA path");
   FHIP_REQUIRE(ctx, ((uintptr_t)workspace & 255) == 0 && ((uintptr_t)x & 15) == 0 &&
@@ -514,7 +518,12 @@ int fhip_gather_conv_wgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *d
                            void *dw, bool *handled) {
   *handled = false;
   const WgradPlan p = make_wgrad_plan(d);
-  if (!p.ok || (((uintptr_t)x | (uintptr_t)dy) & 15) != 0 || !fhip_ctx_scratch_ready(ctx, p.part_bytes))
+  if (!p.ok || (((uintptr_t)x | (uintptr_t)dy) & 15) != 0)
+    return 0;
+  const int rc = fhip_fast_conv_wgrad_direct(ctx, d, dy, x, dw, nullptr, 0, handled);
+  if (*handled || rc != 0)
+    return rc;
+  if (!fhip_ctx_scratch_ready(ctx, p.part_bytes))
     return 0;
   void *scratch = nullptr;
   if (fhip_ctx_scratch(ctx, p.part_bytes, &scratch) != 0)

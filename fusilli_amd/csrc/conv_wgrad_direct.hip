@@ -1,9 +1,9 @@
 // Convolution weight gradient for 3 x 3 filters, straight from X and DY.
 //
-//   DW[k, r, s, c] = sum over n, p, q of DY[n, p, q, k] * X[n, p + r - 1, q + s - 1, c]
+//   DW[k, r, s, c] = sum over n, p, q of DY[n, p, q, k] * X[n, p + r - pad, q + s - pad, c]
 //
 // (channels-last 16-bit tensors, one group, unit strides and dilations,
-// padding 1, images of up to 56 columns, C and K multiples of 32).  As a GEMM
+// padding up to 2 on all sides, DY of up to 56 columns, C and K multiples of 8).  As a GEMM
 // this is skinny: 9 * C * K outputs, reduced over every pixel of the batch, and
 // the reduction runs along the tensors' slow dimension.  The kernel therefore
 //
@@ -16,7 +16,7 @@
 //    MFMA operands out of them with transposing reads: 16 consecutive pixels of
 //    a row are the K extent of one 32 x 32 x 16 MFMA, and a row takes as many
 //    as it has (NKS), not the four of the widest;
-//  * walks the rows of X: row rho pairs with the DY rows rho + 1, rho, rho - 1
+//  * walks the rows of X: row rho pairs with the DY rows rho + pad, rho + pad - 1, rho + pad - 2
 //    (filter rows 0, 1, 2), whose fragments stay in registers for the three
 //    visits, and the three column taps are the same LDS row read one pixel
 //    apart -- six fragment reads feed nine MFMAs;
@@ -60,10 +60,11 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 struct WgDirectArgs {
   const char *x, *dy;
   float *part;
-  int32_t H, W, C, K;
-  int32_t rows;   // of the batch: N * H
+  int32_t H, W, C, K, P, Q;
+  int32_t pad;
+  int32_t rows;   // of X: N * H
   int32_t nparts; // workgroups per (k, c) block
-  int32_t types, ctypes; // blocks, C / 32
+  int32_t types, ctypes; // blocks, C / 32 rounded up
   int32_t total, per_xcd; // types * nparts, an eighth of it rounded up
   uint32_t magic_types, magic_ctypes, magic_h;
   uint32_t x_bytes, dy_bytes;
@@ -138,44 +139,45 @@ conv_wgrad_direct_kernel(WgDirectArgs g) {
   const int first = row0 + (((row1 - row0) * wave) >> 3);
   const int last = row0 + (((row1 - row0) * (wave + 1)) >> 3);
 
-  // A walk over rows [first, last) of the batch, cut into the images' runs.  Step t of a run
-  // that starts at row p0 of its image brings DY row p0 - 1 + t into registers and, from
+  // A walk over rows [first, last) of X, cut into the images' runs.  Step t of a run
+  // that starts at row p0 of its image brings DY row p0 + pad - 2 + t into registers and, from
   // t = 2 on, multiplies X row p0 + t - 2 with the three DY rows held: the newest is
   // filter row 0, the oldest filter row 2.
   struct Walk {
-    int row, p0, n, t; // the run's first row in the batch and in its image, its rows, the step
+    int row, n, t; // the run's first row in X, its rows, the step
+    int y, yrow;   // DY row of step 0 in its image and in the batch
   };
   const int img0 = conv_div(first, a_H, g.magic_h);
-  auto begin = [&](int row, int p0) __attribute__((always_inline)) {
-    const int in_image = a_H - p0, left = last - row;
-    return Walk{row, p0, left < in_image ? left : in_image, 0};
+  auto begin = [&](int row, int p0, int img) __attribute__((always_inline)) {
+    const int in_image = a_H - p0, left = last - row, y = p0 + g.pad - 2;
+    return Walk{row, left < in_image ? left : in_image, 0, y, img * g.P + y};
   };
-  auto step = [&](Walk &w) __attribute__((always_inline)) {
-    if (++w.t == w.n + 2)
-      w = begin(w.row + w.n, 0);
+  auto next = [&](const Walk &w) __attribute__((always_inline)) {
+    return begin(w.row + w.n, 0, conv_div(w.row, a_H, g.magic_h) + 1);
   };
 
   // ---- LDS-DMA lane offsets (relative to a row's first byte) --------------------
   // instruction j fills pixel slots 16 j .. 16 j + 15 of a row slice: lane d
   // carries 16 bytes (8 channels) d % 4 of slot 16 j + d / 4.  X slot t holds
-  // image column t - 1 (slot 0 and the slots past the image are the zero
-  // padding), DY slot t holds column t (zeros past the image).
+  // image column t - pad (the slots outside the image are the zero
+  // padding), DY slot t holds column t (zeros past the image); channels past C or K are zeros.
   uint32_t xrel[R::kX], yrel[R::kY];
 #pragma unroll
   for (int j = 0; j < R::kX; ++j) {
     const int slot = 16 * j + (l >> 2);
-    const int q = slot - 1;
-    xrel[j] = (unsigned)q < (unsigned)a_W
+    const int q = slot - g.pad;
+    xrel[j] = (unsigned)q < (unsigned)a_W && cb * 32 + (l & 3) * 8 < g.C
                   ? (uint32_t)(q * g.C * 2 + cb * 64 + (l & 3) * 16)
                   : 0x80000000u;
     if (j < R::kY)
-      yrel[j < R::kY ? j : 0] = slot < a_W ? (uint32_t)(slot * g.K * 2 + kb * 64 + (l & 3) * 16)
-                                           : 0x80000000u;
+      yrel[j < R::kY ? j : 0] = slot < g.Q && kb * 32 + (l & 3) * 8 < g.K
+                                    ? (uint32_t)(slot * g.K * 2 + kb * 64 + (l & 3) * 16)
+                                    : 0x80000000u;
   }
   const __amdgpu_buffer_rsrc_t rx = wd_rsrc(g.x, g.x_bytes);
   const __amdgpu_buffer_rsrc_t ry = wd_rsrc(g.dy, g.dy_bytes);
   const __amdgpu_buffer_rsrc_t rnone = wd_rsrc(g.x, 0); // every lane reads zero
-  const int x_pitch = a_W * g.C * 2, y_pitch = a_W * g.K * 2;
+  const int x_pitch = a_W * g.C * 2, y_pitch = g.Q * g.K * 2;
 
   const uint32_t wbase = lds0 + (uint32_t)wave * kWdWaveLds;
   // fragment read address inside a row slice: lane l is MFMA row / column
@@ -192,7 +194,7 @@ conv_wgrad_direct_kernel(WgDirectArgs g) {
       acc[t][i] = 0.f;
 
   if (first < last) {
-    Walk ahead = begin(first, first - img0 * a_H), now = ahead;
+    Walk ahead = begin(first, first - img0 * a_H, img0), now = ahead;
     // ring slots of the next loads and the next reads
     uint32_t put_x = 0, put_y = R::kYBase, get_x = 0, get_y = R::kYBase;
     auto turn = [](uint32_t &at, uint32_t by, uint32_t from, uint32_t to) __attribute__((always_inline)) {
@@ -203,9 +205,9 @@ conv_wgrad_direct_kernel(WgDirectArgs g) {
     // share's halo)
     auto issue = [&]() __attribute__((always_inline)) {
       const bool live = ahead.n > 0;
-      const bool y_ok = live && (unsigned)(ahead.p0 - 1 + ahead.t) < (unsigned)a_H, x_ok = live && ahead.t >= 2;
+      const bool y_ok = live && (unsigned)(ahead.y + ahead.t) < (unsigned)g.P, x_ok = live && ahead.t >= 2;
       const __amdgpu_buffer_rsrc_t ys = y_ok ? ry : rnone, xs = x_ok ? rx : rnone;
-      const int y_off = y_ok ? (ahead.row - 1 + ahead.t) * y_pitch : 0;
+      const int y_off = y_ok ? (ahead.yrow + ahead.t) * y_pitch : 0;
       const int x_off = x_ok ? (ahead.row + ahead.t - 2) * x_pitch : 0;
 #pragma unroll
       for (int j = 0; j < R::kX; ++j)
@@ -219,8 +221,8 @@ conv_wgrad_direct_kernel(WgDirectArgs g) {
             0, 0);
       turn(put_x, R::kXBytes, 0, R::kYBase);
       turn(put_y, R::kYBytes, R::kYBase, R::kYBase + R::kD * R::kYBytes);
-      if (live)
-        step(ahead);
+      if (live && ++ahead.t == ahead.n + 2)
+        ahead = next(ahead);
     };
 #pragma unroll
     for (int i = 0; i < R::kD; ++i)
@@ -313,7 +315,7 @@ conv_wgrad_direct_kernel(WgDirectArgs g) {
     using I2 = std::integral_constant<int, 2>;
     // (run by run, the products in a loop of their own: under a branch of one loop over all steps
     // the compiler copies the accumulators about and spills 440 to 880 registers)
-    for (; now.n > 0; now = begin(now.row + now.n, 0)) {
+    for (; now.n > 0; now = next(now)) {
       light(I0{});
       light(I1{});
       for (int left = now.n;;) {
@@ -363,7 +365,7 @@ conv_wgrad_direct_kernel(WgDirectArgs g) {
 }
 
 struct WgDirectSumArgs {
-  int32_t nparts, ctypes;
+  int32_t nparts, ctypes, C, K;
   int64_t sk, sc, sr, ss; // element strides of DW [K, C, R, S]
   int32_t dt;
 };
@@ -398,6 +400,8 @@ conv_wgrad_direct_sum_kernel(WgDirectSumArgs a, const float *part, void *dw) {
   const int kb = type / a.ctypes, cb = type - kb * a.ctypes;
   const int64_t c = cb * 32 + (lane & 31);
   const int r = tap / 3, sx = tap - r * 3;
+  if (c >= a.C || kb * 32 + 8 * (e & 3) + 4 * (lane >> 5) >= a.K)
+    return;
   const int64_t k = kb * 32 + 8 * (e & 3) + 4 * (lane >> 5);
   const float v[4] = {acc[0], acc[1], acc[2], acc[3]};
   fhip_store_float(dw, a.dt, k * a.sk + c * a.sc + r * a.sr + sx * a.ss, a.sk, v);
@@ -426,7 +430,8 @@ bool wd_channels_last(const fhip_tensor_desc &t) {
   return true;
 }
 
-WgDirectPlan make_wd_plan(const fhip_conv_desc *d, int num_cus) {
+// `contract` is 0 for the problems that conv_wgrad.hip reports its workspace for.
+WgDirectPlan make_wd_plan(const fhip_conv_desc *d) {
   WgDirectPlan p;
   const FhipKnobs &knobs = fhip_knobs();
   if (knobs.wgrad_direct == 0)
@@ -446,25 +451,38 @@ WgDirectPlan make_wd_plan(const fhip_conv_desc *d, int num_cus) {
   if (wdt != FHIP_BFLOAT16 && wdt != FHIP_HALF && wdt != FHIP_FLOAT)
     return p;
   const int64_t N = d->x.dim[0], C = d->x.dim[1], H = d->x.dim[2], W = d->x.dim[3];
-  const int64_t K = d->w.dim[0];
+  const int64_t K = d->w.dim[0], P = d->y.dim[2], Q = d->y.dim[3];
   if (d->w.dim[1] != C || d->w.dim[2] != 3 || d->w.dim[3] != 3)
     return p;
   for (int i = 0; i < 2; ++i)
-    if (d->stride[i] != 1 || d->dilation[i] != 1 || d->padding[i] != 1)
+    if (d->stride[i] != 1 || d->dilation[i] != 1 || d->padding[i] != d->padding[0] || d->padding[i] < 0 ||
+        d->padding[i] > 2)
       return p;
-  if (d->y.dim[2] != H || d->y.dim[3] != W || d->y.dim[0] != N || d->y.dim[1] != K)
+  if (P != H + 2 * d->padding[0] - 2 || Q != W + 2 * d->padding[1] - 2 || d->y.dim[0] != N || d->y.dim[1] != K)
     return p;
-  if (C % 32 != 0 || K % 32 != 0 || W > kWdMaxW || W < 1 || H < 1 || N < 1)
+  if (C % 8 != 0 || K % 8 != 0 || Q > kWdMaxW || Q < 1 || P < 1 || N < 1)
     return p;
   if (!wd_channels_last(d->x) || !wd_channels_last(d->y))
     return p;
-  const int64_t x_bytes = N * H * W * C * 2, dy_bytes = N * H * W * K * 2;
+  const int64_t x_bytes = N * H * W * C * 2, dy_bytes = N * P * Q * K * 2;
   if (x_bytes >= (1ll << 31) || dy_bytes >= (1ll << 31))
     return p;
-  const int cus = num_cus > 0 ? num_cus : 256;
-  const int64_t types = (C / 32) * (K / 32);
+  const int64_t types = ((C + 31) / 32) * ((K + 31) / 32);
   if (types > 4096)
     return p;
+  WgDirectArgs &a = p.a;
+  a.H = (int32_t)H, a.W = (int32_t)W, a.C = (int32_t)C, a.K = (int32_t)K;
+  a.P = (int32_t)P, a.Q = (int32_t)Q;
+  a.pad = (int32_t)d->padding[0];
+  a.rows = (int32_t)(N * H);
+  a.types = (int32_t)types, a.ctypes = (int32_t)((C + 31) / 32);
+  a.magic_types = conv_magic(a.types), a.magic_ctypes = conv_magic(a.ctypes), a.magic_h = conv_magic(a.H);
+  a.x_bytes = (uint32_t)x_bytes, a.dy_bytes = (uint32_t)dy_bytes;
+  p.nks = (int)((Q + 15) / 16);
+  p.ok = true;
+  if (C % 32 != 0 || K % 32 != 0 || P != H || Q != W)
+    return p;
+  const int64_t cus = 256;
   // The caller's workspace: the partial sums of workgroups that take whole images, or row chunks
   // of one, a round of them and no fewer.  Saved plans hold its size and are taken only where they equal
   // the plan of today byte for byte (Graph::loadFromArtifact); parts beyond it lie in
@@ -483,16 +501,8 @@ WgDirectPlan make_wd_plan(const fhip_conv_desc *d, int num_cus) {
   const int64_t igroups = (N + ipw - 1) / ipw;
   const int64_t whole = igroups * chunks;
   if (types * whole >= (1ll << 31) / kWdBlock || chunks > 65535 || igroups > 65535)
-    return p;
+    return WgDirectPlan{};
   p.contract = (size_t)(types * whole) * kWdBlock * sizeof(float);
-  WgDirectArgs &a = p.a;
-  a.H = (int32_t)H, a.W = (int32_t)W, a.C = (int32_t)C, a.K = (int32_t)K;
-  a.rows = (int32_t)(N * H);
-  a.types = (int32_t)types, a.ctypes = (int32_t)(C / 32);
-  a.magic_types = conv_magic(a.types), a.magic_ctypes = conv_magic(a.ctypes), a.magic_h = conv_magic(a.H);
-  a.x_bytes = (uint32_t)x_bytes, a.dy_bytes = (uint32_t)dy_bytes;
-  p.nks = (int)((W + 15) / 16);
-  p.ok = true;
   return p;
 }
 
@@ -523,6 +533,16 @@ int wd_parts(const WgDirectArgs &a, int nks, int64_t most) {
   return (int)best;
 }
 
+// Whether it replaces the gathered tiles of conv_wgrad.hip, which take these problems too.  On 58
+// random layers of 8 to 64 images, 7 to 64 rows and 32 to 512 channels it is 1.2 to 1.4 times as fast, twice where their
+// runs fall badly (N24 128 -> 144, 54 x 54 74.8 us, here 34.8; N37 448 -> 208, 8 x 31 55.4 / 28.0), but for small ones
+// (N17 64 -> 80, 10 x 10 9.3 / 10.6; N30 176 -> 48, 7 x 7 10.9 / 11.9).  Gradients stored in f32 stay
+// there: their chains of additions are shorter.
+bool wd_pays(const WgDirectPlan &p, int w_dtype) {
+  const WgDirectArgs &a = p.a;
+  return w_dtype != FHIP_FLOAT && (double)a.C * a.K * ((double)a.rows / a.H * a.P * a.Q) >= 1.4e7;
+}
+
 template <int KIND, int NKS> int wd_launch(fhip_ctx *ctx, const WgDirectArgs &a) {
   auto kernel = conv_wgrad_direct_kernel<KIND, NKS>;
   static FhipOncePerDevice configured;
@@ -548,33 +568,40 @@ template <int KIND> int wd_launch(fhip_ctx *ctx, const WgDirectPlan &p) {
 
 bool fhip_fast_conv_wgrad_direct_applicable(const fhip_conv_desc *d,
                                             size_t *workspace_bytes) {
-  const WgDirectPlan p = make_wd_plan(d, 256);
+  const WgDirectPlan p = make_wd_plan(d);
   if (workspace_bytes)
-    *workspace_bytes = p.ok ? p.contract : 0;
-  return p.ok;
+    *workspace_bytes = p.contract;
+  return p.ok && p.contract != 0;
 }
 
 int fhip_fast_conv_wgrad_direct(fhip_ctx *ctx, const fhip_conv_desc *d,
                                 const void *dy, const void *x, void *dw,
-                                void *workspace) {
+                                void *workspace, size_t workspace_bytes, bool *handled) {
   // planned for 256 compute units whatever the device: the workspace size was
   // answered without one
-  WgDirectPlan p = make_wd_plan(d, 256);
-  FHIP_REQUIRE(ctx, p.ok, "conv wgrad: descriptor not supported by the direct kernel");
+  WgDirectPlan p = make_wd_plan(d);
+  const bool ours = p.ok && p.contract != 0;
+  *handled = ours;
+  if (!p.ok || (!ours && !wd_pays(p, d->w.dtype)))
+    return 0;
   FHIP_REQUIRE(ctx, ((uintptr_t)workspace & 255) == 0 && ((uintptr_t)x & 15) == 0 &&
                         ((uintptr_t)dy & 15) == 0,
                "conv wgrad: workspace must be 256-byte and tensors 16-byte aligned");
   constexpr size_t kBytes = kWdBlock * sizeof(float);
-  const int64_t held = (int64_t)(p.contract / kBytes) / p.a.types;
+  const int64_t held = (int64_t)(workspace_bytes / kBytes) / p.a.types;
   p.a.nparts = wd_parts(p.a, p.nks, (1ll << 31) / kWdBlock / p.a.types);
   void *part = workspace;
   if (p.a.nparts > held) {
     const size_t bytes = (size_t)p.a.types * p.a.nparts * kBytes;
-    if (!fhip_ctx_scratch_ready(ctx, bytes))
+    const bool ready = fhip_ctx_scratch_ready(ctx, bytes);
+    if (!ready && !ours)
+      return 0; // (the gathered tiles fit the workspace)
+    if (!ready)
       p.a.nparts = wd_parts(p.a, p.nks, held);
     else if (fhip_ctx_scratch(ctx, bytes, &part) != 0)
       return 1;
   }
+  *handled = true;
   p.a.total = p.a.types * p.a.nparts;
   p.a.per_xcd = (p.a.total + 7) / 8;
   p.a.x = (const char *)x;
@@ -583,13 +610,13 @@ int fhip_fast_conv_wgrad_direct(fhip_ctx *ctx, const fhip_conv_desc *d,
   if ((p.kind == GK_BF16 ? wd_launch<GK_BF16>(ctx, p) : wd_launch<GK_F16>(ctx, p)) != 0)
     return 1;
   WgDirectSumArgs s;
-  s.nparts = p.a.nparts, s.ctypes = p.a.ctypes;
+  s.nparts = p.a.nparts, s.ctypes = p.a.ctypes, s.C = p.a.C, s.K = p.a.K;
   s.sk = d->w.dim[0] == 1 ? 0 : d->w.stride[0];
   s.sc = d->w.dim[1] == 1 ? 0 : d->w.stride[1];
   s.sr = d->w.dim[2] == 1 ? 0 : d->w.stride[2];
   s.ss = d->w.dim[3] == 1 ? 0 : d->w.stride[3];
   s.dt = d->w.dtype;
-  const int64_t total = (int64_t)(p.a.C / 32) * (p.a.K / 32) * kWdBlock;
+  const int64_t total = (int64_t)p.a.types * kWdBlock;
   hipLaunchKernelGGL(conv_wgrad_direct_sum_kernel, dim3((unsigned)(total / 256)),
                      dim3(256), 0, ctx->stream, s, (const float *)p.a.part, dw);
   FHIP_HIP_CHECK(ctx, hipGetLastError());

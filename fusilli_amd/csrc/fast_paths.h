@@ -72,18 +72,19 @@ int fhip_conv_dgrad_static_setup(fhip_ctx *ctx);
 bool fhip_fast_conv_wgrad_applicable(const fhip_conv_desc *d,
                                      size_t *workspace_bytes);
 int fhip_fast_conv_wgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy,
-                         const void *x, void *dw, void *workspace);
+                         const void *x, void *dw, void *workspace, size_t workspace_bytes);
 int fhip_gather_conv_wgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy,
                            const void *x, void *dw, bool *handled);
 
-// Weight gradient of 3 x 3, padding-1, unit-stride convolutions straight from
-// X and DY (no operand copies): one MFMA kernel plus the sum of its partial
-// results; `*workspace_bytes` of 256-byte aligned workspace hold those.
+// Weight gradient of 3 x 3, unit-stride convolutions straight from X and DY (no operand
+// copies): one MFMA kernel plus the sum of its partial results, in the workspace where it
+// holds them, else in the context's scratch.  The first says for which it reports the workspace; `handled`
+// false: a problem for fhip_fast_conv_wgrad's gathered tiles.
 bool fhip_fast_conv_wgrad_direct_applicable(const fhip_conv_desc *d,
                                             size_t *workspace_bytes);
 int fhip_fast_conv_wgrad_direct(fhip_ctx *ctx, const fhip_conv_desc *d,
                                 const void *dy, const void *x, void *dw,
-                                void *workspace);
+                                void *workspace, size_t workspace_bytes, bool *handled);
 
 // Register-blocked direct kernels for any layout, dtype, group count and 1 - 3
 // spatial dims (conv_direct.hip): the path of the convolutions the MFMA

@@ -58,3 +58,41 @@ def test_direct_weight_gradient_shares(ctx, x, k, steps):
         np.testing.assert_array_equal(got[416:, 256:], oracle.conv_wgrad(dy, xt, [64, 64, 3, 3], [1, 1], [1, 1], [1, 1]))
     else:
         np.testing.assert_array_equal(got, oracle.conv_wgrad(dy.logical(), xt.logical(), w, [1, 1], [1, 1], [1, 1]))
+
+
+# paddings of 0 to 2, channels off the blocks of 32: the same kernel in place of the
+# gathered tiles, whose workspace it is given
+@pytest.mark.parametrize("x,k,pad,steps", [
+    ([16, 48, 48, 32], 48, 2, 3), ([9, 64, 31, 19], 72, 0, 2), ([40, 200, 9, 18], 40, 0, 1),
+    ([60, 32, 20, 58], 32, 0, 4), ([30, 40, 17, 14], 64, 2, 1), ([25, 96, 4, 31], 200, 2, 3),
+    ([12, 136, 16, 54], 24, 2, 4), ([11, 8, 60, 40], 72, 1, 3), ([60, 88, 1, 16], 200, 2, 2),
+])
+@pytest.mark.parametrize("dtype", [capi.BFLOAT16, capi.HALF])
+def test_direct_weight_gradient_of_other_paddings_and_channels(ctx, x, k, pad, steps, dtype):
+    yd = [x[0], k, x[2] + 2 * pad - 2, x[3] + 2 * pad - 2]
+    xt, dy = whole(k, x, dtype, 2), whole(k + 1, yd, dtype, 1)
+    w = [k, x[1], 3, 3]
+    geom = ([pad, pad], [1, 1], [1, 1])
+    ref = oracle.conv_wgrad(dy.logical(), xt.logical(), w, *geom)
+    dw = run_conv_wgrad(ctx, dy, xt, w, *geom, dtype, tuned=None)
+    name = ctx.last_kernel()
+    big = np.prod(yd) * x[1] >= 1.4e7
+    assert name.startswith(f"conv_wgrad_direct steps={steps}" if big else "conv_wgrad_gather"), name
+    np.testing.assert_array_equal(dw.logical(), HT.from_logical(ref, dtype).logical())
+    # stored in f32: the gathered tiles' shorter chains
+    dw = run_conv_wgrad(ctx, dy, xt, w, *geom, dtype, tuned=None, w_dtype=capi.FLOAT)
+    assert ctx.last_kernel().startswith("conv_wgrad_gather"), ctx.last_kernel()
+    np.testing.assert_array_equal(dw.logical(), ref)
+
+
+def test_direct_weight_gradient_meets_no_values_outside(ctx):
+    # infinite values in the channels, rows and columns next to a block's own: each gradient shows its own
+    x, dy = whole(5, [8, 40, 40, 30], capi.BFLOAT16, 2), whole(6, [8, 72, 40, 30], capi.BFLOAT16, 1)
+    xv, w = x.logical().copy(), [72, 40, 3, 3]
+    xv[:, 39] = np.inf
+    dw = run_conv_wgrad(ctx, dy, HT.from_logical(xv, capi.BFLOAT16, oracle.channels_last_strides([8, 40, 40, 30])), w,
+                        [1, 1], [1, 1], [1, 1], capi.BFLOAT16, tuned=None).logical()
+    assert ctx.last_kernel().startswith("conv_wgrad_direct"), ctx.last_kernel()
+    ref = oracle.conv_wgrad(dy.logical(), x.logical(), w, [1, 1], [1, 1], [1, 1])
+    np.testing.assert_array_equal(dw[:, :39], HT.from_logical(ref, capi.BFLOAT16).logical()[:, :39])
+    assert not np.isfinite(dw[:, 39]).any()
