@@ -6,7 +6,7 @@ import pytest
 from fusilli_amd import capi
 from oracle import oracle
 from helpers import HT
-from test_generic_ops_gpu import run_batchnorm, run_conv_wgrad
+from test_generic_ops_gpu import run_batchnorm, run_conv_dgrad, run_conv_wgrad
 
 pytestmark = pytest.mark.gpu
 
@@ -96,3 +96,22 @@ def test_direct_weight_gradient_meets_no_values_outside(ctx):
     ref = oracle.conv_wgrad(dy.logical(), x.logical(), w, [1, 1], [1, 1], [1, 1])
     np.testing.assert_array_equal(dw[:, :39], HT.from_logical(ref, capi.BFLOAT16).logical()[:, :39])
     assert not np.isfinite(dw[:, 39]).any()
+
+
+# the mirrored filter of a data gradient, copied in blocks of 64 x 64: edges of the blocks, groups, and a
+# channel count that the copy takes element by element
+@pytest.mark.parametrize("x,k,w", [
+    ([4, 64, 13, 12], 8, [3, 3]), ([4, 72, 13, 12], 136, [3, 3]), ([2, 192, 9, 30], 64, [5, 1]),
+    ([3, 256, 12, 12], 128, [3, 3]), ([2, 64, 20, 21], 200, [1, 3]), ([2, 64, 20, 21], 100, [3, 3]),
+])
+@pytest.mark.parametrize("groups", [1, 2])
+def test_mirrored_filter(ctx, x, k, w, groups):
+    if groups == 2 and (x[1] % 128 or k % 128):
+        pytest.skip("groups of whole slices")
+    wd = [k, x[1] // groups] + w
+    dy = whole(k, [x[0], k] + x[2:], capi.BFLOAT16, 1)
+    wt = whole(k + 1, wd, capi.BFLOAT16, 2)
+    pad = [(w[0] - 1) // 2, (w[1] - 1) // 2]
+    dx = run_conv_dgrad(ctx, dy, wt, x, pad, [1, 1], [1, 1], capi.BFLOAT16, tuned=None)
+    ref = oracle.conv_dgrad(dy.logical(), wt.logical(), x, pad, [1, 1], [1, 1])
+    np.testing.assert_array_equal(dx.logical(), HT.from_logical(ref, capi.BFLOAT16).logical())
