@@ -23,6 +23,8 @@
 // One training step (us):
 //   N100 3 -> 32, 32 x 32, 3 x 3, f32: fprop 26.2 -> 13.6 -> 12.0, dgrad 60.5 -> 15.0 -> 11.1, wgrad 46.1 -> 13.0
 //   N122 1 -> 64, 57 x 57, 5 x 5, bf16: 136 -> 52.6, 701 -> 78.6 -> 33.0, 495 -> 45.7
+// With elements found by steps, and quotients of uniform values in scalar multiplications, 36 random
+// layers (sums of traced us): fprop 420.8 -> 398.4, dgrad 294.8 -> 287.2, wgrad 314.0 -> 296.
 //
 // Reference semantics: aten.convolution / aten.convolution_backward
 // (reference support/asm_emitter.h:690-701, 868-873, 1030-1035).
@@ -48,13 +50,14 @@ struct CfArgs {
   int32_t lw;                  // columns of the staged X
   uint32_t lw_magic, rows_magic, q_magic, rs_magic, s_magic;
   int32_t xrows;               // most rows of X staged at once
+  int32_t col_step, row_step, c_step; // kCfThreads elements of the staged X
   int32_t tiles;               // forward: workgroups per image; gradients: bands
   int32_t band;                // output (data gradient: input) rows per band
   int32_t quads;               // data gradient: runs of 4 pixels per row,
   int32_t wt;                  // products: columns per band,
   int32_t cb, wpitch, gat, gpitch; // channels per pass, pitch of the filter, where G starts, pitch of a row in G
-  int32_t packed;              // W without gaps, in this order
-  uint32_t w_magic, quads_magic;
+  int32_t packed;              // the filter of an output channel without gaps, in this order
+  uint32_t w_magic, quads_magic, tiles_whole, q_whole;
   DevEpilogue epi;
 };
 
@@ -64,38 +67,83 @@ __device__ __forceinline__ int cf_div(int e, uint32_t magic) {
   return (int)__umulhi((uint32_t)e, magic) + (magic == 0 ? e : 0);
 }
 
+// e / d of uniform values, any e >= 0, whole = (2^32 - 1) / d: a quotient at most one too small, in
+// scalar multiplications (a division is some 30 dependent vector operations)
+__device__ __forceinline__ int cf_div_uniform(int e, int d, uint32_t whole, int *rest) {
+  int q = (int)__umulhi((uint32_t)e, whole);
+  int r = e - q * d;
+  if (r >= d)
+    ++q, r -= d;
+  *rest = r;
+  return q;
+}
+
 // X rows [row0, row0 + rows) of all channels of an image, zeros outside it, as f32, in batches:
-// request() issues a batch's loads, put() waits for them.
-template <typename T> struct CfStageX {
+// request() issues a batch's loads, put() waits for them.  A thread steps from element to element:
+// the first loads wait for what it takes to find them (multiplications of 32 bits are four times as
+// long as additions).  TRIM: no loads behind the last element; in the loop over the bands of a weight
+// gradient with much else in it the branches cost more (f32 N119 3 -> 64, 58 x 58 33.7 us without, 35.5
+// with, one band each N38 3 -> 64, 24 x 24 6.4 and 6.1).
+template <typename T, bool TRIM = true> struct CfStageX {
   static constexpr int kBatch = 8; // loads in flight per thread
   T v[kBatch];
+  // where in an image a load goes, less its first row, and its row there, two to a register, 2^16 - 1
+  // where it is in no column of the image
+  uint32_t at[kBatch];
+  uint32_t row[kBatch / 2];
   uint32_t live;
+  // elements e0 + threadIdx.x + i * kCfThreads
+  __device__ __forceinline__ void find(const CfArgs &g, int e0) {
+    const int total = g.C * g.xrows * g.lw, e = e0 + (int)threadIdx.x;
+    const int cr = cf_div(e, g.lw_magic);
+    int c = cf_div(cr, g.rows_magic), r = cr - c * g.xrows, w = e - cr * g.lw - g.pad_w;
+    const uint32_t sc = (uint32_t)g.xs[1], sr = (uint32_t)g.xs[2];
+    uint32_t p = (uint32_t)c * sc + (uint32_t)r * sr + (uint32_t)w;
+    const uint32_t step = (uint32_t)g.c_step * sc + (uint32_t)g.row_step * sr + (uint32_t)g.col_step;
+    const uint32_t next_row = sr - (uint32_t)g.lw, next_c = sc - (uint32_t)g.xrows * sr;
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      if (TRIM && e0 + i * kCfThreads >= total) // (uniform)
+        break;
+      at[i] = p;
+      const uint32_t mine = c < g.C && (unsigned)w < (unsigned)g.W ? (uint32_t)r : 0xffffu;
+      row[i / 2] = i & 1 ? row[i / 2] | mine << 16 : mine;
+      w += g.col_step, r += g.row_step, c += g.c_step, p += step;
+      if (w >= g.lw - g.pad_w)
+        w -= g.lw, ++r, p += next_row;
+      if (r >= g.xrows)
+        r -= g.xrows, ++c, p += next_c;
+    }
+  }
   __device__ __forceinline__ void request(const CfArgs &g, const T *x, int row0, int rows, int e0) {
     const int total = g.C * g.xrows * g.lw;
+    const int r0 = row0 < 0 ? -row0 : 0, r1 = g.H - row0 < rows ? g.H - row0 : rows; // rows of the image
+    const uint32_t add = (uint32_t)row0 * (uint32_t)g.xs[2];
     live = 0;
 #pragma unroll
     for (int i = 0; i < kBatch; ++i) {
-      const int e = e0 + i * kCfThreads;
-      const int cr = cf_div(e, g.lw_magic), col = e - cr * g.lw;
-      const int c = cf_div(cr, g.rows_magic), r = cr - c * g.xrows;
-      const int h = row0 + r, w = col - g.pad_w;
-      const bool in = e < total && r < rows && (unsigned)h < (unsigned)g.H && (unsigned)w < (unsigned)g.W;
+      if (TRIM && e0 + i * kCfThreads >= total)
+        break;
+      const int r = (int)(i & 1 ? row[i / 2] >> 16 : row[i / 2] & 0xffffu);
+      const bool in = r >= r0 && r < r1;
       // (the load is issued either way: a branch would wait for every value)
-      v[i] = x[in ? c * (int)g.xs[1] + h * (int)g.xs[2] + w * (int)g.xs[3] : 0];
+      v[i] = x[in ? at[i] + add : 0u];
       live |= (uint32_t)in << i;
     }
   }
   __device__ __forceinline__ void put(const CfArgs &g, int e0, float *xl) const {
     const int total = g.C * g.xrows * g.lw;
+    float *to = xl + e0 + threadIdx.x;
 #pragma unroll
     for (int i = 0; i < kBatch; ++i)
-      if (e0 + i * kCfThreads < total)
-        xl[e0 + i * kCfThreads] = (live >> i) & 1 ? (float)v[i] : 0.f;
+      if (e0 + i * kCfThreads + (int)threadIdx.x < total)
+        to[i * kCfThreads] = (live >> i) & 1 ? (float)v[i] : 0.f;
   }
   // all batches from `e0` on
   static __device__ __forceinline__ void stage(const CfArgs &g, const T *x, int row0, int rows, int e0, float *xl) {
     for (; e0 < g.C * g.xrows * g.lw; e0 += kBatch * kCfThreads) {
       CfStageX b;
+      b.find(g, e0);
       b.request(g, x, row0, rows, e0);
       b.put(g, e0, xl);
     }
@@ -138,28 +186,33 @@ __global__ __launch_bounds__(kCfThreads) void conv_few_fprop_kernel(CfArgs g, co
   int *tab = (int *)(ops + FHIP_MAX_EPILOGUE * K16); // where a pair's X lies
   float *xl = (float *)(tab + j4);
   const int tid = threadIdx.x, l = tid & 63, wave = tid >> 6;
-  const int k0 = blockIdx.y * K16;
-  const int n = blockIdx.x / g.tiles, t0 = (blockIdx.x % g.tiles) * kCfThreads;
+  const int k0 = blockIdx.z * K16, n = blockIdx.y, t0 = blockIdx.x * kCfThreads;
   const int pq = g.P * g.Q;
   const int t1 = t0 + kCfThreads < pq ? t0 + kCfThreads : pq;
-  const int p0 = t0 / g.Q, p1 = (t1 - 1) / g.Q;
+  int q0; // (column of the first pixel)
+  const int p0 = cf_div_uniform(t0, g.Q, g.q_whole, &q0), p1 = p0 + cf_div(q0 + t1 - 1 - t0, g.q_magic);
   // Everything a workgroup reads is requested before the first wait: X, the filter, then the
   // fused operations' values per channel.  Nothing looks at a loaded value before that, not
   // even a select (f32 N22 1 -> 16, 28 x 28, 3 x 3 7.3 -> 6.8 us, bf16 N71 1 -> 32, 17 x 17, 5 x 5 9.1 -> 8.3).
   const int row0 = p0 * g.str_h - g.pad_h, xrows = (p1 - p0) * g.str_h + (g.R - 1) * g.dil_h + 1;
   CfStageX<T> xv0;
-  xv0.request(g, x + n * g.xs[0], row0, xrows, tid);
+  xv0.find(g, 0);
+  xv0.request(g, x + n * g.xs[0], row0, xrows, 0);
   constexpr int kBatch = 8;
   const int kk = tid % K16, jt = tid / K16; // this thread's channel, its first pair
   const bool k_in = k0 + kk < g.K;
+  const T *wk = w + (k_in ? k0 + kk : k0) * g.ws[0];
+  // (as many loads as there are pairs, up to a batch; those behind the last pair read the first)
   auto weights = [&](int j0, T (&v)[kBatch]) {
 #pragma unroll
     for (int i = 0; i < kBatch; ++i) {
-      const int j = j0 + i * (kCfThreads / K16);
-      const bool in = j < g.J && k_in;
-      int f;
-      cf_pair(g, in ? j : 0, &f);
-      v[i] = w[in ? (k0 + kk) * g.ws[0] + f : 0];
+      if (j0 - jt + i * (kCfThreads / K16) >= j4) // (uniform)
+        break;
+      int j = j0 + i * (kCfThreads / K16);
+      j = j < g.J ? j : 0;
+      if (!g.packed)
+        cf_pair(g, j, &j);
+      v[i] = wk[j];
     }
   };
   auto put_weights = [&](int j0, const T (&v)[kBatch]) {
@@ -188,8 +241,8 @@ __global__ __launch_bounds__(kCfThreads) void conv_few_fprop_kernel(CfArgs g, co
     int f;
     tab[j] = j < g.J ? cf_pair(g, j, &f) : 0;
   }
-  xv0.put(g, tid, xl);
-  CfStageX<T>::stage(g, x + n * g.xs[0], row0, xrows, tid + CfStageX<T>::kBatch * kCfThreads, xl);
+  xv0.put(g, 0, xl);
+  CfStageX<T>::stage(g, x + n * g.xs[0], row0, xrows, CfStageX<T>::kBatch * kCfThreads, xl);
   put_weights(jt, wv0);
   for (int j0 = jt + kBatch * (kCfThreads / K16); j0 < j4; j0 += kBatch * (kCfThreads / K16)) {
     T v[kBatch];
@@ -214,9 +267,9 @@ __global__ __launch_bounds__(kCfThreads) void conv_few_fprop_kernel(CfArgs g, co
   for (int t = 0; t < 4; ++t) {
     const int m = l & 15;
     int px = first + (m >> 2) * gs + t * ts + (m & 3);
-    px = px < t1 ? px : t1 - 1;
-    const int p = px / g.Q, q = px - p * g.Q;
-    base[t] = (p - p0) * g.str_h * g.lw + q * g.str_w;
+    // (row p and column i - p * Q behind p0's start)
+    const int i = (px < t1 ? px : t1 - 1) - t0 + q0;
+    base[t] = __mul24(i, g.str_w) + __mul24(cf_div(i, g.q_magic), g.str_h * g.lw - g.Q * g.str_w);
   }
   f32x4 acc[4][KT];
 #pragma unroll
@@ -362,9 +415,13 @@ __global__ __launch_bounds__(kCfThreads) void conv_few_wgrad_kernel(CfArgs g, co
 #pragma unroll
     for (int v = 0; v < JT; ++v)
       acc[u][v] = f32x4{0, 0, 0, 0};
+  CfStageX<T, (KT <= 2 && JT <= 3)> xs; // (the same elements of every band)
+  xs.find(g, 0);
   const int items = g.N * g.tiles;
   for (int item = blockIdx.x; item < items; item += gridDim.x) {
-    const int n = item / g.tiles, p0 = (item - n * g.tiles) * g.band;
+    int p0;
+    const int n = cf_div_uniform(item, g.tiles, g.tiles_whole, &p0);
+    p0 *= g.band;
     const int rows = g.P - p0 < g.band ? g.P - p0 : g.band;
     const int np = rows * g.Q;
     const T *src[KT];
@@ -376,9 +433,11 @@ __global__ __launch_bounds__(kCfThreads) void conv_few_wgrad_kernel(CfArgs g, co
     float a[2][KT][4];
     const int px0 = wave * 16 + (l >> 4) * 4;
     cf_load_dy<T, KT>(src, px0, np, a[0]);
+    const int row0 = p0 * g.str_h - g.pad_h, xrows = (rows - 1) * g.str_h + (g.R - 1) * g.dil_h + 1;
+    xs.request(g, x + n * g.xs[0], row0, xrows, 0);
     __syncthreads();
-    CfStageX<T>::stage(g, x + n * g.xs[0], p0 * g.str_h - g.pad_h,
-                       (rows - 1) * g.str_h + (g.R - 1) * g.dil_h + 1, tid, xl);
+    xs.put(g, 0, xl);
+    CfStageX<T>::stage(g, x + n * g.xs[0], row0, xrows, CfStageX<T>::kBatch * kCfThreads, xl);
     __syncthreads();
     auto spend = [&](const float (&b)[KT][4], int px) {
       const int4 at = *(const int4 *)(pixtab + px);
@@ -668,7 +727,9 @@ __global__ __launch_bounds__(1024) void conv_few_dgrad_products_kernel(CfArgs g,
   extern __shared__ __attribute__((aligned(16))) float smem[];
   const int tid = threadIdx.x, l = tid & 63, threads = blockDim.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = threads >> 6;
-  const int n = blockIdx.x / g.tiles, h0 = (blockIdx.x - n * g.tiles) * g.band;
+  int h0;
+  const int n = cf_div_uniform(blockIdx.x, g.tiles, g.tiles_whole, &h0);
+  h0 *= g.band;
   const int w0 = blockIdx.y * g.wt;
   const int rows = g.H - h0 < g.band ? g.H - h0 : g.band, cols = g.W - w0 < g.wt ? g.W - w0 : g.wt;
   // Rows and columns of DY that reach this band (whole rows unless bands are cut).  A row is
@@ -778,7 +839,7 @@ __global__ __launch_bounds__(1024) void conv_few_dgrad_products_kernel(CfArgs g,
         if (first || !held)
           fetch(unit, k0);
         if (first) {
-          if (g.packed)
+          if (g.packed && g.ws[0] == g.J)
             stage(std::true_type{});
           else
             stage(std::false_type{});
@@ -919,6 +980,7 @@ bool cf_args(const fhip_conv_desc *d, const fhip_tensor_desc &y, CfArgs &g) {
   g.P = (int32_t)y.dim[2], g.Q = (int32_t)y.dim[3];
   g.J = (int32_t)J;
   g.rs_magic = cf_magic(g.R * g.S), g.s_magic = cf_magic(g.S);
+  g.q_magic = cf_magic(g.Q), g.q_whole = 0xffffffffu / (uint32_t)g.Q;
   g.pad_h = (int32_t)d->padding[0], g.pad_w = (int32_t)d->padding[1];
   g.str_h = (int32_t)d->stride[0], g.str_w = (int32_t)d->stride[1];
   g.dil_h = (int32_t)d->dilation[0], g.dil_w = (int32_t)d->dilation[1];
@@ -934,6 +996,7 @@ bool cf_args(const fhip_conv_desc *d, const fhip_tensor_desc &y, CfArgs &g) {
   };
   if (!strides(d->x, g.xs) || !strides(d->w, g.ws) || !strides(y, g.ys))
     return false;
+  g.packed = (g.S == 1 || g.ws[3] == 1) && (g.R == 1 || g.ws[2] == g.S) && (g.C == 1 || g.ws[1] == g.R * g.S);
   // X walked along its rows (channels-last tensors have kernels of their own)
   return g.W == 1 || g.xs[3] == 1;
 }
@@ -952,6 +1015,8 @@ bool cf_stage(CfArgs &g, int span, int64_t other, size_t *bytes) {
     return false;
   g.lw = (int32_t)lw, g.lw_magic = cf_magic(g.lw);
   g.xrows = (int32_t)rows, g.rows_magic = cf_magic(g.xrows);
+  g.col_step = kCfThreads % g.lw;
+  g.row_step = kCfThreads / g.lw % g.xrows, g.c_step = kCfThreads / g.lw / g.xrows;
   *bytes = (size_t)(total + other) * 4;
   return true;
 }
@@ -1007,7 +1072,7 @@ int fhip_few_conv_fprop(fhip_ctx *ctx, const fhip_conv_desc *d, const void *x, c
   g.epi = epi;
   *handled = true;
   fhip_note_kernel(ctx, "conv_few fprop channels=%d", kt * 16);
-  const dim3 grid((unsigned)blocks, (unsigned)((g.K + kt * 16 - 1) / (kt * 16)));
+  const dim3 grid((unsigned)g.tiles, (unsigned)g.N, (unsigned)((g.K + kt * 16 - 1) / (kt * 16)));
   cf_by_type(d->x.dtype, [&](auto t) {
     typedef decltype(t) T;
     auto kernel = kt == 4   ? conv_few_fprop_kernel<T, 4>
@@ -1035,7 +1100,7 @@ int fhip_few_conv_wgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy, 
   g.tiles = (g.P + band - 1) / band;
   g.band = (g.P + g.tiles - 1) / g.tiles;
   g.tiles = (g.P + g.band - 1) / g.band;
-  g.q_magic = cf_magic(g.Q);
+  g.tiles_whole = 0xffffffffu / (uint32_t)g.tiles;
   size_t lds = 0;
   const int64_t slots = ((int64_t)g.band * g.Q + 15) / 16 * 16;
   if (slots >= (1 << 14) || !cf_stage(g, g.band, slots, &lds))
@@ -1052,8 +1117,10 @@ int fhip_few_conv_wgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy, 
   const int64_t frags = (int64_t)kblocks * kt * jt * 256;
   if (items >= (1ll << 31) || kblocks > 65535)
     return 0;
-  // two workgroups per compute unit, no more than 8 MB of partial sums
-  int64_t runs = 2 * cus / kblocks, most = (8ll << 20) / (frags * 4);
+  // Two workgroups per compute unit with 64 channels each, as their registers allow, else three (f32
+  // N89 1 -> 32, 57 x 57, 3 x 3 17.9 us with two, 15.9 with three, 17.3 with four; N124 4 -> 16, 37 x 37 11.4, 9.3
+  // and 10.0; N119 3 -> 64, 58 x 58 36.2 with two, 41.1 with three), no more than 8 MB of partial sums.
+  int64_t runs = (kt == 4 ? 2 : 3) * cus / kblocks, most = (8ll << 20) / (frags * 4);
   runs = runs < most ? runs : most;
   runs = runs < items ? runs : items;
   runs = runs < 1 ? 1 : runs;
@@ -1147,7 +1214,6 @@ static int cf_dgrad_products(fhip_ctx *ctx, const fhip_conv_desc *d, CfArgs g, c
     return 0;
   g.gat = (int32_t)((filter + 3) / 4 * 4);
   g.q_magic = cf_magic(g.J);
-  g.packed = (g.S == 1 || g.ws[3] == 1) && (g.R == 1 || g.ws[2] == g.S) && (g.C == 1 || g.ws[1] == rs) && g.ws[0] == g.J;
   const int64_t tiles_w = (g.W + 127) / 128;
   g.wt = (int32_t)((g.W + tiles_w - 1) / tiles_w);
   g.w_magic = cf_magic((g.wt + 3) / 4), g.quads_magic = cf_magic((g.Q + 3) / 4);
@@ -1187,6 +1253,7 @@ static int cf_dgrad_products(fhip_ctx *ctx, const fhip_conv_desc *d, CfArgs g, c
       break;
   }
   g.tiles = (g.H + g.band - 1) / g.band;
+  g.tiles_whole = 0xffffffffu / (uint32_t)g.tiles;
   const int64_t blocks = (int64_t)g.N * g.tiles;
   if (blocks >= (1ll << 23))
     return 0;

@@ -172,3 +172,33 @@ def test_data_gradient_keeps_subnormal_values(ctx, dtype, tiny):
     scale = 12 * wt.logical().flat[0] * tiny
     assert np.array_equal(dx[0, 0, 1:-1, 1:-1], np.full([6, 6], 9 * scale)), dx[0, 0]
     assert np.array_equal(dx[0, :, 0, 0], np.full([3], 4 * scale))
+
+
+# X staged by steps of 256 elements: rows longer than that, channels of fewer elements, several batches
+# of loads, gaps between rows, channels and images; filters that do not lie pair behind pair; more
+# bands than workgroups.  Whole numbers: every sum is exact.
+@pytest.mark.parametrize("x,w,pad,s,d,gaps", [
+    ([2, 3, 6, 300], [16, 3, 3, 3], [1, 1], [1, 1], [1, 1], False),
+    ([3, 9, 2, 3], [20, 9, 3, 3], [1, 1], [1, 1], [1, 1], True),
+    ([2, 12, 40, 31], [17, 12, 3, 3], [1, 1], [1, 1], [1, 1], True),
+    ([2, 4, 25, 256], [30, 4, 5, 5], [2, 2], [2, 1], [1, 3], True),
+    ([2, 1, 1, 700], [8, 1, 1, 5], [0, 7], [1, 3], [1, 2], False),
+    ([2, 2, 700, 1], [8, 2, 5, 1], [3, 0], [2, 1], [1, 1], True),
+    ([200, 3, 40, 40], [16, 3, 3, 3], [1, 1], [1, 1], [1, 1], False),
+])
+@pytest.mark.parametrize("dtype", [capi.FLOAT, capi.BFLOAT16])
+def test_staged_rows(ctx, x, w, pad, s, d, gaps, dtype):
+    rng = np.random.default_rng(x[0] + x[3])
+    pitch, plane = x[3] + 5, x[2] * (x[3] + 5) + 11
+    xt = HT.from_logical(rng.integers(-2, 3, size=x), dtype, [x[1] * plane + 3, plane, pitch, 1] if gaps else None)
+    turned = [w[1] * w[2] * w[3], 1, w[1] * w[3], w[1]]  # channel beside channel
+    wt = HT.from_logical(rng.integers(-1, 2, size=w), dtype, turned if gaps else None)
+    y = run_conv(ctx, xt, wt, pad, s, d, dtype)
+    assert ctx.last_kernel().startswith("conv_few fprop"), ctx.last_kernel()
+    # (sums of at most 112 products of 2 x 1: whole in 16 bits too)
+    np.testing.assert_array_equal(y.logical(), oracle.conv_fprop(xt.logical(), wt.logical(), pad, s, d))
+    dy = HT.from_logical(rng.integers(-1, 2, size=y.dims), dtype)
+    dw = run_conv_wgrad(ctx, dy, xt, w, pad, s, d, dtype, False, tuned=None)
+    assert ctx.last_kernel().startswith("conv_few wgrad"), ctx.last_kernel()
+    ref = oracle.conv_wgrad(dy.logical(), xt.logical(), w, pad, s, d)
+    np.testing.assert_array_equal(dw.logical(), HT.from_logical(ref, dtype).logical())
