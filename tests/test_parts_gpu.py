@@ -16,16 +16,44 @@ def whole(seed, dims, dtype, span):
     return HT.from_logical(v, dtype, oracle.channels_last_strides(dims))
 
 
-# 64 rows of 32 channels per workgroup, 64 lanes per channel that take eight parts a round
-@pytest.mark.parametrize("parts", [1, 2, 63, 64, 65, 449, 511, 512])
-@pytest.mark.parametrize("affine", [capi.FLOAT, capi.HALF])
-def test_batchnorm_parts(ctx, parts, affine):
-    x = whole(parts, [parts, 32, 8, 8], capi.BFLOAT16, 3)
-    one = HT.from_logical(np.ones(32), affine)
-    _, m, _ = run_batchnorm(ctx, x, training=True, eps=1e-3, scale=one, bias=one)
-    assert f"workgroups={parts}" in ctx.last_kernel(), ctx.last_kernel()
+# 64 rows of 32 channels are a round of the row lanes, eight of them a block: blocks on both sides of
+# the rounds of loads that add them, channels in one and several groups, the last one part of a group
+@pytest.mark.parametrize("n,c,parts", [
+    (1, 32, 1), (8, 32, 1), (9, 32, 2), (129, 32, 17), (1032, 32, 129), (2048, 32, 256), (2200, 32, 256),
+    (5, 8, 1), (7, 136, 2), (130, 72, 21), (9, 1032, 3), (13, 2048, 4),
+])
+@pytest.mark.parametrize("dtype,affine", [(capi.BFLOAT16, capi.FLOAT), (capi.FLOAT, capi.HALF)])
+def test_batchnorm_parts(ctx, n, c, parts, dtype, affine):
+    if dtype == capi.FLOAT and c > 1024:
+        pytest.skip("more channels than the kernel takes")
+    x = whole(n, [n, c, 8, 8], dtype, 3)
+    one = HT.from_logical(np.ones(c), affine)
+    y, m, v = run_batchnorm(ctx, x, training=True, eps=1e-3, scale=one, bias=one)
+    if dtype == capi.BFLOAT16:
+        assert ctx.last_kernel().endswith(f"workgroups={parts}"), ctx.last_kernel()
     # (one division and one addition to the pivot, each rounded once)
-    np.testing.assert_allclose(m, x.logical().mean(axis=(0, 2, 3)), rtol=0, atol=3 * 2.0 ** -23)
+    mean = x.logical().mean(axis=(0, 2, 3))
+    np.testing.assert_allclose(m, mean, rtol=0, atol=3 * 2.0 ** -23)
+    # (exact sums: a few roundings of values near one, the last one to Y's type)
+    inv = 1 / np.sqrt(x.logical().astype(np.float64).var(axis=(0, 2, 3)) + 1e-3)
+    np.testing.assert_allclose(v, inv, rtol=2.0 ** -20)
+    ref = (x.logical() - mean[:, None, None]) * inv[:, None, None] + 1
+    step = 2.0 ** -8 if dtype == capi.BFLOAT16 else 2.0 ** -19
+    np.testing.assert_allclose(y.logical() if hasattr(y, "logical") else y, ref, rtol=step, atol=step)
+
+
+# (the pivot is a value of X)
+def test_batchnorm_writes_over_its_input(ctx):
+    x = whole(3, [9, 72, 17, 16], capi.BFLOAT16, 3)
+    y, m, _ = run_batchnorm(ctx, x, training=True, eps=1e-3)
+    d = capi.BatchNormDesc()
+    d.x, d.y, d.training, d.epsilon = x.desc(), x.desc(), 1, 1e-3
+    d.scale_dtype = d.bias_dtype = d.running_dtype = d.stats_dtype = capi.FLOAT
+    mean, inv = HT.empty([72], capi.FLOAT), HT.empty([72], capi.FLOAT)
+    bx, bm, bi = x.upload(ctx), mean.upload(ctx), inv.upload(ctx)
+    ctx.batchnorm_fwd(d, bx, bx, None, None, None, None, bm, bi)
+    np.testing.assert_array_equal(mean.fetch(ctx, bm).logical(), m)
+    np.testing.assert_array_equal(x.fetch(ctx, bx).logical(), y)
 
 
 # gathered tiles: runs of 32-pixel steps, added one by one, four and sixteen at a time
