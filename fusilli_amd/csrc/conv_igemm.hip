@@ -27,6 +27,7 @@ struct ConvPlan {
   ConvGeom geom{};
   int bm = 256, bn = 128;
   bool halo = false;
+  bool for_halo = false; // gather 128 x 128 where the halo tiles would take a second round
   int tile_rows = 0; // halo mode: rows per M tile (<= bm)
   // grouped convolution: one GEMM per group (the kernel's outer batch dim)
   // over the group's channel runs of X, its rows of W and its columns of OUT;
@@ -273,13 +274,21 @@ ConvPlan make_plan(const fhip_conv_desc *d, const fhip_conv_desc *orig = nullptr
          // the gather: 55.6 vs 74 us for C = K = 128, 56 x 56; 24 vs 32 us for
          // C = K = 256, 14 x 14 at N = 32 and 46 vs 52 us at N = 128
       bm = small256 && big ? 256 : (fits128 ? 128 : 0);
-    // ... unless the gather would run its 128 x 128 tiles (eight wavefronts,
-    // two workgroups per compute unit) over two rounds of the machine or more:
-    // C256 -> K64 1 x 1 at 56 x 56 24.8 -> 18.0 us, C = K = 128 3 x 3 at 56 x 56
-    // and N = 64 98 -> 84 us (C = K = 128 at 28 x 28, 196 tiles: halo 16.2, gather 20.7)
-    if (want < 0 && bm == 128 && p.bm == 128 && p.bn == 128 &&
-        ((p.M + 127) / 128) * ((p.N + 127) / 128) * p.groups >= 512)
+    // ... unless the gather runs 128 x 128 tiles (eight wavefronts, two workgroups per compute
+    // unit) where the slab leaves room for one, over more than a round of the machine: bf16 3 x 3
+    // 256 -> 352, 13754 pixels, 324 tiles halo 54.1, gather 40.7 us; 192 -> 192, 49972, 782 tiles
+    // 58.5, 43.0; 5 x 5 64 -> 384, 12150, 285 tiles 39.6, 30.2 (60 layers of 257 to 1056 tiles 1.04 to
+    // 1.5 times, none slower; up to 256 tiles either by a tenth; N = 64 over two rounds of 64-wide
+    // columns 60.4, 48.8).  Two halo workgroups per compute unit win at any count: 64 -> 64, 5 x 5,
+    // 70756 pixels 26.5, gather 50.7; 64 -> 80, 3 x 3, 71424 21.1, 24.2; 64 -> 176, 33300 20.0, 24.
+    // Single taps: C64 -> K64 at 56 x 56.
+    const int64_t tiles128 = ((p.M + 127) / 128) * ((p.N + 127) / 128) * p.groups;
+    const bool two_rounds = p.bm == 128 && p.bn == 128 && tiles128 >= 512;
+    if (want < 0 && bm == 128 && (reach == 0 ? two_rounds : !small128 && (narrow ? two_rounds : tiles128 > 256))) {
       bm = 0;
+      p.bm = p.bn = 128;
+      p.for_halo = !two_rounds;
+    }
     // a single tap has nothing to reuse in the slab (C128 -> K512 at 28 x 28:
     // halo 19.6, gather 12.9 us; C256 -> K1024 at 14 x 14: 13.9, 11.4 us);
     // with one K slice in all the halo kernel's shorter set-up still wins
@@ -384,7 +393,8 @@ bool copies_pay(const ConvResolved &r, int64_t J, bool fused) {
   if (p.halo && p.bm == 256) // (N10 56 -> 256: 28.7 / 34.6, 30.7 / 47.1; 24 -> 384, 37 x 37: 28.8 / 22.4)
     return fused ? J >= 480 || (J >= 280 && full >= 0.68 && fill >= 0.75) || (mn >= 2.4e7 && full >= 0.85)
                  : J >= 480 && seventh && full >= 0.7 && fill >= 0.8;
-  if (p.halo) // (N39 216 -> 352, 30 x 18: 61 / 69, 63 / 73; N32 136 -> 256, 28 x 28: 51 / 39, 54 / 44)
+  // (halo times; on the gather in its place the first one's product 66.2 -> 51.7)
+  if (p.halo || p.for_halo) // (N39 216 -> 352, 30 x 18: 61 / 69, 63 / 73; N32 136 -> 256, 28 x 28: 51 / 39, 54 / 44)
     return ((seventh || ((r.Cp - r.C) * 5 <= r.C && mn * (double)J >= 1.4e10)) && J >= 1000 && fill >= 0.8 &&
             full >= (fused ? 0.75 : 0.8)) ||
            (fused && J >= 400 && J <= 600 && tiles >= 300 && (r.Cp - r.C) * 3 <= r.C);

@@ -643,3 +643,24 @@ def test_conv_gather_repeats_its_bits(ctx):
         got = out.fetch(ctx, do).logical().reshape([15, 2] + ydims[1:])
         assert np.array_equal(got, np.broadcast_to(got[:1], got.shape)), f"launch {i}"
         assert_close(got[0], ref, capi.FLOAT, f"launch {i}", rtol=1e-4)
+
+
+@pytest.mark.parametrize("n,c,hw,k,r,route", [
+    (22, 128, 32, 192, 3, "gather 128x128"),   # 352 tiles, the slab of one workgroup fills a compute unit
+    (16, 128, 32, 192, 3, "halo 128x128"),     # 256: one round
+    (164, 64, 20, 48, 5, "halo 128x64"),       # 513 tiles, two workgroups per compute unit
+    (164, 64, 20, 80, 5, "halo 128x128"),
+    (64, 256, 32, 64, 3, "gather 128x128"),    # 512 tiles of half their width
+])
+def test_conv_halo_and_gather_by_rounds(ctx, n, c, hw, k, r, route):
+    # the batch repeats two images of whole numbers: exact sums, the same in every copy
+    xd, wd = [n, c, hw, hw], [k, c, r, r]
+    rng = np.random.default_rng(n + k)
+    pair = rng.integers(-1, 2, size=[2] + xd[1:]).astype(np.float64)
+    x = HT.from_logical(np.concatenate([pair] * (n // 2)), capi.BFLOAT16, oracle.channels_last_strides(xd))
+    w = HT.from_logical(rng.integers(-1, 2, size=wd), capi.BFLOAT16, oracle.channels_last_strides(wd))
+    pad = [r // 2, r // 2]
+    got = run(ctx, x, w, pad, [1, 1], [1, 1], capi.FLOAT, out_dtype=capi.FLOAT).logical()
+    assert ctx.last_kernel().startswith(f"conv_igemm {route}"), ctx.last_kernel()
+    ref = oracle.conv_fprop(pair, w.logical(), pad, [1, 1], [1, 1])
+    assert np.array_equal(got.reshape([n // 2, 2, k, hw, hw]), np.broadcast_to(ref, [n // 2, 2, k, hw, hw]))
