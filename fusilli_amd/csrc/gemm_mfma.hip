@@ -208,6 +208,18 @@ GemmPlan make_plan(const fhip_matmul_desc *d, bool ragged) {
       }
     }
   }
+  // (the estimate counts 128 x 128 tiles that share a compute unit as two rounds; measured, a round of
+  // 257 to 512 of them is less than half again as long as one of 256: us, 256 x 128 / 128 x 128, bf16
+  // 2048 x 3200 x 3008 47.3 / 42.1, 1856 x 3064 x 3648 55.5 / 47.7, 2812 x 1600 x 256 with GELU 21.8 / 18.1, fp8
+  // 3328 x 1792 x 2432 22.9 / 19.2, int8 1728 x 2656 x 2560 26.6 / 22.6; of 17 such products among 500
+  // random ones the mean takes 8 % less, the slowest 2 % more.  Flat results go either way, int8 569 x
+  // 7296 x 2304 22.9 / 24.3; rows that start inside a cache line are read twice by neighbours on other
+  // compute units, 1264 x 4928 x 2608 47.0 / 54.4; so are the bytes of a row-major B, fp8 832 x 5520 x
+  // 1792 17.5 / 23.6.)
+  const double pairs = tiles(128, 128);
+  if (p.bm == 256 && p.bn == 128 && p.ksplit == 1 && pairs > 256 && pairs <= 512 &&
+      p.N <= 6 * p.M && p.K * elem % kTileKBytes == 0 && (k16 || p.b_kc))
+    p.bm = 128;
   if (fhip_knobs().gemm_tile_bm) {
     const int bm = fhip_knobs().gemm_tile_bm, bn = fhip_knobs().gemm_tile_bn;
     if ((bm == 128 || bm == 256) &&

@@ -232,3 +232,18 @@ def test_chains_of_four(ctx, dtype, m, n, k):
     x = 0.25 * ref_matmul(a, b)
     act = oracle.pointwise(capi.PW["SWISH_FWD"], [x], swish_beta=0.7)
     assert_close(got, 2.0 - (act - bias.logical()), dtype, name)
+
+
+# 257 to 512 tiles of 128 x 128 in place of 256 x 128 ones; flat results, cut slices and row-major bytes
+# stay on those
+@pytest.mark.parametrize("dtype,m,n,k,tb,tile", [
+    (capi.BFLOAT16, 2176, 1984, 1216, False, "128x128"), (capi.HALF, 3177, 1920, 896, True, "128x128"),
+    (capi.FP8E4M3, 3328, 1792, 2432, True, "128x128"), (capi.INT8, 1728, 2656, 2560, True, "128x128"),
+    (capi.INT8, 569, 7296, 2304, True, "256x128"), (capi.BFLOAT16, 1264, 4928, 2608, True, "256x128"),
+    (capi.FP8E4M3, 832, 5520, 1792, False, "256x128"),
+])
+def test_tiles_in_pairs(ctx, dtype, m, n, k, tb, tile):
+    a, b = make_operand(87, 0, m, k, dtype, False), make_operand(87, 1, k, n, dtype, tb)
+    got, name, odt = run(ctx, a, b)
+    assert name.endswith(f"{tile} waves=8 split=1"), name
+    check(got, ref_matmul(a, b), odt, name)
