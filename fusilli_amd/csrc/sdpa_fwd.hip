@@ -443,7 +443,9 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_fwd_kernel(SdpaArgs g) {
       __builtin_amdgcn_s_waitcnt(sd_wait_imm(2 * kLoadsPerTile + 8));
   };
   // kTight: only the next tile's mask, or (three stages, wavefronts 0..3) the K tile behind
-  // the next may be out
+  // the next may be out.  The mask is the youngest load wherever one has been issued behind K and V,
+  // which wavefronts 4..7 do in the vector-ALU phase: they wait for 0 in their first round, whose barrier
+  // comes ahead of that phase.
   auto wait_tight = [&]() {
     if (MASK != 2 && kStagesK == 3 && !team)
       __builtin_amdgcn_s_waitcnt(sd_wait_imm(kLoadsPerTile));
@@ -687,7 +689,9 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_fwd_kernel(SdpaArgs g) {
     // round has landed (which, in the vector-ALU phase, have not been issued
     // yet)
     if (team) {
-      if constexpr (kTight)
+      if constexpr (kTight && FIRST)
+        __builtin_amdgcn_s_waitcnt(sd_wait_imm(0));
+      else if constexpr (kTight)
         wait_tight();
       else
         __builtin_amdgcn_s_waitcnt(sd_wait_imm(kLoadsInValuPhase ? 0 : 2 * kLoadsPerTile));

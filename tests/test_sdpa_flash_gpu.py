@@ -348,7 +348,8 @@ def test_flash_folded_groups(ctx, knobs, layout, hkv, split, sq):
     assert_close(out.logical(), oracle.sdpa(q.logical(), k.logical(), v.logical()), capi.BFLOAT16)
 
 
-@pytest.mark.parametrize("causal,masked,hd", [(False, False, 128), (True, False, 128), (False, True, 64)])
+@pytest.mark.parametrize("causal,masked,hd", [(False, False, 128), (True, False, 128), (False, True, 64),
+                                              (False, True, 128)])
 def test_flash_split_keys_lose_no_precision(ctx, knobs, causal, masked, hd):
     # Probabilities are rounded against each team's reference point: the error against 64 bits may not
     # grow (sums over 100 000 independent roundings; the ratio moves by a percent or so).
@@ -403,3 +404,27 @@ def test_flash_split_keys_dead_rows(ctx, knobs, hd):
     rows = np.arange(96) != 17
     ref = oracle.sdpa(q.logical(), k.logical(), v.logical(), mask=mask.logical())
     assert_close(out[:, :, rows], ref[:, :, rows], capi.HALF)
+
+
+@pytest.mark.parametrize("mdt", [capi.BOOLEAN, capi.BFLOAT16])
+@pytest.mark.parametrize("hd", [128, 64])
+def test_flash_split_keys_mask_on_a_full_machine(ctx, knobs, mdt, hd):
+    # 512 workgroups on the same data, seven key tiles: a tile that is read before all wavefronts' loads of it
+    # have landed differs between copies when memory is busy
+    knobs(SDPA_SPLIT=1)
+    sq, skv = 256, 448
+    q, k, v = (rand(67, i, [1, 1, n, hd], std=1.5) for i, n in enumerate((sq, skv, skv)))
+    m = rand(67, 3, [1, 1, sq, skv])
+    if mdt == capi.BOOLEAN:
+        m = (m > -0.5).astype(np.float64)
+        m[..., -1] = 1
+    mask = HT.from_logical(m, mdt)
+    wide = [HT.from_logical(np.broadcast_to(t, [8, 32] + list(t.shape[2:])), capi.BFLOAT16) for t in (q, k, v)]
+    one = [HT.from_logical(t, capi.BFLOAT16).logical() for t in (q, k, v)]
+    ml = mask.logical()
+    ref = oracle.sdpa(*one, mask=ml.astype(bool) if mdt == capi.BOOLEAN else ml)
+    for launch in range(3):
+        out = run(ctx, *wide, mask=mask).logical()
+        assert ctx.last_kernel().endswith("split"), ctx.last_kernel()
+        assert np.array_equal(out, np.broadcast_to(out[:1, :1], out.shape)), launch
+        assert_close(out[:1, :1], ref, capi.BFLOAT16, f"launch {launch}")
