@@ -113,8 +113,8 @@ def test_direct_weight_gradient_of_other_paddings_and_channels(ctx, x, k, pad, s
     np.testing.assert_array_equal(dw.logical(), ref)
 
 
-def test_direct_weight_gradient_meets_no_values_outside(ctx):
-    # infinite values in the channels, rows and columns next to a block's own: each gradient shows its own
+def test_direct_weight_gradient_meets_no_channels_outside(ctx):
+    # infinite values in the channel next to a gradient's own, in the same blocks
     x, dy = whole(5, [8, 40, 40, 30], capi.BFLOAT16, 2), whole(6, [8, 72, 40, 30], capi.BFLOAT16, 1)
     xv, w = x.logical().copy(), [72, 40, 3, 3]
     xv[:, 39] = np.inf
@@ -124,6 +124,32 @@ def test_direct_weight_gradient_meets_no_values_outside(ctx):
     ref = oracle.conv_wgrad(dy.logical(), x.logical(), w, [1, 1], [1, 1], [1, 1])
     np.testing.assert_array_equal(dw[:, :39], HT.from_logical(ref, capi.BFLOAT16).logical()[:, :39])
     assert not np.isfinite(dw[:, 39]).any()
+
+
+# Infinite values of X in border rows and columns, a channel for each: the taps that meet them show it and no
+# other (DY rows and columns that do not exist are zeros in registers).  Steps of 16 pixels full and not,
+# channels in whole blocks of 32 and off them, every padding.
+@pytest.mark.parametrize("pad", [0, 1, 2])
+@pytest.mark.parametrize("n,p,q,steps", [(60, 17, 14, 1), (16, 40, 30, 2), (20, 27, 32, 2), (12, 36, 45, 3),
+                                         (20, 16, 50, 4), (12, 29, 56, 4), (400, 1, 20, 2), (260, 2, 17, 2)])
+@pytest.mark.parametrize("c,k", [(40, 72), (64, 32)])
+def test_direct_weight_gradient_meets_no_rows_or_columns_outside(ctx, pad, n, p, q, steps, c, k):
+    h, w = p + 2 - 2 * pad, q + 2 - 2 * pad
+    if h < 1:
+        pytest.skip("no rows of X")
+    x, dy = whole(n, [n, c, h, w], capi.BFLOAT16, 2), whole(n + 1, [n, k, p, q], capi.BFLOAT16, 1)
+    xv = x.logical().copy()
+    for i, (axis, at) in enumerate((a, b) for a in (2, 3) for b in (0, 1, 2, -3, -2, -1)):
+        if -xv.shape[axis] <= at < xv.shape[axis]:
+            np.moveaxis(xv[:, 3 * i], axis - 1, 0)[at] = np.inf
+    xt = HT.from_logical(xv, capi.BFLOAT16, oracle.channels_last_strides(xv.shape))
+    geom = ([k, c, 3, 3], [pad, pad], [1, 1], [1, 1])
+    got = run_conv_wgrad(ctx, dy, xt, *geom, capi.BFLOAT16, tuned=None).logical()
+    assert ctx.last_kernel().startswith(f"conv_wgrad_direct steps={steps}"), ctx.last_kernel()
+    ref = HT.from_logical(oracle.conv_wgrad(dy.logical(), xt.logical(), *geom), capi.BFLOAT16).logical()
+    np.testing.assert_array_equal(np.isfinite(got), np.isfinite(ref))
+    assert np.isfinite(ref).any(axis=(0, 2, 3)).sum() > 20  # (and most channels meet none)
+    np.testing.assert_array_equal(got[np.isfinite(ref)], ref[np.isfinite(ref)])
 
 
 # the mirrored filter of a data gradient, copied in blocks of 64 x 64: edges of the blocks, groups, and a
