@@ -77,9 +77,9 @@ int fhip_gather_conv_wgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *d
                            const void *x, void *dw, bool *handled);
 
 // Weight gradient of 3 x 3, unit-stride convolutions straight from X and DY (no operand
-// copies): one MFMA kernel plus the sum of its partial results, in the workspace where it
-// holds them, else in the context's scratch.  The first says for which it reports the workspace; `handled`
-// false: a problem for fhip_fast_conv_wgrad's gathered tiles.
+// copies): one MFMA kernel plus the sum of its partial results, as many as the descriptor's workspace
+// (`workspace_bytes`) holds; without one they lie in the context's scratch.  The first says for which it
+// reports the workspace; `handled` false: a problem for fhip_fast_conv_wgrad's gathered tiles.
 bool fhip_fast_conv_wgrad_direct_applicable(const fhip_conv_desc *d,
                                             size_t *workspace_bytes);
 int fhip_fast_conv_wgrad_direct(fhip_ctx *ctx, const fhip_conv_desc *d,

@@ -1592,7 +1592,7 @@ int fhip_conv_wgrad(fhip_ctx *ctx, const fhip_conv_desc *d, const void *dy,
                  "(fhip_conv_wgrad_workspace_size), got %zu",
                  need, workspace ? workspace_bytes : (size_t)0);
     FHIP_HIP_CHECK(ctx, hipSetDevice(ctx->device));
-    return fhip_fast_conv_wgrad(ctx, d, dy, x, dw, workspace, workspace_bytes);
+    return fhip_fast_conv_wgrad(ctx, d, dy, x, dw, workspace, need);
   }
   dim3 grid;
   FHIP_REQUIRE(ctx, conv_wgrad_grid(d, &grid),

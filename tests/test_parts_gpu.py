@@ -6,7 +6,7 @@ import pytest
 from fusilli_amd import capi
 from oracle import oracle
 from helpers import HT
-from test_generic_ops_gpu import run_batchnorm, run_conv_dgrad, run_conv_wgrad
+from test_generic_ops_gpu import conv_bwd_desc, run_batchnorm, run_conv_dgrad, run_conv_wgrad
 
 pytestmark = pytest.mark.gpu
 
@@ -150,6 +150,26 @@ def test_direct_weight_gradient_meets_no_rows_or_columns_outside(ctx, pad, n, p,
     np.testing.assert_array_equal(np.isfinite(got), np.isfinite(ref))
     assert np.isfinite(ref).any(axis=(0, 2, 3)).sum() > 20  # (and most channels meet none)
     np.testing.assert_array_equal(got[np.isfinite(ref)], ref[np.isfinite(ref)])
+
+
+# Layers for which more parts would be faster than the descriptor's workspace holds, its own and the gathered
+# tiles': all parts lie there all the same (graphs with a workspace each share nothing else).
+@pytest.mark.parametrize("x,k,parts", [([45, 448, 21, 1], 320, 1), ([1, 264, 45, 22], 128, 2)])
+def test_direct_weight_gradient_stays_in_the_workspace(ctx, x, k, parts):
+    xt, dy = whole(k, x, capi.BFLOAT16, 2), whole(k + 1, [x[0], k] + x[2:], capi.BFLOAT16, 1)
+    w, geom = [k, x[1], 3, 3], ([1, 1], [1, 1], [1, 1])
+    dw = HT.empty(w, capi.BFLOAT16, oracle.channels_last_strides(w))
+    d = conv_bwd_desc(xt, dw, dy, *geom)
+    need, used = ctx.conv_wgrad_workspace(d), parts * -(-k // 32) * -(-x[1] // 32) * 9 * 1024
+    assert need >= used * 4
+    space = ctx.to_device(np.full(need // 4, np.nan, np.float32))
+    bdy, bx, bdw = dy.upload(ctx), xt.upload(ctx), dw.upload(ctx)
+    ctx.conv_wgrad(d, bdy, bx, bdw, space)
+    name = ctx.last_kernel()
+    assert name.startswith("conv_wgrad_direct") and name.endswith(f"parts={parts}"), name
+    assert np.isfinite(space.download(np.float32)[:used]).all()
+    ref = HT.from_logical(oracle.conv_wgrad(dy.logical(), xt.logical(), w, *geom), capi.BFLOAT16)
+    np.testing.assert_array_equal(dw.fetch(ctx, bdw).logical(), ref.logical())
 
 
 # the mirrored filter of a data gradient, copied in blocks of 64 x 64: edges of the blocks, groups, and a
