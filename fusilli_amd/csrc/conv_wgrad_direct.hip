@@ -622,7 +622,11 @@ int fhip_fast_conv_wgrad_direct(fhip_ctx *ctx, const fhip_conv_desc *d,
   const int64_t most = (1ll << 31) / kWdBlock / p.a.types, held = (int64_t)(workspace_bytes / kBytes) / p.a.types;
   if (workspace && held < 1)
     return 0;
-  p.a.nparts = wd_parts(p.a, p.nks, workspace && held < most ? held : most);
+  // Gradients stored in f32 show how long a wavefront's chain of additions is: all parts that the workspace has
+  // (error against 64 bits, time: N14 320 -> 480, 24 x 24 in two parts 1.36e-7, 50.8 us, in one 1.87e-7, 44.4; N11
+  // 288 -> 480, 29 x 29 in three 1.26e-7, 41.8, in one 2.05e-7, 41.3; N14 64 -> 192, 14 x 14 in 28 8.2e-8,
+  // 19.5, in five 8.4e-8, 11.3).
+  p.a.nparts = d->w.dtype == FHIP_FLOAT ? (int32_t)held : wd_parts(p.a, p.nks, workspace && held < most ? held : most);
   void *part = workspace;
   if (!workspace) {
     const size_t bytes = (size_t)p.a.types * p.a.nparts * kBytes;

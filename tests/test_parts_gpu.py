@@ -172,6 +172,22 @@ def test_direct_weight_gradient_stays_in_the_workspace(ctx, x, k, parts):
     np.testing.assert_array_equal(dw.fetch(ctx, bdw).logical(), ref.logical())
 
 
+# Gradients stored in f32 keep the parts that their workspace has room for, however few are faster: fewer parts
+# are longer chains of f32 additions.  16-bit gradients take the planner's count.
+@pytest.mark.parametrize("x,k,parts,few", [([14, 320, 24, 24], 480, 2, 1), ([14, 64, 14, 14], 192, 28, 5)])
+@pytest.mark.parametrize("dtype", [capi.FLOAT, capi.BFLOAT16])
+def test_direct_weight_gradient_parts_by_type(ctx, x, k, parts, few, dtype):
+    xt, dy = whole(k, x, capi.BFLOAT16, 2), whole(k + 1, [x[0], k] + x[2:], capi.BFLOAT16, 1)
+    w, geom = [k, x[1], 3, 3], ([1, 1], [1, 1], [1, 1])
+    dw = HT.empty(w, dtype, oracle.channels_last_strides(w))
+    assert ctx.conv_wgrad_workspace(conv_bwd_desc(xt, dw, dy, *geom)) == parts * (k // 32) * (x[1] // 32) * 36864
+    got = run_conv_wgrad(ctx, dy, xt, w, *geom, capi.BFLOAT16, tuned=True, w_dtype=dtype).logical()
+    assert ctx.last_kernel().endswith(f" parts={parts if dtype == capi.FLOAT else few}"), ctx.last_kernel()
+    # (some blocks of a large one)
+    ref = oracle.conv_wgrad(dy.logical()[:, -64:], xt.logical()[:, -64:], [64, 64, 3, 3], *geom)
+    np.testing.assert_array_equal(got[-64:, -64:], HT.from_logical(ref, dtype).logical())
+
+
 # the mirrored filter of a data gradient, copied in blocks of 64 x 64: edges of the blocks, groups, and a
 # channel count that the copy takes element by element
 @pytest.mark.parametrize("x,k,w", [
