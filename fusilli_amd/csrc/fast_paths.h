@@ -114,11 +114,12 @@ bool fhip_fast_sdpa_applicable(const fhip_sdpa_desc *d);
 int fhip_fast_sdpa(fhip_ctx *ctx, const fhip_sdpa_desc *d, const void *q,
                    const void *k, const void *v, const void *mask, void *o);
 
+// Estimate of the tiled kernel where it folds grouped heads or splits the keys between teams, else -1.
+double fhip_flash_sdpa_us(const fhip_sdpa_desc *d);
+
 // Few query rows per key / value head (decode): keys split over workgroups.  For
 // descriptors that fhip_fast_sdpa takes; `handled` false where the tiled kernel is
 // the faster one.
-// Estimate of the tiled kernel where it folds grouped heads or splits the keys between teams, else -1.
-double fhip_flash_sdpa_us(const fhip_sdpa_desc *d);
 int fhip_decode_sdpa(fhip_ctx *ctx, const fhip_sdpa_desc *d, const void *q,
                      const void *k, const void *v, void *o, bool *handled);
 

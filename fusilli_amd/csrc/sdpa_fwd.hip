@@ -33,9 +33,10 @@
 //
 // Where workgroups of 256 rows are few, or fill a round and a little more (SPLIT): 128 rows
 // per workgroup, of which both teams of four wavefronts own the same rows and take every
-// other key tile.  A team has rings of its own (two stages: a round of lead) and loads its own
-// tiles; in the end the teams exchange halves of O^T with their reference points and sums.  A
-// round is a little longer (twice the LDS-DMA) and there are half as many.
+// other key tile.  A team has rings of its own (head dim 64: three stages of K and of V; 128: two of V, and
+// three of K, two under a mask) and loads its own tiles; in the end the teams exchange halves of
+// O^T with their reference points and sums.  A round is a little longer (twice the
+// LDS-DMA) and there are half as many.
 //
 // Reference semantics: aten.scaled_dot_product_attention (reference
 // support/asm_emitter.h:2409-2468, node/sdpa_node.h:36-236), GQA by head
@@ -73,7 +74,6 @@ template <int HD> struct SdShape {
   static constexpr int kChunks = kRowB / 16;       // 16-byte chunks per row
   static constexpr int kRowsPerLoad = 64 / kChunks; // rows of one wave DMA
   static constexpr int kTileB = kBKV * kRowB;      // one K (or V) tile
-  static constexpr int kLoadsPerTile = kTileB / 1024 / kWaves; // per wave
   static constexpr int kOutPitch = kRowB + 16;     // epilogue rows, padded
   static constexpr int kRingB = 2 * kStages * kTileB; // K ring and V ring
   static constexpr int kLdsB = kRingB > kWaves * 32 * kOutPitch
@@ -347,7 +347,7 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_fwd_kernel(SdpaArgs g) {
     koff[j] = (uint32_t)(row * k_rowb + ((p ^ sd_kswz<HD>(row)) << 4));
     voff[j] = (uint32_t)(row * v_rowb + (sd_vchunk<HD>(row, p) << 4));
   }
-  // K tiles live in stages [0, kStages), V tiles in [kStages, 2 kStages).
+  // K tiles live in stages [0, kStagesK) of a ring, V tiles behind them.
   // One buffer descriptor per operand covers the whole (batch, head) slab; the
   // tile's byte offset is added to the lanes' offsets.  Rows at or past Skv
   // read as zeros (out of the descriptor's range), and so do whole tiles past
@@ -468,7 +468,7 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_fwd_kernel(SdpaArgs g) {
           (int)(off[j] + toff), 0, 0, 0);
     }
   };
-  // ring slot (0 .. kStages - 1) -> LDS address
+  // ring slot (0 .. the operand's stages - 1) -> LDS address
   const uint32_t ring = lds0 + (SPLIT ? (uint32_t)team * (uint32_t)(C::split_lds(MASK != 0) / 2) : 0u);
   auto k_stage = [&](int slot) { return ring + (uint32_t)slot * kTileB; };
   auto v_stage = [&](int slot) {
