@@ -2,6 +2,8 @@
 have to grow the context's scratch do without it; on one that has, the scratch that the
 graph names outlives later growth.  Every replay is compared with the eager result of a
 second context."""
+import ctypes
+
 import pytest
 
 from fusilli_amd import capi
@@ -101,10 +103,38 @@ def _channel_means(torch):
     return _reduce(torch, False)
 
 
+# (more parts than the workspace holds would be faster: recorded or not, it bounds them, so the bits agree)
+def _weight_gradient(torch, n, c, h, w, k):
+    cl = lambda n, c, h, w: capi.TensorDesc.make([n, c, h, w], [c * h * w, 1, c * w, c], capi.BFLOAT16)  # noqa: E731
+    x = torch.randn(n, h, w, c, device="cuda", dtype=torch.bfloat16)
+    dy = torch.randn(n, h, w, k, device="cuda", dtype=torch.bfloat16)
+    out = torch.empty(k, 3, 3, c, device="cuda", dtype=torch.bfloat16)
+    d = capi.ConvDesc()
+    d.x, d.w, d.y = cl(n, c, h, w), cl(k, c, 3, 3), cl(n, k, h, w)
+    d.spatial_rank = 2
+    for i in range(2):
+        d.stride[i] = d.dilation[i] = d.padding[i] = 1
+    d.epilogue = capi.make_epilogue([])
+    need = ctypes.c_size_t(0)
+    assert capi.load().fhip_conv_wgrad_workspace_size(ctypes.byref(d), ctypes.byref(need)) == 0
+    space = torch.empty(need.value, device="cuda", dtype=torch.uint8)
+    return x, out, lambda c: c.conv_wgrad(d, dy.data_ptr(), x.data_ptr(), out.data_ptr(), space.data_ptr()), 0.0
+
+
+def _weight_gradient_own(torch):
+    return _weight_gradient(torch, 45, 448, 21, 1, 320)
+
+
+def _weight_gradient_gathered(torch):
+    return _weight_gradient(torch, 1, 264, 45, 22, 128)
+
+
 # what runs where there is scratch
 ROUTES = {_matmul_tiled: "gemm_mfma bf16 128x128 waves=8 split=16",
           _conv_padded: "conv_igemm gather 256x128 split=1 padded=1 groups=1",
-          _conv_split: "conv_igemm gather 128x128 split=8 padded=0 groups=1"}
+          _conv_split: "conv_igemm gather 128x128 split=8 padded=0 groups=1",
+          _weight_gradient_own: "conv_wgrad_direct steps=1 parts=1",
+          _weight_gradient_gathered: "conv_wgrad_direct steps=2 parts=2"}
 
 
 @pytest.mark.parametrize("make", [_norm, _sdpa, _matmul])
@@ -153,7 +183,7 @@ def test_replay_after_scratch_has_grown(make):
 
 
 @pytest.mark.parametrize("make", [_norm, _sdpa, _matmul, _matmul_tiled, _conv_padded, _conv_split, _bias_gradient,
-                                  _channel_means])
+                                  _channel_means, _weight_gradient_own, _weight_gradient_gathered])
 def test_first_call_under_capture(make):
     import torch
     torch.manual_seed(1)
